@@ -9,6 +9,7 @@
 #include "prof.h"
 #include "dion.h"
 #include "ns_flow.h"
+#include "ns_small.h"
 
 namespace {
 
@@ -20,6 +21,19 @@ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // with 128 bytes of padding), so such rows get 128 bytes more.
 inline int padded_pitch(int n, size_t esz) { return ((size_t)n * esz) % 4096 == 0 ? n + (int)(128 / esz) : n; }
 
+inline int round_up(int x, int g) { return (x + g - 1) / g * g; }
+
+// Working dimension of a bf16 product of the batched kernels.  Padding is exact (zero rows and columns go through the
+// iteration unchanged) and buys the K loop without bounds checks: with the padding done inside the staging and update
+// passes instead of on copies, a Muon step over 14 matrices of 1021, 341 and 2731 rows / columns 1.45 -> 0.85 ms.  Whole
+// 256-tiles where that costs at most 7 % more than whole 128-tiles.
+inline int padded_dim(int x) {
+  const int r128 = round_up(x, 128), r256 = round_up(x, 256);
+  return r256 * 100LL <= r128 * 107LL ? r256 : r128;
+}
+
+constexpr size_t FLOW_TAIL_BYTES = 1536;   // behind the counters of a control area: ticket, owner and status words
+
 struct NsLayout {
   int mw = 0, nw = 0, tiles = 0;
   int ldx = 0, lda = 0;   // row pitches of the mw x nw iterates and of the mw x mw Gram / polynomial
@@ -27,20 +41,27 @@ struct NsLayout {
   size_t x_bytes = 0, a_bytes = 0, part_bytes = 0, flow_bytes = 0;  // per matrix
   size_t per_matrix = 0;
   NsLayout() {}
-  NsLayout(int m, int n, int dtype) {
+  // m x n matrices; `small`: the layout of the one-launch kernel for small matrices (ns_small.hip), which never needs
+  // more memory than the other one
+  NsLayout(int m, int n, int dtype, bool small = false) {
     mw = m < n ? m : n;
     nw = m < n ? n : m;
-    tiles = da_stage_tiles(m, n);
+    if (dtype != DA_BF16) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
+    else if (small) { mw = round_up(mw, DA_SMALL_BT); nw = round_up(nw, DA_SMALL_BT); }
+    else { mw = padded_dim(mw); nw = padded_dim(nw); }
+    tiles = da_stage_tiles(m, n, mw, nw);
     esz = dtype == DA_BF16 ? 2 : 4;
     // no padding between matrices: with every pitch a multiple of 8 each one starts 16-byte aligned
     ldx = padded_pitch(nw, esz);
     lda = padded_pitch(mw, esz);
     x_bytes = (size_t)mw * ldx * esz;
     a_bytes = (size_t)mw * lda * esz;
-    part_bytes = align_up((size_t)tiles * sizeof(float) + sizeof(float), 256);
-    // control words of the persistent Newton-Schulz kernel: cb * flow_bytes >= da_ns_flow_ctl_bytes(cb) for cb >= 1
+    part_bytes = align_up((size_t)tiles * sizeof(float), 256);
+    // control words of the persistent Newton-Schulz kernels: cb * flow_bytes >= da_ns_flow_ctl_bytes(cb) for cb >= 1
     // (+ 16: one slot of the table of weight pointers that the last product's epilogue updates)
-    flow_bytes = DA_FLOW_CTR_STRIDE * sizeof(int) + 256 + 16;
+    flow_bytes = DA_FLOW_CTR_STRIDE * sizeof(int) + FLOW_TAIL_BYTES + 16;
+    static_assert(DA_SMALL_CTR_STRIDE <= DA_FLOW_CTR_STRIDE && DA_SMALL_TAIL * sizeof(int) + 128 <= FLOW_TAIL_BYTES,
+                  "the control area serves both");
     per_matrix = 2 * x_bytes + 2 * a_bytes + part_bytes + flow_bytes;
   }
   int chunk(int batch, size_t ws_bytes) const {
@@ -60,9 +81,9 @@ struct NsLayout {
 
 struct NsBuffers {
   char *x0 = nullptr, *x1 = nullptr, *a = nullptr, *b = nullptr;
-  float *partials = nullptr, *divisor = nullptr;
+  float* partials = nullptr;
   int* flow = nullptr;
-  void** xtab = nullptr;   // per-matrix weight pointers (Muon: the last product updates the weights itself)
+  void** xtab = nullptr;   // per-matrix destinations (the last product stores or updates them itself)
   NsBuffers() {}
   NsBuffers(const NsLayout& L, void* ws, int cb) {
     char* p = static_cast<char*>(ws);
@@ -71,9 +92,8 @@ struct NsBuffers {
     a = p; p += L.a_bytes * cb;
     b = p; p += L.a_bytes * cb;
     partials = reinterpret_cast<float*>(p); p += L.part_bytes * cb;
-    divisor = partials + (size_t)L.tiles * cb;
     flow = reinterpret_cast<int*>(p);
-    xtab = reinterpret_cast<void**>(p + (DA_FLOW_CTR_STRIDE * sizeof(int) + 256) * (size_t)cb);
+    xtab = reinterpret_cast<void**>(p + (DA_FLOW_CTR_STRIDE * sizeof(int) + FLOW_TAIL_BYTES) * (size_t)cb);
   }
 };
 
@@ -226,39 +246,208 @@ int ns_iterate(const NsSet* sets, int nsets, int dtype, const float* coeffs, int
   return DA_OK;
 }
 
-int ns_iterate(const NsLayout& L, const NsBuffers& W, int cb, int dtype, const float* coeffs, int steps,
-               int faithful, hipStream_t s, char** result, const int** poison = nullptr) {
-  NsSet one;
-  one.L = L; one.W = W; one.cb = cb;
-  return ns_iterate(&one, 1, dtype, coeffs, steps, faithful, s, result, poison);
+// A bucket of same-shape matrices (m x n, at most DA_MAX_GROUPS of them per call of ns_jobs): sources G (row pitch ldg),
+// momentum M (null: plain cast), destinations X (row pitch ldx): the weights to update, or the result (update == 0).
+struct NsJob {
+  const void* const* G;
+  void* const* M;
+  void* const* X;
+  int cnt, m, n, ldg, ldx;
+  float decay, step;
+};
+struct NsCall {
+  int x_dtype, g_dtype, compute_dtype;   // momentum has the weights' dtype
+  int update;                            // 1: Muon step, 0: Newton-Schulz of the sources
+  float mu;
+  int nesterov;
+  const float* coeffs;
+  int steps;
+  float eps;
+  int faithful;
+};
+
+// Whether the one-launch kernel for small matrices takes these jobs.  Matrices are dealt to eight queues of one XCD's
+// workgroups each; what counts is the longest queue, in 64 x 64 x 64 stages per iteration.  Measured against the batched
+// launches (us per call): 912 stages (16 x 256 x 1024) 141 : 206, 1088 (512 x 512) 129 : 191, 3488 (512 x 2048) 260 : 286,
+// 3600 (768 x 768) 300 : 247, 3648 (64 x 256 x 1024) 348 : 279.
+bool ns_small_wanted(const NsJob* jobs, int nj, const NsCall& c) {
+  if (c.compute_dtype != DA_BF16 || !c.faithful || c.steps < 1 || c.steps > DA_SMALL_MAX_STEPS) return false;
+  if (da_ns_flow_mode() >= 0) return false;   // the caller chose between the other two
+  double load[8] = {0}, worst = 0;
+  int first = 0;
+  for (int i = 0; i < nj; ++i) {
+    const int mw = round_up(jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n, DA_SMALL_BT) / DA_SMALL_BT;
+    const int nw = round_up(jobs[i].m < jobs[i].n ? jobs[i].n : jobs[i].m, DA_SMALL_BT) / DA_SMALL_BT;
+    const double sym = 0.5 * mw * (mw + 1), stages = sym * nw + sym * mw + (double)mw * nw * mw;
+    for (int j = 0; j < jobs[i].cnt; ++j) load[(first + j) & 7] += stages;
+    first += jobs[i].cnt;
+  }
+  for (int q = 0; q < 8; ++q) worst = load[q] > worst ? load[q] : worst;
+  return worst <= 2500.0;
 }
 
-// The weights of `c` matrices starting at X[0] as a device table at `dst`, and the set's update parameters.
-int ns_set_update(NsSet& set, void* const* X, int first, int c, int m, int n, int x_dtype, float decay, float step,
-                  hipStream_t s) {
-  DaPtrTable t{};
-  for (int j = 0; j < c; ++j) t.p[j] = X[j];
-  set.update = 1; set.x_dtype = x_dtype; set.tall = m > n ? 1 : 0; set.x_ld = n; set.decay = decay; set.step = step;
-  return da_upload_ptrs(t, set.W.xtab + first, c, s);
-}
-
-// After a persistent launch that updated the weights itself: NaN in all of them if the launch gave up.
-int ns_poison_weights(void* const* X, int batch, int m, int n, int x_dtype, const int* poison, hipStream_t s) {
-  for (int j0 = 0; j0 < batch; j0 += DA_MAX_PTRS) {
-    const int c = batch - j0 < DA_MAX_PTRS ? batch - j0 : DA_MAX_PTRS;
-    DaPtrTable t{};
-    for (int j = 0; j < c; ++j) t.p[j] = X[j0 + j];
-    const int rc = da_poison_if(t, c, (long long)m * n, x_dtype, poison, s);
+int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStream_t s) {
+  if (nj < 1 || nj > DA_MAX_GROUPS) return DA_ERR_ARG;
+  const bool small = ns_small_wanted(jobs, nj, c);
+  // carve the workspace: every job keeps all of its matrices resident
+  NsSet sets[DA_MAX_GROUPS];
+  char* p = static_cast<char*>(workspace);
+  int total = 0;
+  for (int i = 0; i < nj; ++i) {
+    const NsJob& k = jobs[i];
+    NsSet& S = sets[i];
+    S.L = NsLayout(k.m, k.n, c.compute_dtype, small);
+    S.W = NsBuffers(S.L, p, k.cnt);
+    S.cb = k.cnt;
+    S.update = c.update; S.x_dtype = c.x_dtype; S.tall = k.m > k.n ? 1 : 0; S.x_ld = k.ldx; S.decay = k.decay; S.step = k.step;
+    p += align_up(S.L.per_matrix * (size_t)k.cnt, 256);
+    total += k.cnt;
+  }
+  int* ctl = nullptr;
+  if (small) {
+    // control words of all jobs in one piece: a single job's own area, else behind the last job, in the room that the
+    // jobs' areas leave (FLOW_TAIL_BYTES and more per matrix, of which 8 bytes are used)
+    ctl = sets[0].W.flow;
+    if (nj > 1) {
+      char* q = static_cast<char*>(workspace);
+      for (int i = 0; i < nj; ++i) {
+        NsSet& S = sets[i];
+        S.W = NsBuffers(S.L, q, jobs[i].cnt);
+        S.W.xtab = reinterpret_cast<void**>(S.W.flow);
+        q = reinterpret_cast<char*>(S.W.xtab + jobs[i].cnt);
+        q = static_cast<char*>(workspace) + align_up((size_t)(q - static_cast<char*>(workspace)), 128);
+      }
+      ctl = reinterpret_cast<int*>(q);
+    }
+  }
+  const double xsz = c.x_dtype == DA_BF16 ? 2 : 4, gsz = c.g_dtype == DA_BF16 ? 2 : 4;
+  // momentum update (or cast), staging in wide orientation, Frobenius partial sums
+  for (int i = 0, j0 = 0; i < nj;) {
+    DaStage st;
+    st.ngroups = 0;
+    st.g_dtype = c.g_dtype; st.m_dtype = c.x_dtype; st.w_dtype = c.compute_dtype;
+    st.mu = c.mu; st.nesterov = c.nesterov; st.muon = c.update;
+    st.zero = nullptr; st.nzero = 0; st.status = nullptr; st.preset = 0;
+    if (small && i == 0 && j0 == 0) {
+      st.zero = ctl; st.nzero = total * DA_SMALL_CTR_STRIDE + 8 * DA_SMALL_LINE;
+      st.status = ctl + st.nzero; st.preset = da_ns_flow_fail() ? 1 : 0;
+    }
+    int mats = 0;
+    double bytes = 0;
+    while (i < nj && st.ngroups < DA_MAX_GROUPS && mats < DA_STAGE_MATS) {
+      const NsJob& k = jobs[i];
+      const NsSet& S = sets[i];
+      const int n = k.cnt - j0 < DA_STAGE_MATS - mats ? k.cnt - j0 : DA_STAGE_MATS - mats;
+      DaStageGroup& g = st.g[st.ngroups++];
+      g.wide = S.W.x0 + (size_t)j0 * S.L.x_bytes;
+      g.partials = S.W.partials + (size_t)j0 * S.L.tiles;
+      g.xtab = S.W.xtab + j0;
+      g.rows = k.m; g.cols = k.n; g.ld = k.ldg;
+      g.mw = S.L.mw; g.nw = S.L.nw; g.ldw = S.L.ldx;
+      g.cnt = n;
+      for (int j = 0; j < n; ++j) {
+        st.src[mats + j] = k.G[j0 + j];
+        st.mom[mats + j] = k.M ? k.M[j0 + j] : nullptr;
+        st.dst[mats + j] = k.X[j0 + j];
+      }
+      mats += n;
+      // algorithmic bytes: read G (and M), write M and the working matrix
+      bytes += (double)k.m * k.n * (gsz + (c.update ? 2 * xsz : 0.0) + S.L.esz) * n;
+      j0 += n;
+      if (j0 == k.cnt) { ++i; j0 = 0; }
+    }
+    DaProfScope prof(DA_PROF_STAGE, bytes, s);
+    const int rc = da_stage(st, s);
     if (rc) return rc;
+  }
+  if (small) {
+    // costliest job first, as the kernel deals them
+    DaNsSmallGroup sg[DA_MAX_GROUPS];
+    int order[DA_MAX_GROUPS];
+    double flops = 0.0;
+    for (int i = 0; i < nj; ++i) {
+      const NsLayout& L = sets[i].L;
+      order[i] = i;
+      for (int j = i; j > 0; --j) {
+        const NsLayout &A = sets[order[j - 1]].L, &B = sets[order[j]].L;
+        if ((double)A.mw * A.mw * (3.0 * A.nw + A.mw) >= (double)B.mw * B.mw * (3.0 * B.nw + B.mw)) break;
+        const int t = order[j]; order[j] = order[j - 1]; order[j - 1] = t;
+      }
+      flops += (double)c.steps * jobs[i].cnt * ((double)L.mw * (L.mw + 1.0) * (L.nw + L.mw) + 2.0 * L.mw * L.mw * L.nw);
+    }
+    for (int i = 0; i < nj; ++i) {
+      const NsJob& k = jobs[order[i]];
+      const NsSet& S = sets[order[i]];
+      sg[i] = DaNsSmallGroup{S.W.x0, S.W.x1, S.W.a, S.W.b, (long long)(S.L.x_bytes / 2), (long long)(S.L.a_bytes / 2),
+                             S.L.mw, S.L.nw, S.L.ldx, S.L.lda, k.cnt, S.W.partials, S.L.tiles, S.W.xtab,
+                             c.x_dtype, k.m, k.n, k.ldx, c.update, k.decay, k.step};
+    }
+    DaProfScope prof(DA_PROF_NS_FLOW, flops, s);
+    return da_ns_small(sg, nj, c.coeffs, c.steps, c.eps, ctl, s);
+  }
+  for (int i = 0; i < nj; ++i) {
+    const NsLayout& L = sets[i].L;
+    DaProfScope prof(DA_PROF_NORMALIZE, 2.0 * (double)jobs[i].m * jobs[i].n * L.esz * jobs[i].cnt, s);  // (padding excluded)
+    const int rc = da_normalize(sets[i].W.x0, c.compute_dtype, (long long)(L.x_bytes / L.esz), jobs[i].cnt, sets[i].W.partials,
+                                L.tiles, c.eps, s);
+    if (rc) return rc;
+  }
+  // The last product updates the weights in its epilogue where it has whole tiles of them; otherwise (and for a plain
+  // result) a pass of its own follows.
+  bool whole = c.update != 0;
+  for (int i = 0; i < nj; ++i) {
+    const NsLayout& L = sets[i].L;
+    const int mt = jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n, nt = jobs[i].m < jobs[i].n ? jobs[i].n : jobs[i].m;
+    whole = whole && L.mw == mt && L.nw == nt && (jobs[i].ldx & 7) == 0;
+  }
+  char* res[DA_MAX_GROUPS];
+  const int* poison = nullptr;
+  bool updated = false;
+  int rc = ns_iterate(sets, nj, c.compute_dtype, c.coeffs, c.steps, c.faithful, s, res, &poison, whole ? &updated : nullptr);
+  if (rc) return rc;
+  if (updated && poison) {
+    // a persistent launch that updated the weights itself: NaN in all of them if it gave up
+    DaPtrUploads up{};
+    DaPoisonShape shape{};
+    shape.f32 = c.x_dtype == DA_F32;
+    int count = 0;
+    for (int i = 0; i < nj; ++i)
+      for (int j0 = 0; j0 < jobs[i].cnt; j0 += DA_MAX_PTRS) {
+        const int n = jobs[i].cnt - j0 < DA_MAX_PTRS ? jobs[i].cnt - j0 : DA_MAX_PTRS;
+        for (int j = 0; j < n; ++j) up.t[count].p[j] = jobs[i].X[j0 + j];
+        up.n[count] = n;
+        shape.numel[count] = (long long)jobs[i].m * jobs[i].n;
+        if (++count == DA_MAX_UPLOADS) {
+          rc = da_poison_multi_if(up, count, shape, poison, s);
+          if (rc) return rc;
+          count = 0;
+        }
+      }
+    return count ? da_poison_multi_if(up, count, shape, poison, s) : DA_OK;
+  }
+  for (int i = 0; i < nj && !updated; ++i) {
+    const NsJob& k = jobs[i];
+    const NsLayout& L = sets[i].L;
+    for (int j0 = 0; j0 < k.cnt; j0 += DA_MAX_PTRS) {
+      const int n = k.cnt - j0 < DA_MAX_PTRS ? k.cnt - j0 : DA_MAX_PTRS;
+      DaUnstage us{};
+      for (int j = 0; j < n; ++j) us.x.p[j] = k.X[j0 + j];
+      us.wide = res[i] + (size_t)j0 * L.x_bytes;
+      us.batch = n; us.rows = k.m; us.cols = k.n; us.ld = k.ldx; us.mw = L.mw; us.ldw = L.ldx;
+      us.x_dtype = c.x_dtype; us.w_dtype = c.compute_dtype;
+      us.decay = k.decay; us.step = k.step; us.muon = c.update;
+      us.poison = poison;
+      // algorithmic bytes: read X (update only) and the result, write X
+      DaProfScope prof(DA_PROF_UNSTAGE, (double)k.m * k.n * ((c.update ? 2 : 1) * xsz + L.esz) * n, s);
+      rc = da_unstage(us, s);
+      if (rc) return rc;
+    }
   }
   return DA_OK;
 }
 
-int ns_normalize_chunk(const NsLayout& L, const NsBuffers& W, int cb, int dtype, float eps, hipStream_t s) {
-  DaProfScope prof(DA_PROF_NORMALIZE, 2.0 * (double)L.mw * L.nw * L.esz * cb, s);  // algorithmic bytes (pad excluded)
-  // (the divisor is formed inside the launch from the partial sums: no separate finishing launch)
-  return da_normalize_from_partials(W.x0, dtype, (long long)(L.x_bytes / L.esz), cb, nullptr, W.partials, L.tiles, eps, s);
-}
+// 16-byte alignment of a matrix whose rows are whole 16-byte chunks; rows off that grid need their elements' alignment.
+inline bool misaligned(const void* p, bool chunks, size_t esz) { return ((uintptr_t)p & (chunks ? 15 : esz - 1)) != 0; }
 
 bool dtype_ok(int d) { return d == DA_BF16 || d == DA_F32; }
 
@@ -323,48 +512,29 @@ int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, l
            void* workspace, size_t workspace_bytes, void* stream) {
   if (!G || !out || !coeffs || !workspace || batch <= 0 || m <= 0 || n <= 0 || steps < 0) return DA_ERR_ARG;
   if (!dtype_ok(g_dtype) || !dtype_ok(compute_dtype)) return DA_ERR_DTYPE;
-  if ((m | n | ldg | ldo) & 7) return DA_ERR_ALIGN;
-  if ((g_stride | out_stride) & 7) return DA_ERR_ALIGN;
-  // matrices move as 16-byte chunks; only the workspace, which the library carves up itself, needs 256
-  if (((uintptr_t)G | (uintptr_t)out) & 15) return DA_ERR_ALIGN;
+  const size_t gsz = g_dtype == DA_BF16 ? 2 : 4, osz = compute_dtype == DA_BF16 ? 2 : 4;
+  if (ldg < n || ldo < n) return DA_ERR_ARG;
+  // matrices move as 16-byte chunks where their rows allow that; only the workspace, which the library carves up
+  // itself, needs 256
+  const bool g_chunks = !((n | ldg) & 7), o_chunks = !((n | ldo) & 7);
+  if ((g_chunks && (g_stride & 7)) || (o_chunks && (out_stride & 7))) return DA_ERR_ALIGN;
+  if (misaligned(G, g_chunks, gsz) || misaligned(out, o_chunks, osz)) return DA_ERR_ALIGN;
   if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const NsLayout L(m, n, compute_dtype);
   const int chunk = L.chunk(batch, workspace_bytes);
   if (chunk < 1) return DA_ERR_WORKSPACE;
-  const size_t gsz = g_dtype == DA_BF16 ? 2 : 4;
+  const NsCall call = {compute_dtype, g_dtype, compute_dtype, 0, 0.f, 0, coeffs, steps, eps, faithful};
   for (int b0 = 0; b0 < batch; b0 += chunk) {
     const int cb = batch - b0 < chunk ? batch - b0 : chunk;
-    const NsBuffers W(L, workspace, cb);
-    DaStage st{};
-    for (int i = 0; i < cb; ++i)
-      st.g.p[i] = const_cast<char*>(static_cast<const char*>(G)) + (size_t)(b0 + i) * g_stride * gsz;
-    st.wide = W.x0; st.partials = W.partials;
-    st.batch = cb; st.rows = m; st.cols = n; st.ld = ldg; st.ldw = L.ldx;
-    st.g_dtype = g_dtype; st.m_dtype = g_dtype; st.w_dtype = compute_dtype;
-    st.mu = 0.f; st.nesterov = 0; st.muon = 0;
-    int rc;
-    {
-      DaProfScope prof(DA_PROF_STAGE, (double)m * n * (gsz + L.esz) * cb, s);
-      rc = da_stage_wide(st, s);
+    const void* src[DA_MAX_PTRS];
+    void* dst[DA_MAX_PTRS];
+    for (int i = 0; i < cb; ++i) {
+      src[i] = static_cast<const char*>(G) + (size_t)(b0 + i) * g_stride * gsz;
+      dst[i] = static_cast<char*>(out) + (size_t)(b0 + i) * out_stride * osz;
     }
-    if (rc) return rc;
-    rc = ns_normalize_chunk(L, W, cb, compute_dtype, eps, s);
-    if (rc) return rc;
-    char* res = nullptr;
-    const int* poison = nullptr;
-    rc = ns_iterate(L, W, cb, compute_dtype, coeffs, steps, faithful, s, &res, &poison);
-    if (rc) return rc;
-    DaUnstage us{};
-    us.poison = poison;
-    for (int i = 0; i < cb; ++i) us.x.p[i] = static_cast<char*>(out) + (size_t)(b0 + i) * out_stride * L.esz;
-    us.wide = res; us.batch = cb; us.rows = m; us.cols = n; us.ld = ldo; us.ldw = L.ldx;
-    us.x_dtype = compute_dtype; us.w_dtype = compute_dtype;
-    us.decay = 1.f; us.step = 1.f; us.muon = 0;
-    {
-      DaProfScope prof(DA_PROF_UNSTAGE, 2.0 * (double)m * n * L.esz * cb, s);
-      rc = da_unstage(us, s);
-    }
+    const NsJob job = {src, nullptr, dst, cb, m, n, ldg, ldo, 1.f, 1.f};
+    const int rc = ns_jobs(&job, 1, call, workspace, s);
     if (rc) return rc;
   }
   return DA_OK;
@@ -500,70 +670,38 @@ size_t dion_amd_muon_workspace_bytes(int batch, int m, int n) {
   return NsLayout(m, n, DA_BF16).recommended(batch);
 }
 
+}  // extern "C"
+
+namespace {
+int muon_check(void* const* X, const void* const* G, void* const* M, int batch, int n, int x_dtype, int g_dtype) {
+  const bool chunks = (n & 7) == 0;
+  const size_t xsz = x_dtype == DA_BF16 ? 2 : 4, gsz = g_dtype == DA_BF16 ? 2 : 4;
+  for (int i = 0; i < batch; ++i) {
+    if (!X[i] || !G[i] || !M[i]) return DA_ERR_ARG;
+    if (misaligned(X[i], chunks, xsz) || misaligned(G[i], chunks, gsz) || misaligned(M[i], chunks, xsz)) return DA_ERR_ALIGN;
+  }
+  return DA_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int dion_amd_muon_step(void* const* X, const void* const* G, void* const* M, int batch, int m, int n, int x_dtype,
                        int g_dtype, float mu, int nesterov, float decay, float adjusted_lr, const float* coeffs,
                        int steps, float eps, int faithful, void* workspace, size_t workspace_bytes, void* stream) {
   if (!X || !G || !M || !coeffs || !workspace || batch <= 0 || m <= 0 || n <= 0 || steps < 0) return DA_ERR_ARG;
   if (!dtype_ok(x_dtype) || !dtype_ok(g_dtype)) return DA_ERR_DTYPE;
-  if ((m | n) & 7) return DA_ERR_ALIGN;
   if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
-  for (int i = 0; i < batch; ++i) {
-    if (!X[i] || !G[i] || !M[i]) return DA_ERR_ARG;
-    if (((uintptr_t)X[i] | (uintptr_t)G[i] | (uintptr_t)M[i]) & 15) return DA_ERR_ALIGN;
-  }
+  const int rc = muon_check(X, G, M, batch, n, x_dtype, g_dtype);
+  if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const NsLayout L(m, n, DA_BF16);
   const int chunk = L.chunk(batch, workspace_bytes);
   if (chunk < 1) return DA_ERR_WORKSPACE;
+  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful};
   for (int b0 = 0; b0 < batch; b0 += chunk) {
-    const int cb = batch - b0 < chunk ? batch - b0 : chunk;
-    const NsBuffers W(L, workspace, cb);
-    DaStage st{};
-    for (int i = 0; i < cb; ++i) {
-      st.g.p[i] = const_cast<void*>(G[b0 + i]);
-      st.mom.p[i] = M[b0 + i];
-    }
-    st.wide = W.x0; st.partials = W.partials;
-    st.batch = cb; st.rows = m; st.cols = n; st.ld = n; st.ldw = L.ldx;
-    st.g_dtype = g_dtype; st.m_dtype = x_dtype; st.w_dtype = DA_BF16;
-    st.mu = mu; st.nesterov = nesterov; st.muon = 1;
-    const double xsz = x_dtype == DA_BF16 ? 2 : 4, gsz = g_dtype == DA_BF16 ? 2 : 4;
-    int rc;
-    {
-      // algorithmic bytes: read G and M, write M and the bf16 working matrix
-      DaProfScope prof(DA_PROF_STAGE, (double)m * n * (gsz + 2 * xsz + 2) * cb, s);
-      rc = da_stage_wide(st, s);
-    }
-    if (rc) return rc;
-    rc = ns_normalize_chunk(L, W, cb, DA_BF16, eps, s);
-    if (rc) return rc;
-    char* res = nullptr;
-    const int* poison = nullptr;
-    bool updated = false;
-    NsSet one;
-    one.L = L; one.W = W; one.cb = cb;
-    rc = ns_set_update(one, X + b0, 0, cb, m, n, x_dtype, decay, adjusted_lr, s);
-    if (rc) return rc;
-    rc = ns_iterate(&one, 1, DA_BF16, coeffs, steps, faithful, s, &res, &poison, &updated);
-    if (rc) return rc;
-    if (updated) {
-      if (poison) {
-        rc = ns_poison_weights(X + b0, cb, m, n, x_dtype, poison, s);
-        if (rc) return rc;
-      }
-      continue;
-    }
-    DaUnstage us{};
-    us.poison = poison;
-    for (int i = 0; i < cb; ++i) us.x.p[i] = X[b0 + i];
-    us.wide = res; us.batch = cb; us.rows = m; us.cols = n; us.ld = n; us.ldw = L.ldx;
-    us.x_dtype = x_dtype; us.w_dtype = DA_BF16;
-    us.decay = decay; us.step = adjusted_lr; us.muon = 1;
-    {
-      // algorithmic bytes: read X and the bf16 result, write X
-      DaProfScope prof(DA_PROF_UNSTAGE, (double)m * n * (2 * xsz + 2) * cb, s);
-      rc = da_unstage(us, s);
-    }
+    const NsJob job = {G + b0, M + b0, X + b0, batch - b0 < chunk ? batch - b0 : chunk, m, n, n, n, decay, adjusted_lr};
+    const int rc = ns_jobs(&job, 1, call, workspace, s);
     if (rc) return rc;
   }
   return DA_OK;
@@ -573,27 +711,27 @@ int dion_amd_muon_pre(const void* const* G, void* const* M, void* const* U, int 
                       int m_dtype, float mu, int nesterov, void* stream) {
   if (!G || !M || !U || batch <= 0 || m <= 0 || n <= 0) return DA_ERR_ARG;
   if (!dtype_ok(g_dtype) || !dtype_ok(m_dtype)) return DA_ERR_DTYPE;
-  if (n & 7) return DA_ERR_ALIGN;
+  const bool chunks = (n & 7) == 0;
+  const size_t gsz = g_dtype == DA_BF16 ? 2 : 4, msz = m_dtype == DA_BF16 ? 2 : 4;
   for (int i = 0; i < batch; ++i) {
     if (!G[i] || !M[i] || !U[i]) return DA_ERR_ARG;
-    if (((uintptr_t)G[i] | (uintptr_t)M[i] | (uintptr_t)U[i]) & 15) return DA_ERR_ALIGN;
+    if (misaligned(G[i], chunks, gsz) || misaligned(M[i], chunks, msz) || misaligned(U[i], chunks, 2)) return DA_ERR_ALIGN;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const double gsz = g_dtype == DA_BF16 ? 2 : 4, msz = m_dtype == DA_BF16 ? 2 : 4;
-  for (int b0 = 0; b0 < batch; b0 += DA_MAX_PTRS) {
-    const int cb = batch - b0 < DA_MAX_PTRS ? batch - b0 : DA_MAX_PTRS;
+  for (int b0 = 0; b0 < batch; b0 += DA_STAGE_MATS) {
+    const int cb = batch - b0 < DA_STAGE_MATS ? batch - b0 : DA_STAGE_MATS;
     DaStage st{};
     for (int i = 0; i < cb; ++i) {
-      st.g.p[i] = const_cast<void*>(G[b0 + i]);
-      st.mom.p[i] = M[b0 + i];
-      st.wtab.p[i] = U[b0 + i];
+      st.src[i] = G[b0 + i];
+      st.mom[i] = M[b0 + i];
+      st.dst[i] = U[b0 + i];
     }
-    st.use_wtab = 1; st.wide = nullptr; st.partials = nullptr;
-    st.batch = cb; st.rows = m; st.cols = n; st.ld = n; st.ldw = n;
+    st.ngroups = 1;
+    st.g[0].rows = m; st.g[0].cols = n; st.g[0].ld = n; st.g[0].cnt = cb;
     st.g_dtype = g_dtype; st.m_dtype = m_dtype; st.w_dtype = DA_BF16;
     st.mu = mu; st.nesterov = nesterov; st.muon = 1;
     DaProfScope prof(DA_PROF_STAGE, (double)m * n * (gsz + 2 * msz + 2) * cb, s);
-    const int rc = da_stage_wide(st, s);
+    const int rc = da_stage(st, s);
     if (rc) return rc;
   }
   return DA_OK;
@@ -603,10 +741,11 @@ int dion_amd_muon_post(void* const* X, const void* const* O, int batch, int m, i
                        float decay, float adjusted_lr, void* stream) {
   if (!X || !O || batch <= 0 || m <= 0 || n <= 0) return DA_ERR_ARG;
   if (!dtype_ok(x_dtype) || !dtype_ok(o_dtype)) return DA_ERR_DTYPE;
-  if (n & 7) return DA_ERR_ALIGN;
+  const bool chunks = (n & 7) == 0;
   for (int i = 0; i < batch; ++i) {
     if (!X[i] || !O[i]) return DA_ERR_ARG;
-    if (((uintptr_t)X[i] | (uintptr_t)O[i]) & 15) return DA_ERR_ALIGN;
+    if (misaligned(X[i], chunks, x_dtype == DA_BF16 ? 2 : 4) || misaligned(O[i], chunks, o_dtype == DA_BF16 ? 2 : 4))
+      return DA_ERR_ALIGN;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const double xsz = x_dtype == DA_BF16 ? 2 : 4;
@@ -659,112 +798,20 @@ int dion_amd_muon_step_buckets(const dion_amd_muon_bucket* buckets, int nbuckets
   for (int i = 0; i < nbuckets; ++i) {
     const dion_amd_muon_bucket& k = buckets[i];
     if (!k.X || !k.G || !k.M || k.batch <= 0 || k.m <= 0 || k.n <= 0) return DA_ERR_ARG;
-    if ((k.m | k.n) & 7) return DA_ERR_ALIGN;
-    for (int j = 0; j < k.batch; ++j) {
-      if (!k.X[j] || !k.G[j] || !k.M[j]) return DA_ERR_ARG;
-      if (((uintptr_t)k.X[j] | (uintptr_t)k.G[j] | (uintptr_t)k.M[j]) & 15) return DA_ERR_ALIGN;
-    }
+    const int rc = muon_check(k.X, k.G, k.M, k.batch, k.n, x_dtype, g_dtype);
+    if (rc) return rc;
   }
   if (workspace_bytes < dion_amd_muon_buckets_workspace_bytes(buckets, nbuckets)) return DA_ERR_WORKSPACE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const double xsz = x_dtype == DA_BF16 ? 2 : 4, gsz = g_dtype == DA_BF16 ? 2 : 4;
+  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful};
   for (int r0 = 0; r0 < nbuckets; r0 += DA_MAX_GROUPS) {
     const int nr = nbuckets - r0 < DA_MAX_GROUPS ? nbuckets - r0 : DA_MAX_GROUPS;
-    // carve the workspace: every bucket of this round keeps all of its matrices resident
-    NsSet sets[DA_MAX_GROUPS];
-    char* p = static_cast<char*>(workspace);
+    NsJob jobs[DA_MAX_GROUPS];
     for (int i = 0; i < nr; ++i) {
       const dion_amd_muon_bucket& k = buckets[r0 + i];
-      const NsLayout L(k.m, k.n, DA_BF16);
-      sets[i].L = L;
-      sets[i].W = NsBuffers(L, p, k.batch);
-      sets[i].cb = k.batch;
-      p += align_up(L.per_matrix * (size_t)k.batch, 256);
+      jobs[i] = NsJob{k.G, k.M, k.X, k.batch, k.m, k.n, k.n, k.n, k.decay, k.adjusted_lr};
     }
-    // momentum update, bf16 staging in wide orientation, Frobenius partial sums; then normalise
-    for (int i = 0; i < nr; ++i) {
-      const dion_amd_muon_bucket& k = buckets[r0 + i];
-      const NsLayout& L = sets[i].L;
-      const NsBuffers& W = sets[i].W;
-      for (int j0 = 0; j0 < k.batch; j0 += DA_MAX_PTRS) {
-        const int c = k.batch - j0 < DA_MAX_PTRS ? k.batch - j0 : DA_MAX_PTRS;
-        DaStage st{};
-        for (int j = 0; j < c; ++j) {
-          st.g.p[j] = const_cast<void*>(k.G[j0 + j]);
-          st.mom.p[j] = k.M[j0 + j];
-        }
-        st.wide = W.x0 + (size_t)j0 * L.x_bytes;
-        st.partials = W.partials + (size_t)j0 * L.tiles;
-        st.batch = c; st.rows = k.m; st.cols = k.n; st.ld = k.n; st.ldw = L.ldx;
-        st.g_dtype = g_dtype; st.m_dtype = x_dtype; st.w_dtype = DA_BF16;
-        st.mu = mu; st.nesterov = nesterov; st.muon = 1;
-        DaProfScope prof(DA_PROF_STAGE, (double)k.m * k.n * (gsz + 2 * xsz + 2) * c, s);
-        const int rc = da_stage_wide(st, s);
-        if (rc) return rc;
-      }
-      const int rc = ns_normalize_chunk(L, W, k.batch, DA_BF16, eps, s);
-      if (rc) return rc;
-    }
-    char* res[DA_MAX_GROUPS];
-    const int* poison = nullptr;
-    bool updated = false;
-    // the weights' pointer tables for the last product's epilogue: as few launches as the tables need
-    DaPtrUploads up{};
-    DaPoisonShape shape{};
-    shape.f32 = x_dtype == DA_F32;
-    auto flush_uploads = [&](int count, bool poisoning) -> int {
-      if (count == 0) return DA_OK;
-      return poisoning ? da_poison_multi_if(up, count, shape, poison, s) : da_upload_ptrs_multi(up, count, s);
-    };
-    auto for_all_tables = [&](bool poisoning) -> int {
-      int count = 0;
-      for (int i = 0; i < nr; ++i) {
-        const dion_amd_muon_bucket& k = buckets[r0 + i];
-        for (int j0 = 0; j0 < k.batch; j0 += DA_MAX_PTRS) {
-          const int c = k.batch - j0 < DA_MAX_PTRS ? k.batch - j0 : DA_MAX_PTRS;
-          for (int j = 0; j < c; ++j) up.t[count].p[j] = k.X[j0 + j];
-          up.dst[count] = sets[i].W.xtab + j0;
-          up.n[count] = c;
-          shape.numel[count] = (long long)k.m * k.n;
-          if (++count == DA_MAX_UPLOADS) {
-            const int rc = flush_uploads(count, poisoning);
-            if (rc) return rc;
-            count = 0;
-          }
-        }
-      }
-      return flush_uploads(count, poisoning);
-    };
-    for (int i = 0; i < nr; ++i) {
-      const dion_amd_muon_bucket& k = buckets[r0 + i];
-      NsSet& S = sets[i];
-      S.update = 1; S.x_dtype = x_dtype; S.tall = k.m > k.n ? 1 : 0; S.x_ld = k.n; S.decay = k.decay; S.step = k.adjusted_lr;
-    }
-    int rc = for_all_tables(false);
+    const int rc = ns_jobs(jobs, nr, call, workspace, static_cast<hipStream_t>(stream));
     if (rc) return rc;
-    rc = ns_iterate(sets, nr, DA_BF16, coeffs, steps, faithful, s, res, &poison, &updated);
-    if (rc) return rc;
-    if (updated && poison) {
-      rc = for_all_tables(true);
-      if (rc) return rc;
-    }
-    for (int i = 0; i < nr && !updated; ++i) {
-      const dion_amd_muon_bucket& k = buckets[r0 + i];
-      const NsLayout& L = sets[i].L;
-      for (int j0 = 0; j0 < k.batch; j0 += DA_MAX_PTRS) {
-        const int c = k.batch - j0 < DA_MAX_PTRS ? k.batch - j0 : DA_MAX_PTRS;
-        DaUnstage us{};
-        for (int j = 0; j < c; ++j) us.x.p[j] = k.X[j0 + j];
-        us.wide = res[i] + (size_t)j0 * L.x_bytes;
-        us.batch = c; us.rows = k.m; us.cols = k.n; us.ld = k.n; us.ldw = L.ldx;
-        us.x_dtype = x_dtype; us.w_dtype = DA_BF16;
-        us.decay = k.decay; us.step = k.adjusted_lr; us.muon = 1;
-        us.poison = poison;
-        DaProfScope prof(DA_PROF_UNSTAGE, (double)k.m * k.n * (2 * xsz + 2) * c, s);
-        rc = da_unstage(us, s);
-        if (rc) return rc;
-      }
-    }
   }
   return DA_OK;
 }

@@ -8,28 +8,39 @@ struct DaPtrTable {
   void* p[DA_MAX_PTRS];
 };
 
+// Staging of up to DA_MAX_GROUPS buckets of same-shape matrices in one launch: momentum update (Muon) or plain cast,
+// rounded into working matrices of *wide* orientation (rows <= cols), zero outside the true matrix.
+struct DaStageGroup {
+  void* wide;        // [cnt][mw][ldw]; null: the result of matrix b goes to dst[b], in source orientation, without padding
+  float* partials;   // [cnt][da_stage_tiles(rows, cols, mw, nw)] sums of squares of the result (wide != null)
+  void** xtab;       // optional: receives the dst pointers of the group's matrices
+  int rows, cols;    // source matrices, row pitch ld (momentum: contiguous)
+  int ld;
+  int mw, nw, ldw;   // working matrices: rows, columns and pitch, all multiples of 8, >= min / max (rows, cols)
+  int cnt;
+};
+constexpr int DA_STAGE_MATS = 80;   // matrices per launch: their pointers travel as kernel arguments
 struct DaStage {
-  DaPtrTable g;      // source matrices (rows x cols, row pitch ld)
-  DaPtrTable mom;    // momentum buffers (contiguous rows x cols), Muon mode only
-  void* wide;        // [batch][min(rows,cols)][ldw] working matrices, max(rows,cols) columns used
-  float* partials;   // [batch][da_stage_tiles(rows, cols)]
-  int batch, rows, cols, ld;
-  int ldw;           // row pitch of the working matrices (elements, multiple of 8, >= max(rows,cols))
+  DaStageGroup g[DA_MAX_GROUPS];
+  int ngroups;
+  const void* src[DA_STAGE_MATS];   // all groups' matrices in order: gradients / sources,
+  void* mom[DA_STAGE_MATS];         // momentum buffers (muon), updated in place,
+  void* dst[DA_STAGE_MATS];         // destinations (for xtab, or of the result itself where wide is null)
   int g_dtype, m_dtype, w_dtype;
   float mu;
-  int nesterov;
-  int muon;
-  // Stand-alone momentum pass (no Newton-Schulz behind it): each result keeps the source orientation and goes
-  // to its own matrix wtab.p[b] (rows x cols, contiguous) instead of the batch `wide`; no partial sums.
-  int use_wtab;
-  DaPtrTable wtab;
+  int nesterov, muon;
+  // control memory of the launch behind this one: `nzero` ints to clear and a word that receives `preset`
+  int* zero;
+  int nzero;
+  int* status;
+  int preset;
 };
 
 struct DaUnstage {
   DaPtrTable x;      // destinations (rows x cols, row pitch ld)
-  const void* wide;
+  const void* wide;  // [batch][mw][ldw], of which the min(rows, cols) x max(rows, cols) corner is used
   int batch, rows, cols, ld;
-  int ldw;           // row pitch of the working matrices
+  int mw, ldw;
   int x_dtype, w_dtype;
   float decay, step;
   int muon;
@@ -42,31 +53,21 @@ struct DaUnstage {
   const int* poison;
 };
 
-int da_stage_tiles(int rows, int cols);
-int da_stage_wide(const DaStage& d, hipStream_t s);
-int da_norm_finish(const float* partials, int tiles, int batch, float eps, int bf16_mode, float* divisor,
-                   hipStream_t s);
-int da_normalize(void* wide, int w_dtype, long long per_matrix, int batch, const float* divisor, hipStream_t s);
-// The same with the divisor formed inside the launch from the partial sums of squares (`tiles` per matrix; what
-// da_norm_finish would have written: same order of summation, same roundings).  partials == null: read `divisor`.
-int da_normalize_from_partials(void* wide, int w_dtype, long long per_matrix, int batch, const float* divisor,
-                               const float* partials, int tiles, float eps, hipStream_t s);
+int da_stage_tiles(int rows, int cols, int mw, int nw);
+int da_stage(const DaStage& d, hipStream_t s);
+// W <- W / (||W||_F + eps), the norm from `tiles` partial sums of squares per matrix
+int da_normalize(void* wide, int w_dtype, long long per_matrix, int batch, const float* partials, int tiles, float eps,
+                 hipStream_t s);
 int da_unstage(const DaUnstage& d, hipStream_t s);
-// Up to DA_MAX_UPLOADS pointer tables in one launch: dst[k][i] = t[k].p[i] for i < n[k]; and the same tables as the
-// target of a conditional poisoning (numel[k] contiguous elements per matrix of table k).
+// Conditional poisoning of up to DA_MAX_UPLOADS pointer tables (numel[k] contiguous elements per matrix of table k).
 constexpr int DA_MAX_UPLOADS = 6;
 struct DaPtrUploads {
   DaPtrTable t[DA_MAX_UPLOADS];
-  void** dst[DA_MAX_UPLOADS];
   int n[DA_MAX_UPLOADS];
 };
 struct DaPoisonShape {
   long long numel[DA_MAX_UPLOADS];
   int f32;
 };
-int da_upload_ptrs_multi(const DaPtrUploads& u, int count, hipStream_t s);
+// If *flag != 0 when the kernel runs, every element of the matrices becomes NaN.
 int da_poison_multi_if(const DaPtrUploads& u, int count, const DaPoisonShape& sh, const int* flag, hipStream_t s);
-// dst[i] = t.p[i] for i < n <= DA_MAX_PTRS: a table of per-matrix pointers in device memory
-int da_upload_ptrs(const DaPtrTable& t, void** dst, int n, hipStream_t s);
-// If *flag != 0 when the kernel runs, every element of the n matrices (numel contiguous elements each) becomes NaN.
-int da_poison_if(const DaPtrTable& t, int n, long long numel, int dtype, const int* flag, hipStream_t s);

@@ -86,6 +86,16 @@ __device__ __forceinline__ void dma16(const char* base, unsigned off, unsigned l
                : "v"(off), "s"(u), "s"(__builtin_amdgcn_readfirstlane((int)l))
                : "memory");
 }
+// The same past the L1 (scope bit sc1): for data that another compute unit of the XCD wrote during this launch.
+__device__ __forceinline__ void dma16_l2(const char* base, unsigned off, unsigned l) {
+  const unsigned long long a = reinterpret_cast<unsigned long long>(base);
+  const unsigned long long u = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) |
+                               (unsigned)__builtin_amdgcn_readfirstlane((int)a);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1 sc1"
+               :
+               : "v"(off), "s"(u), "s"(__builtin_amdgcn_readfirstlane((int)l))
+               : "memory");
+}
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ unsigned lds_addr(const char* p) {
   return (unsigned)(uintptr_t)DA_LDS_PTR(const char, p);
@@ -139,6 +149,13 @@ __device__ __forceinline__ unsigned epi_pair(float s0, float s1, float a0, float
 
 typedef __attribute__((address_space(1))) u32x4_t global_u32x4_t;
 __device__ __forceinline__ u32x4_t ldg16(const char* p) { return *(const global_u32x4_t*)p; }
+// 16 bytes past the L1: two 8-byte loads of agent scope
+__device__ __forceinline__ u32x4_t ldg16_l2(const char* p) {
+  const unsigned long long a = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long b = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p + 8), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const u32x4_t v = {(unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)};
+  return v;
+}
 __device__ __forceinline__ void stg16(char* p, u32x4_t v) { *(global_u32x4_t*)p = v; }
 
 __device__ __forceinline__ void wave_sync_lds() {

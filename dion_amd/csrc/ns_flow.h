@@ -31,6 +31,8 @@ const int* da_ns_flow_status_word(const DaNsFlowGroup* g);
 // mode: -1 automatic (DION_AMD_NS_FLOW in the environment, else by workload), 0 never, 1 whenever the shapes
 // allow, 2 the same with an L2 write-back after every tile.  fail (test hook): launches start with the status word set.
 void da_ns_flow_set_mode(int mode);
+int da_ns_flow_mode();   // what set_mode or the environment chose, -1: nothing
+bool da_ns_flow_fail();
 void da_ns_flow_set_fail(int on);
 void da_ns_flow_set_spin_limit(long long ticks);
 // Measurement hook: while enabled, every tile of a launch records the 100 MHz counter at its start, when its

@@ -369,6 +369,13 @@ int da_ns_flow_trace_read(void* dst, int max_tiles, int* tiles) {
   return DA_OK;
 }
 void da_ns_flow_set_mode(int mode) { g_flow_mode.store(mode, std::memory_order_relaxed); }
+int da_ns_flow_mode() {
+  const int mode = g_flow_mode.load(std::memory_order_relaxed);
+  if (mode >= 0) return mode;
+  static const int env = [] { const char* e = getenv("DION_AMD_NS_FLOW"); return e ? atoi(e) : -1; }();
+  return env;
+}
+bool da_ns_flow_fail() { return g_flow_fail.load(std::memory_order_relaxed) != 0; }
 void da_ns_flow_set_fail(int on) { g_flow_fail.store(on, std::memory_order_relaxed); }
 void da_ns_flow_set_spin_limit(long long ticks) { g_flow_spin.store(ticks, std::memory_order_relaxed); }
 
@@ -376,11 +383,7 @@ size_t da_ns_flow_ctl_bytes(int cnt) { return (size_t)cnt * DA_FLOW_CTR_STRIDE *
 
 bool da_ns_flow_applicable(const DaNsFlowGroup* g, int n, int steps, int faithful) {
   if (!faithful) return false;   // (the kernel carries the rounding-faithful epilogues only)
-  int mode = g_flow_mode.load(std::memory_order_relaxed);
-  if (mode < 0) {
-    static const int env = [] { const char* e = getenv("DION_AMD_NS_FLOW"); return e ? atoi(e) : -1; }();
-    mode = env;
-  }
+  const int mode = da_ns_flow_mode();
   if (mode == 0) return false;
   if (n < 1 || n > DA_MAX_GROUPS || steps < 1 || steps > DA_FLOW_MAX_STEPS) return false;
   long long nmat = 0;
@@ -453,12 +456,7 @@ int da_ns_flow(const DaNsFlowGroup* g, int n, const float* coeffs, int steps, in
   r.preset = g_flow_fail.load(std::memory_order_relaxed) ? 1 : 0;
   for (int i = 0; i < 3 * steps; ++i) a.coeffs[i] = coeffs[i];
   a.ngroups = n; a.steps = steps; a.faithful = faithful;
-  int mode = g_flow_mode.load(std::memory_order_relaxed);
-  if (mode < 0) {
-    static const int env = [] { const char* e = getenv("DION_AMD_NS_FLOW"); return e ? atoi(e) : -1; }();
-    mode = env;
-  }
-  a.strict = mode == 2;
+  a.strict = da_ns_flow_mode() == 2;
   const long long spin = g_flow_spin.load(std::memory_order_relaxed);
   a.spin_limit = spin >= 0 ? (unsigned long long)spin : 200000000ull;   // 2 s of the 100 MHz counter
 

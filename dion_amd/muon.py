@@ -178,7 +178,6 @@ class Muon(Optimizer):
         # products are grouped launches, so small buckets share the GPU instead of queueing
         # (the reference overlaps them as async tasks, dion/muon.py:185-270).
         fused = defaultdict(list)
-        crops = []
         for (shape, dtype, gdtype, device), plist in buckets.items():
             states = [self._get_or_initialize_state(p, "muon") for p in plist]
             adjusted_lr = lr if adjust is None else _ADJUST[adjust](lr, shape)
@@ -187,14 +186,6 @@ class Muon(Optimizer):
                 continue
             _lib.require_gpu(plist[0], "Muon.step")
             X, G, M = self._matrix_views(plist, states, group["flatten"])
-            m, n = X[0].shape
-            if m % 8 or n % 8:
-                # step zero-padded copies (exact: see _lib.zero_padded) and crop the results back
-                m8, n8 = _lib.padded_dims(m, n)
-                Xw, Gw, Mw = (_lib.zero_padded(t, m8, n8) for t in (X, G, M))
-                crops.append((X, Xw))
-                crops.append((M, Mw))
-                X, G, M = list(Xw.unbind(0)), list(Gw.unbind(0)), list(Mw.unbind(0))
             fused[(dtype, gdtype, device)].append((X, G, M, float(adjusted_lr)))
 
         decay = 1 - lr * weight_decay
@@ -220,8 +211,6 @@ class Muon(Optimizer):
                 )
             _lib.check(rc, "dion_amd_muon_step_buckets")
             del keep
-        for dst, padded in crops:
-            _lib.crop_back(dst, padded)
 
     @staticmethod
     def _matrix_views(plist: List[Tensor], states: List[dict], flatten: bool):
@@ -261,25 +250,16 @@ class Muon(Optimizer):
         X = [p.view(rows, cols) for p in plist]
         G = [(p.grad if p.grad.is_contiguous() else p.grad.contiguous()).view(rows, cols) for p in plist]
         M = [m.view(rows, cols) for m in Ms]
-        crops = []
-        c8 = cols
-        if cols % 8:
-            # the stages move 16-byte row segments: step zero-padded copies and crop the results back
-            c8 = -(-cols // 8) * 8
-            Xw, Gw, Mw = (_lib.zero_padded(t, rows, c8) for t in (X, G, M))
-            crops = [(X, Xw), (M, Mw)]
-            X, G, M = list(Xw.unbind(0)), list(Gw.unbind(0)), list(Mw.unbind(0))
-        U = torch.empty((len(plist), rows, c8), dtype=torch.bfloat16, device=device)
-        Us = list(U.unbind(0))
+        Us = [torch.empty((rows, cols), dtype=torch.bfloat16, device=device) for _ in plist]
         with torch.cuda.device(device):
             rc = lib.dion_amd_muon_pre(
-                _lib.ptr_array(G), _lib.ptr_array(M), _lib.ptr_array(Us), len(plist), rows, c8,
+                _lib.ptr_array(G), _lib.ptr_array(M), _lib.ptr_array(Us), len(plist), rows, cols,
                 _lib.dtype_code(G[0].dtype), _lib.dtype_code(M[0].dtype), mu.item(), int(bool(group["nesterov"])),
                 _lib.stream_ptr(device))
         _lib.check(rc, "dion_amd_muon_pre")
         O = []
         for p, u in zip(plist, Us):
-            u = u[:, :cols].reshape(p.shape) if c8 != cols else u.view(p.shape)
+            u = u.view(p.shape)
             if group["flatten"] and u.ndim >= 3:
                 v = u.flatten(start_dim=1)
             elif u.ndim >= 4:
@@ -291,10 +271,7 @@ class Muon(Optimizer):
             # bf16 and fp32 go to the library as they are, anything else as fp32
             if o.dtype not in (torch.bfloat16, torch.float32):
                 o = o.to(dtype=torch.float32)
-            o = o.reshape(rows, cols)
-            if c8 != cols:
-                o = torch.nn.functional.pad(o, (0, c8 - cols))
-            o = o.contiguous()
+            o = o.reshape(rows, cols).contiguous()
             if o.data_ptr() % 16:   # (a contiguous view at an odd offset: the kernels move 16-byte segments)
                 o = o.clone()
             O.append(o)
@@ -304,11 +281,9 @@ class Muon(Optimizer):
         alr = adjusted_lr.item() if isinstance(adjusted_lr, Tensor) else float(torch.tensor(adjusted_lr).item())
         with torch.cuda.device(device):
             rc = lib.dion_amd_muon_post(
-                _lib.ptr_array(X), _lib.ptr_array(O), len(plist), rows, c8, _lib.dtype_code(X[0].dtype),
+                _lib.ptr_array(X), _lib.ptr_array(O), len(plist), rows, cols, _lib.dtype_code(X[0].dtype),
                 _lib.dtype_code(O[0].dtype), (1 - lr * weight_decay).item(), alr, _lib.stream_ptr(device))
         _lib.check(rc, "dion_amd_muon_post")
-        for dst, padded in crops:
-            _lib.crop_back(dst, padded)
 
     # ------------------------------------------------------------------ element-wise groups
     def _lion_group_step(self, group: dict):

@@ -377,7 +377,7 @@ int dion_amd_profile_read(int kind, long long* launches, double* total_ms, doubl
  *   "edge_loop"     bf16 products with a ragged dimension on a k-strided operand (Dion's rank-r products at r = 192):
  *                   1 the direct-to-LDS K loop with edge tiles, 0 the bounds-checked K loop, -1 the default (1 unless
  *                   DION_AMD_NO_EDGE_LOOP is set in the environment).  Both give the same bits.
- *   "ns_flow_fail"  test hook: 1 makes every persistent launch start with its status word set, as if a wait had
+ *   "ns_flow_fail"  test hook: 1 makes every persistent launch (and that for small matrices) start with its status word set, as if a wait had
  *                   run into its limit; the results of such a launch are NaN.
  * The value applies to calls that start after this one returns, on every thread.  Unknown name:
  * DION_AMD_ERR_ARG. */
