@@ -6,6 +6,7 @@ import ctypes
 import os
 
 import torch
+from torch.optim import Optimizer, optimizer
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # DION_AMD_LIB names another build of the same library (kernel experiments); default: in-tree
@@ -108,6 +109,33 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host module (`csrc/host.cpp`), bound to the loaded library."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as module
+        except ImportError as exc:
+            raise DionAmdError(f"dion_amd._host is not built or does not load ({exc}). Run `python -m dion_amd.build`.") from exc
+        module.bind(DionAmdError, check, *(_c.cast(getattr(lib, "dion_amd_" + name), _vp).value for name in
+                                           ("muon_buckets_workspace_bytes", "muon_step_buckets", "lion_step", "adamw_step")))
+        _host = module
+    return _host
+
+
+def run_step(opt, step, closure):
+    """`step(opt, closure)` with the registered step hooks.  `Optimizer` wraps every `step` in a profiler range that costs
+    14 us; here that wrapper runs only while a profiler records or hooks are registered."""
+    if (torch.autograd._profiler_enabled() or opt._optimizer_step_pre_hooks or opt._optimizer_step_post_hooks
+            or optimizer._global_optimizer_pre_hooks or optimizer._global_optimizer_post_hooks):
+        return Optimizer.profile_hook_step(step)(opt, closure)
+    return step(opt, closure)
 
 
 def exported_symbols():

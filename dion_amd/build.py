@@ -1,10 +1,12 @@
-"""Builds the gfx950 shared library `dion_amd/libdion_amd.so` from `dion_amd/csrc/*.hip`.
+"""Builds the gfx950 shared library `dion_amd/libdion_amd.so` from `dion_amd/csrc/*.hip`, and the host module
+`dion_amd/_host.so` from `dion_amd/csrc/host.cpp` (a CPython module on PyTorch's C++ interface).
 
 Run as `python -m dion_amd.build`.  hipcc cross-compiles without a GPU present.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,6 +18,7 @@ LIB = os.environ.get("DION_AMD_BUILD_LIB") or os.path.join(HERE, "libdion_amd.so
 if os.environ.get("DION_AMD_BUILD_LIB"):
     OBJ = LIB + ".obj"
 
+HOST_LIB = os.path.join(HERE, "_host.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950",
@@ -55,8 +58,24 @@ def _compile(src):
     return src, obj, res
 
 
+def build_host():
+    """g++ only: no device code in it."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include",
+           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host.cpp"), "-o", HOST_LIB,
+           f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip", f"-Wl,-rpath,{root}/lib"]
+    return subprocess.run(cmd, capture_output=True, text=True)
+
+
 def build(verbose=True, jobs=None):
     os.makedirs(OBJ, exist_ok=True)
+    host = None
+    if not os.environ.get("DION_AMD_BUILD_LIB"):   # (measurement builds write another library, nothing else)
+        host = ThreadPoolExecutor(max_workers=1).submit(build_host)
     srcs = sources()
     jobs = jobs or min(len(srcs), 8)
     objs = []
@@ -72,6 +91,8 @@ def build(verbose=True, jobs=None):
     res = subprocess.run(link, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
+    if host is not None and host.result().returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{host.result().stderr}")
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources")
     return LIB

@@ -25,7 +25,7 @@ from torch import Tensor
 from torch.optim.optimizer import Optimizer, ParamsT
 
 from . import _lib
-from .elementwise_opts import adamw_update_foreach, lion_update_foreach
+from .elementwise_opts import element_group_step
 
 
 @dataclass
@@ -141,8 +141,13 @@ class Dion(Optimizer):
         self._pool = None   # worker threads that enqueue the buckets of a wave side by side
         self._rng = None    # generator of the random sketches (DionReference with qr_method "rcqr")
 
-    @torch.no_grad()
     def step(self, closure=None):
+        return _lib.run_step(self, Dion._step, closure)
+
+    step.hooked = True   # (the hooks and the profiler range of `Optimizer` are run_step's)
+
+    @torch.no_grad()
+    def _step(self, closure=None):
         loss = None
         if closure is not None:
             with torch.enable_grad():
@@ -380,28 +385,14 @@ class Dion(Optimizer):
                 main.wait_stream(stream)
 
     # ------------------------------------------------------------------ element-wise groups
+    def _new_state(self, param: Tensor, group: dict):
+        self._get_or_initialize_state(param, group)
+
     def _lion_group_step(self, group: dict):
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
-        states = [self._get_or_initialize_state(p, group) for p in params]
-        lion_update_foreach(
-            params, [p.grad for p in params], [s["momentum"] for s in states],
-            lr=torch.tensor(group["lr"]), beta1=torch.tensor(group["beta1"]), beta2=torch.tensor(group["beta2"]),
-            weight_decay=torch.tensor(group["weight_decay"]),
-        )
+        element_group_step(self, group, False)
 
     def _adamw_group_step(self, group: dict):
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
-        states = [self._get_or_initialize_state(p, group) for p in params]
-        adamw_update_foreach(
-            params, [p.grad for p in params], [s["momentum"] for s in states], [s["variance"] for s in states],
-            lr=torch.tensor(group["lr"]), beta1=torch.tensor(group["beta1"]), beta2=torch.tensor(group["beta2"]),
-            weight_decay=torch.tensor(group["weight_decay"]), step=torch.tensor(group["step"]),
-            epsilon=torch.tensor(group["epsilon"]),
-        )
+        element_group_step(self, group, True)
 
 
 def _sketch(p_shape, dtype, device, oversample, generator=None) -> Tensor:

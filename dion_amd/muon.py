@@ -6,23 +6,22 @@ arguments and defaults, same param-group keys, same `self.state` layout
 only: `distributed_mesh` must be None.
 
 Per `step()` the matrices of every "muon" group are bucketed by (shape, dtype) -- the
-grouping rule of `create_param_batches` (reference dion/opt_utils.py:48-65) -- and each
-bucket is handed, as arrays of device pointers, to `dion_amd_muon_step`, which runs the
-fused momentum pass, the batched Newton-Schulz GEMMs and the fused weight update on the
-current stream.
+grouping rule of `create_param_batches` (reference dion/opt_utils.py:48-65) -- by the native host
+module (`csrc/host.cpp`) and handed, as arrays of device pointers, to `dion_amd_muon_step_buckets`,
+which runs the fused momentum pass, the batched Newton-Schulz GEMMs and the fused weight update on
+the current stream.
 """
+import ctypes
 import math
 from collections import defaultdict
-from typing import Callable, List, Optional, Tuple
-
-import ctypes
+from typing import Callable, Optional, Tuple
 
 import torch
 from torch import Tensor
 from torch.optim.optimizer import Optimizer, ParamsT
 
 from . import _lib
-from .elementwise_opts import adamw_update_foreach, lion_update_foreach
+from .elementwise_opts import element_group_step
 from .newton_schulz import NS_SCHEDULE_COEFFS, flat_coeffs, zeropower_via_newtonschulz5
 
 
@@ -49,6 +48,7 @@ _ADJUST = {
     "rms_norm": adjust_lr_rms_norm,
     "keller_muon": adjust_lr_keller_muon,
 }
+_ADJUST_CODE = {None: 0, "spectral_norm": 1, "rms_norm": 2, "keller_muon": 3}   # of _host.muon_group
 
 
 class Muon(Optimizer):
@@ -117,8 +117,12 @@ class Muon(Optimizer):
         self._workspace = _lib.Workspace()
         self._coeffs = flat_coeffs(NS_SCHEDULE_COEFFS)
 
-    @torch.no_grad()
     def step(self, closure=None):
+        return _lib.run_step(self, Muon._step, closure)
+
+    step.hooked = True   # (the hooks and the profiler range of `Optimizer` are run_step's)
+
+    def _step(self, closure=None):
         loss = None
         if closure is not None:
             with torch.enable_grad():
@@ -154,83 +158,48 @@ class Muon(Optimizer):
                 state["variance"] = torch.zeros_like(param)
         return state
 
+    def _new_state(self, param: Tensor, group: dict):
+        with torch.no_grad():
+            self._get_or_initialize_state(param, group["algorithm"])
+
     # ------------------------------------------------------------------ muon
     def _muon_group_step(self, group: dict):
         assert all(p.ndim >= 2 for p in group["params"]), "Muon optimizer only supports matrix parameters."
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
         adjust = group["adjust_lr"]
-        if adjust is not None and adjust not in _ADJUST:
+        if adjust not in _ADJUST_CODE:
             raise ValueError(f"Unknown adjust_lr value: {adjust}")
+        if not self._fused:
+            with torch.no_grad():
+                self._muon_group_unfused(group)
+            return
+        # Buckets of one (dtype, grad dtype, device) go to the library together: their Newton-Schulz
+        # products are grouped launches, so small buckets share the GPU instead of queueing
+        # (the reference overlaps them as async tasks, dion/muon.py:185-270).
+        args = (group["params"], self.state, float(group["lr"]), float(group["mu"]), float(group["weight_decay"]),
+                float(group["epsilon"]), group["nesterov"], _ADJUST_CODE[adjust], group["flatten"],
+                ctypes.addressof(self._coeffs), len(NS_SCHEDULE_COEFFS), self._workspace)
+        host = _lib.host()
+        missing = host.muon_group(*args)
+        if missing is not None:
+            for p in missing:
+                self._new_state(p, group)
+            host.muon_group(*args)
 
+    def _muon_group_unfused(self, group: dict):
         # hyper-parameters as 0-dim fp32 tensors, evaluated like reference dion/muon.py:205-208
         lr = torch.tensor(group["lr"])
         mu = torch.tensor(group["mu"])
         weight_decay = torch.tensor(group["weight_decay"])
         epsilon = torch.tensor(group["epsilon"])
-
+        adjust = group["adjust_lr"]
         buckets = defaultdict(list)
-        for p in params:
-            buckets[(p.shape, p.dtype, p.grad.dtype, p.device)].append(p)
-
-        # Buckets of one (dtype, grad dtype, device) go to the library together: their Newton-Schulz
-        # products are grouped launches, so small buckets share the GPU instead of queueing
-        # (the reference overlaps them as async tasks, dion/muon.py:185-270).
-        fused = defaultdict(list)
-        for (shape, dtype, gdtype, device), plist in buckets.items():
+        for p in group["params"]:
+            if p.grad is not None:
+                buckets[(p.shape, p.dtype, p.grad.dtype, p.device)].append(p)
+        for (shape, *_), plist in buckets.items():
             states = [self._get_or_initialize_state(p, "muon") for p in plist]
             adjusted_lr = lr if adjust is None else _ADJUST[adjust](lr, shape)
-            if not self._fused:
-                self._muon_bucket_unfused(plist, states, lr, adjusted_lr, mu, weight_decay, epsilon, group)
-                continue
-            _lib.require_gpu(plist[0], "Muon.step")
-            X, G, M = self._matrix_views(plist, states, group["flatten"])
-            fused[(dtype, gdtype, device)].append((X, G, M, float(adjusted_lr)))
-
-        decay = 1 - lr * weight_decay
-        for (dtype, gdtype, device), items in fused.items():
-            lib = _lib.load()
-            arr = (_lib.MuonBucket * len(items))()
-            keep = []  # pointer arrays (and contiguous gradient copies) must outlive the call
-            for b, (X, G, M, alr) in zip(arr, items):
-                px, pg, pm = _lib.ptr_array(X), _lib.ptr_array(G), _lib.ptr_array(M)
-                keep.append((px, pg, pm, G))
-                b.X, b.G, b.M = (ctypes.cast(a, ctypes.POINTER(ctypes.c_void_p)) for a in (px, pg, pm))
-                b.batch = len(X)
-                b.m, b.n = X[0].shape
-                b.decay = decay.item()
-                b.adjusted_lr = alr
-            ws = self._workspace.get(lib.dion_amd_muon_buckets_workspace_bytes(arr, len(items)), device)
-            with torch.cuda.device(device):
-                rc = lib.dion_amd_muon_step_buckets(
-                    arr, len(items), _lib.dtype_code(dtype), _lib.dtype_code(gdtype),
-                    mu.item(), int(bool(group["nesterov"])),
-                    self._coeffs, len(NS_SCHEDULE_COEFFS), epsilon.item(), 1,
-                    ws.data_ptr(), ws.numel(), _lib.stream_ptr(device),
-                )
-            _lib.check(rc, "dion_amd_muon_step_buckets")
-            del keep
-
-    @staticmethod
-    def _matrix_views(plist: List[Tensor], states: List[dict], flatten: bool):
-        """Split every parameter into the 2-D matrices Newton-Schulz sees (reference dion/muon.py:585-591):
-        `flatten` folds trailing dims of a >=3-D tensor into columns, otherwise leading dims are a batch."""
-        X, G, M = [], [], []
-        for p, st in zip(plist, states):
-            mom = st["momentum"]
-            if not p.is_contiguous() or not mom.is_contiguous():
-                raise _lib.DionAmdError("Muon.step: parameters and momentum buffers must be contiguous")
-            g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
-            if p.ndim == 2:
-                X.append(p); G.append(g); M.append(mom)
-            elif flatten:
-                X.append(p.view(p.size(0), -1)); G.append(g.view(p.size(0), -1)); M.append(mom.view(p.size(0), -1))
-            else:
-                r, c = p.shape[-2:]
-                X.extend(p.view(-1, r, c).unbind(0)); G.extend(g.view(-1, r, c).unbind(0))
-                M.extend(mom.view(-1, r, c).unbind(0))
-        return X, G, M
+            self._muon_bucket_unfused(plist, states, lr, adjusted_lr, mu, weight_decay, epsilon, group)
 
     def _muon_bucket_unfused(self, plist, states, lr, adjusted_lr, mu, weight_decay, epsilon, group):
         """Custom `newton_schulz_func` (the reference's plug-in hook, dion/muon.py:48-49, 122-131): the momentum pass
@@ -287,24 +256,7 @@ class Muon(Optimizer):
 
     # ------------------------------------------------------------------ element-wise groups
     def _lion_group_step(self, group: dict):
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
-        states = [self._get_or_initialize_state(p, "lion") for p in params]
-        lion_update_foreach(
-            params, [p.grad for p in params], [s["momentum"] for s in states],
-            lr=torch.tensor(group["lr"]), beta1=torch.tensor(group["beta1"]), beta2=torch.tensor(group["beta2"]),
-            weight_decay=torch.tensor(group["weight_decay"]),
-        )
+        element_group_step(self, group, False)
 
     def _adamw_group_step(self, group: dict):
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
-        states = [self._get_or_initialize_state(p, "adamw") for p in params]
-        adamw_update_foreach(
-            params, [p.grad for p in params], [s["momentum"] for s in states], [s["variance"] for s in states],
-            lr=torch.tensor(group["lr"]), beta1=torch.tensor(group["beta1"]), beta2=torch.tensor(group["beta2"]),
-            weight_decay=torch.tensor(group["weight_decay"]), step=torch.tensor(group["step"]),
-            epsilon=torch.tensor(group["epsilon"]),
-        )
+        element_group_step(self, group, True)
