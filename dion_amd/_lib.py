@@ -38,7 +38,14 @@ class MuonBucket(ctypes.Structure):
                 ("decay", _f), ("adjusted_lr", _f)]
 
 
+class DionBucket(ctypes.Structure):
+    """`dion_amd_dion_bucket` of include/dion_amd.h."""
+    _fields_ = [("X", _vpp), ("G", _vpp), ("M", _vpp), ("Q", _vpp), ("batch", _i), ("m", _i), ("n", _i), ("r", _i),
+                ("scaled_lr", _f), ("info", _vp)]
+
+
 _bkp = _c.POINTER(MuonBucket)
+_dbp = _c.POINTER(DionBucket)
 
 _SIGNATURES = {
     "dion_amd_version": (_c.c_char_p, []),
@@ -60,6 +67,8 @@ _SIGNATURES = {
                                 _vp, _vp, _sz, _vp]),
     "dion_amd_dion_step_qr": (_i, [_vpp, _vpp, _vpp, _vpp, _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _f, _f, _i, _i, _i,
                                    _vp, _vp, _sz, _vp]),
+    "dion_amd_dion_buckets_workspace_bytes": (_sz, [_dbp, _i, _i, _i, _i, _i]),
+    "dion_amd_dion_step_buckets": (_i, [_dbp, _i, _i, _i, _i, _i, _f, _f, _f, _vp, _sz, _vp]),
     "dion_amd_set_option": (_i, [_c.c_char_p, _i]),
     "dion_amd_orthonormalize_sketch_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "dion_amd_orthonormalize_sketch": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp]),
@@ -124,7 +133,8 @@ def host():
         except ImportError as exc:
             raise DionAmdError(f"dion_amd._host is not built or does not load ({exc}). Run `python -m dion_amd.build`.") from exc
         module.bind(DionAmdError, check, *(_c.cast(getattr(lib, "dion_amd_" + name), _vp).value for name in
-                                           ("muon_buckets_workspace_bytes", "muon_step_buckets", "lion_step", "adamw_step")))
+                                           ("muon_buckets_workspace_bytes", "muon_step_buckets", "lion_step", "adamw_step",
+                                            "dion_buckets_workspace_bytes", "dion_step_buckets")))
         _host = module
     return _host
 

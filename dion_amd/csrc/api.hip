@@ -10,6 +10,7 @@
 #include "dion.h"
 #include "ns_flow.h"
 #include "ns_small.h"
+#include "dion_small.h"
 
 namespace {
 
@@ -329,7 +330,7 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStre
     st.mu = c.mu; st.nesterov = c.nesterov; st.muon = c.update;
     st.zero = nullptr; st.nzero = 0; st.status = nullptr; st.preset = 0;
     if (small && i == 0 && j0 == 0) {
-      st.zero = ctl; st.nzero = total * DA_SMALL_CTR_STRIDE + 8 * DA_SMALL_LINE;
+      st.zero = ctl; st.nzero = total * DA_SMALL_CTR_STRIDE + DA_SMALL_TAIL - 32;
       st.status = ctl + st.nzero; st.preset = da_ns_flow_fail() ? 1 : 0;
     }
     int mats = 0;
@@ -470,6 +471,9 @@ bool fused_bq_enabled() {
   static const bool env_off = getenv("DION_AMD_NO_FUSED_BQ") != nullptr;
   return !env_off;
 }
+
+// Small buckets in one launch (dion_small.hip): -1 by the amount of work, 0 never, 1 whenever possible.
+std::atomic<int> g_opt_dion_small{-1};
 
 // Number of slices (1, 2 or 4) of the inner dimension `mp` for the product R = B^T P (np x r per matrix, `cb`
 // matrices), by the bf16 launcher's own estimate: workgroup rounds x 64-deep stages per tile, a 256 x 256 tile
@@ -648,6 +652,10 @@ int dion_amd_set_option(const char* name, int value) {
   }
   if (strcmp(name, "edge_loop") == 0) {
     da_gemm_bf16_set_edge_loop(value);
+    return DA_OK;
+  }
+  if (strcmp(name, "dion_small") == 0) {
+    g_opt_dion_small.store(value < 0 ? -1 : (value != 0), std::memory_order_relaxed);
     return DA_OK;
   }
   if (strcmp(name, "ns_flow_fail") == 0) {
@@ -1168,3 +1176,46 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
 }
 
 }  // namespace
+
+namespace {
+// fills `g` from the caller's buckets; false: not for the one-launch kernel
+bool dion_small_groups(const dion_amd_dion_bucket* buckets, int n, DaDionSmallGroup* g) {
+  if (!buckets || n < 1 || n > DA_DS_GROUPS) return false;
+  for (int i = 0; i < n; ++i) {
+    const dion_amd_dion_bucket& k = buckets[i];
+    if (!k.X || !k.G || !k.M || !k.Q || k.batch <= 0 || k.m <= 0 || k.n <= 0 || k.r <= 0 || k.r > k.m || k.r > k.n) return false;
+    for (int j = 0; j < k.batch; ++j)
+      if (!k.X[j] || !k.G[j] || !k.M[j] || !k.Q[j]) return false;
+    g[i] = DaDionSmallGroup{k.X, k.G, k.M, k.Q, k.batch, k.m, k.n, k.r, k.scaled_lr, k.info};
+  }
+  return true;
+}
+}  // namespace
+
+extern "C" size_t dion_amd_dion_buckets_workspace_bytes(const dion_amd_dion_bucket* buckets, int nbuckets, int x_dtype,
+                                                        int g_dtype, int m_dtype, int q_dtype) {
+  if (!dtype_ok(x_dtype) || !dtype_ok(g_dtype) || !dtype_ok(m_dtype) || !dtype_ok(q_dtype)) return 0;
+  const int opt = g_opt_dion_small.load(std::memory_order_relaxed);
+  DaDionSmallGroup g[DA_DS_GROUPS];
+  if (opt == 0 || !dion_small_groups(buckets, nbuckets, g)) return 0;
+  const DaDionSmallCall c = {x_dtype, g_dtype, m_dtype, q_dtype, 0.f, 0.f, 0.f, 0};
+  return da_dion_small_bytes(g, nbuckets, c, opt == 1);
+}
+
+extern "C" int dion_amd_dion_step_buckets(const dion_amd_dion_bucket* buckets, int nbuckets, int x_dtype, int g_dtype,
+                                          int m_dtype, int q_dtype, float ef_alpha, float decay, float eps, void* workspace,
+                                          size_t workspace_bytes, void* stream) {
+  if (!workspace) return DA_ERR_ARG;
+  if (!dtype_ok(x_dtype) || !dtype_ok(g_dtype) || !dtype_ok(m_dtype) || !dtype_ok(q_dtype)) return DA_ERR_DTYPE;
+  DaDionSmallGroup g[DA_DS_GROUPS];
+  if (!dion_small_groups(buckets, nbuckets, g)) return DA_ERR_ARG;
+  if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
+  const DaDionSmallCall c = {x_dtype, g_dtype, m_dtype, q_dtype, ef_alpha, decay, eps, da_ns_flow_fail() ? 1 : 0};
+  const size_t need = da_dion_small_bytes(g, nbuckets, c, true);
+  if (need == 0) return DA_ERR_LIMIT;
+  if (workspace_bytes < need) return DA_ERR_WORKSPACE;
+  double flops = 0.0;
+  for (int i = 0; i < nbuckets; ++i) flops += 8.0 * g[i].cnt * g[i].m * (double)g[i].n * g[i].r;
+  DaProfScope prof(DA_PROF_DION_EFUPD, flops, static_cast<hipStream_t>(stream));
+  return da_dion_small(g, nbuckets, c, workspace, static_cast<hipStream_t>(stream));
+}

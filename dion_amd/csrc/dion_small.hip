@@ -1,0 +1,1414 @@
+// The Dion step (reference dion/dion.py:742-875) of a set of small matrices in ONE launch:
+//
+//   B = M + G;  P = B' Q;  P <- orth(P);  R = B'^T P;  Q <- R / (||R||_col + eps);
+//   M <- B - (1 - mu) P R^T;  X <- decay X - lr P Q^T              (B' = B, or B^T when m < n; mp x np, mp >= np)
+//
+// What bounds it: as a sequence of launches a bucket takes 40 to 60 of them (a third of which only find out that the fp64
+// pass of the orthonormaliser is not needed), each a few microseconds of work: a model of 24 matrices of 256 x 256 and
+// 256 x 1024 spent 0.6-0.8 ms, most of it on the host.  Now 0.26 ms, and the host is free after 45 us: four fifths of it is the
+// chain of phases (25 us per diagonal block, 10-15 us per product), not throughput.  Here the step is a list of phases per matrix, cut into tiles;
+// workgroups take tiles from eight queues, one per XCD (flow_queue.h), and a counter per matrix and phase says when the
+// next phase may start.  A matrix stays with one XCD, so its phases meet in one L2.
+//
+// Phases (kinds):  ADD   B = M + G in place, and whether any element is not zero; Q as a padded working matrix
+//                  BQ    P = B' Q                                      64 x 64 tiles
+//                  GRAM  P^T P in fp64, lower 32 x 32 tiles, K slices as slabs of their own
+//                  DIAG0 LOW0 DIAG1 LOW1 ..   P^T P = L L^T and T = L^-1 in blocks of 64, left-looking: DIAGj adds the slabs
+//                        (in order) and the earlier columns' products to block (j, j), factors it and inverts the factor;
+//                        LOWj does the rest of block column j of L and of block row j of T, a task per block
+//                  PT    P T^T in fp64
+//                  FIX   only does anything for a matrix whose pivot range says that cond(P) may leave a visible defect, or
+//                        with a failed pivot: the closed-form second pass of da_orthonormalize in fp64 (defect measured,
+//                        noise columns dropped, P <- P (I - up(P^T P - I)))
+//                  BTP   R = B'^T P                                    64 x 64 (bf16) or 32 x 32 (fp32) tiles
+//                  CNORM column norms, Q_new, Q state                  64 x 64 tiles
+//                  UPD   error feedback and weight update, both products of a 64 x 64 tile of M and X
+// The orthonormaliser is the fp64 CholeskyQR of dion.hip for every matrix: at these sizes the fp64 products cost less than
+// the launches of the two-precision road.  P, R and the products with B run on the matrix cores in the momentum's dtype with
+// the instructions and the order of k of the batched kernels (v_mfma_f32_16x16x32_bf16, in the updates v_mfma_f32_32x32x16_bf16; v_mfma_f32_32x32x2_f32).
+//
+// Coherence.  Every buffer of the workspace is written once and read only after its phase is complete, and the lines of
+// M and X belong to one matrix (128-byte aligned): plain loads cannot meet a stale L1 line.  The exception is M itself,
+// which ADD rewrites: its loads go past the L1 (scope bit sc1), so that no old line stays behind.
+//
+// Shapes: any m, n (rows that are no multiple of 16 bytes move with unaligned accesses), rank up to 256; the working
+// matrices are padded to whole tiles and the tiles' loads fill with zeros.
+#include "dion_small.h"
+#include "flow_queue.h"
+#include "gemm_f64.h"
+#include "mfma_tile.h"
+
+#pragma clang fp contract(off)
+
+namespace {
+
+constexpr int MAX_RT = DA_DS_MAX_RANK / 64;
+enum Kind { ADD, BQ, GRAM, DIAG, LOW, PT = GRAM + 1 + 2 * MAX_RT, FIX, BTP, CNORM, UPD, KINDS };   // DIAGj = DIAG + 2 j, LOWj
+constexpr int CTR_STRIDE = 32;     // ints per matrix: a counter per kind, then the words below
+constexpr int W_NONZERO = 18, W_SICK = 19, W_BAD = 20, W_GRAM2 = 21, W_RANGE = 24;   // (W_RANGE: two doubles)
+static_assert(KINDS <= W_NONZERO, "a counter per kind");
+constexpr int ADD_ELEMS = 8192;
+constexpr int KD = 32;             // depth of an fp32 / fp64 stage
+constexpr int LP = 65;             // pitch of the factorisation's 64 x 64 tile
+constexpr double PIVOT_RATIO = 1e-7;   // as POLISH_PIVOT_RATIO in dion.hip
+constexpr int STAGES64 = 2 * 2 * KD * 66 * 8;   // two stages of two fp64 operands of 64 rows: the largest user of the LDS
+constexpr int SMEM = STAGES64 + 4 * DA_DS_MAX_RANK;
+
+struct GroupDev {
+  void *const *X, *const *G, *const *M, *const *Q;   // device tables
+  char *P, *P2, *R, *Qn, *Qw;         // momentum dtype: [cnt][mpT * 64][rp], [cnt][npT * 64][rp]
+  double* norm;                  // [cnt][nT][rp]: the column norms' shares of BTP's row tiles
+  double *P64, *slab, *L, *T, *A2, *defect;
+  int* words;                    // [cnt][CTR_STRIDE]
+  int* info;
+  int cnt, first;
+  int m, n, r, rp, mp, np, mpT, npT, rT, transposed;
+  int nT;
+  int slices, kslice;            // of the Gram products
+  float scaled_lr;
+};
+
+struct Args {
+  GroupDev g[DA_DS_GROUPS];
+  unsigned* tickets;
+  int* status;
+  unsigned long long spin_limit;
+  int ngroups;
+  int total[DA_QUEUES];          // tasks of every queue
+  int x_f32, g_f32, q_f32;
+  float ef_alpha, decay, eps;
+};
+
+typedef double double2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_un_t __attribute__((ext_vector_type(4), aligned(2)));   // an unaligned 16-byte access
+
+__host__ __device__ inline int tasks_of(const GroupDev& G, int kind, bool bf) {
+  const int t32 = (G.r + 31) >> 5;
+  switch (kind) {
+    case ADD: return (int)(((long long)G.m * G.n + ADD_ELEMS - 1) / ADD_ELEMS) + (G.npT * 64 * G.rp + ADD_ELEMS - 1) / ADD_ELEMS;
+    case BQ: case PT: return G.mpT * G.rT;
+    case GRAM: return t32 * (t32 + 1) / 2 * G.slices;
+    case FIX: return t32 * (t32 + 1) / 2 + G.mpT * G.rT;
+    case BTP: return bf ? G.npT * G.rT : ((G.np + 31) >> 5) * t32;
+    case CNORM: return G.npT * G.rT;
+    case UPD: return G.mpT * G.npT;
+    default: {   // block column j: the diagonal block; the blocks below it and the blocks of row j of the inverse
+      const int j = (kind - DIAG) >> 1;
+      return j >= G.rT ? 0 : ((kind - DIAG) & 1) ? G.rT - 1 : 1;
+    }
+  }
+}
+
+// ---- operands ----------------------------------------------------------------------------------------------------------
+
+// Element (row, k): p[row * ld + k], or p[k * ld + row] when `ks`.  EDGE: a caller's matrix of `rows` x `kmax`, of which
+// anything beyond reads as zero; `last` = its elements - 8.  Otherwise a working matrix, padded to whole tiles.
+template <typename E, bool EDGE> struct Opnd {
+  const E* p;
+  int ld, ks;
+  int rows, kmax;
+  long long last;
+};
+template <typename E> __device__ __forceinline__ Opnd<E, false> work(const void* p, int ld, int ks) {
+  return Opnd<E, false>{static_cast<const E*>(p), ld, ks, 0, 0, 0};
+}
+
+// Eight consecutive elements as they came from memory: converted only when they go to LDS, so that the loads of the next
+// stages stay in flight.
+template <typename E> struct Raw { u32x4_t q[sizeof(E) / 2]; };
+template <typename E> __device__ __forceinline__ Raw<E> load_raw(const E* p) {
+  Raw<E> r;
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(E) / 2); ++i) {
+    const u32x4_un_t x = *reinterpret_cast<const u32x4_un_t*>(reinterpret_cast<const char*>(p) + 16 * i);
+    r.q[i] = x;
+  }
+  return r;
+}
+template <typename T> __device__ __forceinline__ void unpack(const Raw<bf16_t>& r, T (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const unsigned w = r.q[0][i];
+    v[2 * i] = (T)lo_f(w);
+    v[2 * i + 1] = (T)hi_f(w);
+  }
+}
+template <typename T> __device__ __forceinline__ void unpack(const Raw<float>& r, T (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const unsigned w = r.q[i >> 2][i & 3];
+    v[i] = (T)__builtin_bit_cast(float, w);
+  }
+}
+__device__ __forceinline__ void unpack(const Raw<double>& r, double (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const unsigned lo = r.q[i >> 1][2 * (i & 1)], hi = r.q[i >> 1][2 * (i & 1) + 1];
+    v[i] = __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  }
+}
+__device__ __forceinline__ float to_f(bf16_t x) { return bf2f(x); }
+__device__ __forceinline__ float to_f(float x) { return x; }
+
+// Eight elements from element offset `e`, of which n exist; the rest reads as zero.
+template <typename E> __device__ __forceinline__ void load8(const E* p, long long e, int n, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = 0.f;
+  if (n >= 8) {
+    unpack(load_raw(p + e), v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < n) v[i] = to_f(p[e + i]);
+  }
+}
+
+// Chunk c (eight elements) of a TB x depth-D tile: its (row, k) in the tile
+template <int TB, int D>
+__device__ __forceinline__ void chunk_at(int ks, int c, int& row, int& k) {
+  row = ks ? (c % (TB / 8)) * 8 : c / (D / 8);
+  k = ks ? c / (TB / 8) : (c % (D / 8)) * 8;
+}
+template <int TB, int D, typename E, bool EDGE>
+__device__ __forceinline__ Raw<E> fetch_chunk(const Opnd<E, EDGE>& o, int c, int row0, int k0) {
+  int row, k;
+  chunk_at<TB, D>(o.ks, c, row, k);
+  row += row0;
+  k += k0;
+  long long e = o.ks ? (long long)k * o.ld + row : (long long)row * o.ld + k;
+  if (EDGE) e = e < o.last ? e : o.last;   // (inside the matrix whatever the chunk)
+  return load_raw(o.p + e);
+}
+// what of a fetched chunk lies inside a caller's matrix; the rest becomes zero
+template <int TB, int D, typename E>
+__device__ __forceinline__ void mask_chunk(const Opnd<E, true>& o, Raw<E>& r, int c, int row0, int k0) {
+  int row, k;
+  chunk_at<TB, D>(o.ks, c, row, k);
+  row += row0;
+  k += k0;
+  const int n = o.ks ? (k < o.kmax ? o.rows - row : 0) : (row < o.rows ? o.kmax - k : 0);
+  if (n >= 8) return;
+  const long long e = o.ks ? (long long)k * o.ld + row : (long long)row * o.ld + k;
+  if (n > 0 && e > o.last) {   // the matrix's last elements: the load was moved back
+    constexpr int W = 4 / sizeof(E);   // elements per word
+#pragma unroll
+    for (int i = 0; i < 8 / W; ++i) {
+      unsigned w = 0;
+      if (i * W < n) w = sizeof(E) == 4 ? reinterpret_cast<const unsigned*>(o.p + e)[i] : (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i];
+      if (sizeof(E) == 2 && i * W + 1 < n) w |= (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i + 1] << 16;
+      r.q[i >> 2][i & 3] = w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(E) * 2; ++i) {
+      const unsigned w = r.q[i >> 2][i & 3];
+      r.q[i >> 2][i & 3] = sizeof(E) == 4 ? (i < n ? w : 0u) : (2 * i + 1 < n ? w : 2 * i < n ? w & 0xffffu : 0u);
+    }
+  }
+}
+
+// ---- products of fp32 / fp64 tiles: LDS stages [k][row] with a pitch of TB + 2 (fp64) or TB + 4 (fp32) -------------------
+template <typename T, int TB>
+struct Real {
+  static constexpr int P = TB + (sizeof(T) == 8 ? 2 : 4);
+  static constexpr int OPND = KD * P;              // elements of one operand's stage
+  static constexpr int NCH = TB * KD / 8;          // chunks per operand stage (at most one per thread)
+};
+
+struct NoTurn {
+  template <typename V> __device__ __forceinline__ void operator()(V&, int, int) const {}
+};
+template <typename T, int TB, typename E, bool EDGE, typename Turn>
+__device__ __forceinline__ void put_chunk(T* dst, const Opnd<E, EDGE>& o, Raw<E>& r, int c, int row0, int k0, Turn turn) {
+  constexpr int P = Real<T, TB>::P;
+  T v[8];
+  if constexpr (EDGE) mask_chunk<TB, KD>(o, r, c, row0, k0);
+  unpack(r, v);
+  int row, k;
+  chunk_at<TB, KD>(o.ks, c, row, k);
+  turn(v, row0 + row, k0 + k);
+  if (o.ks) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[k * P + row + i] = v[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[(k + i) * P + row] = v[i];
+  }
+}
+
+// K loop of one TB x TB tile:  sum over k in [kbeg, kend) of A(row0 + i, k) B(col0 + j, k), for NB column operands; `mma`
+// accumulates one stage of KD from the operands' LDS buffers (A first); `turn(v, col, k)` maps the chunk (col, k ..) of a column
+// operand on its way to LDS.  Two stages are on the way from memory while a third
+// is multiplied.
+template <typename T, int TB, int NB, typename OA, typename OB, typename Mma, typename Turn>
+__device__ __forceinline__ void real_loop(const OA& A, const OB (&B)[NB], int row0, int col0, int kbeg, int kend, T* lds, int tid,
+                                          Mma mma, Turn turn) {
+  typedef Real<T, TB> L;
+  constexpr int STG = (1 + NB) * L::OPND;
+  const int c = tid & (L::NCH - 1);
+  const bool own = tid < L::NCH;
+  decltype(fetch_chunk<TB, KD>(A, c, row0, kbeg)) va[2];
+  decltype(fetch_chunk<TB, KD>(B[0], c, col0, kbeg)) vb[2][NB];
+  auto fetch = [&](int s, int k0) {
+    va[s] = fetch_chunk<TB, KD>(A, c, row0, k0);
+#pragma unroll
+    for (int o = 0; o < NB; ++o) vb[s][o] = fetch_chunk<TB, KD>(B[o], c, col0, k0);
+  };
+  auto put = [&](int s, int k0) {
+    if (own) {
+      put_chunk<T, TB>(lds + s * STG, A, va[s], c, row0, k0, NoTurn());
+#pragma unroll
+      for (int o = 0; o < NB; ++o) put_chunk<T, TB>(lds + s * STG + (1 + o) * L::OPND, B[o], vb[s][o], c, col0, k0, turn);
+    }
+  };
+  fetch(0, kbeg);
+  if (kbeg + KD < kend) fetch(1, kbeg + KD);
+  put(0, kbeg);
+  for (int k0 = kbeg; k0 < kend; k0 += 2 * KD) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + s * KD;
+      if (k >= kend) break;
+      if (k + 2 * KD < kend) fetch(s, k + 2 * KD);
+      __syncthreads();
+      mma(lds + s * STG);
+      if (k + KD < kend) put(s ^ 1, k + KD);
+    }
+  }
+  __syncthreads();
+}
+
+// fp64 (and fp32 in 32-tiles): v_mfma_*_16x16x4, four wavefronts of TB/2 x TB/2
+template <typename T, int TB>
+struct Acc16 {
+  static constexpr int NBK = TB / 32, P = Real<T, TB>::P, H = TB / 2;
+  typename Mfma<T>::acc_t acc[NBK][NBK];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < NBK; ++i)
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) acc[i][j] = typename Mfma<T>::acc_t{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void stage(const T* sa, const T* sb, int lane, int wm, int wn) {
+#pragma unroll
+    for (int ks = 0; ks < KD / 4; ++ks) {
+      const int k = ks * 4 + (lane >> 4);
+      T af[NBK], bf[NBK];
+#pragma unroll
+      for (int i = 0; i < NBK; ++i) af[i] = sa[k * P + wm * H + i * 16 + (lane & 15)];
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) bf[j] = sb[k * P + wn * H + j * 16 + (lane & 15)];
+#pragma unroll
+      for (int i = 0; i < NBK; ++i)
+#pragma unroll
+        for (int j = 0; j < NBK; ++j) acc[i][j] = Mfma<T>::mma(af[i], bf[j], acc[i][j]);
+    }
+  }
+  // to the staging area d[row][col], pitch TB + 2; ends with a barrier
+  __device__ __forceinline__ void out(T* d, int lane, int wm, int wn) const {
+#pragma unroll
+    for (int i = 0; i < NBK; ++i)
+#pragma unroll
+      for (int j = 0; j < NBK; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          d[(wm * H + i * 16 + Mfma<T>::row(v, lane)) * (TB + 2) + wn * H + j * 16 + (lane & 15)] = acc[i][j][v];
+    __syncthreads();
+  }
+};
+template <typename T, int TB, typename OA, typename OB, typename Turn = NoTurn>
+__device__ __forceinline__ void tile16(const OA& A, const OB& B, int row0, int col0, int kbeg, int kend, T* lds, int tid, int lane,
+                                       int wm, int wn, Turn turn = Turn()) {
+  Acc16<T, TB> acc;
+  acc.clear();
+  const OB Bs[1] = {B};
+  real_loop<T, TB, 1>(A, Bs, row0, col0, kbeg, kend, lds, tid,
+                      [&](const T* st) { acc.stage(st, st + Real<T, TB>::OPND, lane, wm, wn); }, turn);
+  acc.out(lds, lane, wm, wn);
+}
+
+// fp32, 64-tiles: one v_mfma_f32_32x32x2 block per wavefront (the order of k of gemm_f32.hip); element e of `acc` is row
+// (lane & 31), column 8 (e / 4) + 4 (lane / 32) + e % 4 of the wavefront's block.  NB column operands share the row operand.
+template <int NB, typename OA, typename OB>
+__device__ __forceinline__ void tile32x2(const OA& A, const OB (&B)[NB], int row0, int col0, int kend, float* lds, int tid, int lane,
+                                         int wm, int wn, f32x16_t (&acc)[NB]) {
+  constexpr int P = Real<float, 64>::P, OPND = Real<float, 64>::OPND;
+#pragma unroll
+  for (int o = 0; o < NB; ++o)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[o][v] = 0.f;
+  real_loop<float, 64, NB>(A, B, row0, col0, 0, kend, lds, tid, [&](const float* st) {
+#pragma unroll
+    for (int ks = 0; ks < KD / 2; ++ks) {
+      const int k = ks * 2 + (lane >> 5);
+      const float fa = st[k * P + wm * 32 + (lane & 31)];
+#pragma unroll
+      for (int o = 0; o < NB; ++o)
+        acc[o] = __builtin_amdgcn_mfma_f32_32x32x2f32(st[(1 + o) * OPND + k * P + wn * 32 + (lane & 31)], fa, acc[o], 0, 0, 0);
+    }
+  }, NoTurn());
+}
+__device__ __forceinline__ void stage_f32(const f32x16_t& acc, float* stg, int lane, int wm, int wn) {
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    stg[(wm * 32 + (lane & 31)) * 66 + wn * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)] = acc[v];
+}
+
+// ---- products of bf16 tiles: the LDS layouts of gemm_bf16_tile.h, 64-deep stages through registers -----------------------
+// `acc` is called with every stage: the buffers of the row operand and of NB column operands, 8 KB each.
+template <int TB, int D, bool EDGE>
+__device__ __forceinline__ void put_bf16(char* dst, const Opnd<bf16_t, EDGE>& o, Raw<bf16_t>& r, int c, int row0, int k0) {
+  if constexpr (EDGE) mask_chunk<TB, D>(o, r, c, row0, k0);
+  const int q = c >> 3, ch = c & 7;   // (row or k, chunk): 8 chunks of a line either way
+  *reinterpret_cast<u32x4_t*>(dst + q * 128 + (o.ks ? ks_swizzle(ch, q) : kc_swizzle(ch, q)) * 16) = r.q[0];
+}
+template <int NB, bool EDGE, typename Acc>
+__device__ __forceinline__ void tile_bf16(const Opnd<bf16_t, EDGE>& A, const Opnd<bf16_t, false> (&B)[NB], int row0, int col0, int kend,
+                                          char* lds, int tid, Acc acc) {
+  constexpr int OPND = 64 * 64 * 2;
+  constexpr int STG = (1 + NB) * OPND;
+  Raw<bf16_t> v[2][1 + NB][2];   // two stages on the way while a third is multiplied
+  auto fetch = [&](int s2, int k0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v[s2][0][h] = fetch_chunk<64, 64>(A, tid + 256 * h, row0, k0);
+#pragma unroll
+      for (int o = 0; o < NB; ++o) v[s2][1 + o][h] = fetch_chunk<64, 64>(B[o], tid + 256 * h, col0, k0);
+    }
+  };
+  auto put = [&](int s2, int k0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      put_bf16<64, 64>(lds + s2 * STG, A, v[s2][0][h], tid + 256 * h, row0, k0);
+#pragma unroll
+      for (int o = 0; o < NB; ++o) put_bf16<64, 64>(lds + s2 * STG + (1 + o) * OPND, B[o], v[s2][1 + o][h], tid + 256 * h, col0, k0);
+    }
+  };
+  fetch(0, 0);
+  if (64 < kend) fetch(1, 64);
+  put(0, 0);
+  for (int k0 = 0; k0 < kend; k0 += 128) {
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const int k = k0 + s2 * 64;
+      if (k >= kend) break;
+      if (k + 128 < kend) fetch(s2, k + 128);
+      __syncthreads();
+      acc(lds + s2 * STG);
+      if (k + 64 < kend) put(s2 ^ 1, k + 64);
+    }
+  }
+  __syncthreads();
+}
+// P and R: v_mfma_f32_16x16x32_bf16, four 16 x 16 blocks per wavefront, to the staging area (pitch 66)
+template <bool EDGE>
+__device__ __forceinline__ void product_bf16(const Opnd<bf16_t, EDGE>& A, const Opnd<bf16_t, false>& B, int row0, int col0, int kend,
+                                             char* lds, int tid, int lane, int wm, int wn, float* stg) {
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const Opnd<bf16_t, false> Bs[1] = {B};
+  tile_bf16<1>(A, Bs, row0, col0, kend, lds, tid, [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8_t fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        fa[i] = A.ks ? read_frag16<64, true>(st, wm * 32 + i * 16, ks, lane) : read_frag16<64, false>(st, wm * 32 + i * 16, ks, lane);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[j] = read_frag16<64, true>(st + 8192, wn * 32 + j * 16, ks, lane);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    }
+  });
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        stg[(wm * 32 + i * 16 + (lane & 15)) * 66 + wn * 32 + j * 16 + (lane >> 4) * 4 + v] = acc[i][j][v];
+}
+// the updates: v_mfma_f32_32x32x16_bf16 as in the batched update kernel, both products at once
+__device__ __forceinline__ void update_bf16(const Opnd<bf16_t, false>& A, const Opnd<bf16_t, false> (&B)[2], int row0, int col0,
+                                            int kend, char* lds, int tid, int lane, int wm, int wn, f32x16_t (&acc)[2]) {
+#pragma unroll
+  for (int o = 0; o < 2; ++o)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[o][v] = 0.f;
+  tile_bf16<2>(A, B, row0, col0, kend, lds, tid, [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8_t fa = read_frag<64, false>(st, wm * 32, ks, lane);
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+        acc[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_frag<64, false>(st + (1 + o) * 8192, wn * 32, ks, lane), fa, acc[o], 0, 0, 0);
+    }
+  });
+}
+
+// ---- stores ------------------------------------------------------------------------------------------------------------
+
+// eight values at element offset e of a matrix of dtype f32 / bf16, n of them
+__device__ __forceinline__ void store8(char* p, int f32, long long e, int n, const float (&v)[8]) {
+  if (n <= 0) return;
+  if (f32) {
+    float* q = reinterpret_cast<float*>(p) + e;
+    if (n >= 8) {
+      u32x4_un_t x, y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = __builtin_bit_cast(unsigned, v[i]);
+        y[i] = __builtin_bit_cast(unsigned, v[4 + i]);
+      }
+      *reinterpret_cast<u32x4_un_t*>(q) = x;
+      *reinterpret_cast<u32x4_un_t*>(q + 4) = y;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < n) q[i] = v[i];
+    }
+  } else {
+    bf16_t* q = reinterpret_cast<bf16_t*>(p) + e;
+    if (n >= 8) {
+      u32x4_un_t x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = cvt_pk_bf16(v[2 * i], v[2 * i + 1]);
+      *reinterpret_cast<u32x4_un_t*>(q) = x;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < n) q[i] = f2bf(v[i]);
+    }
+  }
+}
+
+// nan_to_num of the dtype; 0 for an all-zero B (reference dion/dion.py:1416-1444)
+template <bool BF>
+__device__ __forceinline__ float guard(float x, bool nonzero, float alt) {
+  const float top = BF ? 3.3895313892515355e38f : 3.4028234663852886e38f;
+  if (BF) x = rbf(x);
+  if (x != x) x = 0.f;
+  else if (x > top) x = top;
+  else if (x < -top) x = -top;
+  return nonzero ? x : alt;
+}
+
+// ---- the serial part of the factorisation: a 64 x 64 diagonal block and its inverse (scheme of cholesky.hip) --------------
+// g: the block (lower triangle), pitch ld, in LDS, from `lds` on or anywhere.  dT receives the inverse factor, transposed (dT[k][x] = D[x][k], pitch LP).
+// A pivot that is not positive zeroes its column and is counted in `bad` (o + column + 1, the first one); `live`: columns
+// of the block that belong to the matrix (the others are identity and leave the pivot range alone).
+struct Quad { double v[4]; };
+__device__ __forceinline__ void diag_factor(const double* g, int ld, char* lds, double* dT, int live, int o, int tid, int lane,
+                                            int wave, int& bad, double& pmin, double& pmax) {
+#pragma clang fp contract(fast)
+  typedef Mfma<double>::acc_t acc_t;
+  double(*scol)[4][64] = reinterpret_cast<double(*)[4][64]>(lds);   // [2]: published block column of S
+  Quad(*yrow)[64] = reinterpret_cast<Quad(*)[64]>(lds + 4096);      // [2]: published row block of Y
+  Quad(*lops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 8192);      // [2]: L block column as MFMA operand
+  Quad(*xops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 12288);     // [2]: X
+  const int lc = lane & 15, lg = lane >> 4;
+  acc_t S[4], Y[4];
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = wave * 16 + Mfma<double>::row(v, lane), j = tj * 16 + lc;
+      S[tj][v] = tj <= wave ? (i >= j ? g[(long long)i * ld + j] : g[(long long)j * ld + i]) : 0.0;
+      Y[tj][v] = i == j ? 1.0 : 0.0;
+    }
+  __syncthreads();   // (the block may lie where the published ones go)
+  if (tid < 128) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) yrow[tid >> 6][tid & 63].v[k] = 0.0;
+  }
+  __syncthreads();
+  auto publish = [&](int q, int buf) {
+    const int tq = q >> 2, qq = q & 3;
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {
+      if (tj == tq && tj <= wave && (lc >> 2) == qq) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) scol[buf][lc & 3][wave * 16 + Mfma<double>::row(v, lane)] = S[tj][v];
+      }
+      if (wave == tq && tj <= wave) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int rr = Mfma<double>::row(v, lane);
+          if ((rr >> 2) == qq) yrow[buf][tj * 16 + lc].v[rr & 3] = Y[tj][v];
+        }
+      }
+    }
+  };
+  publish(0, 0);
+  __syncthreads();
+  for (int cb = 0; cb < 16; ++cb) {
+    const int buf = cb & 1, k0 = cb * 4;
+    double sv[4], a[4][4], di[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sv[k] = scol[buf][k][lane];
+    const Quad yv = yrow[buf][lane];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) a[ii][jj] = scol[buf][jj][k0 + ii];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const double p = a[c][c];
+      const bool ok = __builtin_amdgcn_class(p, 0x100);   // positive normal
+      double rs = ok ? __builtin_amdgcn_rsq(p) : 0.0;     // 2^-27: one step of third order
+      const double err = 1.0 - p * rs * rs;
+      rs = rs + rs * err * (0.5 + 0.375 * err);
+      di[c] = ok ? rs : 0.0;
+      bad = (!ok && bad == 0 && k0 + c < live) ? o + k0 + c + 1 : bad;
+      if (ok && k0 + c < live) {
+        pmin = p < pmin ? p : pmin;
+        pmax = p > pmax ? p : pmax;
+      }
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i) a[i][c] *= di[c];
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i)
+#pragma unroll
+        for (int j = c + 1; j <= i; ++j) a[i][j] -= a[i][c] * a[j][c];
+    }
+    double l[4], x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double tl = sv[k], tx = yv.v[k];
+#pragma unroll
+      for (int m = 0; m < k; ++m) {
+        tl -= l[m] * a[k][m];
+        tx -= a[k][m] * x[m];
+      }
+      l[k] = tl * di[k];
+      x[k] = tx * di[k];
+    }
+    Quad lo, xo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      lo.v[k] = lane > k0 + 3 ? l[k] : 0.0;
+      xo.v[k] = lane <= k0 + k ? x[k] : 0.0;
+    }
+    lops[buf][lane] = lo;
+    xops[buf][lane] = xo;
+    if (wave == (cb & 3)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dT[lane * LP + k0 + k] = xo.v[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (wave * 16 + 15 > k0 + 3) {
+      const double aop = -lops[buf][wave * 16 + lc].v[lg];
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        if (tj <= wave && tj * 16 + 15 > k0 + 3) S[tj] = Mfma<double>::mma(aop, lops[buf][tj * 16 + lc].v[lg], S[tj]);
+        if (tj <= wave && tj * 16 <= k0 + 3) Y[tj] = Mfma<double>::mma(aop, xops[buf][tj * 16 + lc].v[lg], Y[tj]);
+      }
+    }
+    if (cb + 1 < 16) publish(cb + 1, buf ^ 1);
+    __syncthreads();
+  }
+}
+
+// ---- the kernel ----------------------------------------------------------------------------------------------------------
+
+template <bool BF> struct MomentumType { typedef float type; };
+template <> struct MomentumType<true> { typedef bf16_t type; };
+
+template <bool BF>
+__global__ __launch_bounds__(256, 2) void dion_small_kernel(Args a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  __shared__ int sh_ticket[2];
+  __shared__ int sh_words[2];
+  __shared__ int sh_start[128], sh_per[128], sh_wait[128];   // the queue's schedule: entry = kind * ngroups + group
+  static_assert(KINDS * DA_DS_GROUPS <= 128, "one entry each");
+  constexpr int MSZ = BF ? 2 : 4, MT = BF ? DA_BF16 : DA_F32;
+  const int xcd = xcc_id();
+
+  for (int qi = 0; qi < DA_QUEUES; ++qi) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int q = (xcd + qi) & (DA_QUEUES - 1);
+    const int total = a.total[q];
+    if (total <= 0) continue;
+    unsigned* word = a.tickets + q * DA_QUEUE_LINE;
+    int slot = 0;
+    if (tid == 0) sh_ticket[0] = take_ticket(word, xcd, total, false);
+    __syncthreads();
+    if (wave_uniform(sh_ticket[0]) < 0) {
+      __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
+      continue;
+    }
+    // ---- the schedule, phase by phase, group by group: first ticket, tasks per matrix, and what a phase waits for
+    if (tid < 128) {
+      int n = 0;
+      if (tid < KINDS * a.ngroups) {
+        const int k = tid / a.ngroups;
+        const GroupDev& G = a.g[tid - k * a.ngroups];
+        const int per = tasks_of(G, k, BF);
+        n = per * da_in_queue(G.first, G.cnt, q);
+        int w = k == BTP ? PT : k - 1;
+        while (w >= 0 && tasks_of(G, w, BF) == 0) --w;
+        sh_per[tid] = per;
+        sh_wait[tid] = w < 0 ? -1 : (w << 24 | tasks_of(G, w, BF));
+      }
+      sh_start[tid] = n;
+    }
+    __syncthreads();
+    if (tid < 64) {   // exclusive sums of 128 entries by one wavefront
+      const int lo = sh_start[2 * lane], hi = sh_start[2 * lane + 1];
+      int sum = lo + hi;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(sum, o);
+        if (lane >= o) sum += x;
+      }
+      sh_start[2 * lane] = sum - lo - hi;
+      sh_start[2 * lane + 1] = sum - hi;
+    }
+    while (true) {
+      __syncthreads();
+      int t = wave_uniform(sh_ticket[slot]);
+      if (t < 0) break;
+      // (opaque to the compiler: every phase's address arithmetic would move out of this loop and be spilled)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+      // ---- ticket -> (kind, group, matrix, task): the last entry that starts at or before it
+      const int entry = wave_uniform(__popcll(__ballot(sh_start[lane] <= t)) + __popcll(__ballot(sh_start[64 + lane] <= t)) - 1);
+      t -= wave_uniform(sh_start[entry]);
+      const int kind = entry / a.ngroups, per = wave_uniform(sh_per[entry]), wait = wave_uniform(sh_wait[entry]);
+      const GroupDev& G = a.g[entry - kind * a.ngroups];
+      const int kth = wave_uniform(t / per);
+      const int task = wave_uniform(t - kth * per);
+      const int b = wave_uniform(((q - G.first) & 7) + 8 * kth);
+      int* words = G.words + (long long)b * CTR_STRIDE;
+      if (tid == 0) {
+        if (wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
+        int sick = __hip_atomic_load(words + W_SICK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (kind == BTP && sick) wait_count(words + FIX, tasks_of(G, FIX, BF), a.status, a.spin_limit);
+        sh_words[0] = __hip_atomic_load(words + W_NONZERO, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh_words[1] = sick;
+      }
+      __syncthreads();
+      const bool nonzero = sh_words[0] != 0, sick = sh_words[1] != 0;
+      int next = -1;
+      auto ask = [&]() {
+        if (tid == 0) next = take_ticket(word, xcd, total, true);
+      };
+
+      const int rp = G.rp, mpR = G.mpT * 64, npR = G.npT * 64;
+      char* const P = G.P + (long long)b * mpR * rp * MSZ;
+      char* const P2 = G.P2 + (long long)b * mpR * rp * MSZ;
+      char* const R = G.R + (long long)b * npR * rp * MSZ;
+      char* const Qw = G.Qw + (long long)b * npR * rp * MSZ;
+      char* const Qn = G.Qn + (long long)b * npR * rp * MSZ;
+      double* const P64 = G.P64 + (long long)b * mpR * rp;
+      const long long rr = (long long)rp * rp;
+      double* const L = G.L + b * rr;
+      double* const T = G.T + b * rr;
+      char* const M = static_cast<char*>(G.M[b]);
+      typedef typename MomentumType<BF>::type E;    // bf16_t or float
+      const long long last = (long long)G.m * G.n - 8;
+      auto momentum = [&](bool turned) {            // B' (false), B'^T (true)
+        return Opnd<E, true>{reinterpret_cast<const E*>(M), G.n, (G.transposed != 0) != turned, turned ? G.np : G.mp,
+                             turned ? G.mp : G.np, last};
+      };
+      float* const stg = reinterpret_cast<float*>(lds);
+
+      if (kind == ADD) {
+        ask();
+        const long long n = (long long)G.m * G.n;
+        const int mtasks = (int)((n + ADD_ELEMS - 1) / ADD_ELEMS);
+        if (task >= mtasks) {
+          // ---- Q in the momentum's dtype, padded to whole tiles
+          for (int h = 0; h < ADD_ELEMS / 2048; ++h) {
+            const long long e = (long long)(task - mtasks) * ADD_ELEMS + h * 2048 + tid * 8;
+            const int row = (int)(e / rp), col = (int)(e - (long long)row * rp);
+            if (row >= npR) break;
+            const int c = row < G.np ? G.r - col : 0;
+            float v[8];
+            if (a.q_f32) load8(static_cast<const float*>(G.Q[b]), (long long)row * G.r + col, c, v);
+            else load8(static_cast<const bf16_t*>(G.Q[b]), (long long)row * G.r + col, c, v);
+            store8(Qw, !BF, e, 8, v);
+          }
+        } else {
+          const long long e0 = (long long)task * ADD_ELEMS + tid * 8;
+          const bf16_t* const g16 = static_cast<const bf16_t*>(G.G[b]);
+          const float* const g32 = static_cast<const float*>(G.G[b]);
+          bool any = false;
+          auto finish = [&](const Raw<E>& mr, float (&g)[8], long long e, int c) {
+            float m[8];
+            unpack(mr, m);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              m[i] = BF ? rbf(m[i] + g[i]) : m[i] + g[i];
+              if (i < c) any |= m[i] != 0.f;
+            }
+            store8(M, !BF, e, c, m);
+          };
+          if ((long long)(task + 1) * ADD_ELEMS <= n) {   // every load on the way before the first is used
+            Raw<E> mr[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+              for (int i = 0; i < MSZ / 2; ++i) mr[h].q[i] = ldg16_l2(M + (e0 + h * 2048) * MSZ + 16 * i);
+            if (a.g_f32) {
+              Raw<float> gr[4];
+#pragma unroll
+              for (int h = 0; h < 4; ++h) gr[h] = load_raw(g32 + e0 + h * 2048);
+#pragma unroll
+              for (int h = 0; h < 4; ++h) {
+                float g[8];
+                unpack(gr[h], g);
+                finish(mr[h], g, e0 + h * 2048, 8);
+              }
+            } else {
+              Raw<bf16_t> gr[4];
+#pragma unroll
+              for (int h = 0; h < 4; ++h) gr[h] = load_raw(g16 + e0 + h * 2048);
+#pragma unroll
+              for (int h = 0; h < 4; ++h) {
+                float g[8];
+                unpack(gr[h], g);
+                finish(mr[h], g, e0 + h * 2048, 8);
+              }
+            }
+          } else {
+            for (int h = 0; h < 4; ++h) {
+              const long long e = e0 + h * 2048;
+              const int c = n - e >= 8 ? 8 : (int)(n - e);
+              if (c <= 0) break;
+              Raw<E> mr;
+#pragma unroll
+              for (int i = 0; i < MSZ / 2; ++i) mr.q[i] = u32x4_t{0, 0, 0, 0};
+              if (c == 8) {
+#pragma unroll
+                for (int i = 0; i < MSZ / 2; ++i) mr.q[i] = ldg16_l2(M + e * MSZ + 16 * i);
+              } else if (BF) {
+                unsigned w[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                  if (i < c) w[i >> 1] |= (unsigned)__hip_atomic_load(reinterpret_cast<const unsigned short*>(M) + e + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) << (16 * (i & 1));
+                mr.q[0] = u32x4_t{w[0], w[1], w[2], w[3]};
+              } else {
+                unsigned w[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                  w[i] = i < c ? __hip_atomic_load(reinterpret_cast<const unsigned*>(M) + e + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+                mr.q[0] = u32x4_t{w[0], w[1], w[2], w[3]};
+                mr.q[MSZ / 2 - 1] = u32x4_t{w[4], w[5], w[6], w[7]};
+              }
+              float g[8];
+              if (a.g_f32) load8(g32, e, c, g);
+              else load8(g16, e, c, g);
+              finish(mr, g, e, c);
+            }
+          }
+          if (__any(any) && lane == 0)
+            __hip_atomic_store(words + W_NONZERO, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      } else if (kind == BQ || kind == BTP) {
+        // ---- P = B' Q;  R = B'^T P
+        const bool bq = kind == BQ;
+        const int rT = G.rT, rt32 = (G.r + 31) >> 5;
+        const Opnd<E, true> sa = momentum(!bq);
+        const Opnd<E, false> sb = work<E>(bq ? Qw : P2, rp, 1);
+        const int kend = bq ? G.np : G.mp;
+        char* const C = bq ? P : R;
+        // a chunk of the result: rounded and, for R, guarded (an all-zero B keeps Q)
+        auto put = [&](int row0, int col0, int lr, int lc, int pitch) {
+          const int row = row0 + lr, col = col0 + lc;
+          float v[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = stg[lr * pitch + lc + i];
+          if (!bq) {
+            float alt[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) alt[i] = 0.f;
+            if (!nonzero) unpack(load_raw(reinterpret_cast<const E*>(Qw) + (long long)row * rp + col), alt);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = guard<BF>(v[i], nonzero, alt[i]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) stg[lr * pitch + lc + i] = v[i];
+          }
+          store8(C, !BF, (long long)row * rp + col, 8, v);
+        };
+        // the tile's share of the column norms
+        auto norms = [&](int ti, int row0, int col0, int pitch, int tb) {
+          __syncthreads();
+          double* const red = reinterpret_cast<double*>(lds + 64 * 66 * 4);
+          const int c = tid & (tb - 1), g = tid / tb, rows = tb * tb / 256;
+          double s = 0.0;
+          for (int i = g * rows; i < (g + 1) * rows; ++i) {
+            const float v = row0 + i < G.np ? stg[i * pitch + c] : 0.f;
+            s += (double)v * (double)v;
+          }
+          red[tid] = s;
+          __syncthreads();
+          if (tid < tb) {
+            double t = 0.0;
+            for (int i = 0; i < 256 / tb; ++i) t += red[i * tb + tid];
+            G.norm[((long long)b * G.nT + ti) * rp + col0 + tid] = t;
+          }
+        };
+        if (BF || bq) {
+          const int ti = task / rT, tj = task - ti * rT, row0 = wave_uniform(ti) * 64, col0 = wave_uniform(tj) * 64;
+          if constexpr (BF) {
+            product_bf16(sa, sb, row0, col0, kend, lds, tid, lane, wm, wn, stg);
+          } else {
+            f32x16_t acc[1];
+            const Opnd<E, false> sbs[1] = {sb};
+            tile32x2<1>(sa, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc);
+            stage_f32(acc[0], stg, lane, wm, wn);
+          }
+          ask();
+          __syncthreads();
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            put(row0, col0, (tid >> 3) + 32 * h, (tid & 7) * 8, 66);
+          }
+          if (!bq) norms(ti, row0, col0, 66, 64);
+        } else {
+          const int ti = task / rt32, tj = task - ti * rt32, row0 = wave_uniform(ti) * 32, col0 = wave_uniform(tj) * 32;
+          if constexpr (!BF) tile16<float, 32>(sa, sb, row0, col0, 0, kend, stg, tid, lane, wm, wn);
+          ask();
+          if (tid < 128) put(row0, col0, tid >> 2, (tid & 3) * 8, 34);
+          norms(ti, row0, col0, 34, 32);
+        }
+      } else if (kind == GRAM) {
+        // ---- one lower 32 x 32 tile of one K slice of P^T P
+        const int t32 = (G.r + 31) >> 5, per_slice = t32 * (t32 + 1) / 2;
+        const int slice = task / per_slice;
+        int rem = task - slice * per_slice, ti = 0;
+        while (rem > ti) { rem -= ti + 1; ++ti; }
+        ti = wave_uniform(ti);
+        const int tj = wave_uniform(rem);
+        const int kbeg = wave_uniform(slice) * G.kslice, kend = min(kbeg + G.kslice, (G.mp + KD - 1) / KD * KD);
+        const Opnd<E, false> s = work<E>(P, rp, 1);
+        double* const d = reinterpret_cast<double*>(lds);
+        tile16<double, 32>(s, s, ti * 32, tj * 32, kbeg, kend, d, tid, lane, wm, wn);
+        ask();
+        double* const out = G.slab + ((long long)b * G.slices + slice) * rr;
+        for (int e = tid; e < 1024; e += 256) out[(ti * 32 + (e >> 5)) * rp + tj * 32 + (e & 31)] = d[(e >> 5) * 34 + (e & 31)];
+      } else if (kind == FIX && !sick) {
+        ask();   // what nearly every matrix does
+      } else if (kind <= FIX) {
+        // ---- fp64 products of 64-tiles
+        double* const d = reinterpret_cast<double*>(lds);
+        const int rT = G.rT;
+        enum Job { J_DIAG, J_LOW, J_INV, J_PT, J_GRAM2, J_PV };
+        Job job = J_PT;
+        int j = 0, x = 0;            // block column / row
+        int row0 = 0, col0 = 0, kend = 0;
+        Opnd<double, false> sa{}, sb{};
+        if (kind == PT) {            // P T^T (T is triangular)
+          row0 = task / rT * 64;
+          col0 = (task - task / rT * rT) * 64;
+          kend = col0 + 64;
+          sb = work<double>(T, rp, 0);
+        } else if (kind == FIX) {
+          const int t32 = (G.r + 31) >> 5, ng = t32 * (t32 + 1) / 2;
+          if (task < ng) {           // a lower 32 x 32 tile of P64^T P64
+            job = J_GRAM2;
+            int rem = task;
+            while (rem > x) { rem -= x + 1; ++x; }
+            j = rem;
+          } else {
+            job = J_PV;
+            if (tid == 0) wait_count(words + W_GRAM2, ng, a.status, a.spin_limit);
+            row0 = (task - ng) / rT * 64;
+            col0 = (task - ng) % rT * 64;
+            kend = col0 + 64;
+          }
+        } else {
+          j = (kind - DIAG) >> 1;
+          if (!((kind - DIAG) & 1)) {
+            job = J_DIAG; x = j;
+          } else if (task < rT - 1 - j) {
+            job = J_LOW; x = j + 1 + task;
+          } else {
+            job = J_INV; x = task - (rT - 1 - j);
+          }
+          if (job == J_INV) {        // sum over k of L(j, k) T(k, x), x <= k < j
+            sa = work<double>(L + (long long)j * 64 * rp + x * 64, rp, 0);
+            sb = work<double>(T + (long long)x * 64 * rp + x * 64, rp, 1);
+            kend = (j - x) * 64;
+          } else {                   // sum over k < j of L(x, k) L(j, k)^T
+            sa = work<double>(L + (long long)x * 64 * rp, rp, 0);
+            sb = work<double>(L + (long long)j * 64 * rp, rp, 0);
+            kend = j * 64;
+          }
+        }
+        // the tile in d, guarded, to P2
+        auto put_p2 = [&]() {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = guard<BF>((float)d[r * 66 + c + i], nonzero, 0.f);
+            store8(P2, !BF, (long long)(row0 + r) * rp + col0 + c, 8, v);
+          }
+        };
+        row0 = wave_uniform(row0);
+        col0 = wave_uniform(col0);
+        kend = wave_uniform(kend);
+        if (job == J_GRAM2) {
+          const int ti = wave_uniform(x), tj = wave_uniform(j);
+          const Opnd<double, false> p = work<double>(P64, rp, 1);
+          tile16<double, 32>(p, p, ti * 32, tj * 32, 0, (G.mp + KD - 1) / KD * KD, d, tid, lane, wm, wn);
+          ask();
+          double* const out = G.A2 + b * rr;
+          for (int e = tid; e < 1024; e += 256) out[(ti * 32 + (e >> 5)) * rp + tj * 32 + (e & 31)] = d[(e >> 5) * 34 + (e & 31)];
+          // the tile's share of || column of P64^T P64 - I ||^2, by rows and (symmetric) by columns
+          if (tid < 64) {
+            const int i = tid & 31;
+            double s = 0.0;
+            for (int k = 0; k < 32; ++k) {
+              const double v = (tid < 32 ? d[i * 34 + k] : d[k * 34 + i]) - (ti == tj && i == k ? 1.0 : 0.0);
+              s += v * v;
+            }
+            const int c = (tid < 32 ? ti : tj) * 32 + i, t = tid < 32 ? tj : ti;
+            if (tid < 32 || ti != tj) G.defect[((long long)b * rp + c) * (2 * MAX_RT) + t] = s;
+          }
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+          if (tid == 0) __hip_atomic_fetch_add(words + W_GRAM2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else if (job == J_PV) {
+          // P64 V, V = I - up(G2 - I) with the columns that came from noise-level pivots dropped; V^T is formed from the lower
+          // tiles of G2 on the way to LDS
+          __syncthreads();   // thread 0 has waited
+          int* const drop = reinterpret_cast<int*>(lds + STAGES64);
+          if (tid < G.r) {
+            const double* const p = G.defect + ((long long)b * rp + tid) * (2 * MAX_RT);
+            double s = 0.0;
+            for (int t = 0; t < ((G.r + 31) >> 5); ++t) s += p[t];
+            drop[tid] = !(s <= 0.25) ? 1 : 0;
+          } else if (tid < rp) {
+            drop[tid] = 0;
+          }
+          __syncthreads();
+          if (row0 == 0 && col0 == 0 && tid == 0 && G.info &&
+              __hip_atomic_load(words + W_BAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+            for (int c = 0; c < G.r; ++c)
+              if (drop[c]) { G.info[b] = c + 1; break; }
+          }
+          tile16<double, 64>(work<double>(P64, rp, 0), work<double>(G.A2 + b * rr, rp, 0), row0, col0, 0, kend, d, tid, lane, wm, wn,
+                             [&](double (&v)[8], int c, int k) {
+            const bool gone = drop[c] != 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const double y = v[i];
+              const bool on = k + i == c;
+              double u = k + i < c ? -y : (on ? 1.5 - 0.5 * y : 0.0);
+              if (c >= G.r) u = on ? 1.0 : 0.0;               // beyond the rank: the identity
+              if (gone) u = 0.0;                              // a dropped column comes out as zero
+              else if (drop[k + i]) u = on ? 1.0 : 0.0;       // and gives no correction
+              v[i] = u;
+            }
+          });
+          ask();
+          put_p2();
+        } else {
+          typedef Real<double, 64> RD;
+          typedef Opnd<double, false> OD;
+          const OD sd = work<double>(T + (long long)j * 64 * rp + j * 64, rp, 0);   // D, the inverse of the diagonal block's factor
+          const bool two = job == J_LOW || job == J_INV;
+          do {
+            if (kind == PT) tile16<double, 64>(work<E>(P, rp, 0), sb, row0, col0, 0, kend, d, tid, lane, wm, wn);
+            else if (kend > 0) tile16<double, 64>(sa, sb, row0, col0, 0, kend, d, tid, lane, wm, wn);
+            if (job == J_PT) {
+              if (sick) {
+                for (int e = tid; e < 4096; e += 256) P64[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
+              } else {
+                put_p2();
+              }
+              break;
+            }
+            if (job == J_DIAG || two) {
+              Raw<double> dr[2];
+              if (two) {
+                dr[0] = fetch_chunk<64, KD>(sd, tid, 0, 0);
+                dr[1] = fetch_chunk<64, KD>(sd, tid, 0, KD);
+              }
+              double2_t w[8];        // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
+              const int k = (tid & 31) * 2, i0 = tid >> 5;
+#pragma unroll
+              for (int u = 0; u < 8; ++u) w[u] = double2_t{0.0, 0.0};
+              if (job != J_INV) {
+                // the slabs of P^T P in slice order; beyond the rank the matrix is the identity
+                const double* const slab = G.slab + (long long)b * G.slices * rr + (long long)(x * 64 + i0) * rp + j * 64 + k;
+                for (int s = 0; s < G.slices; ++s) {
+                  double2_t y[8];
+#pragma unroll
+                  for (int u = 0; u < 8; ++u) y[u] = *reinterpret_cast<const double2_t*>(slab + s * rr + (long long)u * 8 * rp);
+#pragma unroll
+                  for (int u = 0; u < 8; ++u) w[u] += y[u];
+                }
+                const int lim = ((G.r + 31) >> 5) << 5;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                  const int gi = x * 64 + i0 + 8 * u, gk = j * 64 + k;
+                  if (gi >= G.r || gk >= lim || (gk >> 5) > (gi >> 5)) {   // (not written by GRAM)
+                    w[u][0] = gi >= G.r && gi == gk ? 1.0 : 0.0;
+                    w[u][1] = gi >= G.r && gi == gk + 1 ? 1.0 : 0.0;
+                  }
+                }
+              }
+              if (kend > 0) {
+                const double sign = job == J_INV ? 1.0 : -1.0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                  w[u][0] += sign * d[(i0 + 8 * u) * 66 + k];
+                  w[u][1] += sign * d[(i0 + 8 * u) * 66 + k + 1];
+                }
+              }
+              if (job == J_DIAG) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                  d[(i0 + 8 * u) * 66 + k] = w[u][0];
+                  d[(i0 + 8 * u) * 66 + k + 1] = w[u][1];
+                }
+                __syncthreads();
+                int bad = 0;
+                double pmin = 3e38, pmax = 0.0;
+                double* const range = reinterpret_cast<double*>(words + W_RANGE);
+                if (j > 0) {
+                  bad = __hip_atomic_load(words + W_BAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  pmin = __hip_atomic_load(range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  pmax = __hip_atomic_load(range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                double* const dT = d + 2048;   // behind the 16 KB of the published blocks
+                diag_factor(d, 66, lds, dT, min(64, G.r - j * 64), j * 64, tid, lane, wave, bad, pmin, pmax);
+                double* const Dw = T + (long long)j * 64 * rp + j * 64;
+                for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * LP + (e >> 6)];
+                if (tid == 0) {
+                  __hip_atomic_store(words + W_BAD, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  __hip_atomic_store(range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  __hip_atomic_store(range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  if (j == rT - 1) {
+                    const bool healthy = bad == 0 && pmin >= PIVOT_RATIO * pmax && pmax > 0.0;
+                    __hip_atomic_store(words + W_SICK, healthy ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (G.info) G.info[b] = bad;
+                  }
+                }
+                break;
+              }
+              // second product, both operands to the LDS stages:  L(x, j) = W(x, j) D^T;   T(j, x) = -D W(j, x)
+              __syncthreads();
+              double* const wst = d + (job == J_INV ? RD::OPND : 0);
+              double* const dst = d + (job == J_INV ? 0 : RD::OPND);
+#pragma unroll
+              for (int u = 0; u < 8; ++u) {
+                const int i = i0 + 8 * u;
+                if (job == J_INV) {
+                  wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k] = w[u][0];
+                  wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k + 1] = w[u][1];
+                } else {
+                  wst[(k >> 5) * 2 * RD::OPND + (k & 31) * RD::P + i] = w[u][0];
+                  wst[(k >> 5) * 2 * RD::OPND + ((k + 1) & 31) * RD::P + i] = w[u][1];
+                }
+              }
+              put_chunk<double, 64>(dst, sd, dr[0], tid, 0, 0, NoTurn());
+              put_chunk<double, 64>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
+              __syncthreads();
+              Acc16<double, 64> acc;
+              acc.clear();
+              acc.stage(d, d + RD::OPND, lane, wm, wn);
+              acc.stage(d + 2 * RD::OPND, d + 3 * RD::OPND, lane, wm, wn);
+              __syncthreads();
+              acc.out(d, lane, wm, wn);
+            }
+            double* const out = job == J_INV ? T + (long long)j * 64 * rp + x * 64 : L + (long long)x * 64 * rp + j * 64;
+            const double sign = job == J_INV ? -1.0 : 1.0;
+            for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e >> 6) * 66 + (e & 63)];
+          } while (false);
+          ask();
+        }
+      } else if (kind == CNORM) {
+        // ---- a 64 x 64 tile of R: column norms from the tiles' shares (in order), Q_new in the momentum's dtype and as Q state
+        const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+        double* const red = reinterpret_cast<double*>(lds);
+        float* const den = reinterpret_cast<float*>(lds + 4096);
+        const int ti = wave_uniform(task / G.rT), row0 = ti * 64, col0 = wave_uniform(task - ti * G.rT) * 64;
+        const int limit = BF ? rp : ((G.r + 31) >> 5) << 5;   // columns of R that exist
+        Raw<E> rv[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          rv[h] = load_raw(reinterpret_cast<const E*>(R) + (long long)(row0 + (tid >> 3) + 32 * h) * rp + col0 + (tid & 7) * 8);
+        {
+          double s = 0.0;
+          if (col0 + (tid & 63) < limit)
+            for (int t = tid >> 6; t < G.nT; t += 4) s += G.norm[((long long)b * G.nT + t) * rp + col0 + (tid & 63)];
+          red[tid] = s;
+        }
+        __syncthreads();
+        if (tid < 64) den[tid] = sqrtf((float)(red[tid] + red[64 + tid] + red[128 + tid] + red[192 + tid])) + a.eps;
+        ask();
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int row = row0 + (tid >> 3) + 32 * h, c = (tid & 7) * 8, col = col0 + c;
+          float v[8];
+          unpack(rv[h], v);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            v[i] = v[i] / den[c + i];
+            if (BF) v[i] = rbf(v[i]);
+            if (poisoned) v[i] = __builtin_nanf("");
+            if (row >= G.np || col + i >= G.r) v[i] = 0.f;   // (padding)
+          }
+          store8(Qn, !BF, (long long)row * rp + col, 8, v);
+          store8(static_cast<char*>(G.Q[b]), a.q_f32, (long long)row * G.r + col, row < G.np ? G.r - col : 0, v);
+        }
+      } else if (kind == UPD) {
+        // ---- M += ef_alpha P R^T, X = decay X - lr P Q_new^T on one tile (rows of P, rows of R)
+        const int ti = wave_uniform(task / G.npT), tj = wave_uniform(task - task / G.npT * G.npT);
+        const int row0 = ti * 64, col0 = tj * 64;
+        const bool turned = G.transposed != 0;
+        const Opnd<E, false> sp = work<E>(P2, rp, 0), sr = work<E>(R, rp, 0), sn = work<E>(Qn, rp, 0);
+        const int kend = BF ? rp : ((G.r + 31) >> 5) << 5;   // (what the tiles of BTP have written)
+        char* const X = static_cast<char*>(G.X[b]);
+        float* const stg2 = stg + 64 * 66;
+        // a thread's chunks: stored row, eight consecutive stored columns; inside the matrix M and X are requested before the
+        // products
+        const int tr = turned ? col0 : row0, tc = turned ? row0 : col0;
+        const bool inside = tr + 64 <= G.m && tc + 64 <= G.n;
+        const long long e0 = (long long)(tr + (tid >> 3)) * G.n + tc + (tid & 7) * 8;
+        Raw<E> mr[2];
+        Raw<float> xr[2];      // (bf16 weights: the first quarter)
+        if (inside) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const long long e = e0 + 32LL * h * G.n;
+            mr[h] = load_raw(reinterpret_cast<const E*>(M) + e);
+            if (a.x_f32) xr[h] = load_raw(reinterpret_cast<const float*>(X) + e);
+            else xr[h].q[0] = load_raw(reinterpret_cast<const bf16_t*>(X) + e).q[0];
+          }
+        }
+        f32x16_t acc[2];
+        const Opnd<E, false> sbs[2] = {sr, sn};
+        if constexpr (BF) update_bf16(sp, sbs, row0, col0, kend, lds, tid, lane, wm, wn, acc);
+        else tile32x2<2>(sp, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc);
+        stage_f32(acc[0], stg, lane, wm, wn);
+        stage_f32(acc[1], stg2, lane, wm, wn);
+        ask();
+        __syncthreads();
+        const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+        const float lr = -G.scaled_lr;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
+          const long long e = e0 + 32LL * h * G.n;
+          const int n = tr + r < G.m ? G.n - tc - c : 0;
+          float mv[8], xv[8];
+          if (inside) {
+            unpack(mr[h], mv);
+            if (a.x_f32) unpack(xr[h], xv);
+            else unpack(Raw<bf16_t>{{xr[h].q[0]}}, xv);
+          } else {
+            load8(reinterpret_cast<const E*>(M), e, n, mv);
+            if (a.x_f32) load8(reinterpret_cast<const float*>(X), e, n, xv);
+            else load8(reinterpret_cast<const bf16_t*>(X), e, n, xv);
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int at = turned ? (c + i) * 66 + r : r * 66 + c + i;
+            // the roundings of the reference's separate tensor ops (epi_value in mfma_tile.h)
+            float t1 = stg[at], t2 = stg2[at];
+            if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
+            t1 = a.ef_alpha * t1;
+            t2 = lr * t2;
+            if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
+            mv[i] = mv[i] + t1;
+            float x = a.decay * xv[i];
+            if (!a.x_f32) x = rbf(x);
+            xv[i] = x + t2;
+            if (poisoned) mv[i] = xv[i] = __builtin_nanf("");
+          }
+          store8(M, !BF, e, n, mv);
+          store8(X, a.x_f32, e, n, xv);
+        }
+      } else {
+        ask();   // a phase that a healthy matrix does not need
+      }
+      // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
+      if (tid == 0) sh_ticket[slot ^ 1] = next;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) __hip_atomic_fetch_add(words + kind, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (in the L2)
+      slot ^= 1;
+    }
+    __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
+  }
+}
+
+struct Setup {
+  void* p[4][DA_DS_MATS];   // X, G, M, Q
+  void** dst;               // [4][n]
+  int n;
+  int* zero;
+  int nzero;
+  int* status;
+  int preset;
+};
+__global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < s.n) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s.dst[k * s.n + i] = s.p[k][i];
+  }
+  for (int e = i; e < s.nzero; e += gridDim.x * 256) s.zero[e] = 0;
+  if (i == 0) *s.status = s.preset;
+}
+
+inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+struct Shape {
+  int mp, np, mpT, npT, rT, rp, nT, slices, kslice;
+  Shape(int m, int n, int r, bool bf) {
+    mp = m > n ? m : n;
+    np = m > n ? n : m;
+    mpT = (mp + 63) / 64; npT = (np + 63) / 64; rT = (r + 63) / 64;
+    rp = rT * 64;
+    nT = bf ? npT : (np + 31) / 32;
+    // enough Gram tasks for an XCD's 32 compute units, at least 128 rows each
+    const int t32 = (r + 31) / 32, tiles = t32 * (t32 + 1) / 2;
+    slices = (64 + tiles - 1) / tiles;
+    if (slices > mp / 128) slices = mp / 128;
+    if (slices < 1) slices = 1;
+    kslice = ((mp + slices - 1) / slices + KD - 1) / KD * KD;
+    slices = (mp + kslice - 1) / kslice;
+  }
+};
+
+// lays out one group at p (null: only counts); returns the bytes
+size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, char* base) {
+  size_t o = 0;
+  auto take = [&](size_t n) { char* q = base ? base + o : nullptr; o += up256(n); return q; };
+  const size_t c = (size_t)g.cnt, pm = c * S.mpT * 64 * S.rp, pn = c * S.npT * 64 * S.rp, rr = c * S.rp * S.rp;
+  char* P = take(pm * msz);
+  char* P2 = take(pm * msz);
+  char* R = take(pn * msz);
+  char* Qn = take(pn * msz);
+  char* Qw = take(pn * msz);
+  char* norm = take(c * S.nT * S.rp * 8);
+  double* f64[6];   // P64, slab, L, T, A2, defect
+  for (int i = 0; i < 6; ++i) f64[i] = reinterpret_cast<double*>(take((i == 0 ? pm : i == 1 ? rr * S.slices : i == 5 ? c * S.rp * 2 * MAX_RT : rr) * 8));
+  if (D) {
+    D->P = P; D->P2 = P2; D->R = R; D->Qn = Qn; D->Qw = Qw; D->norm = reinterpret_cast<double*>(norm); D->nT = S.nT;
+    D->P64 = f64[0]; D->slab = f64[1]; D->L = f64[2]; D->T = f64[3]; D->A2 = f64[4]; D->defect = f64[5];
+  }
+  return o;
+}
+
+// control memory: words of all matrices, the queues' lines, the status word's line, the pointer tables
+size_t control_bytes(int mats) { return up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4) + up256((size_t)4 * mats * 8); }
+
+}  // namespace
+
+size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, bool forced) {
+  if (!g || n < 1 || n > DA_DS_GROUPS) return 0;
+  int mats = 0;
+  size_t bytes = 0;
+  // Where the line lies, in microseconds.  One launch: the chain of phases (90 in bf16, 135 in fp32, 60 more per further block of
+  // 64 columns of rank, 100 for a factor as wide as the matrix, which takes FIX) and the tiles of the XCD with the most.  A launch
+  // per product: what the host takes to issue a few hundred of them, 2.5 times that with shapes off the 8-grid (padded
+  // copies), plus the products, in fp32 at a fifth of the bf16 rate.  Measured, one launch against many, layers of four d x d and
+  // two d x 4d: bf16 d 128 r 64: 95 / 400;  256 x4 r 128: 204 / 464;  512 x8 r 32: 366 / 528;  512 x8 r 128: 502 / 534;
+  // 768 x4 r 192: 703 / 506.  fp32 256 x4 r 128: 272 / 559;  768 x4 r 48: 643 / 948;  768 x12 r 192: 3121 / 2259.
+  const bool bf = c.m_dtype == DA_BF16;
+  double load[DA_QUEUES] = {0}, chain = 0.0, other = 0.0;
+  bool padded = false, odd_full = false;
+  for (int i = 0; i < n; ++i) {
+    if (g[i].cnt < 1 || g[i].r < 1 || g[i].r > DA_DS_MAX_RANK || (long long)g[i].m * g[i].n > (1LL << 28) || (long long)g[i].m * g[i].n < 8) return 0;
+    const Shape S(g[i].m, g[i].n, g[i].r, c.m_dtype == DA_BF16);
+    for (int j = 0; j < g[i].cnt; ++j) {
+      // (lines of M and X must not be shared with another matrix; 16-byte loads of M and G by flat offset)
+      if (((uintptr_t)g[i].M[j] | (uintptr_t)g[i].X[j]) & 127) return 0;
+      if (((uintptr_t)g[i].G[j] | (uintptr_t)g[i].Q[j]) & 15) return 0;
+      load[(mats + j) & 7] += (double)S.mpT * S.npT * (bf ? 0.2 + 0.12 * S.rT : 0.25 + 0.25 * S.rT);
+    }
+    const double own = (bf ? 90.0 : 135.0) + 60.0 * (S.rT - 1) + (g[i].r == S.np ? 100.0 : 0.0);
+    chain = own > chain ? own : chain;
+    other += (bf ? 0.008 : 0.04) * g[i].cnt * S.mpT * S.npT * S.rT;
+    // (a full-rank factor of noise has a condition of 1e4 to 1e6, which multiplies every last-bit difference between the roads
+    // from step to step; off the 8-grid, where the other road's second pass works on a padded rank, they do differ)
+    odd_full |= g[i].r == S.np && (g[i].r & 7) != 0;
+    padded |= ((g[i].m | g[i].n) & 7) != 0;
+    mats += g[i].cnt;
+    bytes += lay_out(nullptr, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
+  }
+  if (mats > DA_DS_MATS) return 0;
+  double worst = 0;
+  for (int q = 0; q < DA_QUEUES; ++q) worst = load[q] > worst ? load[q] : worst;
+  other += (bf ? 400.0 : 480.0) * (padded ? 2.5 : 1.0);
+  if (!forced && (odd_full || chain + worst > other)) return 0;
+  return bytes + control_bytes(mats);
+}
+
+int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, void* workspace, hipStream_t s) {
+  Args a{};
+  Setup su;
+  int mats = 0;
+  char* p = static_cast<char*>(workspace);
+  for (int i = 0; i < n; ++i) mats += g[i].cnt;
+  if (mats > DA_DS_MATS || n > DA_DS_GROUPS) return DA_ERR_LIMIT;
+  int* words = reinterpret_cast<int*>(p);
+  a.tickets = reinterpret_cast<unsigned*>(words + (size_t)mats * CTR_STRIDE);
+  a.status = reinterpret_cast<int*>(a.tickets + DA_QUEUES * DA_QUEUE_LINE);
+  su.n = mats;
+  su.zero = words;
+  su.nzero = mats * CTR_STRIDE + DA_QUEUES * DA_QUEUE_LINE;
+  su.status = a.status;
+  su.preset = c.fail;
+  su.dst = reinterpret_cast<void**>(p + up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4));
+  p += control_bytes(mats);
+  int first = 0;
+  for (int i = 0; i < n; ++i) {
+    const Shape S(g[i].m, g[i].n, g[i].r, c.m_dtype == DA_BF16);
+    GroupDev& D = a.g[i];
+    p += lay_out(&D, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, p);
+    D.X = su.dst + first; D.G = su.dst + mats + first; D.M = su.dst + 2 * mats + first; D.Q = su.dst + 3 * mats + first;
+    for (int j = 0; j < g[i].cnt; ++j) {
+      su.p[0][first + j] = g[i].X[j];
+      su.p[1][first + j] = const_cast<void*>(g[i].G[j]);
+      su.p[2][first + j] = g[i].M[j];
+      su.p[3][first + j] = g[i].Q[j];
+    }
+    D.words = words + (size_t)first * CTR_STRIDE;
+    D.info = g[i].info;
+    D.cnt = g[i].cnt; D.first = first;
+    D.m = g[i].m; D.n = g[i].n; D.r = g[i].r; D.rp = S.rp; D.mp = S.mp; D.np = S.np;
+    D.mpT = S.mpT; D.npT = S.npT; D.rT = S.rT; D.transposed = g[i].m < g[i].n ? 1 : 0;
+    D.slices = S.slices; D.kslice = S.kslice;
+    D.scaled_lr = g[i].scaled_lr;
+    first += g[i].cnt;
+  }
+  a.ngroups = n;
+  for (int q = 0; q < DA_QUEUES; ++q)
+    for (int i = 0; i < n; ++i)
+      for (int k = 0; k < KINDS; ++k) a.total[q] += da_in_queue(a.g[i].first, a.g[i].cnt, q) * tasks_of(a.g[i], k, c.m_dtype == DA_BF16);
+  a.spin_limit = 200000000ull;   // 2 s of the 100 MHz counter
+  a.x_f32 = c.x_dtype == DA_F32; a.g_f32 = c.g_dtype == DA_F32; a.q_f32 = c.q_dtype == DA_F32;
+  a.ef_alpha = c.ef_alpha; a.decay = c.decay; a.eps = c.eps;
+  hipLaunchKernelGGL(dion_small_setup_kernel, dim3((unsigned)((su.nzero + 255) / 256)), dim3(256), 0, s, su);
+  int rc = da_launch_status();
+  if (rc) return rc;
+  static DaOncePerDevice configured;
+  rc = configured.run([&]() -> int {
+    DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
+    DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
+    return DA_OK;
+  });
+  if (rc) return rc;
+  const dim3 grid(2 * (unsigned)da_cu_count());
+  if (c.m_dtype == DA_BF16) hipLaunchKernelGGL(dion_small_kernel<true>, grid, dim3(256), SMEM, s, a);
+  else hipLaunchKernelGGL(dion_small_kernel<false>, grid, dim3(256), SMEM, s, a);
+  return da_launch_status();
+}

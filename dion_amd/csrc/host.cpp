@@ -23,10 +23,12 @@ struct Api {
   decltype(&dion_amd_muon_step_buckets) muon_step;
   decltype(&dion_amd_lion_step) lion_step;
   decltype(&dion_amd_adamw_step) adamw_step;
+  decltype(&dion_amd_dion_buckets_workspace_bytes) dion_bytes;
+  decltype(&dion_amd_dion_step_buckets) dion_step;
 } api;
 PyObject* g_error = nullptr;    // _lib.DionAmdError
 PyObject* g_check = nullptr;    // _lib.check(rc, what)
-PyObject *s_momentum, *s_variance, *s_get, *s_buf;
+PyObject *s_momentum, *s_variance, *s_q, *s_get, *s_buf;
 
 struct Failed {};   // a Python exception is set
 
@@ -57,7 +59,8 @@ struct Entry {
 
 // The parameters of `params` that have a gradient, with the state tensors named `keys`.  Appends the parameters without
 // state to `missing` (a Python list) instead.
-void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys, std::vector<Entry>& out, PyObject* missing) {
+void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys, std::vector<Entry>& out, PyObject* missing,
+            std::vector<PyObject*>* objects = nullptr) {
   const Py_ssize_t n = PyList_GET_SIZE(params);
   out.reserve((size_t)n);
   for (Py_ssize_t i = 0; i < n; ++i) {
@@ -76,6 +79,7 @@ void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys,
       continue;
     }
     out.emplace_back();
+    if (objects) objects->push_back(o);
     Entry& e = out.back();
     e.p = p;
     e.g = g;
@@ -226,6 +230,127 @@ PyObject* muon_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
   return nullptr;
 }
 
+// ---- Dion
+
+struct DionBucket {
+  Entry first;                   // shape, dtypes and device of the bucket
+  PyObject* p0;                  // its first parameter (borrowed)
+  std::vector<void*> X, M, Q;
+  std::vector<const void*> G;
+  std::vector<PyObject*> params; // borrowed
+  long long m, n, r;
+};
+
+// dion_group(params, state, lr, mu, weight_decay, epsilon, workspace, info) -> None when the step is done; a list: parameters
+// whose state has to be created first (nothing was done then); a tuple: parameters of the buckets that the one-launch entry
+// point does not take, which are left to the caller.  info(parameter, count): the status words of a bucket (int32 tensor).
+PyObject* dion_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
+  if (na != 8) { PyErr_SetString(PyExc_TypeError, "dion_group: 8 arguments"); return nullptr; }
+  PyObject* missing = nullptr;
+  try {
+    const float lr = (float)PyFloat_AsDouble(a[2]), mu = (float)PyFloat_AsDouble(a[3]), wd = (float)PyFloat_AsDouble(a[4]),
+                eps = (float)PyFloat_AsDouble(a[5]);
+    if (PyErr_Occurred()) return nullptr;
+    at::NoGradGuard no_grad;
+    missing = PyList_New(0);
+    if (!missing) return nullptr;
+    std::vector<Entry> all;
+    std::vector<PyObject*> objects;
+    PyObject* const keys[2] = {s_momentum, s_q};
+    gather(a[0], a[1], keys, 2, all, missing, &objects);
+    if (PyList_GET_SIZE(missing)) return missing;
+    Py_CLEAR(missing);
+
+    std::vector<DionBucket> buckets;
+    for (size_t k = 0; k < all.size(); ++k) {
+      Entry& e = all[k];
+      DionBucket* b = nullptr;
+      for (DionBucket& c : buckets)
+        if (c.first.p.sizes().equals(e.p.sizes()) && c.first.p.scalar_type() == e.p.scalar_type() &&
+            c.first.g.scalar_type() == e.g.scalar_type() && c.first.p.device() == e.p.device()) { b = &c; break; }
+      if (!b) {
+        if (!e.p.is_cuda()) {
+          PyErr_Format(g_error, "Dion.step: tensor is on %s; the MI355X kernels need a GPU tensor (no CPU fallback)",
+                       e.p.device().str().c_str());
+          throw Failed();
+        }
+        buckets.emplace_back();
+        b = &buckets.back();
+        b->first = e;
+        b->p0 = objects[k];
+        b->m = e.p.size(0); b->n = e.p.size(1); b->r = e.s[1].size(1);
+      }
+      if (!e.p.is_contiguous() || !e.s[0].is_contiguous() || !e.s[1].is_contiguous())
+        fail("Dion.step: parameters and optimizer states must be contiguous");
+      if (!e.s[0].sizes().equals(e.p.sizes()) || e.s[1].size(0) != std::min(b->m, b->n) || e.s[1].size(1) != b->r)
+        fail("Dion.step: optimizer states do not fit their parameter");
+      if (!e.g.is_contiguous()) e.g = e.g.contiguous();
+      b->X.push_back(e.p.data_ptr());
+      b->G.push_back(e.g.data_ptr());
+      b->M.push_back(e.s[0].data_ptr());
+      b->Q.push_back(e.s[1].data_ptr());
+      b->params.push_back(objects[k]);
+    }
+
+    // buckets of one set of dtypes and device go to the library together
+    const float decay = 1.f - lr * wd, ef_alpha = -(1.f - mu);
+    std::vector<char> done(buckets.size(), 0);
+    std::vector<dion_amd_dion_bucket> call;
+    std::vector<DionBucket*> members;
+    std::vector<PyObject*> left;
+    for (size_t i = 0; i < buckets.size(); ++i) {
+      if (done[i]) continue;
+      const Entry f = buckets[i].first;
+      call.clear();
+      members.clear();
+      for (size_t j = i; j < buckets.size(); ++j) {
+        DionBucket& b = buckets[j];
+        if (done[j] || b.first.p.scalar_type() != f.p.scalar_type() || b.first.g.scalar_type() != f.g.scalar_type() ||
+            b.first.s[0].scalar_type() != f.s[0].scalar_type() || b.first.s[1].scalar_type() != f.s[1].scalar_type() ||
+            b.first.p.device() != f.p.device())
+          continue;
+        done[j] = 1;
+        members.push_back(&b);
+        const float scale = (float)std::pow((double)b.m / (double)b.n, 0.5);
+        call.push_back({b.X.data(), b.G.data(), b.M.data(), b.Q.data(), (int)b.X.size(), (int)b.m, (int)b.n, (int)b.r, scale * lr, nullptr});
+      }
+      const c10::Device dev = f.p.device();
+      const int xc = dtype_code(f.p.scalar_type()), gc = dtype_code(f.g.scalar_type()), mc = dtype_code(f.s[0].scalar_type()),
+                qc = dtype_code(f.s[1].scalar_type());
+      const size_t need = api.dion_bytes(call.data(), (int)call.size(), xc, gc, mc, qc);
+      if (need == 0) {
+        for (DionBucket* b : members) left.insert(left.end(), b->params.begin(), b->params.end());
+        continue;
+      }
+      for (size_t j = 0; j < members.size(); ++j) {
+        PyObject* cnt = PyLong_FromSize_t(members[j]->X.size());
+        PyObject* t = cnt ? PyObject_CallFunctionObjArgs(a[7], members[j]->p0, cnt, nullptr) : nullptr;
+        Py_XDECREF(cnt);
+        if (!t) throw Failed();
+        call[j].info = static_cast<int*>(THPVariable_Unpack(t).data_ptr());
+        Py_DECREF(t);   // (the optimizer holds it)
+      }
+      char* ws = workspace(a[6], need, dev);
+      const c10::DeviceGuard guard(dev);
+      check(api.dion_step(call.data(), (int)call.size(), xc, gc, mc, qc, ef_alpha, decay, eps, ws, need, stream_of(dev)),
+            "dion_amd_dion_step_buckets");
+    }
+    if (left.empty()) Py_RETURN_NONE;
+    PyObject* rest = PyTuple_New((Py_ssize_t)left.size());
+    if (!rest) return nullptr;
+    for (size_t i = 0; i < left.size(); ++i) {
+      Py_INCREF(left[i]);
+      PyTuple_SET_ITEM(rest, (Py_ssize_t)i, left[i]);
+    }
+    return rest;
+  } catch (const Failed&) {
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+  }
+  Py_XDECREF(missing);
+  return nullptr;
+}
+
 // ---- Lion / AdamW
 
 // (hyper-parameters are evaluated like 0-dim fp32 tensors, reference dion/scalar_opts.py:89-187)
@@ -362,8 +487,8 @@ PyObject* element_lists(PyObject*, PyObject* const* a, Py_ssize_t na) {
 // bind(DionAmdError, check, addresses of the entry points in the order of Api)
 PyObject* bind(PyObject*, PyObject* args) {
   PyObject *err, *chk;
-  unsigned long long f[4];
-  if (!PyArg_ParseTuple(args, "OOKKKK", &err, &chk, f, f + 1, f + 2, f + 3)) return nullptr;
+  unsigned long long f[6];
+  if (!PyArg_ParseTuple(args, "OOKKKKKK", &err, &chk, f, f + 1, f + 2, f + 3, f + 4, f + 5)) return nullptr;
   Py_INCREF(err);
   Py_INCREF(chk);
   g_error = err;
@@ -372,12 +497,15 @@ PyObject* bind(PyObject*, PyObject* args) {
   api.muon_step = reinterpret_cast<decltype(api.muon_step)>(f[1]);
   api.lion_step = reinterpret_cast<decltype(api.lion_step)>(f[2]);
   api.adamw_step = reinterpret_cast<decltype(api.adamw_step)>(f[3]);
+  api.dion_bytes = reinterpret_cast<decltype(api.dion_bytes)>(f[4]);
+  api.dion_step = reinterpret_cast<decltype(api.dion_step)>(f[5]);
   Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, "Entry points of the loaded library."},
     {"muon_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(muon_group)), METH_FASTCALL, "Muon step of a group."},
+    {"dion_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dion_group)), METH_FASTCALL, "Dion step of a group."},
     {"element_group", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(element_group)), METH_FASTCALL,
      "Lion / AdamW step of a group."},
     {"element_lists", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(element_lists)), METH_FASTCALL,
@@ -390,6 +518,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host side of the optimize
 PyMODINIT_FUNC PyInit__host() {
   s_momentum = PyUnicode_InternFromString("momentum");
   s_variance = PyUnicode_InternFromString("variance");
+  s_q = PyUnicode_InternFromString("Q");
   s_get = PyUnicode_InternFromString("get");
   s_buf = PyUnicode_InternFromString("_buf");
   return PyModule_Create(&module);

@@ -6,9 +6,8 @@
 constexpr int DA_SMALL_BT = 64;           // tile edge: working matrices are padded to multiples of it
 constexpr int DA_SMALL_MAX_STEPS = 8;
 constexpr int DA_SMALL_CTR_STRIDE = 32;   // ints of control memory per matrix (one counter per phase)
-// ints behind the counters: a 128-byte line per queue (ticket word, owner word), then the status word's line
-constexpr int DA_SMALL_LINE = 32;
-constexpr int DA_SMALL_TAIL = 9 * DA_SMALL_LINE;
+// ints behind the counters: a line per queue (ticket word, owner word), then the status word's line
+constexpr int DA_SMALL_TAIL = 9 * 32;
 
 // One bucket of `cnt` same-shape wide matrices, mw <= nw multiples of 64, in bf16 working buffers
 // x0, x1: [cnt][mw][ldx], a, b: [cnt][mw][lda].  x0 holds the staged input (not yet divided by its norm), zero outside

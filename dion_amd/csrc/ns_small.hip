@@ -29,13 +29,14 @@
 // instruction, order of k and rounding-faithful epilogue arithmetic are those of gemm_bf16_tile.h, so the products have the
 // same bits as the batched kernel's.
 #include "ns_small.h"
+#include "flow_queue.h"
 #include "gemm_bf16_tile.h"
 
 namespace {
 
 typedef Cfg<64, 2, 2, 16> Sm;
 constexpr int BT = DA_SMALL_BT;
-constexpr int NQ = 8;                      // queues = XCDs
+constexpr int NQ = DA_QUEUES;
 constexpr int NST = 4;                     // LDS stage buffers
 constexpr int STAGE = 2 * BT * BK * 2;     // bytes of one stage: both operands
 constexpr int PITCH = BT + 4;              // floats per row of the epilogue's staging area
@@ -59,7 +60,7 @@ struct GroupDev {
 struct SmallArgs {
   GroupDev g[DA_MAX_GROUPS];
   float coeffs[3 * DA_SMALL_MAX_STEPS];
-  unsigned* tickets;         // [NQ][DA_SMALL_LINE]
+  unsigned* tickets;         // [NQ][DA_QUEUE_LINE]
   int* status;
   unsigned long long spin_limit;
   float eps;
@@ -67,8 +68,7 @@ struct SmallArgs {
   int sym32;                 // the symmetric products in 32 x 32 tiles
 };
 
-__device__ __forceinline__ int ceil8(int x) { return (x + 7) >> 3; }   // x >= -7
-__device__ __forceinline__ int in_queue(const GroupDev& G, int q) { return ceil8(G.first + G.cnt - q) - ceil8(G.first - q); }
+__device__ __forceinline__ int in_queue(const GroupDev& G, int q) { return da_in_queue(G.first, G.cnt, q); }
 // tasks per matrix: kind 0 normalisation, 1 / 2 the symmetric products, 3 X'
 __device__ __forceinline__ int tasks_of(const GroupDev& G, int kind, int sym32) {
   if (kind == 0) return G.tnorm;
@@ -120,27 +120,6 @@ __device__ __forceinline__ Item decode(const SmallArgs& a, int q, int t) {
     }
   }
   return r;
-}
-
-__device__ __forceinline__ unsigned long long now_ticks() { return __builtin_amdgcn_s_memrealtime(); }
-
-// Next ticket of a queue for a workgroup on XCD `xcd`, or -1: the queue is used up or belongs to another XCD.  word[0] is
-// the ticket counter, word[1] the owner (XCD + 1).  Only the owner's workgroups touch the counter, so its atomics need no
-// more than the XCD's own L2 (workgroup scope: no sc1 bit): of agent scope they take 130 ns each, one after the other,
-// 8 us for the 64 tiles of a 512 x 512 product.
-__device__ __forceinline__ int take_ticket(unsigned* word, int xcd, int total, bool owned) {
-  const unsigned me = (unsigned)(xcd + 1);
-  if (!owned) {
-    unsigned cur = __hip_atomic_load(word + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (cur == 0) {
-      unsigned expect = 0;
-      cur = __hip_atomic_compare_exchange_strong(word + 1, &expect, me, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT) ? me : expect;
-    }
-    if (cur != me) return -1;
-  }
-  const unsigned idx = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  return idx < (unsigned)total ? (int)idx : -1;
 }
 
 // Waits until at most the loads of n stages behind the one needed are in flight: four direct-to-LDS loads each, completed
@@ -312,7 +291,7 @@ __global__ __launch_bounds__(256, 2) void ns_small_kernel(SmallArgs a) {
   const int lane = tid & 63;
   const int wave = wave_uniform(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int xcd = (int)(__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u);   // XCC_ID
+  const int xcd = xcc_id();
 
   for (int qi = 0; qi < NQ; ++qi) {
     const int q = (xcd + qi) & (NQ - 1);
@@ -325,7 +304,7 @@ __global__ __launch_bounds__(256, 2) void ns_small_kernel(SmallArgs a) {
     total = total * a.steps + norms;
     if (total <= 0) continue;
     int slot = 0;
-    if (tid == 0) sh_ticket[0] = take_ticket(a.tickets + q * DA_SMALL_LINE, xcd, total, false);
+    if (tid == 0) sh_ticket[0] = take_ticket(a.tickets + q * DA_QUEUE_LINE, xcd, total, false);
     while (true) {
       __syncthreads();
       const int t = wave_uniform(sh_ticket[slot]);
@@ -341,18 +320,7 @@ __global__ __launch_bounds__(256, 2) void ns_small_kernel(SmallArgs a) {
         if (w.phase > 0) {
           // the product this tile reads must be complete for its matrix
           const int want = tasks_of(G, w.phase == 1 ? 0 : (w.kind == 1 ? 3 : w.kind - 1), a.sym32);
-          unsigned spins = 0;
-          unsigned long long t0 = 0;
-          while (__hip_atomic_load(ctr - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
-            // (the status word and the clock every 32nd time only: each load is a round trip to the L2)
-            if ((spins++ & 31) != 31) continue;
-            if (t0 == 0) t0 = now_ticks();
-            if (now_ticks() - t0 > a.spin_limit ||
-                __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-              __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              break;
-            }
-          }
+          wait_count(ctr - 1, want, a.status, a.spin_limit);
         }
       }
       __syncthreads();
@@ -360,7 +328,7 @@ __global__ __launch_bounds__(256, 2) void ns_small_kernel(SmallArgs a) {
       int next = -1;   // (thread 0) the next ticket, asked for when this task is on its way: not earlier, or a waiting
                        // workgroup would hold two tasks of a phase while others have none
       auto ask = [&]() {
-        if (tid == 0) next = take_ticket(a.tickets + q * DA_SMALL_LINE, xcd, total, true);
+        if (tid == 0) next = take_ticket(a.tickets + q * DA_QUEUE_LINE, xcd, total, true);
       };
       if (w.kind == 0) {
         // ---- X <- X / (||X||_F + eps), the divisor from the matrix's partial sums (the order and the roundings of
@@ -621,7 +589,7 @@ int da_ns_small(const DaNsSmallGroup* g, int n, const float* coeffs, int steps, 
   a.ngroups = n; a.steps = steps; a.eps = eps;
   int* tail = ctl + (size_t)first * DA_SMALL_CTR_STRIDE;
   a.tickets = reinterpret_cast<unsigned*>(tail);
-  a.status = tail + NQ * DA_SMALL_LINE;
+  a.status = tail + NQ * DA_QUEUE_LINE;
   a.spin_limit = 200000000ull;   // 2 s of the 100 MHz counter
   // 32-tiles for the symmetric products while those of every queue fit one and a half rounds of its 64 workgroups
   long long most = 0;

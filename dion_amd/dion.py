@@ -5,8 +5,9 @@ arguments, defaults, validation errors, param-group keys and `self.state` layout
 (`state[p]["momentum"]`, `state[p]["Q"]`, plus `"variance"` for AdamW groups).  One GPU only:
 `replicate_mesh`, `outer_shard_mesh` and `inner_shard_mesh` must be None.
 
-Per `step()` the matrices of every "dion" group are bucketed by (shape, dtype) and each bucket
-goes, as arrays of device pointers, to `dion_amd_dion_step_qr`: B = M + G, the tall-skinny MFMA
+Per `step()` the matrices of every "dion" group are bucketed by (shape, dtype).  Buckets of small matrices go to
+`dion_amd_dion_step_buckets` together, the whole step as one launch (gathered natively, `_host.dion_group`).  Any other
+bucket goes, as arrays of device pointers, to `dion_amd_dion_step_qr`: B = M + G, the tall-skinny MFMA
 GEMMs P = B Q and R = B^T P, a CholeskyQR orthonormalisation of P on the device (an fp32 pass on the bf16 matrix
 cores, an fp64 pass for the factors whose measured defect asks for it, a closed-form polishing step; no host
 synchronisation), the column normalisation that yields the next Q, and error feedback and weight update as one
@@ -240,15 +241,39 @@ class Dion(Optimizer):
         state["Q"] = torch.randn(q_shape, device=param.device, dtype=q_dtype)
 
     # ------------------------------------------------------------------ dion
+    def _bucket_info(self, p: Tensor, count: int) -> Tensor:
+        """Status words of p's bucket (see `cholesky_info`)."""
+        key = (p.shape, p.dtype, p.grad.dtype, p.device)
+        info = self._info.get(key)
+        if info is None or info.numel() != count:
+            info = self._info[key] = torch.zeros(count, dtype=torch.int32, device=p.device)
+        return info
+
     def _dion_group_step(self, group: dict):
-        params = [p for p in group["params"] if p.grad is not None]
-        if not params:
-            return
-        for p in params:
-            if p.ndim > 2:
+        for p in group["params"]:
+            if p.ndim > 2 and p.grad is not None:
                 raise NotImplementedError(
                     f"Tensors with more than 2 dimensions are not supported. Got {p.ndim}D tensor."
                 )
+        if self._REFERENCE_OPTIONS:
+            # (sketches, several power iterations, the choice of QR method: bucket by bucket)
+            self._dion_params_step(group, [p for p in group["params"] if p.grad is not None])
+            return
+        args = (group["params"], self.state, float(group["lr"]), float(group["mu"]), float(group["weight_decay"]),
+                float(group["epsilon"]), self._workspaces[0], self._bucket_info)
+        host = _lib.host()
+        left = host.dion_group(*args)
+        if isinstance(left, list):
+            for p in left:
+                self._get_or_initialize_state(p, group)
+            left = host.dion_group(*args)
+        if left:
+            self._dion_params_step(group, left)
+
+    def _dion_params_step(self, group: dict, params):
+        """The buckets of `params`, each with launches of its own on a stream of its own."""
+        if not params:
+            return
         # hyper-parameters as 0-dim fp32 tensors, evaluated like reference dion/dion.py:327-331, 852, 859-870
         lr = torch.tensor(group["lr"])
         mu = torch.tensor(group["mu"])
@@ -266,10 +291,7 @@ class Dion(Optimizer):
             _lib.require_gpu(plist[0], "Dion.step")
             for p in plist:
                 self._get_or_initialize_state(p, group)
-            key = (shape, dtype, gdtype, device)
-            info = self._info.get(key)
-            if info is None or info.numel() != len(plist):
-                self._info[key] = torch.zeros(len(plist), dtype=torch.int32, device=device)
+            self._bucket_info(plist[0], len(plist))
         slots = min(len(buckets), self._max_concurrent_tasks)
         # A bucket's step is one library call that enqueues a few hundred launches on the bucket's stream.  With
         # several buckets the calls of a wave (one bucket per stream) are made by worker threads side by side: at a

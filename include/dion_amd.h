@@ -303,6 +303,27 @@ int dion_amd_dion_step_qr(void* const* X, const void* const* G, void* const* M, 
                           int power_iters, int qr_method,
                           int* info, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Several buckets of small matrices in one call and ONE launch (after a small set-up launch): replaces the task generator
+ * and the task runtime around dion_update_ddp for a set of buckets (reference dion/dion.py:234-385, dion/opt_utils.py
+ * AsyncRuntime).  Same update as dion_amd_dion_step with power_iters 1, orthonormaliser in fp64 throughout; any m, n, rank up
+ * to 256; rows may have any length, X and M must be 128-byte aligned, G and Q 16-byte.
+ * dion_amd_dion_buckets_workspace_bytes returns 0 when this entry point does not take the buckets (ranks, alignment, more
+ * than 8 buckets or 96 matrices) or when the per-bucket entry points are faster (much work): use those then. */
+typedef struct dion_amd_dion_bucket {
+  void* const* X;        /* HOST arrays of `batch` device pointers, as in dion_amd_dion_step */
+  const void* const* G;
+  void* const* M;
+  void* const* Q;
+  int batch, m, n, r;
+  float scaled_lr;       /* sqrt(m / n) * lr */
+  int* info;             /* device, `batch` ints, may be NULL */
+} dion_amd_dion_bucket;
+size_t dion_amd_dion_buckets_workspace_bytes(const dion_amd_dion_bucket* buckets, int nbuckets, int x_dtype, int g_dtype,
+                                             int m_dtype, int q_dtype);
+int dion_amd_dion_step_buckets(const dion_amd_dion_bucket* buckets, int nbuckets, int x_dtype, int g_dtype, int m_dtype,
+                               int q_dtype, float ef_alpha, float decay, float eps,
+                               void* workspace, size_t workspace_bytes, void* stream);
+
 /* The reference's randomised Cholesky QR with the random sketch GIVEN by the caller (the async `orthogonalize`,
  * reference dion/dion.py:1274-1308, whose sketch comes from generate_random_sketch_matrix, 1221-1263; the same
  * sequence in dion/dion_reference.py:764-787):
@@ -377,6 +398,8 @@ int dion_amd_profile_read(int kind, long long* launches, double* total_ms, doubl
  *   "edge_loop"     bf16 products with a ragged dimension on a k-strided operand (Dion's rank-r products at r = 192):
  *                   1 the direct-to-LDS K loop with edge tiles, 0 the bounds-checked K loop, -1 the default (1 unless
  *                   DION_AMD_NO_EDGE_LOOP is set in the environment).  Both give the same bits.
+ *   "dion_small"    whether dion_amd_dion_buckets_workspace_bytes takes buckets of small matrices: 1 whenever it can, 0 never,
+ *                   -1 the default (up to an amount of work per XCD).
  *   "ns_flow_fail"  test hook: 1 makes every persistent launch (and that for small matrices) start with its status word set, as if a wait had
  *                   run into its limit; the results of such a launch are NaN.
  * The value applies to calls that start after this one returns, on every thread.  Unknown name:
