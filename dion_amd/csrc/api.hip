@@ -33,6 +33,24 @@ inline int padded_dim(int x) {
   return r256 * 100LL <= r128 * 107LL ? r256 : r128;
 }
 
+// Whether the buckets of one grouped call all go to whole 256-tiles: a grouped product runs 256-tiles only where every member
+// has them, so one member on the 128-grid costs all of them a third more per multiply-add.  (14 of 2368 x 2368 and 7 each of
+// 7040 x 2368 and 2368 x 7040 with 14 of 789 x 2368, padded to 896: 22.0 ms, padded to 1024: 17.3 ms.)
+template <typename Bucket, typename Count>
+bool grid256(const Bucket* k, int n, Count count) {
+  double nat = 0.0, big = 0.0;
+  bool on = false, off = false;
+  for (int i = 0; i < n; ++i) {
+    const int mw = k[i].m < k[i].n ? k[i].m : k[i].n, nw = k[i].m < k[i].n ? k[i].n : k[i].m;
+    auto cost = [&](double a, double b) { return count(k[i]) * a * a * (3.0 * b + a); };
+    const int am = padded_dim(mw), an = padded_dim(nw), bm = round_up(mw, 256), bn = round_up(nw, 256);
+    (am == bm && an == bn ? on : off) = true;
+    nat += cost(am, an);
+    big += cost(bm, bn);
+  }
+  return on && off && big <= 1.33 * nat;
+}
+
 constexpr size_t FLOW_TAIL_BYTES = 1536;   // behind the counters of a control area: ticket, owner and status words
 
 struct NsLayout {
@@ -43,12 +61,13 @@ struct NsLayout {
   size_t per_matrix = 0;
   NsLayout() {}
   // m x n matrices; `small`: the layout of the one-launch kernel for small matrices (ns_small.hip), which never needs
-  // more memory than the other one
-  NsLayout(int m, int n, int dtype, bool small = false) {
+  // more memory than the other one; `all256`: see grid256
+  NsLayout(int m, int n, int dtype, bool small = false, bool all256 = false) {
     mw = m < n ? m : n;
     nw = m < n ? n : m;
     if (dtype != DA_BF16) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
     else if (small) { mw = round_up(mw, DA_SMALL_BT); nw = round_up(nw, DA_SMALL_BT); }
+    else if (all256) { mw = round_up(mw, 256); nw = round_up(nw, 256); }
     else { mw = padded_dim(mw); nw = padded_dim(nw); }
     tiles = da_stage_tiles(m, n, mw, nw);
     esz = dtype == DA_BF16 ? 2 : 4;
@@ -290,6 +309,7 @@ bool ns_small_wanted(const NsJob* jobs, int nj, const NsCall& c) {
 int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStream_t s) {
   if (nj < 1 || nj > DA_MAX_GROUPS) return DA_ERR_ARG;
   const bool small = ns_small_wanted(jobs, nj, c);
+  const bool all256 = grid256(jobs, nj, [](const NsJob& k) { return k.cnt; });
   // carve the workspace: every job keeps all of its matrices resident
   NsSet sets[DA_MAX_GROUPS];
   char* p = static_cast<char*>(workspace);
@@ -297,7 +317,7 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStre
   for (int i = 0; i < nj; ++i) {
     const NsJob& k = jobs[i];
     NsSet& S = sets[i];
-    S.L = NsLayout(k.m, k.n, c.compute_dtype, small);
+    S.L = NsLayout(k.m, k.n, c.compute_dtype, small, all256);
     S.W = NsBuffers(S.L, p, k.cnt);
     S.cb = k.cnt;
     S.update = c.update; S.x_dtype = c.x_dtype; S.tall = k.m > k.n ? 1 : 0; S.x_ld = k.ldx; S.decay = k.decay; S.step = k.step;
@@ -788,9 +808,11 @@ size_t dion_amd_muon_buckets_workspace_bytes(const dion_amd_muon_bucket* buckets
   size_t worst = 0;
   for (int r0 = 0; r0 < nbuckets; r0 += DA_MAX_GROUPS) {
     size_t need = 0;
-    for (int i = r0; i < nbuckets && i < r0 + DA_MAX_GROUPS; ++i) {
+    const int nr = nbuckets - r0 < DA_MAX_GROUPS ? nbuckets - r0 : DA_MAX_GROUPS;
+    const bool all256 = grid256(buckets + r0, nr, [](const dion_amd_muon_bucket& k) { return k.batch; });
+    for (int i = r0; i < r0 + nr; ++i) {
       if (buckets[i].batch <= 0 || buckets[i].m <= 0 || buckets[i].n <= 0) return 0;
-      need += align_up(NsLayout(buckets[i].m, buckets[i].n, DA_BF16).per_matrix * (size_t)buckets[i].batch, 256);
+      need += align_up(NsLayout(buckets[i].m, buckets[i].n, DA_BF16, false, all256).per_matrix * (size_t)buckets[i].batch, 256);
     }
     if (need > worst) worst = need;
   }
