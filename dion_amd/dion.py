@@ -15,6 +15,7 @@ pass over M and X.
 """
 import math
 import os
+import threading
 from collections import defaultdict
 from concurrent.futures import ThreadPoolExecutor
 from concurrent.futures import wait as wait_futures
@@ -137,7 +138,6 @@ class Dion(Optimizer):
         # launches that cannot fill the GPU, so buckets overlap nearly for free.
         self._max_concurrent_tasks = 3
         self._workspaces = [_lib.Workspace() for _ in range(self._max_concurrent_tasks)]
-        self._streams = {}
         self._info = {}
         self._pool = None   # worker threads that enqueue the buckets of a wave side by side
         self._rng = None    # generator of the random sketches (DionReference with qr_method "rcqr")
@@ -316,10 +316,7 @@ class Dion(Optimizer):
                     if slots == 1:
                         stream = main
                     else:
-                        pool = self._streams.setdefault(device, [])
-                        while len(pool) < slots:
-                            pool.append(torch.cuda.Stream(device=device))
-                        stream = pool[slot]
+                        stream = _side_streams(device, slots)[slot]
                         if (device, slot) not in forked:
                             stream.wait_stream(main)   # gradients and earlier updates were produced on `main`
                             forked[(device, slot)] = (main, stream)
@@ -415,6 +412,21 @@ class Dion(Optimizer):
 
     def _adamw_group_step(self, group: dict):
         element_group_step(self, group, True)
+
+
+_side = threading.local()
+
+
+def _side_streams(device, count):
+    """The calling thread's side streams on `device`, at least `count` of them.
+
+    One set for all optimizers of a thread: the runtime deals streams to four hardware queues as they are created, and a
+    set that includes the queue of the main stream serialises the buckets (a step of two buckets of 3968 x 1792, rank 448,
+    with an embedding of 29747 x 1792 under Lion: 0.83 ms on the first optimizer's streams, 1.29 ms on the second one's)."""
+    streams = _side.__dict__.setdefault("streams", {}).setdefault(device, [])
+    while len(streams) < count:
+        streams.append(torch.cuda.Stream(device=device))
+    return streams
 
 
 def _sketch(p_shape, dtype, device, oversample, generator=None) -> Tensor:
