@@ -2,6 +2,8 @@
 // guard, dtype casts, the NaN / all-zero fix-up of P and R, the column normalisation that
 // turns R into the next Q, and the host-side driver of the orthonormalisation (one blocked
 // CholeskyQR pass in fp64: Gram -> Cholesky -> triangular solve, then closed-form polishing passes).
+#include "orth_flow.h"
+#include "ns_flow.h"
 #include "dion.h"
 #include "gemm_f64.h"
 #include "prof.h"
@@ -424,22 +426,30 @@ struct OrthWs {
   double* pstat;   // 2 per matrix: smallest and largest pivot of the fp64 factorisation
   int* polish;     // per matrix: 1 = the fp64 pass's result goes through the polishing pass
   int* direct;     // per matrix: 1 = it is the result as it is
+  double* defect;  // one-launch pass over flagged matrices: the columns' defects by 32-tiles
+  int* flow_ctl;   // ... and its control words
   size_t bytes;
   OrthWs(void* ws, int batch, int rows, int r) {
     const size_t pr = (size_t)rows * r * batch, rr = (size_t)r * r * batch;
+    // (padded to whole tiles for the one-launch pass over flagged matrices, which works in the same places)
+    const size_t rp = (size_t)((r + 63) / 64) * 64, pr64 = (size_t)((rows + 63) / 64) * 64 * rp * batch, rr64 = rp * rp * batch;
+    const size_t fsl = (size_t)da_orth_flow_slices(rows, r);
     const int sp = gram_slices(batch, rows, r);
     char* p = static_cast<char*>(ws);
     auto take = [&](size_t n) { char* q = p; p += orth_align(n); return q; };
-    P0 = reinterpret_cast<double*>(take(pr * 8));
+    P0 = reinterpret_cast<double*>(take(pr64 * 8));
     Pf = reinterpret_cast<float*>(take(pr * 4));
     Ph = reinterpret_cast<bf16_t*>(take(pr * 2));
-    G = reinterpret_cast<double*>(take(rr * 8));
-    L = reinterpret_cast<double*>(take(rr * 8));
-    W = reinterpret_cast<double*>(take(rr * 8));
+    G = reinterpret_cast<double*>(take(rr64 * 8));
+    L = reinterpret_cast<double*>(take(rr64 * 8));
+    W = reinterpret_cast<double*>(take(rr64 * 8));
     // K-slice outputs: `sp` slices of the fp64 / fp32 Gram kernels, or two fp32 slabs per slice of the bf16 one
     const size_t slabs16 = (size_t)2 * gram16_slices(batch, rows, r, 1, nullptr);   // (one product has the most slices)
     const size_t part_a = rr * 8 * (sp > 2 ? sp : 2), part_b = rr * 4 * slabs16;
-    part = reinterpret_cast<double*>(take(part_a > part_b ? part_a : part_b));
+    const size_t part_c = rr64 * 8 * fsl, part_ab = part_a > part_b ? part_a : part_b;
+    part = reinterpret_cast<double*>(take(part_ab > part_c ? part_ab : part_c));
+    defect = reinterpret_cast<double*>(take(rp * (rp / 32) * 8 * batch));
+    flow_ctl = reinterpret_cast<int*>(take(((size_t)batch + 9) * DA_ORTH_FLOW_CTL * 4));
     rowdef = reinterpret_cast<float*>(take((size_t)r * batch * 4));
     rowdef_part = reinterpret_cast<float*>(take((size_t)((r + 63) / 64) * r * batch * 4));
     need = reinterpret_cast<int*>(take((size_t)batch * 4));
@@ -1267,6 +1277,9 @@ int da_orthonormalize(const void* P, void* out, int dtype, int batch, int rows, 
     if (rc) return rc;
   }
   // ---- fp64 pass: on the flagged matrices, or on all of them
+  if (fast && da_orth_flow_applicable(batch, rows, r))   // (one launch, which as a rule finds none)
+    return da_orth_flow(P, out, dtype, batch, rows, r, r_live, w.need, info,
+                        DaOrthFlow{w.P0, w.part, w.L, w.W, w.G, w.defect, w.flow_ctl}, da_ns_flow_fail() ? 1 : 0, s);
   const DaGate gate = fast ? DaGate{w.need, 1} : all;
   rc = da_cvt_to_f64(P, dtype, w.P0, pr, batch, gate, s);
   if (rc) return rc;

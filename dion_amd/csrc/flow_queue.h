@@ -11,6 +11,16 @@ __host__ __device__ inline int ceil8(int x) { return (x + 7) >> 3; }   // x >= -
 // how many of the matrices first .. first + cnt - 1 (in dealing order) belong to queue q
 __host__ __device__ inline int da_in_queue(int first, int cnt, int q) { return ceil8(first + cnt - q) - ceil8(first - q); }
 
+// The kernel's arguments (its first and only parameter, of type A), opaque to the compiler: read again where they are used.  Hoisted
+// out of a persistent loop they take more scalar registers than there are, and are spilled.
+template <typename A>
+__device__ __forceinline__ const A& fresh_args() {
+  typedef const __attribute__((address_space(4))) A* ptr_t;
+  ptr_t p = (ptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const A*)p;
+}
+
 __device__ __forceinline__ int xcc_id() { return (int)(__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7u); }
 __device__ __forceinline__ unsigned long long now_ticks() { return __builtin_amdgcn_s_memrealtime(); }
 

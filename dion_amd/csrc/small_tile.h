@@ -1,0 +1,712 @@
+// Tile products and the serial part of a factorisation for the one-launch kernels (dion_small.hip, orth_flow.hip): 256 threads,
+// operands from memory through registers into LDS, products on the matrix cores in bf16, fp32 and fp64.
+#pragma once
+#include "gemm_f64.h"
+#include "mfma_tile.h"
+
+#pragma clang fp contract(off)
+
+namespace {
+
+constexpr int KD = 32;             // depth of an fp32 / fp64 stage
+constexpr int LP = 65;             // pitch of the factorisation's 64 x 64 tile
+constexpr int STAGES64 = 2 * 2 * KD * 66 * 8;   // two stages of two fp64 operands of 64 rows: the largest user of the LDS
+
+typedef double double2_t __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_un_t __attribute__((ext_vector_type(4), aligned(2)));   // an unaligned 16-byte access
+
+// ---- operands ----------------------------------------------------------------------------------------------------------
+
+// Element (row, k): p[row * ld + k], or p[k * ld + row] when `ks`.  EDGE: a caller's matrix of `rows` x `kmax`, of which
+// anything beyond reads as zero; `last` = its elements - 8.  Otherwise a working matrix, padded to whole tiles.
+template <typename E, bool EDGE> struct Opnd {
+  const E* p;
+  int ld, ks;
+  int rows, kmax;
+  long long last;
+};
+template <typename E> __device__ __forceinline__ Opnd<E, false> work(const void* p, int ld, int ks) {
+  return Opnd<E, false>{static_cast<const E*>(p), ld, ks, 0, 0, 0};
+}
+
+// Eight consecutive elements as they came from memory: converted only when they go to LDS, so that the loads of the next
+// stages stay in flight.
+template <typename E> struct Raw { u32x4_t q[sizeof(E) / 2]; };
+template <typename E> __device__ __forceinline__ Raw<E> load_raw(const E* p) {
+  Raw<E> r;
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(E) / 2); ++i) {
+    const u32x4_un_t x = *reinterpret_cast<const u32x4_un_t*>(reinterpret_cast<const char*>(p) + 16 * i);
+    r.q[i] = x;
+  }
+  return r;
+}
+template <typename T> __device__ __forceinline__ void unpack(const Raw<bf16_t>& r, T (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const unsigned w = r.q[0][i];
+    v[2 * i] = (T)lo_f(w);
+    v[2 * i + 1] = (T)hi_f(w);
+  }
+}
+template <typename T> __device__ __forceinline__ void unpack(const Raw<float>& r, T (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const unsigned w = r.q[i >> 2][i & 3];
+    v[i] = (T)__builtin_bit_cast(float, w);
+  }
+}
+__device__ __forceinline__ void unpack(const Raw<double>& r, double (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const unsigned lo = r.q[i >> 1][2 * (i & 1)], hi = r.q[i >> 1][2 * (i & 1) + 1];
+    v[i] = __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+  }
+}
+__device__ __forceinline__ float to_f(bf16_t x) { return bf2f(x); }
+__device__ __forceinline__ float to_f(float x) { return x; }
+
+// Eight elements from element offset `e`, of which n exist; the rest reads as zero.
+template <typename E> __device__ __forceinline__ void load8(const E* p, long long e, int n, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = 0.f;
+  if (n >= 8) {
+    unpack(load_raw(p + e), v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < n) v[i] = to_f(p[e + i]);
+  }
+}
+
+// Chunk c (eight elements) of a TB x depth-D tile: its (row, k) in the tile
+template <int TB, int D>
+__device__ __forceinline__ void chunk_at(int ks, int c, int& row, int& k) {
+  row = ks ? (c % (TB / 8)) * 8 : c / (D / 8);
+  k = ks ? c / (TB / 8) : (c % (D / 8)) * 8;
+}
+template <int TB, int D, typename E, bool EDGE>
+__device__ __forceinline__ Raw<E> fetch_chunk(const Opnd<E, EDGE>& o, int c, int row0, int k0) {
+  int row, k;
+  chunk_at<TB, D>(o.ks, c, row, k);
+  row += row0;
+  k += k0;
+  long long e = o.ks ? (long long)k * o.ld + row : (long long)row * o.ld + k;
+  if (EDGE) e = e < o.last ? e : o.last;   // (inside the matrix whatever the chunk)
+  return load_raw(o.p + e);
+}
+// what of a fetched chunk lies inside a caller's matrix; the rest becomes zero
+template <int TB, int D, typename E>
+__device__ __forceinline__ void mask_chunk(const Opnd<E, true>& o, Raw<E>& r, int c, int row0, int k0) {
+  int row, k;
+  chunk_at<TB, D>(o.ks, c, row, k);
+  row += row0;
+  k += k0;
+  const int n = o.ks ? (k < o.kmax ? o.rows - row : 0) : (row < o.rows ? o.kmax - k : 0);
+  if (n >= 8) return;
+  const long long e = o.ks ? (long long)k * o.ld + row : (long long)row * o.ld + k;
+  if (n > 0 && e > o.last) {   // the matrix's last elements: the load was moved back
+    constexpr int W = 4 / sizeof(E);   // elements per word
+#pragma unroll
+    for (int i = 0; i < 8 / W; ++i) {
+      unsigned w = 0;
+      if (i * W < n) w = sizeof(E) == 4 ? reinterpret_cast<const unsigned*>(o.p + e)[i] : (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i];
+      if (sizeof(E) == 2 && i * W + 1 < n) w |= (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i + 1] << 16;
+      r.q[i >> 2][i & 3] = w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(E) * 2; ++i) {
+      const unsigned w = r.q[i >> 2][i & 3];
+      r.q[i >> 2][i & 3] = sizeof(E) == 4 ? (i < n ? w : 0u) : (2 * i + 1 < n ? w : 2 * i < n ? w & 0xffffu : 0u);
+    }
+  }
+}
+
+// ---- products of fp32 / fp64 tiles: LDS stages [k][row] with a pitch of TB + 2 (fp64) or TB + 4 (fp32) -------------------
+template <typename T, int TB>
+struct Real {
+  static constexpr int P = TB + (sizeof(T) == 8 ? 2 : 4);
+  static constexpr int OPND = KD * P;              // elements of one operand's stage
+  static constexpr int NCH = TB * KD / 8;          // chunks per operand stage (at most one per thread)
+};
+
+struct NoTurn {
+  template <typename V> __device__ __forceinline__ void operator()(V&, int, int) const {}
+};
+template <typename T, int TB, typename E, bool EDGE, typename Turn>
+__device__ __forceinline__ void put_chunk(T* dst, const Opnd<E, EDGE>& o, Raw<E>& r, int c, int row0, int k0, Turn turn) {
+  constexpr int P = Real<T, TB>::P;
+  T v[8];
+  if constexpr (EDGE) mask_chunk<TB, KD>(o, r, c, row0, k0);
+  unpack(r, v);
+  int row, k;
+  chunk_at<TB, KD>(o.ks, c, row, k);
+  turn(v, row0 + row, k0 + k);
+  if (o.ks) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[k * P + row + i] = v[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dst[(k + i) * P + row] = v[i];
+  }
+}
+
+// K loop of one TB x TB tile:  sum over k in [kbeg, kend) of A(row0 + i, k) B(col0 + j, k), for NB column operands; `mma`
+// accumulates one stage of KD from the operands' LDS buffers (A first); `turn(v, col, k)` maps the chunk (col, k ..) of a column
+// operand on its way to LDS.  Two stages are on the way from memory while a third
+// is multiplied; of fp64 64-tiles one (its products take 1.7 us and two stages too many registers).
+template <typename T, int TB, int NB, typename OA, typename OB, typename Mma, typename Turn>
+__device__ __forceinline__ void real_loop(const OA& A, const OB (&B)[NB], int row0, int col0, int kbeg, int kend, T* lds, int tid,
+                                          Mma mma, Turn turn) {
+  typedef Real<T, TB> L;
+  constexpr int STG = (1 + NB) * L::OPND;
+  const int c = tid & (L::NCH - 1);
+  const bool own = tid < L::NCH;
+  decltype(fetch_chunk<TB, KD>(A, c, row0, kbeg)) va[2];
+  decltype(fetch_chunk<TB, KD>(B[0], c, col0, kbeg)) vb[2][NB];
+  auto fetch = [&](int s, int k0) {
+    va[s] = fetch_chunk<TB, KD>(A, c, row0, k0);
+#pragma unroll
+    for (int o = 0; o < NB; ++o) vb[s][o] = fetch_chunk<TB, KD>(B[o], c, col0, k0);
+  };
+  auto put = [&](int s, int k0) {
+    if (own) {
+      put_chunk<T, TB>(lds + s * STG, A, va[s], c, row0, k0, NoTurn());
+#pragma unroll
+      for (int o = 0; o < NB; ++o) put_chunk<T, TB>(lds + s * STG + (1 + o) * L::OPND, B[o], vb[s][o], c, col0, k0, turn);
+    }
+  };
+  constexpr int AHEAD = sizeof(T) == 8 && TB == 64 ? 1 : 2;
+  fetch(0, kbeg);
+  if (AHEAD == 2 && kbeg + KD < kend) fetch(1, kbeg + KD);
+  put(0, kbeg);
+  for (int k0 = kbeg; k0 < kend; k0 += 2 * KD) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = k0 + s * KD;
+      if (k >= kend) break;
+      if (k + AHEAD * KD < kend) fetch(AHEAD == 2 ? s : s ^ 1, k + AHEAD * KD);
+      __syncthreads();
+      mma(lds + s * STG);
+      if (k + KD < kend) put(s ^ 1, k + KD);
+    }
+  }
+  __syncthreads();
+}
+
+// fp64 (and fp32 in 32-tiles): v_mfma_*_16x16x4, four wavefronts of TB/2 x TB/2
+template <typename T, int TB>
+struct Acc16 {
+  static constexpr int NBK = TB / 32, P = Real<T, TB>::P, H = TB / 2;
+  typename Mfma<T>::acc_t acc[NBK][NBK];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < NBK; ++i)
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) acc[i][j] = typename Mfma<T>::acc_t{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void stage(const T* sa, const T* sb, int lane, int wm, int wn) {
+#pragma unroll
+    for (int ks = 0; ks < KD / 4; ++ks) {
+      const int k = ks * 4 + (lane >> 4);
+      T af[NBK], bf[NBK];
+#pragma unroll
+      for (int i = 0; i < NBK; ++i) af[i] = sa[k * P + wm * H + i * 16 + (lane & 15)];
+#pragma unroll
+      for (int j = 0; j < NBK; ++j) bf[j] = sb[k * P + wn * H + j * 16 + (lane & 15)];
+#pragma unroll
+      for (int i = 0; i < NBK; ++i)
+#pragma unroll
+        for (int j = 0; j < NBK; ++j) acc[i][j] = Mfma<T>::mma(af[i], bf[j], acc[i][j]);
+    }
+  }
+  // to the staging area d[row][col], pitch TB + 2; ends with a barrier
+  __device__ __forceinline__ void out(T* d, int lane, int wm, int wn) const {
+#pragma unroll
+    for (int i = 0; i < NBK; ++i)
+#pragma unroll
+      for (int j = 0; j < NBK; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          d[(wm * H + i * 16 + Mfma<T>::row(v, lane)) * (TB + 2) + wn * H + j * 16 + (lane & 15)] = acc[i][j][v];
+    __syncthreads();
+  }
+};
+template <typename T, int TB, typename OA, typename OB, typename Turn = NoTurn>
+__device__ __forceinline__ void tile16(const OA& A, const OB& B, int row0, int col0, int kbeg, int kend, T* lds, int tid, int lane,
+                                       int wm, int wn, Turn turn = Turn()) {
+  Acc16<T, TB> acc;
+  acc.clear();
+  const OB Bs[1] = {B};
+  real_loop<T, TB, 1>(A, Bs, row0, col0, kbeg, kend, lds, tid,
+                      [&](const T* st) { acc.stage(st, st + Real<T, TB>::OPND, lane, wm, wn); }, turn);
+  acc.out(lds, lane, wm, wn);
+}
+
+// fp32, 64-tiles: one v_mfma_f32_32x32x2 block per wavefront (the order of k of gemm_f32.hip); element e of `acc` is row
+// (lane & 31), column 8 (e / 4) + 4 (lane / 32) + e % 4 of the wavefront's block.  NB column operands share the row operand.
+template <int NB, typename OA, typename OB>
+__device__ __forceinline__ void tile32x2(const OA& A, const OB (&B)[NB], int row0, int col0, int kend, float* lds, int tid, int lane,
+                                         int wm, int wn, f32x16_t (&acc)[NB]) {
+  constexpr int P = Real<float, 64>::P, OPND = Real<float, 64>::OPND;
+#pragma unroll
+  for (int o = 0; o < NB; ++o)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[o][v] = 0.f;
+  real_loop<float, 64, NB>(A, B, row0, col0, 0, kend, lds, tid, [&](const float* st) {
+#pragma unroll
+    for (int ks = 0; ks < KD / 2; ++ks) {
+      const int k = ks * 2 + (lane >> 5);
+      const float fa = st[k * P + wm * 32 + (lane & 31)];
+#pragma unroll
+      for (int o = 0; o < NB; ++o)
+        acc[o] = __builtin_amdgcn_mfma_f32_32x32x2f32(st[(1 + o) * OPND + k * P + wn * 32 + (lane & 31)], fa, acc[o], 0, 0, 0);
+    }
+  }, NoTurn());
+}
+__device__ __forceinline__ void stage_f32(const f32x16_t& acc, float* stg, int lane, int wm, int wn) {
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    stg[(wm * 32 + (lane & 31)) * 66 + wn * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)] = acc[v];
+}
+
+// ---- products of bf16 tiles: the LDS layouts of gemm_bf16_tile.h, 64-deep stages through registers -----------------------
+// `acc` is called with every stage: the buffers of the row operand and of NB column operands, 8 KB each.
+template <int TB, int D, bool EDGE>
+__device__ __forceinline__ void put_bf16(char* dst, const Opnd<bf16_t, EDGE>& o, Raw<bf16_t>& r, int c, int row0, int k0) {
+  if constexpr (EDGE) mask_chunk<TB, D>(o, r, c, row0, k0);
+  const int q = c >> 3, ch = c & 7;   // (row or k, chunk): 8 chunks of a line either way
+  *reinterpret_cast<u32x4_t*>(dst + q * 128 + (o.ks ? ks_swizzle(ch, q) : kc_swizzle(ch, q)) * 16) = r.q[0];
+}
+template <int NB, bool EDGE, typename Acc>
+__device__ __forceinline__ void tile_bf16(const Opnd<bf16_t, EDGE>& A, const Opnd<bf16_t, false> (&B)[NB], int row0, int col0, int kend,
+                                          char* lds, int tid, Acc acc) {
+  constexpr int OPND = 64 * 64 * 2;
+  constexpr int STG = (1 + NB) * OPND;
+  Raw<bf16_t> v[2][1 + NB][2];   // two stages on the way while a third is multiplied
+  auto fetch = [&](int s2, int k0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v[s2][0][h] = fetch_chunk<64, 64>(A, tid + 256 * h, row0, k0);
+#pragma unroll
+      for (int o = 0; o < NB; ++o) v[s2][1 + o][h] = fetch_chunk<64, 64>(B[o], tid + 256 * h, col0, k0);
+    }
+  };
+  auto put = [&](int s2, int k0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      put_bf16<64, 64>(lds + s2 * STG, A, v[s2][0][h], tid + 256 * h, row0, k0);
+#pragma unroll
+      for (int o = 0; o < NB; ++o) put_bf16<64, 64>(lds + s2 * STG + (1 + o) * OPND, B[o], v[s2][1 + o][h], tid + 256 * h, col0, k0);
+    }
+  };
+  fetch(0, 0);
+  if (64 < kend) fetch(1, 64);
+  put(0, 0);
+  for (int k0 = 0; k0 < kend; k0 += 128) {
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      const int k = k0 + s2 * 64;
+      if (k >= kend) break;
+      if (k + 128 < kend) fetch(s2, k + 128);
+      __syncthreads();
+      acc(lds + s2 * STG);
+      if (k + 64 < kend) put(s2 ^ 1, k + 64);
+    }
+  }
+  __syncthreads();
+}
+// P and R: v_mfma_f32_16x16x32_bf16, four 16 x 16 blocks per wavefront, to the staging area (pitch 66)
+template <bool EDGE>
+__device__ __forceinline__ void product_bf16(const Opnd<bf16_t, EDGE>& A, const Opnd<bf16_t, false>& B, int row0, int col0, int kend,
+                                             char* lds, int tid, int lane, int wm, int wn, float* stg) {
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const Opnd<bf16_t, false> Bs[1] = {B};
+  tile_bf16<1>(A, Bs, row0, col0, kend, lds, tid, [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8_t fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        fa[i] = A.ks ? read_frag16<64, true>(st, wm * 32 + i * 16, ks, lane) : read_frag16<64, false>(st, wm * 32 + i * 16, ks, lane);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) fb[j] = read_frag16<64, true>(st + 8192, wn * 32 + j * 16, ks, lane);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    }
+  });
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        stg[(wm * 32 + i * 16 + (lane & 15)) * 66 + wn * 32 + j * 16 + (lane >> 4) * 4 + v] = acc[i][j][v];
+}
+// the updates: v_mfma_f32_32x32x16_bf16 as in the batched update kernel, both products at once
+__device__ __forceinline__ void update_bf16(const Opnd<bf16_t, false>& A, const Opnd<bf16_t, false> (&B)[2], int row0, int col0,
+                                            int kend, char* lds, int tid, int lane, int wm, int wn, f32x16_t (&acc)[2]) {
+#pragma unroll
+  for (int o = 0; o < 2; ++o)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[o][v] = 0.f;
+  tile_bf16<2>(A, B, row0, col0, kend, lds, tid, [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8_t fa = read_frag<64, false>(st, wm * 32, ks, lane);
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+        acc[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_frag<64, false>(st + (1 + o) * 8192, wn * 32, ks, lane), fa, acc[o], 0, 0, 0);
+    }
+  });
+}
+
+// ---- stores ------------------------------------------------------------------------------------------------------------
+
+// eight values at element offset e of a matrix of dtype f32 / bf16, n of them
+__device__ __forceinline__ void store8(char* p, int f32, long long e, int n, const float (&v)[8]) {
+  if (n <= 0) return;
+  if (f32) {
+    float* q = reinterpret_cast<float*>(p) + e;
+    if (n >= 8) {
+      u32x4_un_t x, y;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = __builtin_bit_cast(unsigned, v[i]);
+        y[i] = __builtin_bit_cast(unsigned, v[4 + i]);
+      }
+      *reinterpret_cast<u32x4_un_t*>(q) = x;
+      *reinterpret_cast<u32x4_un_t*>(q + 4) = y;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < n) q[i] = v[i];
+    }
+  } else {
+    bf16_t* q = reinterpret_cast<bf16_t*>(p) + e;
+    if (n >= 8) {
+      u32x4_un_t x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = cvt_pk_bf16(v[2 * i], v[2 * i + 1]);
+      *reinterpret_cast<u32x4_un_t*>(q) = x;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < n) q[i] = f2bf(v[i]);
+    }
+  }
+}
+
+// nan_to_num of the dtype; 0 for an all-zero B (reference dion/dion.py:1416-1444)
+template <bool BF>
+__device__ __forceinline__ float guard(float x, bool nonzero, float alt) {
+  const float top = BF ? 3.3895313892515355e38f : 3.4028234663852886e38f;
+  if (BF) x = rbf(x);
+  if (x != x) x = 0.f;
+  else if (x > top) x = top;
+  else if (x < -top) x = -top;
+  return nonzero ? x : alt;
+}
+
+// ---- the serial part of the factorisation: a 64 x 64 diagonal block and its inverse (scheme of cholesky.hip) --------------
+// g: the block (lower triangle), pitch ld, in LDS, from `lds` on or anywhere.  dT receives the inverse factor, transposed (dT[k][x] = D[x][k], pitch LP).
+// A pivot that is not positive zeroes its column and is counted in `bad` (o + column + 1, the first one); `live`: columns
+// of the block that belong to the matrix (the others are identity and leave the pivot range alone).
+struct Quad { double v[4]; };
+__device__ __forceinline__ void diag_factor(const double* g, int ld, char* lds, double* dT, int live, int o, int tid, int lane,
+                                            int wave, int& bad, double& pmin, double& pmax) {
+#pragma clang fp contract(fast)
+  typedef Mfma<double>::acc_t acc_t;
+  double(*scol)[4][64] = reinterpret_cast<double(*)[4][64]>(lds);   // [2]: published block column of S
+  Quad(*yrow)[64] = reinterpret_cast<Quad(*)[64]>(lds + 4096);      // [2]: published row block of Y
+  Quad(*lops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 8192);      // [2]: L block column as MFMA operand
+  Quad(*xops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 12288);     // [2]: X
+  const int lc = lane & 15, lg = lane >> 4;
+  acc_t S[4], Y[4];
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = wave * 16 + Mfma<double>::row(v, lane), j = tj * 16 + lc;
+      S[tj][v] = tj <= wave ? (i >= j ? g[(long long)i * ld + j] : g[(long long)j * ld + i]) : 0.0;
+      Y[tj][v] = i == j ? 1.0 : 0.0;
+    }
+  __syncthreads();   // (the block may lie where the published ones go)
+  if (tid < 128) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) yrow[tid >> 6][tid & 63].v[k] = 0.0;
+  }
+  __syncthreads();
+  auto publish = [&](int q, int buf) {
+    const int tq = q >> 2, qq = q & 3;
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {
+      if (tj == tq && tj <= wave && (lc >> 2) == qq) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) scol[buf][lc & 3][wave * 16 + Mfma<double>::row(v, lane)] = S[tj][v];
+      }
+      if (wave == tq && tj <= wave) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int rr = Mfma<double>::row(v, lane);
+          if ((rr >> 2) == qq) yrow[buf][tj * 16 + lc].v[rr & 3] = Y[tj][v];
+        }
+      }
+    }
+  };
+  publish(0, 0);
+  __syncthreads();
+  for (int cb = 0; cb < 16; ++cb) {
+    const int buf = cb & 1, k0 = cb * 4;
+    double sv[4], a[4][4], di[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sv[k] = scol[buf][k][lane];
+    const Quad yv = yrow[buf][lane];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) a[ii][jj] = scol[buf][jj][k0 + ii];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const double p = a[c][c];
+      const bool ok = __builtin_amdgcn_class(p, 0x100);   // positive normal
+      double rs = ok ? __builtin_amdgcn_rsq(p) : 0.0;     // 2^-27: one step of third order
+      const double err = 1.0 - p * rs * rs;
+      rs = rs + rs * err * (0.5 + 0.375 * err);
+      di[c] = ok ? rs : 0.0;
+      bad = (!ok && bad == 0 && k0 + c < live) ? o + k0 + c + 1 : bad;
+      if (ok && k0 + c < live) {
+        pmin = p < pmin ? p : pmin;
+        pmax = p > pmax ? p : pmax;
+      }
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i) a[i][c] *= di[c];
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i)
+#pragma unroll
+        for (int j = c + 1; j <= i; ++j) a[i][j] -= a[i][c] * a[j][c];
+    }
+    double l[4], x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double tl = sv[k], tx = yv.v[k];
+#pragma unroll
+      for (int m = 0; m < k; ++m) {
+        tl -= l[m] * a[k][m];
+        tx -= a[k][m] * x[m];
+      }
+      l[k] = tl * di[k];
+      x[k] = tx * di[k];
+    }
+    Quad lo, xo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      lo.v[k] = lane > k0 + 3 ? l[k] : 0.0;
+      xo.v[k] = lane <= k0 + k ? x[k] : 0.0;
+    }
+    lops[buf][lane] = lo;
+    xops[buf][lane] = xo;
+    if (wave == (cb & 3)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dT[lane * LP + k0 + k] = xo.v[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (wave * 16 + 15 > k0 + 3) {
+      const double aop = -lops[buf][wave * 16 + lc].v[lg];
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        if (tj <= wave && tj * 16 + 15 > k0 + 3) S[tj] = Mfma<double>::mma(aop, lops[buf][tj * 16 + lc].v[lg], S[tj]);
+        if (tj <= wave && tj * 16 <= k0 + 3) Y[tj] = Mfma<double>::mma(aop, xops[buf][tj * 16 + lc].v[lg], Y[tj]);
+      }
+    }
+    if (cb + 1 < 16) publish(cb + 1, buf ^ 1);
+    __syncthreads();
+  }
+}
+
+// ---- the blocked fp64 Cholesky factorisation  P^T P = L L^T,  T = L^-1  in blocks of 64, as tasks -------------------------
+// P^T P comes as lower 32 x 32 tiles in K slices (slab: [slices][rp][rp], rp = 64 rT); columns r .. rp - 1 are the identity.
+struct Factor {
+  const double* slab;
+  double *L, *T;               // rp x rp; of L the blocks below the diagonal, of T those on and below it
+  int slices, r, rp, rT;
+  int *bad, *sick, *info;      // first failed pivot (column + 1); outcome: pivot range below `ratio` or a failed pivot; info may be null
+  double* range;               // smallest and largest pivot so far
+  double ratio;
+};
+// Left-looking.  `diag`: block (j, j) -- the slabs added in order, less the products of the earlier columns -- is factored and
+// the factor inverted.  Otherwise task 0 .. rT - 2: a block of column j of L below the diagonal or of block row j of T.
+__device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, int task, char* lds, int tid, int lane, int wave, int wm,
+                                            int wn) {
+  typedef Real<double, 64> RD;
+  enum Job { J_DIAG, J_LOW, J_INV };
+  double* const d = reinterpret_cast<double*>(lds);
+  double *const L = F.L, *const T = F.T;
+  const int rp = F.rp, rT = F.rT;
+  const long long rr = (long long)rp * rp;
+  const Job job = diag ? J_DIAG : task < rT - 1 - j ? J_LOW : J_INV;
+  const int x = diag ? j : job == J_LOW ? j + 1 + task : task - (rT - 1 - j);
+  const int kend = wave_uniform((job == J_INV ? j - x : j) * 64);
+  // J_INV: sum over k of L(j, k) T(k, x), x <= k < j;  else: sum over k < j of L(x, k) L(j, k)^T
+  const Opnd<double, false> sa = work<double>(job == J_INV ? L + (long long)j * 64 * rp + x * 64 : L + (long long)x * 64 * rp, rp, 0);
+  const Opnd<double, false> sb = job == J_INV ? work<double>(T + (long long)x * 64 * rp + x * 64, rp, 1)
+                                              : work<double>(L + (long long)j * 64 * rp, rp, 0);
+  const Opnd<double, false> sd = work<double>(T + (long long)j * 64 * rp + j * 64, rp, 0);   // D, the inverse of the diagonal block's factor
+  if (kend > 0) tile16<double, 64>(sa, sb, 0, 0, 0, kend, d, tid, lane, wm, wn);
+  double2_t w[8];        // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
+  const int k = (tid & 31) * 2, i0 = tid >> 5;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) w[u] = double2_t{0.0, 0.0};
+  if (job != J_INV) {
+    // the slabs of P^T P in slice order; beyond the rank the matrix is the identity
+    const double* const slab = F.slab + (long long)(x * 64 + i0) * rp + j * 64 + k;
+    for (int s = 0; s < F.slices; ++s) {
+      double2_t y[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) y[u] = *reinterpret_cast<const double2_t*>(slab + s * rr + (long long)u * 8 * rp);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[u] += y[u];
+    }
+    const int lim = ((F.r + 31) >> 5) << 5;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int gi = x * 64 + i0 + 8 * u, gk = j * 64 + k;
+      if (gi >= F.r || gk >= lim || (gk >> 5) > (gi >> 5)) {   // (not written by GRAM)
+        w[u][0] = gi >= F.r && gi == gk ? 1.0 : 0.0;
+        w[u][1] = gi >= F.r && gi == gk + 1 ? 1.0 : 0.0;
+      }
+    }
+  }
+  if (kend > 0) {
+    const double sign = job == J_INV ? 1.0 : -1.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      w[u][0] += sign * d[(i0 + 8 * u) * 66 + k];
+      w[u][1] += sign * d[(i0 + 8 * u) * 66 + k + 1];
+    }
+  }
+  if (job == J_DIAG) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      d[(i0 + 8 * u) * 66 + k] = w[u][0];
+      d[(i0 + 8 * u) * 66 + k + 1] = w[u][1];
+    }
+    __syncthreads();
+    int bad = 0;
+    double pmin = 3e38, pmax = 0.0;
+    double* const range = F.range;
+    if (j > 0) {
+      bad = __hip_atomic_load(F.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      pmin = __hip_atomic_load(range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      pmax = __hip_atomic_load(range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    double* const dT = d + 2048;   // behind the 16 KB of the published blocks
+    diag_factor(d, 66, lds, dT, min(64, F.r - j * 64), j * 64, tid, lane, wave, bad, pmin, pmax);
+    double* const Dw = T + (long long)j * 64 * rp + j * 64;
+    for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * LP + (e >> 6)];
+    if (tid == 0) {
+      __hip_atomic_store(F.bad, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (j == rT - 1) {
+        const bool healthy = bad == 0 && pmin >= F.ratio * pmax && pmax > 0.0;
+        __hip_atomic_store(F.sick, healthy ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (F.info) *F.info = bad;
+      }
+    }
+    return;
+  }
+  // second product, both operands to the LDS stages:  L(x, j) = W(x, j) D^T;   T(j, x) = -D W(j, x)
+  Raw<double> dr[2];
+  dr[0] = fetch_chunk<64, KD>(sd, tid, 0, 0);
+  dr[1] = fetch_chunk<64, KD>(sd, tid, 0, KD);
+  __syncthreads();
+  double* const wst = d + (job == J_INV ? RD::OPND : 0);
+  double* const dst = d + (job == J_INV ? 0 : RD::OPND);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int i = i0 + 8 * u;
+    if (job == J_INV) {
+      wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k] = w[u][0];
+      wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k + 1] = w[u][1];
+    } else {
+      wst[(k >> 5) * 2 * RD::OPND + (k & 31) * RD::P + i] = w[u][0];
+      wst[(k >> 5) * 2 * RD::OPND + ((k + 1) & 31) * RD::P + i] = w[u][1];
+    }
+  }
+  put_chunk<double, 64>(dst, sd, dr[0], tid, 0, 0, NoTurn());
+  put_chunk<double, 64>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
+  __syncthreads();
+  Acc16<double, 64> acc;
+  acc.clear();
+  acc.stage(d, d + RD::OPND, lane, wm, wn);
+  acc.stage(d + 2 * RD::OPND, d + 3 * RD::OPND, lane, wm, wn);
+  __syncthreads();
+  acc.out(d, lane, wm, wn);
+  double* const out = job == J_INV ? T + (long long)j * 64 * rp + x * 64 : L + (long long)x * 64 * rp + j * 64;
+  const double sign = job == J_INV ? -1.0 : 1.0;
+  for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e >> 6) * 66 + (e & 63)];
+}
+
+// One lower 32 x 32 tile (number t of t32 (t32 + 1) / 2) of S^T S over rows [kbeg, kend) of S, into out (pitch rp) and d (pitch 34)
+template <typename OP>
+__device__ __forceinline__ void gram_tile(const OP& S, int t, int kbeg, int kend, double* out, int rp, double* d, int tid, int lane, int wm,
+                                          int wn, int& ti, int& tj) {
+  int i = 0;
+  while (t > i) { t -= i + 1; ++i; }
+  ti = wave_uniform(i);
+  tj = wave_uniform(t);
+  tile16<double, 32>(S, S, ti * 32, tj * 32, kbeg, kend, d, tid, lane, wm, wn);
+  for (int e = tid; e < 1024; e += 256) out[(long long)(ti * 32 + (e >> 5)) * rp + tj * 32 + (e & 31)] = d[(e >> 5) * 34 + (e & 31)];
+}
+// the tile's share of || column of S^T S - I ||^2, by rows and (symmetric) by columns: defect[column][32-tile]
+__device__ __forceinline__ void gram_defect(const double* d, double* defect, int pitch, int ti, int tj, int tid) {
+  if (tid >= 64) return;
+  const int i = tid & 31;
+  double s = 0.0;
+  for (int k = 0; k < 32; ++k) {
+    const double v = (tid < 32 ? d[i * 34 + k] : d[k * 34 + i]) - (ti == tj && i == k ? 1.0 : 0.0);
+    s += v * v;
+  }
+  const int c = (tid < 32 ? ti : tj) * 32 + i, t = tid < 32 ? tj : ti;
+  if (tid < 32 || ti != tj) defect[(long long)c * pitch + t] = s;
+}
+// drop[c]: column c came from a noise-level pivot (columns 0 .. rp - 1)
+__device__ __forceinline__ void find_dropped(const double* defect, int pitch, int r, int rp, unsigned char* drop, int tid) {
+  for (int c = tid; c < rp; c += 256) {
+    double s = 0.0;
+    if (c < r)
+      for (int t = 0; t < ((r + 31) >> 5); ++t) s += defect[(long long)c * pitch + t];
+    drop[c] = !(s <= 0.25) ? 1 : 0;
+  }
+  __syncthreads();
+}
+// A 64 x 64 tile of S V into d, V = I - up(S^T S - I) without the dropped columns; V^T is formed from the lower tiles of S^T S
+// on the way to LDS
+__device__ __forceinline__ void polish_tile(const double* S, const double* gram, int r, int rp, const unsigned char* drop, int row0, int col0,
+                                            double* d, int tid, int lane, int wm, int wn) {
+  tile16<double, 64>(work<double>(S, rp, 0), work<double>(gram, rp, 0), row0, col0, 0, col0 + 64, d, tid, lane, wm, wn,
+                     [&](double (&v)[8], int c, int k) {
+    const bool gone = drop[c] != 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const double y = v[i];
+      const bool on = k + i == c;
+      double u = k + i < c ? -y : (on ? 1.5 - 0.5 * y : 0.0);
+      if (c >= r) u = on ? 1.0 : 0.0;                 // beyond the rank: the identity
+      if (gone) u = 0.0;                              // a dropped column comes out as zero
+      else if (drop[k + i]) u = on ? 1.0 : 0.0;       // and gives no correction
+      v[i] = u;
+    }
+  });
+}
+
+}  // namespace
