@@ -1277,7 +1277,7 @@ int da_orthonormalize(const void* P, void* out, int dtype, int batch, int rows, 
     if (rc) return rc;
   }
   // ---- fp64 pass: on the flagged matrices, or on all of them
-  if (fast && da_orth_flow_applicable(batch, rows, r))   // (one launch, which as a rule finds none)
+  if (fast && da_orth_flow_applicable(rows, r))   // (one launch, which as a rule finds none)
     return da_orth_flow(P, out, dtype, batch, rows, r, r_live, w.need, info,
                         DaOrthFlow{w.P0, w.part, w.L, w.W, w.G, w.defect, w.flow_ctl}, da_ns_flow_fail() ? 1 : 0, s);
   const DaGate gate = fast ? DaGate{w.need, 1} : all;

@@ -12,7 +12,7 @@ struct DaOrthFlow {
 };
 int da_orth_flow_slices(int rows, int r);
 // Whether the launch takes factors of these dimensions and is the better one for them.
-bool da_orth_flow_applicable(int batch, int rows, int r);
+bool da_orth_flow_applicable(int rows, int r);
 // out[b] <- orth(P[b]) for the matrices with need[b] != 0 (out may be P); info[b] as da_orthonormalize.
 int da_orth_flow(const void* P, void* out, int dtype, int batch, int rows, int r, int r_live, const int* need, int* info,
                  const DaOrthFlow& w, int fail, hipStream_t s);

@@ -3,14 +3,14 @@
 //
 // What bounds it: nothing, as a rule -- no matrix is flagged and the launch returns at once (5 us).  As a launch per product the
 // same took 28 to 60 launches that each found out for themselves that there is nothing to do: 75 us of a bucket of rank 192,
-// 250 us of one of rank 512, and the host's time to issue them.  For a flagged matrix it is the scheme of dion_small.hip: tasks
+// and the host's time to issue them (72 bf16 matrices, rank 192: a step 835 -> 727 us).  For a flagged matrix it is the scheme of dion_small.hip: tasks
 // from eight queues, one per XCD (flow_queue.h), a matrix stays with one XCD, counters say when a phase may start:
 //   GRAM   P^T P in fp64, lower 32 x 32 tiles, K slices as slabs of their own
 //   DIAGj, LOWj   blocked Cholesky factor and its inverse, left-looking (factor_task)
 //   PT     S = P L^-T in fp64
 //   FIX    the closed form of a second pass: S^T S, columns from noise-level pivots dropped, out = S (I - up(S^T S - I))
-// A flagged matrix keeps one XCD busy: large ones with few others beside them are left to the launches per product, which
-// spread over the chip (da_orth_flow_applicable).
+// A flagged matrix keeps one XCD busy: large ones are left to the launches per product, which spread over the chip
+// (da_orth_flow_applicable).
 #include "orth_flow.h"
 #include "flow_queue.h"
 #include "small_tile.h"
@@ -211,15 +211,16 @@ int da_orth_flow_slices(int rows, int r) {
   return (rows + kslice - 1) / kslice;
 }
 
-// One XCD does 5 to 6 TFLOP/s of fp64: a flagged matrix of 3072 x 768 takes about 1.5 ms on it.  Beyond that, with fewer matrices
-// than XCDs, the launches per product (which use the whole chip) keep the rare case bounded.
-bool da_orth_flow_applicable(int batch, int rows, int r) {
-  return (r + 63) / 64 <= MAX_RT && (long long)rows * r >= 8 && (batch >= DA_QUEUES || (double)rows * r * r <= 2.2e9);
+// Where the line lies: a flagged matrix has one XCD to itself at best, the launches per product the whole chip.  A full-rank
+// factor of a fresh Q is flagged (12 of 3072 x 768 each in two buckets: 13.4 ms a step in one launch, 7.4 ms in many), so the
+// work per matrix is kept to what one XCD does in about half a millisecond.
+bool da_orth_flow_applicable(int rows, int r) {
+  return (r + 63) / 64 <= MAX_RT && (long long)rows * r >= 8 && (double)rows * r * r <= 4e8;
 }
 
 int da_orth_flow(const void* P, void* out, int dtype, int batch, int rows, int r, int r_live, const int* need, int* info,
                  const DaOrthFlow& w, int fail, hipStream_t s) {
-  if (!da_orth_flow_applicable(batch, rows, r)) return DA_ERR_LIMIT;
+  if (!da_orth_flow_applicable(rows, r)) return DA_ERR_LIMIT;
   static DaOncePerDevice configured;
   int rc = configured.run([&]() -> int {
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(orth_flow_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));

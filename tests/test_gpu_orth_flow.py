@@ -21,7 +21,7 @@ def _factors(batch, rows, r, cond):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("batch,rows,r", [(1, 300, 27), (4, 512, 64), (10, 1001, 65), (3, 1100, 200), (17, 264, 33), (2, 2100, 520)])
+@pytest.mark.parametrize("batch,rows,r", [(1, 300, 27), (4, 512, 64), (10, 1001, 65), (3, 1100, 200), (17, 264, 33), (2, 1500, 260)])
 def test_flagged_factors_match_householder(dev, dtype, batch, rows, r):
     from dion_amd import _lib
     from dion_amd.newton_schulz import orthonormalize
