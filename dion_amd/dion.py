@@ -27,7 +27,7 @@ from torch import Tensor
 from torch.optim.optimizer import Optimizer, ParamsT
 
 from . import _lib
-from .elementwise_opts import element_group_step
+from .elementwise_opts import element_groups_step
 
 
 @dataclass
@@ -169,10 +169,8 @@ class Dion(Optimizer):
 
         for group in dion_groups:
             self._dion_group_step(group)
-        for group in lion_groups:
-            self._lion_group_step(group)
-        for group in adamw_groups:
-            self._adamw_group_step(group)
+        element_groups_step(self, lion_groups, False)
+        element_groups_step(self, adamw_groups, True)
         return loss
 
     @torch.no_grad()
@@ -407,11 +405,6 @@ class Dion(Optimizer):
     def _new_state(self, param: Tensor, group: dict):
         self._get_or_initialize_state(param, group)
 
-    def _lion_group_step(self, group: dict):
-        element_group_step(self, group, False)
-
-    def _adamw_group_step(self, group: dict):
-        element_group_step(self, group, True)
 
 
 _side = threading.local()

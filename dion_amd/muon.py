@@ -21,7 +21,7 @@ from torch import Tensor
 from torch.optim.optimizer import Optimizer, ParamsT
 
 from . import _lib
-from .elementwise_opts import element_group_step
+from .elementwise_opts import element_groups_step
 from .newton_schulz import NS_SCHEDULE_COEFFS, flat_coeffs, zeropower_via_newtonschulz5
 
 
@@ -143,10 +143,8 @@ class Muon(Optimizer):
 
         for group in muon_groups:
             self._muon_group_step(group)
-        for group in lion_groups:
-            self._lion_group_step(group)
-        for group in adamw_groups:
-            self._adamw_group_step(group)
+        element_groups_step(self, lion_groups, False)
+        element_groups_step(self, adamw_groups, True)
         return loss
 
     # ------------------------------------------------------------------ state
@@ -255,8 +253,3 @@ class Muon(Optimizer):
         _lib.check(rc, "dion_amd_muon_post")
 
     # ------------------------------------------------------------------ element-wise groups
-    def _lion_group_step(self, group: dict):
-        element_group_step(self, group, False)
-
-    def _adamw_group_step(self, group: dict):
-        element_group_step(self, group, True)
