@@ -57,7 +57,8 @@ struct GroupDev {
   double *P64, *slab, *L, *T, *A2, *defect;
   int* words;                    // [cnt][CTR_STRIDE]
   int* info;
-  int cnt, first;
+  int cnt;
+  unsigned char nq[DA_QUEUES], at[DA_QUEUES];   // matrices in every queue; where their numbers begin in Args::order
   int m, n, r, rp, mp, np, mpT, npT, rT, transposed;
   int nT;
   int slices, kslice;            // of the Gram products
@@ -71,6 +72,7 @@ struct Args {
   unsigned long long spin_limit;
   int ngroups;
   int total[DA_QUEUES];          // tasks of every queue
+  unsigned char order[DA_DS_MATS];   // the matrices' numbers within their group, by group and queue
   int x_f32, g_f32, q_f32;
   float ef_alpha, decay, eps;
 };
@@ -104,6 +106,7 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
   __shared__ int sh_ticket[2];
   __shared__ int sh_words[2];
   __shared__ int sh_start[128], sh_per[128], sh_wait[128];   // the queue's schedule: entry = kind * ngroups + group
+  __shared__ unsigned char sh_at[128], sh_order[DA_DS_MATS];
   static_assert(KINDS * DA_DS_GROUPS <= 128, "one entry each");
   constexpr int MSZ = BF ? 2 : 4, MT = BF ? DA_BF16 : DA_F32;
   const int xcd = xcc_id();
@@ -128,13 +131,15 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
         const int k = tid / args.ngroups;
         const GroupDev& G = args.g[tid - k * args.ngroups];
         const int per = tasks_of(G, k, BF);
-        n = per * da_in_queue(G.first, G.cnt, q);
+        n = per * G.nq[q];
         int w = k == BTP ? PT : k - 1;
         while (w >= 0 && tasks_of(G, w, BF) == 0) --w;
         sh_per[tid] = per;
+        sh_at[tid] = G.at[q];
         sh_wait[tid] = w < 0 ? -1 : (w << 24 | tasks_of(G, w, BF));
       }
       sh_start[tid] = n;
+      if (tid < DA_DS_MATS) sh_order[tid] = args.order[tid];
     }
     __syncthreads();
     if (tid < 64) {   // exclusive sums of 128 entries by one wavefront
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
       const GroupDev& G = a.g[entry - kind * a.ngroups];
       const int kth = wave_uniform(t / per);
       const int task = wave_uniform(t - kth * per);
-      const int b = wave_uniform(((q - G.first) & 7) + 8 * kth);
+      const int b = wave_uniform((int)sh_order[sh_at[entry] + kth]);
       int* words = G.words + (long long)b * CTR_STRIDE;
       if (tid == 0) {
         if (wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
@@ -593,6 +598,34 @@ size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, 
 // control memory: words of all matrices, the queues' lines, the status word's line, the pointer tables
 size_t control_bytes(int mats) { return up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4) + up256((size_t)4 * mats * 8); }
 
+// Matrices to queues: the costliest first, each to the queue with the least to do so far.  (Dealt in the order of the buckets, 14
+// matrices of 1021, 341 and 2731 rows / columns left two XCDs with a tenth of the others' work: 730 us, so 670.)  Returns the
+// work of the fullest queue in microseconds (see da_dion_small_bytes); queue[i] of matrix i, in the order of the groups.
+double deal(const DaDionSmallGroup* g, int n, bool bf, unsigned char* queue) {
+  double load[DA_QUEUES] = {0}, cost[DA_DS_GROUPS];
+  int sorted[DA_DS_GROUPS], first[DA_DS_GROUPS];
+  for (int i = 0, mats = 0; i < n; ++i) {
+    const Shape S(g[i].m, g[i].n, g[i].r, bf);
+    cost[i] = (double)S.mpT * S.npT * (bf ? 0.2 + 0.12 * S.rT : 0.25 + 0.25 * S.rT);
+    first[i] = mats;
+    mats += g[i].cnt;
+    int k = i;
+    for (; k > 0 && cost[sorted[k - 1]] < cost[i]; --k) sorted[k] = sorted[k - 1];
+    sorted[k] = i;
+  }
+  for (int k = 0; k < n; ++k)
+    for (int j = 0; j < g[sorted[k]].cnt; ++j) {
+      int q = 0;
+      for (int x = 1; x < DA_QUEUES; ++x)
+        if (load[x] < load[q]) q = x;
+      load[q] += cost[sorted[k]];
+      if (queue) queue[first[sorted[k]] + j] = (unsigned char)q;
+    }
+  double worst = 0.0;
+  for (int q = 0; q < DA_QUEUES; ++q) worst = load[q] > worst ? load[q] : worst;
+  return worst;
+}
+
 }  // namespace
 
 size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, bool forced) {
@@ -606,7 +639,7 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
   // two d x 4d: bf16 d 128 r 64: 95 / 400;  256 x4 r 128: 204 / 464;  512 x8 r 32: 366 / 528;  512 x8 r 128: 502 / 534;
   // 768 x4 r 192: 703 / 506.  fp32 256 x4 r 128: 272 / 559;  768 x4 r 48: 643 / 948;  768 x12 r 192: 3121 / 2259.
   const bool bf = c.m_dtype == DA_BF16;
-  double load[DA_QUEUES] = {0}, chain = 0.0, other = 0.0;
+  double chain = 0.0, other = 0.0;
   bool padded = false, odd_full = false;
   for (int i = 0; i < n; ++i) {
     if (g[i].cnt < 1 || g[i].r < 1 || g[i].r > DA_DS_MAX_RANK || (long long)g[i].m * g[i].n > (1LL << 28) || (long long)g[i].m * g[i].n < 8) return 0;
@@ -615,7 +648,6 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
       // (lines of M and X must not be shared with another matrix; 16-byte loads of M and G by flat offset)
       if (((uintptr_t)g[i].M[j] | (uintptr_t)g[i].X[j]) & 127) return 0;
       if (((uintptr_t)g[i].G[j] | (uintptr_t)g[i].Q[j]) & 15) return 0;
-      load[(mats + j) & 7] += (double)S.mpT * S.npT * (bf ? 0.2 + 0.12 * S.rT : 0.25 + 0.25 * S.rT);
     }
     const double own = (bf ? 90.0 : 135.0) + 60.0 * (S.rT - 1) + (g[i].r == S.np ? 100.0 : 0.0);
     chain = own > chain ? own : chain;
@@ -628,8 +660,7 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
     bytes += lay_out(nullptr, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
   }
   if (mats > DA_DS_MATS) return 0;
-  double worst = 0;
-  for (int q = 0; q < DA_QUEUES; ++q) worst = load[q] > worst ? load[q] : worst;
+  const double worst = deal(g, n, bf, nullptr);
   other += (bf ? 400.0 : 480.0) * (padded ? 2.5 : 1.0);
   if (!forced && (odd_full || chain + worst > other)) return 0;
   return bytes + control_bytes(mats);
@@ -652,7 +683,9 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   su.preset = c.fail;
   su.dst = reinterpret_cast<void**>(p + up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4));
   p += control_bytes(mats);
-  int first = 0;
+  unsigned char queue[DA_DS_MATS];
+  deal(g, n, c.m_dtype == DA_BF16, queue);
+  int first = 0, at = 0;
   for (int i = 0; i < n; ++i) {
     const Shape S(g[i].m, g[i].n, g[i].r, c.m_dtype == DA_BF16);
     GroupDev& D = a.g[i];
@@ -666,7 +699,13 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
     }
     D.words = words + (size_t)first * CTR_STRIDE;
     D.info = g[i].info;
-    D.cnt = g[i].cnt; D.first = first;
+    D.cnt = g[i].cnt;
+    for (int q = 0; q < DA_QUEUES; ++q) {
+      D.at[q] = (unsigned char)at;
+      for (int j = 0; j < g[i].cnt; ++j)
+        if (queue[first + j] == q) a.order[at++] = (unsigned char)j;
+      D.nq[q] = (unsigned char)(at - D.at[q]);
+    }
     D.m = g[i].m; D.n = g[i].n; D.r = g[i].r; D.rp = S.rp; D.mp = S.mp; D.np = S.np;
     D.mpT = S.mpT; D.npT = S.npT; D.rT = S.rT; D.transposed = g[i].m < g[i].n ? 1 : 0;
     D.slices = S.slices; D.kslice = S.kslice;
@@ -676,7 +715,7 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   a.ngroups = n;
   for (int q = 0; q < DA_QUEUES; ++q)
     for (int i = 0; i < n; ++i)
-      for (int k = 0; k < KINDS; ++k) a.total[q] += da_in_queue(a.g[i].first, a.g[i].cnt, q) * tasks_of(a.g[i], k, c.m_dtype == DA_BF16);
+      for (int k = 0; k < KINDS; ++k) a.total[q] += a.g[i].nq[q] * tasks_of(a.g[i], k, c.m_dtype == DA_BF16);
   a.spin_limit = 200000000ull;   // 2 s of the 100 MHz counter
   a.x_f32 = c.x_dtype == DA_F32; a.g_f32 = c.g_dtype == DA_F32; a.q_f32 = c.q_dtype == DA_F32;
   a.ef_alpha = c.ef_alpha; a.decay = c.decay; a.eps = c.eps;
