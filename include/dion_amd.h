@@ -13,8 +13,11 @@
  *     synchronises with the host.
  *   - Matrices are row-major.  dtype codes: DION_AMD_BF16 / _F32 / _F64.
  *   - Return value: 0 ok; <0 argument error (DION_AMD_ERR_*); >0 a hipError_t.
- *   - Alignment: bf16 matrices need every dimension, pitch and batch stride to be a
- *     multiple of 8 elements and 16-byte aligned base pointers (fp32: multiples of 4).
+ *   - Alignment: the matrix-product, orthonormalisation and per-bucket Dion entry points need every
+ *     bf16 dimension, pitch and batch stride to be a multiple of 8 elements and 16-byte aligned base
+ *     pointers (fp32: multiples of 4).  Newton-Schulz, Muon and dion_amd_dion_step_buckets take any
+ *     dimensions; base pointers must be 16-byte aligned where rows are whole 16-byte pieces, else
+ *     aligned to their elements.
  *     A `workspace` pointer must be 256-byte aligned (the library carves it up itself).
  *     Violations return DION_AMD_ERR_ALIGN; nothing is launched.
  */
@@ -153,7 +156,7 @@ int dion_amd_muon_step(void* const* X, const void* const* G, void* const* M,
  * dion_amd_muon_pre replaces muon_update_pre_orthogonalize (reference dion/muon.py:525-552):
  * per matrix  M <- mu M + G (G cast to M's dtype first);  U = bf16(nesterov ? mu M + G : M),
  * with the reference's rounding after every tensor op.  G, M, U: HOST arrays of `batch` device
- * pointers to contiguous m x n matrices (n a multiple of 8); U receives bf16.
+ * pointers to contiguous m x n matrices; U receives bf16.
  *
  * dion_amd_muon_post replaces muon_update_post_orthogonalize (reference dion/muon.py:556-573):
  * X <- decay X;  X <- X - r_O(adjusted_lr O)  for O of the same shape in o_dtype (bf16 or f32: whatever the
