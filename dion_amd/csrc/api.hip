@@ -399,9 +399,11 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStre
     for (int i = 0; i < nj; ++i) {
       const NsJob& k = jobs[order[i]];
       const NsSet& S = sets[order[i]];
+      int vec = (k.ldx & 7) == 0;
+      for (int j = 0; j < k.cnt; ++j) vec = vec && ((uintptr_t)k.X[j] & 15) == 0;
       sg[i] = DaNsSmallGroup{S.W.x0, S.W.x1, S.W.a, S.W.b, (long long)(S.L.x_bytes / 2), (long long)(S.L.a_bytes / 2),
                              S.L.mw, S.L.nw, S.L.ldx, S.L.lda, k.cnt, S.W.partials, S.L.tiles, S.W.xtab,
-                             c.x_dtype, k.m, k.n, k.ldx, c.update, k.decay, k.step};
+                             c.x_dtype, k.m, k.n, k.ldx, c.update, vec, k.decay, k.step};
     }
     DaProfScope prof(DA_PROF_NS_FLOW, flops, s);
     return da_ns_small(sg, nj, c.coeffs, c.steps, c.eps, ctl, s);
@@ -467,7 +469,8 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStre
   return DA_OK;
 }
 
-// 16-byte alignment of a matrix whose rows are whole 16-byte chunks; rows off that grid need their elements' alignment.
+// 16-byte alignment of matrices on the 8-element grid (`chunks`); others need their elements' alignment: the staging and
+// update passes look at the addresses and move such matrices with unaligned accesses.
 inline bool misaligned(const void* p, bool chunks, size_t esz) { return ((uintptr_t)p & (chunks ? 15 : esz - 1)) != 0; }
 
 bool dtype_ok(int d) { return d == DA_BF16 || d == DA_F32; }
@@ -542,7 +545,7 @@ int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, l
   // itself, needs 256
   const bool g_chunks = !((n | ldg) & 7), o_chunks = !((n | ldo) & 7);
   if ((g_chunks && (g_stride & 7)) || (o_chunks && (out_stride & 7))) return DA_ERR_ALIGN;
-  if (misaligned(G, g_chunks, gsz) || misaligned(out, o_chunks, osz)) return DA_ERR_ALIGN;
+  if (misaligned(G, g_chunks && !(m & 7), gsz) || misaligned(out, o_chunks && !(m & 7), osz)) return DA_ERR_ALIGN;
   if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const NsLayout L(m, n, compute_dtype);
@@ -701,8 +704,8 @@ size_t dion_amd_muon_workspace_bytes(int batch, int m, int n) {
 }  // extern "C"
 
 namespace {
-int muon_check(void* const* X, const void* const* G, void* const* M, int batch, int n, int x_dtype, int g_dtype) {
-  const bool chunks = (n & 7) == 0;
+int muon_check(void* const* X, const void* const* G, void* const* M, int batch, int m, int n, int x_dtype, int g_dtype) {
+  const bool chunks = ((m | n) & 7) == 0;
   const size_t xsz = x_dtype == DA_BF16 ? 2 : 4, gsz = g_dtype == DA_BF16 ? 2 : 4;
   for (int i = 0; i < batch; ++i) {
     if (!X[i] || !G[i] || !M[i]) return DA_ERR_ARG;
@@ -720,7 +723,7 @@ int dion_amd_muon_step(void* const* X, const void* const* G, void* const* M, int
   if (!X || !G || !M || !coeffs || !workspace || batch <= 0 || m <= 0 || n <= 0 || steps < 0) return DA_ERR_ARG;
   if (!dtype_ok(x_dtype) || !dtype_ok(g_dtype)) return DA_ERR_DTYPE;
   if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
-  const int rc = muon_check(X, G, M, batch, n, x_dtype, g_dtype);
+  const int rc = muon_check(X, G, M, batch, m, n, x_dtype, g_dtype);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const NsLayout L(m, n, DA_BF16);
@@ -828,7 +831,7 @@ int dion_amd_muon_step_buckets(const dion_amd_muon_bucket* buckets, int nbuckets
   for (int i = 0; i < nbuckets; ++i) {
     const dion_amd_muon_bucket& k = buckets[i];
     if (!k.X || !k.G || !k.M || k.batch <= 0 || k.m <= 0 || k.n <= 0) return DA_ERR_ARG;
-    const int rc = muon_check(k.X, k.G, k.M, k.batch, k.n, x_dtype, g_dtype);
+    const int rc = muon_check(k.X, k.G, k.M, k.batch, k.m, k.n, x_dtype, g_dtype);
     if (rc) return rc;
   }
   if (workspace_bytes < dion_amd_muon_buckets_workspace_bytes(buckets, nbuckets)) return DA_ERR_WORKSPACE;

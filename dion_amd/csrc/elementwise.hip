@@ -169,7 +169,7 @@ struct StageArgs {
   int tiles[DA_MAX_GROUPS];      // blocks per matrix
 };
 
-// VEC: the rows of every group are whole 16-byte chunks
+// VEC: the rows of every group are whole, 16-byte aligned chunks
 template <typename TG, typename TM, typename TW, bool VEC>
 __global__ __launch_bounds__(256, VEC ? 5 : 4) void stage_kernel(StageArgs a) {
   __shared__ float red[4];
@@ -374,7 +374,7 @@ struct UnstageArgs {
   const int* poison;  // optional device word: non-zero = the working matrices are invalid, the result becomes NaN
 };
 
-// VEC: the rows of x (and of wtab's matrices) are whole 16-byte chunks
+// VEC: the rows of x (and of wtab's matrices) are whole, 16-byte aligned chunks
 template <typename TX, typename TW, bool TALL, bool VEC>
 __global__ __launch_bounds__(256) void unstage_kernel(UnstageArgs<TX, TW> a) {
   __shared__ float tile[TALL ? TS : 1][TS + 1];
@@ -475,10 +475,20 @@ __global__ __launch_bounds__(256) void unstage_kernel(UnstageArgs<TX, TW> a) {
   }
 }
 
+inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// The vector form is for rows of whole 16-byte chunks at 16-byte aligned addresses: a matrix off the 8-element grid may start
+// anywhere (33 rows of 64 elements: whole chunks, but wherever the caller's view begins).
 template <typename TG, typename TM, typename TW>
 int stage_launch(const StageArgs& a, hipStream_t s) {
   bool vec = true;
-  for (int i = 0; i < a.d.ngroups; ++i) vec = vec && !((a.d.g[i].ld | a.d.g[i].cols) & 7);
+  for (int i = 0, mat = 0; i < a.d.ngroups; ++i) {
+    const DaStageGroup& g = a.d.g[i];
+    vec = vec && !((g.ld | g.cols) & 7);
+    for (int b = 0; vec && b < g.cnt; ++b)
+      vec = aligned16(a.d.src[mat + b]) && (!a.d.muon || aligned16(a.d.mom[mat + b])) && (g.wide || aligned16(a.d.dst[mat + b]));
+    mat += g.cnt;
+  }
   const dim3 grid((unsigned)a.blk0[DA_MAX_GROUPS]);
   if (vec) hipLaunchKernelGGL((stage_kernel<TG, TM, TW, true>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((stage_kernel<TG, TM, TW, false>), grid, dim3(256), 0, s, a);
@@ -492,7 +502,8 @@ int stage_dispatch_w(const StageArgs& a, hipStream_t s) {
 
 template <typename TX, typename TW>
 int unstage_launch(const DaUnstage& d, hipStream_t s) {
-  const bool vec = !((d.ld | (d.use_wtab ? d.ldw : 0) | d.cols) & 7);
+  bool vec = !((d.ld | (d.use_wtab ? d.ldw : 0) | d.cols) & 7);
+  for (int b = 0; vec && b < d.batch; ++b) vec = aligned16(d.x.p[b]) && (!d.use_wtab || aligned16(d.wtab.p[b]));
   UnstageArgs<TX, TW> a{d.x, static_cast<const TW*>(d.wide), d.rows, d.cols, d.ld, d.mw, d.ldw, d.decay, d.step, d.muon, d.use_wtab, d.wtab, d.poison};
   const bool tall = d.rows > d.cols && !d.use_wtab;
   const int tiles = tall ? ((a.rows + TS - 1) / TS) * ((a.cols + TS - 1) / TS)

@@ -13,6 +13,7 @@ constexpr int DA_SMALL_TAIL = 9 * 32;
 // x0, x1: [cnt][mw][ldx], a, b: [cnt][mw][lda].  x0 holds the staged input (not yet divided by its norm), zero outside
 // the true matrix; partials: [cnt][ptiles] sums of squares of the staged input.
 // tab: device table of `cnt` destination matrices (rows x cols, row pitch ld, dtype), stored transposed when rows > cols.
+// vec: every destination row is whole 16-byte chunks (pitch a multiple of 8 elements, base 16-byte aligned).
 // update 1: W <- r_W(r_W(W * decay) - r_bf16(X' * step)); 0: W <- X' (bf16 destinations).
 struct DaNsSmallGroup {
   char *x0, *x1, *a, *b;
@@ -21,7 +22,7 @@ struct DaNsSmallGroup {
   const float* partials;
   int ptiles;
   void* const* tab;
-  int dtype, rows, cols, ld, update;
+  int dtype, rows, cols, ld, update, vec;
   float decay, step;
 };
 

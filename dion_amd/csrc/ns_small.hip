@@ -579,7 +579,7 @@ int da_ns_small(const DaNsSmallGroup* g, int n, const float* coeffs, int steps, 
     D.tnorm = (int)(((long long)G.mw * G.ldx + NORM_ELEMS - 1) / NORM_ELEMS);
     D.cnt = G.cnt; D.first = first;
     D.dtype = G.dtype; D.rows = G.rows; D.cols = G.cols; D.ld = G.ld; D.update = G.update;
-    D.vec = (G.ld % 8) == 0;
+    D.vec = G.vec;
     D.decay = G.decay; D.step = G.step;
     first += G.cnt;
     tickets += (long long)G.cnt * (D.tnorm + steps * (D.tm * (D.tm + 1) + D.tm * D.tn));

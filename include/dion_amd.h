@@ -15,9 +15,10 @@
  *   - Return value: 0 ok; <0 argument error (DION_AMD_ERR_*); >0 a hipError_t.
  *   - Alignment: the matrix-product, orthonormalisation and per-bucket Dion entry points need every
  *     bf16 dimension, pitch and batch stride to be a multiple of 8 elements and 16-byte aligned base
- *     pointers (fp32: multiples of 4).  Newton-Schulz, Muon and dion_amd_dion_step_buckets take any
- *     dimensions; base pointers must be 16-byte aligned where rows are whole 16-byte pieces, else
- *     aligned to their elements.
+ *     pointers (fp32: multiples of 4).  Newton-Schulz and Muon take any dimensions; base pointers must
+ *     be 16-byte aligned where both dimensions and the pitch are multiples of 8, else aligned to their
+ *     elements (dion_amd_muon_pre / _post: where the row length is a multiple of 8; batch strides:
+ *     multiples of 8 where row length and pitch are).  dion_amd_dion_step_buckets has its own rule.
  *     A `workspace` pointer must be 256-byte aligned (the library carves it up itself).
  *     Violations return DION_AMD_ERR_ALIGN; nothing is launched.
  */

@@ -339,3 +339,50 @@ def test_muon_hook_returning_fp32_keeps_its_precision(dev):
         for i, p in enumerate(params):
             assert torch.equal(opt.state[p]["momentum"].cpu(), Mo[i]), (step, i)
             assert torch.equal(p.detach().cpu(), Xo[i]), (step, i)
+
+
+# ------------------------------------------------------------------ views that start anywhere
+def _view(shape, shift, dtype, gen, dev, scale):
+    """A contiguous `shape` view `shift` elements into a flat buffer, and the buffer."""
+    numel = shape[0] * shape[1]
+    flat = (torch.randn(numel + shift + 8, generator=gen, device=dev) * scale).to(dtype)
+    return flat[shift:shift + numel].view(shape), flat
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shapes", [
+    [(33, 64), (64, 33), (33, 65), (17, 8)],                   # one launch
+    [(1021, 1024), (1024, 1021)] * 2,                          # batched products, separate update pass
+    [(33, 64), (64, 64)],                                      # a bucket on the grid beside one off it (the latter aligned)
+])
+def test_matrices_off_the_8_grid_may_start_anywhere(dev, shapes, dtype):
+    """Weights, gradients and momentum as views at odd offsets of flat buffers give the bits of aligned copies, and leave what
+    lies around the view alone."""
+    from dion_amd import Muon, zeropower_via_newtonschulz5
+
+    gen = torch.Generator(device=dev).manual_seed(11)
+    runs = {False: [], True: []}
+    for i, s in enumerate(shapes):
+        shift = 0 if s[0] % 8 == 0 and s[1] % 8 == 0 else (1, 3, 4, 5)[i % 4]
+        views = [_view(s, shift, dtype, gen, dev, scale) for scale in (0.02, 1e-3, 3e-3)]
+        for moved in (False, True):
+            x, g, m = ((v, f) if moved else (v.clone(), None) for v, f in views)
+            runs[moved].append((x, g, m))
+    around = [[f.clone() for f in (x[1], g[1], m[1])] for x, g, m in runs[True]]
+    for s, (x, g, m) in zip(shapes, runs[True]):
+        assert torch.equal(zeropower_via_newtonschulz5(g[0]), zeropower_via_newtonschulz5(g[0].clone()))
+    for moved in (False, True):
+        params = [torch.nn.Parameter(x[0]) for x, _, _ in runs[moved]]
+        opt = Muon(params, lr=0.02, mu=0.95, weight_decay=0.01, nesterov=True)
+        for p, (_, g, m) in zip(params, runs[moved]):
+            p.grad = g[0]
+            opt.state[p]["momentum"] = m[0]
+        opt.step()
+    torch.cuda.synchronize()
+    for s, a, b, old in zip(shapes, runs[False], runs[True], around):
+        assert torch.isfinite(b[0][0].float()).all() and not torch.equal(b[0][1], old[0])
+        for k, name in enumerate(("weights", "gradient", "momentum")):
+            assert torch.equal(a[k][0], b[k][0]), (s, name)
+            shift, numel = b[k][0].storage_offset(), s[0] * s[1]
+            new = b[k][1]
+            assert torch.equal(new[:shift], old[k][:shift]) and torch.equal(new[shift + numel:], old[k][shift + numel:]), (s, name)

@@ -1,0 +1,48 @@
+"""CPU-side contract of the entry points and of the host module: what they accept, what they refuse, and how often they run what
+a user registered.  Nothing is launched: library calls end at a workspace of no bytes, steps at a missing GPU."""
+import ctypes
+
+import pytest
+import torch
+
+ALIGN, WORKSPACE = -2, -3
+BASE = 0x7F0000000000     # addresses that are looked at, never followed
+
+
+def _pointers(offset, count=2):
+    return (ctypes.c_void_p * count)(*[BASE + i * (1 << 24) + offset for i in range(count)])
+
+
+@pytest.mark.parametrize("m,n", [(33, 64), (64, 33), (33, 65), (1, 8), (4095, 4096)])
+def test_matrices_off_the_8_grid_need_only_the_alignment_of_their_elements(m, n):
+    """A view into a flat buffer may start anywhere when a dimension is no multiple of 8 (reference dion/muon.py:525-573 takes
+    any tensor): the check behind the addresses, that of the workspace's size, is the one that answers."""
+    from dion_amd import _lib
+
+    lib = _lib.load()
+    coeffs = _lib.float_array([1.0, 1.0, 1.0])
+    for code, size in ((_lib.BF16, 2), (_lib.F32, 4)):
+        for offset, want in ((0, WORKSPACE), (size, WORKSPACE), (8, WORKSPACE), (size // 2, ALIGN)):
+            ptrs = _pointers(offset)
+            rc = lib.dion_amd_newton_schulz(BASE + offset, code, m * n, n, BASE, m * n, n, 1, m, n, coeffs, 1, 1e-7, _lib.BF16, 1,
+                                            BASE, 0, None)
+            assert rc == want, (m, n, code, offset)
+            assert lib.dion_amd_muon_step(ptrs, ptrs, ptrs, 2, m, n, code, code, 0.9, 0, 1.0, 0.1, coeffs, 1, 1e-7, 1,
+                                          BASE, 0, None) == want
+            k = _lib.MuonBucket()
+            k.X = k.G = k.M = ctypes.cast(ptrs, ctypes.POINTER(ctypes.c_void_p))
+            k.batch, k.m, k.n, k.decay, k.adjusted_lr = 2, m, n, 1.0, 0.1
+            assert lib.dion_amd_muon_step_buckets(ctypes.byref(k), 1, code, code, 0.9, 0, coeffs, 1, 1e-7, 1, BASE, 0, None) == want
+
+
+def test_matrices_on_the_8_grid_need_16_byte_alignment():
+    from dion_amd import _lib
+
+    lib = _lib.load()
+    coeffs = _lib.float_array([1.0, 1.0, 1.0])
+    for offset, want in ((0, WORKSPACE), (16, WORKSPACE), (8, ALIGN)):
+        ptrs = _pointers(offset)
+        assert lib.dion_amd_newton_schulz(BASE + offset, _lib.BF16, 0, 64, BASE, 0, 64, 1, 32, 64, coeffs, 1, 1e-7, _lib.BF16, 1,
+                                          BASE, 0, None) == want
+        assert lib.dion_amd_muon_step(ptrs, ptrs, ptrs, 2, 32, 64, _lib.F32, _lib.F32, 0.9, 0, 1.0, 0.1, coeffs, 1, 1e-7, 1,
+                                      BASE, 0, None) == want
