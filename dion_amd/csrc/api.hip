@@ -33,6 +33,18 @@ inline int padded_dim(int x) {
   return r256 * 100LL <= r128 * 107LL ? r256 : r128;
 }
 
+// Whether the working matrices of m x n matrices are padded to whole tiles: not where that makes them more than 1.7 times as
+// large (a thin matrix: the factors of a low-rank adapter).  Those keep the 8-element grid and the K loop with bounds checks,
+// as their passes over memory cost more than that loop.  Muon steps, us, 8-grid : padded, by how much the padding adds:
+//   x 8     224 of 16 x 4096 and of 4096 x 16   1203 : 2194 (workspace 115 : 939 MiB)     256 of 8 x 8192 (x 16)  1284 : 2456
+//   x 2     224 of 64 x 4096 and of 4096 x 64   1794 : 2312 (462 : 939)                   128 of 136 x 4096 (x 1.88)  1285 : 1418
+//   x 1.78  512 of 72 x 1024   655 : 753
+//   x 1.64  512 of 200 x 200   720 : 631, 256 of 300 x 300   834 : 947      x 1.45  96 of 264 x 2048   1128 : 1143
+//   x 1.36  24 of 1096 x 1096  1689 : 1188                                   x 1.21  4 of 648 x 10000   1388 : 1048
+inline bool padding_pays(int mw, int nw) {
+  return (double)padded_dim(mw) * padded_dim(nw) <= 1.7 * round_up(mw, 8) * (double)round_up(nw, 8);
+}
+
 // Whether the buckets of one grouped call all go to whole 256-tiles: a grouped product runs 256-tiles only where every member
 // has them, so one member on the 128-grid costs all of them a third more per multiply-add.  (14 of 2368 x 2368 and 7 each of
 // 7040 x 2368 and 2368 x 7040 with 14 of 789 x 2368, padded to 896: 22.0 ms, padded to 1024: 17.3 ms.)
@@ -42,6 +54,7 @@ bool grid256(const Bucket* k, int n, Count count) {
   bool on = false, off = false;
   for (int i = 0; i < n; ++i) {
     const int mw = k[i].m < k[i].n ? k[i].m : k[i].n, nw = k[i].m < k[i].n ? k[i].n : k[i].m;
+    if (!padding_pays(mw, nw)) continue;   // (on the 8-grid whatever the others do, and in launches of their own)
     auto cost = [&](double a, double b) { return count(k[i]) * a * a * (3.0 * b + a); };
     const int am = padded_dim(mw), an = padded_dim(nw), bm = round_up(mw, 256), bn = round_up(nw, 256);
     (am == bm && an == bn ? on : off) = true;
@@ -49,6 +62,25 @@ bool grid256(const Bucket* k, int n, Count count) {
     big += cost(bm, bn);
   }
   return on && off && big <= 1.33 * nat;
+}
+
+// Whether the one-launch kernel for small matrices has little enough work with these buckets (`count` of each).  Matrices are
+// dealt to eight queues of one XCD's workgroups each; what counts is the longest queue, in 64 x 64 x 64 stages per iteration.
+// Measured against the batched launches (us per call): 912 stages (16 x 256 x 1024) 141 : 206, 1088 (512 x 512) 129 : 191,
+// 3488 (512 x 2048) 260 : 286, 3600 (768 x 768) 300 : 247, 3648 (64 x 256 x 1024) 348 : 279.
+template <typename Bucket, typename Count>
+bool small_enough(const Bucket* k, int n, Count count) {
+  double load[8] = {0}, worst = 0;
+  int first = 0;
+  for (int i = 0; i < n; ++i) {
+    const int mw = round_up(k[i].m < k[i].n ? k[i].m : k[i].n, DA_SMALL_BT) / DA_SMALL_BT;
+    const int nw = round_up(k[i].m < k[i].n ? k[i].n : k[i].m, DA_SMALL_BT) / DA_SMALL_BT;
+    const double sym = 0.5 * mw * (mw + 1), stages = sym * nw + sym * mw + (double)mw * nw * mw;
+    for (int j = 0; j < count(k[i]); ++j) load[(first + j) & 7] += stages;
+    first = (first + count(k[i])) & 7;
+  }
+  for (int q = 0; q < 8; ++q) worst = load[q] > worst ? load[q] : worst;
+  return worst <= 2500.0;
 }
 
 constexpr size_t FLOW_TAIL_BYTES = 1536;   // behind the counters of a control area: ticket, owner and status words
@@ -60,13 +92,13 @@ struct NsLayout {
   size_t x_bytes = 0, a_bytes = 0, part_bytes = 0, flow_bytes = 0;  // per matrix
   size_t per_matrix = 0;
   NsLayout() {}
-  // m x n matrices; `small`: the layout of the one-launch kernel for small matrices (ns_small.hip), which never needs
-  // more memory than the other one; `all256`: see grid256
+  // m x n matrices; `small`: the layout of the one-launch kernel for small matrices (ns_small.hip); `all256`: see grid256
   NsLayout(int m, int n, int dtype, bool small = false, bool all256 = false) {
     mw = m < n ? m : n;
     nw = m < n ? n : m;
     if (dtype != DA_BF16) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
     else if (small) { mw = round_up(mw, DA_SMALL_BT); nw = round_up(nw, DA_SMALL_BT); }
+    else if (!padding_pays(mw, nw)) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
     else if (all256) { mw = round_up(mw, 256); nw = round_up(nw, 256); }
     else { mw = padded_dim(mw); nw = padded_dim(nw); }
     tiles = da_stage_tiles(m, n, mw, nw);
@@ -90,14 +122,26 @@ struct NsLayout {
     if (c > DA_MAX_PTRS) c = DA_MAX_PTRS;
     return (int)c;
   }
-  size_t recommended(int batch) const {
-    size_t c = ((size_t)4 << 30) / per_matrix;
-    if (c < 1) c = 1;
-    if (c > (size_t)batch) c = batch;
-    if (c > DA_MAX_PTRS) c = DA_MAX_PTRS;
-    return c * per_matrix;
-  }
+  // whole tiles in both dimensions: the products of such matrices share launches without bounds checks
+  bool whole_tiles() const { return mw % 128 == 0 && nw % 128 == 0; }
 };
+
+// Recommended workspace for a bucket: 4 GiB of matrices at most, and room for the layout of the one-launch kernel (whole
+// 64-tiles, which a thin matrix does not have otherwise) where that kernel would take as many matrices at a time.
+size_t ns_workspace_bytes(int batch, int m, int n, int dtype) {
+  const NsLayout L(m, n, dtype);
+  size_t c = ((size_t)4 << 30) / L.per_matrix;
+  if (c < 1) c = 1;
+  if (c > (size_t)batch) c = batch;
+  if (c > DA_MAX_PTRS) c = DA_MAX_PTRS;
+  size_t bytes = c * L.per_matrix;
+  struct { int m, n; } shape = {m, n};
+  if (dtype == DA_BF16 && small_enough(&shape, 1, [&](const decltype(shape)&) { return (int)c; })) {
+    const size_t small = align_up(NsLayout(m, n, dtype, true).per_matrix * c, 256);
+    bytes = bytes > small ? bytes : small;
+  }
+  return bytes;
+}
 
 struct NsBuffers {
   char *x0 = nullptr, *x1 = nullptr, *a = nullptr, *b = nullptr;
@@ -286,29 +330,82 @@ struct NsCall {
   int faithful;
 };
 
-// Whether the one-launch kernel for small matrices takes these jobs.  Matrices are dealt to eight queues of one XCD's
-// workgroups each; what counts is the longest queue, in 64 x 64 x 64 stages per iteration.  Measured against the batched
-// launches (us per call): 912 stages (16 x 256 x 1024) 141 : 206, 1088 (512 x 512) 129 : 191, 3488 (512 x 2048) 260 : 286,
-// 3600 (768 x 768) 300 : 247, 3648 (64 x 256 x 1024) 348 : 279.
-bool ns_small_wanted(const NsJob* jobs, int nj, const NsCall& c) {
-  if (c.compute_dtype != DA_BF16 || !c.faithful || c.steps < 1 || c.steps > DA_SMALL_MAX_STEPS) return false;
-  if (da_ns_flow_mode() >= 0) return false;   // the caller chose between the other two
-  double load[8] = {0}, worst = 0;
-  int first = 0;
-  for (int i = 0; i < nj; ++i) {
-    const int mw = round_up(jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n, DA_SMALL_BT) / DA_SMALL_BT;
-    const int nw = round_up(jobs[i].m < jobs[i].n ? jobs[i].n : jobs[i].m, DA_SMALL_BT) / DA_SMALL_BT;
-    const double sym = 0.5 * mw * (mw + 1), stages = sym * nw + sym * mw + (double)mw * nw * mw;
-    for (int j = 0; j < jobs[i].cnt; ++j) load[(first + j) & 7] += stages;
-    first += jobs[i].cnt;
+// The iterations of `n` of the staged and normalised sets, and what becomes of their results.
+int ns_finish(const NsJob* jobs, const NsSet* sets, const int* order, int n, const NsCall& c, hipStream_t s) {
+  const double xsz = c.x_dtype == DA_BF16 ? 2 : 4;
+  NsSet part[DA_MAX_GROUPS];
+  // The last product updates the weights in its epilogue where it has whole tiles of them; otherwise (and for a plain
+  // result) a pass of its own follows.
+  bool whole = c.update != 0;
+  for (int i = 0; i < n; ++i) {
+    part[i] = sets[order[i]];
+    const NsJob& k = jobs[order[i]];
+    const int mt = k.m < k.n ? k.m : k.n, nt = k.m < k.n ? k.n : k.m;
+    whole = whole && part[i].L.mw == mt && part[i].L.nw == nt && (k.ldx & 7) == 0;
   }
-  for (int q = 0; q < 8; ++q) worst = load[q] > worst ? load[q] : worst;
-  return worst <= 2500.0;
+  char* res[DA_MAX_GROUPS];
+  const int* poison = nullptr;
+  bool updated = false;
+  int rc = ns_iterate(part, n, c.compute_dtype, c.coeffs, c.steps, c.faithful, s, res, &poison, whole ? &updated : nullptr);
+  if (rc) return rc;
+  if (updated && poison) {
+    // a persistent launch that updated the weights itself: NaN in all of them if it gave up
+    DaPtrUploads up{};
+    DaPoisonShape shape{};
+    shape.f32 = c.x_dtype == DA_F32;
+    int count = 0;
+    for (int i = 0; i < n; ++i) {
+      const NsJob& k = jobs[order[i]];
+      for (int j0 = 0; j0 < k.cnt; j0 += DA_MAX_PTRS) {
+        const int cnt = k.cnt - j0 < DA_MAX_PTRS ? k.cnt - j0 : DA_MAX_PTRS;
+        for (int j = 0; j < cnt; ++j) up.t[count].p[j] = k.X[j0 + j];
+        up.n[count] = cnt;
+        shape.numel[count] = (long long)k.m * k.n;
+        if (++count == DA_MAX_UPLOADS) {
+          rc = da_poison_multi_if(up, count, shape, poison, s);
+          if (rc) return rc;
+          count = 0;
+        }
+      }
+    }
+    return count ? da_poison_multi_if(up, count, shape, poison, s) : DA_OK;
+  }
+  for (int i = 0; i < n && !updated; ++i) {
+    const NsJob& k = jobs[order[i]];
+    const NsLayout& L = part[i].L;
+    for (int j0 = 0; j0 < k.cnt; j0 += DA_MAX_PTRS) {
+      const int cnt = k.cnt - j0 < DA_MAX_PTRS ? k.cnt - j0 : DA_MAX_PTRS;
+      DaUnstage us{};
+      for (int j = 0; j < cnt; ++j) us.x.p[j] = k.X[j0 + j];
+      us.wide = res[i] + (size_t)j0 * L.x_bytes;
+      us.batch = cnt; us.rows = k.m; us.cols = k.n; us.ld = k.ldx; us.mw = L.mw; us.ldw = L.ldx;
+      us.x_dtype = c.x_dtype; us.w_dtype = c.compute_dtype;
+      us.decay = k.decay; us.step = k.step; us.muon = c.update;
+      us.poison = poison;
+      // algorithmic bytes: read X (update only) and the result, write X
+      DaProfScope prof(DA_PROF_UNSTAGE, (double)k.m * k.n * ((c.update ? 2 : 1) * xsz + L.esz) * cnt, s);
+      rc = da_unstage(us, s);
+      if (rc) return rc;
+    }
+  }
+  return DA_OK;
 }
 
-int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStream_t s) {
+// Whether the one-launch kernel for small matrices takes these jobs.
+bool ns_small_wanted(const NsJob* jobs, int nj, const NsCall& c, size_t workspace_bytes) {
+  if (c.compute_dtype != DA_BF16 || !c.faithful || c.steps < 1 || c.steps > DA_SMALL_MAX_STEPS) return false;
+  if (da_ns_flow_mode() >= 0) return false;   // the caller chose between the other two
+  if (!small_enough(jobs, nj, [](const NsJob& k) { return k.cnt; })) return false;
+  // (a workspace sized by the queries holds this layout; a smaller one that holds the other takes the batched launches)
+  size_t need = 0;
+  for (int i = 0; i < nj; ++i)
+    need += align_up(NsLayout(jobs[i].m, jobs[i].n, c.compute_dtype, true).per_matrix * (size_t)jobs[i].cnt, 256);
+  return need <= workspace_bytes;
+}
+
+int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, size_t workspace_bytes, hipStream_t s) {
   if (nj < 1 || nj > DA_MAX_GROUPS) return DA_ERR_ARG;
-  const bool small = ns_small_wanted(jobs, nj, c);
+  const bool small = ns_small_wanted(jobs, nj, c, workspace_bytes);
   const bool all256 = grid256(jobs, nj, [](const NsJob& k) { return k.cnt; });
   // carve the workspace: every job keeps all of its matrices resident
   NsSet sets[DA_MAX_GROUPS];
@@ -415,58 +512,17 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, hipStre
                                 L.tiles, c.eps, s);
     if (rc) return rc;
   }
-  // The last product updates the weights in its epilogue where it has whole tiles of them; otherwise (and for a plain
-  // result) a pass of its own follows.
-  bool whole = c.update != 0;
-  for (int i = 0; i < nj; ++i) {
-    const NsLayout& L = sets[i].L;
-    const int mt = jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n, nt = jobs[i].m < jobs[i].n ? jobs[i].n : jobs[i].m;
-    whole = whole && L.mw == mt && L.nw == nt && (jobs[i].ldx & 7) == 0;
-  }
-  char* res[DA_MAX_GROUPS];
-  const int* poison = nullptr;
-  bool updated = false;
-  int rc = ns_iterate(sets, nj, c.compute_dtype, c.coeffs, c.steps, c.faithful, s, res, &poison, whole ? &updated : nullptr);
-  if (rc) return rc;
-  if (updated && poison) {
-    // a persistent launch that updated the weights itself: NaN in all of them if it gave up
-    DaPtrUploads up{};
-    DaPoisonShape shape{};
-    shape.f32 = c.x_dtype == DA_F32;
-    int count = 0;
+  // Matrices in whole tiles and others in launches of their own: one member that needs the checked K loop puts it on all
+  // of a grouped launch (and keeps the persistent kernel and the update in the last epilogue from all of them).
+  int order[DA_MAX_GROUPS], nwhole = 0;
+  for (int pass = 0, k = 0; pass < 2; ++pass)
     for (int i = 0; i < nj; ++i)
-      for (int j0 = 0; j0 < jobs[i].cnt; j0 += DA_MAX_PTRS) {
-        const int n = jobs[i].cnt - j0 < DA_MAX_PTRS ? jobs[i].cnt - j0 : DA_MAX_PTRS;
-        for (int j = 0; j < n; ++j) up.t[count].p[j] = jobs[i].X[j0 + j];
-        up.n[count] = n;
-        shape.numel[count] = (long long)jobs[i].m * jobs[i].n;
-        if (++count == DA_MAX_UPLOADS) {
-          rc = da_poison_multi_if(up, count, shape, poison, s);
-          if (rc) return rc;
-          count = 0;
-        }
-      }
-    return count ? da_poison_multi_if(up, count, shape, poison, s) : DA_OK;
+      if ((c.compute_dtype != DA_BF16 || sets[i].L.whole_tiles()) == (pass == 0)) { order[k++] = i; nwhole += pass == 0; }
+  if (nwhole) {
+    const int rc = ns_finish(jobs, sets, order, nwhole, c, s);
+    if (rc) return rc;
   }
-  for (int i = 0; i < nj && !updated; ++i) {
-    const NsJob& k = jobs[i];
-    const NsLayout& L = sets[i].L;
-    for (int j0 = 0; j0 < k.cnt; j0 += DA_MAX_PTRS) {
-      const int n = k.cnt - j0 < DA_MAX_PTRS ? k.cnt - j0 : DA_MAX_PTRS;
-      DaUnstage us{};
-      for (int j = 0; j < n; ++j) us.x.p[j] = k.X[j0 + j];
-      us.wide = res[i] + (size_t)j0 * L.x_bytes;
-      us.batch = n; us.rows = k.m; us.cols = k.n; us.ld = k.ldx; us.mw = L.mw; us.ldw = L.ldx;
-      us.x_dtype = c.x_dtype; us.w_dtype = c.compute_dtype;
-      us.decay = k.decay; us.step = k.step; us.muon = c.update;
-      us.poison = poison;
-      // algorithmic bytes: read X (update only) and the result, write X
-      DaProfScope prof(DA_PROF_UNSTAGE, (double)k.m * k.n * ((c.update ? 2 : 1) * xsz + L.esz) * n, s);
-      rc = da_unstage(us, s);
-      if (rc) return rc;
-    }
-  }
-  return DA_OK;
+  return nwhole < nj ? ns_finish(jobs, sets, order + nwhole, nj - nwhole, c, s) : DA_OK;
 }
 
 // 16-byte alignment of matrices on the 8-element grid (`chunks`); others need their elements' alignment: the staging and
@@ -527,7 +583,7 @@ const char* dion_amd_version(void) { return "dion_amd 0.1 (gfx950)"; }
 
 size_t dion_amd_ns_workspace_bytes(int batch, int m, int n, int compute_dtype) {
   if (batch <= 0 || m <= 0 || n <= 0 || !dtype_ok(compute_dtype)) return 0;
-  return NsLayout(m, n, compute_dtype).recommended(batch);
+  return ns_workspace_bytes(batch, m, n, compute_dtype);
 }
 
 }  // extern "C"
@@ -561,7 +617,7 @@ int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, l
       dst[i] = static_cast<char*>(out) + (size_t)(b0 + i) * out_stride * osz;
     }
     const NsJob job = {src, nullptr, dst, cb, m, n, ldg, ldo, 1.f, 1.f};
-    const int rc = ns_jobs(&job, 1, call, workspace, s);
+    const int rc = ns_jobs(&job, 1, call, workspace, workspace_bytes, s);
     if (rc) return rc;
   }
   return DA_OK;
@@ -698,7 +754,7 @@ int dion_amd_ns_flow_trace_read(void* host_dst, int max_tiles, int* tiles) {
 
 size_t dion_amd_muon_workspace_bytes(int batch, int m, int n) {
   if (batch <= 0 || m <= 0 || n <= 0) return 0;
-  return NsLayout(m, n, DA_BF16).recommended(batch);
+  return ns_workspace_bytes(batch, m, n, DA_BF16);
 }
 
 }  // extern "C"
@@ -732,7 +788,7 @@ int dion_amd_muon_step(void* const* X, const void* const* G, void* const* M, int
   const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful};
   for (int b0 = 0; b0 < batch; b0 += chunk) {
     const NsJob job = {G + b0, M + b0, X + b0, batch - b0 < chunk ? batch - b0 : chunk, m, n, n, n, decay, adjusted_lr};
-    const int rc = ns_jobs(&job, 1, call, workspace, s);
+    const int rc = ns_jobs(&job, 1, call, workspace, workspace_bytes, s);
     if (rc) return rc;
   }
   return DA_OK;
@@ -810,14 +866,19 @@ size_t dion_amd_muon_buckets_workspace_bytes(const dion_amd_muon_bucket* buckets
   if (!buckets || nbuckets <= 0) return 0;
   size_t worst = 0;
   for (int r0 = 0; r0 < nbuckets; r0 += DA_MAX_GROUPS) {
-    size_t need = 0;
+    size_t need = 0, need_small = 0;
     const int nr = nbuckets - r0 < DA_MAX_GROUPS ? nbuckets - r0 : DA_MAX_GROUPS;
-    const bool all256 = grid256(buckets + r0, nr, [](const dion_amd_muon_bucket& k) { return k.batch; });
-    for (int i = r0; i < r0 + nr; ++i) {
+    const auto count = [](const dion_amd_muon_bucket& k) { return k.batch; };
+    for (int i = r0; i < r0 + nr; ++i)
       if (buckets[i].batch <= 0 || buckets[i].m <= 0 || buckets[i].n <= 0) return 0;
-      need += align_up(NsLayout(buckets[i].m, buckets[i].n, DA_BF16, false, all256).per_matrix * (size_t)buckets[i].batch, 256);
+    const bool all256 = grid256(buckets + r0, nr, count);
+    for (int i = r0; i < r0 + nr; ++i) {
+      const dion_amd_muon_bucket& k = buckets[i];
+      need += align_up(NsLayout(k.m, k.n, DA_BF16, false, all256).per_matrix * (size_t)k.batch, 256);
+      need_small += align_up(NsLayout(k.m, k.n, DA_BF16, true).per_matrix * (size_t)k.batch, 256);
     }
     if (need > worst) worst = need;
+    if (need_small > worst && small_enough(buckets + r0, nr, count)) worst = need_small;
   }
   return worst;
 }
@@ -843,7 +904,7 @@ int dion_amd_muon_step_buckets(const dion_amd_muon_bucket* buckets, int nbuckets
       const dion_amd_muon_bucket& k = buckets[r0 + i];
       jobs[i] = NsJob{k.G, k.M, k.X, k.batch, k.m, k.n, k.n, k.n, k.decay, k.adjusted_lr};
     }
-    const int rc = ns_jobs(jobs, nr, call, workspace, static_cast<hipStream_t>(stream));
+    const int rc = ns_jobs(jobs, nr, call, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     if (rc) return rc;
   }
   return DA_OK;

@@ -386,3 +386,42 @@ def test_matrices_off_the_8_grid_may_start_anywhere(dev, shapes, dtype):
             shift, numel = b[k][0].storage_offset(), s[0] * s[1]
             new = b[k][1]
             assert torch.equal(new[:shift], old[k][:shift]) and torch.equal(new[shift + numel:], old[k][shift + numel:]), (s, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("buckets", [
+    [(300, 16, 1000), (300, 1000, 16), (8, 768, 768), (8, 72, 768)],      # thin buckets beside one in whole tiles
+    [(17, 1, 40000), (9, 136, 4096), (9, 4096, 136), (40, 9, 5001)],      # one row; just past the limit; off the 8-grid
+    [(48, 768, 768), (16, 768, 1024), (64, 24, 768)],                     # beside the persistent launch
+])
+def test_thin_matrices_in_a_large_call_equal_single_calls(dev, buckets, dtype):
+    """Matrices that padding to whole tiles would blow up keep the 8-grid and run in launches of their own, beside the padded
+    ones.  A matrix alone goes through the one-launch kernel on 64-tiles: the same products in the same order of k, so the weights
+    and momentum are the same bits."""
+    from dion_amd import Muon
+
+    gen = torch.Generator(device=dev).manual_seed(13)
+    X, G = [], []
+    for count, m, n in buckets:
+        X.append([(torch.randn(m, n, generator=gen, device=dev) * 0.02).to(dtype) for _ in range(count)])
+        G.append([(torch.randn(m, n, generator=gen, device=dev) * 1e-3).to(dtype) for _ in range(count)])
+
+    def step(xs, gs):
+        params = [torch.nn.Parameter(x.clone()) for x in xs]
+        opt = Muon(params, lr=0.02, mu=0.95, weight_decay=0.01, nesterov=True)
+        for _ in range(2):
+            for p, g in zip(params, gs):
+                p.grad = g
+            opt.step()
+        torch.cuda.synchronize()
+        return [(p.detach(), opt.state[p]["momentum"]) for p in params]
+
+    together = step(sum(X, []), sum(G, []))
+    at = 0
+    for (count, m, n), xs, gs in zip(buckets, X, G):
+        for k in (0, count - 1):
+            (x, mom), = step([xs[k]], [gs[k]])
+            assert torch.isfinite(x.float()).all() and not torch.equal(x, xs[k])
+            assert torch.equal(together[at + k][0], x), (m, n, k, "weights")
+            assert torch.equal(together[at + k][1], mom), (m, n, k, "momentum")
+        at += count

@@ -46,3 +46,50 @@ def test_matrices_on_the_8_grid_need_16_byte_alignment():
                                           BASE, 0, None) == want
         assert lib.dion_amd_muon_step(ptrs, ptrs, ptrs, 2, 32, 64, _lib.F32, _lib.F32, 0.9, 0, 1.0, 0.1, coeffs, 1, 1e-7, 1,
                                       BASE, 0, None) == want
+
+
+def _buckets(spec):
+    from dion_amd import _lib
+
+    arr = (_lib.MuonBucket * len(spec))()
+    for k, (batch, m, n) in zip(arr, spec):
+        k.batch, k.m, k.n = batch, m, n
+    return arr
+
+
+def _unpadded(batch, m, n):
+    """Two iterates and two Gram-sized matrices in bf16 with every dimension and pitch on the 8-grid (and off multiples of 4 KiB),
+    the partial sums and control words: what the iteration cannot do without, per bucket."""
+    m, n = sorted((-(-m // 8) * 8, -(-n // 8) * 8))
+    pitch = lambda k: k + (64 if k * 2 % 4096 == 0 else 0)
+    return batch * (2 * 2 * m * pitch(n) + 2 * 2 * m * pitch(m) + 4 * (m // 32 + 1) * (n // 64 + 2) + 4096)
+
+
+@pytest.mark.parametrize("spec", [
+    [(224, 16, 4096), (224, 4096, 16)],             # the factors of a low-rank adapter: 115 MiB, padded to tiles 939
+    [(224, 64, 4096), (224, 4096, 64)],
+    [(128, 136, 4096)], [(1600, 72, 72)], [(32, 24, 50000)], [(256, 8, 8192)],
+    [(48, 768, 768), (96, 16, 768)],                # beside a bucket on the tile grid
+    [(256, 300, 300)], [(24, 1096, 1096)], [(4, 648, 10000)], [(14, 341, 1021)],
+])
+def test_workspace_of_thin_matrices_is_not_a_multiple_of_their_own_size(spec):
+    """Padding to whole tiles may add 70 per cent to the working matrices, not a factor of eight (a call of more work than the
+    one-launch kernel takes)."""
+    from dion_amd import _lib
+
+    lib = _lib.load()
+    got = lib.dion_amd_muon_buckets_workspace_bytes(_buckets(spec), len(spec))
+    assert 0 < got <= 1.75 * sum(_unpadded(*k) for k in spec)
+
+
+def test_workspace_holds_either_layout():
+    """Few thin matrices go to the one-launch kernel, whose tiles are 64 wide: the queries make room for that."""
+    from dion_amd import _lib
+
+    lib = _lib.load()
+    tiles = 3 * 2 * (2 * 64 * 4096 + 2 * 64 * 64)
+    assert lib.dion_amd_muon_buckets_workspace_bytes(_buckets([(3, 16, 4096)]), 1) >= tiles
+    assert lib.dion_amd_ns_workspace_bytes(3, 16, 4096, _lib.BF16) >= tiles
+    assert lib.dion_amd_muon_workspace_bytes(3, 4096, 16) >= tiles
+    # one matrix of a batch that goes through in chunks
+    assert lib.dion_amd_ns_workspace_bytes(1, 16, 4096, _lib.F32) < 4 * 4 * 16 * 4096
