@@ -85,6 +85,10 @@ bool small_enough(const Bucket* k, int n, Count count) {
 
 constexpr size_t FLOW_TAIL_BYTES = 1536;   // behind the counters of a control area: ticket, owner and status words
 
+// The grid of the working matrices' dimensions: whole tiles of the batched products where padding pays, whole 64-tiles (the
+// one-launch kernel for small matrices, ns_small.hip), whole 256-tiles where padding pays (see grid256), or 16-byte chunks only.
+enum NsGrid { NS_TILES, NS_TILES64, NS_TILES256, NS_CHUNKS };
+
 struct NsLayout {
   int mw = 0, nw = 0, tiles = 0;
   int ldx = 0, lda = 0;   // row pitches of the mw x nw iterates and of the mw x mw Gram / polynomial
@@ -92,14 +96,12 @@ struct NsLayout {
   size_t x_bytes = 0, a_bytes = 0, part_bytes = 0, flow_bytes = 0;  // per matrix
   size_t per_matrix = 0;
   NsLayout() {}
-  // m x n matrices; `small`: the layout of the one-launch kernel for small matrices (ns_small.hip); `all256`: see grid256
-  NsLayout(int m, int n, int dtype, bool small = false, bool all256 = false) {
+  NsLayout(int m, int n, int dtype, NsGrid grid = NS_TILES) {
     mw = m < n ? m : n;
     nw = m < n ? n : m;
-    if (dtype != DA_BF16) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
-    else if (small) { mw = round_up(mw, DA_SMALL_BT); nw = round_up(nw, DA_SMALL_BT); }
-    else if (!padding_pays(mw, nw)) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
-    else if (all256) { mw = round_up(mw, 256); nw = round_up(nw, 256); }
+    if (dtype == DA_BF16 && grid == NS_TILES64) { mw = round_up(mw, DA_SMALL_BT); nw = round_up(nw, DA_SMALL_BT); }
+    else if (dtype != DA_BF16 || grid == NS_CHUNKS || !padding_pays(mw, nw)) { mw = round_up(mw, 8); nw = round_up(nw, 8); }
+    else if (grid == NS_TILES256) { mw = round_up(mw, 256); nw = round_up(nw, 256); }
     else { mw = padded_dim(mw); nw = padded_dim(nw); }
     tiles = da_stage_tiles(m, n, mw, nw);
     esz = dtype == DA_BF16 ? 2 : 4;
@@ -137,7 +139,7 @@ size_t ns_workspace_bytes(int batch, int m, int n, int dtype) {
   size_t bytes = c * L.per_matrix;
   struct { int m, n; } shape = {m, n};
   if (dtype == DA_BF16 && small_enough(&shape, 1, [&](const decltype(shape)&) { return (int)c; })) {
-    const size_t small = align_up(NsLayout(m, n, dtype, true).per_matrix * c, 256);
+    const size_t small = align_up(NsLayout(m, n, dtype, NS_TILES64).per_matrix * c, 256);
     bytes = bytes > small ? bytes : small;
   }
   return bytes;
@@ -328,6 +330,7 @@ struct NsCall {
   int steps;
   float eps;
   int faithful;
+  NsGrid grid;                           // NS_TILES, or NS_CHUNKS for a workspace that holds no padded matrix
 };
 
 // The iterations of `n` of the staged and normalised sets, and what becomes of their results.
@@ -399,7 +402,7 @@ bool ns_small_wanted(const NsJob* jobs, int nj, const NsCall& c, size_t workspac
   // (a workspace sized by the queries holds this layout; a smaller one that holds the other takes the batched launches)
   size_t need = 0;
   for (int i = 0; i < nj; ++i)
-    need += align_up(NsLayout(jobs[i].m, jobs[i].n, c.compute_dtype, true).per_matrix * (size_t)jobs[i].cnt, 256);
+    need += align_up(NsLayout(jobs[i].m, jobs[i].n, c.compute_dtype, NS_TILES64).per_matrix * (size_t)jobs[i].cnt, 256);
   return need <= workspace_bytes;
 }
 
@@ -414,7 +417,7 @@ int ns_jobs(const NsJob* jobs, int nj, const NsCall& c, void* workspace, size_t 
   for (int i = 0; i < nj; ++i) {
     const NsJob& k = jobs[i];
     NsSet& S = sets[i];
-    S.L = NsLayout(k.m, k.n, c.compute_dtype, small, all256);
+    S.L = NsLayout(k.m, k.n, c.compute_dtype, small ? NS_TILES64 : (all256 ? NS_TILES256 : c.grid));
     S.W = NsBuffers(S.L, p, k.cnt);
     S.cb = k.cnt;
     S.update = c.update; S.x_dtype = c.x_dtype; S.tall = k.m > k.n ? 1 : 0; S.x_ld = k.ldx; S.decay = k.decay; S.step = k.step;
@@ -592,7 +595,7 @@ namespace {
 
 int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, long long out_stride, int ldo,
            int batch, int m, int n, const float* coeffs, int steps, float eps, int compute_dtype, int faithful,
-           void* workspace, size_t workspace_bytes, void* stream) {
+           void* workspace, size_t workspace_bytes, void* stream, NsGrid grid = NS_TILES) {
   if (!G || !out || !coeffs || !workspace || batch <= 0 || m <= 0 || n <= 0 || steps < 0) return DA_ERR_ARG;
   if (!dtype_ok(g_dtype) || !dtype_ok(compute_dtype)) return DA_ERR_DTYPE;
   const size_t gsz = g_dtype == DA_BF16 ? 2 : 4, osz = compute_dtype == DA_BF16 ? 2 : 4;
@@ -604,10 +607,10 @@ int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, l
   if (misaligned(G, g_chunks && !(m & 7), gsz) || misaligned(out, o_chunks && !(m & 7), osz)) return DA_ERR_ALIGN;
   if ((uintptr_t)workspace & 255) return DA_ERR_ALIGN;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const NsLayout L(m, n, compute_dtype);
+  const NsLayout L(m, n, compute_dtype, grid);
   const int chunk = L.chunk(batch, workspace_bytes);
   if (chunk < 1) return DA_ERR_WORKSPACE;
-  const NsCall call = {compute_dtype, g_dtype, compute_dtype, 0, 0.f, 0, coeffs, steps, eps, faithful};
+  const NsCall call = {compute_dtype, g_dtype, compute_dtype, 0, 0.f, 0, coeffs, steps, eps, faithful, grid};
   for (int b0 = 0; b0 < batch; b0 += chunk) {
     const int cb = batch - b0 < chunk ? batch - b0 : chunk;
     const void* src[DA_MAX_PTRS];
@@ -626,7 +629,10 @@ int ns_run(const void* G, int g_dtype, long long g_stride, int ldg, void* out, l
 // Working memory of dion_amd_newton_schulz_static: one array per GPU, part of the library's device image (it lives
 // as long as the process).  Host code never uses the array's name as an address: `static_scratch()` asks the
 // runtime for the device address on the current GPU, once per device, and hands that pointer on.
-static __device__ __align__(256) unsigned char scratch[DION_AMD_STATIC_SCRATCH_BYTES];
+// The announced size is for the matrices: the control words of the one-launch kernels, 1280 bytes a matrix beyond the
+// persistent kernel's, come on top.
+constexpr size_t SCRATCH_BYTES = DION_AMD_STATIC_SCRATCH_BYTES + FLOW_TAIL_BYTES - 256;
+static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 constexpr int DA_MAX_DEVICES = 64;
 void* g_scratch_ptr[DA_MAX_DEVICES];
 std::mutex g_scratch_mutex;
@@ -664,13 +670,16 @@ int dion_amd_newton_schulz_static(const void* G, int g_dtype, long long g_stride
                                   int steps, float eps, int compute_dtype, int faithful, void* stream) {
   if (batch <= 0 || m <= 0 || n <= 0) return DA_ERR_ARG;
   if (!dtype_ok(compute_dtype)) return DA_ERR_DTYPE;
-  // one matrix's working set must fit the array (a batch then goes through it in chunks)
-  if (NsLayout(m, n, compute_dtype).per_matrix > (size_t)DION_AMD_STATIC_SCRATCH_BYTES) return DA_ERR_LIMIT;
+  // one matrix's working set must fit the array (a batch then goes through it in chunks): padded to whole tiles, or else
+  // without padding (648 x 10000: 32.4 MiB and 26.3)
+  NsGrid grid = NS_TILES;
+  if (NsLayout(m, n, compute_dtype).per_matrix > SCRATCH_BYTES) grid = NS_CHUNKS;
+  if (NsLayout(m, n, compute_dtype, grid).per_matrix > SCRATCH_BYTES) return DA_ERR_LIMIT;
   void* ws = nullptr;
   const int rc = static_scratch(&ws);
   if (rc) return rc;
   return ns_run(G, g_dtype, g_stride, ldg, out, out_stride, ldo, batch, m, n, coeffs, steps, eps, compute_dtype,
-                faithful, ws, DION_AMD_STATIC_SCRATCH_BYTES, stream);
+                faithful, ws, SCRATCH_BYTES, stream, grid);
 }
 
 int dion_amd_syrk(const void* A, long long a_stride, int lda, void* C, long long c_stride, int ldc, int batch, int m,
@@ -785,7 +794,7 @@ int dion_amd_muon_step(void* const* X, const void* const* G, void* const* M, int
   const NsLayout L(m, n, DA_BF16);
   const int chunk = L.chunk(batch, workspace_bytes);
   if (chunk < 1) return DA_ERR_WORKSPACE;
-  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful};
+  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful, NS_TILES};
   for (int b0 = 0; b0 < batch; b0 += chunk) {
     const NsJob job = {G + b0, M + b0, X + b0, batch - b0 < chunk ? batch - b0 : chunk, m, n, n, n, decay, adjusted_lr};
     const int rc = ns_jobs(&job, 1, call, workspace, workspace_bytes, s);
@@ -874,8 +883,8 @@ size_t dion_amd_muon_buckets_workspace_bytes(const dion_amd_muon_bucket* buckets
     const bool all256 = grid256(buckets + r0, nr, count);
     for (int i = r0; i < r0 + nr; ++i) {
       const dion_amd_muon_bucket& k = buckets[i];
-      need += align_up(NsLayout(k.m, k.n, DA_BF16, false, all256).per_matrix * (size_t)k.batch, 256);
-      need_small += align_up(NsLayout(k.m, k.n, DA_BF16, true).per_matrix * (size_t)k.batch, 256);
+      need += align_up(NsLayout(k.m, k.n, DA_BF16, all256 ? NS_TILES256 : NS_TILES).per_matrix * (size_t)k.batch, 256);
+      need_small += align_up(NsLayout(k.m, k.n, DA_BF16, NS_TILES64).per_matrix * (size_t)k.batch, 256);
     }
     if (need > worst) worst = need;
     if (need_small > worst && small_enough(buckets + r0, nr, count)) worst = need_small;
@@ -896,7 +905,7 @@ int dion_amd_muon_step_buckets(const dion_amd_muon_bucket* buckets, int nbuckets
     if (rc) return rc;
   }
   if (workspace_bytes < dion_amd_muon_buckets_workspace_bytes(buckets, nbuckets)) return DA_ERR_WORKSPACE;
-  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful};
+  const NsCall call = {x_dtype, g_dtype, DA_BF16, 1, mu, nesterov, coeffs, steps, eps, faithful, NS_TILES};
   for (int r0 = 0; r0 < nbuckets; r0 += DA_MAX_GROUPS) {
     const int nr = nbuckets - r0 < DA_MAX_GROUPS ? nbuckets - r0 : DA_MAX_GROUPS;
     NsJob jobs[DA_MAX_GROUPS];

@@ -93,3 +93,28 @@ def test_workspace_holds_either_layout():
     assert lib.dion_amd_muon_workspace_bytes(3, 4096, 16) >= tiles
     # one matrix of a batch that goes through in chunks
     assert lib.dion_amd_ns_workspace_bytes(1, 16, 4096, _lib.F32) < 4 * 4 * 16 * 4096
+
+
+@pytest.mark.parametrize("m,n", [
+    (648, 10000), (10000, 648), (640, 10000),
+    # working sets without padding within a kilobyte of the array
+    (200, 41736), (232, 35920), (400, 20568), (536, 15112), (616, 13000), (1072, 6752), (1232, 5576), (1304, 5128),
+])
+def test_static_newton_schulz_takes_what_fits_without_padding(m, n):
+    """The working set that has to fit the array is the one on the 8-grid: 26.3 MiB for 648 x 10000, which padding makes 32.4.
+    (A misaligned source: the call ends at that check, or here at the missing GPU, and nothing is launched.)"""
+    from dion_amd import _lib
+
+    coeffs = _lib.float_array([1.0, 1.0, 1.0])
+    args = (BASE + 1, _lib.BF16, m * n, n, BASE, m * n, n, 1, m, n, coeffs, 1, 1e-7, _lib.BF16, 1, None)
+    rc = _lib.load().dion_amd_newton_schulz_static(*args)
+    assert rc == ALIGN or rc > 0, rc
+
+
+@pytest.mark.parametrize("m,n", [(4096, 4096), (648, 13000), (64, 200000)])
+def test_static_newton_schulz_refuses_what_does_not_fit(m, n):
+    from dion_amd import _lib
+
+    coeffs = _lib.float_array([1.0, 1.0, 1.0])
+    args = (BASE + 1, _lib.BF16, m * n, n, BASE, m * n, n, 1, m, n, coeffs, 1, 1e-7, _lib.BF16, 1, None)
+    assert _lib.load().dion_amd_newton_schulz_static(*args) == -5

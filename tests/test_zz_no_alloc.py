@@ -65,3 +65,13 @@ def test_static_newton_schulz_rejects_what_does_not_fit(dev):
     assert bool((out == 7.0).all())   # nothing was launched
     with pytest.raises(_lib.DionAmdError, match="limit"):
         _lib.check(rc, "dion_amd_newton_schulz_static")
+
+
+@pytest.mark.parametrize("m,n", [(648, 10000), (9990, 641), (16, 200000)])
+def test_static_newton_schulz_without_padding(dev, m, n):
+    """A matrix that fits the array only without padding to whole tiles: the products add the same terms in the same order."""
+    from dion_amd import _lib
+
+    G = torch.randn((2, m, n), generator=torch.Generator(device=dev).manual_seed(10), device=dev).bfloat16()
+    got, ref = _both(_lib.load(), _lib, G, torch.bfloat16, dev)
+    assert torch.isfinite(got.float()).all() and torch.equal(got, ref)
