@@ -24,7 +24,7 @@ from typing import Any, Dict, Optional, Tuple
 
 import torch
 from torch import Tensor
-from torch.optim.optimizer import Optimizer, ParamsT
+from torch.optim.optimizer import ParamsT
 
 from . import _lib
 from .elementwise_opts import element_groups_step
@@ -46,7 +46,7 @@ def _enqueue_dion_step(fn, device, args):
     return fn(*args)
 
 
-class Dion(Optimizer):
+class Dion(_lib.HookedOptimizer):
     _REFERENCE_OPTIONS = False   # True in DionReference: power_iters >= 1 and all three qr_method names
     """
     Dion (https://arxiv.org/abs/2504.05295) for a single MI355X.
@@ -142,13 +142,8 @@ class Dion(Optimizer):
         self._pool = None   # worker threads that enqueue the buckets of a wave side by side
         self._rng = None    # generator of the random sketches (DionReference with qr_method "rcqr")
 
-    def step(self, closure=None):
-        return _lib.run_step(self, Dion._step, closure)
-
-    step.hooked = True   # (the hooks and the profiler range of `Optimizer` are run_step's)
-
     @torch.no_grad()
-    def _step(self, closure=None):
+    def step(self, closure=None):
         loss = None
         if closure is not None:
             with torch.enable_grad():

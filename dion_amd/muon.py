@@ -18,7 +18,7 @@ from typing import Callable, Optional, Tuple
 
 import torch
 from torch import Tensor
-from torch.optim.optimizer import Optimizer, ParamsT
+from torch.optim.optimizer import ParamsT
 
 from . import _lib
 from .elementwise_opts import element_groups_step
@@ -51,7 +51,7 @@ _ADJUST = {
 _ADJUST_CODE = {None: 0, "spectral_norm": 1, "rms_norm": 2, "keller_muon": 3}   # of _host.muon_group
 
 
-class Muon(Optimizer):
+class Muon(_lib.HookedOptimizer):
     """
     Muon for a single MI355X.
 
@@ -118,11 +118,6 @@ class Muon(Optimizer):
         self._coeffs = flat_coeffs(NS_SCHEDULE_COEFFS)
 
     def step(self, closure=None):
-        return _lib.run_step(self, Muon._step, closure)
-
-    step.hooked = True   # (the hooks and the profiler range of `Optimizer` are run_step's)
-
-    def _step(self, closure=None):
         loss = None
         if closure is not None:
             with torch.enable_grad():

@@ -118,3 +118,89 @@ def test_static_newton_schulz_refuses_what_does_not_fit(m, n):
     coeffs = _lib.float_array([1.0, 1.0, 1.0])
     args = (BASE + 1, _lib.BF16, m * n, n, BASE, m * n, n, 1, m, n, coeffs, 1, 1e-7, _lib.BF16, 1, None)
     assert _lib.load().dion_amd_newton_schulz_static(*args) == -5
+
+
+# ------------------------------------------------------------------ step hooks
+def _optimizers():
+    from dion_amd import Dion, DionReference, Muon
+
+    return [Muon, Dion, DionReference]
+
+
+def _record(opt):
+    seen = []
+    opt.register_step_pre_hook(lambda o, args, kwargs: seen.append(("pre", args, kwargs)))
+    opt.register_step_post_hook(lambda o, args, kwargs: seen.append(("post", args, kwargs)))
+    return seen
+
+
+def _parameters():
+    return [torch.nn.Parameter(torch.zeros(8, 8))]     # without gradients: a step has nothing to do
+
+
+@pytest.mark.parametrize("cls", _optimizers())
+@pytest.mark.parametrize("plain_first", [False, True])
+def test_step_hooks_run_once_in_a_subclass(cls, plain_first):
+    """A subclass whose step() calls super().step(): hooks act once per step, whether or not the class itself has been
+    instantiated before, and through as many levels as there are."""
+    class Mine(cls):
+        def step(self, closure=None):
+            return super().step(closure)
+
+    class Deeper(Mine):
+        def step(self, closure=None):
+            return super().step(closure=closure)
+
+    class Inherits(Deeper):
+        pass
+
+    if plain_first:
+        cls(_parameters()).step()
+    for kind in (Mine, Deeper, Inherits, cls):
+        opt = kind(_parameters())
+        seen = _record(opt)
+        for n in (1, 2):
+            assert opt.step() is None
+            assert [s[0] for s in seen] == ["pre", "post"] * n, kind
+        assert opt.param_groups[0]["step"] == 2
+        with pytest.raises(ZeroDivisionError):
+            opt.step(lambda: 1 / 0)
+        del seen[:]
+        assert opt.step(lambda: 7) == 7                 # an exception leaves nothing behind
+        assert [s[0] for s in seen] == ["pre", "post"], kind
+
+
+@pytest.mark.parametrize("cls", _optimizers())
+def test_step_hooks_get_the_arguments_of_the_call(cls):
+    """As torch's own optimizers hand them on."""
+    closure = lambda: None
+    calls = [lambda o: o.step(), lambda o: o.step(closure), lambda o: o.step(closure=closure)]
+    want, got = [], []
+    for kind, out in ((torch.optim.SGD, want), (cls, got)):
+        opt = kind(_parameters(), lr=0.1)
+        seen = _record(opt)
+        for call in calls:
+            call(opt)
+        out += [(when, len(args), args[1:], kwargs, args[0] is opt) for when, args, kwargs in seen]
+    assert got == want
+
+
+@pytest.mark.parametrize("cls", _optimizers())
+def test_global_hooks_and_the_profiler_see_every_step(cls):
+    from torch.optim.optimizer import register_optimizer_step_post_hook, register_optimizer_step_pre_hook
+
+    opt, seen = cls(_parameters()), []
+    handles = [register_optimizer_step_pre_hook(lambda o, a, k: seen.append("pre")),
+               register_optimizer_step_post_hook(lambda o, a, k: seen.append("post"))]
+    opt.step()
+    for h in handles:
+        h.remove()
+    opt.step()
+    assert seen == ["pre", "post"]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        opt.step()
+    assert [e.name for e in prof.events()].count(f"Optimizer.step#{cls.__name__}.step") == 1
+    scheduler = torch.optim.lr_scheduler.LambdaLR(opt, lambda epoch: 1.0)     # (it wraps the bound method)
+    opt.step()
+    scheduler.step()
+    assert opt.param_groups[0]["step"] == 4
