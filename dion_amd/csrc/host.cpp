@@ -57,14 +57,23 @@ struct Entry {
   at::Tensor s[2];
 };
 
-// The parameters of `params` that have a gradient, with the state tensors named `keys`.  Appends the parameters without
-// state to `missing` (a Python list) instead.
+// A reference of our own; null: a Python exception is set.
+struct Ref {
+  PyObject* p;
+  explicit Ref(PyObject* o) : p(o) { if (!p) throw Failed(); }
+  ~Ref() { Py_DECREF(p); }
+  Ref(const Ref&) = delete;
+  Ref& operator=(const Ref&) = delete;
+};
+
+// The parameters of `params` (a tuple) that have a gradient, with the state tensors named `keys`.  Appends the parameters
+// without state to `missing` (a Python list) instead.
 void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys, std::vector<Entry>& out, PyObject* missing,
             std::vector<PyObject*>* objects = nullptr) {
-  const Py_ssize_t n = PyList_GET_SIZE(params);
+  const Py_ssize_t n = PyTuple_GET_SIZE(params);
   out.reserve((size_t)n);
   for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject* o = PyList_GET_ITEM(params, i);
+    PyObject* o = PyTuple_GET_ITEM(params, i);
     if (!THPVariable_Check(o)) {
       PyErr_SetString(PyExc_TypeError, "parameters must be tensors");
       throw Failed();
@@ -153,10 +162,11 @@ PyObject* muon_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
     const int steps = (int)PyLong_AsLong(a[10]);
     if (PyErr_Occurred()) return nullptr;
     at::NoGradGuard no_grad;
+    const Ref params(PySequence_Tuple(a[0]));   // (any collection; it keeps them while this call lasts)
     missing = PyList_New(0);
     if (!missing) return nullptr;
     std::vector<Entry> all;
-    gather(a[0], a[1], &s_momentum, 1, all, missing);
+    gather(params.p, a[1], &s_momentum, 1, all, missing);
     if (PyList_GET_SIZE(missing)) return missing;
     Py_CLEAR(missing);
 
@@ -252,12 +262,13 @@ PyObject* dion_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
                 eps = (float)PyFloat_AsDouble(a[5]);
     if (PyErr_Occurred()) return nullptr;
     at::NoGradGuard no_grad;
+    const Ref params(PySequence_Tuple(a[0]));
     missing = PyList_New(0);
     if (!missing) return nullptr;
     std::vector<Entry> all;
     std::vector<PyObject*> objects;
     PyObject* const keys[2] = {s_momentum, s_q};
-    gather(a[0], a[1], keys, 2, all, missing, &objects);
+    gather(params.p, a[1], keys, 2, all, missing, &objects);
     if (PyList_GET_SIZE(missing)) return missing;
     Py_CLEAR(missing);
 
@@ -434,11 +445,12 @@ PyObject* element_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
     Scalars s;
     if (!scalars(a + 3, s)) return nullptr;
     at::NoGradGuard no_grad;
+    const Ref params(PySequence_Tuple(a[1]));
     missing = PyList_New(0);
     if (!missing) return nullptr;
     std::vector<Entry> all;
     PyObject* const keys[2] = {s_momentum, s_variance};
-    gather(a[1], a[2], keys, adamw ? 2 : 1, all, missing);
+    gather(params.p, a[2], keys, adamw ? 2 : 1, all, missing);
     if (PyList_GET_SIZE(missing)) return missing;
     Py_CLEAR(missing);
     elementwise_run(adamw, all, adamw ? "adamw_update_foreach" : "lion_update_foreach", s.lr, s.b1, s.b2, s.wd, s.step, s.eps);
@@ -460,6 +472,11 @@ PyObject* element_lists(PyObject*, PyObject* const* a, Py_ssize_t na) {
     Scalars s;
     if (!scalars(a + 5, s)) return nullptr;
     at::NoGradGuard no_grad;
+    for (int k = 0; k < (adamw ? 4 : 3); ++k)
+      if (!PyList_Check(a[1 + k]) || PyList_GET_SIZE(a[1 + k]) != PyList_GET_SIZE(a[1])) {
+        PyErr_SetString(PyExc_TypeError, "expected lists of equal length");
+        return nullptr;
+      }
     const Py_ssize_t n = PyList_GET_SIZE(a[1]);
     std::vector<Entry> all((size_t)n);
     for (Py_ssize_t i = 0; i < n; ++i) {

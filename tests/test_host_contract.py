@@ -204,3 +204,32 @@ def test_global_hooks_and_the_profiler_see_every_step(cls):
     opt.step()
     scheduler.step()
     assert opt.param_groups[0]["step"] == 4
+
+
+# ------------------------------------------------------------------ what the native module is handed
+def _groups():
+    """One optimizer for every road through the native module: Muon, Dion and both element-wise algorithms."""
+    from dion_amd import Dion, Muon
+
+    return [(Muon, "muon"), (Muon, "lion"), (Muon, "adamw"), (Dion, "dion"), (Dion, "lion"), (Dion, "adamw")]
+
+
+@pytest.mark.parametrize("cls,algorithm", _groups())
+@pytest.mark.parametrize("kind", [tuple, list, lambda ps: dict.fromkeys(ps)])
+def test_parameters_of_a_group_may_be_any_collection(cls, algorithm, kind):
+    """`group["params"]` is walked, not assumed to be a list."""
+    from dion_amd import _lib
+
+    params = [torch.nn.Parameter(torch.zeros(8, 8)) for _ in range(5)]
+    opt = cls([dict(params=params, algorithm=algorithm)])
+    opt.param_groups[0]["params"] = kind(params)
+    opt.step()                                    # no gradients: nothing to do
+    params[3].grad = torch.zeros(8, 8)
+    with pytest.raises(_lib.DionAmdError, match="tensor is on cpu"):
+        opt.step()
+    assert list(opt.state) == [params[3]]
+    opt.param_groups[0]["params"] = kind([])
+    opt.step()
+    opt.param_groups[0]["params"] = 3
+    with pytest.raises(TypeError):
+        opt.step()
