@@ -195,6 +195,12 @@ def require_gpu(t, what):
         )
 
 
+def require_states(missing, what):
+    """`missing`: None, or the parameters that the host module still found without a state after it was created."""
+    if missing is not None:
+        raise DionAmdError(f"{what}: the optimizer state of {len(missing)} parameter(s) is empty after its initialisation")
+
+
 def stream_ptr(device=None):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 

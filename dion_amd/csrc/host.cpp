@@ -61,10 +61,32 @@ struct Entry {
 struct Ref {
   PyObject* p;
   explicit Ref(PyObject* o) : p(o) { if (!p) throw Failed(); }
-  ~Ref() { Py_DECREF(p); }
+  Ref(Ref&& o) : p(o.p) { o.p = nullptr; }
+  ~Ref() { Py_XDECREF(p); }
   Ref(const Ref&) = delete;
   Ref& operator=(const Ref&) = delete;
 };
+
+// map[key] for a dict or any other mapping; `none` (borrowed) where there is no such key.
+Ref lookup(PyObject* map, PyObject* key, PyObject* none) {
+  PyObject* v;
+  if (PyDict_Check(map)) {
+    v = PyDict_GetItemWithError(map, key);
+    Py_XINCREF(v);
+    if (!v && PyErr_Occurred()) throw Failed();
+  } else {
+    v = PyObject_GetItem(map, key);
+    if (!v) {
+      if (!PyErr_ExceptionMatches(PyExc_KeyError)) throw Failed();
+      PyErr_Clear();
+    }
+  }
+  if (!v) {
+    v = none;
+    Py_INCREF(v);
+  }
+  return Ref(v);
+}
 
 // The parameters of `params` (a tuple) that have a gradient, with the state tensors named `keys`.  Appends the parameters
 // without state to `missing` (a Python list) instead.
@@ -81,9 +103,10 @@ void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys,
     const at::Tensor& p = THPVariable_Unpack(o);
     const at::Tensor& g = p.grad();
     if (!g.defined()) continue;
-    PyObject* st = PyDict_GetItemWithError(state, o);
-    if (!st && PyErr_Occurred()) throw Failed();
-    if (!st || !PyDict_Check(st) || PyDict_GET_SIZE(st) == 0) {
+    const Ref st = lookup(state, o, Py_None);
+    const int there = PyObject_IsTrue(st.p);   // (an empty state, as `Optimizer.state` makes them, is to be filled)
+    if (there < 0) throw Failed();
+    if (!there) {
       if (PyList_Append(missing, o)) throw Failed();
       continue;
     }
@@ -93,12 +116,12 @@ void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys,
     e.p = p;
     e.g = g;
     for (int k = 0; k < nkeys; ++k) {
-      PyObject* t = PyDict_GetItemWithError(st, keys[k]);
-      if (!t || !THPVariable_Check(t)) {
-        if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, keys[k]);
+      const Ref t = lookup(st.p, keys[k], Py_None);
+      if (!THPVariable_Check(t.p)) {
+        PyErr_SetObject(PyExc_KeyError, keys[k]);
         throw Failed();
       }
-      e.s[k] = THPVariable_Unpack(t);
+      e.s[k] = THPVariable_Unpack(t.p);
     }
   }
 }

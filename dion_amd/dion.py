@@ -260,6 +260,8 @@ class Dion(_lib.HookedOptimizer):
             for p in left:
                 self._get_or_initialize_state(p, group)
             left = host.dion_group(*args)
+            if isinstance(left, list):
+                _lib.require_states(left, "Dion.step")
         if left:
             self._dion_params_step(group, left)
 

@@ -46,4 +46,4 @@ def element_groups_step(opt, groups, adamw):
         if missing is not None:
             for p in missing:
                 opt._new_state(p, members[0])
-            host.element_group(*args)
+            _lib.require_states(host.element_group(*args), f"{type(opt).__name__}.step")

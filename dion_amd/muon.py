@@ -176,7 +176,7 @@ class Muon(_lib.HookedOptimizer):
         if missing is not None:
             for p in missing:
                 self._new_state(p, group)
-            host.muon_group(*args)
+            _lib.require_states(host.muon_group(*args), "Muon.step")
 
     def _muon_group_unfused(self, group: dict):
         # hyper-parameters as 0-dim fp32 tensors, evaluated like reference dion/muon.py:205-208

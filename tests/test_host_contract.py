@@ -233,3 +233,41 @@ def test_parameters_of_a_group_may_be_any_collection(cls, algorithm, kind):
     opt.param_groups[0]["params"] = 3
     with pytest.raises(TypeError):
         opt.step()
+
+
+@pytest.mark.parametrize("cls,algorithm", _groups())
+def test_a_state_that_stays_missing_is_an_error(cls, algorithm):
+    """A parameter whose state is not there after it was asked for is not skipped in silence."""
+    from dion_amd import _lib
+
+    class Forgets(cls):
+        def _get_or_initialize_state(self, param, algo):
+            return {}
+
+    p = torch.nn.Parameter(torch.zeros(8, 8))
+    p.grad = torch.zeros(8, 8)
+    opt = Forgets([dict(params=[p], algorithm=algorithm)])
+    with pytest.raises(_lib.DionAmdError, match="state"):
+        opt.step()
+
+
+@pytest.mark.parametrize("cls,algorithm", _groups())
+def test_a_state_may_be_any_mapping(cls, algorithm):
+    """What is not a dict is asked for its tensors like one; one that lacks a tensor is a KeyError."""
+    from collections import UserDict
+
+    from dion_amd import _lib
+
+    p = torch.nn.Parameter(torch.zeros(8, 8))
+    p.grad = torch.zeros(8, 8)
+    opt = cls([dict(params=[p], algorithm=algorithm)])
+    for state in (UserDict, dict):
+        opt.state[p] = state(momentum=torch.zeros(8, 8), variance=torch.zeros(8, 8), Q=torch.zeros(8, 8))
+        with pytest.raises(_lib.DionAmdError, match="tensor is on cpu"):
+            opt.step()
+        opt.state[p] = state(other=torch.zeros(8, 8))
+        with pytest.raises(KeyError, match="momentum"):
+            opt.step()
+    opt.state = UserDict({p: dict(momentum=torch.zeros(8, 8), variance=torch.zeros(8, 8), Q=torch.zeros(8, 8))})
+    with pytest.raises(_lib.DionAmdError, match="tensor is on cpu"):
+        opt.step()
