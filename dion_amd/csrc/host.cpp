@@ -195,6 +195,10 @@ PyObject* muon_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
 
     std::vector<MuonBucket> buckets;
     for (Entry& e : all) {
+      // (the library reads as many elements of the gradient and the momentum as the parameter has, the momentum in its dtype)
+      if (e.s[0].numel() != e.p.numel() || e.s[0].scalar_type() != e.p.scalar_type() || e.s[0].device() != e.p.device() ||
+          e.g.numel() != e.p.numel() || e.g.device() != e.p.device())
+        fail("Muon.step: gradient and momentum do not fit their parameter");
       MuonBucket* b = nullptr;
       for (MuonBucket& c : buckets)
         if (c.p0.sizes().equals(e.p.sizes()) && c.p0.scalar_type() == e.p.scalar_type() && c.gtype == e.g.scalar_type() &&

@@ -271,3 +271,29 @@ def test_a_state_may_be_any_mapping(cls, algorithm):
     opt.state = UserDict({p: dict(momentum=torch.zeros(8, 8), variance=torch.zeros(8, 8), Q=torch.zeros(8, 8))})
     with pytest.raises(_lib.DionAmdError, match="tensor is on cpu"):
         opt.step()
+
+
+@pytest.mark.parametrize("shape,flatten,momentum", [
+    ((8, 16), False, (8, 8)), ((8, 16), False, (8, 32)), ((3, 8, 16), False, (2, 8, 16)), ((3, 8, 16), True, (3, 8)),
+    ((4, 8), False, (0, 8)),
+])
+def test_muon_refuses_a_momentum_of_another_size(shape, flatten, momentum):
+    """A buffer that is not as large as its parameter would be read and written out of its bounds."""
+    from dion_amd import Muon, _lib
+
+    p = torch.nn.Parameter(torch.zeros(shape))
+    p.grad = torch.zeros(shape)
+    opt = Muon([p], flatten=flatten)
+    opt.state[p]["momentum"] = torch.zeros(momentum)
+    with pytest.raises(_lib.DionAmdError, match="do not fit"):
+        opt.step()
+    opt.state[p]["momentum"] = torch.zeros(shape, dtype=torch.bfloat16)      # half the bytes
+    with pytest.raises(_lib.DionAmdError, match="do not fit"):
+        opt.step()
+    opt.state[p]["momentum"] = torch.zeros(p.numel()).view(shape)
+    with pytest.raises(_lib.DionAmdError, match="tensor is on cpu"):
+        opt.step()
+    p.data = torch.zeros((2 * shape[0],) + shape[1:])                        # the gradient is the old one's
+    opt.state[p]["momentum"] = torch.zeros(p.shape)
+    with pytest.raises(_lib.DionAmdError, match="do not fit"):
+        opt.step()
