@@ -51,6 +51,13 @@ void check(int rc, const char* what) {
   throw Failed();
 }
 
+// The interpreter lock is released while the library is called (argument checks, pointer tables and launches, 5 to 50 us):
+// other threads of the program run meanwhile.  Whatever the call is handed is held by references of the caller's own.
+struct Unlocked {
+  PyThreadState* saved = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(saved); }
+};
+
 // One parameter with its gradient and its states.
 struct Entry {
   at::Tensor p, g;
@@ -127,25 +134,17 @@ void gather(PyObject* params, PyObject* state, PyObject* const* keys, int nkeys,
 }
 
 // `nbytes` of workspace on `dev` from a _lib.Workspace
-char* workspace(PyObject* ws, size_t nbytes, c10::Device dev) {
-  PyObject* buf = PyObject_GetAttr(ws, s_buf);
-  if (!buf) throw Failed();
-  char* p = nullptr;
-  if (THPVariable_Check(buf)) {
-    const at::Tensor& t = THPVariable_Unpack(buf);
-    if ((size_t)t.numel() >= nbytes && t.device() == dev) p = static_cast<char*>(t.data_ptr());
+at::Tensor workspace(PyObject* ws, size_t nbytes, c10::Device dev) {
+  {
+    const Ref buf(PyObject_GetAttr(ws, s_buf));
+    if (THPVariable_Check(buf.p)) {
+      const at::Tensor& t = THPVariable_Unpack(buf.p);
+      if ((size_t)t.numel() >= nbytes && t.device() == dev) return t;
+    }
   }
-  Py_DECREF(buf);
-  if (p) return p;
-  PyObject* d = THPDevice_New(dev);
-  PyObject* n = PyLong_FromSize_t(nbytes);
-  PyObject* t = d && n ? PyObject_CallMethodObjArgs(ws, s_get, n, d, nullptr) : nullptr;
-  Py_XDECREF(d);
-  Py_XDECREF(n);
-  if (!t) throw Failed();
-  p = static_cast<char*>(THPVariable_Unpack(t).data_ptr());
-  Py_DECREF(t);   // (the workspace object holds it)
-  return p;
+  const Ref d(THPDevice_New(dev)), n(PyLong_FromSize_t(nbytes));
+  const Ref t(PyObject_CallMethodObjArgs(ws, s_get, n.p, d.p, nullptr));
+  return THPVariable_Unpack(t.p);
 }
 
 void* stream_of(c10::Device dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
@@ -253,10 +252,15 @@ PyObject* muon_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
       const c10::Device dev = f.p0.device();
       const int xc = dtype_code(f.p0.scalar_type()), gc = dtype_code(f.gtype);
       const size_t need = api.muon_bytes(call.data(), (int)call.size());
-      char* ws = workspace(a[11], need, dev);
+      const at::Tensor ws = workspace(a[11], need, dev);
       const c10::DeviceGuard guard(dev);
-      check(api.muon_step(call.data(), (int)call.size(), xc, gc, mu, nesterov, coeffs, steps, eps, 1, ws, need, stream_of(dev)),
-            "dion_amd_muon_step_buckets");
+      int rc;
+      {
+        const Unlocked unlocked;
+        rc = api.muon_step(call.data(), (int)call.size(), xc, gc, mu, nesterov, coeffs, steps, eps, 1, ws.data_ptr(), need,
+                           stream_of(dev));
+      }
+      check(rc, "dion_amd_muon_step_buckets");
     }
     Py_RETURN_NONE;
   } catch (const Failed&) {
@@ -335,6 +339,7 @@ PyObject* dion_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
     std::vector<char> done(buckets.size(), 0);
     std::vector<dion_amd_dion_bucket> call;
     std::vector<DionBucket*> members;
+    std::vector<at::Tensor> infos;
     std::vector<PyObject*> left;
     for (size_t i = 0; i < buckets.size(); ++i) {
       if (done[i]) continue;
@@ -360,18 +365,21 @@ PyObject* dion_group(PyObject*, PyObject* const* a, Py_ssize_t na) {
         for (DionBucket* b : members) left.insert(left.end(), b->params.begin(), b->params.end());
         continue;
       }
+      infos.clear();
       for (size_t j = 0; j < members.size(); ++j) {
-        PyObject* cnt = PyLong_FromSize_t(members[j]->X.size());
-        PyObject* t = cnt ? PyObject_CallFunctionObjArgs(a[7], members[j]->p0, cnt, nullptr) : nullptr;
-        Py_XDECREF(cnt);
-        if (!t) throw Failed();
-        call[j].info = static_cast<int*>(THPVariable_Unpack(t).data_ptr());
-        Py_DECREF(t);   // (the optimizer holds it)
+        const Ref cnt(PyLong_FromSize_t(members[j]->X.size()));
+        const Ref t(PyObject_CallFunctionObjArgs(a[7], members[j]->p0, cnt.p, nullptr));
+        infos.push_back(THPVariable_Unpack(t.p));
+        call[j].info = static_cast<int*>(infos.back().data_ptr());
       }
-      char* ws = workspace(a[6], need, dev);
+      const at::Tensor ws = workspace(a[6], need, dev);
       const c10::DeviceGuard guard(dev);
-      check(api.dion_step(call.data(), (int)call.size(), xc, gc, mc, qc, ef_alpha, decay, eps, ws, need, stream_of(dev)),
-            "dion_amd_dion_step_buckets");
+      int rc;
+      {
+        const Unlocked unlocked;
+        rc = api.dion_step(call.data(), (int)call.size(), xc, gc, mc, qc, ef_alpha, decay, eps, ws.data_ptr(), need, stream_of(dev));
+      }
+      check(rc, "dion_amd_dion_step_buckets");
     }
     if (left.empty()) Py_RETURN_NONE;
     PyObject* rest = PyTuple_New((Py_ssize_t)left.size());
@@ -441,14 +449,16 @@ void elementwise_run(bool adamw, std::vector<Entry>& all, const char* what, floa
     const c10::Device dev = f.p.device();
     const int xc = dtype_code(f.p.scalar_type()), gc = dtype_code(f.g.scalar_type()), mc = dtype_code(f.s[0].scalar_type());
     const c10::DeviceGuard guard(dev);
-    if (adamw)
-      check(api.adamw_step(X.data(), G.data(), M.data(), V.data(), numel.data(), (int)X.size(), xc, gc, mc,
-                           dtype_code(f.s[1].scalar_type()), adjusted, 1.f - beta1, 1.f - beta2, decay, bc2, eps, stream_of(dev)),
-            "dion_amd_adamw_step");
-    else
-      check(api.lion_step(X.data(), G.data(), M.data(), numel.data(), (int)X.size(), xc, gc, mc, lr, 1.f - beta1, 1.f - beta2,
-                          decay, stream_of(dev)),
-            "dion_amd_lion_step");
+    const int vc = adamw ? dtype_code(f.s[1].scalar_type()) : 0;
+    int rc;
+    {
+      const Unlocked unlocked;
+      rc = adamw ? api.adamw_step(X.data(), G.data(), M.data(), V.data(), numel.data(), (int)X.size(), xc, gc, mc, vc, adjusted,
+                                  1.f - beta1, 1.f - beta2, decay, bc2, eps, stream_of(dev))
+                 : api.lion_step(X.data(), G.data(), M.data(), numel.data(), (int)X.size(), xc, gc, mc, lr, 1.f - beta1,
+                                 1.f - beta2, decay, stream_of(dev));
+    }
+    check(rc, adamw ? "dion_amd_adamw_step" : "dion_amd_lion_step");
   }
 }
 
