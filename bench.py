@@ -58,7 +58,8 @@ WORKLOADS = {
     "scalar_gpt_small": dict(kind="scalar", shapes=[(50304, 768)] * 2 + [(768,)] * 25, seed=6,
                              desc="Lion on the GPT-small embedding and norms, AdamW on lm_head (50304x768 each), bf16"),
 }
-GEMM_KINDS = ("ns_syrk", "ns_poly", "ns_axpy", "ns_flow", "gemm", "dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_ef_upd")
+GEMM_KINDS = ("ns_syrk", "ns_poly", "ns_axpy", "ns_flow", "gemm", "dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_ef_upd",
+              "dion_small")
 
 
 def make_problem(shapes, seed, dtype, device="cpu"):
@@ -287,7 +288,7 @@ def roofline_of(res, kind, workload=None, hbm_bytes=None):
                     traffic=MEASURED_TRAFFIC_BYTES.get((workload, "scalar_opt")), avg_launch_ms=round(ms / n, 5),
                     bytes_per_launch=work / n)
     cands = [k for k in (("ns_syrk", "ns_poly", "ns_axpy", "ns_flow") if kind == "muon"
-                         else ("dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_ef_upd")) if k in prof]
+                         else ("dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_ef_upd", "dion_small")) if k in prof]
     dom = max(cands, key=lambda k: prof[k][1])
     n, ms, work = prof[dom]
     if kind == "dion" and hbm_bytes is not None and dom in hbm_bytes:

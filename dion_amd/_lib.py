@@ -261,7 +261,8 @@ def set_option(name, value):
     check(load().dion_amd_set_option(name.encode(), int(value)), f"dion_amd_set_option({name!r})")
 
 PROF_KINDS = ("ns_syrk", "ns_poly", "ns_axpy", "stage", "normalize", "unstage", "gemm",
-              "dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_orth", "dion_elem", "scalar_opt", "dion_ef_upd", "ns_flow")
+              "dion_bq", "dion_btp", "dion_ef", "dion_upd", "dion_orth", "dion_elem", "scalar_opt", "dion_ef_upd", "ns_flow",
+              "dion_small")
 
 
 def profile_read():

@@ -1311,6 +1311,6 @@ extern "C" int dion_amd_dion_step_buckets(const dion_amd_dion_bucket* buckets, i
   if (workspace_bytes < need) return DA_ERR_WORKSPACE;
   double flops = 0.0;
   for (int i = 0; i < nbuckets; ++i) flops += 8.0 * g[i].cnt * g[i].m * (double)g[i].n * g[i].r;
-  DaProfScope prof(DA_PROF_DION_EFUPD, flops, static_cast<hipStream_t>(stream));
+  DaProfScope prof(DA_PROF_DION_SMALL, flops, static_cast<hipStream_t>(stream));
   return da_dion_small(g, nbuckets, c, workspace, static_cast<hipStream_t>(stream));
 }

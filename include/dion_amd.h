@@ -378,7 +378,8 @@ int dion_amd_dion_step_sketch(void* const* X, const void* const* G, void* const*
 #define DION_AMD_PROF_SCALAR_OPT 13
 #define DION_AMD_PROF_DION_EFUPD 14
 #define DION_AMD_PROF_NS_FLOW 15
-#define DION_AMD_PROF_KINDS 16
+#define DION_AMD_PROF_DION_SMALL 16   /* a whole Dion step of small matrices (dion_amd_dion_step_buckets) */
+#define DION_AMD_PROF_KINDS 17
 int dion_amd_profile_enable(int on);
 int dion_amd_profile_reset(void);
 /* Waits for the recorded events of `kind`; returns launch count, summed milliseconds and

@@ -95,3 +95,22 @@ def test_a_small_dion_launch_that_gave_up_poisons_the_result(dev, option):
     option("ns_flow_fail", 0)
     out, _ = _run(dev, [(96, 160), (160, 96)], F32, 0.5, 1, 1)
     assert all(torch.isfinite(t).all() for tri in out for t in tri)
+
+
+def test_the_profile_books_the_one_launch_step_as_itself(dev, option):
+    """A step of small matrices is one kind of its own with the step's flops: no update pass, no orthonormaliser ran."""
+    from dion_amd import _lib
+
+    lib, shapes = _lib.load(), [(96, 160), (160, 96)]
+    option("dion_small", 1)
+    try:
+        _lib.check(lib.dion_amd_profile_reset(), "reset")
+        _lib.check(lib.dion_amd_profile_enable(1), "enable")
+        _run(dev, shapes, F32, 0.5, 1, 3)
+        prof = _lib.profile_read()
+    finally:
+        lib.dion_amd_profile_enable(0)
+        lib.dion_amd_profile_reset()
+    assert set(prof) == {"dion_small"}
+    launches, ms, work = prof["dion_small"]
+    assert launches == 3 and ms > 0 and work == 3 * 2 * 8.0 * 96 * 160 * 48

@@ -297,3 +297,19 @@ def test_muon_refuses_a_momentum_of_another_size(shape, flatten, momentum):
     opt.state[p]["momentum"] = torch.zeros(p.shape)
     with pytest.raises(_lib.DionAmdError, match="do not fit"):
         opt.step()
+
+
+def test_profile_kinds_have_the_names_of_the_header():
+    import os
+    import re
+
+    from dion_amd import _lib
+
+    header = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "dion_amd.h")).read()
+    kinds = {int(v): k for k, v in re.findall(r"#define DION_AMD_PROF_([A-Z_]+) (\d+)", header) if k != "KINDS"}
+    assert sorted(kinds) == list(range(len(_lib.PROF_KINDS)))
+    assert int(re.search(r"DION_AMD_PROF_KINDS (\d+)", header).group(1)) == len(kinds)
+    assert [kinds[i].lower().replace("_", "") for i in sorted(kinds)] == [n.replace("_", "") for n in _lib.PROF_KINDS]
+    lib = _lib.load()
+    out = (ctypes.c_longlong(), ctypes.c_double(), ctypes.c_double())
+    assert [lib.dion_amd_profile_read(k, *(ctypes.byref(o) for o in out)) for k in (len(kinds) - 1, len(kinds))] == [0, -1]
