@@ -114,3 +114,96 @@ def test_the_profile_books_the_one_launch_step_as_itself(dev, option):
     assert set(prof) == {"dion_small"}
     launches, ms, work = prof["dion_small"]
     assert launches == 3 and ms > 0 and work == 3 * 2 * 8.0 * 96 * 160 * 48
+
+
+def _agree(shapes, runs, tol):
+    for i, (a, b) in enumerate(zip(*runs)):
+        for name, x, y in zip(("X", "M", "Q"), a, b):
+            e = rel_fro(y, x)
+            assert torch.isfinite(y.float()).all() and e <= tol, (i, shapes[i], name, e)
+
+
+@pytest.mark.parametrize("shapes", [
+    [(64, 96)] * 60 + [(96, 64)] * 36,                                  # the most matrices one launch takes
+    [(64, 96)] * 60 + [(96, 64)] * 37,                                  # one more: bucket by bucket
+    [(32 + 8 * i, 64 + 8 * i) for i in range(8)],                       # the most buckets
+    [(32 + 8 * i, 64 + 8 * i) for i in range(9)],                       # one more
+    [(64, 96)] * 200 + [(40, 72)],
+])
+def test_groups_around_the_limits_of_one_launch(dev, option, shapes):
+    runs = []
+    for mode in (0, 1):
+        option("dion_small", mode)
+        out, opt = _run(dev, shapes, F32, 0.5, 8, 2)
+        runs.append(out)
+        assert all(opt.state[p]["Q"].abs().sum() > 0 for p in opt.param_groups[0]["params"])
+    _agree(shapes, runs, 2e-5)
+    if len(shapes) > 96 or len(set(shapes)) > 8:                        # both took the same road
+        for a, b in zip(*runs):
+            assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_a_group_split_between_both_roads(dev, option):
+    """Matrices of two dtypes in one group: the few fp32 ones go out in one launch, the many bf16 ones bucket by bucket, and every
+    parameter is stepped exactly once."""
+    from dion_amd import Dion
+
+    shapes = [(64, 96)] * 5 + [(96, 64)] * 60 + [(128, 64)] * 50 + [(64, 64)] * 3
+    dtypes = [F32] * 5 + [BF] * 110 + [F32] * 3
+    runs = []
+    for mode in (0, -1):
+        option("dion_small", mode)
+        gen = torch.Generator(device=dev).manual_seed(8)
+        torch.manual_seed(8)
+        params = [torch.nn.Parameter((torch.randn(s, generator=gen, device=dev) * 0.02).to(d)) for s, d in zip(shapes, dtypes)]
+        opt = Dion(params, lr=0.02, rank_fraction=0.5)
+        for p in params:      # (in one order, whichever road creates them)
+            opt._get_or_initialize_state(p, opt.param_groups[0])
+        for _ in range(2):
+            for p in params:
+                p.grad = (torch.randn(p.shape, generator=gen, device=dev) * 1e-2).to(p.dtype)
+            opt.step()
+        torch.cuda.synchronize()
+        runs.append([(p.detach(), opt.state[p]["momentum"], opt.state[p]["Q"]) for p in params])
+        assert len(opt.cholesky_info()) == 4 and all(int(v.max()) == 0 for v in opt.cholesky_info().values())
+    fp32 = [i for i, d in enumerate(dtypes) if d == F32 and shapes[i][0] != shapes[i][1]]
+    _agree([shapes[i] for i in fp32], [[r[i] for i in fp32] for r in runs], 2e-5)
+    for i, (a, b) in enumerate(zip(*runs)):
+        if dtypes[i] == BF:
+            assert all(torch.equal(x, y) for x, y in zip(a, b)), i
+        else:
+            assert rel_fro(b[0], a[0]) <= 2e-5 and rel_fro(b[1], a[1]) <= 2e-5, i
+
+
+@pytest.mark.parametrize("shape,shift", [((96, 160), 8), ((160, 96), 24), ((33, 64), 1), ((77, 53), 3)])
+def test_dion_weights_off_the_128_byte_grid(dev, option, shape, shift):
+    """Views of flat buffers that are only 16-byte aligned (off the 8-grid: aligned to their elements) are left to the bucket
+    launches: the bits of aligned copies on that road, and nothing around the views is touched."""
+    from dion_amd import Dion
+
+    option("dion_small", 0)
+    runs, numel = [], shape[0] * shape[1]
+    for moved in (False, True):
+        gen = torch.Generator(device=dev).manual_seed(9)
+        torch.manual_seed(9)
+        flats, params = [], []
+        for _ in range(3):
+            x = torch.randn(shape, generator=gen, device=dev) * 0.02
+            if moved:
+                flat = torch.full((numel + shift + 40,), 7.0, device=dev)
+                flat[shift:shift + numel] = x.flatten()
+                x = flat[shift:shift + numel].view(shape)
+                assert x.data_ptr() % 128
+                flats.append(flat)
+            params.append(torch.nn.Parameter(x))
+        opt = Dion(params, lr=0.02, rank_fraction=0.5)
+        for p in params:
+            p.grad = torch.randn(shape, generator=gen, device=dev) * 1e-2
+        opt.step()
+        torch.cuda.synchronize()
+        runs.append([(p.detach().clone(), opt.state[p]["momentum"], opt.state[p]["Q"]) for p in params])
+        for flat in flats:
+            assert (flat[:shift] == 7).all() and (flat[shift + numel:] == 7).all()
+        option("dion_small", 1)
+    for a, b in zip(*runs):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))

@@ -425,3 +425,35 @@ def test_thin_matrices_in_a_large_call_equal_single_calls(dev, buckets, dtype):
             assert torch.equal(together[at + k][0], x), (m, n, k, "weights")
             assert torch.equal(together[at + k][1], mom), (m, n, k, "momentum")
         at += count
+
+
+@pytest.mark.parametrize("shapes", [
+    [(256, 256)] * 3 + [(512, 256)], [(768, 768)] * 48 + [(768, 1024)] * 8 + [(1024, 768)] * 8])
+def test_weights_off_the_128_byte_grid(dev, shapes):
+    """Neighbouring matrices that share a cache line (16-byte aligned views of one flat buffer), through the one-launch kernel
+    and through the updates in a product's epilogue: the bits of matrices with buffers of their own."""
+    from dion_amd import Muon
+
+    results = []
+    for shared in (False, True):
+        gen = torch.Generator(device=dev).manual_seed(12)
+        total = sum(a * b for a, b in shapes) + 64
+        flat, at, params = torch.zeros(total, dtype=torch.bfloat16, device=dev), 8, []
+        for a, b in shapes:
+            x = (torch.randn(a, b, generator=gen, device=dev) * 0.02).bfloat16()
+            if shared:
+                view = flat[at:at + a * b].view(a, b)
+                view.copy_(x)
+                at += a * b
+                x = view
+                assert x.data_ptr() % 128 != 0 and x.data_ptr() % 16 == 0
+            params.append(torch.nn.Parameter(x))
+        opt = Muon(params, lr=0.02, mu=0.95, weight_decay=0.01)
+        for _ in range(2):
+            for p in params:
+                p.grad = (torch.randn(p.shape, generator=gen, device=dev) * 1e-3).bfloat16()
+            opt.step()
+        torch.cuda.synchronize()
+        results.append([p.detach().clone() for p in params])
+    for s, a, b in zip(shapes, *results):
+        assert torch.equal(a, b), s

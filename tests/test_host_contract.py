@@ -313,3 +313,32 @@ def test_profile_kinds_have_the_names_of_the_header():
     lib = _lib.load()
     out = (ctypes.c_longlong(), ctypes.c_double(), ctypes.c_double())
     assert [lib.dion_amd_profile_read(k, *(ctypes.byref(o) for o in out)) for k in (len(kinds) - 1, len(kinds))] == [0, -1]
+
+
+def test_what_the_one_launch_dion_step_takes():
+    """Up to 96 matrices in 8 buckets, weights and momentum on the 128-byte grid, gradients and Q on the 16-byte one."""
+    from dion_amd import _lib
+
+    lib = _lib.load()
+
+    def need(spec, x=0, m=0, g=0, q=0):
+        arr, keep = (_lib.DionBucket * len(spec))(), []
+        for k, (count, rows, cols) in zip(arr, spec):
+            tables = [_pointers(off, count) for off in (x, g, m, q)]
+            keep.append(tables)
+            k.X, k.G, k.M, k.Q = (ctypes.cast(t, ctypes.POINTER(ctypes.c_void_p)) for t in tables)
+            k.batch, k.m, k.n, k.r, k.scaled_lr = count, rows, cols, min(rows, cols) // 2, 0.1
+        return lib.dion_amd_dion_buckets_workspace_bytes(arr, len(spec), _lib.F32, _lib.F32, _lib.F32, _lib.F32)
+
+    buckets = [(2, 32 + 8 * i, 64 + 8 * i) for i in range(9)]
+    try:
+        _lib.set_option("dion_small", 1)
+        assert need([(96, 64, 96)]) > 0 and need([(60, 64, 96), (36, 96, 64)]) > 0 and need(buckets[:8]) > 0
+        assert need([(97, 64, 96)]) == 0 and need([(60, 64, 96), (37, 96, 64)]) == 0 and need(buckets) == 0
+        assert need([(2, 64, 96)], g=16, q=16, x=128, m=256) > 0
+        for kw in (dict(x=64), dict(m=16), dict(g=8), dict(q=4)):
+            assert need([(2, 64, 96)], **kw) == 0, kw
+        _lib.set_option("dion_small", 0)
+        assert need([(2, 64, 96)]) == 0
+    finally:
+        _lib.set_option("dion_small", -1)
