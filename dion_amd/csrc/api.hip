@@ -66,8 +66,11 @@ bool grid256(const Bucket* k, int n, Count count) {
 
 // Whether the one-launch kernel for small matrices has little enough work with these buckets (`count` of each).  Matrices are
 // dealt to eight queues of one XCD's workgroups each; what counts is the longest queue, in 64 x 64 x 64 stages per iteration.
-// Measured against the batched launches (us per call): 912 stages (16 x 256 x 1024) 141 : 206, 1088 (512 x 512) 129 : 191,
-// 3488 (512 x 2048) 260 : 286, 3600 (768 x 768) 300 : 247, 3648 (64 x 256 x 1024) 348 : 279.
+// Measured against the batched launches (us per call), below the line: 912 stages (16 x 256 x 1024) 148 : 208, 1088 (512 x 512)
+// 131 : 191, 1888 (512 x 1024) 173 : 222, 2280 (40 x 256 x 1024) 247 : 251, 2480 (320 x 128 x 512) 529 : 744; above it:
+// 2688 (512 x 1536) 216 : 255, 2736 (48 x 256 x 1024) 262 : 259, 2880 (160 x 256 x 256) 365 : 502, 3488 (512 x 2048) 267 : 286,
+// 3600 (768 x 768) 296 : 248, 3648 (64 x 256 x 1024) 341 : 278.  The line is on the safe side: the roads cross at 2700 at the
+// earliest (many matrices of a middling size) and by 3600 for all.
 template <typename Bucket, typename Count>
 bool small_enough(const Bucket* k, int n, Count count) {
   double load[8] = {0}, worst = 0;

@@ -5,7 +5,7 @@
 //
 // What bounds it: as a sequence of launches a bucket takes 40 to 60 of them (a third of which only find out that the fp64
 // pass of the orthonormaliser is not needed), each a few microseconds of work: a model of 24 matrices of 256 x 256 and
-// 256 x 1024 spent 0.6-0.8 ms, most of it on the host.  Now 0.26 ms, and the host is free after 45 us: four fifths of it is the
+// 256 x 1024 spent 0.6-0.8 ms, most of it on the host.  Now 0.25 ms, and the host is free after 38 us: four fifths of it is the
 // chain of phases (25 us per diagonal block, 10-15 us per product), not throughput.  Here the step is a list of phases per matrix, cut into tiles;
 // workgroups take tiles from eight queues, one per XCD (flow_queue.h), and a counter per matrix and phase says when the
 // next phase may start.  A matrix stays with one XCD, so its phases meet in one L2.
