@@ -180,9 +180,9 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
       }
       __syncthreads();
       const bool nonzero = sh_words[0] != 0, sick = sh_words[1] != 0;
-      int next = -1;
+      unsigned next = DA_NO_TICKET;
       auto ask = [&]() {
-        if (tid == 0) next = take_ticket(word, xcd, total, true);
+        if (tid == 0) next = request_ticket(word);
       };
 
       const int rp = G.rp, mpR = G.mpT * 64, npR = G.npT * 64;
@@ -526,7 +526,7 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
         ask();   // a phase that a healthy matrix does not need
       }
       // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
-      if (tid == 0) sh_ticket[slot ^ 1] = next;
+      if (tid == 0) sh_ticket[slot ^ 1] = ticket_of(next, total);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (tid == 0) __hip_atomic_fetch_add(words + kind, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (in the L2)

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
         }
       }
       __syncthreads();
-      int next = -1;
+      unsigned next = DA_NO_TICKET;
       const long long rr = (long long)rp * rp, last = (long long)a.rows * a.r - 8;
       const E* const P = reinterpret_cast<const E*>(a.P) + b * ((long long)a.rows * a.r);
       double* const S = a.w.P64 + b * ((long long)a.mT * 64 * rp);
@@ -139,12 +139,12 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
         int ti, tj;
         gram_tile(p, task - slice * ng, kbeg, min(kbeg + a.kslice, (a.rows + KD - 1) / KD * KD), a.w.slab + (b * a.slices + slice) * rr, rp,
                   d, tid, lane, wm, wn, ti, tj);
-        if (tid == 0) next = take_ticket(word, xcd, total, true);
+        if (tid == 0) next = request_ticket(word);
       } else if (fix && task < ng) {
         counter = words + W_GRAM2;
         int ti, tj;
         gram_tile(work<double>(S, rp, 1), task, 0, (a.rows + KD - 1) / KD * KD, a.w.gram + b * rr, rp, d, tid, lane, wm, wn, ti, tj);
-        if (tid == 0) next = take_ticket(word, xcd, total, true);
+        if (tid == 0) next = request_ticket(word);
         gram_defect(d, defect, 2 * rT, ti, tj, tid);
       } else if (pt || fix) {
         const int t2 = fix ? task - ng : task, row0 = wave_uniform(t2 / rT) * 64, col0 = wave_uniform(t2 % rT) * 64;
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
           }
           polish_tile(S, a.w.gram + b * rr, a.r_live, rp, drop, row0, col0, d, tid, lane, wm, wn);
         }
-        if (tid == 0) next = take_ticket(word, xcd, total, true);
+        if (tid == 0) next = request_ticket(word);
         if (pt) {
           for (int e = tid; e < 4096; e += 256) S[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
         } else {
@@ -180,10 +180,10 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
         const Factor F = {a.w.slab + b * a.slices * rr, a.w.L + b * rr, a.w.T + b * rr, a.slices, a.r_live, rp, rT,
                           words + W_BAD, words + W_SICK, a.info + b, reinterpret_cast<double*>(words + W_RANGE), 0.0};
         factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn);
-        if (tid == 0) next = take_ticket(word, xcd, total, true);
+        if (tid == 0) next = request_ticket(word);
       }
       // ---- publish: every wavefront's stores are acknowledged, then the counter moves
-      if (tid == 0) sh_ticket[slot ^ 1] = next;
+      if (tid == 0) sh_ticket[slot ^ 1] = ticket_of(next, total);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (tid == 0) __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (in the L2)
