@@ -3,7 +3,7 @@
 // diagonal block on the matrix cores and inverts the triangular factor (redundantly -- the factor is
 // the serial part; a few workgroups per matrix repeat it rather than wait for one), then they share
 // the 64 x 64 pieces of what depends on it:
-//   role 0            : stores L_jj and its inverse D_j (the diagonal block of W, see below),
+//   role 0            : stores the inverse D_j of L_jj (the diagonal block of W, see below),
 //   roles 1 .. below  : one 64-row tile of the panel   L[i, j] = A[i, j] D_j^T,
 //   roles above that  : one 64-column tile of          W[j, c] = -D_j L[j, c],  c < j,
 // where W is the block-lower-triangular matrix with which the triangular solve of P becomes one
@@ -18,7 +18,7 @@
 // the later steps read: the separate update launch between two steps is gone.
 // No host synchronisation: a failed pivot is recorded in a device-side info word, mirroring
 // torch.linalg.cholesky_ex's `info`.
-#include "gemm_f64.h"
+#include "diag64.h"
 
 // fp64 factorisation: fused multiply-adds are welcome here (the build disables contraction
 // globally for the kernels that reproduce the reference's bf16 rounding points)
@@ -27,25 +27,7 @@
 namespace {
 
 constexpr int NB = DA_CHOL_NB;
-constexpr int LP = NB + 1;   // LDS pitch of the operand tiles (doubles): transposed stores stay nearly conflict-free
-
-// The 64 x 64 diagonal block S and the inverse-in-progress Y live in matrix-core accumulators: wavefront w of
-// the four holds tile row w (rows 16 w .. 16 w + 15) of both as 16 x 16 tiles.  Right-looking with 4-wide block
-// columns.  Per block step every wavefront reads the published block column of S (64 x 4) and row block of Y
-// (4 x 64) from LDS and repeats the serial part on its own SIMD instead of waiting for one owner: the 4 x 4
-// diagonal factor (the same instructions in every lane), then lane = row forms its row of the L block column
-// by forward substitution and lane = column its column of X = L_cc^-1 Y_c (rows 4 cb .. 4 cb + 3 of the inverse,
-// final after this).  Both go to LDS as MFMA operands, the two rank-4 updates S -= L_c L_c^T, Y -= L_c X are
-// v_mfma_*_16x16x4 instructions on the wavefront's own tiles, and the wavefronts publish the next block column / row
-// block.  One workgroup barrier per 4 columns; the published blocks and the operands are double-buffered.
-template <typename T> __device__ __forceinline__ T rsqrt_seed(T p);
-template <> __device__ __forceinline__ double rsqrt_seed<double>(double p) { return __builtin_amdgcn_rsq(p); }
-template <> __device__ __forceinline__ float rsqrt_seed<float>(float p) { return __builtin_amdgcn_rsqf(p); }
-// a positive normal number (false for NaN, infinities, zero and denormals, which the estimate does not handle)
-__device__ __forceinline__ bool usable_pivot(double p) { return __builtin_amdgcn_class(p, 0x100); }
-__device__ __forceinline__ bool usable_pivot(float p) { return __builtin_amdgcn_classf(p, 0x100); }
-
-template <typename T> struct Quad { T v[4]; };
+constexpr int LP = DIAG_P;   // LDS pitch of the operand tiles: transposed stores stay nearly conflict-free
 
 template <typename T, bool INV>
 __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __restrict__ Lmat,
@@ -54,11 +36,6 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
                                                         const int* gate, int gate_want, int o_prev, int c_end, int per, int t_row, int n_t,
                                                         int t_inline, T* __restrict__ pstat) {
   typedef typename Mfma<T>::acc_t acc_t;
-  typedef Quad<T> quad_t;
-  __shared__ __attribute__((aligned(16))) T scol[2][4][NB];     // published block column of S: [column][row]
-  __shared__ __attribute__((aligned(16))) quad_t yrow[2][NB];   // published row block of Y:    [column] -> 4 rows
-  __shared__ __attribute__((aligned(16))) quad_t lops[2][NB];   // L block column as MFMA operand (0 in finished rows)
-  __shared__ __attribute__((aligned(16))) quad_t xops[2][NB];   // X, [column] -> 4 rows
   extern __shared__ __attribute__((aligned(16))) unsigned char opnd_raw[];   // two k-major 64 x 64 operand tiles
   T* const opnd = reinterpret_cast<T*>(opnd_raw);
   // grid (matrix, workgroup of the matrix): the matrices' workgroups 0 are dispatched first, the update-only
@@ -67,14 +44,15 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
   if (gate && (gate[b] != 0) != (gate_want != 0)) return;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lc = lane & 15, lg = lane >> 4;
-  // D_j transposed (dT[k][x] = D[x][k], zero outside the nb x nb lower triangle) and, for role 0, L_jj (in `op`)
+  // D_j transposed (dT[k][x] = D[x][k], zero outside the nb x nb lower triangle); `op`: the factorisation's work area, then
+  // the operand tiles of the products
   T* const dT = opnd;
   T* const op = opnd + NB * LP;
   // deferred mode: L[j, p] k-major (ljT[k][n] = L[o + n][o_prev + k]), behind the role buffers
   T* const ljT = opnd + (INV ? 5 : 2) * NB * LP;
   const bool defer = o_prev >= 0;
   const T* g = G + (long long)b * sG + (long long)o * r + o;
-  // The workgroups of one matrix share its roles round-robin (role 0: L_jj, D_j and the status word; 1 .. below:
+  // The workgroups of one matrix share its roles round-robin (role 0: D_j and the status word; 1 .. below:
   // panel tiles; the rest: W tiles).  The operand tile of a product does not depend on this step's factor: it is
   // requested now, 16 elements per thread, and the next one while the previous product runs.
   const int nroles = 1 + below + ((!INV || t_inline) ? o / NB : 0);
@@ -161,7 +139,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
         DA_STORE_TILE(pb0, pb1, pb2, pb3, pa + NB * LP, false);  // opb[kk][n] = T[64 k + kk][64 c + n]
       };
       if (!have_first) fetch_t(c, c);
-      __syncthreads();   // the buffers may still be read (role 0's copy, a previous product)
+      __syncthreads();   // the buffers may still be read (a previous product)
       put(0);
       for (int k = c; k < jb; ++k) {
         const int buf = (k - c) & 1;
@@ -260,7 +238,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
     DA_LOAD_TILE(lj0, lj1, lj2, lj3, Lmat + (long long)b * sG + (long long)o * r + o_prev, nb, NB);
     DA_STORE_TILE(lj0, lj1, lj2, lj3, ljT, true);
   }
-  acc_t S[4], Y[4];
+  acc_t S[4];
 #pragma unroll
   for (int tj = 0; tj < 4; ++tj)
 #pragma unroll
@@ -268,7 +246,6 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
       const int i = wave * 16 + Mfma<T>::row(v, lane), j = tj * 16 + lc;
       // identity padding beyond nb keeps the padded part inert
       S[tj][v] = (tj <= wave && i < nb && j < nb) ? g[(long long)i * r + j] : (i == j ? T(1) : T(0));
-      Y[tj][v] = (i == j) ? T(1) : T(0);
     }
   if (defer) {
     __syncthreads();   // ljT is in place
@@ -299,142 +276,27 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
   // (the two tiles of a T role would stay in registers through the whole factor loop: those are requested after it)
   const bool early = role < nroles && !(INV && role > below);
   if (early) fetch(role);
-  if (tid < 2 * NB) {
-    // columns right of the diagonal tile of a row block are never published: they read as zero
-    quad_t z;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) z.v[k] = T(0);
-    yrow[tid >> 6][tid & 63] = z;
-  }
-  __syncthreads();
-
-  // Block q (columns / rows 4 q .. 4 q + 3) of the current S and Y into buffer `buf`.
-  auto publish = [&](int q, int buf) {
-    const int tq = q >> 2, qq = q & 3;
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-      if (tj == tq && tj <= wave && (lc >> 2) == qq) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) scol[buf][lc & 3][wave * 16 + Mfma<T>::row(v, lane)] = S[tj][v];
+  diag_factor64(S, op, dT, nb, nb, lane, wave, [&](int failed, T pmin, T pmax) {
+    if (wg != 0 || lane != 0) return;
+    // (`fresh`: the first block column of a factorisation starts the matrix's status word)
+    if (fresh || (failed != 0 && info[b] == 0)) info[b] = failed ? o + failed : 0;
+    // pivot range of the matrix so far (the squares of R's diagonal: their ratio bounds cond(R)^2 from below)
+    if (pstat) {
+      if (o > 0) {
+        pmin = pstat[2 * b] < pmin ? pstat[2 * b] : pmin;
+        pmax = pstat[2 * b + 1] > pmax ? pstat[2 * b + 1] : pmax;
       }
-      if (wave == tq && tj <= wave) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int rr = Mfma<T>::row(v, lane);
-          if ((rr >> 2) == qq) yrow[buf][tj * 16 + lc].v[rr & 3] = Y[tj][v];
-        }
-      }
+      pstat[2 * b] = pmin;
+      pstat[2 * b + 1] = pmax;
     }
-  };
-  publish(0, 0);
-  __syncthreads();
-
-  constexpr int NEWTON = sizeof(T) == 8 ? 2 : 0;   // the hardware estimate is good to 1 ulp in fp32, ~2^-27 in fp64
-  int bad = 0;                                     // first failed pivot (every lane computes the same)
-  T pmin = T(3e38), pmax = T(0);                   // smallest and largest usable pivot of this block column
-  for (int cb = 0; cb < NB / 4; ++cb) {
-    const int buf = cb & 1, k0 = cb * 4;
-    quad_t sv;                             // lane = row: S[lane][k0 ..]
-#pragma unroll
-    for (int k = 0; k < 4; ++k) sv.v[k] = scol[buf][k][lane];
-    const quad_t yv = yrow[buf][lane];     // lane = column: Y[k0 ..][lane]
-    T a[4][4];
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const quad_t d = *reinterpret_cast<const quad_t*>(&scol[buf][jj][k0]);   // the same address in every lane
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) a[ii][jj] = d.v[ii];
-    }
-    // unblocked Cholesky of the 4 x 4 diagonal block: a[i][j], j < i becomes L_cc, di[] the inverse diagonal
-    T di[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const T p = a[c][c];
-      const bool ok = usable_pivot(p);
-      // 1/sqrt(p) from the hardware estimate plus Newton steps: this chain is the critical path of the whole
-      // factorisation and the library sqrt + divide are four times as long
-      T rs = ok ? rsqrt_seed<T>(p) : T(0);
-#pragma unroll
-      for (int it = 0; it < NEWTON; ++it) rs = rs * (T(1.5) - T(0.5) * p * rs * rs);
-      di[c] = ok ? rs : T(0);
-      bad = (!ok && bad == 0 && k0 + c < nb) ? o + k0 + c + 1 : bad;
-      if (ok && k0 + c < nb) {
-        pmin = p < pmin ? p : pmin;
-        pmax = p > pmax ? p : pmax;
-      }
-#pragma unroll
-      for (int i = c + 1; i < 4; ++i) a[i][c] *= di[c];
-#pragma unroll
-      for (int i = c + 1; i < 4; ++i)
-#pragma unroll
-        for (int j = c + 1; j <= i; ++j) a[i][j] -= a[i][c] * a[j][c];
-    }
-    // row `lane` of the L block column and column `lane` of X, by forward substitution with L_cc
-    T l[4], x[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      T tl = sv.v[k], tx = yv.v[k];
-#pragma unroll
-      for (int m = 0; m < k; ++m) {
-        tl -= l[m] * a[k][m];
-        tx -= a[k][m] * x[m];
-      }
-      l[k] = tl * di[k];
-      x[k] = tx * di[k];
-    }
-    quad_t lo, xo, lfin;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      lo.v[k] = lane > k0 + 3 ? l[k] : T(0);               // finished rows take no part in the updates
-      lfin.v[k] = lane >= k0 + k ? l[k] : T(0);            // L_jj: zero above the diagonal
-      xo.v[k] = (lane <= k0 + k && k0 + k < nb) ? x[k] : T(0);
-    }
-    lops[buf][lane] = lo;     // (every wavefront writes the same values; each reads back after its own writes)
-    xops[buf][lane] = xo;
-    if (wave == (cb & 3)) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) dT[lane * LP + k0 + k] = lane < nb ? xo.v[k] : T(0);
-      if (wg == 0) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) op[lane * LP + k0 + k] = lfin.v[k];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (wave * 16 + 15 > k0 + 3) {
-      const T aop = -lops[buf][wave * 16 + lc].v[lg];
-#pragma unroll
-      for (int tj = 0; tj < 4; ++tj) {
-        if (tj <= wave && tj * 16 + 15 > k0 + 3) S[tj] = Mfma<T>::mma(aop, lops[buf][tj * 16 + lc].v[lg], S[tj]);
-        if (tj <= wave && tj * 16 <= k0 + 3) Y[tj] = Mfma<T>::mma(aop, xops[buf][tj * 16 + lc].v[lg], Y[tj]);
-      }
-    }
-    if (cb + 1 < NB / 4) publish(cb + 1, buf ^ 1);
-    __syncthreads();
-  }
+  });
 
   // ---- the 64 x 64 x 64 products that depend on the factor: C[m][n] = sum_k opa[k][m] * opb[k][n]
   if (wg == 0) {
-    T* l = Lmat + (long long)b * sG + (long long)o * r + o;
     T* w = (INV ? Tmat : Wmat) + (long long)b * sG + (long long)o * r + o;
     for (int e = tid; e < NB * NB; e += 256) {
       const int i = e >> 6, j = e & 63;
-      if (i < nb && j < nb) {
-        l[(long long)i * r + j] = op[i * LP + j];
-        w[(long long)i * r + j] = dT[j * LP + i];
-      }
-    }
-    // (`fresh`: the first block column of a factorisation starts the matrix's status word)
-    if (tid == 0 && (fresh || (bad != 0 && info[b] == 0))) info[b] = bad;
-    // pivot range of the matrix so far (the squares of R's diagonal: their ratio bounds cond(R)^2 from below)
-    if (tid == 0 && pstat) {
-      T mn = pmin, mx = pmax;
-      if (o > 0) {
-        mn = pstat[2 * b] < mn ? pstat[2 * b] : mn;
-        mx = pstat[2 * b + 1] > mx ? pstat[2 * b + 1] : mx;
-      }
-      pstat[2 * b] = mn;
-      pstat[2 * b + 1] = mx;
+      if (i < nb && j < nb) w[(long long)i * r + j] = dT[j * LP + i];
     }
   }
   if (role < nroles && !early) fetch(role);
@@ -474,7 +336,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
         pa3[i] -= op[(trow + 48) * LP + tcol + i];
       }
     }
-    __syncthreads();   // `op` may still be read (role 0's copy, the previous product's MFMAs)
+    __syncthreads();   // `op` may still be read (the previous product's MFMAs)
     // panel: opa[k][m] = A[row0 + m][o + k];  W: opb[k][n] = L[o + k][col0 + n]
     DA_STORE_TILE(pa0, pa1, pa2, pa3, op, panel);
     const int next = role + per;

@@ -72,8 +72,8 @@ int da_cvt_from_f32(const float* src, void* dst, int dst_dtype, long long per, i
 
 // Block-column step j = o / 64 of the blocked lower Cholesky G = L L^T of each r x r matrix
 // G[b] (o a multiple of 64; nb = 64 except for a ragged last block): factors the nb x nb diagonal
-// block at offset o (the trailing updates of earlier steps already applied to G), writes L_jj and
-// the panel L[o+nb.., o..o+nb] into Lmat[b], and row block j of W[b] (D_j = L_jj^-1 on the
+// block at offset o (the trailing updates of earlier steps already applied to G), writes the panel
+// L[o+nb.., o..o+nb] into Lmat[b] (L_jj itself is not stored), and row block j of W[b] (D_j = L_jj^-1 on the
 // diagonal, -D_j L[j, c] left of it).  A non-positive or non-finite pivot zeroes that column (of
 // L_jj and of D_j) and records (o + column + 1) in info[b] if it is the matrix's first failure.
 // `gate`: as in RealGemmDesc.

@@ -1,7 +1,7 @@
 // Tile products and the serial part of a factorisation for the one-launch kernels (dion_small.hip, orth_flow.hip): 256 threads,
 // operands from memory through registers into LDS, products on the matrix cores in bf16, fp32 and fp64.
 #pragma once
-#include "gemm_f64.h"
+#include "diag64.h"
 #include "mfma_tile.h"
 
 #pragma clang fp contract(off)
@@ -9,7 +9,6 @@
 namespace {
 
 constexpr int KD = 32;             // depth of an fp32 / fp64 stage
-constexpr int LP = 65;             // pitch of the factorisation's 64 x 64 tile
 constexpr int STAGES64 = 2 * 2 * KD * 66 * 8;   // two stages of two fp64 operands of 64 rows: the largest user of the LDS
 
 typedef double double2_t __attribute__((ext_vector_type(2)));
@@ -415,123 +414,6 @@ __device__ __forceinline__ float guard(float x, bool nonzero, float alt) {
   return nonzero ? x : alt;
 }
 
-// ---- the serial part of the factorisation: a 64 x 64 diagonal block and its inverse (scheme of cholesky.hip) --------------
-// g: the block (lower triangle), pitch ld, in LDS, from `lds` on or anywhere.  dT receives the inverse factor, transposed (dT[k][x] = D[x][k], pitch LP).
-// A pivot that is not positive zeroes its column and is counted in `bad` (o + column + 1, the first one); `live`: columns
-// of the block that belong to the matrix (the others are identity and leave the pivot range alone).
-struct Quad { double v[4]; };
-__device__ __forceinline__ void diag_factor(const double* g, int ld, char* lds, double* dT, int live, int o, int tid, int lane,
-                                            int wave, int& bad, double& pmin, double& pmax) {
-#pragma clang fp contract(fast)
-  typedef Mfma<double>::acc_t acc_t;
-  double(*scol)[4][64] = reinterpret_cast<double(*)[4][64]>(lds);   // [2]: published block column of S
-  Quad(*yrow)[64] = reinterpret_cast<Quad(*)[64]>(lds + 4096);      // [2]: published row block of Y
-  Quad(*lops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 8192);      // [2]: L block column as MFMA operand
-  Quad(*xops)[64] = reinterpret_cast<Quad(*)[64]>(lds + 12288);     // [2]: X
-  const int lc = lane & 15, lg = lane >> 4;
-  acc_t S[4], Y[4];
-#pragma unroll
-  for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int i = wave * 16 + Mfma<double>::row(v, lane), j = tj * 16 + lc;
-      S[tj][v] = tj <= wave ? (i >= j ? g[(long long)i * ld + j] : g[(long long)j * ld + i]) : 0.0;
-      Y[tj][v] = i == j ? 1.0 : 0.0;
-    }
-  __syncthreads();   // (the block may lie where the published ones go)
-  if (tid < 128) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) yrow[tid >> 6][tid & 63].v[k] = 0.0;
-  }
-  __syncthreads();
-  auto publish = [&](int q, int buf) {
-    const int tq = q >> 2, qq = q & 3;
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-      if (tj == tq && tj <= wave && (lc >> 2) == qq) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) scol[buf][lc & 3][wave * 16 + Mfma<double>::row(v, lane)] = S[tj][v];
-      }
-      if (wave == tq && tj <= wave) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int rr = Mfma<double>::row(v, lane);
-          if ((rr >> 2) == qq) yrow[buf][tj * 16 + lc].v[rr & 3] = Y[tj][v];
-        }
-      }
-    }
-  };
-  publish(0, 0);
-  __syncthreads();
-  for (int cb = 0; cb < 16; ++cb) {
-    const int buf = cb & 1, k0 = cb * 4;
-    double sv[4], a[4][4], di[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) sv[k] = scol[buf][k][lane];
-    const Quad yv = yrow[buf][lane];
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) a[ii][jj] = scol[buf][jj][k0 + ii];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const double p = a[c][c];
-      const bool ok = __builtin_amdgcn_class(p, 0x100);   // positive normal
-      double rs = ok ? __builtin_amdgcn_rsq(p) : 0.0;     // 2^-27: one step of third order
-      const double err = 1.0 - p * rs * rs;
-      rs = rs + rs * err * (0.5 + 0.375 * err);
-      di[c] = ok ? rs : 0.0;
-      bad = (!ok && bad == 0 && k0 + c < live) ? o + k0 + c + 1 : bad;
-      if (ok && k0 + c < live) {
-        pmin = p < pmin ? p : pmin;
-        pmax = p > pmax ? p : pmax;
-      }
-#pragma unroll
-      for (int i = c + 1; i < 4; ++i) a[i][c] *= di[c];
-#pragma unroll
-      for (int i = c + 1; i < 4; ++i)
-#pragma unroll
-        for (int j = c + 1; j <= i; ++j) a[i][j] -= a[i][c] * a[j][c];
-    }
-    double l[4], x[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      double tl = sv[k], tx = yv.v[k];
-#pragma unroll
-      for (int m = 0; m < k; ++m) {
-        tl -= l[m] * a[k][m];
-        tx -= a[k][m] * x[m];
-      }
-      l[k] = tl * di[k];
-      x[k] = tx * di[k];
-    }
-    Quad lo, xo;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      lo.v[k] = lane > k0 + 3 ? l[k] : 0.0;
-      xo.v[k] = lane <= k0 + k ? x[k] : 0.0;
-    }
-    lops[buf][lane] = lo;
-    xops[buf][lane] = xo;
-    if (wave == (cb & 3)) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) dT[lane * LP + k0 + k] = xo.v[k];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (wave * 16 + 15 > k0 + 3) {
-      const double aop = -lops[buf][wave * 16 + lc].v[lg];
-#pragma unroll
-      for (int tj = 0; tj < 4; ++tj) {
-        if (tj <= wave && tj * 16 + 15 > k0 + 3) S[tj] = Mfma<double>::mma(aop, lops[buf][tj * 16 + lc].v[lg], S[tj]);
-        if (tj <= wave && tj * 16 <= k0 + 3) Y[tj] = Mfma<double>::mma(aop, xops[buf][tj * 16 + lc].v[lg], Y[tj]);
-      }
-    }
-    if (cb + 1 < 16) publish(cb + 1, buf ^ 1);
-    __syncthreads();
-  }
-}
-
 // ---- the blocked fp64 Cholesky factorisation  P^T P = L L^T,  T = L^-1  in blocks of 64, as tasks -------------------------
 // P^T P comes as lower 32 x 32 tiles in K slices (slab: [slices][rp][rp], rp = 64 rT); columns r .. rp - 1 are the identity.
 struct Factor {
@@ -600,28 +482,37 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
       d[(i0 + 8 * u) * 66 + k + 1] = w[u][1];
     }
     __syncthreads();
-    int bad = 0;
-    double pmin = 3e38, pmax = 0.0;
-    double* const range = F.range;
-    if (j > 0) {
-      bad = __hip_atomic_load(F.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      pmin = __hip_atomic_load(range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      pmax = __hip_atomic_load(range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    double* const dT = d + 2048;   // behind the 16 KB of the published blocks
-    diag_factor(d, 66, lds, dT, min(64, F.r - j * 64), j * 64, tid, lane, wave, bad, pmin, pmax);
-    double* const Dw = T + (long long)j * 64 * rp + j * 64;
-    for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * LP + (e >> 6)];
-    if (tid == 0) {
+    Mfma<double>::acc_t S[4];
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = wave * 16 + Mfma<double>::row(v, lane), col = tj * 16 + (lane & 15);
+        S[tj][v] = tj <= wave ? (row >= col ? d[row * 66 + col] : d[col * 66 + row]) : 0.0;
+      }
+    __syncthreads();   // (the block lies where the factorisation works)
+    double* const dT = d + DIAG_W;
+    static_assert(2 * DIAG_W * 8 <= STAGES64, "the work area and the inverse factor");
+    diag_factor64(S, d, dT, min(64, F.r - j * 64), 64, lane, wave, [&](int failed, double pmin, double pmax) {
+      if (lane != 0) return;
+      int bad = failed ? j * 64 + failed : 0;
+      if (j > 0) {
+        const int before = __hip_atomic_load(F.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before) bad = before;
+        pmin = fmin(pmin, __hip_atomic_load(F.range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        pmax = fmax(pmax, __hip_atomic_load(F.range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      }
       __hip_atomic_store(F.bad, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(F.range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(F.range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (j == rT - 1) {
         const bool healthy = bad == 0 && pmin >= F.ratio * pmax && pmax > 0.0;
         __hip_atomic_store(F.sick, healthy ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (F.info) *F.info = bad;
       }
-    }
+    });
+    double* const Dw = T + (long long)j * 64 * rp + j * 64;
+    for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * DIAG_P + (e >> 6)];
     return;
   }
   // second product, both operands to the LDS stages:  L(x, j) = W(x, j) D^T;   T(j, x) = -D W(j, x)

@@ -1,0 +1,54 @@
+"""The 64 x 64 diagonal block of the blocked Cholesky factorisations (csrc/diag64.h), through the orthonormaliser: ranks at the edges of
+its panels of 16 columns, and columns of zeros, whose pivots fail, at their first and last columns."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS32 = 2.0**-24
+
+
+def _factor(m, r, seed):
+    """Columns of a random orthonormal basis with scales between 1 and 4 and a mixing that keeps the condition below 20."""
+    g = torch.Generator().manual_seed(seed)
+    U = torch.linalg.qr(torch.randn(m, r, generator=g, dtype=torch.float64))[0]
+    V = torch.linalg.qr(torch.randn(r, r, generator=g, dtype=torch.float64))[0]
+    return (U * torch.linspace(1, 4, r, dtype=torch.float64)) @ V
+
+
+def _q64(P):
+    """Thin-QR factor with a positive diagonal of R, in 64 bits."""
+    Q, R = torch.linalg.qr(P.double())
+    return Q * torch.sign(torch.diagonal(R))
+
+
+@pytest.mark.parametrize("r", [1, 8, 15, 16, 17, 24, 40, 48, 63, 64, 65, 80, 127, 128, 200])
+@pytest.mark.parametrize("qr_method", ["qr", "cqr"])
+def test_ranks_at_the_edges_of_the_panels(r, qr_method):
+    from dion_amd.newton_schulz import orthonormalize
+
+    m = 4 * r + 24
+    P = torch.stack([_factor(m, r, s) for s in range(3)]).float()
+    # fp64 pass: the result is rounded once, 2^-24 of an entry, which is at most 1; and the pass works in fp64.
+    # fp32 pass alone: sums of m products of fp32 numbers, and the condition (4) squared: 16 eps sqrt(m) a column and a
+    # hundred times that as the safe side.
+    passes = 1 if qr_method == "qr" else 2
+    tol = 4 * EPS32 if qr_method == "qr" else 100 * 16 * EPS32 * m**0.5
+    Q, info = orthonormalize(P.cuda(), passes=passes, qr_method=qr_method, return_info=True)
+    assert not info.any()
+    for b in range(3):
+        assert (Q[b].cpu().double() - _q64(P[b])).norm() <= tol * r**0.5
+
+
+@pytest.mark.parametrize("col", [0, 5, 15, 16, 31, 32, 47, 48, 63, 64, 79])
+def test_a_column_of_zeros_is_dropped_and_reported(col):
+    from dion_amd.newton_schulz import orthonormalize
+
+    m, r = 300, 80
+    P = torch.stack([_factor(m, r, s) for s in range(2)]).float()
+    P[1, :, col] = 0
+    Q, info = orthonormalize(P.cuda(), passes=1, qr_method="qr", return_info=True)
+    assert info.tolist() == [0, col + 1]
+    assert not Q[1, :, col].any()
+    keep = [j for j in range(r) if j != col]
+    assert (Q[1].cpu().double()[:, keep] - _q64(P[1][:, keep])).norm() <= 4 * EPS32 * r**0.5
+    assert (Q[0].cpu().double() - _q64(P[0])).norm() <= 4 * EPS32 * r**0.5
