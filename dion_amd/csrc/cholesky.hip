@@ -3,13 +3,10 @@
 // diagonal block on the matrix cores and inverts the triangular factor (redundantly -- the factor is
 // the serial part; a few workgroups per matrix repeat it rather than wait for one), then they share
 // the 64 x 64 pieces of what depends on it:
-//   role 0            : stores the inverse D_j of L_jj (the diagonal block of W, see below),
-//   roles 1 .. below  : one 64-row tile of the panel   L[i, j] = A[i, j] D_j^T,
-//   roles above that  : one 64-column tile of          W[j, c] = -D_j L[j, c],  c < j,
-// where W is the block-lower-triangular matrix with which the triangular solve of P becomes one
-// in-place GEMM per block column:  P[:, j] <- P[:, 0 .. j] W[j, 0 .. j]^T.
-// A second form of the kernel (INV) writes, instead of W's row block, row block j of T = L^-1 itself:
-//   T[j, j] = D_j,   T[j, c] = -D_j sum_{k = c .. j-1} L[j, k] T[k, c],   c < j,
+//   role 0            : stores the inverse D_j of L_jj,
+//   roles 1 .. below  : one 64-row tile of the panel   L[i, j] = A[i, j] D_j^T.
+// A second form of the kernel (INV) writes row block j of T = L^-1 as well,
+//   roles above that  : T[j, j] = D_j,   T[j, c] = -D_j sum_{k = c .. j-1} L[j, k] T[k, c],   c < j,
 // for the callers that need the inverse factor as a matrix.
 // Deferred trailing update (o_prev >= 0): the rank-64 update of the previous step, A[i, c] -= L[i, p] L[c, p]^T
 // (p = the previous block column), has not been applied to the matrix.  This launch applies it where it needs it
@@ -31,7 +28,7 @@ constexpr int LP = DIAG_P;   // LDS pitch of the operand tiles: transposed store
 
 template <typename T, bool INV>
 __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __restrict__ Lmat,
-                                                        T* __restrict__ Wmat, T* __restrict__ Tmat, long long sG, int r,
+                                                        T* __restrict__ Tmat, long long sG, int r,
                                                         int o, int nb, int below, int* __restrict__ info, int fresh,
                                                         const int* gate, int gate_want, int o_prev, int c_end, int per, int t_row, int n_t,
                                                         int t_inline, T* __restrict__ pstat) {
@@ -53,9 +50,9 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
   const bool defer = o_prev >= 0;
   const T* g = G + (long long)b * sG + (long long)o * r + o;
   // The workgroups of one matrix share its roles round-robin (role 0: D_j and the status word; 1 .. below:
-  // panel tiles; the rest: W tiles).  The operand tile of a product does not depend on this step's factor: it is
+  // panel tiles; the rest: T tiles).  The operand tile of a product does not depend on this step's factor: it is
   // requested now, 16 elements per thread, and the next one while the previous product runs.
-  const int nroles = 1 + below + ((!INV || t_inline) ? o / NB : 0);
+  const int nroles = 1 + below + (INV && t_inline ? o / NB : 0);
   // row block of T that the T roles work on: this step's, or an earlier one in the workgroups that only do that
   int t_o = o, t_nb = nb;
   // A 64 x 64 tile in registers: thread t holds the four elements (row (t >> 4) + 16 q, columns 4 (t & 15) .. + 3),
@@ -260,17 +257,14 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
     }
   }
   auto fetch = [&](int role) __attribute__((always_inline)) {
-    const bool panel = role <= below;
-    if (INV && !panel) {
+    if (INV && role > below) {
       fetch_t(role - 1 - below, role - 1 - below);
-      return;
-    }
-    const int row0 = o + nb + (role - 1) * NB;
-    if (panel) {
+    } else {
+      const int row0 = o + nb + (role - 1) * NB;
       DA_LOAD_TILE(pa0, pa1, pa2, pa3, G + (long long)b * sG + (long long)row0 * r + o, r - row0 < NB ? r - row0 : NB, nb);
       // (deferred update: L[i, p] as well)
       if (defer) DA_LOAD_TILE(pb0, pb1, pb2, pb3, Lmat + (long long)b * sG + (long long)row0 * r + o_prev, r - row0 < NB ? r - row0 : NB, NB);
-    } else DA_LOAD_TILE(pa0, pa1, pa2, pa3, Lmat + (long long)b * sG + (long long)o * r + (role - 1 - below) * NB, nb, NB);
+    }
   };
   int role = wg == 0 ? per : wg;   // this workgroup's first product (`per` workgroups share the roles)
   // (the two tiles of a T role would stay in registers through the whole factor loop: those are requested after it)
@@ -293,7 +287,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
 
   // ---- the 64 x 64 x 64 products that depend on the factor: C[m][n] = sum_k opa[k][m] * opb[k][n]
   if (wg == 0) {
-    T* w = (INV ? Tmat : Wmat) + (long long)b * sG + (long long)o * r + o;
+    T* w = Tmat + (long long)b * sG + (long long)o * r + o;
     for (int e = tid; e < NB * NB; e += 256) {
       const int i = e >> 6, j = e & 63;
       if (i < nb && j < nb) w[(long long)i * r + j] = dT[j * LP + i];
@@ -301,14 +295,13 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
   }
   if (role < nroles && !early) fetch(role);
   while (role < nroles) {
-    const bool panel = role <= below;
-    if (INV && !panel) {
+    if (INV && role > below) {
       const int next = role + per;
       t_tile(role - 1 - below, o / NB, true, next < nroles ? next : -1, fetch);
       role = next;
       continue;
     }
-    if (defer && panel) {
+    if (defer) {
       // the deferred update of this tile first:  A[i, j] -= L[i, p] L[j, p]^T
       __syncthreads();                                 // `op` may still be read
       DA_STORE_TILE(pb0, pb1, pb2, pb3, op, true);     // opa[k][m] = L[i, p][m][k]
@@ -337,25 +330,19 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
       }
     }
     __syncthreads();   // `op` may still be read (the previous product's MFMAs)
-    // panel: opa[k][m] = A[row0 + m][o + k];  W: opb[k][n] = L[o + k][col0 + n]
-    DA_STORE_TILE(pa0, pa1, pa2, pa3, op, panel);
+    DA_STORE_TILE(pa0, pa1, pa2, pa3, op, true);   // opa[k][m] = A[row0 + m][o + k]
     const int next = role + per;
     if (next < nroles) fetch(next);   // in flight during this role's product
     __syncthreads();
-    const int row0 = panel ? o + nb + (role - 1) * NB : o;
-    const int col0 = panel ? o : (role - 1 - below) * NB;   // (W: col0 + 64 <= o)
-    const int rows_ok = panel ? (r - row0 < NB ? r - row0 : NB) : nb;
-    const int cols_ok = panel ? nb : NB;
-    const T* opa = panel ? op : dT;
-    const T* opb = panel ? dT : op;
+    const int row0 = o + nb + (role - 1) * NB;
+    const int rows_ok = r - row0 < NB ? r - row0 : NB;
     acc_t acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-    mma_tile(opa, opb, acc);
-    T* dst = (panel ? Lmat : Wmat) + (long long)b * sG + (long long)row0 * r + col0;
-    const T sign = panel ? T(1) : T(-1);
+    mma_tile(op, dT, acc);
+    T* dst = Lmat + (long long)b * sG + (long long)row0 * r + o;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -364,7 +351,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
         for (int v = 0; v < 4; ++v) {
           const int m = wm * 32 + i * 16 + Mfma<T>::row(v, lane);
           const int n = wn * 32 + j * 16 + (lane & 15);
-          if (m < rows_ok && n < cols_ok) dst[(long long)m * r + n] = sign * acc[i][j][v];
+          if (m < rows_ok && n < nb) dst[(long long)m * r + n] = acc[i][j][v];
         }
     role = next;
   }
@@ -374,7 +361,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
 #undef DA_STORE_TILE
 
 template <typename T, bool INV>
-int chol_step(T* G, T* Lmat, T* Wmat, T* Tmat, long long sG, int r, int o, int nb, int* info, int batch,
+int chol_step(T* G, T* Lmat, T* Tmat, long long sG, int r, int o, int nb, int* info, int batch,
               DaGate gate, bool fresh, int o_prev, int c_end, int t_row, int t_inline, T* pstat, hipStream_t s) {
   if (nb <= 0 || nb > NB || o < 0 || o + nb > r || (o % NB) != 0 || batch <= 0 || batch > 65535) return DA_ERR_ARG;
   if (o_prev >= 0 && (o_prev != o - NB || c_end < o + nb || c_end > r)) return DA_ERR_ARG;
@@ -385,7 +372,7 @@ int chol_step(T* G, T* Lmat, T* Wmat, T* Tmat, long long sG, int r, int o, int n
   // workgroups per matrix: as many as fit one per CU over the batch (the factorisation every workgroup repeats is
   // bound by fp64 instruction issue, which two workgroups on a CU would share: 384 instead of 256 in flight cost
   // 3 % of the orthonormaliser on a 48-matrix bucket), never more than there are roles
-  const int nroles = 1 + below + ((!INV || t_inline) ? o / NB : 0);
+  const int nroles = 1 + below + (INV && t_inline ? o / NB : 0);
   if (t_row >= 0 && (!INV || t_row < 1 || t_row * NB >= o)) return DA_ERR_ARG;   // an earlier row with tiles left of its diagonal
   int per = 256 / batch;
   if (per < 1) per = 1;
@@ -413,25 +400,25 @@ int chol_step(T* G, T* Lmat, T* Wmat, T* Tmat, long long sG, int r, int o, int n
     const int cap = 512 / batch > 1 ? 512 / batch : 1;
     n_t = t_row < cap ? t_row : cap;
   }
-  hipLaunchKernelGGL((chol_step_kernel<T, INV>), dim3(batch, per + n_t + extra), dim3(256), smem, s, G, Lmat, Wmat, Tmat, sG, r,
+  hipLaunchKernelGGL((chol_step_kernel<T, INV>), dim3(batch, per + n_t + extra), dim3(256), smem, s, G, Lmat, Tmat, sG, r,
                      o, nb, below, info, fresh ? 1 : 0, gate.flags, gate.want, o_prev, c_end, per, t_row, n_t, t_inline, pstat);
   return da_launch_status();
 }
 
 }  // namespace
 
-int da_chol_step(double* G, double* Lmat, double* Wmat, long long sG, int r, int o, int nb, int* info,
+int da_chol_step(double* G, double* Lmat, double* Dmat, long long sG, int r, int o, int nb, int* info,
                  int batch, DaGate gate, hipStream_t s, int o_prev, int c_end, double* pstat) {
-  return chol_step<double, false>(G, Lmat, Wmat, nullptr, sG, r, o, nb, info, batch, gate, false, o_prev, c_end, -1, 1, pstat, s);
+  return chol_step<double, false>(G, Lmat, Dmat, sG, r, o, nb, info, batch, gate, false, o_prev, c_end, -1, 1, pstat, s);
 }
-int da_chol_step_f32(float* G, float* Lmat, float* Wmat, long long sG, int r, int o, int nb, int* info,
+int da_chol_step_f32(float* G, float* Lmat, float* Dmat, long long sG, int r, int o, int nb, int* info,
                      int batch, DaGate gate, hipStream_t s, int o_prev, int c_end) {
   // the fp32 pass keeps its status in a word of its own, which its first block column initialises
-  return chol_step<float, false>(G, Lmat, Wmat, nullptr, sG, r, o, nb, info, batch, gate, o == 0, o_prev, c_end, -1, 1, nullptr, s);
+  return chol_step<float, false>(G, Lmat, Dmat, sG, r, o, nb, info, batch, gate, o == 0, o_prev, c_end, -1, 1, nullptr, s);
 }
 int da_chol_step_f32_inv(float* G, float* Lmat, float* Tmat, long long sG, int r, int o, int nb, int* info,
                          int batch, DaGate gate, hipStream_t s, int o_prev, int c_end, int t_row, int t_inline) {
-  return chol_step<float, true>(G, Lmat, nullptr, Tmat, sG, r, o, nb, info, batch, gate, o == 0, o_prev, c_end, t_row,
+  return chol_step<float, true>(G, Lmat, Tmat, sG, r, o, nb, info, batch, gate, o == 0, o_prev, c_end, t_row,
                                 t_inline, nullptr, s);
 }
 int da_chol_trow_f32(float* Lmat, float* Tmat, long long sG, int r, int t_row, int batch, DaGate gate, hipStream_t s) {
@@ -440,8 +427,7 @@ int da_chol_trow_f32(float* Lmat, float* Tmat, long long sG, int r, int t_row, i
   const int cap = 512 / batch > 1 ? 512 / batch : 1;
   const int n_t = t_row < cap ? t_row : cap;
   // (the attribute is set by the first factorisation step, which always precedes this launch)
-  hipLaunchKernelGGL((chol_step_kernel<float, true>), dim3(batch, n_t), dim3(256), smem, s, static_cast<float*>(nullptr), Lmat,
-                     static_cast<float*>(nullptr), Tmat, sG, r, t_row * NB, r - t_row * NB < NB ? r - t_row * NB : NB, 0,
+  hipLaunchKernelGGL((chol_step_kernel<float, true>), dim3(batch, n_t), dim3(256), smem, s, static_cast<float*>(nullptr), Lmat, Tmat, sG, r, t_row * NB, r - t_row * NB < NB ? r - t_row * NB : NB, 0,
                      static_cast<int*>(nullptr), 0, gate.flags, gate.want, -1, 0, 0, t_row, n_t, 0, static_cast<float*>(nullptr));
   return da_launch_status();
 }

@@ -416,7 +416,7 @@ struct OrthWs {
   bf16_t* Ph;      // ... bf16 copy of Pf (operand of the correction product)
   double* G;       // r x r per matrix (fp64, or fp32 in the same place): Gram matrix
   double* L;       // Cholesky factor; later the correction factor of the polishing pass
-  double* W;       // inverse-factor blocks
+  double* W;       // inverses of the factor's diagonal blocks; the fp32 pass: the inverse factor
   double* part;    // K-slice outputs of a sliced Gram product
   float* rowdef;   // r per matrix: squared defect of each row of the polishing pass's Gram matrix
   float* rowdef_part;   // ... as partial sums per 64-column block
@@ -592,7 +592,7 @@ int gram(const T* P, T* G, T* part, int batch, int rows, int r, int r_live, floa
 // Most 64 x 64 tiles (over the batch) a trailing update may have to ride along in the next step's launch.
 const long long DA_CHOL_DEFER_TILES = [] { const char* e = getenv("DION_AMD_CHOL_DEFER_TILES"); const long long v = e ? atoll(e) : 0; return v > 0 ? v : 256; }();
 
-// Panel width (in 64-column steps) of the two-level blocking of chol_factor / apply_rinv.
+// Panel width (in 64-column steps) of the two-level blocking of chol_factor.
 int chol_panel_steps(int nblk, bool fallback) {
   static const int pw_env = [] {
     const char* e = getenv("DION_AMD_CHOL_PANEL");
@@ -604,8 +604,8 @@ int chol_panel_steps(int nblk, bool fallback) {
   return fallback ? nblk : pw_env;
 }
 
-// Blocked lower Cholesky G = L L^T of each r x r matrix (G is overwritten), with the inverse-factor blocks W that
-// apply_rinv uses.
+// Blocked lower Cholesky G = L L^T of each r x r matrix (G is overwritten); the diagonal blocks of W receive the inverses of
+// the diagonal blocks of L, for da_solve_rows.
 template <typename T>
 int chol_factor(T* G, T* L, T* W, int batch, int r, int* info, DaGate gate, hipStream_t s, T* pstat = nullptr) {
   const int NB = DA_CHOL_NB;
@@ -620,7 +620,6 @@ int chol_factor(T* G, T* L, T* W, int batch, int r, int* info, DaGate gate, hipS
   // (the rank-64 updates inside a panel ride along in the next step's launch instead of taking one of their own)
   static const bool defer = [] { const char* e = getenv("DION_AMD_CHOL_NO_DEFER"); return !(e && atoi(e)); }();
   bool pending = false;   // the previous step left its update to the next launch
-  // blocked lower Cholesky G = L L^T, building W alongside
   for (int j = 0; j < nblk; ++j) {
     const int o = j * NB, nb = r - o < NB ? r - o : NB, rest = r - o - nb;
     const int p0 = j / pw * pw * NB;                       // first column of the panel
@@ -664,51 +663,6 @@ int chol_factor(T* G, T* L, T* W, int batch, int r, int* info, DaGate gate, hipS
   return DA_OK;
 }
 
-// P0 <- P0 R^-1 with R = L^T (L, W from chol_factor), in place, `rows` rows per matrix.
-template <typename T>
-int apply_rinv(T* P0, const T* L, const T* W, int batch, int rows, int r, DaGate gate, hipStream_t s) {
-  const int NB = DA_CHOL_NB;
-  const int nblk = (r + NB - 1) / NB;
-  const long long pr = (long long)rows * r, rr = (long long)r * r;
-  const int pw = chol_panel_steps(nblk, gate.flags != nullptr);
-  int rc = DA_OK;
-  // By the panels of the factorisation: first the solved columns left of the panel are
-  // taken out of it in one product,
-  //   P0[:, panel] -= P0[:, 0 .. p0] L[panel, 0 .. p0]^T
-  // then block column by block column inside it
-  //   P0[:, j] <- P0[:, p0 .. j] W[j, p0 .. j]^T
-  // (each workgroup owns 64 rows and the one 64-column output tile, and has read all it needs of
-  // those rows before it stores)
-  for (int j = 0; j < nblk; ++j) {
-    const int o = j * NB, nb = r - o < NB ? r - o : NB;
-    const int p0 = j / pw * pw * NB;
-    const int pe = p0 + pw * NB < r ? p0 + pw * NB : r;
-    if (o == p0 && p0 > 0) {
-      RealGemmDesc<T> u{};
-      u.batch = batch;
-      u.A = P0; u.sA = pr; u.lda = r; u.a_kstrided = 0;
-      u.B = L + (long long)p0 * r; u.sB = rr; u.ldb = r; u.b_kstrided = 0;
-      u.C = P0 + p0; u.sC = pr; u.ldc = r;
-      u.E = u.C; u.sE = pr; u.lde = r;
-      u.M = rows; u.N = pe - p0; u.K = p0; u.alpha = -1.0; u.beta = 1.0;
-      u.gate = gate.flags; u.gate_want = gate.want;
-      rc = gemm_real(u, s);
-      if (rc) return rc;
-    }
-    RealGemmDesc<T> a{};
-    a.batch = batch;
-    a.A = P0 + p0; a.sA = pr; a.lda = r; a.a_kstrided = 0;
-    a.B = W + (long long)o * r + p0; a.sB = rr; a.ldb = r; a.b_kstrided = 0;
-    a.C = P0 + o; a.sC = pr; a.ldc = r;
-    a.E = nullptr;
-    a.M = rows; a.N = nb; a.K = o + nb - p0; a.alpha = 1.0; a.beta = 0.0;
-    a.gate = gate.flags; a.gate_want = gate.want;
-    rc = gemm_real(a, s);
-    if (rc) return rc;
-  }
-  return DA_OK;
-}
-
 // One blocked CholeskyQR pass in precision T, in place:  P <- P R^-1  with  P^T P = R^T R.
 template <typename T>
 int cholqr_pass(T* P0, T* G, T* L, T* W, T* part, int batch, int rows, int r, int r_live, int* info, DaGate gate,
@@ -717,7 +671,7 @@ int cholqr_pass(T* P0, T* G, T* L, T* W, T* part, int batch, int rows, int r, in
   if (rc) return rc;
   rc = chol_factor<T>(G, L, W, batch, r, info, gate, s, pstat);
   if (rc) return rc;
-  return apply_rinv<T>(P0, L, W, batch, rows, r, gate, s);
+  return da_solve_rows(P0, L, W, batch, rows, r, gate, s);
 }
 
 // V = I - up(G - I) for each r x r Gram matrix G of an almost orthonormal P, where up() keeps the strict
@@ -986,28 +940,28 @@ int gram16(const bf16_t* H, const bf16_t* Lo, float* G, float* part, int batch, 
   return da_launch_status();
 }
 
-// T = identity (r x r per matrix)
-__global__ __launch_bounds__(256) void eye_kernel(float* __restrict__ T, long long rr, int r) {
-  const long long b = blockIdx.y;
-  const int i = blockIdx.x;
-  for (int j = threadIdx.x; j < r; j += 256) T[b * rr + (long long)i * r + j] = i == j ? 1.f : 0.f;
-}
-
-// Tcat[k][0 .. r) = bf16(T[k][:]), Tcat[k][r .. 2r) = bf16(T[k][:] - that): T to 16 bits as two bf16 factors
-// `stacked`: [T_hi; T_lo] (2r x r) instead of [T_hi | T_lo] (r x 2r).  `lower`: the source holds L^-1 (lower
-// triangular, blocks of 64 above the diagonal never written) and T = R^-1 is its transpose.
-__global__ __launch_bounds__(256) void split_factor_kernel(const float* __restrict__ T, bf16_t* __restrict__ Tcat,
-                                                           long long rr, int r, int stacked, int lower) {
-  const long long b = blockIdx.y;
-  const int k = blockIdx.x;
-  const float* t = T + b * rr + (long long)k * r;
-  bf16_t* o = Tcat + b * 2 * rr + (long long)k * (stacked ? r : 2 * r);
-  const long long lo = stacked ? rr : r;
-  for (int j = threadIdx.x; j < r; j += 256) {
-    const float v = !lower ? t[j] : ((j >> 6) >= (k >> 6) ? T[b * rr + (long long)j * r + k] : 0.f);
+// T = R^-1 to 16 bits as two bf16 factors, side by side [T_hi | T_lo] (r x 2r) or `stacked` [T_hi; T_lo] (2r x r), from its
+// transpose Li = L^-1 (lower triangular; what lies in blocks of 64 above the diagonal was never written and counts as zero).  A
+// 64 x 64 tile per workgroup, turned in LDS (read along the columns of Li, a line of its own for every lane, it took 25 us and
+// more for 12 matrices of rank 768 instead of 12).
+__global__ __launch_bounds__(256) void split_factor_kernel(const float* __restrict__ Li, bf16_t* __restrict__ Tcat,
+                                                           long long rr, int r, int stacked) {
+  __shared__ float tile[64][65];
+  const long long b = blockIdx.z;
+  const int k0 = blockIdx.y * 64, j0 = blockIdx.x * 64;   // rows and columns of T
+  const int c = threadIdx.x & 63, q = threadIdx.x >> 6;
+  if (j0 >= k0) {
+    for (int i = q; i < 64; i += 4)
+      tile[i][c] = j0 + i < r && k0 + c < r ? Li[b * rr + (long long)(j0 + i) * r + k0 + c] : 0.f;
+  }
+  __syncthreads();
+  if (j0 + c >= r) return;
+  for (int i = q; i < 64 && k0 + i < r; i += 4) {
+    bf16_t* const o = Tcat + b * 2 * rr + (long long)(k0 + i) * (stacked ? r : 2 * r) + j0 + c;
+    const float v = j0 >= k0 ? tile[c][i] : 0.f;
     const bf16_t h = f2bf(v);
-    o[j] = h;
-    o[lo + j] = f2bf(v - bf2f(h));
+    o[0] = h;
+    o[stacked ? rr : r] = f2bf(v - bf2f(h));
   }
 }
 
@@ -1046,28 +1000,23 @@ int fast16_pass(const bf16_t* P, const OrthWs& w, int batch, int rows, int r, in
   const DaGate all{nullptr, 0};
   float* G = reinterpret_cast<float*>(w.G);
   float* L = reinterpret_cast<float*>(w.L);
-  float* W = reinterpret_cast<float*>(w.W);
-  float* T = W + rr * batch;                          // second half of W's room
-  bf16_t* Tcat = reinterpret_cast<bf16_t*>(w.L);      // over the factor L, which is dead once W is complete
+  float* T = reinterpret_cast<float*>(w.W);
+  bf16_t* Tcat = reinterpret_cast<bf16_t*>(w.L);      // over the factor L, which is dead once T is complete
   float* C2 = reinterpret_cast<float*>(w.P0);         // rows x 2r fp32 = the room of the fp64 copy
   bf16_t* Lo = reinterpret_cast<bf16_t*>(w.Pf);
   float* part = reinterpret_cast<float*>(w.part);
   int rc = gram16(P, nullptr, G, part, batch, rows, r, r_live, nullptr, nullptr, all, s);
   if (rc) return rc;
-  // (the steps write the rows of L^-1 themselves: no W, no recurrence on the identity afterwards)
-  static const bool inv_rows = [] { const char* e = getenv("DION_AMD_ORTH_NO_INV"); return !(e && atoi(e)); }();
   // (every step's trailing update rides along in the next step's launch)
   static const bool defer = [] { const char* e = getenv("DION_AMD_CHOL_NO_DEFER"); return !(e && atoi(e)); }();
   static const bool lag_on = [] { const char* e = getenv("DION_AMD_CHOL_NO_TLAG"); return !(e && atoi(e)); }();
-  const bool lag = inv_rows && lag_on && nblk >= 4;   // (short chains: the extra launch at the end costs what the lag saves)
+  const bool lag = lag_on && nblk >= 4;   // (short chains: the extra launch at the end costs what the lag saves)
   bool pending = false;
   for (int j = 0; j < nblk; ++j) {
     const int o = j * NB, nb = r - o < NB ? r - o : NB, rest = r - o - nb;
     const int o_prev = pending ? o - NB : -1;
     // (the rows of L^-1 lag one step behind: row j - 1 is formed by workgroups of step j's launch that do nothing else)
-    rc = inv_rows ? da_chol_step_f32_inv(G, L, T, rr, r, o, nb, w.info32, batch, all, s, o_prev, r,
-                                         lag && j >= 2 ? j - 1 : -1, lag ? 0 : 1)
-                  : da_chol_step_f32(G, L, W, rr, r, o, nb, w.info32, batch, all, s, o_prev, r);
+    rc = da_chol_step_f32_inv(G, L, T, rr, r, o, nb, w.info32, batch, all, s, o_prev, r, lag && j >= 2 ? j - 1 : -1, lag ? 0 : 1);
     pending = false;
     if (rc) return rc;
     if (rest <= 0) break;
@@ -1088,29 +1037,12 @@ int fast16_pass(const bf16_t* P, const OrthWs& w, int batch, int rows, int r, in
     rc = da_chol_trow_f32(L, T, rr, r, nblk - 1, batch, all, s);
     if (rc) return rc;
   }
-  if (!inv_rows) {
-    hipLaunchKernelGGL(eye_kernel, dim3((unsigned)r, (unsigned)batch), dim3(256), 0, s, T, rr, r);
-    rc = da_launch_status();
-    if (rc) return rc;
-  }
-  for (int j = 0; j < nblk && !inv_rows; ++j) {
-    const int o = j * NB, nb = r - o < NB ? r - o : NB;
-    Gemm32Desc a{};
-    a.batch = batch;
-    a.A = T; a.sA = rr; a.lda = r; a.a_kstrided = 0;
-    a.B = W + (long long)o * r; a.sB = rr; a.ldb = r; a.b_kstrided = 0;
-    a.C = T + o; a.sC = rr; a.ldc = r;
-    // rows below block j of T are zero in these columns (T is upper triangular): only rows < o + nb are needed
-    a.M = o + nb; a.N = nb; a.K = o + nb; a.alpha = 1.0; a.beta = 0.0;
-    rc = da_gemm_f32s(a, s);
-    if (rc) return rc;
-  }
   // P1 = P T_hi + P T_lo.  With whole 64-deep stages (r a multiple of 64) it is ONE accumulation over the stacked
   // factor [T_hi; T_lo], P read twice along k, and the product leaves the kernel as h + l; otherwise the two
   // products go side by side into an fp32 matrix and a pass of its own adds and splits them.
   const bool stacked = r % 64 == 0 && rows % 128 == 0 && (Lo - w.Ph) % 8 == 0;
-  hipLaunchKernelGGL(split_factor_kernel, dim3((unsigned)r, (unsigned)batch), dim3(256), 0, s, T, Tcat, rr, r,
-                     stacked ? 1 : 0, inv_rows ? 1 : 0);
+  hipLaunchKernelGGL(split_factor_kernel, dim3((unsigned)nblk, (unsigned)nblk, (unsigned)batch), dim3(256), 0, s, T, Tcat, rr, r,
+                     stacked ? 1 : 0);
   rc = da_launch_status();
   if (rc) return rc;
   if (stacked) {
@@ -1384,7 +1316,7 @@ int da_orthonormalize_sketch(const void* P, const void* S, void* out, int dtype,
   // ---- P1 = P R1^-1
   rc = da_cvt_to_f64(P, dtype, w.P0, pr, batch, all, s);
   if (rc) return rc;
-  rc = apply_rinv<double>(w.P0, w.L, w.W, batch, rows, r, all, s);
+  rc = da_solve_rows(w.P0, w.L, w.W, batch, rows, r, all, s);
   if (rc) return rc;
   // ---- Cholesky QR of the preconditioned factor
   rc = cholqr_pass<double>(w.P0, w.G, w.L, w.W, w.part, batch, rows, r, r_live, info, all, s);

@@ -70,11 +70,16 @@ int da_cvt_f32_to_bf16(const float* src, bf16_t* low, long long per, int batch, 
 // dst (bf16 / f32) <- src (f32)
 int da_cvt_from_f32(const float* src, void* dst, int dst_dtype, long long per, int batch, DaGate gate, hipStream_t s);
 
+// P[b] <- P[b] L[b]^-T in place, P: rows x r, L: the blocks below the diagonal of a lower Cholesky factor in blocks of 64, D: the
+// inverses of its diagonal blocks (r x r arrays with those blocks filled), as da_chol_step leaves them.
+int da_solve_rows(double* P, const double* L, const double* D, int batch, int rows, int r, DaGate g, hipStream_t s);
+int da_solve_rows(float* P, const float* L, const float* D, int batch, int rows, int r, DaGate g, hipStream_t s);
+
 // Block-column step j = o / 64 of the blocked lower Cholesky G = L L^T of each r x r matrix
 // G[b] (o a multiple of 64; nb = 64 except for a ragged last block): factors the nb x nb diagonal
 // block at offset o (the trailing updates of earlier steps already applied to G), writes the panel
-// L[o+nb.., o..o+nb] into Lmat[b] (L_jj itself is not stored), and row block j of W[b] (D_j = L_jj^-1 on the
-// diagonal, -D_j L[j, c] left of it).  A non-positive or non-finite pivot zeroes that column (of
+// L[o+nb.., o..o+nb] into Lmat[b] (L_jj itself is not stored), and D_j = L_jj^-1 into the
+// diagonal block j of Dmat[b].  A non-positive or non-finite pivot zeroes that column (of
 // L_jj and of D_j) and records (o + column + 1) in info[b] if it is the matrix's first failure.
 // `gate`: as in RealGemmDesc.
 // o_prev >= 0 (= o - 64): the trailing update of the previous step, A[i, c] -= L[i, p] L[c, p]^T with p the
@@ -83,11 +88,11 @@ int da_cvt_from_f32(const float* src, void* dst, int dst_dtype, long long per, i
 // so that no separate update launch runs between two steps.  Columns >= c_end are left to the caller.
 // pstat (fp64 form, may be null): two words per matrix, the smallest and the largest pivot met so far (step o == 0
 // starts them): the squares of R's diagonal, whose ratio bounds cond(R)^2 from below.
-int da_chol_step(double* G, double* Lmat, double* Wmat, long long sG, int r, int o, int nb, int* info,
+int da_chol_step(double* G, double* Lmat, double* Dmat, long long sG, int r, int o, int nb, int* info,
                  int batch, DaGate gate, hipStream_t s, int o_prev = -1, int c_end = 0, double* pstat = nullptr);
-int da_chol_step_f32(float* G, float* Lmat, float* Wmat, long long sG, int r, int o, int nb, int* info,
+int da_chol_step_f32(float* G, float* Lmat, float* Dmat, long long sG, int r, int o, int nb, int* info,
                      int batch, DaGate gate, hipStream_t s, int o_prev = -1, int c_end = 0);
-// The same step, but instead of the row block of W it writes row block j of T = L^-1 itself into Tmat (lower
+// The same step, but instead of D_j alone it writes row block j of T = L^-1 itself into Tmat (lower
 // triangular, row-major): T[j, j] = D_j and T[j, c] = -D_j sum_{k = c .. j-1} L[j, k] T[k, c] for c < j, from the
 // rows of T that the earlier steps left.  After the last step Tmat holds L^-1 (blocks above the diagonal untouched).
 // t_inline = 0: the step leaves the tiles of its row of T left of the diagonal to a later launch (it writes D_j only);

@@ -5,18 +5,121 @@
 //
 //   C[b] (M x N) = alpha * sum_k Aop[b](i,k) * Bop[b](j,k) + beta * E[b]
 //
-// 256 threads (2 x 2 wavefronts) per 64 x 64 tile, 16 k per stage; each wavefront owns
-// 32 x 32 as 2 x 2 accumulators of 16 x 16.  LDS tiles are k-major [16][64] doubles for
-// either operand layout, so the one-double-per-lane MFMA operands are conflict-free reads.
-// Double buffered: the global loads of the next stage are in flight during the MFMAs.
+// 256 threads (2 x 2 wavefronts) per 64 x 64 tile; each wavefront owns 32 x 32 as 2 x 2 accumulators of 16 x 16.
+// Interior tiles run a ring of two stages filled by direct-to-LDS loads (ring_loop): a stage 128 bytes deep costs a wavefront four
+// load instructions and no registers, ALU work or LDS stores, and its 16 KB leave room for five workgroups on a compute unit.
+// 48 Gram products of 768 x 768: 394 us with stages through registers, 375 now (63 TFLOP/s of 78.6); with rings of three and four
+// stages, three and two workgroups, 453 and 532: what hides the latency here are the other workgroups.
+// Other tiles go through registers, 16 k per stage, k-major LDS tiles, with the loads of the next stage in flight during the MFMAs.
 // The same template is instantiated for fp32 (v_mfma_f32_16x16x4_f32; the polishing passes); the
 // result may be stored as fp32 or bf16, and a block-triangular B operand shortens the sum per
 // column tile.
 #include "gemm_f64.h"
+#include "mfma_tile.h"
 
 namespace {
 
-constexpr int BK = 16;
+constexpr int RK = 16;             // depth of a stage through registers
+
+// ---- the K loop of interior tiles: direct-to-LDS loads, a ring of two stages ------------------------------------------------
+// A stage is 128 bytes deep: 16 k (fp64) or 32 k (fp32).  LDS layouts of an operand of R rows:
+//   k-contiguous: [R][128 bytes], 16-byte chunks exchanged by (row >> 1) & 7: the 16 rows x 4 k of an operand read cover every bank once;
+//   k-strided:    [depth][R elements] as in memory, chunks exchanged by k so that the k of a read fall into different banks.
+template <typename T> struct Ring {
+  static constexpr int D = 128 / (int)sizeof(T);                     // depth
+  static constexpr int EPC = 16 / (int)sizeof(T);                    // elements of a chunk
+  static constexpr int bytes(int rows) { return rows * 128; }
+  // chunk exchange of a k-strided row
+  static __device__ __forceinline__ int ks_chunk(int c, int k) { return sizeof(T) == 8 ? c ^ ((k & 1) << 3) : c ^ ((k & 3) << 2); }
+};
+// Requests one operand's stage: wavefront instruction i of R / 8 in all fills the 1 KB block i, lane p its p-th 16 bytes.
+template <typename T, bool KS, int R>
+struct RingAddr {
+  static constexpr int PER = R / 32;          // instructions per wavefront (4 wavefronts)
+  const char* base;
+  unsigned off[PER];
+  unsigned step;
+  __device__ __forceinline__ RingAddr(const T* p, int ld, int row0, int k0, int wave, int lane) {
+    typedef Ring<T> G;
+    if (!KS) {
+      base = reinterpret_cast<const char*>(p + (long long)row0 * ld + k0);
+      step = 128u;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int row = (i * 4 + wave) * 8 + (lane >> 3);
+        off[i] = (unsigned)(row * ld) * (unsigned)sizeof(T) + (unsigned)((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+      }
+    } else {
+      constexpr int CPR = R * (int)sizeof(T) / 16;   // chunks of a k-row
+      base = reinterpret_cast<const char*>(p + (long long)k0 * ld + row0);
+      step = (unsigned)(G::D * ld) * (unsigned)sizeof(T);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int c = (i * 4 + wave) * 64 + lane, k = c / CPR;
+        off[i] = (unsigned)(k * ld) * (unsigned)sizeof(T) + (unsigned)G::ks_chunk(c % CPR, k) * 16u;
+      }
+    }
+  }
+  __device__ __forceinline__ void request(unsigned lds, int wave) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      dma16(base, off[i], lds + (i * 4 + wave) * 1024);
+      off[i] += step;
+    }
+  }
+};
+template <typename T, bool KS, int R> __device__ __forceinline__ T ring_read(const char* st, int row, int k) {
+  if (!KS) {
+    const int byte = k * (int)sizeof(T);
+    return *reinterpret_cast<const T*>(st + row * 128 + (((byte >> 4) ^ ((row >> 1) & 7)) << 4) + (byte & 15));
+  }
+  const int byte = row * (int)sizeof(T);
+  return *reinterpret_cast<const T*>(st + k * (R * (int)sizeof(T)) + (Ring<T>::ks_chunk(byte >> 4, k) << 4) + (byte & 15));
+}
+// a tile's operand within reach of 32-bit offsets
+template <typename T, bool KS> __device__ __forceinline__ bool ring_span(int ld, int K) {
+  return (long long)(KS ? K : 64) * ld * (long long)sizeof(T) + (KS ? 512 : (long long)K * (long long)sizeof(T)) < (1LL << 32);
+}
+// acc[TI][2] += A-rows (RA of them from m0) x B-rows (64 from n0) over KT stages from k0; lds: 2 * 128 * (RA + 64) bytes, free on
+// entry.  No barrier behind the last stage.
+template <typename T, bool A_KS, bool B_KS, int RA>
+__device__ __forceinline__ void ring_loop(typename Mfma<T>::acc_t (&acc)[RA / 32][2], const T* A, int lda, int m0, const T* B, int ldb, int n0,
+                                          int k0, int KT, char* lds, int lane, int wave, int wm, int wn) {
+  typedef Ring<T> G;
+  constexpr int TI = RA / 32, ST = 128 * (RA + 64);
+  if (KT <= 0) return;
+  RingAddr<T, A_KS, RA> ra(A, lda, m0, k0, wave, lane);
+  RingAddr<T, B_KS, 64> rb(B, ldb, n0, k0, wave, lane);
+  const unsigned l0 = lds_addr(lds);
+  const int lc = lane & 15, lg = lane >> 4;
+  ra.request(l0, wave);
+  rb.request(l0 + RA * 128, wave);
+  for (int kt = 0; kt < KT; ++kt) {
+    dma_wait();
+    __syncthreads();
+    if (kt + 1 < KT) {   // into the buffer whose last readers are past the barrier
+      const unsigned st = l0 + ((kt + 1) & 1) * ST;
+      ra.request(st, wave);
+      rb.request(st + RA * 128, wave);
+    }
+    const char* const sa = lds + (kt & 1) * ST;
+    const char* const sb = sa + RA * 128;
+#pragma unroll
+    for (int ks = 0; ks < G::D / 4; ++ks) {
+      const int k = ks * 4 + lg;
+      T af[TI], bf[2];
+#pragma unroll
+      for (int i = 0; i < TI; ++i) af[i] = ring_read<T, A_KS, RA>(sa, wm * (RA / 2) + i * 16 + lc, k);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bf[j] = ring_read<T, B_KS, 64>(sb, wn * 32 + j * 16 + lc, k);
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = Mfma<T>::mma(af[i], bf[j], acc[i][j]);
+    }
+  }
+}
+
 
 template <bool KS, typename T>
 __device__ __forceinline__ void fetch(T (&v)[4], const T* __restrict__ base, int ld, int row0, int k0,
@@ -35,15 +138,6 @@ __device__ __forceinline__ void fetch(T (&v)[4], const T* __restrict__ base, int
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (outer < outer_n && inner + e < inner_n) ? p[e] : T(0);
   }
-}
-
-// Interior tiles (all rows and k in range, 16-byte aligned rows): the same four elements with no checks.
-template <typename T>
-__device__ __forceinline__ void fetch_fast(T (&v)[4], const T* __restrict__ p) {
-  typedef T pair_t __attribute__((ext_vector_type(2)));
-  const pair_t lo = *reinterpret_cast<const pair_t*>(p);
-  const pair_t hi = *reinterpret_cast<const pair_t*>(p + 2);
-  v[0] = lo.x; v[1] = lo.y; v[2] = hi.x; v[3] = hi.y;
 }
 
 // One 64-row slice of a stage goes to the k-major LDS tile lds[k][row] (row pitch BTt).
@@ -67,8 +161,10 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
   constexpr int H = BTt / 64;        // 64-row slices per operand stage
   constexpr int WT = BTt / 2;        // wavefront tile
   constexpr int TI = WT / 16;        // 16 x 16 accumulators per wavefront and direction
-  __shared__ T lds_a[2][BK * BTt];
-  __shared__ T lds_b[2][BK * BTt];
+  static_assert(BTt == 64, "the tile of the K loop");
+  __shared__ __attribute__((aligned(16))) char lds[2 * 128 * 128];
+  T* const lds_a = reinterpret_cast<T*>(lds);
+  T* const lds_b = lds_a + 2 * RK * BTt;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int tiles_m = (d.M + BTt - 1) / BTt, tiles_n = (d.N + BTt - 1) / BTt;
@@ -106,7 +202,7 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
     for (int j = 0; j < TI; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
   // double buffered: the global loads of stage s+1 are in flight while stage s is multiplied
-  const int KT_all = (Keff + BK - 1) / BK;
+  const int KT_all = (Keff + RK - 1) / RK;
   const int per_split = (KT_all + (int)gridDim.y - 1) / (int)gridDim.y;
   const int kt0 = split * per_split;
   const int KT = KT_all - kt0 < per_split ? KT_all - kt0 : per_split;   // may be <= 0 for the last slices
@@ -114,19 +210,19 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
 #define DA_RFETCH(kt)                                                                               \
   do {                                                                                              \
     _Pragma("unroll") for (int h = 0; h < H; ++h) {                                                 \
-      fetch<A_KS>(pa[h], A, d.lda, m0 + 64 * h, (kt) * BK, d.M, Keff, tid);                         \
-      fetch<B_KS>(pb[h], B, d.ldb, n0 + 64 * h, (kt) * BK, d.N, Keff, tid);                         \
+      fetch<A_KS>(pa[h], A, d.lda, m0 + 64 * h, (kt) * RK, d.M, Keff, tid);                         \
+      fetch<B_KS>(pb[h], B, d.ldb, n0 + 64 * h, (kt) * RK, d.N, Keff, tid);                         \
     }                                                                                               \
   } while (0)
 #define DA_RPUT(buf)                                                                                \
   do {                                                                                              \
     _Pragma("unroll") for (int h = 0; h < H; ++h) {                                                 \
-      put<A_KS, BTt>(lds_a[buf] + 64 * h, pa[h], tid);                                              \
-      put<B_KS, BTt>(lds_b[buf] + 64 * h, pb[h], tid);                                              \
+      put<A_KS, BTt>(lds_a + (buf) * RK * BTt + 64 * h, pa[h], tid);                                              \
+      put<B_KS, BTt>(lds_b + (buf) * RK * BTt + 64 * h, pb[h], tid);                                              \
     }                                                                                               \
   } while (0)
 #define DA_RMMA(sa, sb)                                                                             \
-  _Pragma("unroll") for (int ks = 0; ks < BK / 4; ++ks) {                                           \
+  _Pragma("unroll") for (int ks = 0; ks < RK / 4; ++ks) {                                           \
     const int k = ks * 4 + (lane >> 4);                                                             \
     T af[TI], bfv[TI];                                                                              \
     _Pragma("unroll") for (int i = 0; i < TI; ++i) af[i] = (sa)[k * BTt + wm * WT + i * 16 + (lane & 15)];  \
@@ -134,57 +230,23 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
     _Pragma("unroll") for (int i = 0; i < TI; ++i)                                                  \
       _Pragma("unroll") for (int j = 0; j < TI; ++j) acc[i][j] = Mfma<T>::mma(af[i], bfv[j], acc[i][j]);    \
   }
-  // Interior tile with 16-byte aligned operand rows: the stage loads need no range or alignment checks and
-  // walk precomputed pointers.  (With the checks the loop issues ~380 scalar and vector ALU instructions per
-  // stage around 16 MFMAs, more issue time than the MFMAs take.)
-  const bool interior = m0 + BTt <= d.M && n0 + BTt <= d.N && Keff % BK == 0 &&
+  // Interior tile with 16-byte aligned operand rows, whole stages, operands within reach of the loads' 32-bit offsets
+  const bool interior = m0 + BTt <= d.M && n0 + BTt <= d.N && Keff % Ring<T>::D == 0 && kt0 * RK % Ring<T>::D == 0 && KT * RK % Ring<T>::D == 0 &&
+                        ring_span<T, A_KS>(d.lda, Keff) && ring_span<T, B_KS>(d.ldb, Keff) &&
                         ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 &&
                         (((long long)d.lda | (long long)d.ldb) * (long long)sizeof(T)) % 16 == 0;
   if (interior) {
-    // the thread's first element of each operand and the distance between stages
-    const T* pA[H];
-    const T* pB[H];
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-      pA[h] = A_KS ? A + (long long)(kt0 * BK + (tid >> 4)) * d.lda + m0 + 64 * h + (tid & 15) * 4
-                   : A + (long long)(m0 + 64 * h + (tid >> 2)) * d.lda + kt0 * BK + (tid & 3) * 4;
-      pB[h] = B_KS ? B + (long long)(kt0 * BK + (tid >> 4)) * d.ldb + n0 + 64 * h + (tid & 15) * 4
-                   : B + (long long)(n0 + 64 * h + (tid >> 2)) * d.ldb + kt0 * BK + (tid & 3) * 4;
-    }
-    const long long stepA = A_KS ? (long long)BK * d.lda : BK, stepB = B_KS ? (long long)BK * d.ldb : BK;
-#define DA_RFETCH_FAST()                                                                            \
-  do {                                                                                              \
-    _Pragma("unroll") for (int h = 0; h < H; ++h) {                                                 \
-      fetch_fast(pa[h], pA[h]);                                                                     \
-      fetch_fast(pb[h], pB[h]);                                                                     \
-      pA[h] += stepA;                                                                               \
-      pB[h] += stepB;                                                                               \
-    }                                                                                               \
-  } while (0)
-    if (KT > 0) {
-      DA_RFETCH_FAST();
-      DA_RPUT(0);
-    }
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      const T* sa = lds_a[kt & 1];
-      const T* sb = lds_b[kt & 1];
-      const bool more = kt + 1 < KT;
-      if (more) DA_RFETCH_FAST();
-      DA_RMMA(sa, sb)
-      if (more) DA_RPUT((kt + 1) & 1);
-      __syncthreads();
-    }
-#undef DA_RFETCH_FAST
+    ring_loop<T, A_KS, B_KS, 64>(acc, A, d.lda, m0, B, d.ldb, n0, kt0 * RK, KT * RK / Ring<T>::D, lds, lane, wave, wm, wn);
   } else {
+
     if (KT > 0) {
       DA_RFETCH(kt0);
       DA_RPUT(0);
     }
     __syncthreads();
     for (int kt = 0; kt < KT; ++kt) {
-      const T* sa = lds_a[kt & 1];
-      const T* sb = lds_b[kt & 1];
+      const T* sa = lds_a + (kt & 1) * RK * BTt;
+      const T* sb = lds_b + (kt & 1) * RK * BTt;
       const bool more = kt + 1 < KT;
       if (more) DA_RFETCH(kt0 + kt + 1);
       DA_RMMA(sa, sb)
@@ -261,6 +323,156 @@ int launch(const RealGemmDesc<T>& d, hipStream_t s) {
   if (auto_split) split = da_auto_split(blocks, d.K);
   if (split > 1 && d.split_stride < (long long)d.sC * d.batch) return DA_ERR_ARG;
   return launch_bt<T, A_KS, B_KS, SYM, BTt>(d, split, s);
+}
+
+// ---- P <- P R^-1 with R = L^T: all block columns in one launch -------------------------------------------------------------
+//
+//   X(:, j) = (P(:, j) - sum over k < j of X(:, k) L(j, k)^T) D_j^T,  D_j = L_jj^-1,  j in blocks of 64
+//
+// A workgroup owns SR rows of one matrix and walks its block columns: the sum is the K loop of the GEMM above on the X it has stored
+// itself (it reads its own stores back through its compute unit's L1), the difference goes to LDS as the operand of the
+// product with D_j, whose fragments come straight from memory.
+//
+// What bounds it: the fp64 matrix cores, and the last workgroups: SR = 32 gives a 768-row matrix 24 of them, five to a compute unit
+// at a time (the registers are held to that), so that a bucket of a few dozen matrices runs in one round.  48 matrices of
+// 768 x 768: 585 us, 40 TFLOP/s; as fifteen products over panels of four block columns (1 launch each) 570 us plus 85 us for the
+// blocks of the panels' inverses, which are no longer needed; and as the pass over flagged matrices one launch that finds
+// nothing instead of one per block column.  (Four workgroups a compute unit: 618.)
+// Workgroups of one matrix stay on one XCD (they read the same L) once there are eight matrices.
+constexpr int SR = 32;
+template <typename T, bool INTERIOR>
+__device__ __forceinline__ void solve_rows_of(T* __restrict__ P, const T* __restrict__ L, const T* __restrict__ D, int rows, int r, int row0,
+                                              T* lds, int tid, int lane, int wm, int wn) {
+  typedef typename Mfma<T>::acc_t acc_t;
+  constexpr int CB = 64;
+  const int lc = lane & 15, lg = lane >> 4;
+  T* const la = lds;                     // checked loop: [2][RK][SR]
+  T* const lb = lds + 2 * RK * SR;       // ... [2][RK][CB]
+  for (int n0 = 0; n0 < r; n0 += CB) {
+    const int nb = INTERIOR || r - n0 >= CB ? CB : r - n0;
+    acc_t old[2], acc[2];
+    T* const own = P + (long long)(row0 + wm * 16) * r + n0 + wn * 32 + lc;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int m = Mfma<T>::row(v, lane);
+        old[j][v] = INTERIOR || (row0 + wm * 16 + m < rows && wn * 32 + j * 16 + lc < nb) ? own[(long long)m * r + j * 16] : T(0);
+        acc[j][v] = T(0);
+      }
+    if constexpr (INTERIOR) {
+      // (what this workgroup stored is read back past nothing but its own L1: the stores are acknowledged first)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      acc_t ac2[1][2] = {{acc[0], acc[1]}};
+      if (n0 > 0) ring_loop<T, false, false, SR>(ac2, P, r, row0, L, r, n0, 0, n0 / Ring<T>::D, reinterpret_cast<char*>(lds), lane, wm * 2 + wn, wm, wn);
+      acc[0] = ac2[0][0];
+      acc[1] = ac2[0][1];
+      __syncthreads();
+    } else {
+      const int KT = n0 / RK;
+      T pa[4], pb[4];
+      auto stage_in = [&](int kt) __attribute__((always_inline)) {
+        if (tid < 4 * SR) fetch<false>(pa, P, r, row0, kt * RK, rows, n0, tid);
+        fetch<false>(pb, L, r, n0, kt * RK, n0 + nb, n0, tid);
+      };
+      auto stage_out = [&](int buf) __attribute__((always_inline)) {
+        if (tid < 4 * SR) put<false, SR>(la + buf * RK * SR, pa, tid);
+        put<false, CB>(lb + buf * RK * CB, pb, tid);
+      };
+      if (KT > 0) {
+        stage_in(0);
+        stage_out(0);
+      }
+      __syncthreads();
+      for (int kt = 0; kt < KT; ++kt) {
+        const T* const sa = la + (kt & 1) * RK * SR;
+        const T* const sb = lb + (kt & 1) * RK * CB;
+        const bool more = kt + 1 < KT;
+        if (more) stage_in(kt + 1);
+#pragma unroll
+        for (int ks = 0; ks < RK / 4; ++ks) {
+          const int k = ks * 4 + lg;
+          const T af = sa[k * SR + wm * 16 + lc];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[j] = Mfma<T>::mma(af, sb[k * CB + wn * 32 + j * 16 + lc], acc[j]);
+        }
+        if (more) stage_out((kt + 1) & 1);
+        __syncthreads();
+      }
+    }
+    // the difference, [column][row], then its product with D_j^T: D[n][k] at n = 32 wn + 16 j + lc, k = 4 ks + lg
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        lds[(wn * 32 + j * 16 + lc) * SR + wm * 16 + Mfma<T>::row(v, lane)] = old[j][v] - acc[j][v];
+        acc[j][v] = T(0);
+      }
+    __syncthreads();
+    const T* const dj = D + (long long)(n0 + wn * 32 + lc) * r + n0 + lg;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {   // (in quarters: the registers decide how many workgroups a compute unit holds)
+      T df[2][CB / 16];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int ks = 0; ks < CB / 16; ++ks) {
+          const int k = h * (CB / 4) + ks * 4;
+          df[j][ks] = INTERIOR || (wn * 32 + j * 16 + lc < nb && k + lg < nb) ? dj[(long long)j * 16 * r + k] : T(0);
+        }
+#pragma unroll
+      for (int ks = 0; ks < CB / 16; ++ks) {
+        const T af = lds[(h * (CB / 4) + ks * 4 + lg) * SR + wm * 16 + lc];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = Mfma<T>::mma(af, df[j][ks], acc[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int m = Mfma<T>::row(v, lane);
+        if (INTERIOR || (row0 + wm * 16 + m < rows && wn * 32 + j * 16 + lc < nb)) own[(long long)m * r + j * 16] = acc[j][v];
+      }
+    __syncthreads();   // the stored columns are the next block column's operand; the buffers are free
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 5) void solve_rows_kernel(T* __restrict__ Pm, const T* __restrict__ Lm, const T* __restrict__ Dm, int rows,
+                                                         int r, int batch, int blocks, int spread, const int* gate, int gate_want) {
+  __shared__ __attribute__((aligned(16))) T lds[2 * 128 * (SR + 64) / sizeof(T)];
+  static_assert(2 * 128 * (SR + 64) / sizeof(T) >= 64 * SR && 128 / sizeof(T) >= RK, "room for the difference and for the stages of the checked loop");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int b, blk;
+  if (spread) {
+    b = blockIdx.x / blocks;
+    blk = blockIdx.x - b * blocks;
+  } else {
+    const int idx = blockIdx.x >> 3, m = idx / blocks;
+    b = m * 8 + (blockIdx.x & 7);
+    blk = idx - m * blocks;
+  }
+  if (b >= batch || (gate && (gate[b] != 0) != (gate_want != 0))) return;
+  T* const P = Pm + (long long)b * rows * r;
+  const T* const L = Lm + (long long)b * r * r;
+  const T* const D = Dm + (long long)b * r * r;
+  const int row0 = blk * SR;
+  const bool interior = row0 + SR <= rows && r % 64 == 0 && ((reinterpret_cast<uintptr_t>(Pm) | reinterpret_cast<uintptr_t>(Lm)) & 15) == 0;
+  if (interior) solve_rows_of<T, true>(P, L, D, rows, r, row0, lds, tid, lane, wave >> 1, wave & 1);
+  else solve_rows_of<T, false>(P, L, D, rows, r, row0, lds, tid, lane, wave >> 1, wave & 1);
+}
+
+template <typename T>
+int solve_rows(T* P, const T* L, const T* D, int batch, int rows, int r, DaGate g, hipStream_t s) {
+  if (!P || !L || !D || batch <= 0 || rows <= 0 || r <= 0) return DA_ERR_ARG;
+  const int blocks = (rows + SR - 1) / SR;
+  const int spread = batch < 8 ? 1 : 0;
+  const long long grid = (long long)blocks * (spread ? batch : (batch + 7) / 8 * 8);
+  if (grid > 0x7fffffffLL) return DA_ERR_LIMIT;
+  hipLaunchKernelGGL(solve_rows_kernel<T>, dim3((unsigned)grid), dim3(256), 0, s, P, L, D, rows, r, batch, blocks, spread, g.flags, g.want);
+  return da_launch_status();
 }
 
 // Element-wise conversions of `batch` matrices of `per` contiguous elements; blockIdx.y = matrix.
@@ -357,6 +569,12 @@ int cvt_up(const void* src, int src_dtype, R* dst, long long per, int batch, DaG
 
 int da_gemm_f64(const Gemm64Desc& d, hipStream_t s) { return gemm_real<double>(d, s); }
 int da_gemm_f32s(const Gemm32Desc& d, hipStream_t s) { return gemm_real<float>(d, s); }
+int da_solve_rows(double* P, const double* L, const double* D, int batch, int rows, int r, DaGate g, hipStream_t s) {
+  return solve_rows<double>(P, L, D, batch, rows, r, g, s);
+}
+int da_solve_rows(float* P, const float* L, const float* D, int batch, int rows, int r, DaGate g, hipStream_t s) {
+  return solve_rows<float>(P, L, D, batch, rows, r, g, s);
+}
 
 int da_cvt_to_f64(const void* src, int src_dtype, double* dst, long long per, int batch, DaGate g, hipStream_t s) {
   return cvt_up<double>(src, src_dtype, dst, per, batch, g, s);

@@ -1,5 +1,6 @@
-"""The 64 x 64 diagonal block of the blocked Cholesky factorisations (csrc/diag64.h), through the orthonormaliser: ranks at the edges of
-its panels of 16 columns, and columns of zeros, whose pivots fail, at their first and last columns."""
+"""The 64 x 64 diagonal block of the blocked Cholesky factorisations (csrc/diag64.h) and the triangular solve behind them
+(csrc/gemm_f64.hip), through the orthonormaliser: ranks at the edges of the block's panels of 16 columns, columns of zeros, whose
+pivots fail, at their first and last columns, whole and ragged rows, one and several matrices to an XCD."""
 import pytest
 import torch
 
@@ -52,3 +53,16 @@ def test_a_column_of_zeros_is_dropped_and_reported(col):
     keep = [j for j in range(r) if j != col]
     assert (Q[1].cpu().double()[:, keep] - _q64(P[1][:, keep])).norm() <= 4 * EPS32 * r**0.5
     assert (Q[0].cpu().double() - _q64(P[0])).norm() <= 4 * EPS32 * r**0.5
+
+
+@pytest.mark.parametrize("batch, m, r", [(1, 64, 64), (3, 352, 192), (8, 64, 64), (9, 100, 64), (11, 288, 128), (17, 129, 65), (2, 1000, 320)])
+@pytest.mark.parametrize("qr_method", ["qr", "cqr"])
+def test_solve_over_batches_and_ragged_rows(batch, m, r, qr_method):
+    from dion_amd.newton_schulz import orthonormalize
+
+    P = torch.stack([_factor(m, r, s) for s in range(batch)]).float()
+    passes = 1 if qr_method == "qr" else 2
+    tol = 4 * EPS32 if qr_method == "qr" else 100 * 16 * EPS32 * m**0.5   # (as above)
+    Q = orthonormalize(P.cuda(), passes=passes, qr_method=qr_method).cpu().double()
+    for b in range(batch):
+        assert (Q[b] - _q64(P[b])).norm() <= tol * r**0.5
