@@ -126,6 +126,11 @@ struct GemmDesc {
   // over is rounded to bf16 as well and stored c2_off elements after C -- the result as two bf16 matrices.
   int a_kwrap;
   long long c2_off;
+  // bf16 kernel, optional.  k_tri: B (k-strided; with a_kwrap every copy of it) is upper triangular, B(k, n) = 0 for k > n: a column
+  // tile only sums k below its end, and the longest sums start first.  Half the K loop of a wide factor's products with its
+  // inverse Cholesky factor: a Dion step at rank 768 (12 layers, d 768, ff 3072) 3652 -> 3602 us, at rank 512 within the
+  // noise.  (The checked K loop sums the zeros as well: the same bits for a finite A.)
+  int k_tri;
   // bf16 kernel, optional.  k_slices > 1: the sum over k is cut into that many slices of k_slice elements (a multiple
   // of 64; the last one may be shorter) that run as tiles of their own; slice s stores its partial product as
   // matrices s * batch ... s * batch + batch - 1 of C, which therefore holds k_slices * batch matrices sC apart,

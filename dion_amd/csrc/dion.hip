@@ -759,6 +759,7 @@ int correction_bf16(const float* in, const bf16_t* in_low, void* out, int out_dt
   c.sE = pr; c.lde = r;
   c.M = rows; c.N = r; c.K = r;
   c.epilogue = DA_EPI_AXPBY; c.s0 = 1.f; c.s1 = -1.f; c.faithful = 0;
+  c.k_tri = 1;
   c.gate = gate.flags; c.gate_want = gate.want;
   return da_gemm_bf16(c, s);
 }
@@ -1052,6 +1053,7 @@ int fast16_pass(const bf16_t* P, const OrthWs& w, int batch, int rows, int r, in
     c.B = Tcat; c.sB = 2 * rr; c.ldb = r; c.b_kstrided = 1;
     c.C = w.Ph; c.sC = pr; c.ldc = r; c.c_dtype = DA_BF16; c.c2_off = Lo - w.Ph;
     c.M = rows; c.N = r; c.K = 2 * r;
+    c.k_tri = 1;
     c.epilogue = DA_EPI_STORE; c.s1 = 1.f; c.faithful = 0;
     rc = da_gemm_bf16(c, s);
     if (rc || !second_gram) return rc;

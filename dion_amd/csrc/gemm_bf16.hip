@@ -103,6 +103,7 @@ __device__ __forceinline__ TileId decode_tile(const GemmDesc& d, int bid, int nb
     r.ti = t / tiles_n;
     r.tj = t - r.ti * tiles_n;
   }
+  if (!SYM && d.k_tri) r.tj = tiles_n - 1 - r.tj;   // (the longest sums first)
   return r;
 }
 
@@ -164,9 +165,22 @@ __global__ __launch_bounds__(C::NT) void gemm_bf16_kernel(GemmArgs args) {
   const bf16_t* B = (d.Btab ? static_cast<const bf16_t*>(d.Btab[b]) : static_cast<const bf16_t*>(d.B) + (long long)b * d.sB) +
                     k0 * (B_KS ? d.ldb : 1);
 
+  int a_wrap = -1;       // (a triangular B: the rows past the tile's last column are left out of every copy)
+  unsigned b_jump = 0;
+  if (B_KS && !SYM && MODE != DA_LOOP_CHECKED && d.k_tri) {
+    const int whole = d.a_kwrap ? d.a_kwrap : dK, part = whole < n0 + BT ? whole : n0 + BT;
+    if (d.a_kwrap) {
+      a_wrap = part;
+      b_jump = (unsigned)((long long)(whole - part) * d.ldb * 2);
+      dK = dK / whole * part;
+    } else {
+      dK = part;
+    }
+  }
+
   typename C::acc_t acc[TMI][TNJ];
   gemm_tile_k_loop<C, A_KS, B_KS, MODE>(acc, d, A, B, dK, m0, n0, lds, tid, lane, wave, wm, wn, DaNoHook(),
-                                        SYM && ti == tj && A == B && dK <= args.diag_k);
+                                        SYM && ti == tj && A == B && dK <= args.diag_k, a_wrap, b_jump);
   if (trace) ts1 = __builtin_amdgcn_s_memrealtime();
   epilogue<C, SYM, MODE == DA_LOOP_INTERIOR>(acc, d, lds, tile.b, ti, tj, m0, n0, wave, lane, wm, wn);
   if (trace) {
@@ -309,6 +323,7 @@ int check_desc(const GemmDesc& d) {
   if (d.a_kwrap && (d.a_kwrap < 0 || d.a_kstrided || d.a_kwrap % BK || d.K % d.a_kwrap)) return DA_ERR_ARG;
   if (d.c2_off && (d.c_dtype != DA_BF16 || d.epilogue != DA_EPI_STORE || d.faithful || d.symmetric || (d.c2_off & 7)))
     return DA_ERR_ARG;
+  if (d.k_tri && (d.symmetric || !d.b_kstrided || d.k_slices > 1 || (d.a_kwrap ? d.a_kwrap : d.K) < d.N)) return DA_ERR_ARG;
   if (d.k_slices < 0 || (d.k_slices > 1 && (d.k_slice <= 0 || d.k_slice % BK || (long long)(d.k_slices - 1) * d.k_slice >= d.K ||
                                             (long long)d.k_slices * d.k_slice < d.K || d.c_dtype != DA_F32 ||
                                             d.epilogue != DA_EPI_STORE || d.Ctab || d.a_kwrap || d.c2_off || d.symmetric)))

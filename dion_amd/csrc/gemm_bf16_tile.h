@@ -403,12 +403,14 @@ constexpr int DA_LOOP_CHECKED = 0, DA_LOOP_INTERIOR = 1, DA_LOOP_EDGE = 2;
 // wavefront has waited for all of its outstanding memory operations by then, stores of earlier work included.
 // `same_panel` (direct-to-LDS forms, both operands k-contiguous): the two operands are the same rows of the same
 // matrix -- a diagonal tile of X X^T or A A -- so one panel is staged and both fragment sets are read from it.
+// `a_wrap`, `b_jump` (direct-to-LDS forms): A is read again from its first column after a_wrap of its columns instead of
+// GemmDesc::a_kwrap of them, and B then goes on b_jump bytes further.
 struct DaNoHook { __device__ __forceinline__ void operator()() const {} };
 template <typename C, bool A_KS, bool B_KS, int MODE, typename Hook = DaNoHook>
 __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, const bf16_t* A,
                                                  const bf16_t* B, int dK, int m0, int n0, char* lds, int tid, int lane,
                                                  int wave, int wm, int wn, Hook after_first_stage = Hook(),
-                                                 bool same_panel = false) {
+                                                 bool same_panel = false, int a_wrap = -1, unsigned b_jump = 0) {
   constexpr bool FULL = MODE != DA_LOOP_CHECKED;   // the direct-to-LDS K loop
   constexpr int BT = C::BT, TMI = C::TMI, TNJ = C::TNJ, NCH = C::NCH, NW = C::NT / 64;
   constexpr int A_BYTES = Tile<BT, A_KS>::bytes;
@@ -467,11 +469,11 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
           dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
     }                                                                                              \
     koff_a += (unsigned)(sa.tstep * 2);                                                            \
-    if (koff_a == wrap_a) koff_a = 0;                                                              \
     koff_b += (unsigned)(sb.tstep * 2);                                                            \
+    if (koff_a == wrap_a) { koff_a = 0; koff_b += b_jump; }                                        \
   } while (0)
     unsigned koff_a = 0, koff_b = 0;   // byte offset of the stage within the operand (< 4 GiB: checked by the launcher)
-    const unsigned wrap_a = (unsigned)d.a_kwrap * 2u;   // A read again from its first column (0: never, koff_a > 0 here)
+    const unsigned wrap_a = (unsigned)(a_wrap < 0 ? d.a_kwrap : a_wrap) * 2u;   // A read again from its first column (0: never, koff_a > 0 here)
     DA_DMA(lds);
     dma_wait();
     __syncthreads();
@@ -609,11 +611,11 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
           dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
     }                                                                                              \
     koff_a += (unsigned)(sa.tstep * 2);                                                            \
-    if (koff_a == wrap_a) koff_a = 0;                                                              \
     koff_b += (unsigned)(sb.tstep * 2);                                                            \
+    if (koff_a == wrap_a) { koff_a = 0; koff_b += b_jump; }                                        \
   } while (0)
     unsigned koff_a = 0, koff_b = 0;
-    const unsigned wrap_a = (unsigned)d.a_kwrap * 2u;
+    const unsigned wrap_a = (unsigned)(a_wrap < 0 ? d.a_kwrap : a_wrap) * 2u;
     DA16_DMA(lds);
     dma_wait();
     __syncthreads();

@@ -1,6 +1,7 @@
 """The 64 x 64 diagonal block of the blocked Cholesky factorisations (csrc/diag64.h) and the triangular solve behind them
 (csrc/gemm_f64.hip), through the orthonormaliser: ranks at the edges of the block's panels of 16 columns, columns of zeros, whose
-pivots fail, at their first and last columns, whole and ragged rows, one and several matrices to an XCD."""
+pivots fail, at their first and last columns, whole and ragged rows, one and several matrices to an XCD; and the bf16 products
+with the triangular factors (csrc/gemm_bf16.hip)."""
 import pytest
 import torch
 
@@ -66,3 +67,23 @@ def test_solve_over_batches_and_ragged_rows(batch, m, r, qr_method):
     Q = orthonormalize(P.cuda(), passes=passes, qr_method=qr_method).cpu().double()
     for b in range(batch):
         assert (Q[b] - _q64(P[b])).norm() <= tol * r**0.5
+
+
+@pytest.mark.parametrize("batch, r", [(1, 128), (2, 136), (1, 320), (1, 520), (2, 768)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_products_with_triangular_factors(batch, r, dtype):
+    """P T and the correction, whose column tiles stop their sums at the triangle's edge (one, whole and ragged tiles)."""
+    from dion_amd.newton_schulz import orthonormalize
+
+    m = 4 * r
+    P = torch.stack([_factor(m, r, s) for s in range(batch)]).to(dtype)
+    one = orthonormalize(P.cuda(), qr_method="cqr").cpu().double()
+    two = orthonormalize(P.cuda(), qr_method="rcqr").cpu().double()
+    # Storing: half an ulp of every entry.  cqr: fp32 sums of m products, the condition squared (as above).  rcqr: the
+    # defect D that cqr leaves, squared, and the two bf16 operands of its correction; the fp32 product P T, condition 4.
+    ulp = (2.0**-9 if dtype == torch.bfloat16 else EPS32) * r**0.5
+    for b in range(batch):
+        q = _q64(P[b])
+        assert (one[b] - q).norm() <= ulp + 100 * 16 * EPS32 * m**0.5 * r**0.5
+        D = 0.0 if dtype == torch.bfloat16 else float((one[b].T @ one[b] - torch.eye(r, dtype=torch.float64)).norm())
+        assert (two[b] - q).norm() <= ulp + D * D + 2.0**-8 * D + 16 * 4 * EPS32 * r**0.5
