@@ -1,17 +1,17 @@
-// The Dion step (reference dion/dion.py:742-875) of a set of small matrices in ONE launch:
+// The Dion step (reference dion/dion.py:742-875) of a set of small matrices in three launches:
 //
 //   B = M + G;  P = B' Q;  P <- orth(P);  R = B'^T P;  Q <- R / (||R||_col + eps);
 //   M <- B - (1 - mu) P R^T;  X <- decay X - lr P Q^T              (B' = B, or B^T when m < n; mp x np, mp >= np)
 //
 // What bounds it: as a sequence of launches a bucket takes 40 to 60 of them (a third of which only find out that the fp64
 // pass of the orthonormaliser is not needed), each a few microseconds of work: a model of 24 matrices of 256 x 256 and
-// 256 x 1024 spent 0.6-0.8 ms, most of it on the host.  Now 0.25 ms, and the host is free after 38 us: four fifths of it is the
-// chain of phases (25 us per diagonal block, 10-15 us per product), not throughput.  Here the step is a list of phases per matrix, cut into tiles;
+// 256 x 1024 spent 0.6-0.8 ms, most of it on the host; here 0.19 ms, three quarters of it the chain of phases (15-24 us per
+// diagonal block, 10-15 us per product), not throughput.  The element-wise ends, B = M + G and the update, are launches over the
+// whole GPU; what lies between is a list of phases per matrix, cut into tiles, in one launch:
 // workgroups take tiles from eight queues, one per XCD (flow_queue.h), and a counter per matrix and phase says when the
 // next phase may start.  A matrix stays with one XCD, so its phases meet in one L2.
 //
-// Phases (kinds):  ADD   B = M + G in place, and whether any element is not zero; Q as a padded working matrix
-//                  BQ    P = B' Q                                      64 x 64 tiles
+// Phases (kinds):  BQ    P = B' Q                                      64 x 64 tiles
 //                  GRAM  P^T P in fp64, lower 32 x 32 tiles, K slices as slabs of their own
 //                  DIAG0 LOW0 DIAG1 LOW1 ..   P^T P = L L^T and T = L^-1 in blocks of 64, left-looking: DIAGj adds the slabs
 //                        (in order) and the earlier columns' products to block (j, j), factors it and inverts the factor;
@@ -22,18 +22,17 @@
 //                        noise columns dropped, P <- P (I - up(P^T P - I)))
 //                  BTP   R = B'^T P                                    64 x 64 (bf16) or 32 x 32 (fp32) tiles
 //                  CNORM column norms, Q_new, Q state                  64 x 64 tiles
-//                  UPD   error feedback and weight update, both products of a 64 x 64 tile of M and X
 // The orthonormaliser is the fp64 CholeskyQR of dion.hip for every matrix: at these sizes the fp64 products cost less than
 // the launches of the two-precision road.  P, R and the products with B run on the matrix cores in the momentum's dtype with
 // the instructions and the order of k of the batched kernels (v_mfma_f32_16x16x32_bf16, in the updates v_mfma_f32_32x32x16_bf16; v_mfma_f32_32x32x2_f32).
 //
-// Coherence.  Every buffer of the workspace is written once and read only after its phase is complete, and the lines of
-// M and X belong to one matrix (128-byte aligned): plain loads cannot meet a stale L1 line.  The exception is M itself,
-// which ADD rewrites: its loads go past the L1 (scope bit sc1), so that no old line stays behind.
+// Coherence.  Every buffer of the workspace is written once and read only after its phase is complete, and M and X change in
+// other launches: plain loads cannot meet a stale L1 line.
 //
 // Shapes: any m, n (rows that are no multiple of 16 bytes move with unaligned accesses), rank up to 256; the working
 // matrices are padded to whole tiles and the tiles' loads fill with zeros.
 #include "dion_small.h"
+#include <type_traits>
 #include "flow_queue.h"
 #include "small_tile.h"
 
@@ -42,13 +41,15 @@
 namespace {
 
 constexpr int MAX_RT = DA_DS_MAX_RANK / 64;
-enum Kind { ADD, BQ, GRAM, DIAG, LOW, PT = GRAM + 1 + 2 * MAX_RT, FIX, BTP, CNORM, UPD, KINDS };   // DIAGj = DIAG + 2 j, LOWj
+enum Kind { BQ, GRAM, DIAG, LOW, PT = GRAM + 1 + 2 * MAX_RT, FIX, BTP, CNORM, KINDS };   // DIAGj = DIAG + 2 j, LOWj
 constexpr int CTR_STRIDE = 32;     // ints per matrix: a counter per kind, then the words below
 constexpr int W_NONZERO = 18, W_SICK = 19, W_BAD = 20, W_GRAM2 = 21, W_RANGE = 24;   // (W_RANGE: two doubles)
 static_assert(KINDS <= W_NONZERO, "a counter per kind");
 constexpr int ADD_ELEMS = 8192;
 constexpr double PIVOT_RATIO = 1e-7;   // as POLISH_PIVOT_RATIO in dion.hip
 constexpr int SMEM = STAGES64 + DA_DS_MAX_RANK;
+constexpr int SMEM_UPDATE = 2 * 3 * Real<float, 64>::OPND * 4;   // two stages of three fp32 operands; the bf16 ones and the two products staged behind them are smaller
+static_assert(SMEM_UPDATE >= 2 * 3 * 64 * 64 * 2 && SMEM_UPDATE >= 2 * 64 * 66 * 4 && 3 * SMEM_UPDATE <= 160 * 1024, "LDS of the update");
 
 struct GroupDev {
   void *const *X, *const *G, *const *M, *const *Q;   // device tables
@@ -57,10 +58,12 @@ struct GroupDev {
   double *P64, *slab, *L, *T, *A2, *defect;
   int* words;                    // [cnt][CTR_STRIDE]
   int* info;
+  int* any;                      // [cnt][mchunks]: a chunk of B with an element that is not zero
   int cnt;
   unsigned char nq[DA_QUEUES], at[DA_QUEUES];   // matrices in every queue; where their numbers begin in Args::order
   int m, n, r, rp, mp, np, mpT, npT, rT, transposed;
   int nT;
+  int mchunks;                   // of ADD_ELEMS elements
   int slices, kslice;            // of the Gram products
   float scaled_lr;
 };
@@ -81,13 +84,11 @@ struct Args {
 __host__ __device__ inline int tasks_of(const GroupDev& G, int kind, bool bf) {
   const int t32 = (G.r + 31) >> 5;
   switch (kind) {
-    case ADD: return (int)(((long long)G.m * G.n + ADD_ELEMS - 1) / ADD_ELEMS) + (G.npT * 64 * G.rp + ADD_ELEMS - 1) / ADD_ELEMS;
     case BQ: case PT: return G.mpT * G.rT;
     case GRAM: return t32 * (t32 + 1) / 2 * G.slices;
     case FIX: return t32 * (t32 + 1) / 2 + G.mpT * G.rT;
     case BTP: return bf ? G.npT * G.rT : ((G.np + 31) >> 5) * t32;
     case CNORM: return G.npT * G.rT;
-    case UPD: return G.mpT * G.npT;
     default: {   // block column j: the diagonal block; the blocks below it and the blocks of row j of the inverse
       const int j = (kind - DIAG) >> 1;
       return j >= G.rT ? 0 : ((kind - DIAG) & 1) ? G.rT - 1 : 1;
@@ -202,102 +203,15 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
       };
       float* const stg = reinterpret_cast<float*>(lds);
 
-      if (kind == ADD) {
-        ask();
-        const long long n = (long long)G.m * G.n;
-        const int mtasks = (int)((n + ADD_ELEMS - 1) / ADD_ELEMS);
-        if (task >= mtasks) {
-          // ---- Q in the momentum's dtype, padded to whole tiles
-          for (int h = 0; h < ADD_ELEMS / 2048; ++h) {
-            const long long e = (long long)(task - mtasks) * ADD_ELEMS + h * 2048 + tid * 8;
-            const int row = (int)(e / rp), col = (int)(e - (long long)row * rp);
-            if (row >= npR) break;
-            const int c = row < G.np ? G.r - col : 0;
-            float v[8];
-            if (a.q_f32) load8(static_cast<const float*>(G.Q[b]), (long long)row * G.r + col, c, v);
-            else load8(static_cast<const bf16_t*>(G.Q[b]), (long long)row * G.r + col, c, v);
-            store8(Qw, !BF, e, 8, v);
-          }
-        } else {
-          const long long e0 = (long long)task * ADD_ELEMS + tid * 8;
-          const bf16_t* const g16 = static_cast<const bf16_t*>(G.G[b]);
-          const float* const g32 = static_cast<const float*>(G.G[b]);
-          bool any = false;
-          auto finish = [&](const Raw<E>& mr, float (&g)[8], long long e, int c) {
-            float m[8];
-            unpack(mr, m);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              m[i] = BF ? rbf(m[i] + g[i]) : m[i] + g[i];
-              if (i < c) any |= m[i] != 0.f;
-            }
-            store8(M, !BF, e, c, m);
-          };
-          if ((long long)(task + 1) * ADD_ELEMS <= n) {   // every load on the way before the first is used
-            Raw<E> mr[4];
-#pragma unroll
-            for (int h = 0; h < 4; ++h)
-#pragma unroll
-              for (int i = 0; i < MSZ / 2; ++i) mr[h].q[i] = ldg16_l2(M + (e0 + h * 2048) * MSZ + 16 * i);
-            if (a.g_f32) {
-              Raw<float> gr[4];
-#pragma unroll
-              for (int h = 0; h < 4; ++h) gr[h] = load_raw(g32 + e0 + h * 2048);
-#pragma unroll
-              for (int h = 0; h < 4; ++h) {
-                float g[8];
-                unpack(gr[h], g);
-                finish(mr[h], g, e0 + h * 2048, 8);
-              }
-            } else {
-              Raw<bf16_t> gr[4];
-#pragma unroll
-              for (int h = 0; h < 4; ++h) gr[h] = load_raw(g16 + e0 + h * 2048);
-#pragma unroll
-              for (int h = 0; h < 4; ++h) {
-                float g[8];
-                unpack(gr[h], g);
-                finish(mr[h], g, e0 + h * 2048, 8);
-              }
-            }
-          } else {
-            for (int h = 0; h < 4; ++h) {
-              const long long e = e0 + h * 2048;
-              const int c = n - e >= 8 ? 8 : (int)(n - e);
-              if (c <= 0) break;
-              Raw<E> mr;
-#pragma unroll
-              for (int i = 0; i < MSZ / 2; ++i) mr.q[i] = u32x4_t{0, 0, 0, 0};
-              if (c == 8) {
-#pragma unroll
-                for (int i = 0; i < MSZ / 2; ++i) mr.q[i] = ldg16_l2(M + e * MSZ + 16 * i);
-              } else if (BF) {
-                unsigned w[4] = {0, 0, 0, 0};
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                  if (i < c) w[i >> 1] |= (unsigned)__hip_atomic_load(reinterpret_cast<const unsigned short*>(M) + e + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) << (16 * (i & 1));
-                mr.q[0] = u32x4_t{w[0], w[1], w[2], w[3]};
-              } else {
-                unsigned w[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                  w[i] = i < c ? __hip_atomic_load(reinterpret_cast<const unsigned*>(M) + e + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-                mr.q[0] = u32x4_t{w[0], w[1], w[2], w[3]};
-                mr.q[MSZ / 2 - 1] = u32x4_t{w[4], w[5], w[6], w[7]};
-              }
-              float g[8];
-              if (a.g_f32) load8(g32, e, c, g);
-              else load8(g16, e, c, g);
-              finish(mr, g, e, c);
-            }
-          }
-          if (__any(any) && lane == 0)
-            __hip_atomic_store(words + W_NONZERO, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      } else if (kind == BQ || kind == BTP) {
+      if (kind == BQ || kind == BTP) {
         // ---- P = B' Q;  R = B'^T P
         const bool bq = kind == BQ;
         const int rT = G.rT, rt32 = (G.r + 31) >> 5;
+        if (bq && task == 0) {   // has any element of B been found not to be zero?
+          bool any = false;
+          for (int i = tid; i < G.mchunks; i += 256) any |= G.any[(long long)b * G.mchunks + i] != 0;
+          if (__any(any) && lane == 0) __hip_atomic_store(words + W_NONZERO, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         const Opnd<E, true> sa = momentum(!bq);
         const Opnd<E, false> sb = work<E>(bq ? Qw : P2, rp, 1);
         const int kend = bq ? G.np : G.mp;
@@ -454,74 +368,6 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
           store8(Qn, !BF, (long long)row * rp + col, 8, v);
           store8(static_cast<char*>(G.Q[b]), a.q_f32, (long long)row * G.r + col, row < G.np ? G.r - col : 0, v);
         }
-      } else if (kind == UPD) {
-        // ---- M += ef_alpha P R^T, X = decay X - lr P Q_new^T on one tile (rows of P, rows of R)
-        const int ti = wave_uniform(task / G.npT), tj = wave_uniform(task - task / G.npT * G.npT);
-        const int row0 = ti * 64, col0 = tj * 64;
-        const bool turned = G.transposed != 0;
-        const Opnd<E, false> sp = work<E>(P2, rp, 0), sr = work<E>(R, rp, 0), sn = work<E>(Qn, rp, 0);
-        const int kend = BF ? rp : ((G.r + 31) >> 5) << 5;   // (what the tiles of BTP have written)
-        char* const X = static_cast<char*>(G.X[b]);
-        float* const stg2 = stg + 64 * 66;
-        // a thread's chunks: stored row, eight consecutive stored columns; inside the matrix M and X are requested before the
-        // products
-        const int tr = turned ? col0 : row0, tc = turned ? row0 : col0;
-        const bool inside = tr + 64 <= G.m && tc + 64 <= G.n;
-        const long long e0 = (long long)(tr + (tid >> 3)) * G.n + tc + (tid & 7) * 8;
-        Raw<E> mr[2];
-        Raw<float> xr[2];      // (bf16 weights: the first quarter)
-        if (inside) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const long long e = e0 + 32LL * h * G.n;
-            mr[h] = load_raw(reinterpret_cast<const E*>(M) + e);
-            if (a.x_f32) xr[h] = load_raw(reinterpret_cast<const float*>(X) + e);
-            else xr[h].q[0] = load_raw(reinterpret_cast<const bf16_t*>(X) + e).q[0];
-          }
-        }
-        f32x16_t acc[2];
-        const Opnd<E, false> sbs[2] = {sr, sn};
-        if constexpr (BF) update_bf16(sp, sbs, row0, col0, kend, lds, tid, lane, wm, wn, acc);
-        else tile32x2<2>(sp, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc);
-        stage_f32(acc[0], stg, lane, wm, wn);
-        stage_f32(acc[1], stg2, lane, wm, wn);
-        ask();
-        __syncthreads();
-        const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-        const float lr = -G.scaled_lr;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
-          const long long e = e0 + 32LL * h * G.n;
-          const int n = tr + r < G.m ? G.n - tc - c : 0;
-          float mv[8], xv[8];
-          if (inside) {
-            unpack(mr[h], mv);
-            if (a.x_f32) unpack(xr[h], xv);
-            else unpack(Raw<bf16_t>{{xr[h].q[0]}}, xv);
-          } else {
-            load8(reinterpret_cast<const E*>(M), e, n, mv);
-            if (a.x_f32) load8(reinterpret_cast<const float*>(X), e, n, xv);
-            else load8(reinterpret_cast<const bf16_t*>(X), e, n, xv);
-          }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int at = turned ? (c + i) * 66 + r : r * 66 + c + i;
-            // the roundings of the reference's separate tensor ops (epi_value in mfma_tile.h)
-            float t1 = stg[at], t2 = stg2[at];
-            if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
-            t1 = a.ef_alpha * t1;
-            t2 = lr * t2;
-            if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
-            mv[i] = mv[i] + t1;
-            float x = a.decay * xv[i];
-            if (!a.x_f32) x = rbf(x);
-            xv[i] = x + t2;
-            if (poisoned) mv[i] = xv[i] = __builtin_nanf("");
-          }
-          store8(M, !BF, e, n, mv);
-          store8(X, a.x_f32, e, n, xv);
-        }
       } else {
         ask();   // a phase that a healthy matrix does not need
       }
@@ -536,23 +382,198 @@ __global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
   }
 }
 
+struct SetupGroup {
+  int end;                      // the group's last block + 1
+  int first, mblocks, per;      // its first matrix; blocks of a matrix for M, for M and Q
+  int m, n, r, rp, np, npR;
+  char* Qw;
+  int* any;
+};
 struct Setup {
   void* p[4][DA_DS_MATS];   // X, G, M, Q
   void** dst;               // [4][n]
   int n;
   int* zero;
-  int nzero;
+  int nzero, zblocks;
   int* status;
   int preset;
+  int ngroups, g_f32, q_f32;
+  SetupGroup g[DA_DS_GROUPS];
 };
+// The pointers and the counters of the step (the first blocks); B = M + G in place and the note which chunks of it are not all
+// zeros; Q as a padded working matrix.  Bound by memory: 5.5 TB/s, 24 us for 14 matrices of 341 to 2731 rows (22 million elements).
+// As a phase of the queues, where an XCD's 64 workgroups wait for their loads and then for their stores, it took 98 us.
+template <bool BF>
 __global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < s.n) {
+  typedef typename MomentumType<BF>::type E;
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < s.zblocks) {
+    const int i = blockIdx.x * 256 + tid;
+    if (i < s.n) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s.dst[k * s.n + i] = s.p[k][i];
+      for (int k = 0; k < 4; ++k) s.dst[k * s.n + i] = s.p[k][i];
+    }
+    for (int e = i; e < s.nzero; e += s.zblocks * 256) s.zero[e] = 0;
+    if (i == 0) *s.status = s.preset;
+    return;
   }
-  for (int e = i; e < s.nzero; e += gridDim.x * 256) s.zero[e] = 0;
-  if (i == 0) *s.status = s.preset;
+  int t = blockIdx.x - s.zblocks, gi = 0, begin = 0;
+  while (t >= s.g[gi].end) begin = s.g[gi++].end;
+  const SetupGroup& G = s.g[gi];
+  t -= begin;
+  const int b = t / G.per, task = t - b * G.per, mat = G.first + b;
+  if (task >= G.mblocks) {
+    // ---- Q in the momentum's dtype, padded to whole tiles
+    for (int h = 0; h < ADD_ELEMS / 2048; ++h) {
+      const long long e = (long long)(task - G.mblocks) * ADD_ELEMS + h * 2048 + tid * 8;
+      const int row = (int)(e / G.rp), col = (int)(e - (long long)row * G.rp);
+      if (row >= G.npR) break;
+      const int c = row < G.np ? G.r - col : 0;
+      float v[8];
+      if (s.q_f32) load8(static_cast<const float*>(s.p[3][mat]), (long long)row * G.r + col, c, v);
+      else load8(static_cast<const bf16_t*>(s.p[3][mat]), (long long)row * G.r + col, c, v);
+      store8(G.Qw + (long long)b * G.npR * G.rp * sizeof(E), !BF, e, 8, v);
+    }
+    return;
+  }
+  // ---- M + G: every load of a whole chunk on the way before the first is used
+  const long long n = (long long)G.m * G.n, e0 = (long long)task * ADD_ELEMS + tid * 8;
+  char* const M = static_cast<char*>(s.p[2][mat]);
+  const E* const m = reinterpret_cast<const E*>(M);
+  const bf16_t* const g16 = static_cast<const bf16_t*>(s.p[1][mat]);
+  const float* const g32 = static_cast<const float*>(s.p[1][mat]);
+  bool any = false;
+  auto finish = [&](float (&mv)[8], const float (&gv)[8], long long e, int c) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      mv[i] = BF ? rbf(mv[i] + gv[i]) : mv[i] + gv[i];
+      if (i < c) any |= mv[i] != 0.f;
+    }
+    store8(M, !BF, e, c, mv);
+  };
+  auto whole = [&](auto g) {
+    Raw<E> mr[4];
+    Raw<typename std::remove_const<typename std::remove_pointer<decltype(g)>::type>::type> gr[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) { mr[h] = load_raw(m + e0 + h * 2048); gr[h] = load_raw(g + e0 + h * 2048); }
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      float mv[8], gv[8];
+      unpack(mr[h], mv);
+      unpack(gr[h], gv);
+      finish(mv, gv, e0 + h * 2048, 8);
+    }
+  };
+  if ((long long)(task + 1) * ADD_ELEMS <= n) {
+    if (s.g_f32) whole(g32);
+    else whole(g16);
+  } else {
+    for (int h = 0; h < 4; ++h) {
+      const long long e = e0 + h * 2048;
+      const int c = n - e >= 8 ? 8 : (int)(n - e);
+      if (c <= 0) break;
+      float mv[8], gv[8];
+      load8(m, e, c, mv);
+      if (s.g_f32) load8(g32, e, c, gv);
+      else load8(g16, e, c, gv);
+      finish(mv, gv, e, c);
+    }
+  }
+  any = __syncthreads_or(any);
+  if (tid == 0) G.any[(long long)b * G.mblocks + task] = any;
+}
+
+// Error feedback and weight update, M += ef_alpha P R^T and X = decay X - lr P Q_new^T: a 64 x 64 tile (rows of P, rows of R) per
+// workgroup, three workgroups to a compute unit, the tiles of an XCD next to each other (it keeps their R and Q_new in its L2).
+// A launch of its own: bound by the latency of a tile's loads, it was a phase of the queues at two workgroups to a compute unit
+// (the registers of the factorisation) and with a matrix to an XCD.  155 -> 66 us (14 matrices as above, rank 256 and 86; the whole
+// step 607 -> 458); fp32, 24 matrices of 256 x 256 and 256 x 1024 at rank 128: 22 -> 27, but the step 222 -> 203 with both ends out.
+template <bool BF>
+__global__ __launch_bounds__(256, 3) void dion_small_update_kernel(Args a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename MomentumType<BF>::type E;
+  constexpr int MSZ = BF ? 2 : 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const int q = blockIdx.x & 7, each = gridDim.x >> 3, rest = gridDim.x & 7;
+  int t = q * each + min(q, rest) + (blockIdx.x >> 3), gi = 0;   // (workgroups go to the XCDs in turn)
+  for (;; ++gi) {
+    const int mine = a.g[gi].cnt * a.g[gi].mpT * a.g[gi].npT;
+    if (t < mine || gi + 1 == a.ngroups) break;
+    t -= mine;
+  }
+  const GroupDev& G = a.g[gi];
+  const int b = t / (G.mpT * G.npT), task = t - b * (G.mpT * G.npT);
+  const int rp = G.rp;
+  const char* const P2 = G.P2 + (long long)b * G.mpT * 64 * rp * MSZ;
+  const char* const R = G.R + (long long)b * G.npT * 64 * rp * MSZ;
+  const char* const Qn = G.Qn + (long long)b * G.npT * 64 * rp * MSZ;
+  char* const M = static_cast<char*>(G.M[b]);
+  float* const stg = reinterpret_cast<float*>(lds);
+  const int ti = wave_uniform(task / G.npT), tj = wave_uniform(task - task / G.npT * G.npT);
+  const int row0 = ti * 64, col0 = tj * 64;
+  const bool turned = G.transposed != 0;
+  const Opnd<E, false> sp = work<E>(P2, rp, 0), sr = work<E>(R, rp, 0), sn = work<E>(Qn, rp, 0);
+  const int kend = BF ? rp : ((G.r + 31) >> 5) << 5;   // (what the tiles of BTP have written)
+  char* const X = static_cast<char*>(G.X[b]);
+  float* const stg2 = stg + 64 * 66;
+  // a thread's chunks: stored row, eight consecutive stored columns; inside the matrix M and X are requested before the
+  // products
+  const int tr = turned ? col0 : row0, tc = turned ? row0 : col0;
+  const bool inside = tr + 64 <= G.m && tc + 64 <= G.n;
+  const long long e0 = (long long)(tr + (tid >> 3)) * G.n + tc + (tid & 7) * 8;
+  Raw<E> mr[2];
+  Raw<float> xr[2];      // (bf16 weights: the first quarter)
+  if (inside) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const long long e = e0 + 32LL * h * G.n;
+      mr[h] = load_raw(reinterpret_cast<const E*>(M) + e);
+      if (a.x_f32) xr[h] = load_raw(reinterpret_cast<const float*>(X) + e);
+      else xr[h].q[0] = load_raw(reinterpret_cast<const bf16_t*>(X) + e).q[0];
+    }
+  }
+  f32x16_t acc[2];
+  const Opnd<E, false> sbs[2] = {sr, sn};
+  if constexpr (BF) update_bf16(sp, sbs, row0, col0, kend, lds, tid, lane, wm, wn, acc);
+  else tile32x2<2>(sp, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc);
+  stage_f32(acc[0], stg, lane, wm, wn);
+  stage_f32(acc[1], stg2, lane, wm, wn);
+  __syncthreads();
+  const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  const float lr = -G.scaled_lr;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
+    const long long e = e0 + 32LL * h * G.n;
+    const int n = tr + r < G.m ? G.n - tc - c : 0;
+    float mv[8], xv[8];
+    if (inside) {
+      unpack(mr[h], mv);
+      if (a.x_f32) unpack(xr[h], xv);
+      else unpack(Raw<bf16_t>{{xr[h].q[0]}}, xv);
+    } else {
+      load8(reinterpret_cast<const E*>(M), e, n, mv);
+      if (a.x_f32) load8(reinterpret_cast<const float*>(X), e, n, xv);
+      else load8(reinterpret_cast<const bf16_t*>(X), e, n, xv);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at = turned ? (c + i) * 66 + r : r * 66 + c + i;
+      // the roundings of the reference's separate tensor ops (epi_value in mfma_tile.h)
+      float t1 = stg[at], t2 = stg2[at];
+      if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
+      t1 = a.ef_alpha * t1;
+      t2 = lr * t2;
+      if (BF) { t1 = rbf(t1); t2 = rbf(t2); }
+      mv[i] = mv[i] + t1;
+      float x = a.decay * xv[i];
+      if (!a.x_f32) x = rbf(x);
+      xv[i] = x + t2;
+      if (poisoned) mv[i] = xv[i] = __builtin_nanf("");
+    }
+    store8(M, !BF, e, n, mv);
+    store8(X, a.x_f32, e, n, xv);
+  }
 }
 
 inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -575,6 +596,8 @@ struct Shape {
   }
 };
 
+inline int mchunks(int m, int n) { return (int)(((long long)m * n + ADD_ELEMS - 1) / ADD_ELEMS); }
+
 // lays out one group at p (null: only counts); returns the bytes
 size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, char* base) {
   size_t o = 0;
@@ -586,9 +609,11 @@ size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, 
   char* Qn = take(pn * msz);
   char* Qw = take(pn * msz);
   char* norm = take(c * S.nT * S.rp * 8);
+  char* any = take(c * mchunks(g.m, g.n) * 4);
   double* f64[6];   // P64, slab, L, T, A2, defect
   for (int i = 0; i < 6; ++i) f64[i] = reinterpret_cast<double*>(take((i == 0 ? pm : i == 1 ? rr * S.slices : i == 5 ? c * S.rp * 2 * MAX_RT : rr) * 8));
   if (D) {
+    D->any = reinterpret_cast<int*>(any); D->mchunks = mchunks(g.m, g.n);
     D->P = P; D->P2 = P2; D->R = R; D->Qn = Qn; D->Qw = Qw; D->norm = reinterpret_cast<double*>(norm); D->nT = S.nT;
     D->P64 = f64[0]; D->slab = f64[1]; D->L = f64[2]; D->T = f64[3]; D->A2 = f64[4]; D->defect = f64[5];
   }
@@ -669,6 +694,7 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
 int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, void* workspace, hipStream_t s) {
   Args a{};
   Setup su;
+  const bool bf = c.m_dtype == DA_BF16;
   int mats = 0;
   char* p = static_cast<char*>(workspace);
   for (int i = 0; i < n; ++i) mats += g[i].cnt;
@@ -686,8 +712,9 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   unsigned char queue[DA_DS_MATS];
   deal(g, n, c.m_dtype == DA_BF16, queue);
   int first = 0, at = 0;
+  long long adds = 0, tiles = 0;
   for (int i = 0; i < n; ++i) {
-    const Shape S(g[i].m, g[i].n, g[i].r, c.m_dtype == DA_BF16);
+    const Shape S(g[i].m, g[i].n, g[i].r, bf);
     GroupDev& D = a.g[i];
     p += lay_out(&D, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, p);
     D.X = su.dst + first; D.G = su.dst + mats + first; D.M = su.dst + 2 * mats + first; D.Q = su.dst + 3 * mats + first;
@@ -710,6 +737,13 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
     D.mpT = S.mpT; D.npT = S.npT; D.rT = S.rT; D.transposed = g[i].m < g[i].n ? 1 : 0;
     D.slices = S.slices; D.kslice = S.kslice;
     D.scaled_lr = g[i].scaled_lr;
+    SetupGroup& U = su.g[i];
+    U.first = first;
+    U.mblocks = D.mchunks; U.per = D.mchunks + (S.npT * 64 * S.rp + ADD_ELEMS - 1) / ADD_ELEMS;
+    U.end = (int)(adds += (long long)g[i].cnt * U.per);
+    U.m = g[i].m; U.n = g[i].n; U.r = g[i].r; U.rp = S.rp; U.np = S.np; U.npR = S.npT * 64;
+    U.Qw = D.Qw; U.any = D.any;
+    tiles += (long long)g[i].cnt * S.mpT * S.npT;
     first += g[i].cnt;
   }
   a.ngroups = n;
@@ -719,18 +753,25 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   a.spin_limit = 200000000ull;   // 2 s of the 100 MHz counter
   a.x_f32 = c.x_dtype == DA_F32; a.g_f32 = c.g_dtype == DA_F32; a.q_f32 = c.q_dtype == DA_F32;
   a.ef_alpha = c.ef_alpha; a.decay = c.decay; a.eps = c.eps;
-  hipLaunchKernelGGL(dion_small_setup_kernel, dim3((unsigned)((su.nzero + 255) / 256)), dim3(256), 0, s, su);
-  int rc = da_launch_status();
-  if (rc) return rc;
+  su.zblocks = (su.nzero + 255) / 256;
+  su.ngroups = n; su.g_f32 = c.g_dtype == DA_F32; su.q_f32 = c.q_dtype == DA_F32;
   static DaOncePerDevice configured;
-  rc = configured.run([&]() -> int {
+  int rc = configured.run([&]() -> int {
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
     return DA_OK;
   });
   if (rc) return rc;
-  const dim3 grid(2 * (unsigned)da_cu_count());
-  if (c.m_dtype == DA_BF16) hipLaunchKernelGGL(dion_small_kernel<true>, grid, dim3(256), SMEM, s, a);
-  else hipLaunchKernelGGL(dion_small_kernel<false>, grid, dim3(256), SMEM, s, a);
+  const dim3 setup((unsigned)(su.zblocks + adds)), grid(2 * (unsigned)da_cu_count()), update((unsigned)tiles), block(256);
+  if (bf) hipLaunchKernelGGL(dion_small_setup_kernel<true>, setup, block, 0, s, su);
+  else hipLaunchKernelGGL(dion_small_setup_kernel<false>, setup, block, 0, s, su);
+  rc = da_launch_status();
+  if (rc) return rc;
+  if (bf) hipLaunchKernelGGL(dion_small_kernel<true>, grid, block, SMEM, s, a);
+  else hipLaunchKernelGGL(dion_small_kernel<false>, grid, block, SMEM, s, a);
+  rc = da_launch_status();
+  if (rc) return rc;
+  if (bf) hipLaunchKernelGGL(dion_small_update_kernel<true>, update, block, SMEM_UPDATE, s, a);
+  else hipLaunchKernelGGL(dion_small_update_kernel<false>, update, block, SMEM_UPDATE, s, a);
   return da_launch_status();
 }

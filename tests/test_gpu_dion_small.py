@@ -32,6 +32,9 @@ def _run(dev, shapes, dtype, fraction, multiple, steps, mu=0.95, kind="random"):
             g = torch.randn(p.shape, generator=gen, device=dev) * 1e-2
             if kind == "zero":
                 g.zero_()
+            elif isinstance(kind, int):     # zeros but for one element
+                v = g.flatten()[kind].item()
+                g.zero_().view(-1)[kind] = v
             elif kind == "deficient":
                 g[:, g.size(1) // 4:] = 0
                 g[g.size(0) // 4:, :] = 0
@@ -84,6 +87,19 @@ def test_small_dion_kernel_zero_and_deficient_gradients(dev, option, dtype):
                 assert rel_fro(b[2], a[2]) <= (1e-6 if dtype == F32 else 5e-3)
             else:
                 assert rel_fro(b[1], a[1]) <= (1e-4 if dtype == F32 else 1e-2), (i, rel_fro(b[1], a[1]))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("at", [0, 8191, 8192, 100 * 161 - 3, -1])
+def test_one_element_is_found_wherever_it_is(dev, option, dtype, at):
+    """B is not zero if one element is (the chunks of the pass that adds the gradient hold 8192): Q is not kept."""
+    shapes, runs = [(100, 161), (161, 100)], []
+    for mode, kind in ((0, at), (1, at), (1, "zero")):
+        option("dion_small", mode)
+        runs.append(_run(dev, shapes, dtype, 0.5, 1, 1, kind=kind)[0])
+    for a, b, zero in zip(*runs):
+        assert rel_fro(b[1], a[1]) <= (1e-4 if dtype == F32 else 1e-2)
+        assert rel_fro(b[2], zero[2]) > 0.5
 
 
 def test_a_small_dion_launch_that_gave_up_poisons_the_result(dev, option):
