@@ -557,7 +557,7 @@ bool fused_bq_enabled() {
   return !env_off;
 }
 
-// Small buckets in one launch (dion_small.hip): -1 by the amount of work, 0 never, 1 whenever possible.
+// All small buckets together (dion_small.hip): -1 by the amount of work, 0 never, 1 whenever possible.
 std::atomic<int> g_opt_dion_small{-1};
 
 // Number of slices (1, 2 or 4) of the inner dimension `mp` for the product R = B^T P (np x r per matrix, `cb`

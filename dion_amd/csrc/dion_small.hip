@@ -1,33 +1,38 @@
-// The Dion step (reference dion/dion.py:742-875) of a set of small matrices in three launches:
+// The Dion step (reference dion/dion.py:742-875) of a set of small matrices, all buckets at once:
 //
 //   B = M + G;  P = B' Q;  P <- orth(P);  R = B'^T P;  Q <- R / (||R||_col + eps);
 //   M <- B - (1 - mu) P R^T;  X <- decay X - lr P Q^T              (B' = B, or B^T when m < n; mp x np, mp >= np)
 //
 // What bounds it: as a sequence of launches a bucket takes 40 to 60 of them (a third of which only find out that the fp64
 // pass of the orthonormaliser is not needed), each a few microseconds of work: a model of 24 matrices of 256 x 256 and
-// 256 x 1024 spent 0.6-0.8 ms, most of it on the host; here 0.19 ms, three quarters of it the chain of phases (15-24 us per
-// diagonal block, 10-15 us per product), not throughput.  The element-wise ends, B = M + G and the update, are launches over the
-// whole GPU; what lies between is a list of phases per matrix, cut into tiles, in one launch:
-// workgroups take tiles from eight queues, one per XCD (flow_queue.h), and a counter per matrix and phase says when the
-// next phase may start.  A matrix stays with one XCD, so its phases meet in one L2.
+// 256 x 1024 spent 0.6-0.8 ms, most of it on the host; here 0.18 ms for ten launches, of which the factorisation, a chain of
+// 64-column steps, takes a third.
 //
-// Phases (kinds):  BQ    P = B' Q                                      64 x 64 tiles
-//                  GRAM  P^T P in fp64, lower 32 x 32 tiles, K slices as slabs of their own
-//                  DIAG0 LOW0 DIAG1 LOW1 ..   P^T P = L L^T and T = L^-1 in blocks of 64, left-looking: DIAGj adds the slabs
-//                        (in order) and the earlier columns' products to block (j, j), factors it and inverts the factor;
-//                        LOWj does the rest of block column j of L and of block row j of T, a task per block
-//                  PT    P T^T in fp64
-//                  FIX   only does anything for a matrix whose pivot range says that cond(P) may leave a visible defect, or
-//                        with a failed pivot: the closed-form second pass of da_orthonormalize in fp64 (defect measured,
-//                        noise columns dropped, P <- P (I - up(P^T P - I)))
-//                  BTP   R = B'^T P                                    64 x 64 (bf16) or 32 x 32 (fp32) tiles
-//                  CNORM column norms, Q_new, Q state                  64 x 64 tiles
+// Launches, each over all tiles of all matrices, at as many workgroups to a compute unit as its own registers and LDS allow:
+//   set-up  B = M + G in place, and where any element is not zero; Q as a padded working matrix
+//   BQ      P = B' Q                                      64 x 64 tiles
+//   GRAM    P^T P in fp64, lower tiles, K slices as slabs of their own
+//   CHAIN   P^T P = L L^T and T = L^-1 in blocks of 64, left-looking, in phases DIAG0 LOW0 DIAG1 LOW1 ..: DIAGj adds the slabs (in
+//           order) and the earlier columns' products to block (j, j), factors it and inverts the factor; LOWj does the rest of
+//           block column j of L and of block row j of T, a task per block.  Workgroups take tasks from eight queues, one per XCD
+//           (flow_queue.h), a counter per matrix and phase says when the next phase may start, and a matrix stays with one XCD.
+//   PT      P T^T in fp64
+//   FIXG, FIXP  only do anything for a matrix whose pivot range says that cond(P) may leave a visible defect, or with a failed
+//           pivot: the closed-form second pass of da_orthonormalize in fp64 (defect measured, noise columns dropped,
+//           P <- P (I - up(P^T P - I)))
+//   BTP     R = B'^T P                                    64 x 64 (bf16) or 32 x 32 (fp32) tiles
+//   CNORM   column norms, Q_new, Q state                  64 x 64 tiles
+//   UPD     error feedback and weight update              64 x 64 tiles
+// All but CHAIN used to be phases of the queues: two workgroups to a compute unit (the factorisation's registers), a matrix's tiles on
+// one XCD's 64 workgroups, and a ticket and a counter for every tile.  14 bf16 matrices of 341 to 2731 rows at rank 256 and 86 (us,
+// as phases / as launches): set-up 98 / 24, BQ 52 / 31, GRAM 62 / 41, PT 62 / 59, FIX 16 / 9, BTP 48 / 41, CNORM 7 / 9, UPD 155 / 67;
+// the step 622 / 416.  24 fp32 matrices of 256 x 256 and 256 x 1024 at rank 128: 218 / 196.
 // The orthonormaliser is the fp64 CholeskyQR of dion.hip for every matrix: at these sizes the fp64 products cost less than
 // the launches of the two-precision road.  P, R and the products with B run on the matrix cores in the momentum's dtype with
 // the instructions and the order of k of the batched kernels (v_mfma_f32_16x16x32_bf16, in the updates v_mfma_f32_32x32x16_bf16; v_mfma_f32_32x32x2_f32).
 //
-// Coherence.  Every buffer of the workspace is written once and read only after its phase is complete, and M and X change in
-// other launches: plain loads cannot meet a stale L1 line.
+// Coherence in CHAIN.  What it reads is of an earlier launch or written once, and read only after its phase is complete: plain loads
+// cannot meet a stale L1 line.
 //
 // Shapes: any m, n (rows that are no multiple of 16 bytes move with unaligned accesses), rank up to 256; the working
 // matrices are padded to whole tiles and the tiles' loads fill with zeros.
@@ -41,21 +46,26 @@
 namespace {
 
 constexpr int MAX_RT = DA_DS_MAX_RANK / 64;
-enum Kind { BQ, GRAM, DIAG, LOW, PT = GRAM + 1 + 2 * MAX_RT, FIX, BTP, CNORM, KINDS };   // DIAGj = DIAG + 2 j, LOWj
-constexpr int CTR_STRIDE = 32;     // ints per matrix: a counter per kind, then the words below
-constexpr int W_NONZERO = 18, W_SICK = 19, W_BAD = 20, W_GRAM2 = 21, W_RANGE = 24;   // (W_RANGE: two doubles)
-static_assert(KINDS <= W_NONZERO, "a counter per kind");
+// The launches behind the set-up; CHAIN is the factorisation, whose phases DIAGj (2 j), LOWj (2 j + 1) are one launch.
+enum Kind { BQ, GRAM, CHAIN, PT, FIXG, FIXP, BTP, CNORM, UPD, KINDS };
+constexpr int PHASES = 2 * MAX_RT;
+constexpr int CTR_STRIDE = 32;     // ints per matrix: a counter per phase, then the words below
+constexpr int W_NONZERO = 18, W_SICK = 19, W_BAD = 20, W_RANGE = 24;   // (W_RANGE: two doubles)
+static_assert(PHASES <= W_NONZERO, "a counter per phase");
 constexpr int ADD_ELEMS = 8192;
 constexpr double PIVOT_RATIO = 1e-7;   // as POLISH_PIVOT_RATIO in dion.hip
-constexpr int SMEM = STAGES64 + DA_DS_MAX_RANK;
-constexpr int SMEM_UPDATE = 2 * 3 * Real<float, 64>::OPND * 4;   // two stages of three fp32 operands; the bf16 ones and the two products staged behind them are smaller
+constexpr int SMEM = STAGES64 + DA_DS_MAX_RANK;                  // fp64 64-tiles: two workgroups to a compute unit
+constexpr int SMEM_TILE = 2 * 2 * Real<float, 64>::OPND * 4;     // two stages of two operands of fp32 64-tiles, fp64 32-tiles: four
+constexpr int SMEM_UPDATE = 2 * 3 * Real<float, 64>::OPND * 4;   // of three operands: three
+static_assert(SMEM_TILE >= 2 * 2 * 64 * 64 * 2 && SMEM_TILE >= 64 * 66 * 8 && SMEM_TILE >= 2 * 2 * Real<double, 32>::OPND * 8 &&
+              4 * (SMEM_TILE + 1024) <= 160 * 1024, "LDS of the products");
 static_assert(SMEM_UPDATE >= 2 * 3 * 64 * 64 * 2 && SMEM_UPDATE >= 2 * 64 * 66 * 4 && 3 * SMEM_UPDATE <= 160 * 1024, "LDS of the update");
 
 struct GroupDev {
-  void *const *X, *const *G, *const *M, *const *Q;   // device tables
+  void *const *X, *const *M, *const *Q;   // device tables
   char *P, *P2, *R, *Qn, *Qw;         // momentum dtype: [cnt][mpT * 64][rp], [cnt][npT * 64][rp]
   double* norm;                  // [cnt][nT][rp]: the column norms' shares of BTP's row tiles
-  double *P64, *slab, *L, *T, *A2, *defect;
+  double *P64, *slab, *L, *T, *A2, *defect;   // (A2: T^T until the second pass's Gram product)
   int* words;                    // [cnt][CTR_STRIDE]
   int* info;
   int* any;                      // [cnt][mchunks]: a chunk of B with an element that is not zero
@@ -76,310 +86,49 @@ struct Args {
   int ngroups;
   int total[DA_QUEUES];          // tasks of every queue
   unsigned char order[DA_DS_MATS];   // the matrices' numbers within their group, by group and queue
-  int x_f32, g_f32, q_f32;
+  int x_f32, q_f32;
   float ef_alpha, decay, eps;
 };
 
-
-__host__ __device__ inline int tasks_of(const GroupDev& G, int kind, bool bf) {
+// lower tiles of P^T P
+__host__ __device__ inline int gram_tiles(int r, bool bf) {
+  const int t = bf ? (r + 63) >> 6 : (r + 31) >> 5;
+  return t * (t + 1) / 2;
+}
+// workgroups of a launch per matrix
+__host__ __device__ inline int tiles_of(const GroupDev& G, Kind kind, bool bf) {
   const int t32 = (G.r + 31) >> 5;
   switch (kind) {
-    case BQ: case PT: return G.mpT * G.rT;
-    case GRAM: return t32 * (t32 + 1) / 2 * G.slices;
-    case FIX: return t32 * (t32 + 1) / 2 + G.mpT * G.rT;
+    case BQ: case PT: case FIXP: return G.mpT * G.rT;
+    case GRAM: return gram_tiles(G.r, bf) * G.slices;
+    case FIXG: return gram_tiles(G.r, false);
     case BTP: return bf ? G.npT * G.rT : ((G.np + 31) >> 5) * t32;
     case CNORM: return G.npT * G.rT;
-    default: {   // block column j: the diagonal block; the blocks below it and the blocks of row j of the inverse
-      const int j = (kind - DIAG) >> 1;
-      return j >= G.rT ? 0 : ((kind - DIAG) & 1) ? G.rT - 1 : 1;
-    }
+    case UPD: return G.mpT * G.npT;
+    default: return 0;
   }
 }
-
-// ---- the kernel ----------------------------------------------------------------------------------------------------------
+// tasks of a phase of the factorisation: the diagonal block; the blocks below it and the blocks of row j of the inverse
+__host__ __device__ inline int tasks_of(const GroupDev& G, int phase) {
+  return (phase >> 1) >= G.rT ? 0 : (phase & 1) ? G.rT - 1 : 1;
+}
 
 template <bool BF> struct MomentumType { typedef float type; };
 template <> struct MomentumType<true> { typedef bf16_t type; };
 
-template <bool BF>
-__global__ __launch_bounds__(256, 2) void dion_small_kernel(Args args) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  __shared__ int sh_ticket[2];
-  __shared__ int sh_words[2];
-  __shared__ int sh_start[128], sh_per[128], sh_wait[128];   // the queue's schedule: entry = kind * ngroups + group
-  __shared__ unsigned char sh_at[128], sh_order[DA_DS_MATS];
-  static_assert(KINDS * DA_DS_GROUPS <= 128, "one entry each");
-  constexpr int MSZ = BF ? 2 : 4, MT = BF ? DA_BF16 : DA_F32;
-  const int xcd = xcc_id();
-
-  for (int qi = 0; qi < DA_QUEUES; ++qi) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int q = (xcd + qi) & (DA_QUEUES - 1);
-    const int total = args.total[q];
-    if (total <= 0) continue;
-    unsigned* word = args.tickets + q * DA_QUEUE_LINE;
-    int slot = 0;
-    if (tid == 0) sh_ticket[0] = take_ticket(word, xcd, total, false);
-    __syncthreads();
-    if (wave_uniform(sh_ticket[0]) < 0) {
-      __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
-      continue;
-    }
-    // ---- the schedule, phase by phase, group by group: first ticket, tasks per matrix, and what a phase waits for
-    if (tid < 128) {
-      int n = 0;
-      if (tid < KINDS * args.ngroups) {
-        const int k = tid / args.ngroups;
-        const GroupDev& G = args.g[tid - k * args.ngroups];
-        const int per = tasks_of(G, k, BF);
-        n = per * G.nq[q];
-        int w = k == BTP ? PT : k - 1;
-        while (w >= 0 && tasks_of(G, w, BF) == 0) --w;
-        sh_per[tid] = per;
-        sh_at[tid] = G.at[q];
-        sh_wait[tid] = w < 0 ? -1 : (w << 24 | tasks_of(G, w, BF));
-      }
-      sh_start[tid] = n;
-      if (tid < DA_DS_MATS) sh_order[tid] = args.order[tid];
-    }
-    __syncthreads();
-    if (tid < 64) {   // exclusive sums of 128 entries by one wavefront
-      const int lo = sh_start[2 * lane], hi = sh_start[2 * lane + 1];
-      int sum = lo + hi;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int x = __shfl_up(sum, o);
-        if (lane >= o) sum += x;
-      }
-      sh_start[2 * lane] = sum - lo - hi;
-      sh_start[2 * lane + 1] = sum - hi;
-    }
-    while (true) {
-      __syncthreads();
-      int t = wave_uniform(sh_ticket[slot]);
-      if (t < 0) break;
-      // (opaque to the compiler: every phase's address arithmetic would move out of this loop and be spilled)
-      int tid = threadIdx.x;
-      asm volatile("" : "+v"(tid));
-      const int lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
-      const Args& a = fresh_args<Args>();
-      // ---- ticket -> (kind, group, matrix, task): the last entry that starts at or before it
-      const int entry = wave_uniform(__popcll(__ballot(sh_start[lane] <= t)) + __popcll(__ballot(sh_start[64 + lane] <= t)) - 1);
-      t -= wave_uniform(sh_start[entry]);
-      const int kind = entry / a.ngroups, per = wave_uniform(sh_per[entry]), wait = wave_uniform(sh_wait[entry]);
-      const GroupDev& G = a.g[entry - kind * a.ngroups];
-      const int kth = wave_uniform(t / per);
-      const int task = wave_uniform(t - kth * per);
-      const int b = wave_uniform((int)sh_order[sh_at[entry] + kth]);
-      int* words = G.words + (long long)b * CTR_STRIDE;
-      if (tid == 0) {
-        if (wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
-        int sick = __hip_atomic_load(words + W_SICK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (kind == BTP && sick) wait_count(words + FIX, tasks_of(G, FIX, BF), a.status, a.spin_limit);
-        sh_words[0] = __hip_atomic_load(words + W_NONZERO, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sh_words[1] = sick;
-      }
-      __syncthreads();
-      const bool nonzero = sh_words[0] != 0, sick = sh_words[1] != 0;
-      unsigned next = DA_NO_TICKET;
-      auto ask = [&]() {
-        if (tid == 0) next = request_ticket(word);
-      };
-
-      const int rp = G.rp, mpR = G.mpT * 64, npR = G.npT * 64;
-      char* const P = G.P + (long long)b * mpR * rp * MSZ;
-      char* const P2 = G.P2 + (long long)b * mpR * rp * MSZ;
-      char* const R = G.R + (long long)b * npR * rp * MSZ;
-      char* const Qw = G.Qw + (long long)b * npR * rp * MSZ;
-      char* const Qn = G.Qn + (long long)b * npR * rp * MSZ;
-      double* const P64 = G.P64 + (long long)b * mpR * rp;
-      const long long rr = (long long)rp * rp;
-      char* const M = static_cast<char*>(G.M[b]);
-      typedef typename MomentumType<BF>::type E;    // bf16_t or float
-      const long long last = (long long)G.m * G.n - 8;
-      auto momentum = [&](bool turned) {            // B' (false), B'^T (true)
-        return Opnd<E, true>{reinterpret_cast<const E*>(M), G.n, (G.transposed != 0) != turned, turned ? G.np : G.mp,
-                             turned ? G.mp : G.np, last};
-      };
-      float* const stg = reinterpret_cast<float*>(lds);
-
-      if (kind == BQ || kind == BTP) {
-        // ---- P = B' Q;  R = B'^T P
-        const bool bq = kind == BQ;
-        const int rT = G.rT, rt32 = (G.r + 31) >> 5;
-        if (bq && task == 0) {   // has any element of B been found not to be zero?
-          bool any = false;
-          for (int i = tid; i < G.mchunks; i += 256) any |= G.any[(long long)b * G.mchunks + i] != 0;
-          if (__any(any) && lane == 0) __hip_atomic_store(words + W_NONZERO, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        const Opnd<E, true> sa = momentum(!bq);
-        const Opnd<E, false> sb = work<E>(bq ? Qw : P2, rp, 1);
-        const int kend = bq ? G.np : G.mp;
-        char* const C = bq ? P : R;
-        // a chunk of the result: rounded and, for R, guarded (an all-zero B keeps Q)
-        auto put = [&](int row0, int col0, int lr, int lc, int pitch) {
-          const int row = row0 + lr, col = col0 + lc;
-          float v[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = stg[lr * pitch + lc + i];
-          if (!bq) {
-            float alt[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) alt[i] = 0.f;
-            if (!nonzero) unpack(load_raw(reinterpret_cast<const E*>(Qw) + (long long)row * rp + col), alt);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = guard<BF>(v[i], nonzero, alt[i]);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) stg[lr * pitch + lc + i] = v[i];
-          }
-          store8(C, !BF, (long long)row * rp + col, 8, v);
-        };
-        // the tile's share of the column norms
-        auto norms = [&](int ti, int row0, int col0, int pitch, int tb) {
-          __syncthreads();
-          double* const red = reinterpret_cast<double*>(lds + 64 * 66 * 4);
-          const int c = tid & (tb - 1), g = tid / tb, rows = tb * tb / 256;
-          double s = 0.0;
-          for (int i = g * rows; i < (g + 1) * rows; ++i) {
-            const float v = row0 + i < G.np ? stg[i * pitch + c] : 0.f;
-            s += (double)v * (double)v;
-          }
-          red[tid] = s;
-          __syncthreads();
-          if (tid < tb) {
-            double t = 0.0;
-            for (int i = 0; i < 256 / tb; ++i) t += red[i * tb + tid];
-            G.norm[((long long)b * G.nT + ti) * rp + col0 + tid] = t;
-          }
-        };
-        if (BF || bq) {
-          const int ti = task / rT, tj = task - ti * rT, row0 = wave_uniform(ti) * 64, col0 = wave_uniform(tj) * 64;
-          if constexpr (BF) {
-            product_bf16(sa, sb, row0, col0, kend, lds, tid, lane, wm, wn, stg);
-          } else {
-            f32x16_t acc[1];
-            const Opnd<E, false> sbs[1] = {sb};
-            tile32x2<1>(sa, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc);
-            stage_f32(acc[0], stg, lane, wm, wn);
-          }
-          ask();
-          __syncthreads();
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            put(row0, col0, (tid >> 3) + 32 * h, (tid & 7) * 8, 66);
-          }
-          if (!bq) norms(ti, row0, col0, 66, 64);
-        } else {
-          const int ti = task / rt32, tj = task - ti * rt32, row0 = wave_uniform(ti) * 32, col0 = wave_uniform(tj) * 32;
-          if constexpr (!BF) tile16<float, 32>(sa, sb, row0, col0, 0, kend, stg, tid, lane, wm, wn);
-          ask();
-          if (tid < 128) put(row0, col0, tid >> 2, (tid & 3) * 8, 34);
-          norms(ti, row0, col0, 34, 32);
-        }
-      } else if (kind == GRAM) {
-        // ---- one lower 32 x 32 tile of one K slice of P^T P
-        const int t32 = (G.r + 31) >> 5, per_slice = t32 * (t32 + 1) / 2;
-        const int slice = wave_uniform(task / per_slice), kbeg = slice * G.kslice;
-        int ti, tj;
-        gram_tile(work<E>(P, rp, 1), task - slice * per_slice, kbeg, min(kbeg + G.kslice, (G.mp + KD - 1) / KD * KD),
-                  G.slab + ((long long)b * G.slices + slice) * rr, rp, reinterpret_cast<double*>(lds), tid, lane, wm, wn, ti, tj);
-        ask();
-      } else if (kind == FIX && !sick) {
-        ask();   // what nearly every matrix does
-      } else if (kind < PT) {
-        const Factor F = {G.slab + (long long)b * G.slices * rr, G.L + b * rr, G.T + b * rr, G.slices, G.r, rp, G.rT,
-                          words + W_BAD, words + W_SICK, G.info ? G.info + b : nullptr, reinterpret_cast<double*>(words + W_RANGE), PIVOT_RATIO};
-        factor_task(F, (kind - DIAG) >> 1, !((kind - DIAG) & 1), task, lds, tid, lane, wave, wm, wn);
-        ask();
-      } else if (kind == PT || kind == FIX) {
-        double* const d = reinterpret_cast<double*>(lds);
-        const int rT = G.rT, t32 = (G.r + 31) >> 5, ng = t32 * (t32 + 1) / 2;
-        if (kind == FIX && task < ng) {
-          int ti, tj;
-          gram_tile(work<double>(P64, rp, 1), task, 0, (G.mp + KD - 1) / KD * KD, G.A2 + b * rr, rp, d, tid, lane, wm, wn, ti, tj);
-          ask();
-          gram_defect(d, G.defect + (long long)b * rp * (2 * MAX_RT), 2 * MAX_RT, ti, tj, tid);
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
-          if (tid == 0) __hip_atomic_fetch_add(words + W_GRAM2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        } else {
-          const int t = kind == PT ? task : task - ng;
-          const int row0 = wave_uniform(t / rT) * 64, col0 = wave_uniform(t % rT) * 64;
-          if (kind == PT) {   // P T^T (T is triangular)
-            tile16<double, 64>(work<E>(P, rp, 0), work<double>(G.T + b * rr, rp, 0), row0, col0, 0, col0 + 64, d, tid, lane, wm, wn);
-          } else {
-            if (tid == 0) wait_count(words + W_GRAM2, ng, a.status, a.spin_limit);
-            __syncthreads();
-            unsigned char* const drop = reinterpret_cast<unsigned char*>(lds + STAGES64);
-            find_dropped(G.defect + (long long)b * rp * (2 * MAX_RT), 2 * MAX_RT, G.r, rp, drop, tid);
-            if (t == 0 && tid == 0 && G.info && __hip_atomic_load(words + W_BAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-              for (int c = 0; c < G.r; ++c)
-                if (drop[c]) { G.info[b] = c + 1; break; }
-            }
-            polish_tile(P64, G.A2 + b * rr, G.r, rp, drop, row0, col0, d, tid, lane, wm, wn);
-          }
-          ask();
-          if (kind == PT && sick) {
-            for (int e = tid; e < 4096; e += 256) P64[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
-          } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
-              float v[8];
-#pragma unroll
-              for (int i = 0; i < 8; ++i) v[i] = guard<BF>((float)d[r * 66 + c + i], nonzero, 0.f);
-              store8(P2, !BF, (long long)(row0 + r) * rp + col0 + c, 8, v);
-            }
-          }
-        }
-      } else if (kind == CNORM) {
-        // ---- a 64 x 64 tile of R: column norms from the tiles' shares (in order), Q_new in the momentum's dtype and as Q state
-        const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-        double* const red = reinterpret_cast<double*>(lds);
-        float* const den = reinterpret_cast<float*>(lds + 4096);
-        const int ti = wave_uniform(task / G.rT), row0 = ti * 64, col0 = wave_uniform(task - ti * G.rT) * 64;
-        const int limit = BF ? rp : ((G.r + 31) >> 5) << 5;   // columns of R that exist
-        Raw<E> rv[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          rv[h] = load_raw(reinterpret_cast<const E*>(R) + (long long)(row0 + (tid >> 3) + 32 * h) * rp + col0 + (tid & 7) * 8);
-        {
-          double s = 0.0;
-          if (col0 + (tid & 63) < limit)
-            for (int t = tid >> 6; t < G.nT; t += 4) s += G.norm[((long long)b * G.nT + t) * rp + col0 + (tid & 63)];
-          red[tid] = s;
-        }
-        __syncthreads();
-        if (tid < 64) den[tid] = sqrtf((float)(red[tid] + red[64 + tid] + red[128 + tid] + red[192 + tid])) + a.eps;
-        ask();
-        __syncthreads();
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int row = row0 + (tid >> 3) + 32 * h, c = (tid & 7) * 8, col = col0 + c;
-          float v[8];
-          unpack(rv[h], v);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            v[i] = v[i] / den[c + i];
-            if (BF) v[i] = rbf(v[i]);
-            if (poisoned) v[i] = __builtin_nanf("");
-            if (row >= G.np || col + i >= G.r) v[i] = 0.f;   // (padding)
-          }
-          store8(Qn, !BF, (long long)row * rp + col, 8, v);
-          store8(static_cast<char*>(G.Q[b]), a.q_f32, (long long)row * G.r + col, row < G.np ? G.r - col : 0, v);
-        }
-      } else {
-        ask();   // a phase that a healthy matrix does not need
-      }
-      // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
-      if (tid == 0) sh_ticket[slot ^ 1] = ticket_of(next, total);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tid == 0) __hip_atomic_fetch_add(words + kind, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (in the L2)
-      slot ^= 1;
-    }
-    __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
+// A workgroup's tile.  The tiles of a launch are dealt in eight runs, one to an XCD (which workgroups reach in turn): the tiles of a
+// matrix meet in one L2.
+struct Where { int g, b, task; };
+template <Kind KIND, bool BF>
+__device__ __forceinline__ Where my_tile(const Args& a) {
+  const int q = blockIdx.x & 7, each = gridDim.x >> 3, rest = gridDim.x & 7;
+  int t = q * each + min(q, rest) + (blockIdx.x >> 3), g = 0, per;
+  for (;; ++g) {
+    per = tiles_of(a.g[g], KIND, BF);
+    if (t < a.g[g].cnt * per || g + 1 == a.ngroups) break;
+    t -= a.g[g].cnt * per;
   }
+  return {g, t / per, t % per};
 }
 
 struct SetupGroup {
@@ -390,8 +139,8 @@ struct SetupGroup {
   int* any;
 };
 struct Setup {
-  void* p[4][DA_DS_MATS];   // X, G, M, Q
-  void** dst;               // [4][n]
+  void* p[4][DA_DS_MATS];   // X, M, Q, G
+  void** dst;               // [3][n]: X, M, Q
   int n;
   int* zero;
   int nzero, zblocks;
@@ -402,7 +151,6 @@ struct Setup {
 };
 // The pointers and the counters of the step (the first blocks); B = M + G in place and the note which chunks of it are not all
 // zeros; Q as a padded working matrix.  Bound by memory: 5.5 TB/s, 24 us for 14 matrices of 341 to 2731 rows (22 million elements).
-// As a phase of the queues, where an XCD's 64 workgroups wait for their loads and then for their stores, it took 98 us.
 template <bool BF>
 __global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
   typedef typename MomentumType<BF>::type E;
@@ -411,7 +159,7 @@ __global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
     const int i = blockIdx.x * 256 + tid;
     if (i < s.n) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) s.dst[k * s.n + i] = s.p[k][i];
+      for (int k = 0; k < 3; ++k) s.dst[k * s.n + i] = s.p[k][i];
     }
     for (int e = i; e < s.nzero; e += s.zblocks * 256) s.zero[e] = 0;
     if (i == 0) *s.status = s.preset;
@@ -430,18 +178,18 @@ __global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
       if (row >= G.npR) break;
       const int c = row < G.np ? G.r - col : 0;
       float v[8];
-      if (s.q_f32) load8(static_cast<const float*>(s.p[3][mat]), (long long)row * G.r + col, c, v);
-      else load8(static_cast<const bf16_t*>(s.p[3][mat]), (long long)row * G.r + col, c, v);
+      if (s.q_f32) load8(static_cast<const float*>(s.p[2][mat]), (long long)row * G.r + col, c, v);
+      else load8(static_cast<const bf16_t*>(s.p[2][mat]), (long long)row * G.r + col, c, v);
       store8(G.Qw + (long long)b * G.npR * G.rp * sizeof(E), !BF, e, 8, v);
     }
     return;
   }
   // ---- M + G: every load of a whole chunk on the way before the first is used
   const long long n = (long long)G.m * G.n, e0 = (long long)task * ADD_ELEMS + tid * 8;
-  char* const M = static_cast<char*>(s.p[2][mat]);
+  char* const M = static_cast<char*>(s.p[1][mat]);
   const E* const m = reinterpret_cast<const E*>(M);
-  const bf16_t* const g16 = static_cast<const bf16_t*>(s.p[1][mat]);
-  const float* const g32 = static_cast<const float*>(s.p[1][mat]);
+  const bf16_t* const g16 = static_cast<const bf16_t*>(s.p[3][mat]);
+  const float* const g32 = static_cast<const float*>(s.p[3][mat]);
   bool any = false;
   auto finish = [&](float (&mv)[8], const float (&gv)[8], long long e, int c) {
 #pragma unroll
@@ -483,26 +231,305 @@ __global__ __launch_bounds__(256) void dion_small_setup_kernel(Setup s) {
   if (tid == 0) G.any[(long long)b * G.mblocks + task] = any;
 }
 
+// P = B' Q;  R = B'^T P: a 64 x 64 tile (of R in fp32 32 x 32).  Bound by the latency of a tile's stages.
+template <bool BF, bool bq>
+__global__ __launch_bounds__(256, 4) void dion_small_product_kernel(Args a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename MomentumType<BF>::type E;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const Where w = my_tile<bq ? BQ : BTP, BF>(a);
+  const GroupDev& G = a.g[w.g];
+  const int b = w.b, task = w.task, rp = G.rp;
+  const long long prow = (long long)b * G.mpT * 64 * rp * sizeof(E), rrow = (long long)b * G.npT * 64 * rp * sizeof(E);
+  char *const P = G.P + prow, *const P2 = G.P2 + prow, *const R = G.R + rrow, *const Qw = G.Qw + rrow;
+  float* const stg = reinterpret_cast<float*>(lds);
+  const int rT = G.rT, rt32 = (G.r + 31) >> 5;
+  if (bq && task == 0) {   // has any element of B been found not to be zero?
+    bool any = false;
+    for (int i = tid; i < G.mchunks; i += 256) any |= G.any[(long long)b * G.mchunks + i] != 0;
+    if (__any(any) && lane == 0) __hip_atomic_store(G.words + b * CTR_STRIDE + W_NONZERO, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const bool nonzero = G.words[b * CTR_STRIDE + W_NONZERO] != 0;   // (of R: of the launch before)
+  const bool turn = (G.transposed != 0) == bq;   // B' is B^T, or R takes B'^T
+  auto with_layout = [&](auto body) {   // (the layout known to the compiler: no branch in the K loop)
+    const E* const M = static_cast<const E*>(G.M[b]);
+    const int rows = bq ? G.mp : G.np, kmax = bq ? G.np : G.mp;
+    const long long last = (long long)G.m * G.n - 8;
+    if (turn) body(Opnd<E, true>{M, G.n, 1, rows, kmax, last});
+    else body(Opnd<E, true>{M, G.n, 0, rows, kmax, last});
+  };
+  const Opnd<E, false> sb = work<E>(bq ? Qw : P2, rp, 1);
+  const int kend = bq ? G.np : G.mp;
+  char* const C = bq ? P : R;
+  // a chunk of the result: rounded and, for R, guarded (an all-zero B keeps Q)
+  auto put = [&](int row0, int col0, int lr, int lc, int pitch) {
+    const int row = row0 + lr, col = col0 + lc;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = row < (bq ? G.mp : G.np) ? stg[lr * pitch + lc + i] : 0.f;
+    if (!bq) {
+      float alt[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) alt[i] = 0.f;
+      if (!nonzero) unpack(load_raw(reinterpret_cast<const E*>(Qw) + (long long)row * rp + col), alt);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = guard<BF>(v[i], nonzero, alt[i]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) stg[lr * pitch + lc + i] = v[i];
+    }
+    store8(C, !BF, (long long)row * rp + col, 8, v);
+  };
+  // the tile's share of the column norms
+  auto norms = [&](int ti, int row0, int col0, int pitch, int tb) {
+    __syncthreads();
+    double* const red = reinterpret_cast<double*>(lds + 64 * 66 * 4);
+    const int c = tid & (tb - 1), g = tid / tb, rows = tb * tb / 256;
+    double s = 0.0;
+    for (int i = g * rows; i < (g + 1) * rows; ++i) {
+      const float v = row0 + i < G.np ? stg[i * pitch + c] : 0.f;
+      s += (double)v * (double)v;
+    }
+    red[tid] = s;
+    __syncthreads();
+    if (tid < tb) {
+      double t = 0.0;
+      for (int i = 0; i < 256 / tb; ++i) t += red[i * tb + tid];
+      G.norm[((long long)b * G.nT + ti) * rp + col0 + tid] = t;
+    }
+  };
+  if (BF || bq) {
+    const int ti = task / rT, tj = task - ti * rT, row0 = wave_uniform(ti) * 64, col0 = wave_uniform(tj) * 64;
+    if constexpr (BF) {
+      with_layout([&](const Opnd<E, true>& sa) { product_bf16(sa, sb, row0, col0, kend, lds, tid, lane, wm, wn, stg); });
+    } else {
+      f32x16_t acc[1];
+      const Opnd<E, false> sbs[1] = {sb};
+      with_layout([&](const Opnd<E, true>& sa) { tile32x2<1>(sa, sbs, row0, col0, kend, stg, tid, lane, wm, wn, acc); });
+      stage_f32(acc[0], stg, lane, wm, wn);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      put(row0, col0, (tid >> 3) + 32 * h, (tid & 7) * 8, 66);
+    }
+    if (!bq) norms(ti, row0, col0, 66, 64);
+  } else {
+    const int ti = task / rt32, tj = task - ti * rt32, row0 = wave_uniform(ti) * 32, col0 = wave_uniform(tj) * 32;
+    if constexpr (!BF) with_layout([&](const Opnd<E, true>& sa) { tile16<float, 32>(sa, sb, row0, col0, 0, kend, stg, tid, lane, wm, wn); });
+    if (tid < 128) put(row0, col0, tid >> 2, (tid & 3) * 8, 34);
+    norms(ti, row0, col0, 34, 32);
+  }
+}
+
+// One lower tile of one K slice of P^T P: 64 x 64 of a bf16 P, 32 x 32 of an fp32 one.  Bound by the fp64 matrix cores: 41 us for
+// 1.8 GFLOP in bf16 (32 x 32 tiles through fp64 stages: 64).
+template <bool BF>
+__global__ __launch_bounds__(256, BF ? 3 : 4) void dion_small_gram_kernel(Args a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename MomentumType<BF>::type E;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const Where w = my_tile<GRAM, BF>(a);
+  const GroupDev& G = a.g[w.g];
+  const int rp = G.rp, n = gram_tiles(G.r, BF), slice = w.task / n, kbeg = slice * G.kslice;
+  const E* const P = reinterpret_cast<const E*>(G.P) + (long long)w.b * G.mpT * 64 * rp;
+  double *const out = G.slab + ((long long)w.b * G.slices + slice) * rp * rp, *const d = reinterpret_cast<double*>(lds);
+  if constexpr (BF) {
+    int ti = 0, tj = w.task - slice * n;
+    while (tj > ti) tj -= ++ti;
+    gram64_bf16(P + (long long)kbeg * rp, rp, ti * 64, tj * 64, min(G.kslice, G.mpT * 64 - kbeg), lds, tid, lane, wm, wn);
+    for (int e = tid; e < 4096; e += 256) out[(long long)(ti * 64 + (e >> 6)) * rp + tj * 64 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
+  } else {
+    int ti, tj;
+    gram_tile(work<E>(P, rp, 1), w.task - slice * n, kbeg, min(kbeg + G.kslice, (G.mp + KD - 1) / KD * KD), out, rp, d, tid, lane, wm, wn, ti, tj);
+  }
+}
+
+// The factorisation: phases of a matrix one after the other, tasks from the queue of its XCD.
+__global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  __shared__ int sh_ticket[2];
+  __shared__ int sh_start[64], sh_per[64], sh_wait[64];   // the queue's schedule: entry = phase * ngroups + group
+  __shared__ unsigned char sh_at[64];
+  static_assert(PHASES * DA_DS_GROUPS <= 64, "one entry each");
+  const int xcd = xcc_id();
+
+  for (int qi = 0; qi < DA_QUEUES; ++qi) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int q = (xcd + qi) & (DA_QUEUES - 1);
+    const int total = args.total[q];
+    if (total <= 0) continue;
+    unsigned* word = args.tickets + q * DA_QUEUE_LINE;
+    int slot = 0;
+    if (tid == 0) sh_ticket[0] = take_ticket(word, xcd, total, false);
+    __syncthreads();
+    if (wave_uniform(sh_ticket[0]) < 0) {
+      __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
+      continue;
+    }
+    // ---- the schedule, phase by phase, group by group: first ticket, tasks per matrix, and what a phase waits for
+    if (tid < 64) {
+      int n = 0;
+      if (tid < PHASES * args.ngroups) {
+        const int k = tid / args.ngroups;
+        const GroupDev& G = args.g[tid - k * args.ngroups];
+        const int per = tasks_of(G, k);
+        n = per * G.nq[q];
+        int w = k - 1;
+        while (w >= 0 && tasks_of(G, w) == 0) --w;
+        sh_per[tid] = per;
+        sh_at[tid] = G.at[q];
+        sh_wait[tid] = w < 0 ? -1 : (w << 24 | tasks_of(G, w));
+      }
+      int sum = n;   // exclusive sums
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(sum, o);
+        if (lane >= o) sum += x;
+      }
+      sh_start[tid] = sum - n;
+    }
+    while (true) {
+      __syncthreads();
+      int t = wave_uniform(sh_ticket[slot]);
+      if (t < 0) break;
+      // (opaque to the compiler: every phase's address arithmetic would move out of this loop and be spilled)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+      const Args& a = fresh_args<Args>();
+      // ---- ticket -> (phase, group, matrix, task): the last entry that starts at or before it
+      const int entry = wave_uniform(__popcll(__ballot(lane < PHASES * a.ngroups && sh_start[lane] <= t)) - 1);
+      t -= wave_uniform(sh_start[entry]);
+      const int phase = entry / a.ngroups, per = wave_uniform(sh_per[entry]), wait = wave_uniform(sh_wait[entry]);
+      const GroupDev& G = a.g[entry - phase * a.ngroups];
+      const int kth = wave_uniform(t / per);
+      const int task = wave_uniform(t - kth * per);
+      const int b = wave_uniform((int)a.order[sh_at[entry] + kth]);
+      int* words = G.words + (long long)b * CTR_STRIDE;
+      if (tid == 0 && wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
+      __syncthreads();
+      const long long rr = (long long)G.rp * G.rp;
+      const Factor F = {G.slab + (long long)b * G.slices * rr, G.L + b * rr, G.T + b * rr, G.A2 + b * rr, G.slices, G.r, G.rp, G.rT,
+                        words + W_BAD, words + W_SICK, G.info ? G.info + b : nullptr, reinterpret_cast<double*>(words + W_RANGE), PIVOT_RATIO};
+      factor_task(F, phase >> 1, (phase & 1) == 0, task, lds, tid, lane, wave, wm, wn);
+      // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
+      unsigned next = DA_NO_TICKET;
+      if (tid == 0) next = request_ticket(word);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (tid == 0) sh_ticket[slot ^ 1] = ticket_of(next, total);
+      __syncthreads();
+      if (tid == 0) __hip_atomic_fetch_add(words + phase, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (in the L2)
+      slot ^= 1;
+    }
+    __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
+  }
+}
+
+// P T^T in fp64 (PT; bound by the fp64 matrix cores, 59 us for 1.8 GFLOP; through LDS stages 75); for a matrix that needs it the second pass: P^T P (FIXG), P <- P (I - up(P^T P - I)) (FIXP).
+template <Kind KIND, bool BF>
+__global__ __launch_bounds__(256, KIND == FIXG ? 4 : KIND == PT ? 3 : 2) void dion_small_orth_kernel(Args a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  typedef typename MomentumType<BF>::type E;
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const Where w = my_tile<KIND, BF>(a);
+  const GroupDev& G = a.g[w.g];
+  const int b = w.b, t = w.task, rp = G.rp;
+  const int* const words = G.words + (long long)b * CTR_STRIDE;
+  const bool sick = words[W_SICK] != 0, nonzero = words[W_NONZERO] != 0;
+  if (KIND != PT && !sick) return;   // what nearly every matrix does
+  const long long rr = (long long)rp * rp, prow = (long long)b * G.mpT * 64 * rp;
+  double *const P64 = G.P64 + prow, *const d = reinterpret_cast<double*>(lds);
+  double* const defect = G.defect + (long long)b * rp * (2 * MAX_RT);
+  if constexpr (KIND == FIXG) {
+    int ti, tj;
+    gram_tile(work<double>(P64, rp, 1), t, 0, (G.mp + KD - 1) / KD * KD, G.A2 + b * rr, rp, d, tid, lane, wm, wn, ti, tj);
+    gram_defect(d, defect, 2 * MAX_RT, ti, tj, tid);
+    return;
+  }
+  const int row0 = t / G.rT * 64, col0 = t % G.rT * 64;
+  if constexpr (KIND == PT) {   // (T is triangular)
+    direct64<false>(reinterpret_cast<const E*>(G.P) + prow + (long long)row0 * rp, rp, G.A2 + b * rr + col0, rp, col0 + 64, d, lane, wm, wn);
+    if (sick) {
+      for (int e = tid; e < 4096; e += 256) P64[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
+      return;
+    }
+  } else {
+    unsigned char* const drop = reinterpret_cast<unsigned char*>(lds + STAGES64);
+    find_dropped(defect, 2 * MAX_RT, G.r, rp, drop, tid);
+    if (t == 0 && tid == 0 && G.info && words[W_BAD] == 0) {
+      for (int c = 0; c < G.r; ++c)
+        if (drop[c]) { G.info[b] = c + 1; break; }
+    }
+    polish_tile(P64, G.A2 + b * rr, G.r, rp, drop, row0, col0, d, tid, lane, wm, wn);
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = guard<BF>((float)d[r * 66 + c + i], nonzero, 0.f);
+    store8(G.P2 + prow * sizeof(E), !BF, (long long)(row0 + r) * rp + col0 + c, 8, v);
+  }
+}
+
+// A 64 x 64 tile of R: column norms from the tiles' shares (in order), Q_new in the momentum's dtype and as Q state.
+template <bool BF>
+__global__ __launch_bounds__(256) void dion_small_cnorm_kernel(Args a) {
+  __shared__ double red[256];
+  __shared__ float den[64];
+  typedef typename MomentumType<BF>::type E;
+  const int tid = threadIdx.x;
+  const Where w = my_tile<CNORM, BF>(a);
+  const GroupDev& G = a.g[w.g];
+  const int b = w.b, task = w.task, rp = G.rp;
+  const long long rrow = (long long)b * G.npT * 64 * rp * sizeof(E);
+  const char* const R = G.R + rrow;
+  char* const Qn = G.Qn + rrow;
+  const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  const int ti = wave_uniform(task / G.rT), row0 = ti * 64, col0 = wave_uniform(task - ti * G.rT) * 64;
+  const int limit = BF ? rp : ((G.r + 31) >> 5) << 5;   // columns of R that exist
+  Raw<E> rv[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    rv[h] = load_raw(reinterpret_cast<const E*>(R) + (long long)(row0 + (tid >> 3) + 32 * h) * rp + col0 + (tid & 7) * 8);
+  {
+    double s = 0.0;
+    if (col0 + (tid & 63) < limit)
+      for (int t = tid >> 6; t < G.nT; t += 4) s += G.norm[((long long)b * G.nT + t) * rp + col0 + (tid & 63)];
+    red[tid] = s;
+  }
+  __syncthreads();
+  if (tid < 64) den[tid] = sqrtf((float)(red[tid] + red[64 + tid] + red[128 + tid] + red[192 + tid])) + a.eps;
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int row = row0 + (tid >> 3) + 32 * h, c = (tid & 7) * 8, col = col0 + c;
+    float v[8];
+    unpack(rv[h], v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = v[i] / den[c + i];
+      if (BF) v[i] = rbf(v[i]);
+      if (poisoned) v[i] = __builtin_nanf("");
+      if (row >= G.np || col + i >= G.r) v[i] = 0.f;   // (padding)
+    }
+    store8(Qn, !BF, (long long)row * rp + col, 8, v);
+    store8(static_cast<char*>(G.Q[b]), a.q_f32, (long long)row * G.r + col, row < G.np ? G.r - col : 0, v);
+  }
+}
+
 // Error feedback and weight update, M += ef_alpha P R^T and X = decay X - lr P Q_new^T: a 64 x 64 tile (rows of P, rows of R) per
 // workgroup, three workgroups to a compute unit, the tiles of an XCD next to each other (it keeps their R and Q_new in its L2).
-// A launch of its own: bound by the latency of a tile's loads, it was a phase of the queues at two workgroups to a compute unit
-// (the registers of the factorisation) and with a matrix to an XCD.  155 -> 66 us (14 matrices as above, rank 256 and 86; the whole
-// step 607 -> 458); fp32, 24 matrices of 256 x 256 and 256 x 1024 at rank 128: 22 -> 27, but the step 222 -> 203 with both ends out.
+// Bound by the latency of a tile's loads.
 template <bool BF>
 __global__ __launch_bounds__(256, 3) void dion_small_update_kernel(Args a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   typedef typename MomentumType<BF>::type E;
   constexpr int MSZ = BF ? 2 : 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_uniform(tid >> 6), wm = wave >> 1, wn = wave & 1;
-  const int q = blockIdx.x & 7, each = gridDim.x >> 3, rest = gridDim.x & 7;
-  int t = q * each + min(q, rest) + (blockIdx.x >> 3), gi = 0;   // (workgroups go to the XCDs in turn)
-  for (;; ++gi) {
-    const int mine = a.g[gi].cnt * a.g[gi].mpT * a.g[gi].npT;
-    if (t < mine || gi + 1 == a.ngroups) break;
-    t -= mine;
-  }
-  const GroupDev& G = a.g[gi];
-  const int b = t / (G.mpT * G.npT), task = t - b * (G.mpT * G.npT);
+  const Where w = my_tile<UPD, BF>(a);
+  const GroupDev& G = a.g[w.g];
+  const int b = w.b, task = w.task;
   const int rp = G.rp;
   const char* const P2 = G.P2 + (long long)b * G.mpT * 64 * rp * MSZ;
   const char* const R = G.R + (long long)b * G.npT * 64 * rp * MSZ;
@@ -580,21 +607,29 @@ inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct Shape {
   int mp, np, mpT, npT, rT, rp, nT, slices, kslice;
-  Shape(int m, int n, int r, bool bf) {
+  Shape(int m, int n, int r, bool bf, int rows = 128) {
     mp = m > n ? m : n;
     np = m > n ? n : m;
     mpT = (mp + 63) / 64; npT = (np + 63) / 64; rT = (r + 63) / 64;
     rp = rT * 64;
     nT = bf ? npT : (np + 31) / 32;
-    // enough Gram tasks for an XCD's 32 compute units, at least 128 rows each
-    const int t32 = (r + 31) / 32, tiles = t32 * (t32 + 1) / 2;
-    slices = (64 + tiles - 1) / tiles;
-    if (slices > mp / 128) slices = mp / 128;
+    // K slices: about `rows` rows to a Gram tile, at least 128, in whole stages
+    const int deep = bf ? 64 : KD;
+    slices = mp / (rows > 128 ? rows : 128);
     if (slices < 1) slices = 1;
-    kslice = ((mp + slices - 1) / slices + KD - 1) / KD * KD;
+    kslice = ((mp + slices - 1) / slices + deep - 1) / deep * deep;
     slices = (mp + kslice - 1) / kslice;
   }
 };
+
+// Rows to a Gram tile for one tile to a compute unit (32 x 32 tiles: four): the fp64 matrix cores bound the launch, whose time is that of
+// the unit with the most; and every K slice is a slab that the factorisation adds up.
+inline int gram_rows(const DaDionSmallGroup* g, int n, bool bf) {
+  long long rows = 0;
+  for (int i = 0; i < n; ++i) rows += (long long)g[i].cnt * gram_tiles(g[i].r, bf) * (g[i].m > g[i].n ? g[i].m : g[i].n);
+  const long long per = rows / (bf ? 256 : 1024);
+  return per < 1 ? 1 : per > (1 << 30) ? 1 << 30 : (int)per;
+}
 
 inline int mchunks(int m, int n) { return (int)(((long long)m * n + ADD_ELEMS - 1) / ADD_ELEMS); }
 
@@ -621,7 +656,7 @@ size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, 
 }
 
 // control memory: words of all matrices, the queues' lines, the status word's line, the pointer tables
-size_t control_bytes(int mats) { return up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4) + up256((size_t)4 * mats * 8); }
+size_t control_bytes(int mats) { return up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4) + up256((size_t)3 * mats * 8); }
 
 // Matrices to queues: the costliest first, each to the queue with the least to do so far.  (Dealt in the order of the buckets, 14
 // matrices of 1021, 341 and 2731 rows / columns left two XCDs with a tenth of the others' work: 730 us, so 670.)  Returns the
@@ -651,6 +686,33 @@ double deal(const DaDionSmallGroup* g, int n, bool bf, unsigned char* queue) {
   return worst;
 }
 
+template <bool BF>
+int launch_all(const Args& a, hipStream_t s) {
+  static DaOncePerDevice configured;
+  int rc = configured.run([&]() -> int {
+    const void* const wide[] = {reinterpret_cast<const void*>(dion_small_chain_kernel), reinterpret_cast<const void*>(dion_small_orth_kernel<FIXP, BF>)};
+    for (const void* f : wide) DA_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
+    return DA_OK;
+  });
+  auto launch = [&](void (*kernel)(Args), Kind kind, int smem) {
+    long long n = kind == CHAIN ? 2 * da_cu_count() : 0;
+    for (int i = 0; kind != CHAIN && i < a.ngroups; ++i) n += (long long)a.g[i].cnt * tiles_of(a.g[i], kind, BF);
+    if (rc) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(256), smem, s, a);
+    rc = da_launch_status();
+  };
+  launch(dion_small_product_kernel<BF, true>, BQ, SMEM_TILE);
+  launch(dion_small_gram_kernel<BF>, GRAM, SMEM_TILE);
+  launch(dion_small_chain_kernel, CHAIN, SMEM);
+  launch(dion_small_orth_kernel<PT, BF>, PT, SMEM_TILE);
+  launch(dion_small_orth_kernel<FIXG, BF>, FIXG, SMEM_TILE);
+  launch(dion_small_orth_kernel<FIXP, BF>, FIXP, SMEM);
+  launch(dion_small_product_kernel<BF, false>, BTP, SMEM_TILE);
+  launch(dion_small_cnorm_kernel<BF>, CNORM, 0);
+  launch(dion_small_update_kernel<BF>, UPD, SMEM_UPDATE);
+  return rc;
+}
+
 }  // namespace
 
 size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, bool forced) {
@@ -664,6 +726,7 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
   // two d x 4d: bf16 d 128 r 64: 95 / 400;  256 x4 r 128: 204 / 464;  512 x8 r 32: 366 / 528;  512 x8 r 128: 502 / 534;
   // 768 x4 r 192: 703 / 506.  fp32 256 x4 r 128: 272 / 559;  768 x4 r 48: 643 / 948;  768 x12 r 192: 3121 / 2259.
   const bool bf = c.m_dtype == DA_BF16;
+  const int rows = gram_rows(g, n, bf);
   double chain = 0.0, other = 0.0;
   bool padded = false, odd_full = false;
   for (int i = 0; i < n; ++i) {
@@ -682,7 +745,7 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
     odd_full |= g[i].r == S.np && (g[i].r & 7) != 0;
     padded |= ((g[i].m | g[i].n) & 7) != 0;
     mats += g[i].cnt;
-    bytes += lay_out(nullptr, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
+    bytes += lay_out(nullptr, g[i], Shape(g[i].m, g[i].n, g[i].r, bf, rows), c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
   }
   if (mats > DA_DS_MATS) return 0;
   const double worst = deal(g, n, bf, nullptr);
@@ -712,17 +775,18 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   unsigned char queue[DA_DS_MATS];
   deal(g, n, c.m_dtype == DA_BF16, queue);
   int first = 0, at = 0;
-  long long adds = 0, tiles = 0;
+  long long adds = 0;
+  const int rows = gram_rows(g, n, bf);
   for (int i = 0; i < n; ++i) {
-    const Shape S(g[i].m, g[i].n, g[i].r, bf);
+    const Shape S(g[i].m, g[i].n, g[i].r, bf, rows);
     GroupDev& D = a.g[i];
     p += lay_out(&D, g[i], S, c.m_dtype == DA_BF16 ? 2 : 4, p);
-    D.X = su.dst + first; D.G = su.dst + mats + first; D.M = su.dst + 2 * mats + first; D.Q = su.dst + 3 * mats + first;
+    D.X = su.dst + first; D.M = su.dst + mats + first; D.Q = su.dst + 2 * mats + first;
     for (int j = 0; j < g[i].cnt; ++j) {
       su.p[0][first + j] = g[i].X[j];
-      su.p[1][first + j] = const_cast<void*>(g[i].G[j]);
-      su.p[2][first + j] = g[i].M[j];
-      su.p[3][first + j] = g[i].Q[j];
+      su.p[1][first + j] = g[i].M[j];
+      su.p[2][first + j] = g[i].Q[j];
+      su.p[3][first + j] = const_cast<void*>(g[i].G[j]);
     }
     D.words = words + (size_t)first * CTR_STRIDE;
     D.info = g[i].info;
@@ -743,35 +807,21 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
     U.end = (int)(adds += (long long)g[i].cnt * U.per);
     U.m = g[i].m; U.n = g[i].n; U.r = g[i].r; U.rp = S.rp; U.np = S.np; U.npR = S.npT * 64;
     U.Qw = D.Qw; U.any = D.any;
-    tiles += (long long)g[i].cnt * S.mpT * S.npT;
     first += g[i].cnt;
   }
   a.ngroups = n;
   for (int q = 0; q < DA_QUEUES; ++q)
     for (int i = 0; i < n; ++i)
-      for (int k = 0; k < KINDS; ++k) a.total[q] += a.g[i].nq[q] * tasks_of(a.g[i], k, c.m_dtype == DA_BF16);
+      for (int k = 0; k < PHASES; ++k) a.total[q] += a.g[i].nq[q] * tasks_of(a.g[i], k);
   a.spin_limit = 200000000ull;   // 2 s of the 100 MHz counter
-  a.x_f32 = c.x_dtype == DA_F32; a.g_f32 = c.g_dtype == DA_F32; a.q_f32 = c.q_dtype == DA_F32;
+  a.x_f32 = c.x_dtype == DA_F32; a.q_f32 = c.q_dtype == DA_F32;
   a.ef_alpha = c.ef_alpha; a.decay = c.decay; a.eps = c.eps;
   su.zblocks = (su.nzero + 255) / 256;
   su.ngroups = n; su.g_f32 = c.g_dtype == DA_F32; su.q_f32 = c.q_dtype == DA_F32;
-  static DaOncePerDevice configured;
-  int rc = configured.run([&]() -> int {
-    DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
-    DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(dion_small_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM));
-    return DA_OK;
-  });
-  if (rc) return rc;
-  const dim3 setup((unsigned)(su.zblocks + adds)), grid(2 * (unsigned)da_cu_count()), update((unsigned)tiles), block(256);
+  const dim3 block(256), setup((unsigned)(su.zblocks + adds));
   if (bf) hipLaunchKernelGGL(dion_small_setup_kernel<true>, setup, block, 0, s, su);
   else hipLaunchKernelGGL(dion_small_setup_kernel<false>, setup, block, 0, s, su);
-  rc = da_launch_status();
+  const int rc = da_launch_status();
   if (rc) return rc;
-  if (bf) hipLaunchKernelGGL(dion_small_kernel<true>, grid, block, SMEM, s, a);
-  else hipLaunchKernelGGL(dion_small_kernel<false>, grid, block, SMEM, s, a);
-  rc = da_launch_status();
-  if (rc) return rc;
-  if (bf) hipLaunchKernelGGL(dion_small_update_kernel<true>, update, block, SMEM_UPDATE, s, a);
-  else hipLaunchKernelGGL(dion_small_update_kernel<false>, update, block, SMEM_UPDATE, s, a);
-  return da_launch_status();
+  return bf ? launch_all<true>(a, s) : launch_all<false>(a, s);
 }

@@ -1,4 +1,4 @@
-// Ticket queues of the one-launch kernels for small matrices (ns_small.hip, dion_small.hip): eight queues, one per XCD.
+// Ticket queues of the kernels for small matrices that run a chain of phases (ns_small.hip, dion_small.hip): eight queues, one per XCD.
 #pragma once
 #include "common.h"
 

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
         }
         if (tid == 0) next = request_ticket(word);
         if (pt) {
-          for (int e = tid; e < 4096; e += 256) S[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = d[(e >> 6) * 66 + (e & 63)];
+          for (int e = tid; e < 4096; e += 256) S[(long long)(row0 + (e >> 6)) * rp + col0 + (e & 63)] = row0 + (e >> 6) < a.rows ? d[(e >> 6) * 66 + (e & 63)] : 0.0;
         } else {
           const bool poisoned = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
           char* const out = a.out + b * ((long long)a.rows * a.r) * (long long)sizeof(E);
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
           }
         }
       } else {
-        const Factor F = {a.w.slab + b * a.slices * rr, a.w.L + b * rr, a.w.T + b * rr, a.slices, a.r_live, rp, rT,
+        const Factor F = {a.w.slab + b * a.slices * rr, a.w.L + b * rr, a.w.T + b * rr, nullptr, a.slices, a.r_live, rp, rT,
                           words + W_BAD, words + W_SICK, a.info + b, reinterpret_cast<double*>(words + W_RANGE), 0.0};
         factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn);
         if (tid == 0) next = request_ticket(word);

@@ -28,6 +28,10 @@ template <typename E> __device__ __forceinline__ Opnd<E, false> work(const void*
   return Opnd<E, false>{static_cast<const E*>(p), ld, ks, 0, 0, 0};
 }
 
+// Pointers read from a table point to the compiler knows not what: a generic (flat) load counts as an LDS access as well, and every
+// wait for an LDS read waits for it too.  These are global memory.
+#define DA_GLOBAL __attribute__((address_space(1)))
+
 // Eight consecutive elements as they came from memory: converted only when they go to LDS, so that the loads of the next
 // stages stay in flight.
 template <typename E> struct Raw { u32x4_t q[sizeof(E) / 2]; };
@@ -35,7 +39,7 @@ template <typename E> __device__ __forceinline__ Raw<E> load_raw(const E* p) {
   Raw<E> r;
 #pragma unroll
   for (int i = 0; i < (int)(sizeof(E) / 2); ++i) {
-    const u32x4_un_t x = *reinterpret_cast<const u32x4_un_t*>(reinterpret_cast<const char*>(p) + 16 * i);
+    const u32x4_un_t x = *(const DA_GLOBAL u32x4_un_t*)(reinterpret_cast<const char*>(p) + 16 * i);
     r.q[i] = x;
   }
   return r;
@@ -74,7 +78,7 @@ template <typename E> __device__ __forceinline__ void load8(const E* p, long lon
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      if (i < n) v[i] = to_f(p[e + i]);
+      if (i < n) v[i] = to_f(*(const DA_GLOBAL E*)(p + e + i));
   }
 }
 
@@ -109,8 +113,8 @@ __device__ __forceinline__ void mask_chunk(const Opnd<E, true>& o, Raw<E>& r, in
 #pragma unroll
     for (int i = 0; i < 8 / W; ++i) {
       unsigned w = 0;
-      if (i * W < n) w = sizeof(E) == 4 ? reinterpret_cast<const unsigned*>(o.p + e)[i] : (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i];
-      if (sizeof(E) == 2 && i * W + 1 < n) w |= (unsigned)reinterpret_cast<const unsigned short*>(o.p + e)[2 * i + 1] << 16;
+      if (i * W < n) w = sizeof(E) == 4 ? ((const DA_GLOBAL unsigned*)(o.p + e))[i] : (unsigned)((const DA_GLOBAL unsigned short*)(o.p + e))[2 * i];
+      if (sizeof(E) == 2 && i * W + 1 < n) w |= (unsigned)((const DA_GLOBAL unsigned short*)(o.p + e))[2 * i + 1] << 16;
       r.q[i >> 2][i & 3] = w;
     }
   } else {
@@ -133,11 +137,11 @@ struct Real {
 struct NoTurn {
   template <typename V> __device__ __forceinline__ void operator()(V&, int, int) const {}
 };
-template <typename T, int TB, typename E, bool EDGE, typename Turn>
+template <typename T, int TB, bool MASK, typename E, bool EDGE, typename Turn>
 __device__ __forceinline__ void put_chunk(T* dst, const Opnd<E, EDGE>& o, Raw<E>& r, int c, int row0, int k0, Turn turn) {
   constexpr int P = Real<T, TB>::P;
   T v[8];
-  if constexpr (EDGE) mask_chunk<TB, KD>(o, r, c, row0, k0);
+  if constexpr (EDGE && MASK) mask_chunk<TB, KD>(o, r, c, row0, k0);
   unpack(r, v);
   int row, k;
   chunk_at<TB, KD>(o.ks, c, row, k);
@@ -151,10 +155,71 @@ __device__ __forceinline__ void put_chunk(T* dst, const Opnd<E, EDGE>& o, Raw<E>
   }
 }
 
+// The stages 0 .. n - 1 of a K loop through registers and two LDS buffers: `fetch(set, i)` requests stage i, `put(set, i, buffer,
+// mask)` writes it to LDS, `acc(buffer)` multiplies.  With two register sets (AHEAD) two stages are on the way from memory while a
+// third is multiplied.  The leading `full` stages need no mask, and the loop over them has no branch: where a fetch or a masked
+// write is conditional the paths meet with an unknown number of loads on the way, and the compiler waits for all of them, so that every
+// stage took a whole trip to memory (14 matrices of 341 to 2731 rows: P = B Q 36 -> 31 us, R = B^T P 52 -> 41).  Past the end the last
+// stage is fetched again.
+struct Masked { static constexpr bool value = true; };
+struct Unmasked { static constexpr bool value = false; };
+template <int AHEAD, typename Fetch, typename Put, typename Acc>
+__device__ __forceinline__ void staged_loop(int n, int full, Fetch fetch, Put put, Acc acc) {
+  const int last = n - 1;
+  int i = 0;
+  fetch(0, 0);
+  if (AHEAD == 2) fetch(1, min(1, last));
+  if (full > 0) put(0, 0, 0, Unmasked());
+  else put(0, 0, 0, Masked());
+  if (AHEAD == 2) {
+    for (; i + 3 <= full; i += 2) {
+      fetch(0, min(i + 2, last));
+      __syncthreads();
+      acc(0);
+      put(1, i + 1, 1, Unmasked());
+      fetch(1, min(i + 3, last));
+      __syncthreads();
+      acc(1);
+      put(0, i + 2, 0, Unmasked());
+    }
+  } else {
+    for (; i + 3 <= full; i += 2) {
+      fetch(0, i + 1);
+      __syncthreads();
+      acc(0);
+      put(0, i + 1, 1, Unmasked());
+      fetch(0, i + 2);
+      __syncthreads();
+      acc(1);
+      put(0, i + 2, 0, Unmasked());
+    }
+  }
+  for (; i < n; i += 2) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = i + s;
+      if (k >= n) break;
+      if (k + AHEAD < n) fetch(AHEAD == 2 ? s : 0, k + AHEAD);
+      __syncthreads();
+      acc(s);
+      if (k + 1 < n) {
+        if (k + 1 < full) put(AHEAD == 2 ? s ^ 1 : 0, k + 1, s ^ 1, Unmasked());
+        else put(AHEAD == 2 ? s ^ 1 : 0, k + 1, s ^ 1, Masked());
+      }
+    }
+  }
+  __syncthreads();
+}
+// how many of n stages, D deep from kbeg on, no chunk of which reaches past the operand's k (of a caller's matrix never the last one,
+// where a load may have been moved back; rows past its end are read as whatever lies there, and the caller drops their results)
+template <typename E> __device__ __forceinline__ int full_stages(const Opnd<E, false>&, int, int n, int) { return n; }
+template <typename E> __device__ __forceinline__ int full_stages(const Opnd<E, true>& o, int kbeg, int n, int D) {
+  return max(0, min(n - 1, (o.kmax - kbeg) / D));
+}
+
 // K loop of one TB x TB tile:  sum over k in [kbeg, kend) of A(row0 + i, k) B(col0 + j, k), for NB column operands; `mma`
 // accumulates one stage of KD from the operands' LDS buffers (A first); `turn(v, col, k)` maps the chunk (col, k ..) of a column
-// operand on its way to LDS.  Two stages are on the way from memory while a third
-// is multiplied; of fp64 64-tiles one (its products take 1.7 us and two stages too many registers).
+// operand on its way to LDS.  Of fp64 64-tiles one stage is on the way (two take too many registers).
 template <typename T, int TB, int NB, typename OA, typename OB, typename Mma, typename Turn>
 __device__ __forceinline__ void real_loop(const OA& A, const OB (&B)[NB], int row0, int col0, int kbeg, int kend, T* lds, int tid,
                                           Mma mma, Turn turn) {
@@ -162,36 +227,25 @@ __device__ __forceinline__ void real_loop(const OA& A, const OB (&B)[NB], int ro
   constexpr int STG = (1 + NB) * L::OPND;
   const int c = tid & (L::NCH - 1);
   const bool own = tid < L::NCH;
+  const int n = (kend - kbeg + KD - 1) / KD;
   decltype(fetch_chunk<TB, KD>(A, c, row0, kbeg)) va[2];
   decltype(fetch_chunk<TB, KD>(B[0], c, col0, kbeg)) vb[2][NB];
-  auto fetch = [&](int s, int k0) {
+  staged_loop<sizeof(T) == 8 && TB == 64 ? 1 : 2>(n, min(full_stages(A, kbeg, n, KD), full_stages(B[0], kbeg, n, KD)),
+      [&](int s, int i) {
+    const int k0 = kbeg + i * KD;
     va[s] = fetch_chunk<TB, KD>(A, c, row0, k0);
 #pragma unroll
     for (int o = 0; o < NB; ++o) vb[s][o] = fetch_chunk<TB, KD>(B[o], c, col0, k0);
-  };
-  auto put = [&](int s, int k0) {
+  },
+      [&](int s, int i, int buf, auto mask) {
+    const int k0 = kbeg + i * KD;
     if (own) {
-      put_chunk<T, TB>(lds + s * STG, A, va[s], c, row0, k0, NoTurn());
+      put_chunk<T, TB, decltype(mask)::value>(lds + buf * STG, A, va[s], c, row0, k0, NoTurn());
 #pragma unroll
-      for (int o = 0; o < NB; ++o) put_chunk<T, TB>(lds + s * STG + (1 + o) * L::OPND, B[o], vb[s][o], c, col0, k0, turn);
+      for (int o = 0; o < NB; ++o) put_chunk<T, TB, decltype(mask)::value>(lds + buf * STG + (1 + o) * L::OPND, B[o], vb[s][o], c, col0, k0, turn);
     }
-  };
-  constexpr int AHEAD = sizeof(T) == 8 && TB == 64 ? 1 : 2;
-  fetch(0, kbeg);
-  if (AHEAD == 2 && kbeg + KD < kend) fetch(1, kbeg + KD);
-  put(0, kbeg);
-  for (int k0 = kbeg; k0 < kend; k0 += 2 * KD) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int k = k0 + s * KD;
-      if (k >= kend) break;
-      if (k + AHEAD * KD < kend) fetch(AHEAD == 2 ? s : s ^ 1, k + AHEAD * KD);
-      __syncthreads();
-      mma(lds + s * STG);
-      if (k + KD < kend) put(s ^ 1, k + KD);
-    }
-  }
-  __syncthreads();
+  },
+      [&](int buf) { mma(lds + buf * STG); });
 }
 
 // fp64 (and fp32 in 32-tiles): v_mfma_*_16x16x4, four wavefronts of TB/2 x TB/2
@@ -243,6 +297,68 @@ __device__ __forceinline__ void tile16(const OA& A, const OB& B, int row0, int c
   acc.out(lds, lane, wm, wn);
 }
 
+// A 64 x 64 fp64 tile of two working matrices without LDS stages: every wavefront loads the operands of its 32 x 32 block as the
+// fragments that the instruction takes, a 32-deep step ahead of the products and with no barrier between steps.  Lane l holds
+// eight consecutive k of row (or column) l % 16, from 8 (l / 16) on, and the sum over k runs over them in parallel:
+// k = 8 (l / 16) + s in the s-th product.  fp64 operands are k-strided (KS): 16 lanes of a load read 128 consecutive bytes; with k
+// consecutive every lane reads a line of its own, and the L1's look-ups take longer than the products.
+template <typename E, bool KS> struct DirectFrag {
+  Raw<E> r;
+  __device__ __forceinline__ void load(const E* p, int ld, int lane) { r = load_raw(p + (long long)(lane & 15) * ld + (lane >> 4) * 8); }
+  __device__ __forceinline__ void get(double (&v)[8]) const { unpack(r, v); }
+};
+template <> struct DirectFrag<double, true> {   // (k-strided)
+  double r[8];
+  __device__ __forceinline__ void load(const double* p, int ld, int lane) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = p[(long long)((lane >> 4) * 8 + i) * ld + (lane & 15)];
+  }
+  __device__ __forceinline__ void get(double (&v)[8]) const {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = r[i];
+  }
+};
+// A (the tile's first row and k = 0 at A) times B (k-strided, the tile's first column and k = 0 at B) over k < kend (a multiple of
+// 64), to the staging area as tile16 leaves it.
+template <bool KSA, typename E>
+__device__ __forceinline__ void direct64(const E* A, int lda, const double* B, int ldb, int kend, double* d, int lane, int wm, int wn) {
+  Acc16<double, 64> acc;
+  acc.clear();
+  DirectFrag<E, KSA> fa[2][2];
+  DirectFrag<double, true> fb[2][2];
+  A += wm * 32LL * (KSA ? 1 : lda);
+  B += wn * 32;
+  auto fetch = [&](int s, int k0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fa[s][i].load(KSA ? A + (long long)k0 * lda + i * 16 : A + (long long)i * 16 * lda + k0, lda, lane);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) fb[s][j].load(B + (long long)k0 * ldb + j * 16, ldb, lane);
+    __builtin_amdgcn_sched_barrier(0);   // (here, and not behind the products)
+  };
+  auto products = [&](int s) {
+    double a[2][8], b[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fa[s][i].get(a[i]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) fb[s][j].get(b[j]);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc.acc[i][j] = Mfma<double>::mma(a[i][u], b[j][u], acc.acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  fetch(0, 0);
+  for (int k = 0; k < kend; k += 64) {   // (the last step is fetched twice: no load in a branch, as in staged_loop)
+    fetch(1, k + 32);
+    products(0);
+    fetch(0, min(k + 64, kend - 32));
+    products(1);
+  }
+  acc.out(d, lane, wm, wn);
+}
+
 // fp32, 64-tiles: one v_mfma_f32_32x32x2 block per wavefront (the order of k of gemm_f32.hip); element e of `acc` is row
 // (lane & 31), column 8 (e / 4) + 4 (lane / 32) + e % 4 of the wavefront's block.  NB column operands share the row operand.
 template <int NB, typename OA, typename OB>
@@ -272,9 +388,9 @@ __device__ __forceinline__ void stage_f32(const f32x16_t& acc, float* stg, int l
 
 // ---- products of bf16 tiles: the LDS layouts of gemm_bf16_tile.h, 64-deep stages through registers -----------------------
 // `acc` is called with every stage: the buffers of the row operand and of NB column operands, 8 KB each.
-template <int TB, int D, bool EDGE>
+template <int TB, int D, bool MASK, bool EDGE>
 __device__ __forceinline__ void put_bf16(char* dst, const Opnd<bf16_t, EDGE>& o, Raw<bf16_t>& r, int c, int row0, int k0) {
-  if constexpr (EDGE) mask_chunk<TB, D>(o, r, c, row0, k0);
+  if constexpr (EDGE && MASK) mask_chunk<TB, D>(o, r, c, row0, k0);
   const int q = c >> 3, ch = c & 7;   // (row or k, chunk): 8 chunks of a line either way
   *reinterpret_cast<u32x4_t*>(dst + q * 128 + (o.ks ? ks_swizzle(ch, q) : kc_swizzle(ch, q)) * 16) = r.q[0];
 }
@@ -283,38 +399,27 @@ __device__ __forceinline__ void tile_bf16(const Opnd<bf16_t, EDGE>& A, const Opn
                                           char* lds, int tid, Acc acc) {
   constexpr int OPND = 64 * 64 * 2;
   constexpr int STG = (1 + NB) * OPND;
-  Raw<bf16_t> v[2][1 + NB][2];   // two stages on the way while a third is multiplied
-  auto fetch = [&](int s2, int k0) {
+  const int n = (kend + 63) / 64;
+  Raw<bf16_t> v[2][1 + NB][2];
+  staged_loop<2>(n, full_stages(A, 0, n, 64),
+      [&](int s, int i) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      v[s2][0][h] = fetch_chunk<64, 64>(A, tid + 256 * h, row0, k0);
+      v[s][0][h] = fetch_chunk<64, 64>(A, tid + 256 * h, row0, i * 64);
 #pragma unroll
-      for (int o = 0; o < NB; ++o) v[s2][1 + o][h] = fetch_chunk<64, 64>(B[o], tid + 256 * h, col0, k0);
+      for (int o = 0; o < NB; ++o) v[s][1 + o][h] = fetch_chunk<64, 64>(B[o], tid + 256 * h, col0, i * 64);
     }
-  };
-  auto put = [&](int s2, int k0) {
+  },
+      [&](int s, int i, int buf, auto mask) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      put_bf16<64, 64>(lds + s2 * STG, A, v[s2][0][h], tid + 256 * h, row0, k0);
+      put_bf16<64, 64, decltype(mask)::value>(lds + buf * STG, A, v[s][0][h], tid + 256 * h, row0, i * 64);
 #pragma unroll
-      for (int o = 0; o < NB; ++o) put_bf16<64, 64>(lds + s2 * STG + (1 + o) * OPND, B[o], v[s2][1 + o][h], tid + 256 * h, col0, k0);
+      for (int o = 0; o < NB; ++o)
+        put_bf16<64, 64, false>(lds + buf * STG + (1 + o) * OPND, B[o], v[s][1 + o][h], tid + 256 * h, col0, i * 64);
     }
-  };
-  fetch(0, 0);
-  if (64 < kend) fetch(1, 64);
-  put(0, 0);
-  for (int k0 = 0; k0 < kend; k0 += 128) {
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const int k = k0 + s2 * 64;
-      if (k >= kend) break;
-      if (k + 128 < kend) fetch(s2, k + 128);
-      __syncthreads();
-      acc(lds + s2 * STG);
-      if (k + 64 < kend) put(s2 ^ 1, k + 64);
-    }
-  }
-  __syncthreads();
+  },
+      [&](int buf) { acc(lds + buf * STG); });
 }
 // P and R: v_mfma_f32_16x16x32_bf16, four 16 x 16 blocks per wavefront, to the staging area (pitch 66)
 template <bool EDGE>
@@ -349,6 +454,34 @@ __device__ __forceinline__ void product_bf16(const Opnd<bf16_t, EDGE>& A, const 
       for (int v = 0; v < 4; ++v)
         stg[(wm * 32 + i * 16 + (lane & 15)) * 66 + wn * 32 + j * 16 + (lane >> 4) * 4 + v] = acc[i][j][v];
 }
+// A 64 x 64 tile of P^T P in fp64 over k < kend rows of a bf16 working matrix (at the tiles' first rows), to the staging area as
+// tile16 leaves it.  The stages stay bf16 in the LDS, a fragment's elements become fp64 on their way into the products (as fp64 the
+// LDS would carry four times the bytes, and 32 x 32 tiles twice that).  Lane l's eight k of a fragment are 8 (l / 16) on.
+__device__ __forceinline__ void gram64_bf16(const bf16_t* P, int rp, int row0, int col0, int kend, char* lds, int tid, int lane, int wm,
+                                            int wn) {
+  Acc16<double, 64> acc;
+  acc.clear();
+  const Opnd<bf16_t, false> o = work<bf16_t>(P, rp, 1), Bs[1] = {o};
+  tile_bf16<1>(o, Bs, row0, col0, kend, lds, tid, [&](const char* st) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      double a[2][8], b[2][8];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x8_t fa = read_frag16<64, true>(st, wm * 32 + i * 16, ks, lane), fb = read_frag16<64, true>(st + 8192, wn * 32 + i * 16, ks, lane);
+        unpack(Raw<bf16_t>{{__builtin_bit_cast(u32x4_t, fa)}}, a[i]);
+        unpack(Raw<bf16_t>{{__builtin_bit_cast(u32x4_t, fb)}}, b[i]);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc.acc[i][j] = Mfma<double>::mma(a[i][u], b[j][u], acc.acc[i][j]);
+    }
+  });
+  acc.out(reinterpret_cast<double*>(lds), lane, wm, wn);
+}
 // the updates: v_mfma_f32_32x32x16_bf16 as in the batched update kernel, both products at once
 __device__ __forceinline__ void update_bf16(const Opnd<bf16_t, false>& A, const Opnd<bf16_t, false> (&B)[2], int row0, int col0,
                                             int kend, char* lds, int tid, int lane, int wm, int wn, f32x16_t (&acc)[2]) {
@@ -373,7 +506,7 @@ __device__ __forceinline__ void update_bf16(const Opnd<bf16_t, false>& A, const 
 __device__ __forceinline__ void store8(char* p, int f32, long long e, int n, const float (&v)[8]) {
   if (n <= 0) return;
   if (f32) {
-    float* q = reinterpret_cast<float*>(p) + e;
+    DA_GLOBAL float* const q = (DA_GLOBAL float*)p + e;
     if (n >= 8) {
       u32x4_un_t x, y;
 #pragma unroll
@@ -381,20 +514,20 @@ __device__ __forceinline__ void store8(char* p, int f32, long long e, int n, con
         x[i] = __builtin_bit_cast(unsigned, v[i]);
         y[i] = __builtin_bit_cast(unsigned, v[4 + i]);
       }
-      *reinterpret_cast<u32x4_un_t*>(q) = x;
-      *reinterpret_cast<u32x4_un_t*>(q + 4) = y;
+      *(DA_GLOBAL u32x4_un_t*)q = x;
+      *(DA_GLOBAL u32x4_un_t*)(q + 4) = y;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         if (i < n) q[i] = v[i];
     }
   } else {
-    bf16_t* q = reinterpret_cast<bf16_t*>(p) + e;
+    DA_GLOBAL bf16_t* const q = (DA_GLOBAL bf16_t*)p + e;
     if (n >= 8) {
       u32x4_un_t x;
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[i] = cvt_pk_bf16(v[2 * i], v[2 * i + 1]);
-      *reinterpret_cast<u32x4_un_t*>(q) = x;
+      *(DA_GLOBAL u32x4_un_t*)q = x;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
@@ -418,7 +551,7 @@ __device__ __forceinline__ float guard(float x, bool nonzero, float alt) {
 // P^T P comes as lower 32 x 32 tiles in K slices (slab: [slices][rp][rp], rp = 64 rT); columns r .. rp - 1 are the identity.
 struct Factor {
   const double* slab;
-  double *L, *T;               // rp x rp; of L the blocks below the diagonal, of T those on and below it
+  double *LT, *T, *TT;         // rp x rp; the blocks of L^T above the diagonal, of T on and below it, of T^T (if wanted, or null)
   int slices, r, rp, rT;
   int *bad, *sick, *info;      // first failed pivot (column + 1); outcome: pivot range below `ratio` or a failed pivot; info may be null
   double* range;               // smallest and largest pivot so far
@@ -431,18 +564,18 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
   typedef Real<double, 64> RD;
   enum Job { J_DIAG, J_LOW, J_INV };
   double* const d = reinterpret_cast<double*>(lds);
-  double *const L = F.L, *const T = F.T;
+  double *const LT = F.LT, *const T = F.T;
   const int rp = F.rp, rT = F.rT;
   const long long rr = (long long)rp * rp;
   const Job job = diag ? J_DIAG : task < rT - 1 - j ? J_LOW : J_INV;
   const int x = diag ? j : job == J_LOW ? j + 1 + task : task - (rT - 1 - j);
   const int kend = wave_uniform((job == J_INV ? j - x : j) * 64);
   // J_INV: sum over k of L(j, k) T(k, x), x <= k < j;  else: sum over k < j of L(x, k) L(j, k)^T
-  const Opnd<double, false> sa = work<double>(job == J_INV ? L + (long long)j * 64 * rp + x * 64 : L + (long long)x * 64 * rp, rp, 0);
-  const Opnd<double, false> sb = job == J_INV ? work<double>(T + (long long)x * 64 * rp + x * 64, rp, 1)
-                                              : work<double>(L + (long long)j * 64 * rp, rp, 0);
   const Opnd<double, false> sd = work<double>(T + (long long)j * 64 * rp + j * 64, rp, 0);   // D, the inverse of the diagonal block's factor
-  if (kend > 0) tile16<double, 64>(sa, sb, 0, 0, 0, kend, d, tid, lane, wm, wn);
+  if (kend > 0) {
+    if (job == J_INV) direct64<true>(LT + (long long)x * 64 * rp + j * 64, rp, T + (long long)x * 64 * rp + x * 64, rp, kend, d, lane, wm, wn);
+    else direct64<true>(LT + x * 64, rp, LT + j * 64, rp, kend, d, lane, wm, wn);
+  }
   double2_t w[8];        // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
   const int k = (tid & 31) * 2, i0 = tid >> 5;
 #pragma unroll
@@ -450,12 +583,20 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
   if (job != J_INV) {
     // the slabs of P^T P in slice order; beyond the rank the matrix is the identity
     const double* const slab = F.slab + (long long)(x * 64 + i0) * rp + j * 64 + k;
-    for (int s = 0; s < F.slices; ++s) {
-      double2_t y[8];
+    for (int s0 = 0; s0 < F.slices; s0 += 4) {   // four slabs on the way at a time
+      double2_t y[4][8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) y[u] = *reinterpret_cast<const double2_t*>(slab + s * rr + (long long)u * 8 * rp);
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < F.slices) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] += y[u];
+          for (int u = 0; u < 8; ++u) y[s][u] = *reinterpret_cast<const double2_t*>(slab + (s0 + s) * rr + (long long)u * 8 * rp);
+        }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (s0 + s < F.slices) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) w[u] += y[s][u];
+        }
     }
     const int lim = ((F.r + 31) >> 5) << 5;
 #pragma unroll
@@ -513,6 +654,10 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
     });
     double* const Dw = T + (long long)j * 64 * rp + j * 64;
     for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * DIAG_P + (e >> 6)];
+    if (F.TT) {
+      double* const Dt = F.TT + (long long)j * 64 * rp + j * 64;
+      for (int e = tid; e < 4096; e += 256) Dt[(long long)(e >> 6) * rp + (e & 63)] = dT[(e >> 6) * DIAG_P + (e & 63)];
+    }
     return;
   }
   // second product, both operands to the LDS stages:  L(x, j) = W(x, j) D^T;   T(j, x) = -D W(j, x)
@@ -533,8 +678,8 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
       wst[(k >> 5) * 2 * RD::OPND + ((k + 1) & 31) * RD::P + i] = w[u][1];
     }
   }
-  put_chunk<double, 64>(dst, sd, dr[0], tid, 0, 0, NoTurn());
-  put_chunk<double, 64>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
+  put_chunk<double, 64, false>(dst, sd, dr[0], tid, 0, 0, NoTurn());
+  put_chunk<double, 64, false>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
   __syncthreads();
   Acc16<double, 64> acc;
   acc.clear();
@@ -542,9 +687,15 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
   acc.stage(d + 2 * RD::OPND, d + 3 * RD::OPND, lane, wm, wn);
   __syncthreads();
   acc.out(d, lane, wm, wn);
-  double* const out = job == J_INV ? T + (long long)j * 64 * rp + x * 64 : L + (long long)x * 64 * rp + j * 64;
-  const double sign = job == J_INV ? -1.0 : 1.0;
-  for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e >> 6) * 66 + (e & 63)];
+  if (job == J_INV) {
+    double* const out = T + (long long)j * 64 * rp + x * 64;
+    for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = -d[(e >> 6) * 66 + (e & 63)];
+  }
+  double* const turned = job == J_LOW ? LT + (long long)j * 64 * rp + x * 64 : F.TT ? F.TT + (long long)x * 64 * rp + j * 64 : nullptr;
+  if (turned) {
+    const double sign = job == J_INV ? -1.0 : 1.0;
+    for (int e = tid; e < 4096; e += 256) turned[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e & 63) * 66 + (e >> 6)];
+  }
 }
 
 // One lower 32 x 32 tile (number t of t32 (t32 + 1) / 2) of S^T S over rows [kbeg, kend) of S, into out (pitch rp) and d (pitch 34)

@@ -223,3 +223,14 @@ def test_dion_weights_off_the_128_byte_grid(dev, option, shape, shift):
         option("dion_small", 1)
     for a, b in zip(*runs):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("ms", [(127, 128, 129, 200), (191, 192, 193, 264), (255, 256, 257, 264), (319, 320, 321, 449)])
+def test_numbers_of_stages_and_ragged_ends(dev, option, dtype, ms):
+    """K loops of two to eight stages whose last one is whole, one element deep or ragged, B by rows and by columns."""
+    shapes, runs = [(m, 72) for m in ms] + [(77, m) for m in ms], []
+    for mode in (0, 1):
+        option("dion_small", mode)
+        runs.append(_run(dev, shapes, dtype, 0.5, 1, 2)[0])
+    _agree(shapes, runs, 2e-5 if dtype == F32 else 1e-2)   # (as above)
