@@ -51,25 +51,27 @@ struct GemmArgs {
 
 // Which output tile a workgroup owns.  Workgroups are dealt round-robin to the 8 XCDs (each
 // with its own L2), so consecutive *logical* tiles -- which share an operand panel -- are
-// mapped to the same XCD when the grid divides evenly.
+// mapped to the same XCD.
 struct TileId { int b, ti, tj; };
 
 template <int BT, bool SYM>
-__device__ __forceinline__ TileId decode_tile(const GemmDesc& d, int bid, int nblk, bool xcd_aligned, int interleave) {
+__device__ __forceinline__ TileId decode_tile(const GemmDesc& d, int bid, int nblk, int interleave) {
   const int tiles_m = (d.M + BT - 1) / BT;
   const int tiles_n = (d.N + BT - 1) / BT;
   const int per_batch = SYM ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
-  if (xcd_aligned && (nblk & 7) == 0) {
+  {
     // `interleave`: the XCDs take turns at runs of G logical tiles (a super-tile; an eighth of a symmetric matrix), so
     // that all eight work on the same matrix at the same time; otherwise each XCD owns a contiguous eighth of the launch
     const bool sup = !SYM && (((tiles_m % 8) == 0 && (tiles_n % 4) == 0) || ((tiles_m % 4) == 0 && (tiles_n % 8) == 0));
     const int G = sup ? 32 : ((SYM && (per_batch & 7) == 0) ? per_batch >> 3 : 0);
     const int nfull = (interleave && G > 0) ? nblk - nblk % (8 * G) : 0;
+    const int xcd = bid & 7;   // (of one XCD: the workgroups of a residue)
     if (bid < nfull) {
-      const int xcd = bid & 7, idx = bid >> 3;
+      const int idx = bid >> 3;
       bid = ((idx / G) * 8 + xcd) * G + idx % G;
     } else {   // (the rest of the launch, or all of it: a contiguous eighth per XCD)
-      bid = nfull + ((bid - nfull) & 7) * ((nblk - nfull) >> 3) + ((bid - nfull) >> 3);
+      const int rest = nblk - nfull, more = rest & 7;
+      bid = nfull + xcd * (rest >> 3) + (xcd < more ? xcd : more) + ((bid - nfull) >> 3);
     }
   }
   TileId r;
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(C::NT) void gemm_bf16_kernel(GemmArgs args) {
   const int lane = tid & 63;
   const int wave = wave_uniform(tid >> 6);
   const int wm = wave / C::WGN, wn = wave % C::WGN;
-  const TileId tile = decode_tile<BT, SYM>(d, (int)blockIdx.x - blk0, args.start[grp + 1] - blk0, (blk0 & 7) == 0, (args.interleave >> grp) & 1);
+  const TileId tile = decode_tile<BT, SYM>(d, (int)blockIdx.x - blk0, args.start[grp + 1] - blk0, (args.interleave >> grp) & 1);
   const int ti = tile.ti, tj = tile.tj;
   // with K slices the tile index counts (slice, matrix) pairs: the slice's partial product is matrix tile.b of C
   int b = tile.b, dK = d.K;
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(C::NT) void gemm_bf16_kernel(GemmArgs args) {
     dK = d.K - (int)k0 < d.k_slice ? d.K - (int)k0 : d.k_slice;
   }
   if (d.gate && (d.gate[b] != 0) != (d.gate_want != 0)) return;   // (before any barrier: the whole workgroup leaves)
-  const int m0 = ti * BT, n0 = tj * BT;
+  const int m0 = C::SLIDE ? min(ti * BT, d.M - BT) : ti * BT, n0 = C::SLIDE ? min(tj * BT, d.N - BT) : tj * BT;
   const bf16_t* A = (d.Atab ? static_cast<const bf16_t*>(d.Atab[b]) + d.a_off : static_cast<const bf16_t*>(d.A) + (long long)b * d.sA) +
                     k0 * (A_KS ? d.lda : 1);
   const bf16_t* B = (d.Btab ? static_cast<const bf16_t*>(d.Btab[b]) : static_cast<const bf16_t*>(d.B) + (long long)b * d.sB) +
@@ -246,8 +248,9 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
   constexpr int epi = (C::NT / 64) * 32 * (C::WCOLS + 4) * 4;
   constexpr int smem = stage2 > epi ? stage2 : epi;
   auto kfull = gemm_bf16_kernel<C, A_KS, B_KS, SYM, DA_LOOP_INTERIOR>;
-  auto kedge = gemm_bf16_kernel<C, A_KS, B_KS, SYM, (A_KS || B_KS) && !SYM ? DA_LOOP_EDGE : DA_LOOP_CHECKED>;
-  auto kgen = gemm_bf16_kernel<C, A_KS, B_KS, SYM, DA_LOOP_CHECKED>;
+  constexpr int CHECKED = C::SLIDE ? DA_LOOP_INTERIOR : DA_LOOP_CHECKED;
+  auto kedge = gemm_bf16_kernel<C, A_KS, B_KS, SYM, (A_KS || B_KS) && !SYM ? DA_LOOP_EDGE : CHECKED>;
+  auto kgen = gemm_bf16_kernel<C, A_KS, B_KS, SYM, CHECKED>;
   static DaOncePerDevice configured;
   const int rc_cfg = configured.run([&]() -> int {
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kfull), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
@@ -260,7 +263,7 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
   args.n = n;
   args.trace = g_tile_trace.load(std::memory_order_relaxed) ? 1 : 0;
 
-  const bool full = all_interior(d, n, BT);
+  const bool full = C::SLIDE || all_interior(d, n, BT);
   static const bool edge_env = [] { const char* e = getenv("DION_AMD_NO_EDGE_LOOP"); return !(e && atoi(e)); }();
   const int edge_opt = g_opt_edge_loop.load(std::memory_order_relaxed);
   const bool edge_on = edge_opt >= 0 ? edge_opt != 0 : edge_env;
@@ -357,16 +360,35 @@ double launch_cost(const GemmDesc* d, int n, int slots, double unit) {
 
 typedef Cfg<256, 2, 4> Big;
 typedef Cfg<128, 2, 2> Small;
+// Symmetric products: six row and three column blocks to a wavefront, as many LDS reads as the reads' rate allows under the products.
+typedef Cfg<192, 2, 4> Mid;
 typedef Cfg<256, 2, 4, 32> Big32;      // (GemmDesc::mi32)
 typedef Cfg<128, 2, 2, 32> Small32;
+
+// Whether 192 x 192 tiles can run: every operand at least a tile, whole stages, 32-bit offsets (as all_interior); the last tile of
+// a dimension is moved back over its neighbour, whose results it computes again, the same bits, so E must not be C.
+bool slide_ok(const GemmDesc* d, int n) {
+  for (int g = 0; g < n; ++g) {
+    if (!d[g].symmetric || d[g].M < Mid::BT || d[g].K % BK || d[g].Ctab || d[g].Etab || d[g].E == d[g].C) return false;
+    if (da_tile_span_bytes(false, Mid::BT, d[g].lda, d[g].K) >= (1LL << 32) || da_tile_span_bytes(false, Mid::BT, d[g].ldb, d[g].K) >= (1LL << 32)) return false;
+  }
+  return true;
+}
 
 // Tile choice by cost model: 256 x 256 tiles run one per CU, 128 x 128 tiles two per CU; a small
 // tile does a quarter of the work on half a CU at about 2/3 of the large tile's MFMA efficiency
 // (measured on grouped Newton-Schulz products of 768-wide matrices).
 // Interior-only (direct-to-LDS) eligibility wins over either.
+// Symmetric products have 192 x 192 tiles as well: half a matrix of tiles leaves a chip of 256 units idle more often (136 tiles
+// of 256 x 256 of a 4096 x 4096 result, 253 of 192 x 192).  A 64-deep stage of one takes 1.0 us, of a 256-tile 1.5, of two
+// 128-tiles on a unit 1.08, of one alone 0.8, and every launch takes its rounds times that.  X X^T (us, 128 / 192 / 256):
+// 4096 x 14336 393 / 224 / 314;  2 of 4096 x 4096 192 / 143 / 199;  8192 x 8192 699 / 530 / 597;  6 of 1536 x 6144 109 / 93 / 142;
+// 3072 x 8192 128 / 116 / 183;  and not: 5 of 4096 x 4096 414 / 358 / 320;  5120 x 5120 180 / 163 / 126;  2048 x 8192 98 / 114 / 179;
+// 24 of 1024 x 4096 141 / 137 / 107;  12 of 1024 x 1024 25 / 27 / 34.
 int choose_tile(const GemmDesc* d, int n) {
   static const int forced = [] { const char* e = getenv("DION_AMD_TILE"); return e ? atoi(e) : 0; }();
   if (forced == 128 || forced == 256) return forced;
+  if (forced == 192 && d[0].symmetric && slide_ok(d, n)) return forced;
   bool fits_big = true;
   // (a 192-wide product fills three quarters of a 256-tile: still cheaper than one and a half 128-tiles -- rank-192
   // P = BQ 34 -> 29.5 us per GPT-small bucket)
@@ -377,7 +399,15 @@ int choose_tile(const GemmDesc* d, int n) {
   const bool full_small = all_interior(d, n, 128) || (may_edge && edge_loop_ok(d, n, 128));
   const double cost_big = launch_cost<Big>(d, n, 256, 4.0);
   const double cost_small = launch_cost<Small>(d, n, 512, 3.0);
-  return fits_big && (full_big || !full_small) && cost_big <= cost_small ? 256 : 128;
+  const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
+  if (d[0].symmetric && slide_ok(d, n)) {
+    long long mid = 0, small = 0;
+    for (int g = 0; g < n; ++g) { mid += tiles_of<Mid>(d[g]); small += tiles_of<Small>(d[g]); }
+    // (against 128-tiles two to a unit, which hide one another's epilogues, only where sliding computes little again)
+    const double other = big ? cost_big : small <= 256 || 2.25 * mid > 1.15 * small ? 0.75 * cost_small : cost_small;
+    if (launch_cost<Mid>(d, n, 256, 2.75) < other) return Mid::BT;
+  }
+  return big ? 256 : 128;
 }
 
 }  // namespace
@@ -404,8 +434,9 @@ int da_gemm_bf16_grouped(const GemmDesc* din, int n, hipStream_t stream) {
     if (choose_tile(d, n) == 256) return launch<Big32, false, false, false>(d, n, stream);
     return launch<Small32, false, false, false>(d, n, stream);
   }
-  if (choose_tile(d, n) == 256) return dispatch_layout<Big>(d, n, stream);
-  return dispatch_layout<Small>(d, n, stream);
+  const int bt = choose_tile(d, n);
+  if (bt == Mid::BT) return launch<Mid, false, false, true>(d, n, stream);
+  return bt == 256 ? dispatch_layout<Big>(d, n, stream) : dispatch_layout<Small>(d, n, stream);
 }
 
 void da_gemm_bf16_set_edge_loop(int v) { g_opt_edge_loop.store(v < 0 ? -1 : (v != 0), std::memory_order_relaxed); }

@@ -33,6 +33,8 @@ struct Cfg {
   static constexpr int NCH = BT * 8 / NT;          // 16-byte chunks per thread per operand stage
   static constexpr int WROWS = BT / WGM, WCOLS = BT / WGN;
   static constexpr int NB = WROWS / 32;            // 32-row bands of a wavefront's sub-tile (the epilogue's unit)
+  // the last row and column of tiles lies against the matrix's end, over part of its neighbour (gemm_bf16.hip, Mid)
+  static constexpr bool SLIDE = BT == 192;
   typedef typename AccOf<MI>::type acc_t;
 };
 
@@ -141,7 +143,8 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   constexpr int PITCH = W + 4;       // floats; 16-byte aligned rows, conflict-free float4 writes
   constexpr int CPR = W / 8;         // 8-column chunks per row
   constexpr int RPP = 64 / CPR;      // rows per pass of the wavefront
-  constexpr int NPASS = 32 / RPP;
+  constexpr int NPASS = (32 + RPP - 1) / RPP;
+  constexpr bool ODD = 64 % CPR != 0;   // (six chunks to a row: ten rows a pass, four lanes and most of the last pass idle)
   constexpr int CSZ = CF32 ? 4 : 2;
   constexpr int NV = CF32 ? 2 : 1;   // 16-byte vectors per 8 elements
   float* stg = reinterpret_cast<float*>(lds) + wave * (32 * PITCH);
@@ -157,7 +160,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
                             : d.Etab ? static_cast<const char*>(d.Etab[b])
                                      : static_cast<const char*>(d.E) + (long long)b * d.sE * CSZ;
   const int lr = lane / CPR, c8 = (lane % CPR) * 8;
-  const bool col_ok = FULL || wn0 + c8 < dN;
+  const bool col_ok = (FULL || wn0 + c8 < dN) && (!ODD || lane < RPP * CPR);
   char* const Wbase = UPD ? static_cast<char*>(d.upd_tab[b]) : nullptr;
   constexpr bool w_f32 = WF32;   // (a compile-time variant: the prefetch buffers differ in size)
   constexpr int wsz = w_f32 ? 4 : 2;
@@ -169,7 +172,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   u32x4_t ev[DEPTH][NPASS][NV];
   // the weights a band updates are requested when the band starts, ahead of its staging through LDS and of the
   // arithmetic on E (two vectors per 8 elements when they are fp32)
-  constexpr int NWP = UPD == 2 ? (W / 64) * 4 : NPASS;
+  constexpr int NWP = UPD == 2 ? (W + 63) / 64 * 4 : NPASS;
   constexpr int NWV = WF32 ? 2 : 1;
   u32x4_t wv[NWP][NWV];
   auto weight_ptr = [&](int band, int pass) -> char* {
@@ -196,7 +199,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
       const u32x4_t z = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int h = 0; h < NV; ++h) dst[pass][h] = z;
-      if (col_ok && (FULL || m < dM)) {
+      if (col_ok && (FULL || m < dM) && (!ODD || pass * RPP + lr < 32)) {
         const char* Ep = Ebase + ((long long)m * lde + wn0 + c8) * CSZ;
 #pragma unroll
         for (int h = 0; h < NV; ++h) dst[pass][h] = ldg16(Ep + 16 * h);
@@ -244,7 +247,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
     for (int pass = 0; pass < NPASS; ++pass) {
       const int r = pass * RPP + lr;
       const int m = band_m + r;
-      if (col_ok && (FULL || m < dM)) {
+      if (col_ok && (FULL || m < dM) && (!ODD || r < 32)) {
         float* sp = stg + r * PITCH + c8;
         const float4 a0 = *reinterpret_cast<const float4*>(sp);
         const float4 a1 = *reinterpret_cast<const float4*>(sp + 4);
@@ -317,11 +320,11 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
       wave_sync_lds();
       // C^T: row n of the mirrored tile holds 32 consecutive m of this band
 #pragma unroll
-      for (int pass = 0; pass < (W / 64) * 4; ++pass) {
+      for (int pass = 0; pass < (W + 63) / 64 * 4; ++pass) {
         const int nl = (pass >> 2) * 64 + lane;
         const int mg = (pass & 3) * 8;
         const int n = wn0 + nl, m = band_m + mg;
-        if (FULL || (n < dN && m < dM)) {  // M is a multiple of 8 for symmetric outputs
+        if ((FULL || (n < dN && m < dM)) && (W % 64 == 0 || nl < W)) {  // M is a multiple of 8 for symmetric outputs
           float v[8];
 #pragma unroll
           for (int q = 0; q < 8; ++q) v[q] = stg[(mg + q) * PITCH + nl];

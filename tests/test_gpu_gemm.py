@@ -124,3 +124,21 @@ def test_alignment_is_rejected(dev):
     A = torch.randn(64, 36, dtype=torch.bfloat16, device=dev)  # K = 36 is not a multiple of 8
     with pytest.raises(_lib.DionAmdError):
         gemm(A, A)
+
+
+@pytest.mark.parametrize("batch, m, k", [(60, 384, 64), (32, 520, 136), (26, 576, 192), (1, 3080, 64), (16, 776, 3072), (1, 3912, 128)])
+def test_symmetric_products_in_tiles_that_slide(dev, batch, m, k):
+    """Batches whose symmetric products take 192-tiles, the last ones moved back over their neighbours (or k not in whole stages: not), give
+    the bits of one matrix at a time, which takes 128-tiles, and exactly symmetric ones."""
+    from dion_amd.newton_schulz import ns_line_1, ns_line_2
+
+    torch.manual_seed(2)
+    A = torch.randn(batch, m, k, dtype=torch.bfloat16, device=dev)
+    got = ns_line_1(A)
+    assert torch.equal(got, got.mT)
+    assert rel_fro(got[-1], A[-1].cpu().double() @ A[-1].cpu().double().mT) < 6e-3     # (as in test_ns_line_1)
+    got2 = ns_line_2(got, alpha=0.5, beta=-1.5) if m % 64 == 0 else got
+    for b in {0, batch // 2, batch - 1}:
+        if batch > 1:
+            assert torch.equal(ns_line_1(A[b]), got[b])
+            assert m % 64 or torch.equal(ns_line_2(got[b], alpha=0.5, beta=-1.5), got2[b])
