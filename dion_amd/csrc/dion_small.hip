@@ -406,12 +406,13 @@ __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
       const int task = wave_uniform(t - kth * per);
       const int b = wave_uniform((int)a.order[sh_at[entry] + kth]);
       int* words = G.words + (long long)b * CTR_STRIDE;
-      if (tid == 0 && wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
-      __syncthreads();
       const long long rr = (long long)G.rp * G.rp;
       const Factor F = {G.slab + (long long)b * G.slices * rr, G.L + b * rr, G.T + b * rr, G.A2 + b * rr, G.slices, G.r, G.rp, G.rT,
                         words + W_BAD, words + W_SICK, G.info ? G.info + b : nullptr, reinterpret_cast<double*>(words + W_RANGE), PIVOT_RATIO};
-      factor_task(F, phase >> 1, (phase & 1) == 0, task, lds, tid, lane, wave, wm, wn);
+      factor_task(F, phase >> 1, (phase & 1) == 0, task, lds, tid, lane, wave, wm, wn, [&] {
+        if (tid == 0 && wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
+        __syncthreads();
+      });
       // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
       unsigned next = DA_NO_TICKET;
       if (tid == 0) next = request_ticket(word);

@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
       } else {
         const Factor F = {a.w.slab + b * a.slices * rr, a.w.L + b * rr, a.w.T + b * rr, nullptr, a.slices, a.r_live, rp, rT,
                           words + W_BAD, words + W_SICK, a.info + b, reinterpret_cast<double*>(words + W_RANGE), 0.0};
-        factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn);
+        factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn, [] {});
         if (tid == 0) next = request_ticket(word);
       }
       // ---- publish: every wavefront's stores are acknowledged, then the counter moves

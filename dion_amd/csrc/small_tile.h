@@ -559,8 +559,10 @@ struct Factor {
 };
 // Left-looking.  `diag`: block (j, j) -- the slabs added in order, less the products of the earlier columns -- is factored and
 // the factor inverted.  Otherwise task 0 .. rT - 2: a block of column j of L below the diagonal or of block row j of T.
+// `wait` (all threads) returns when the phases before are complete; P^T P has been for long, and is loaded ahead of it.
+template <typename Wait>
 __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, int task, char* lds, int tid, int lane, int wave, int wm,
-                                            int wn) {
+                                            int wn, Wait wait) {
   typedef Real<double, 64> RD;
   enum Job { J_DIAG, J_LOW, J_INV };
   double* const d = reinterpret_cast<double*>(lds);
@@ -572,10 +574,6 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
   const int kend = wave_uniform((job == J_INV ? j - x : j) * 64);
   // J_INV: sum over k of L(j, k) T(k, x), x <= k < j;  else: sum over k < j of L(x, k) L(j, k)^T
   const Opnd<double, false> sd = work<double>(T + (long long)j * 64 * rp + j * 64, rp, 0);   // D, the inverse of the diagonal block's factor
-  if (kend > 0) {
-    if (job == J_INV) direct64<true>(LT + (long long)x * 64 * rp + j * 64, rp, T + (long long)x * 64 * rp + x * 64, rp, kend, d, lane, wm, wn);
-    else direct64<true>(LT + x * 64, rp, LT + j * 64, rp, kend, d, lane, wm, wn);
-  }
   double2_t w[8];        // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
   const int k = (tid & 31) * 2, i0 = tid >> 5;
 #pragma unroll
@@ -607,6 +605,11 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
         w[u][1] = gi >= F.r && gi == gk + 1 ? 1.0 : 0.0;
       }
     }
+  }
+  wait();
+  if (kend > 0) {
+    if (job == J_INV) direct64<true>(LT + (long long)x * 64 * rp + j * 64, rp, T + (long long)x * 64 * rp + x * 64, rp, kend, d, lane, wm, wn);
+    else direct64<true>(LT + x * 64, rp, LT + j * 64, rp, kend, d, lane, wm, wn);
   }
   if (kend > 0) {
     const double sign = job == J_INV ? 1.0 : -1.0;
