@@ -13,9 +13,9 @@
 //   BQ      P = B' Q                                      64 x 64 tiles
 //   GRAM    P^T P in fp64, lower tiles, K slices as slabs of their own
 //   CHAIN   P^T P = L L^T and T = L^-1 in blocks of 64, left-looking, in phases DIAG0 LOW0 DIAG1 LOW1 ..: DIAGj adds the slabs (in
-//           order) and the earlier columns' products to block (j, j), factors it and inverts the factor; LOWj does the rest of
-//           block column j of L and of block row j of T, a task per block.  Workgroups take tasks from eight queues, one per XCD
-//           (flow_queue.h), a counter per matrix and phase says when the next phase may start, and a matrix stays with one XCD.
+//           order), forms block (j, j - 1) of L and factors and inverts block (j, j); LOWj does the rest of block column j of L and
+//           of block row j of T, a task per block (factor_task).  Workgroups take tasks from eight queues, one per XCD
+//           (flow_queue.h), a counter per matrix and phase says when a later one may start, and a matrix stays with one XCD.
 //   PT      P T^T in fp64
 //   FIXG, FIXP  only do anything for a matrix whose pivot range says that cond(P) may leave a visible defect, or with a failed
 //           pivot: the closed-form second pass of da_orthonormalize in fp64 (defect measured, noise columns dropped,
@@ -26,7 +26,7 @@
 // All but CHAIN used to be phases of the queues: two workgroups to a compute unit (the factorisation's registers), a matrix's tiles on
 // one XCD's 64 workgroups, and a ticket and a counter for every tile.  14 bf16 matrices of 341 to 2731 rows at rank 256 and 86 (us,
 // as phases / as launches): set-up 98 / 24, BQ 52 / 31, GRAM 62 / 41, PT 62 / 59, FIX 16 / 9, BTP 48 / 41, CNORM 7 / 9, UPD 155 / 67;
-// the step 622 / 416.  24 fp32 matrices of 256 x 256 and 256 x 1024 at rank 128: 218 / 196.
+// the step 622 / 416, by now 385.  24 fp32 matrices of 256 x 256 and 256 x 1024 at rank 128: 218 / 196, by now 185.
 // The orthonormaliser is the fp64 CholeskyQR of dion.hip for every matrix: at these sizes the fp64 products cost less than
 // the launches of the two-precision road.  P, R and the products with B run on the matrix cores in the momentum's dtype with
 // the instructions and the order of k of the batched kernels (v_mfma_f32_16x16x32_bf16, in the updates v_mfma_f32_32x32x16_bf16; v_mfma_f32_32x32x2_f32).
@@ -108,9 +108,9 @@ __host__ __device__ inline int tiles_of(const GroupDev& G, Kind kind, bool bf) {
     default: return 0;
   }
 }
-// tasks of a phase of the factorisation: the diagonal block; the blocks below it and the blocks of row j of the inverse
+// tasks of a phase of the factorisation
 __host__ __device__ inline int tasks_of(const GroupDev& G, int phase) {
-  return (phase >> 1) >= G.rT ? 0 : (phase & 1) ? G.rT - 1 : 1;
+  return (phase >> 1) >= G.rT ? 0 : (phase & 1) ? low_tasks(G.rT, phase >> 1) : 1;
 }
 
 template <bool BF> struct MomentumType { typedef float type; };
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256, BF ? 3 : 4) void dion_small_gram_kernel(Args a
 __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   __shared__ int sh_ticket[2];
-  __shared__ int sh_start[64], sh_per[64], sh_wait[64];   // the queue's schedule: entry = phase * ngroups + group
+  __shared__ int sh_start[64], sh_per[64];   // the queue's schedule: entry = phase * ngroups + group
   __shared__ unsigned char sh_at[64];
   static_assert(PHASES * DA_DS_GROUPS <= 64, "one entry each");
   const int xcd = xcc_id();
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
       __syncthreads();   // thread 0 rewrites sh_ticket for the next queue
       continue;
     }
-    // ---- the schedule, phase by phase, group by group: first ticket, tasks per matrix, and what a phase waits for
+    // ---- the schedule, phase by phase, group by group: first ticket and tasks per matrix
     if (tid < 64) {
       int n = 0;
       if (tid < PHASES * args.ngroups) {
@@ -374,11 +374,8 @@ __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
         const GroupDev& G = args.g[tid - k * args.ngroups];
         const int per = tasks_of(G, k);
         n = per * G.nq[q];
-        int w = k - 1;
-        while (w >= 0 && tasks_of(G, w) == 0) --w;
         sh_per[tid] = per;
         sh_at[tid] = G.at[q];
-        sh_wait[tid] = w < 0 ? -1 : (w << 24 | tasks_of(G, w));
       }
       int sum = n;   // exclusive sums
 #pragma unroll
@@ -400,7 +397,7 @@ __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
       // ---- ticket -> (phase, group, matrix, task): the last entry that starts at or before it
       const int entry = wave_uniform(__popcll(__ballot(lane < PHASES * a.ngroups && sh_start[lane] <= t)) - 1);
       t -= wave_uniform(sh_start[entry]);
-      const int phase = entry / a.ngroups, per = wave_uniform(sh_per[entry]), wait = wave_uniform(sh_wait[entry]);
+      const int phase = entry / a.ngroups, per = wave_uniform(sh_per[entry]);
       const GroupDev& G = a.g[entry - phase * a.ngroups];
       const int kth = wave_uniform(t / per);
       const int task = wave_uniform(t - kth * per);
@@ -409,10 +406,14 @@ __global__ __launch_bounds__(256, 2) void dion_small_chain_kernel(Args args) {
       const long long rr = (long long)G.rp * G.rp;
       const Factor F = {G.slab + (long long)b * G.slices * rr, G.L + b * rr, G.T + b * rr, G.A2 + b * rr, G.slices, G.r, G.rp, G.rT,
                         words + W_BAD, words + W_SICK, G.info ? G.info + b : nullptr, reinterpret_cast<double*>(words + W_RANGE), PIVOT_RATIO};
-      factor_task(F, phase >> 1, (phase & 1) == 0, task, lds, tid, lane, wave, wm, wn, [&] {
-        if (tid == 0 && wait >= 0) wait_count(words + (wait >> 24), wait & 0xffffff, a.status, a.spin_limit);
+      auto wait_phase = [&](int before) {
+        if (before < 0) return;
+        if (tid == 0) wait_count(words + before, tasks_of(G, before), a.status, a.spin_limit);
         __syncthreads();
-      });
+      };
+      const bool diag = (phase & 1) == 0;
+      factor_task(F, phase >> 1, diag, task, lds, tid, lane, wave, wm, wn, [&] { wait_phase(diag ? phase - 3 : phase - 2); },
+                  [&] { wait_phase(diag ? phase - 2 : phase - 1); });
       // ---- publish: every wavefront's stores are acknowledged, then the matrix's counter moves
       unsigned next = DA_NO_TICKET;
       if (tid == 0) next = request_ticket(word);

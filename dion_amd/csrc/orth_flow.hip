@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
       }
       if (tid < 128) {
         const int per = tid >= entries ? 0 : tid == 0 ? ng * args.slices : tid == entries - 2 ? args.mT * rT : tid == entries - 1 ? ng + args.mT * rT
-                        : (tid & 1) ? 1 : rT - 1;
+                        : (tid & 1) ? 1 : low_tasks(rT, (tid - 1) >> 1);
         sh_per[tid] = per;
         sh_start[tid] = per * nf;
       }
@@ -121,7 +121,9 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
         } else if (entry == 1) {
           wait_count(words + CTR_GRAM, ng * a.slices, a.status, a.spin_limit);
         } else {
-          wait_count(words + CTR_FACTOR, pt ? rT * rT : j * rT + ((entry & 1) ? 0 : 1), a.status, a.spin_limit);
+          // one counter for the phases, rT - 1 tasks to a column (the last: rT): DIAG(j - 1) and what is before it, LOW(j - 2)
+          // included, which no later task could stand in for; LOWj likewise
+          wait_count(words + CTR_FACTOR, pt ? (rT - 1) * (rT - 1) + rT : ((entry & 1) ? j - 1 : j) * (rT - 1) + 1, a.status, a.spin_limit);
         }
       }
       __syncthreads();
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void orth_flow_kernel(Args args) {
       } else {
         const Factor F = {a.w.slab + b * a.slices * rr, a.w.L + b * rr, a.w.T + b * rr, nullptr, a.slices, a.r_live, rp, rT,
                           words + W_BAD, words + W_SICK, a.info + b, reinterpret_cast<double*>(words + W_RANGE), 0.0};
-        factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn, [] {});
+        factor_task(F, (entry - 1) >> 1, (entry & 1) != 0, task, lds, tid, lane, wave, wm, wn, [] {}, [] {});
         if (tid == 0) next = request_ticket(word);
       }
       // ---- publish: every wavefront's stores are acknowledged, then the counter moves

@@ -557,30 +557,35 @@ struct Factor {
   double* range;               // smallest and largest pivot so far
   double ratio;
 };
-// Left-looking.  `diag`: block (j, j) -- the slabs added in order, less the products of the earlier columns -- is factored and
-// the factor inverted.  Otherwise task 0 .. rT - 2: a block of column j of L below the diagonal or of block row j of T.
-// `wait` (all threads) returns when the phases before are complete; P^T P has been for long, and is loaded ahead of it.
-template <typename Wait>
+// Left-looking.  DIAGj forms block (j, j - 1) of L from the inverse of the diagonal block before, takes its products off block (j, j),
+// factors that and inverts the factor: the chain of the phases is one task per column of blocks, and the rest, `low_tasks` per column,
+// runs beside it: blocks of column j of L from (j + 2, j) down, and blocks of block row j of T.  (With all of column j a phase
+// between DIAGj and DIAG(j + 1) a column took 33 us, so 28.)
+// `before` (all threads) returns when LOW(j - 2) resp. LOW(j - 1) is complete, `wait` when DIAG(j - 1) resp. DIAGj is; P^T P has been for
+// long.  What a wait does not stand before is done ahead of it.
+__host__ __device__ inline int low_tasks(int rT, int j) { return (rT - 2 - j > 0 ? rT - 2 - j : 0) + j; }
+template <typename Before, typename Wait>
 __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, int task, char* lds, int tid, int lane, int wave, int wm,
-                                            int wn, Wait wait) {
+                                            int wn, Before before, Wait wait) {
   typedef Real<double, 64> RD;
   enum Job { J_DIAG, J_LOW, J_INV };
   double* const d = reinterpret_cast<double*>(lds);
+  double* const d2 = d + 64 * 66;
+  static_assert(2 * 64 * 66 * 8 <= STAGES64, "two blocks");
   double *const LT = F.LT, *const T = F.T;
-  const int rp = F.rp, rT = F.rT;
+  const int rp = F.rp, rT = F.rT, nlow = max(0, rT - 2 - j);
   const long long rr = (long long)rp * rp;
-  const Job job = diag ? J_DIAG : task < rT - 1 - j ? J_LOW : J_INV;
-  const int x = diag ? j : job == J_LOW ? j + 1 + task : task - (rT - 1 - j);
-  const int kend = wave_uniform((job == J_INV ? j - x : j) * 64);
-  // J_INV: sum over k of L(j, k) T(k, x), x <= k < j;  else: sum over k < j of L(x, k) L(j, k)^T
-  const Opnd<double, false> sd = work<double>(T + (long long)j * 64 * rp + j * 64, rp, 0);   // D, the inverse of the diagonal block's factor
-  double2_t w[8];        // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
+  const Job job = diag ? J_DIAG : task < nlow ? J_LOW : J_INV;
+  const int x = diag ? j : job == J_LOW ? j + 2 + task : task - nlow;
+  const int jd = diag ? j - 1 : j;   // the column of blocks whose L(x, jd) is formed
+  const Opnd<double, false> sd = work<double>(T + (long long)jd * 64 * rp + jd * 64, rp, 0);   // D, the inverse of its diagonal block's factor
+  double2_t own[8];              // element pair u: row (tid + 256 u) / 32, columns 2 ((tid + 256 u) % 32)
   const int k = (tid & 31) * 2, i0 = tid >> 5;
+  // block (x, jb) of P^T P: the slabs in slice order; beyond the rank the matrix is the identity
+  auto gram_block = [&](double2_t (&w)[8], int jb) {
 #pragma unroll
-  for (int u = 0; u < 8; ++u) w[u] = double2_t{0.0, 0.0};
-  if (job != J_INV) {
-    // the slabs of P^T P in slice order; beyond the rank the matrix is the identity
-    const double* const slab = F.slab + (long long)(x * 64 + i0) * rp + j * 64 + k;
+    for (int u = 0; u < 8; ++u) w[u] = double2_t{0.0, 0.0};
+    const double* const slab = F.slab + (long long)(x * 64 + i0) * rp + jb * 64 + k;
     for (int s0 = 0; s0 < F.slices; s0 += 4) {   // four slabs on the way at a time
       double2_t y[4][8];
 #pragma unroll
@@ -599,105 +604,135 @@ __device__ __forceinline__ void factor_task(const Factor& F, int j, bool diag, i
     const int lim = ((F.r + 31) >> 5) << 5;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int gi = x * 64 + i0 + 8 * u, gk = j * 64 + k;
+      const int gi = x * 64 + i0 + 8 * u, gk = jb * 64 + k;
       if (gi >= F.r || gk >= lim || (gk >> 5) > (gi >> 5)) {   // (not written by GRAM)
         w[u][0] = gi >= F.r && gi == gk ? 1.0 : 0.0;
         w[u][1] = gi >= F.r && gi == gk + 1 ? 1.0 : 0.0;
       }
     }
-  }
-  wait();
-  if (kend > 0) {
-    if (job == J_INV) direct64<true>(LT + (long long)x * 64 * rp + j * 64, rp, T + (long long)x * 64 * rp + x * 64, rp, kend, d, lane, wm, wn);
-    else direct64<true>(LT + x * 64, rp, LT + j * 64, rp, kend, d, lane, wm, wn);
-  }
-  if (kend > 0) {
-    const double sign = job == J_INV ? 1.0 : -1.0;
+  };
+  // w += sign * the product that lies in d
+  auto add = [&](double2_t (&w)[8], double sign) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       w[u][0] += sign * d[(i0 + 8 * u) * 66 + k];
       w[u][1] += sign * d[(i0 + 8 * u) * 66 + k + 1];
     }
-  }
-  if (job == J_DIAG) {
+    __syncthreads();
+  };
+  auto park = [&](const double2_t (&w)[8]) {   // a block out of the way of the products' registers; every thread its own elements
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      d[(i0 + 8 * u) * 66 + k] = w[u][0];
-      d[(i0 + 8 * u) * 66 + k + 1] = w[u][1];
+      d2[(i0 + 8 * u) * 66 + k] = w[u][0];
+      d2[(i0 + 8 * u) * 66 + k + 1] = w[u][1];
     }
+  };
+  if (job == J_LOW || (job == J_DIAG && j > 0)) {
+    double2_t w[8];
+    gram_block(w, jd);
+    park(w);
+  }
+  if (job == J_DIAG) gram_block(own, j);
+  before();
+  if (job == J_DIAG && j > 1) {   // the columns up to j - 2 of row j
+    direct64<true>(LT + j * 64, rp, LT + j * 64, rp, jd * 64, d, lane, wm, wn);
+    add(own, -1.0);
+  }
+  wait();
+  if (job == J_INV)      // sum over k of L(j, k) T(k, x), x <= k < j
+    direct64<true>(LT + (long long)x * 64 * rp + j * 64, rp, T + (long long)x * 64 * rp + x * 64, rp, (j - x) * 64, d, lane, wm, wn);
+  else if (jd > 0)       // sum over k < jd of L(x, k) L(jd, k)^T
+    direct64<true>(LT + x * 64, rp, LT + jd * 64, rp, jd * 64, d, lane, wm, wn);
+  if (jd >= 0) {
+    double2_t w[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) w[u] = job == J_INV ? double2_t{0.0, 0.0} : double2_t{d2[(i0 + 8 * u) * 66 + k], d2[(i0 + 8 * u) * 66 + k + 1]};
+    if (job == J_INV) add(w, 1.0);
+    else if (jd > 0) add(w, -1.0);
+    else __syncthreads();
+    // second product, both operands to the LDS stages:  L(x, jd) = W(x, jd) D^T;   T(j, x) = -D W(j, x)
+    Raw<double> dr[2];
+    dr[0] = fetch_chunk<64, KD>(sd, tid, 0, 0);
+    dr[1] = fetch_chunk<64, KD>(sd, tid, 0, KD);
+    double* const wst = d + (job == J_INV ? RD::OPND : 0);
+    double* const dst = d + (job == J_INV ? 0 : RD::OPND);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + 8 * u;
+      if (job == J_INV) {
+        wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k] = w[u][0];
+        wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k + 1] = w[u][1];
+      } else {
+        wst[(k >> 5) * 2 * RD::OPND + (k & 31) * RD::P + i] = w[u][0];
+        wst[(k >> 5) * 2 * RD::OPND + ((k + 1) & 31) * RD::P + i] = w[u][1];
+      }
+    }
+    put_chunk<double, 64, false>(dst, sd, dr[0], tid, 0, 0, NoTurn());
+    put_chunk<double, 64, false>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
     __syncthreads();
-    Mfma<double>::acc_t S[4];
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = wave * 16 + Mfma<double>::row(v, lane), col = tj * 16 + (lane & 15);
-        S[tj][v] = tj <= wave ? (row >= col ? d[row * 66 + col] : d[col * 66 + row]) : 0.0;
-      }
-    __syncthreads();   // (the block lies where the factorisation works)
-    double* const dT = d + DIAG_W;
-    static_assert(2 * DIAG_W * 8 <= STAGES64, "the work area and the inverse factor");
-    diag_factor64(S, d, dT, min(64, F.r - j * 64), 64, lane, wave, [&](int failed, double pmin, double pmax) {
-      if (lane != 0) return;
-      int bad = failed ? j * 64 + failed : 0;
-      if (j > 0) {
-        const int before = __hip_atomic_load(F.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before) bad = before;
-        pmin = fmin(pmin, __hip_atomic_load(F.range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        pmax = fmax(pmax, __hip_atomic_load(F.range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      }
-      __hip_atomic_store(F.bad, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(F.range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(F.range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (j == rT - 1) {
-        const bool healthy = bad == 0 && pmin >= F.ratio * pmax && pmax > 0.0;
-        __hip_atomic_store(F.sick, healthy ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (F.info) *F.info = bad;
-      }
-    });
-    double* const Dw = T + (long long)j * 64 * rp + j * 64;
-    for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * DIAG_P + (e >> 6)];
-    if (F.TT) {
-      double* const Dt = F.TT + (long long)j * 64 * rp + j * 64;
-      for (int e = tid; e < 4096; e += 256) Dt[(long long)(e >> 6) * rp + (e & 63)] = dT[(e >> 6) * DIAG_P + (e & 63)];
-    }
-    return;
-  }
-  // second product, both operands to the LDS stages:  L(x, j) = W(x, j) D^T;   T(j, x) = -D W(j, x)
-  Raw<double> dr[2];
-  dr[0] = fetch_chunk<64, KD>(sd, tid, 0, 0);
-  dr[1] = fetch_chunk<64, KD>(sd, tid, 0, KD);
-  __syncthreads();
-  double* const wst = d + (job == J_INV ? RD::OPND : 0);
-  double* const dst = d + (job == J_INV ? 0 : RD::OPND);
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int i = i0 + 8 * u;
+    Acc16<double, 64> acc;
+    acc.clear();
+    acc.stage(d, d + RD::OPND, lane, wm, wn);
+    acc.stage(d + 2 * RD::OPND, d + 3 * RD::OPND, lane, wm, wn);
+    __syncthreads();
+    acc.out(d, lane, wm, wn);
     if (job == J_INV) {
-      wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k] = w[u][0];
-      wst[(i >> 5) * 2 * RD::OPND + (i & 31) * RD::P + k + 1] = w[u][1];
-    } else {
-      wst[(k >> 5) * 2 * RD::OPND + (k & 31) * RD::P + i] = w[u][0];
-      wst[(k >> 5) * 2 * RD::OPND + ((k + 1) & 31) * RD::P + i] = w[u][1];
+      double* const out = T + (long long)j * 64 * rp + x * 64;
+      for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = -d[(e >> 6) * 66 + (e & 63)];
+    }
+    double* const turned = job != J_INV ? LT + (long long)jd * 64 * rp + x * 64 : F.TT ? F.TT + (long long)x * 64 * rp + j * 64 : nullptr;
+    if (turned) {
+      const double sign = job == J_INV ? -1.0 : 1.0;
+      for (int e = tid; e < 4096; e += 256) turned[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e & 63) * 66 + (e >> 6)];
     }
   }
-  put_chunk<double, 64, false>(dst, sd, dr[0], tid, 0, 0, NoTurn());
-  put_chunk<double, 64, false>(dst + 2 * RD::OPND, sd, dr[1], tid, 0, KD, NoTurn());
+  if (job != J_DIAG) return;
+  // ---- the diagonal block: wavefront w holds its 16 x 16 blocks (w, 0 .. w)
+  park(own);
   __syncthreads();
-  Acc16<double, 64> acc;
-  acc.clear();
-  acc.stage(d, d + RD::OPND, lane, wm, wn);
-  acc.stage(d + 2 * RD::OPND, d + 3 * RD::OPND, lane, wm, wn);
-  __syncthreads();
-  acc.out(d, lane, wm, wn);
-  if (job == J_INV) {
-    double* const out = T + (long long)j * 64 * rp + x * 64;
-    for (int e = tid; e < 4096; e += 256) out[(long long)(e >> 6) * rp + (e & 63)] = -d[(e >> 6) * 66 + (e & 63)];
+  Mfma<double>::acc_t S[4];
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = wave * 16 + Mfma<double>::row(v, lane), col = tj * 16 + (lane & 15);
+      S[tj][v] = tj <= wave ? (row >= col ? d2[row * 66 + col] : d2[col * 66 + row]) : 0.0;
+    }
+  if (j > 0) {   // less L(j, j - 1) L(j, j - 1)^T
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks) {
+      const double a = -d[(wave * 16 + (lane & 15)) * 66 + ks * 4 + (lane >> 4)];
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj)
+        if (tj <= wave) S[tj] = Mfma<double>::mma(a, d[(tj * 16 + (lane & 15)) * 66 + ks * 4 + (lane >> 4)], S[tj]);
+    }
   }
-  double* const turned = job == J_LOW ? LT + (long long)j * 64 * rp + x * 64 : F.TT ? F.TT + (long long)x * 64 * rp + j * 64 : nullptr;
-  if (turned) {
-    const double sign = job == J_INV ? -1.0 : 1.0;
-    for (int e = tid; e < 4096; e += 256) turned[(long long)(e >> 6) * rp + (e & 63)] = sign * d[(e & 63) * 66 + (e >> 6)];
+  __syncthreads();   // (the blocks lie where the factorisation works)
+  double* const dT = d + DIAG_W;
+  static_assert(2 * DIAG_W * 8 <= STAGES64, "the work area and the inverse factor");
+  diag_factor64(S, d, dT, min(64, F.r - j * 64), 64, lane, wave, [&](int failed, double pmin, double pmax) {
+    if (lane != 0) return;
+    int bad = failed ? j * 64 + failed : 0;
+    if (j > 0) {
+      const int before = __hip_atomic_load(F.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (before) bad = before;
+      pmin = fmin(pmin, __hip_atomic_load(F.range, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      pmax = fmax(pmax, __hip_atomic_load(F.range + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    __hip_atomic_store(F.bad, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(F.range, pmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(F.range + 1, pmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (j == rT - 1) {
+      const bool healthy = bad == 0 && pmin >= F.ratio * pmax && pmax > 0.0;
+      __hip_atomic_store(F.sick, healthy ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (F.info) *F.info = bad;
+    }
+  });
+  double* const Dw = T + (long long)j * 64 * rp + j * 64;
+  for (int e = tid; e < 4096; e += 256) Dw[(long long)(e >> 6) * rp + (e & 63)] = dT[(e & 63) * DIAG_P + (e >> 6)];
+  if (F.TT) {
+    double* const Dt = F.TT + (long long)j * 64 * rp + j * 64;
+    for (int e = tid; e < 4096; e += 256) Dt[(long long)(e >> 6) * rp + (e & 63)] = dT[(e >> 6) * DIAG_P + (e & 63)];
   }
 }
 
