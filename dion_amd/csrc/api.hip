@@ -1187,7 +1187,7 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
         }
         if (rc) return rc;
         // all-zero / NaN guard on P   (reference dion/dion.py:847, 1416-1444)
-        rc = da_fix(P, nullptr, m_dtype, sP, cb, nonzero, s);
+        rc = da_fix(P, m_dtype, sP, cb, nonzero, s);
         if (rc) return rc;
       }
       // ---- R = B^T P   (reference dion/dion.py:839)
@@ -1216,13 +1216,14 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
         rc = gemm_group(gs, slices, m_dtype, s, DA_PROF_DION_BTP);
         if (rc) return rc;
         DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);
-        rc = da_fix_sum(parts, slices, pstride, R, Qc, m_dtype, sQ, cb, nonzero, s);
+        // (the orthonormaliser is done with its fp64 scratch: the column sums take its head)
+        rc = da_fix_colsum(parts, slices, pstride, R, Qc, m_dtype, np, r, cb, nonzero, reinterpret_cast<double*>(orth_ws), s);
         if (rc) return rc;
       } else {
         rc = gemm_any(g, m_dtype, s, DA_PROF_DION_BTP);
         if (rc) return rc;
         DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);
-        rc = da_fix(R, Qc, m_dtype, sQ, cb, nonzero, s);
+        rc = da_fix_colsum(nullptr, 0, 0, R, Qc, m_dtype, np, r, cb, nonzero, reinterpret_cast<double*>(orth_ws), s);
         if (rc) return rc;
       }
     }  // power iterations
@@ -1254,7 +1255,6 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
     // ---- Q_new = column-normalised R   (reference dion/dion.py:856, 875, 1460-1491, 1533-1561)
     {
       DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);
-      // the orthonormaliser is done with its fp64 scratch: reuse its head for the column sums
       rc = da_colnorm(R, Qn, m_dtype, tq, q_dtype, np, r, rank, eps, cb, reinterpret_cast<double*>(orth_ws), s);
       if (rc) return rc;
     }

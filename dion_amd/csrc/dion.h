@@ -12,15 +12,16 @@ int da_add_grad(const DaPtrTable& m, const DaPtrTable& g, int m_dtype, int g_dty
 // dst[b] (rows x ld, contiguous batch) <- table[b] (rows x cols contiguous), columns beyond cols zeroed; ld % 8 == 0.
 int da_cast_table(const DaPtrTable& src, int s_dtype, void* dst, int d_dtype, int rows, int cols, int ld, int batch,
                   hipStream_t s);
-int da_fix(void* v, const void* alt, int dtype, long long n, int batch, const int* nonzero, hipStream_t s);
-// v[b] <- fix(round(part[0][b] + ... + part[parts-1][b])): the partial sums (fp32, n elements per matrix, slice k
-// at part + k * pstride) of a product whose inner dimension was cut into slices.
-int da_fix_sum(const float* part, int parts, long long pstride, void* v, const void* alt, int dtype, long long n,
-               int batch, const int* nonzero, hipStream_t s);
-// R, qn: rows x r (r % 8 == 0); the Q state receives the first q_cols columns as a contiguous rows x q_cols
-// matrix.  `sums` is scratch for (1 + min(ceil(rows / 64), 1024)) * batch * r doubles.
+int da_fix(void* v, int dtype, long long n, int batch, const int* nonzero, hipStream_t s);
+// R (rows x r, r % 8 == 0) fixed up, `alt` in its place for an all-zero B, and its columns' sums of squares in slices of rows:
+// min(ceil(rows / 64), 64) * batch * r doubles.  parts > 0: R is round(part[0][b] + ... + part[parts - 1][b]), the partial sums (fp32,
+// rows * r elements per matrix, slice k at part + k * pstride) of a product whose inner dimension was cut into slices.
+int da_fix_colsum(const float* part, int parts, long long pstride, void* R, const void* alt, int dtype, int rows, int r, int batch,
+                  const int* nonzero, double* sums, hipStream_t s);
+// qn = R with normalised columns, both rows x r; the Q state receives the first q_cols columns as a contiguous rows x q_cols
+// matrix.  `sums`: da_fix_colsum's of R.
 int da_colnorm(const void* R, void* qn, int m_dtype, const DaPtrTable& q, int q_dtype, int rows, int r, int q_cols,
-               float eps, int batch, double* sums, hipStream_t s);
+               float eps, int batch, const double* sums, hipStream_t s);
 
 // CholeskyQR (passes = 1) / CholeskyQR2 (passes = 2) of `batch` contiguous matrices P[b]
 // (rows x r, dtype bf16 or f32): one pass with fp64 Gram, Cholesky and triangular solve, then

@@ -132,135 +132,131 @@ __global__ __launch_bounds__(256) void cast_table_pitched_kernel(DaPtrTable st, 
   }
 }
 
-// v <- nan_to_num(v) * nonzero + alt * (1 - nonzero)      (alt may be null: treated as 0)
+// nan_to_num of the dtype; `alt` for an all-zero B
 template <typename T>
-__global__ __launch_bounds__(256) void fix_kernel(T* V, const T* alt, long long n, const int* nonzero) {
+__device__ __forceinline__ float fixed(float x, bool nz, float alt) {
+  if (x != x) x = 0.f;
+  else if (x > V8<T>::maxval()) x = V8<T>::maxval();
+  else if (x < -V8<T>::maxval()) x = -V8<T>::maxval();
+  return nz ? x : alt;
+}
+
+// v <- nan_to_num(v) * nonzero
+template <typename T>
+__global__ __launch_bounds__(256) void fix_kernel(T* V, long long n, const int* nonzero) {
   const int b = blockIdx.y;
   const bool nz = nonzero[b] != 0;
   T* p = V + (long long)b * n;
-  const T* a = alt ? alt + (long long)b * n : nullptr;
   for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (long long)gridDim.x * 256 * 8) {
-    float v[8], q[8];
+    float v[8];
     V8<T>::load(p + i, v);
-    if (a && !nz) V8<T>::load(a + i, q);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = v[e];
-      if (x != x) x = 0.f;
-      else if (x > V8<T>::maxval()) x = V8<T>::maxval();
-      else if (x < -V8<T>::maxval()) x = -V8<T>::maxval();
-      v[e] = nz ? x : (a ? q[e] : 0.f);
-    }
+    for (int e = 0; e < 8; ++e) v[e] = fixed<T>(v[e], nz, 0.f);
     V8<T>::store(p + i, v);
   }
 }
 
-// The same fix-up for a product that was computed as `parts` partial sums over slices of its inner dimension
-// (fp32, `pstride` elements apart): v <- round(sum of the parts), then as fix_kernel.
+// R <- nan_to_num(R) * nonzero + alt * (1 - nonzero), and the sums of its squared columns over a slice of rows, in fp64: 64 columns of
+// a slice per workgroup.  `parts`: R is a product in that many partial sums over slices of its inner dimension (fp32, `pstride`
+// elements apart), added and rounded here; 0: R holds it.  Bound by memory, and by the launches that stand in a row between R and the
+// update: two, which were four (fix-up, column sums, their sum, normalisation), and a pass over R less.  12 layers of d 768, ff 3072:
+// step at rank 768 3587 -> 3560 us, at rank 192 698 -> 696.
 template <typename T>
-__global__ __launch_bounds__(256) void fix_sum_kernel(const float* __restrict__ part, int parts, long long pstride,
-                                                      T* V, const T* alt, long long n, const int* nonzero) {
-  const int b = blockIdx.y;
+__global__ __launch_bounds__(256) void fix_colsum_kernel(const float* __restrict__ part, int parts, long long pstride, T* __restrict__ R,
+                                                         const T* __restrict__ alt, int rows, int r, int rows_per_slice,
+                                                         const int* __restrict__ nonzero, double* __restrict__ sums) {
+  __shared__ double red[32][64 + 1];
+  __shared__ double run[4][64];
+  const int b = blockIdx.z, c8 = (threadIdx.x & 7) * 8, row = threadIdx.x >> 3, col = blockIdx.x * 64 + c8;
   const bool nz = nonzero[b] != 0;
-  T* p = V + (long long)b * n;
-  const float* s0 = part + (long long)b * n;
-  const T* a = alt ? alt + (long long)b * n : nullptr;
-  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (long long)gridDim.x * 256 * 8) {
-    float v[8], q[8];
-    V8<float>::load(s0 + i, v);
-    for (int k = 1; k < parts; ++k) {
-      float t[8];
-      V8<float>::load(s0 + k * pstride + i, t);
+  const long long base = (long long)b * rows * r;
+  const int i0 = blockIdx.y * rows_per_slice;
+  const int i1 = i0 + rows_per_slice < rows ? i0 + rows_per_slice : rows;
+  double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (col < r)   // (r is a multiple of 8)
+    for (int i = i0 + row; i < i1; i += 32) {
+      const long long at = base + (long long)i * r + col;
+      float v[8], q[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (parts) {
+        V8<float>::load(part + at, v);
+        for (int k = 1; k < parts; ++k) {
+          float t[8];
+          V8<float>::load(part + k * pstride + at, t);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += t[e];
-    }
-    if (a && !nz) V8<T>::load(a + i, q);
+          for (int e = 0; e < 8; ++e) v[e] += t[e];
+        }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = V8<T>::round(v[e]);
-      if (x != x) x = 0.f;
-      else if (x > V8<T>::maxval()) x = V8<T>::maxval();
-      else if (x < -V8<T>::maxval()) x = -V8<T>::maxval();
-      v[e] = nz ? x : (a ? q[e] : 0.f);
+        for (int e = 0; e < 8; ++e) v[e] = V8<T>::round(v[e]);
+      } else {
+        V8<T>::load(R + at, v);
+      }
+      if (!nz) V8<T>::load(alt + at, q);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] = fixed<T>(v[e], nz, q[e]);
+        s[e] += (double)v[e] * (double)v[e];
+      }
+      V8<T>::store(R + at, v);
     }
-    V8<T>::store(p + i, v);
-  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) red[row][c8 + e] = s[e];
+  __syncthreads();
+  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+  double t = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) t += red[g * 8 + i][c];
+  run[g][c] = t;
+  __syncthreads();
+  if (g == 0 && blockIdx.x * 64 + c < r)
+    sums[((long long)blockIdx.y * gridDim.z + b) * r + blockIdx.x * 64 + c] = (run[0][c] + run[1][c]) + (run[2][c] + run[3][c]);
 }
 
 // Column normalisation of R[b] (rows x r, TM): Qn = R / (sqrt(sum_rows R^2) + eps), computed in
 // fp32 (column sums accumulated in fp64), stored as TM into qn[b] and, cast to TQ, into the
 // optimizer's Q state (its first q_cols columns: the working matrices may carry zero columns up to a
-// multiple of 8).  Three launches: partial column sums over row slices, their sum in slice order (so the
-// result does not depend on which workgroup finishes first), then a fully parallel normalise pass.
-template <typename TM>
-__global__ __launch_bounds__(256) void colsum_kernel(const TM* __restrict__ R, double* __restrict__ part, int rows, int r,
-                                                     int rows_per_slice) {
-  __shared__ double red[4][64];
-  const int b = blockIdx.z;
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int g = threadIdx.x >> 6;
-  const TM* Rb = R + (long long)b * rows * r;
-  const int i0 = blockIdx.y * rows_per_slice;
-  const int i1 = i0 + rows_per_slice < rows ? i0 + rows_per_slice : rows;
-  double s = 0.0;
-  if (c < r)
-    for (int i = i0 + g; i < i1; i += 4) {
-      const float v = ld_as_float<TM>(Rb + (long long)i * r + c);
-      s += (double)v * (double)v;
-    }
-  red[g][threadIdx.x & 63] = s;
-  __syncthreads();
-  if (g == 0 && c < r) {
-    const double t = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
-    part[((long long)blockIdx.y * gridDim.z + b) * r + c] = t;
-  }
-}
-
-// sums[b][c] = sum over the slices of part[k][b][c], in a fixed order: 64 columns per workgroup, the slices cut into
-// four contiguous runs (one per wavefront, each added in slice order), the four run sums added in run order
-__global__ __launch_bounds__(256) void colsum_finish_kernel(const double* __restrict__ part, double* __restrict__ sums,
-                                                            int slices, long long per_slice) {
-  __shared__ double run[4][64];
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const long long i = (long long)blockIdx.x * 64 + lane;
-  const int per_run = (slices + 3) / 4;
-  const int k0 = q * per_run, k1 = k0 + per_run < slices ? k0 + per_run : slices;
-  double s = 0.0;
-  if (i < per_slice)
-    for (int k = k0; k < k1; ++k) s += part[k * per_slice + i];
-  run[q][lane] = s;
-  __syncthreads();
-  if (q == 0 && i < per_slice) sums[i] = ((run[0][lane] + run[1][lane]) + run[2][lane]) + run[3][lane];
-}
-
+// multiple of 8).  The column sums come by slices of rows (fix_colsum_kernel) and are added in a fixed order by every workgroup, 64 columns of
+// NORM_ROWS rows, for itself.
+constexpr int NORM_ROWS = 256, NORM_SLICES = 64;
 template <typename TM, typename TQ>
-__global__ __launch_bounds__(256) void colscale_kernel(const TM* __restrict__ R, TM* __restrict__ qn, DaPtrTable qt,
-                                                       const double* __restrict__ sums, long long n, int r, int q_cols,
-                                                       float eps) {
-  const int b = blockIdx.y;
-  const TM* Rb = R + (long long)b * n;
-  TM* Qn = qn + (long long)b * n;
+__global__ __launch_bounds__(256) void colnorm_kernel(const TM* __restrict__ R, TM* __restrict__ qn, DaPtrTable qt,
+                                                      const double* __restrict__ sums, int slices, int rows, int r, int q_cols, float eps) {
+  __shared__ double run[4][64];
+  __shared__ float den[64];
+  const int b = blockIdx.z, lane = threadIdx.x & 63, q4 = threadIdx.x >> 6;
+  {
+    const int c = blockIdx.x * 64 + lane, per_run = (slices + 3) / 4;
+    const int k1 = (q4 + 1) * per_run < slices ? (q4 + 1) * per_run : slices;
+    double s = 0.0;
+    if (c < r)
+      for (int k = q4 * per_run; k < k1; ++k) s += sums[((long long)k * gridDim.z + b) * r + c];
+    run[q4][lane] = s;
+  }
+  __syncthreads();
+  if (q4 == 0) den[lane] = sqrtf((float)(((run[0][lane] + run[1][lane]) + run[2][lane]) + run[3][lane])) + eps;
+  __syncthreads();
+  const int c8 = (threadIdx.x & 7) * 8, col = blockIdx.x * 64 + c8;
+  if (col >= r) return;
+  const long long base = (long long)b * rows * r;
   TQ* Q = static_cast<TQ*>(qt.p[b]);
-  const double* sb = sums + (long long)b * r;
-  for (long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (long long)gridDim.x * 256 * 8) {
-    const int c0 = (int)(i % r);  // r is a multiple of 8: the 8 elements stay in one row
-    float v[8], q[8];
-    V8<TM>::load(Rb + i, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float d = sqrtf((float)sb[c0 + e]) + eps;
-      v[e] = V8<TM>::round(v[e] / d);     // cast back to R's dtype (reference dion/dion.py:1490)
-      q[e] = v[e];
+  // (the grid has a workgroup per NORM_ROWS rows up to the largest grid: beyond, each takes several)
+  for (long long i = (long long)blockIdx.y * NORM_ROWS + (threadIdx.x >> 3), in = 0; i < rows; i += 32, ++in) {
+    if (in && in % (NORM_ROWS / 32) == 0) {
+      i += ((long long)gridDim.y - 1) * NORM_ROWS;
+      if (i >= rows) break;
     }
-    V8<TM>::store(Qn + i, v);
+    const long long at = i * r + col;
+    float v[8];
+    V8<TM>::load(R + base + at, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = V8<TM>::round(v[e] / den[c8 + e]);     // cast back to R's dtype (reference dion/dion.py:1490)
+    V8<TM>::store(qn + base + at, v);
     // Q <- Q_new.to(Q.dtype) (reference dion/dion.py:1559-1561); the state has q_cols <= r columns, contiguous
     if (q_cols == r) {
-      V8<TQ>::store(Q + i, q);
+      V8<TQ>::store(Q + at, v);
     } else {
-      const long long row = i / r;
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        if (c0 + e < q_cols) st_from_float<TQ>(Q + row * q_cols + c0 + e, q[e]);
+        if (col + e < q_cols) st_from_float<TQ>(Q + i * q_cols + col + e, v[e]);
     }
   }
 }
@@ -324,60 +320,52 @@ int da_cast_table(const DaPtrTable& src, int s_dtype, void* dst, int d_dtype, in
   return da_launch_status();
 }
 
-int da_fix(void* v, const void* alt, int dtype, long long n, int batch, const int* nonzero, hipStream_t s) {
+int da_fix(void* v, int dtype, long long n, int batch, const int* nonzero, hipStream_t s) {
   if (n & 7) return DA_ERR_ALIGN;
   dim3 grid(ew_blocks(n), batch);
   if (dtype == DA_BF16)
-    hipLaunchKernelGGL(fix_kernel<bf16_t>, grid, dim3(256), 0, s, static_cast<bf16_t*>(v), static_cast<const bf16_t*>(alt), n, nonzero);
+    hipLaunchKernelGGL(fix_kernel<bf16_t>, grid, dim3(256), 0, s, static_cast<bf16_t*>(v), n, nonzero);
   else if (dtype == DA_F32)
-    hipLaunchKernelGGL(fix_kernel<float>, grid, dim3(256), 0, s, static_cast<float*>(v), static_cast<const float*>(alt), n, nonzero);
+    hipLaunchKernelGGL(fix_kernel<float>, grid, dim3(256), 0, s, static_cast<float*>(v), n, nonzero);
   else
     return DA_ERR_DTYPE;
   return da_launch_status();
 }
 
-int da_fix_sum(const float* part, int parts, long long pstride, void* v, const void* alt, int dtype, long long n,
-               int batch, const int* nonzero, hipStream_t s) {
-  if ((n & 7) || (pstride & 7) || parts < 1) return DA_ERR_ALIGN;
-  dim3 grid(ew_blocks(n), batch);
+namespace {
+// slices of rows of the column sums: 64 rows or more (two to a thread), enough of them to read R at the memory system's rate and few
+// enough for every workgroup of the normalisation to add them up
+int norm_slices(int rows) { return rows < 64 * NORM_SLICES ? (rows + 63) / 64 : NORM_SLICES; }
+}  // namespace
+
+int da_fix_colsum(const float* part, int parts, long long pstride, void* R, const void* alt, int dtype, int rows, int r, int batch,
+                  const int* nonzero, double* sums, hipStream_t s) {
+  if (r & 7) return DA_ERR_ALIGN;
+  const int slices = norm_slices(rows), rps = (rows + slices - 1) / slices;
+  const dim3 grid((r + 63) / 64, slices, batch);
   if (dtype == DA_BF16)
-    hipLaunchKernelGGL(fix_sum_kernel<bf16_t>, grid, dim3(256), 0, s, part, parts, pstride, static_cast<bf16_t*>(v), static_cast<const bf16_t*>(alt), n, nonzero);
+    hipLaunchKernelGGL(fix_colsum_kernel<bf16_t>, grid, dim3(256), 0, s, part, parts, pstride, static_cast<bf16_t*>(R), static_cast<const bf16_t*>(alt), rows, r, rps, nonzero, sums);
   else if (dtype == DA_F32)
-    hipLaunchKernelGGL(fix_sum_kernel<float>, grid, dim3(256), 0, s, part, parts, pstride, static_cast<float*>(v), static_cast<const float*>(alt), n, nonzero);
+    hipLaunchKernelGGL(fix_colsum_kernel<float>, grid, dim3(256), 0, s, part, parts, pstride, static_cast<float*>(R), static_cast<const float*>(alt), rows, r, rps, nonzero, sums);
   else
     return DA_ERR_DTYPE;
   return da_launch_status();
 }
 
 int da_colnorm(const void* R, void* qn, int m_dtype, const DaPtrTable& q, int q_dtype, int rows, int r, int q_cols,
-               float eps, int batch, double* sums, hipStream_t s) {
+               float eps, int batch, const double* sums, hipStream_t s) {
   if ((r & 7) || q_cols < 1 || q_cols > r) return DA_ERR_ALIGN;
-  const long long ns = (long long)batch * r;
-  // 64 rows per workgroup (16 per row group): enough workgroups to pull R at the memory system's rate
-  int slices = (rows + 63) / 64;
-  if (slices > 1024) slices = 1024;
-  const int rps = (rows + slices - 1) / slices;
-  double* part = sums + ns;   // [slices][batch][r]
-  dim3 g1((r + 63) / 64, slices, batch);
-  if (m_dtype == DA_BF16)
-    hipLaunchKernelGGL(colsum_kernel<bf16_t>, g1, dim3(256), 0, s, static_cast<const bf16_t*>(R), part, rows, r, rps);
-  else if (m_dtype == DA_F32)
-    hipLaunchKernelGGL(colsum_kernel<float>, g1, dim3(256), 0, s, static_cast<const float*>(R), part, rows, r, rps);
-  else
-    return DA_ERR_DTYPE;
-  hipLaunchKernelGGL(colsum_finish_kernel, dim3((unsigned)((ns + 63) / 64)), dim3(256), 0, s, part, sums, slices, ns);
-  const long long n = (long long)rows * r;
-  dim3 g2(ew_blocks(n), batch);
-  if (m_dtype == DA_BF16 && q_dtype == DA_BF16)
-    hipLaunchKernelGGL((colscale_kernel<bf16_t, bf16_t>), g2, dim3(256), 0, s, static_cast<const bf16_t*>(R), static_cast<bf16_t*>(qn), q, sums, n, r, q_cols, eps);
-  else if (m_dtype == DA_BF16 && q_dtype == DA_F32)
-    hipLaunchKernelGGL((colscale_kernel<bf16_t, float>), g2, dim3(256), 0, s, static_cast<const bf16_t*>(R), static_cast<bf16_t*>(qn), q, sums, n, r, q_cols, eps);
-  else if (m_dtype == DA_F32 && q_dtype == DA_BF16)
-    hipLaunchKernelGGL((colscale_kernel<float, bf16_t>), g2, dim3(256), 0, s, static_cast<const float*>(R), static_cast<float*>(qn), q, sums, n, r, q_cols, eps);
-  else if (m_dtype == DA_F32 && q_dtype == DA_F32)
-    hipLaunchKernelGGL((colscale_kernel<float, float>), g2, dim3(256), 0, s, static_cast<const float*>(R), static_cast<float*>(qn), q, sums, n, r, q_cols, eps);
-  else
-    return DA_ERR_DTYPE;
+  const int slices = norm_slices(rows);
+  const int blocks = (rows + NORM_ROWS - 1) / NORM_ROWS;
+  const dim3 grid((r + 63) / 64, blocks < 65535 ? blocks : 65535, batch);
+#define DA_COLNORM(TM, TQ) \
+  hipLaunchKernelGGL((colnorm_kernel<TM, TQ>), grid, dim3(256), 0, s, static_cast<const TM*>(R), static_cast<TM*>(qn), q, sums, slices, rows, r, q_cols, eps)
+  if (m_dtype == DA_BF16 && q_dtype == DA_BF16) DA_COLNORM(bf16_t, bf16_t);
+  else if (m_dtype == DA_BF16 && q_dtype == DA_F32) DA_COLNORM(bf16_t, float);
+  else if (m_dtype == DA_F32 && q_dtype == DA_BF16) DA_COLNORM(float, bf16_t);
+  else if (m_dtype == DA_F32 && q_dtype == DA_F32) DA_COLNORM(float, float);
+  else return DA_ERR_DTYPE;
+#undef DA_COLNORM
   return da_launch_status();
 }
 

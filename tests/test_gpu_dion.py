@@ -526,3 +526,24 @@ def test_orthonormalize_with_an_injected_sketch(dev, dtype, rows, r, batch):
         assert orth <= (ORTH_TOL if dtype == torch.float32 else 5e-2 * (r ** 0.5) / 8)
     with pytest.raises(ValueError):
         orthonormalize(Pd, sketch=S, qr_method="cqr")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n, r", [(72, 24), (264, 13), (4096, 72), (4200, 40)])
+def test_columns_of_q_have_unit_norm(dev, dtype, n, r):
+    """The column sums come in slices of 64 rows up to 4096 rows and of more beyond, the columns in blocks of 64, Q without the
+    working matrices' padding."""
+    from dion_amd import Dion, _lib
+
+    _lib.set_option("dion_small", 0)
+    try:
+        torch.manual_seed(3)
+        p = torch.nn.Parameter((torch.randn(n, n + 8, device=dev) * 0.02).to(dtype))
+        opt = Dion([p], lr=0.01, rank_fraction=(r - 0.5) / n, rank_multiple_of=1)
+        p.grad = torch.randn(n, n + 8, device=dev).to(dtype)
+        opt.step()
+        q = opt.state[p]["Q"].cpu().double()
+    finally:
+        _lib.set_option("dion_small", -1)
+    # every entry is rounded once, relatively by 2^-9 (2^-24 in fp32, and the norm and the division as well)
+    assert q.shape[1] == r and (q.norm(dim=0) - 1).abs().max() <= (2.0**-9 if dtype == torch.bfloat16 else 4 * 2.0**-24)
