@@ -660,15 +660,13 @@ size_t lay_out(GroupDev* D, const DaDionSmallGroup& g, const Shape& S, int msz, 
 // control memory: words of all matrices, the queues' lines, the status word's line, the pointer tables
 size_t control_bytes(int mats) { return up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4) + up256((size_t)3 * mats * 8); }
 
-// Matrices to queues: the costliest first, each to the queue with the least to do so far.  (Dealt in the order of the buckets, 14
-// matrices of 1021, 341 and 2731 rows / columns left two XCDs with a tenth of the others' work: 730 us, so 670.)  Returns the
-// work of the fullest queue in microseconds (see da_dion_small_bytes); queue[i] of matrix i, in the order of the groups.
-double deal(const DaDionSmallGroup* g, int n, bool bf, unsigned char* queue) {
-  double load[DA_QUEUES] = {0}, cost[DA_DS_GROUPS];
-  int sorted[DA_DS_GROUPS], first[DA_DS_GROUPS];
+// Matrices to queues: those with the longest factorisation first, each to the queue with the least to do so far; queue[i] of matrix i,
+// in the order of the groups.
+void deal(const DaDionSmallGroup* g, int n, unsigned char* queue) {
+  int load[DA_QUEUES] = {0}, cost[DA_DS_GROUPS], sorted[DA_DS_GROUPS], first[DA_DS_GROUPS];
   for (int i = 0, mats = 0; i < n; ++i) {
-    const Shape S(g[i].m, g[i].n, g[i].r, bf);
-    cost[i] = (double)S.mpT * S.npT * (bf ? 0.2 + 0.12 * S.rT : 0.25 + 0.25 * S.rT);
+    const int rT = (g[i].r + 63) / 64;
+    cost[i] = rT * rT;
     first[i] = mats;
     mats += g[i].cnt;
     int k = i;
@@ -681,11 +679,8 @@ double deal(const DaDionSmallGroup* g, int n, bool bf, unsigned char* queue) {
       for (int x = 1; x < DA_QUEUES; ++x)
         if (load[x] < load[q]) q = x;
       load[q] += cost[sorted[k]];
-      if (queue) queue[first[sorted[k]] + j] = (unsigned char)q;
+      queue[first[sorted[k]] + j] = (unsigned char)q;
     }
-  double worst = 0.0;
-  for (int q = 0; q < DA_QUEUES; ++q) worst = load[q] > worst ? load[q] : worst;
-  return worst;
 }
 
 template <bool BF>
@@ -721,15 +716,18 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
   if (!g || n < 1 || n > DA_DS_GROUPS) return 0;
   int mats = 0;
   size_t bytes = 0;
-  // Where the line lies, in microseconds.  One launch: the chain of phases (90 in bf16, 135 in fp32, 60 more per further block of
-  // 64 columns of rank, 100 for a factor as wide as the matrix, which takes FIX) and the tiles of the XCD with the most.  A launch
-  // per product: what the host takes to issue a few hundred of them, 2.5 times that with shapes off the 8-grid (padded
-  // copies), plus the products, in fp32 at a fifth of the bf16 rate.  Measured, one launch against many, layers of four d x d and
-  // two d x 4d: bf16 d 128 r 64: 95 / 400;  256 x4 r 128: 204 / 464;  512 x8 r 32: 366 / 528;  512 x8 r 128: 502 / 534;
-  // 768 x4 r 192: 703 / 506.  fp32 256 x4 r 128: 272 / 559;  768 x4 r 48: 643 / 948;  768 x12 r 192: 3121 / 2259.
+  // Where the line lies, in microseconds.  All buckets together: ten launches and the factorisation (45, and 35 per 64 columns of
+  // rank; 70 for a factor as wide as the matrix, which takes the second pass), and per 64 x 64 tile of a matrix its passes and its
+  // products.  A launch per product: what the host takes to issue a few hundred of them, 2.5 times that with shapes off the 8-grid
+  // (padded copies), plus the products.  Measured, together / by buckets, layers of four d x d and two d x 4d:
+  // bf16 128 x2 r 64: 74 / 503;  512 x8 r 128: 260 / 477;  512 x2 r 256: 245 / 518;  768 x1 r 192: 192 / 406;  768 x4 r 192: 360 / 508;
+  // 768 x12 r 48: 460 / 503;  1024 x1 r 256: 288 / 507;  1024 x4 r 64: 283 / 511;  2048 x1 r 63: 294 / 502;  256 x4 r 256: 280 / 484;
+  // and not: 768 x12 r 192: 1002 / 711;  1024 x4 r 256: 709 / 532 (2048 x1 r 256: 552 / 597 is given away);
+  // fp32 256 x4 r 128: 171 / 512;  768 x4 r 48: 406 / 944;  1024 x2 r 256: 1004 / 1416;  2048 x1 r 256: 1743 / 2445;  and not 768 x12 r 192:
+  // 2470 / 2345;  bf16 off the grid 1021 x4 r 255: 745 / 1863;  2043 x1 r 255: 585 / 960.
   const bool bf = c.m_dtype == DA_BF16;
   const int rows = gram_rows(g, n, bf);
-  double chain = 0.0, other = 0.0;
+  double chain = 0.0, work = 0.0, other = 0.0;
   bool padded = false, odd_full = false;
   for (int i = 0; i < n; ++i) {
     if (g[i].cnt < 1 || g[i].r < 1 || g[i].r > DA_DS_MAX_RANK || (long long)g[i].m * g[i].n > (1LL << 28) || (long long)g[i].m * g[i].n < 8) return 0;
@@ -739,9 +737,10 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
       if (((uintptr_t)g[i].M[j] | (uintptr_t)g[i].X[j]) & 127) return 0;
       if (((uintptr_t)g[i].G[j] | (uintptr_t)g[i].Q[j]) & 15) return 0;
     }
-    const double own = (bf ? 90.0 : 135.0) + 60.0 * (S.rT - 1) + (g[i].r == S.np ? 100.0 : 0.0);
+    const double own = 45.0 + 35.0 * S.rT + (g[i].r == S.np ? 70.0 : 0.0), tiles = (double)g[i].cnt * S.mpT * S.npT;
     chain = own > chain ? own : chain;
-    other += (bf ? 0.008 : 0.04) * g[i].cnt * S.mpT * S.npT * S.rT;
+    work += tiles * (bf ? 0.010 + 0.0085 * S.rT : 0.020 + 0.028 * S.rT);
+    other += tiles * S.rT * (bf ? 0.004 : 0.028);
     // (a full-rank factor of noise has a condition of 1e4 to 1e6, which multiplies every last-bit difference between the roads
     // from step to step; off the 8-grid, where the other road's second pass works on a padded rank, they do differ)
     odd_full |= g[i].r == S.np && (g[i].r & 7) != 0;
@@ -750,9 +749,8 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
     bytes += lay_out(nullptr, g[i], Shape(g[i].m, g[i].n, g[i].r, bf, rows), c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
   }
   if (mats > DA_DS_MATS) return 0;
-  const double worst = deal(g, n, bf, nullptr);
   other += (bf ? 400.0 : 480.0) * (padded ? 2.5 : 1.0);
-  if (!forced && (odd_full || chain + worst > other)) return 0;
+  if (!forced && (odd_full || chain + work > other)) return 0;
   return bytes + control_bytes(mats);
 }
 
@@ -775,7 +773,7 @@ int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, vo
   su.dst = reinterpret_cast<void**>(p + up256((size_t)mats * CTR_STRIDE * 4 + (DA_QUEUES + 1) * DA_QUEUE_LINE * 4));
   p += control_bytes(mats);
   unsigned char queue[DA_DS_MATS];
-  deal(g, n, c.m_dtype == DA_BF16, queue);
+  deal(g, n, queue);
   int first = 0, at = 0;
   long long adds = 0;
   const int rows = gram_rows(g, n, bf);

@@ -234,3 +234,15 @@ def test_numbers_of_stages_and_ragged_ends(dev, option, dtype, ms):
         option("dion_small", mode)
         runs.append(_run(dev, shapes, dtype, 0.5, 1, 2)[0])
     _agree(shapes, runs, 2e-5 if dtype == F32 else 1e-2)   # (as above)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("shapes, fraction", [
+    ([(768, 768)] * 4 + [(768, 3072), (3072, 768)], 0.25), ([(1024, 1024), (4096, 1024)], 0.25), ([(2048, 2048), (2048, 520)], 1 / 32)])
+def test_medium_matrices(dev, option, dtype, shapes, fraction):
+    """Widths and ranks up to where the rule takes all buckets together."""
+    runs = []
+    for mode in (0, -1):
+        option("dion_small", mode)
+        runs.append(_run(dev, shapes, dtype, fraction, 8, 2)[0])
+    _agree(shapes, runs, 2e-5 if dtype == F32 else 1e-2)   # (as above)
