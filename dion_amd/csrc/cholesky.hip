@@ -26,6 +26,142 @@ namespace {
 constexpr int NB = DA_CHOL_NB;
 constexpr int LP = DIAG_P;   // LDS pitch of the operand tiles: transposed stores stay nearly conflict-free
 
+// The fp64 block in sixteen steps of 4 columns.  diag_factor64 takes 8.2 us where this takes 14, but in another order of operations, and
+// this is the road of full-rank square factors: their next step multiplies a changed last bit by conditions of 1e9 and more, up to
+// whole elements of Q's last columns (12 layers of d 768 at rank 768 with it: 3610 us a step, 3690 so; the second step's Q off by
+// up to three times its elements' root mean square).  Factors of lower rank do not mind, nor the fp32 pass, which is polished.
+//
+// S and the inverse-in-progress Y live in matrix-core accumulators: wavefront w of the four holds tile row w (rows 16 w .. 16 w + 15) of
+// both as 16 x 16 tiles.  Right-looking with 4-wide block columns.  Per block step every wavefront reads the published block
+// column of S (64 x 4) and row block of Y (4 x 64) from LDS and repeats the serial part on its own SIMD instead of waiting for
+// one owner: the 4 x 4 diagonal factor (the same instructions in every lane), then lane = row forms its row of the L block column
+// by forward substitution and lane = column its column of X = L_cc^-1 Y_c (rows 4 cb .. 4 cb + 3 of the inverse, final after
+// this).  Both go to LDS as MFMA operands, the two rank-4 updates S -= L_c L_c^T, Y -= L_c X are v_mfma_f64_16x16x4 on the
+// wavefront's own tiles, and the wavefronts publish the next block column / row block.  One workgroup barrier per 4 columns; the
+// published blocks and the operands are double-buffered.  Arguments as diag_factor64's (live = keep = nb).
+template <typename Pivots>
+__device__ __forceinline__ void diag_by_fours(typename Mfma<double>::acc_t (&S)[4], double* work, double* dT, int nb, int lane, int wave, Pivots pivots) {
+  typedef double T;
+  typedef typename Mfma<T>::acc_t acc_t;
+  struct __attribute__((aligned(16))) quad_t { T v[4]; };
+  T* const scol = work;                                          // [2][4][NB]: published block column of S, [column][row]
+  quad_t* const yrow = reinterpret_cast<quad_t*>(work + 8 * NB); // [2][NB]: published row block of Y, [column] -> 4 rows
+  quad_t* const lops = yrow + 2 * NB;                            // [2][NB]: L block column as MFMA operand (0 in finished rows)
+  quad_t* const xops = lops + 2 * NB;                            // [2][NB]: X, [column] -> 4 rows
+  static_assert(8 * NB + 3 * 2 * NB * 4 <= DIAG_W, "the work area");
+  const int lc = lane & 15, lg = lane >> 4;
+  acc_t Y[4];
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Y[tj][v] = wave * 16 + Mfma<T>::row(v, lane) == tj * 16 + lc ? T(1) : T(0);
+  for (int e = wave * 64 + lane; e < 2 * NB; e += 256) {
+    // columns right of the diagonal tile of a row block are never published: they read as zero
+    quad_t z;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z.v[k] = T(0);
+    yrow[e] = z;
+  }
+  __syncthreads();
+  // block q (columns / rows 4 q .. 4 q + 3) of the current S and Y into buffer `buf`
+  auto publish = [&](int q, int buf) {
+    const int tq = q >> 2, qq = q & 3;
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {
+      if (tj == tq && tj <= wave && (lc >> 2) == qq) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) scol[(buf * 4 + (lc & 3)) * NB + wave * 16 + Mfma<T>::row(v, lane)] = S[tj][v];
+      }
+      if (wave == tq && tj <= wave) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int rr = Mfma<T>::row(v, lane);
+          if ((rr >> 2) == qq) yrow[buf * NB + tj * 16 + lc].v[rr & 3] = Y[tj][v];
+        }
+      }
+    }
+  };
+  publish(0, 0);
+  __syncthreads();
+  int bad = 0;                                     // first failed pivot (every lane computes the same)
+  T pmin = T(3e38), pmax = T(0);                   // smallest and largest usable pivot of this block column
+  for (int cb = 0; cb < NB / 4; ++cb) {
+    const int buf = cb & 1, k0 = cb * 4;
+    quad_t sv;                                    // lane = row: S[lane][k0 ..]
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sv.v[k] = scol[(buf * 4 + k) * NB + lane];
+    const quad_t yv = yrow[buf * NB + lane];       // lane = column: Y[k0 ..][lane]
+    T a[4][4];
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const quad_t d = *reinterpret_cast<const quad_t*>(&scol[(buf * 4 + jj) * NB + k0]);   // the same address in every lane
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) a[ii][jj] = d.v[ii];
+    }
+    // unblocked Cholesky of the 4 x 4 diagonal block: a[i][j], j < i becomes L_cc, di[] the inverse diagonal
+    T di[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const T p = a[c][c];
+      const bool ok = usable_pivot(p);
+      // 1/sqrt(p) from the hardware estimate (2^-27) plus Newton steps
+      T rs = ok ? rsqrt_seed<T>(p) : T(0);
+#pragma unroll
+      for (int it = 0; it < 2; ++it) rs = rs * (T(1.5) - T(0.5) * p * rs * rs);
+      di[c] = ok ? rs : T(0);
+      bad = (!ok && bad == 0 && k0 + c < nb) ? k0 + c + 1 : bad;
+      if (ok && k0 + c < nb) {
+        pmin = p < pmin ? p : pmin;
+        pmax = p > pmax ? p : pmax;
+      }
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i) a[i][c] *= di[c];
+#pragma unroll
+      for (int i = c + 1; i < 4; ++i)
+#pragma unroll
+        for (int j = c + 1; j <= i; ++j) a[i][j] -= a[i][c] * a[j][c];
+    }
+    // row `lane` of the L block column and column `lane` of X, by forward substitution with L_cc
+    T l[4], x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      T tl = sv.v[k], tx = yv.v[k];
+#pragma unroll
+      for (int m = 0; m < k; ++m) {
+        tl -= l[m] * a[k][m];
+        tx -= a[k][m] * x[m];
+      }
+      l[k] = tl * di[k];
+      x[k] = tx * di[k];
+    }
+    quad_t lo, xo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      lo.v[k] = lane > k0 + 3 ? l[k] : T(0);               // finished rows take no part in the updates
+      xo.v[k] = (lane <= k0 + k && k0 + k < nb) ? x[k] : T(0);
+    }
+    lops[buf * NB + lane] = lo;     // (every wavefront writes the same values; each reads back after its own writes)
+    xops[buf * NB + lane] = xo;
+    if (wave == (cb & 3)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dT[lane * LP + k0 + k] = lane < nb ? xo.v[k] : T(0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (wave * 16 + 15 > k0 + 3) {
+      const T aop = -lops[buf * NB + wave * 16 + lc].v[lg];
+#pragma unroll
+      for (int tj = 0; tj < 4; ++tj) {
+        if (tj <= wave && tj * 16 + 15 > k0 + 3) S[tj] = Mfma<T>::mma(aop, lops[buf * NB + tj * 16 + lc].v[lg], S[tj]);
+        if (tj <= wave && tj * 16 <= k0 + 3) Y[tj] = Mfma<T>::mma(aop, xops[buf * NB + tj * 16 + lc].v[lg], Y[tj]);
+      }
+    }
+    if (cb + 1 < NB / 4) publish(cb + 1, buf ^ 1);
+    __syncthreads();
+  }
+  if (wave == 0) pivots(bad, pmin, pmax);
+}
+
 template <typename T, bool INV>
 __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __restrict__ Lmat,
                                                         T* __restrict__ Tmat, long long sG, int r,
@@ -270,7 +406,7 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
   // (the two tiles of a T role would stay in registers through the whole factor loop: those are requested after it)
   const bool early = role < nroles && !(INV && role > below);
   if (early) fetch(role);
-  diag_factor64(S, op, dT, nb, nb, lane, wave, [&](int failed, T pmin, T pmax) {
+  auto pivots = [&](int failed, T pmin, T pmax) {
     if (wg != 0 || lane != 0) return;
     // (`fresh`: the first block column of a factorisation starts the matrix's status word)
     if (fresh || (failed != 0 && info[b] == 0)) info[b] = failed ? o + failed : 0;
@@ -283,7 +419,9 @@ __global__ __launch_bounds__(256) void chol_step_kernel(T* __restrict__ G, T* __
       pstat[2 * b] = pmin;
       pstat[2 * b + 1] = pmax;
     }
-  });
+  };
+  if constexpr (sizeof(T) == 8) diag_by_fours(S, op, dT, nb, lane, wave, pivots);
+  else diag_factor64(S, op, dT, nb, nb, lane, wave, pivots);
 
   // ---- the 64 x 64 x 64 products that depend on the factor: C[m][n] = sum_k opa[k][m] * opb[k][n]
   if (wg == 0) {

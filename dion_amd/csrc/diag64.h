@@ -1,4 +1,4 @@
-// The serial part of the blocked Cholesky factorisations (cholesky.hip, small_tile.h): a 64 x 64 diagonal block S = L L^T and
+// The serial part of the blocked Cholesky factorisations (cholesky.hip in fp32, small_tile.h): a 64 x 64 diagonal block S = L L^T and
 // T = L^-1 by one workgroup of four wavefronts, fp64 or fp32.
 //
 // What bounds it: the chain of 64 dependent columns -- pivot, reciprocal square root, one column of L, update of the next column --
@@ -12,7 +12,8 @@
 // Measured, one workgroup: fp64 19 800 cycles (8.2 us; 10 600 of them the columns), fp32 16 100 (6.7 us).  Sixteen steps of 4
 // columns, each with a round trip through LDS, a barrier and rank-4 updates of S and of the whole inverse, took 33 700 in
 // fp64, and 46 400 the first time (cold instruction cache; now 22 200): 24 fp32 matrices of 256 x 256 and
-// 256 x 1024 at rank 128 under Dion 241.9 -> 217.8 us a step; GPT-small's 72 at rank 192 725 -> 696 us, at rank 768 3959 -> 3764 us.
+// 256 x 1024 at rank 128 under Dion 241.9 -> 217.8 us a step; GPT-small's 72 at rank 192 725 -> 696 us.
+// (The fp64 steps of cholesky.hip keep their own, see there.)
 #pragma once
 #include "gemm_f64.h"
 
