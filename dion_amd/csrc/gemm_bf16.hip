@@ -401,11 +401,17 @@ int choose_tile(const GemmDesc* d, int n) {
   const double cost_small = launch_cost<Small>(d, n, 512, 3.0);
   const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
   if (d[0].symmetric && slide_ok(d, n)) {
-    long long mid = 0, small = 0;
-    for (int g = 0; g < n; ++g) { mid += tiles_of<Mid>(d[g]); small += tiles_of<Small>(d[g]); }
-    // (against 128-tiles two to a unit, which hide one another's epilogues, only where sliding computes little again)
-    const double other = big ? cost_big : small <= 256 || 2.25 * mid > 1.15 * small ? 0.75 * cost_small : cost_small;
-    if (launch_cost<Mid>(d, n, 256, 2.75) < other) return Mid::BT;
+    long long mid = 0, small = 0, matrices = 0;
+    for (int g = 0; g < n; ++g) { mid += tiles_of<Mid>(d[g]); small += tiles_of<Small>(d[g]); matrices += d[g].batch; }
+    const double cost_mid = launch_cost<Mid>(d, n, 256, 2.75);
+    if (big) {
+      // (several matrices over many rounds: 4 of 4096 x 10560, a round in twelve less by this count, were 1.4 % slower)
+      if (cost_mid * (mid > 512 && matrices > 1 ? 1.1 : 1.0) < cost_big) return Mid::BT;
+    } else if (small > 256 && 2.25 * mid <= 1.15 * small && cost_mid * (mid > 256 ? 1.13 : 1.0) < cost_small) {
+      // (128-tiles two to a unit hide one another's epilogues: only where sliding computes little again, and over several
+      // rounds, where a 192-tile's stage takes 1.12 us, only for a round less)
+      return Mid::BT;
+    }
   }
   return big ? 256 : 128;
 }
