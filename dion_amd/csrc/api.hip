@@ -1276,7 +1276,7 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
 }  // namespace
 
 namespace {
-// fills `g` from the caller's buckets; false: not for the one-launch kernel
+// fills `g` from the caller's buckets; false: not for the kernels of small matrices
 bool dion_small_groups(const dion_amd_dion_bucket* buckets, int n, DaDionSmallGroup* g) {
   if (!buckets || n < 1 || n > DA_DS_GROUPS) return false;
   for (int i = 0; i < n; ++i) {

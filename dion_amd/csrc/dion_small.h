@@ -1,10 +1,10 @@
-// Host-side interface of the small-matrix Dion kernel (dion_small.hip): the whole step of a set of small matrices in one
-// launch.
+// Host-side interface of the small-matrix Dion kernels (dion_small.hip): the whole step of a set of small matrices in ten
+// launches over all of them.
 #pragma once
 #include "common.h"
 
-constexpr int DA_DS_GROUPS = 8;          // buckets per launch
-constexpr int DA_DS_MATS = 96;           // matrices per launch (their pointers travel as arguments of the set-up launch)
+constexpr int DA_DS_GROUPS = 8;          // buckets together
+constexpr int DA_DS_MATS = 96;           // matrices together (their pointers travel as arguments of the set-up launch)
 constexpr int DA_DS_MAX_RANK = 256;
 
 // A bucket of `cnt` same-shape matrices: X, G, M (m x n, contiguous), Q (min(m, n) x r, contiguous), host arrays of device
@@ -24,7 +24,7 @@ struct DaDionSmallCall {
   int fail;   // test hook: start with the status word set
 };
 
-// Bytes of workspace, or 0 when the launch does not take these buckets (ranks, alignment of the matrices; `forced`: without
+// Bytes of workspace, or 0 when they do not take these buckets (ranks, alignment of the matrices; `forced`: without
 // the rule on the amount of work).
 size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, bool forced);
 int da_dion_small(const DaDionSmallGroup* g, int n, const DaDionSmallCall& c, void* workspace, hipStream_t s);

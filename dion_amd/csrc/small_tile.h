@@ -1,4 +1,4 @@
-// Tile products and the serial part of a factorisation for the one-launch kernels (dion_small.hip, orth_flow.hip): 256 threads,
+// Tile products and the serial part of a factorisation for the kernels of small matrices and flagged factors (dion_small.hip, orth_flow.hip): 256 threads,
 // operands from memory through registers into LDS, products on the matrix cores in bf16, fp32 and fp64.
 #pragma once
 #include "diag64.h"

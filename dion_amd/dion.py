@@ -6,7 +6,7 @@ arguments, defaults, validation errors, param-group keys and `self.state` layout
 `replicate_mesh`, `outer_shard_mesh` and `inner_shard_mesh` must be None.
 
 Per `step()` the matrices of every "dion" group are bucketed by (shape, dtype).  Buckets of small matrices go to
-`dion_amd_dion_step_buckets` together, the whole step as one launch (gathered natively, `_host.dion_group`).  Any other
+`dion_amd_dion_step_buckets` together, the whole step in ten launches (gathered natively, `_host.dion_group`).  Any other
 bucket goes, as arrays of device pointers, to `dion_amd_dion_step_qr`: B = M + G, the tall-skinny MFMA
 GEMMs P = B Q and R = B^T P, a CholeskyQR orthonormalisation of P on the device (an fp32 pass on the bf16 matrix
 cores, an fp64 pass for the factors whose measured defect asks for it, a closed-form polishing step; no host
