@@ -309,7 +309,7 @@ int dion_amd_dion_step_qr(void* const* X, const void* const* G, void* const* M, 
                           int power_iters, int qr_method,
                           int* info, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Several buckets of small matrices in one call and ONE launch (after a small set-up launch): replaces the task generator
+/* Several buckets of small matrices in one call, ten launches over all of them: replaces the task generator
  * and the task runtime around dion_update_ddp for a set of buckets (reference dion/dion.py:234-385, dion/opt_utils.py
  * AsyncRuntime).  Same update as dion_amd_dion_step with power_iters 1, orthonormaliser in fp64 throughout; any m, n, rank up
  * to 256; rows may have any length, X and M must be 128-byte aligned, G and Q 16-byte.
