@@ -210,11 +210,15 @@ __device__ __forceinline__ void staged_loop(int n, int full, Fetch fetch, Put pu
   }
   __syncthreads();
 }
-// how many of n stages, D deep from kbeg on, no chunk of which reaches past the operand's k (of a caller's matrix never the last one,
-// where a load may have been moved back; rows past its end are read as whatever lies there, and the caller drops their results)
+// how many of n stages, D deep from kbeg on, no chunk of which reaches past the operand's k or was loaded from another place than its
+// own (fetch_chunk moves a load that would pass the matrix's end back; rows past the operand's end are read as whatever lies there,
+// and the caller drops their results).  Of a caller's matrix the last stage never counts.  A k-strided chunk starts at k ld + row:
+// ahead of the last k it is moved only where k ld > m n - 8, which takes rows shorter than eight elements, and then the last 7 / ld
+// of the k before it are; they may lie in the stage before (ld = 3 and 65 k in stages of 64: k = 63).
 template <typename E> __device__ __forceinline__ int full_stages(const Opnd<E, false>&, int, int n, int) { return n; }
 template <typename E> __device__ __forceinline__ int full_stages(const Opnd<E, true>& o, int kbeg, int n, int D) {
-  return max(0, min(n - 1, (o.kmax - kbeg) / D));
+  const int own = o.ks && o.ld < 8 ? o.kmax - 7 / o.ld : o.kmax;   // the k whose chunks lie where they belong
+  return max(0, min(n - 1, (own - kbeg) / D));
 }
 
 // K loop of one TB x TB tile:  sum over k in [kbeg, kend) of A(row0 + i, k) B(col0 + j, k), for NB column operands; `mma`

@@ -246,3 +246,21 @@ def test_medium_matrices(dev, option, dtype, shapes, fraction):
         option("dion_small", mode)
         runs.append(_run(dev, shapes, dtype, fraction, 8, 2)[0])
     _agree(shapes, runs, 2e-5 if dtype == F32 else 1e-2)   # (as above)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("n, rank, ms", [
+    (3, 2, (65, 97, 129, 193, 257)),                    # (in bf16 stages of 64 k, in fp32 of 32)
+    (2, 1, (65, 66, 97, 98, 129, 130)),
+    (1, 1, (33, 39, 65, 71, 72, 135)),
+    (5, 3, (65, 129)), (7, 4, (97, 193)), (9, 5, (65, 129)),
+])
+def test_tall_matrices_of_a_few_columns(dev, option, dtype, n, rank, ms):
+    """B'^T P of matrices whose rows are shorter than the eight elements of a load: the loads of the last rows are moved back, also
+    where the last stage of the K loop is shorter than they are many."""
+    shapes, runs = [(m, n) for m in ms], []
+    for mode in (0, 1):
+        option("dion_small", mode)
+        runs.append(_run(dev, shapes, dtype, rank / n, 1, 1, mu=0.5)[0])
+        assert all(q.shape == (n, rank) for _, _, q in runs[-1])
+    _agree(shapes, runs, 2e-5 if dtype == F32 else 1e-2)   # (as above)
