@@ -366,7 +366,8 @@ typedef Cfg<256, 2, 4, 32> Big32;      // (GemmDesc::mi32)
 typedef Cfg<128, 2, 2, 32> Small32;
 
 // Whether 192 x 192 tiles can run: every operand at least a tile, whole stages, 32-bit offsets (as all_interior); the last tile of
-// a dimension is moved back over its neighbour, whose results it computes again, the same bits, so E must not be C.
+// a dimension is moved back over its neighbour, whose results it computes again, the same bits, so E must not be C.  (An E that is not
+// symmetric gives E(m, n) above the diagonal and on the diagonal tiles and E(n, m) elsewhere, as with the other tiles: epilogue_impl.)
 bool slide_ok(const GemmDesc* d, int n) {
   for (int g = 0; g < n; ++g) {
     if (!d[g].symmetric || d[g].M < Mid::BT || d[g].K % BK || d[g].Ctab || d[g].Etab || d[g].E == d[g].C) return false;

@@ -318,12 +318,16 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
     }
     if (SYM && mirror) {
       wave_sync_lds();
-      // C^T: row n of the mirrored tile holds 32 consecutive m of this band
+      // C^T: row n of the mirrored tile holds 32 consecutive m of this band.  Where sliding tiles overlap, what a diagonal tile stores
+      // (from E itself) is left to it: with E(m, n) here and E(n, m) there, an E that is not symmetric would leave either.
+      const int n_own = C::SLIDE && n0 + C::BT >= dN ? (dN - 1) / C::BT * C::BT : 0;
+      const int m_end = C::SLIDE ? dM - C::BT : 0;
 #pragma unroll
       for (int pass = 0; pass < (W + 63) / 64 * 4; ++pass) {
         const int nl = (pass >> 2) * 64 + lane;
         const int mg = (pass & 3) * 8;
         const int n = wn0 + nl, m = band_m + mg;
+        if (C::SLIDE && (n < n_own || m >= m_end)) continue;
         if ((FULL || (n < dN && m < dM)) && (W % 64 == 0 || nl < W)) {  // M is a multiple of 8 for symmetric outputs
           float v[8];
 #pragma unroll

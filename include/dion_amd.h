@@ -101,7 +101,9 @@ int dion_amd_syrk(const void* A, long long a_stride, int lda,
                   int batch, int m, int k, int dtype, void* stream);
 
 /* Replaces ns_line_2 (reference dion/newton_schulz_triton.py:261-302):
- * C_b = alpha * A_b A_b^T + beta * A_b for symmetric A_b (m x m). */
+ * C_b = alpha * A_b A_b^T + beta * A_b for symmetric A_b (m x m).  The tiles above and on the
+ * diagonal are computed, the others mirrored: of an A_b that is not symmetric the addend of an
+ * element below the diagonal is that element or its mirror image, depending on the tile size. */
 int dion_amd_sym_poly(const void* A, long long a_stride, int lda,
                       void* C, long long c_stride, int ldc,
                       int batch, int m, float alpha, float beta,

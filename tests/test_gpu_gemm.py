@@ -142,3 +142,19 @@ def test_symmetric_products_in_tiles_that_slide(dev, batch, m, k):
         if batch > 1:
             assert torch.equal(ns_line_1(A[b]), got[b])
             assert m % 64 or torch.equal(ns_line_2(got[b], alpha=0.5, beta=-1.5), got2[b])
+
+
+@pytest.mark.parametrize("m", [2944, 3008, 4096])
+def test_ns_line_2_of_a_matrix_that_is_not_symmetric(dev, m):
+    """Sizes whose 192-tiles overlap at the end of the matrix: no element may depend on which of two tiles stores last.  Above the
+    diagonal and on the diagonal tiles the addend is the element itself, elsewhere its mirror image."""
+    from dion_amd.newton_schulz import ns_line_2
+
+    torch.manual_seed(5)
+    A = torch.randn(m, m).bfloat16()
+    block = torch.arange(m) // 192
+    row, col = block[:, None], block[None, :]
+    own = (row <= col) | ((torch.arange(m)[:, None] >= m - 192) & (torch.arange(m)[None, :] >= m - 192))
+    want = torch.where(own, A, A.mT)
+    for _ in range(3):
+        assert torch.equal(ns_line_2(A.to(dev), alpha=0.0, beta=1.0).cpu(), want)
