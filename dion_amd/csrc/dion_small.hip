@@ -722,13 +722,14 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
   // (padded copies), plus the products.  Measured, together / by buckets, layers of four d x d and two d x 4d:
   // bf16 128 x2 r 64: 74 / 503;  512 x8 r 128: 260 / 477;  512 x2 r 256: 245 / 518;  768 x1 r 192: 192 / 406;  768 x4 r 192: 360 / 508;
   // 768 x12 r 48: 460 / 503;  1024 x1 r 256: 288 / 507;  1024 x4 r 64: 283 / 511;  2048 x1 r 63: 294 / 502;
-  // and not: 768 x12 r 192: 1002 / 711;  1024 x4 r 256: 709 / 532 (2048 x1 r 256: 552 / 597 and 256 x4 r 256: 280 / 484 are given away);
+  // 256 x4 r 256: 287 / 506;  200 x1 r 200: 184 / 485;  four of 256 x 256 alone r 256: 193 / 269;  and not: 768 x12 r 192: 1002 / 711;
+  // 1024 x4 r 256: 709 / 532 (2048 x1 r 256: 552 / 597 is given away);
   // fp32 256 x4 r 128: 171 / 512;  768 x4 r 48: 406 / 944;  1024 x2 r 256: 1004 / 1416;  2048 x1 r 256: 1743 / 2445;  and not 768 x12 r 192:
   // 2470 / 2345;  bf16 off the grid 1021 x4 r 255: 745 / 1863;  2043 x1 r 255: 585 / 960.
   const bool bf = c.m_dtype == DA_BF16;
   const int rows = gram_rows(g, n, bf);
   double chain = 0.0, work = 0.0, other = 0.0;
-  bool padded = false, odd_full = false, wide_full = false;
+  bool padded = false, odd_full = false;
   for (int i = 0; i < n; ++i) {
     if (g[i].cnt < 1 || g[i].r < 1 || g[i].r > DA_DS_MAX_RANK || (long long)g[i].m * g[i].n > (1LL << 28) || (long long)g[i].m * g[i].n < 8) return 0;
     const Shape S(g[i].m, g[i].n, g[i].r, c.m_dtype == DA_BF16);
@@ -741,18 +742,18 @@ size_t da_dion_small_bytes(const DaDionSmallGroup* g, int n, const DaDionSmallCa
     chain = own > chain ? own : chain;
     work += tiles * (bf ? 0.010 + 0.0085 * S.rT : 0.020 + 0.028 * S.rT);
     other += tiles * S.rT * (bf ? 0.004 : 0.028);
-    // (a full-rank factor of noise has a condition of 1e4 to 1e6, which multiplies every last-bit difference between the roads
-    // from step to step; off the 8-grid, where the other road's second pass works on a padded rank, they do differ, and in bf16
-    // beyond 192 columns a flipped rounding comes back two steps later as whole elements of Q's last columns)
+    // (A full-rank factor of noise has a condition of 1e4 to 1e6, which multiplies every last-bit difference between the roads from step
+    // to step.  Off the 8-grid the other road's second pass works on a padded rank, and such factors stay with it.  On the grid
+    // neither road is the closer one to a step in 64 bits: 4 of 256 x 256 in bf16, first and third step, error of Q 7.95e-2 and
+    // 4.76e-2 on both, the digits that differ are the fifth and later.)
     odd_full |= g[i].r == S.np && (g[i].r & 7) != 0;
-    wide_full |= bf && g[i].r == S.np && S.rT > 3;
     padded |= ((g[i].m | g[i].n) & 7) != 0;
     mats += g[i].cnt;
     bytes += lay_out(nullptr, g[i], Shape(g[i].m, g[i].n, g[i].r, bf, rows), c.m_dtype == DA_BF16 ? 2 : 4, nullptr);
   }
   if (mats > DA_DS_MATS) return 0;
   other += (bf ? 400.0 : 480.0) * (padded ? 2.5 : 1.0);
-  if (!forced && (odd_full || (wide_full && !padded) || chain + work > other)) return 0;
+  if (!forced && (odd_full || chain + work > other)) return 0;
   return bytes + control_bytes(mats);
 }
 

@@ -229,3 +229,29 @@ def test_generate_random_sketch_matrix_shape_and_scale():
         generate_random_sketch_matrix(torch.zeros(10, 4))
     with pytest.raises(TypeError):
         generate_random_sketch_matrix(torch.zeros(1, 10, 4), shard_mesh_dim=0)
+
+
+@pytest.mark.parametrize("shapes, together", [
+    ([(200, 200)] * 4 + [(800, 200), (200, 800)], True),            # full rank beyond 192 columns, on the 8-grid
+    ([(256, 256)] * 4, True),
+    ([(256, 512), (512, 256)], True),
+    (([(256, 256)] * 4 + [(1024, 256), (256, 1024)]) * 4, True),
+    ([(201, 201)] * 4, False),                                      # off the grid
+    ([(264, 264)] * 4, False),                                      # beyond the ranks that are taken together
+    (([(256, 256)] * 2 + [(4096, 256)] * 10) * 8, False),           # more work than the launches together are faster for
+])
+def test_full_rank_bf16_factors_go_together_by_their_work(shapes, together):
+    """Whether a set of buckets is stepped together is asked without a GPU; the pointers are only looked at for alignment."""
+    import ctypes
+
+    from dion_amd import _lib
+
+    sets = {s: shapes.count(s) for s in shapes}
+    buckets, held = (_lib.DionBucket * len(sets))(), []
+    for bucket, ((m, n), count) in zip(buckets, sets.items()):
+        pointers = (ctypes.c_void_p * count)(*[4096 * (i + 1) for i in range(count)])
+        held.append(pointers)
+        bucket.X = bucket.G = bucket.M = bucket.Q = pointers
+        bucket.batch, bucket.m, bucket.n, bucket.r = count, m, n, min(m, n)
+    bf, f32 = _lib.dtype_code(torch.bfloat16), _lib.dtype_code(torch.float32)
+    assert (_lib.load().dion_amd_dion_buckets_workspace_bytes(buckets, len(sets), bf, bf, bf, f32) > 0) == together
