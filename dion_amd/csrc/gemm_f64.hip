@@ -338,7 +338,8 @@ int launch(const RealGemmDesc<T>& d, hipStream_t s) {
 // 768 x 768: 585 us, 40 TFLOP/s; as fifteen products over panels of four block columns (1 launch each) 570 us plus 85 us for the
 // blocks of the panels' inverses, which are no longer needed; and as the pass over flagged matrices one launch that finds
 // nothing instead of one per block column.  (Four workgroups a compute unit: 618.)
-// Workgroups of one matrix stay on one XCD (they read the same L) once there are eight matrices.
+// Eight matrices at a time go to the eight XCDs (a matrix's workgroups read the same L), the up to seven that are left to all of them:
+// to one XCD each they left the others idle (12 matrices of 3072 x 768: the whole orthonormaliser 1628 us, so 1508; 9: 1482 / 1284).
 constexpr int SR = 32;
 template <typename T, bool INTERIOR>
 __device__ __forceinline__ void solve_rows_of(T* __restrict__ P, const T* __restrict__ L, const T* __restrict__ D, int rows, int r, int row0,
@@ -441,20 +442,17 @@ __device__ __forceinline__ void solve_rows_of(T* __restrict__ P, const T* __rest
 
 template <typename T>
 __global__ __launch_bounds__(256, 5) void solve_rows_kernel(T* __restrict__ Pm, const T* __restrict__ Lm, const T* __restrict__ Dm, int rows,
-                                                         int r, int batch, int blocks, int spread, const int* gate, int gate_want) {
+                                                         int r, int batch, int blocks, const int* gate, int gate_want) {
   __shared__ __attribute__((aligned(16))) T lds[2 * 128 * (SR + 64) / sizeof(T)];
   static_assert(2 * 128 * (SR + 64) / sizeof(T) >= 64 * SR && 128 / sizeof(T) >= RK, "room for the difference and for the stages of the checked loop");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int b, blk;
-  if (spread) {
-    b = blockIdx.x / blocks;
-    blk = blockIdx.x - b * blocks;
-  } else {
+  int b = blockIdx.x / blocks, blk = blockIdx.x - b * blocks;
+  if ((int)blockIdx.x < (batch & ~7) * blocks) {
     const int idx = blockIdx.x >> 3, m = idx / blocks;
     b = m * 8 + (blockIdx.x & 7);
     blk = idx - m * blocks;
   }
-  if (b >= batch || (gate && (gate[b] != 0) != (gate_want != 0))) return;
+  if (gate && (gate[b] != 0) != (gate_want != 0)) return;
   T* const P = Pm + (long long)b * rows * r;
   const T* const L = Lm + (long long)b * r * r;
   const T* const D = Dm + (long long)b * r * r;
@@ -468,10 +466,9 @@ template <typename T>
 int solve_rows(T* P, const T* L, const T* D, int batch, int rows, int r, DaGate g, hipStream_t s) {
   if (!P || !L || !D || batch <= 0 || rows <= 0 || r <= 0) return DA_ERR_ARG;
   const int blocks = (rows + SR - 1) / SR;
-  const int spread = batch < 8 ? 1 : 0;
-  const long long grid = (long long)blocks * (spread ? batch : (batch + 7) / 8 * 8);
+  const long long grid = (long long)blocks * batch;
   if (grid > 0x7fffffffLL) return DA_ERR_LIMIT;
-  hipLaunchKernelGGL(solve_rows_kernel<T>, dim3((unsigned)grid), dim3(256), 0, s, P, L, D, rows, r, batch, blocks, spread, g.flags, g.want);
+  hipLaunchKernelGGL(solve_rows_kernel<T>, dim3((unsigned)grid), dim3(256), 0, s, P, L, D, rows, r, batch, blocks, g.flags, g.want);
   return da_launch_status();
 }
 

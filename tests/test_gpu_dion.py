@@ -129,6 +129,19 @@ def test_orthonormalize_batch_and_rank_deficient(dev):
     assert torch.equal(orthonormalize(P[0].to(dev)), Q[0])
 
 
+@pytest.mark.parametrize("batch", [1, 7, 8, 9, 12, 17])
+def test_orthonormalize_deals_any_number_of_matrices(dev, batch):
+    """The fp64 pass over whole and broken groups of eight matrices (its triangular solve deals them to the XCDs by eights)."""
+    from dion_amd.newton_schulz import orthonormalize
+
+    torch.manual_seed(6)
+    P = torch.randn(batch, 200, 72)
+    Q = orthonormalize(P.to(dev), qr_method="qr").double().cpu()
+    for q, p in zip(Q, P):
+        ref = torch.linalg.qr(p.double())[0]
+        assert rel_fro(_sign_align(q, ref), ref) <= 1e-6      # cond(P) = 4: fp64 throughout, rounded once to fp32 (6e-8)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_orthonormalize_numerically_rank_deficient(dev, dtype):
     """P = A B of rank 96 < r = 128: the dependent columns have pivots at round-off level of either sign.  They must
