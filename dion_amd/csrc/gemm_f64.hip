@@ -140,34 +140,35 @@ __device__ __forceinline__ void fetch(T (&v)[4], const T* __restrict__ base, int
   }
 }
 
-// One 64-row slice of a stage goes to the k-major LDS tile lds[k][row] (row pitch BTt).
-template <bool KS, int BTt, typename T>
+// A stage goes to the k-major LDS tile lds[k][row] (row pitch P).
+template <bool KS, int P, typename T>
 __device__ __forceinline__ void put(T* lds, const T (&v)[4], int tid) {
   if (!KS) {
     const int r = tid >> 2, k4 = (tid & 3) * 4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) lds[(k4 + e) * BTt + r] = v[e];
+    for (int e = 0; e < 4; ++e) lds[(k4 + e) * P + r] = v[e];
   } else {
     const int k = tid >> 4, r4 = (tid & 15) * 4;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) lds[k * BTt + r4 + e] = v[e];
+    for (int e = 0; e < 4; ++e) lds[k * P + r4 + e] = v[e];
   }
 }
 
-// BTt x BTt output tile, 256 threads as 2 x 2 wavefronts of (BTt / 2) x (BTt / 2) each.
-template <typename T, bool A_KS, bool B_KS, bool SYM, int BTt>
+// BT x BT output tile, 256 threads as 2 x 2 wavefronts of (BT / 2) x (BT / 2) each.  (Tiles of 128 -- half the operand bytes per flop, but
+// 200 VGPRs and 64 KB of LDS in fp64, two workgroups per CU instead of five -- were 10 % slower on the orthonormaliser's large
+// products and equal on the small ones.)
+constexpr int BT = 64;
+template <typename T, bool A_KS, bool B_KS, bool SYM>
 __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
   typedef typename Mfma<T>::acc_t acc_t;
-  constexpr int H = BTt / 64;        // 64-row slices per operand stage
-  constexpr int WT = BTt / 2;        // wavefront tile
+  constexpr int WT = BT / 2;         // wavefront tile
   constexpr int TI = WT / 16;        // 16 x 16 accumulators per wavefront and direction
-  static_assert(BTt == 64, "the tile of the K loop");
   __shared__ __attribute__((aligned(16))) char lds[2 * 128 * 128];
   T* const lds_a = reinterpret_cast<T*>(lds);
-  T* const lds_b = lds_a + 2 * RK * BTt;
+  T* const lds_b = lds_a + 2 * RK * BT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int tiles_m = (d.M + BTt - 1) / BTt, tiles_n = (d.N + BTt - 1) / BTt;
+  const int tiles_m = (d.M + BT - 1) / BT, tiles_n = (d.N + BT - 1) / BT;
   const bool tri = SYM || d.lower_only;
   // SYM: M == N; lower_only: M >= N, column tile c holds the tiles_m - c row tiles from the diagonal down
   const int per_batch = tri ? tiles_n * tiles_m - tiles_n * (tiles_n - 1) / 2 : tiles_m * tiles_n;
@@ -190,10 +191,10 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
     ti = t / tiles_n;
     tj = t - ti * tiles_n;
   }
-  const int m0 = ti * BTt, n0 = tj * BTt;
+  const int m0 = ti * BT, n0 = tj * BT;
   const T* A = d.A + (long long)b * d.sA;
   const T* B = d.B + (long long)b * d.sB;
-  const int Keff = d.k_tri && n0 + BTt < d.K ? n0 + BTt : d.K;
+  const int Keff = d.k_tri && n0 + BT < d.K ? n0 + BT : d.K;
 
   acc_t acc[TI][TI];
 #pragma unroll
@@ -206,32 +207,28 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
   const int per_split = (KT_all + (int)gridDim.y - 1) / (int)gridDim.y;
   const int kt0 = split * per_split;
   const int KT = KT_all - kt0 < per_split ? KT_all - kt0 : per_split;   // may be <= 0 for the last slices
-  T pa[H][4], pb[H][4];
+  T pa[4], pb[4];
 #define DA_RFETCH(kt)                                                                               \
   do {                                                                                              \
-    _Pragma("unroll") for (int h = 0; h < H; ++h) {                                                 \
-      fetch<A_KS>(pa[h], A, d.lda, m0 + 64 * h, (kt) * RK, d.M, Keff, tid);                         \
-      fetch<B_KS>(pb[h], B, d.ldb, n0 + 64 * h, (kt) * RK, d.N, Keff, tid);                         \
-    }                                                                                               \
+    fetch<A_KS>(pa, A, d.lda, m0, (kt) * RK, d.M, Keff, tid);                                       \
+    fetch<B_KS>(pb, B, d.ldb, n0, (kt) * RK, d.N, Keff, tid);                                       \
   } while (0)
 #define DA_RPUT(buf)                                                                                \
   do {                                                                                              \
-    _Pragma("unroll") for (int h = 0; h < H; ++h) {                                                 \
-      put<A_KS, BTt>(lds_a + (buf) * RK * BTt + 64 * h, pa[h], tid);                                              \
-      put<B_KS, BTt>(lds_b + (buf) * RK * BTt + 64 * h, pb[h], tid);                                              \
-    }                                                                                               \
+    put<A_KS, BT>(lds_a + (buf) * RK * BT, pa, tid);                                                \
+    put<B_KS, BT>(lds_b + (buf) * RK * BT, pb, tid);                                                \
   } while (0)
 #define DA_RMMA(sa, sb)                                                                             \
   _Pragma("unroll") for (int ks = 0; ks < RK / 4; ++ks) {                                           \
     const int k = ks * 4 + (lane >> 4);                                                             \
     T af[TI], bfv[TI];                                                                              \
-    _Pragma("unroll") for (int i = 0; i < TI; ++i) af[i] = (sa)[k * BTt + wm * WT + i * 16 + (lane & 15)];  \
-    _Pragma("unroll") for (int j = 0; j < TI; ++j) bfv[j] = (sb)[k * BTt + wn * WT + j * 16 + (lane & 15)]; \
+    _Pragma("unroll") for (int i = 0; i < TI; ++i) af[i] = (sa)[k * BT + wm * WT + i * 16 + (lane & 15)];  \
+    _Pragma("unroll") for (int j = 0; j < TI; ++j) bfv[j] = (sb)[k * BT + wn * WT + j * 16 + (lane & 15)]; \
     _Pragma("unroll") for (int i = 0; i < TI; ++i)                                                  \
       _Pragma("unroll") for (int j = 0; j < TI; ++j) acc[i][j] = Mfma<T>::mma(af[i], bfv[j], acc[i][j]);    \
   }
   // Interior tile with 16-byte aligned operand rows, whole stages, operands within reach of the loads' 32-bit offsets
-  const bool interior = m0 + BTt <= d.M && n0 + BTt <= d.N && Keff % Ring<T>::D == 0 && kt0 * RK % Ring<T>::D == 0 && KT * RK % Ring<T>::D == 0 &&
+  const bool interior = m0 + BT <= d.M && n0 + BT <= d.N && Keff % Ring<T>::D == 0 && kt0 * RK % Ring<T>::D == 0 && KT * RK % Ring<T>::D == 0 &&
                         ring_span<T, A_KS>(d.lda, Keff) && ring_span<T, B_KS>(d.ldb, Keff) &&
                         ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 &&
                         (((long long)d.lda | (long long)d.ldb) * (long long)sizeof(T)) % 16 == 0;
@@ -245,8 +242,8 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
     }
     __syncthreads();
     for (int kt = 0; kt < KT; ++kt) {
-      const T* sa = lds_a + (kt & 1) * RK * BTt;
-      const T* sb = lds_b + (kt & 1) * RK * BTt;
+      const T* sa = lds_a + (kt & 1) * RK * BT;
+      const T* sb = lds_b + (kt & 1) * RK * BT;
       const bool more = kt + 1 < KT;
       if (more) DA_RFETCH(kt0 + kt + 1);
       DA_RMMA(sa, sb)
@@ -297,32 +294,22 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(RealGemmDesc<T> d) {
       }
 }
 
-template <typename T, int BTt>
+template <typename T>
 long long blocks_of(const RealGemmDesc<T>& d) {
-  const long long tiles_m = (d.M + BTt - 1) / BTt, tiles_n = (d.N + BTt - 1) / BTt;
+  const long long tiles_m = (d.M + BT - 1) / BT, tiles_n = (d.N + BT - 1) / BT;
   return ((d.symmetric || d.lower_only) ? tiles_n * tiles_m - tiles_n * (tiles_n - 1) / 2 : tiles_m * tiles_n) * d.batch;
-}
-
-template <typename T, bool A_KS, bool B_KS, bool SYM, int BTt>
-int launch_bt(const RealGemmDesc<T>& d, int split, hipStream_t s) {
-  const long long blocks = blocks_of<T, BTt>(d);
-  if (blocks <= 0 || blocks > 0x7fffffffLL) return DA_ERR_LIMIT;
-  hipLaunchKernelGGL((gemm_f64_kernel<T, A_KS, B_KS, SYM, BTt>), dim3((unsigned)blocks, split), dim3(256), 0, s, d);
-  return da_launch_status();
 }
 
 template <typename T, bool A_KS, bool B_KS, bool SYM>
 int launch(const RealGemmDesc<T>& d, hipStream_t s) {
-  // Only the 64-wide tile is instantiated: the 128-wide one (half the operand bytes per flop, but 200 VGPRs
-  // and 64 KB of LDS in fp64, i.e. two workgroups per CU instead of five) measured 10 % slower on the
-  // orthonormaliser's large products and equal on the small ones.
-  constexpr int BTt = 64;
-  const long long blocks = blocks_of<T, BTt>(d);
+  const long long blocks = blocks_of(d);
   const bool auto_split = d.split_k < 0 && !d.E && d.c_store == DA_STORE_NATIVE;
   int split = d.split_k > 1 && !d.E ? d.split_k : 1;
   if (auto_split) split = da_auto_split(blocks, d.K);
   if (split > 1 && d.split_stride < (long long)d.sC * d.batch) return DA_ERR_ARG;
-  return launch_bt<T, A_KS, B_KS, SYM, BTt>(d, split, s);
+  if (blocks <= 0 || blocks > 0x7fffffffLL) return DA_ERR_LIMIT;
+  hipLaunchKernelGGL((gemm_f64_kernel<T, A_KS, B_KS, SYM>), dim3((unsigned)blocks, split), dim3(256), 0, s, d);
+  return da_launch_status();
 }
 
 // ---- P <- P R^-1 with R = L^T: all block columns in one launch -------------------------------------------------------------
