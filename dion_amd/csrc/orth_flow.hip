@@ -214,7 +214,7 @@ int da_orth_flow_slices(int rows, int r) {
 }
 
 // Where the line lies: a flagged matrix has one XCD to itself at best, the launches per product the whole chip.  A full-rank
-// factor of a fresh Q is flagged (12 of 3072 x 768 each in two buckets: 13.4 ms a step in one launch, 7.4 ms in many), so the
+// factor of a fresh Q is flagged (12 of 3072 x 768 each in two buckets: 13.4 ms a step in one launch, 6.8 ms in many), so the
 // work per matrix is kept to what one XCD does in about half a millisecond.
 bool da_orth_flow_applicable(int rows, int r) {
   return (r + 63) / 64 <= MAX_RT && (long long)rows * r >= 8 && (double)rows * r * r <= 4e8;
