@@ -5,7 +5,7 @@
 //
 // What bounds it: as a sequence of launches a bucket takes 40 to 60 of them (a third of which only find out that the fp64
 // pass of the orthonormaliser is not needed), each a few microseconds of work: a model of 24 matrices of 256 x 256 and
-// 256 x 1024 spent 0.6-0.8 ms, most of it on the host; here 0.18 ms for ten launches, of which the factorisation, a chain of
+// 256 x 1024 spent 0.6-0.8 ms, most of it on the host; here 0.17 ms for ten launches, of which the factorisation, a chain of
 // 64-column steps, takes a third.
 //
 // Launches, each over all tiles of all matrices, at as many workgroups to a compute unit as its own registers and LDS allow:
@@ -26,7 +26,8 @@
 // All but CHAIN used to be phases of the queues: two workgroups to a compute unit (the factorisation's registers), a matrix's tiles on
 // one XCD's 64 workgroups, and a ticket and a counter for every tile.  14 bf16 matrices of 341 to 2731 rows at rank 256 and 86 (us,
 // as phases / as launches): set-up 98 / 24, BQ 52 / 31, GRAM 62 / 41, PT 62 / 59, FIX 16 / 9, BTP 48 / 41, CNORM 7 / 9, UPD 155 / 67;
-// the step 622 / 416, by now 385.  24 fp32 matrices of 256 x 256 and 256 x 1024 at rank 128: 218 / 196, by now 185.
+// the step 622 / 416, by now 407 (several states in turn; 385 on one).  24 fp32 matrices of 256 x 256 and 256 x 1024 at rank 128: 218 / 196,
+// by now 188 with the element-wise groups.
 // The orthonormaliser is the fp64 CholeskyQR of dion.hip for every matrix: at these sizes the fp64 products cost less than
 // the launches of the two-precision road.  P, R and the products with B run on the matrix cores in the momentum's dtype with
 // the instructions and the order of k of the batched kernels (v_mfma_f32_16x16x32_bf16, in the updates v_mfma_f32_32x32x16_bf16; v_mfma_f32_32x32x2_f32).

@@ -1,4 +1,4 @@
-"""The one-launch Dion kernel for small matrices (reference dion/dion.py:742-875) against the bucket-by-bucket launches (option
+"""The Dion step of small matrices taken together, ten launches over all of them (reference dion/dion.py:742-875), against the bucket-by-bucket launches (option
 "dion_small" = 0), which the oracle checks: shapes around the 32 / 64 tile edges, ranks around the blocks of the factorisation,
 rows off every alignment, more and fewer matrices than queues, zero and rank-deficient gradients."""
 import pytest
