@@ -4,14 +4,12 @@
 //
 //   C[b] (M x N) = epilogue( sum_k Aop[b](i,k) * Bop[b](j,k) )
 //
-// Work decomposition: one workgroup per BT x BT output tile.  Two shapes are built:
-//   * BT = 256, 8 wavefronts (2 x 4): each wavefront owns 128 x 64 as 8 x 4 accumulator blocks of
-//     16 x 16 (4 x 2 of 32 x 32 in the other form).  Two wavefronts share a SIMD, so while one waits
-//     for LDS or a barrier the other keeps the matrix core busy; LDS traffic is 12 fragment reads per
-//     32 MFMAs of a 32-deep k-step.
-//   * BT = 128, 4 wavefronts (2 x 2), 64 x 64 each: for problems too small to fill the
-//     256 CUs with large tiles.
-// The K loop advances 64 elements per stage and is double buffered through LDS.
+// Work decomposition: one workgroup of four wavefronts (2 x 2) per BT x BT output tile:
+//   * BT = 256, a CU each: 128 x 128 per wavefront as 8 x 8 accumulator blocks of 16 x 16, so that LDS is read for 128 KB a
+//     stage (eight wavefronts of 128 x 64, as the bounds-checked form and GemmDesc::mi32 have them, read 192 KB and are bound by it).
+//   * BT = 192, symmetric products, a CU each.
+//   * BT = 128, two to a CU: for problems too small to fill the 256 CUs with large tiles.
+// The K loop advances 64 elements per stage and is double buffered through LDS (gemm_tile_k_loop_quad).
 //
 // Operand staging in LDS:
 //   * k-contiguous operand (rows x K in memory): tile [BT][64] of 16-byte chunks, chunk
@@ -23,7 +21,7 @@
 //     fragment is fetched with two ds_read_b64_tr_b16 (the LDS transpose read of CDNA4),
 //     which hands each lane the four k-consecutive values of its own column.  No register
 //     shuffles, no second copy of X.
-// Interior tiles are staged with direct-to-LDS loads (global_load_lds_dwordx4): no staging
+// Interior tiles are staged with direct-to-LDS loads (buffer_load_dwordx4 ... lds): no staging
 // registers and no ds_write instructions; the swizzles are applied to the global address.
 //
 // The MFMA is issued with the operands swapped (D' = Bfrag x Afrag^T), so that a lane ends
@@ -45,7 +43,6 @@ struct GemmArgs {
   int start[DA_MAX_GROUPS + 1];
   int n;
   int trace;   // 1: every workgroup records its time stamps (measurement hook)
-  int diag_k;  // diagonal tiles of a symmetric product stage one panel for both operands when K is at most this
   int interleave;   // bit g: group g's tiles are dealt to the XCDs in turns (see decode_tile)
 };
 
@@ -112,8 +109,7 @@ __device__ __forceinline__ TileId decode_tile(const GemmDesc& d, int bid, int nb
 // ---------------------------------------------------------------------------------------
 // One kernel, two K loops, three modes.
 //   DA_LOOP_INTERIOR: every tile is interior (M, N multiples of BT, K a multiple of 64).  Stages are
-//     fetched with direct-to-LDS loads issued one stage ahead; the only wait is the
-//     vmcnt(0) in front of the per-stage barrier.  No bounds checks anywhere.
+//     fetched with direct-to-LDS loads up to two stages ahead.  No bounds checks anywhere.
 //   DA_LOOP_EDGE: the same K loop for products whose ragged dimension belongs to a k-strided operand (its chunks
 //     are kept inside the matrix) and whose other operand has whole tiles; the epilogue checks bounds.  Dion's
 //     rank-r products at a rank that is not a multiple of the tile edge (r = 192).
@@ -182,9 +178,10 @@ __global__ __launch_bounds__(C::NT) void gemm_bf16_kernel(GemmArgs args) {
 
   typename C::acc_t acc[TMI][TNJ];
   gemm_tile_k_loop<C, A_KS, B_KS, MODE>(acc, d, A, B, dK, m0, n0, lds, tid, lane, wave, wm, wn, DaNoHook(),
-                                        SYM && ti == tj && A == B && dK <= args.diag_k, a_wrap, b_jump);
+                                        a_wrap, b_jump);
   if (trace) ts1 = __builtin_amdgcn_s_memrealtime();
-  epilogue<C, SYM, MODE == DA_LOOP_INTERIOR>(acc, d, lds, tile.b, ti, tj, m0, n0, wave, lane, wm, wn);
+  constexpr bool UNCHECKED = MODE != DA_LOOP_CHECKED;
+  epilogue<C, SYM, MODE == DA_LOOP_INTERIOR, C::split(UNCHECKED, A_KS), C::split(UNCHECKED, B_KS)>(acc, d, lds, tile.b, ti, tj, m0, n0, wave, lane, wm, wn);
   if (trace) {
     __syncthreads();
     if (tid == 0) {
@@ -241,16 +238,19 @@ long long tiles_of(const GemmDesc& d) {
 // bounds-checked K loop, 1 the direct-to-LDS loop with edge tiles where it applies.
 std::atomic<int> g_opt_edge_loop{-1};
 
-template <typename C, bool A_KS, bool B_KS, bool SYM>
+// C: interior and edge tiles, CG: the bounds-checked form (of the same tile edge).
+template <typename C, typename CG, bool A_KS, bool B_KS, bool SYM>
 int launch(const GemmDesc* d, int n, hipStream_t stream) {
   constexpr int BT = C::BT;
+  static_assert(CG::BT == BT, "");
   constexpr int stage2 = 2 * (Tile<BT, A_KS>::bytes + Tile<BT, B_KS>::bytes);
-  constexpr int epi = (C::NT / 64) * 32 * (C::WCOLS + 4) * 4;
-  constexpr int smem = stage2 > epi ? stage2 : epi;
+  constexpr int epi = (C::NT / 64) * 32 * (C::WCOLS + 4) * 4, epi_g = (CG::NT / 64) * 32 * (CG::WCOLS + 4) * 4;
+  constexpr int smem = stage2 > epi ? (stage2 > epi_g ? stage2 : epi_g) : (epi > epi_g ? epi : epi_g);
   auto kfull = gemm_bf16_kernel<C, A_KS, B_KS, SYM, DA_LOOP_INTERIOR>;
   constexpr int CHECKED = C::SLIDE ? DA_LOOP_INTERIOR : DA_LOOP_CHECKED;
-  auto kedge = gemm_bf16_kernel<C, A_KS, B_KS, SYM, (A_KS || B_KS) && !SYM ? DA_LOOP_EDGE : CHECKED>;
-  auto kgen = gemm_bf16_kernel<C, A_KS, B_KS, SYM, CHECKED>;
+  constexpr bool EDGE = (A_KS || B_KS) && !SYM;
+  auto kgen = gemm_bf16_kernel<CG, A_KS, B_KS, SYM, CHECKED>;
+  auto kedge = gemm_bf16_kernel<std::conditional_t<EDGE, C, CG>, A_KS, B_KS, SYM, EDGE ? DA_LOOP_EDGE : CHECKED>;
   static DaOncePerDevice configured;
   const int rc_cfg = configured.run([&]() -> int {
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kfull), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
@@ -267,7 +267,7 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
   static const bool edge_env = [] { const char* e = getenv("DION_AMD_NO_EDGE_LOOP"); return !(e && atoi(e)); }();
   const int edge_opt = g_opt_edge_loop.load(std::memory_order_relaxed);
   const bool edge_on = edge_opt >= 0 ? edge_opt != 0 : edge_env;
-  const bool edge = !full && edge_on && (A_KS || B_KS) && !SYM && edge_loop_ok(d, n, BT);
+  const bool edge = !full && edge_on && EDGE && edge_loop_ok(d, n, BT);
   long long blocks = 0;
   for (int g = 0; g < n; ++g) {
     args.d[g] = d[g];
@@ -278,10 +278,6 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
     if (blocks > 0x7fffffffLL) return DA_ERR_LIMIT;
   }
   for (int g = n; g <= DA_MAX_GROUPS; ++g) args.start[g] = (int)blocks;
-  // A diagonal tile that stages one panel runs ahead of the tiles it shares that panel with.  In a launch of a few
-  // rounds that shortens the tail (Llama-8B layer: X X^T 0.81 -> 0.77 ms); over many rounds of a long K the tiles
-  // lose each other in the L2 (32 x 4096 x 14336: 1.7 x the fetched bytes, 6.93 -> 7.35 ms), so there only up to
-  // K = 4096 (bA + cAA: 2 % faster with it).  DION_AMD_DIAG_K overrides the limit (0: never).
   // With a contiguous eighth of the launch per XCD the eight XCDs work on eight different matrices.  A launch whose
   // operands exceed the 256 MB Infinity Cache has the XCDs take turns at the tiles of one matrix instead: a panel then
   // comes from HBM once and for the other XCDs from that cache (32 x 4096 x 14336: X' = aX + BX 13.5 -> 13.0 ms,
@@ -293,22 +289,21 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
     const double bytes = 2.0 * d[g].batch * ((double)d[g].M * d[g].K + (SYM ? 0.0 : (double)d[g].N * d[g].K));
     if (il_env >= 0 ? il_env != 0 : bytes > 512.0 * 1048576.0) args.interleave |= 1 << g;
   }
-  static const int diag_k_env = [] { const char* e = getenv("DION_AMD_DIAG_K"); return e ? atoi(e) : -1; }();
-  args.diag_k = diag_k_env >= 0 ? diag_k_env : (blocks <= 4LL * da_cu_count() ? 0x7fffffff : 4096);
   for (int g = 0; g < n; ++g)   // the weight-update epilogue exists for interior tiles of plain bf16 AXPBY products
     if (d[g].upd_tab && (!full || SYM || d[g].c_dtype != DA_BF16 || d[g].epilogue != DA_EPI_AXPBY)) return DA_ERR_ARG;
-  hipLaunchKernelGGL(full ? kfull : (edge ? kedge : kgen), dim3((unsigned)blocks), dim3(C::NT), smem, stream, args);
+  hipLaunchKernelGGL(full ? kfull : (edge ? kedge : kgen), dim3((unsigned)blocks), dim3(full || edge ? C::NT : CG::NT), smem,
+                     stream, args);
   return da_launch_status();
 }
 
-template <typename C>
+template <typename C, typename CG>
 int dispatch_layout(const GemmDesc* d, int n, hipStream_t stream) {
   const GemmDesc& f = d[0];
-  if (f.symmetric) return launch<C, false, false, true>(d, n, stream);
-  if (!f.a_kstrided && !f.b_kstrided) return launch<C, false, false, false>(d, n, stream);
-  if (!f.a_kstrided && f.b_kstrided) return launch<C, false, true, false>(d, n, stream);
-  if (f.a_kstrided && !f.b_kstrided) return launch<C, true, false, false>(d, n, stream);
-  return launch<C, true, true, false>(d, n, stream);
+  if (f.symmetric) return launch<C, CG, false, false, true>(d, n, stream);
+  if (!f.a_kstrided && !f.b_kstrided) return launch<C, CG, false, false, false>(d, n, stream);
+  if (!f.a_kstrided && f.b_kstrided) return launch<C, CG, false, true, false>(d, n, stream);
+  if (f.a_kstrided && !f.b_kstrided) return launch<C, CG, true, false, false>(d, n, stream);
+  return launch<C, CG, true, true, false>(d, n, stream);
 }
 
 int check_desc(const GemmDesc& d) {
@@ -334,15 +329,15 @@ int check_desc(const GemmDesc& d) {
   return DA_OK;
 }
 
-// Estimated duration of the launch with tile configuration C, in units of "one 64-deep stage of a
-// 256 x 256 tile on a whole CU": groups are taken longest-K first (the order they are launched
-// in), `slots` tiles run at a time, the last group's partial round is rounded up, and no launch
-// is shorter than its longest tile.
+// Estimated duration of the launch with tile configuration C, in quarters of "one 64-deep stage of a 256 x 256 tile on a
+// whole CU": groups are taken longest-K first (the order they are launched in), `slots` tiles run at a time, a stage of a round
+// of them costs `unit`, a tile's start and end `ends` stages.  The last group's partial round is rounded up, where tiles run two
+// to a CU (`half` < 1) to `half` a round while it has one for each CU.  No launch is shorter than its longest tile.
 template <typename C>
-double launch_cost(const GemmDesc* d, int n, int slots, double unit) {
+double launch_cost(const GemmDesc* d, int n, int slots, double unit, double ends, double half) {
   double level = 0.0, longest = 0.0;
   for (int g = 0; g < n; ++g) {
-    const double kt = (double)(((d[g].k_slices > 1 ? d[g].k_slice : d[g].K) + BK - 1) / BK);
+    const double kt = (double)(((d[g].k_slices > 1 ? d[g].k_slice : d[g].K) + BK - 1) / BK) + ends;
     const double rounds = (double)tiles_of<C>(d[g]) / slots;
     if (g + 1 < n) {
       level += rounds * kt;
@@ -351,17 +346,18 @@ double launch_cost(const GemmDesc* d, int n, int slots, double unit) {
       const double frac = level > 0.0 ? 0.5 : 0.0;
       double r = rounds - frac;
       if (r < 0.0) r = 0.0;
-      level += ((double)(long long)(r + 0.999999)) * kt;
+      const double whole = (double)(long long)r, part = r - whole;
+      level += (whole + (part <= 0.0 ? 0.0 : part <= 0.5 ? half : 1.0)) * kt;
     }
-    if (kt > longest) longest = kt;
+    if (half * kt > longest) longest = half * kt;
   }
   return unit * (level > longest ? level : longest);
 }
 
-typedef Cfg<256, 2, 4> Big;
+typedef Cfg<256, 2, 2> Big;
+typedef Cfg<256, 2, 4> BigChecked;     // (the operand stages go through registers: eight wavefronts)
 typedef Cfg<128, 2, 2> Small;
-// Symmetric products: six row and three column blocks to a wavefront, as many LDS reads as the reads' rate allows under the products.
-typedef Cfg<192, 2, 4> Mid;
+typedef Cfg<192, 2, 2> Mid;            // (symmetric products)
 typedef Cfg<256, 2, 4, 32> Big32;      // (GemmDesc::mi32)
 typedef Cfg<128, 2, 2, 32> Small32;
 
@@ -376,16 +372,17 @@ bool slide_ok(const GemmDesc* d, int n) {
   return true;
 }
 
-// Tile choice by cost model: 256 x 256 tiles run one per CU, 128 x 128 tiles two per CU; a small
-// tile does a quarter of the work on half a CU at about 2/3 of the large tile's MFMA efficiency
-// (measured on grouped Newton-Schulz products of 768-wide matrices).
-// Interior-only (direct-to-LDS) eligibility wins over either.
-// Symmetric products have 192 x 192 tiles as well: half a matrix of tiles leaves a chip of 256 units idle more often (136 tiles
-// of 256 x 256 of a 4096 x 4096 result, 253 of 192 x 192).  A 64-deep stage of one takes 1.0 us, of a 256-tile 1.5, of two
-// 128-tiles on a unit 1.08, of one alone 0.8, and every launch takes its rounds times that.  X X^T (us, 128 / 192 / 256):
-// 4096 x 14336 393 / 224 / 314;  2 of 4096 x 4096 192 / 143 / 199;  8192 x 8192 699 / 530 / 597;  6 of 1536 x 6144 109 / 93 / 142;
-// 3072 x 8192 128 / 116 / 183;  and not: 5 of 4096 x 4096 414 / 358 / 320;  5120 x 5120 180 / 163 / 126;  2048 x 8192 98 / 114 / 179;
-// 24 of 1024 x 4096 141 / 137 / 107;  12 of 1024 x 1024 25 / 27 / 34.
+// Tile choice by cost model: 256 x 256 tiles run one per CU, 128 x 128 tiles two per CU, 192 x 192 tiles (symmetric products:
+// 136 tiles of 256 x 256 of a 4096 x 4096 result leave half the chip idle, 253 of 192 x 192 fill it) one.  Of two 128-tiles a stage
+// takes 0.7 of a 256-tile's time for half its work, of one alone 0.4, of a 192-tile 0.7; the constants are the best of a grid over the
+// 38 products of which these are some.  Interior-only (direct-to-LDS) eligibility wins over either.
+// X X^T (us, 128 / 192 / 256): 4096 x 14336 334 / 260 / 310;  2 of 4096 x 4096 161 / 147 / 189;  8192 x 8192 720 / 515 / 544;  6 of
+// 1536 x 6144 89 / 96 / 131;  3072 x 8192 102 / 113 / 159;  5 of 4096 x 4096 364 / 353 / 317;  5120 x 5120 183 / 165 / 131;
+// 2048 x 8192 61 / 105 / 150;  24 of 1024 x 4096 113 / 136 / 104;  12 of 1024 x 1024 24 / 30 / 37;  48 of 768 x 768 40 / 47 / 52.
+// B X, B of m x m (us, 128 / 256): 3072 x 8192 141 / 148;  3 of 2048 x 5632 148 / 160;  12 of 1024 x 1024 34 / 37;  48 of 768 x 768
+// 56 / 59;  and not: 12 of 768 x 3072 61 / 58;  5120 x 5120 293 / 235;  4096 x 14336 518 / 435.
+// Plain stores have less for two tiles to hide of one another.  (M, N, K), operands k-contiguous (c) or k-strided (s): 48 of
+// (768, 768, 768) c s 64 / 58, s s 62 / 57, c c 52 / 54;  12 of (3072, 768, 768) c s 61 / 55;  12 of (768, 768, 3072) c s 47 / 67.
 int choose_tile(const GemmDesc* d, int n) {
   static const int forced = [] { const char* e = getenv("DION_AMD_TILE"); return e ? atoi(e) : 0; }();
   if (forced == 128 || forced == 256) return forced;
@@ -398,19 +395,21 @@ int choose_tile(const GemmDesc* d, int n) {
   const bool may_edge = !d[0].symmetric && (d[0].a_kstrided || d[0].b_kstrided);
   const bool full_big = all_interior(d, n, 256) || (may_edge && edge_loop_ok(d, n, 256));
   const bool full_small = all_interior(d, n, 128) || (may_edge && edge_loop_ok(d, n, 128));
-  const double cost_big = launch_cost<Big>(d, n, 256, 4.0);
-  const double cost_small = launch_cost<Small>(d, n, 512, 3.0);
+  // A symmetric product with an addend: where a caller's addend is not symmetric the tile edge decides which of E(m, n) and E(n, m)
+  // an element gets.  Its rule (constants of an older K loop, up to 12 % from the best edge for b A + c A A) stays as it is for that.
+  const bool addend = d[0].symmetric && d[0].epilogue == DA_EPI_AXPBY;
+  const double cost_big = launch_cost<Big>(d, n, 256, 4.0, addend ? 0.0 : 3.0, 1.0);
+  const double cost_small = addend ? launch_cost<Small>(d, n, 512, 3.0, 0.0, 1.0)
+                                   : launch_cost<Small>(d, n, 512, may_edge && d[0].epilogue == DA_EPI_STORE ? 3.0 : 2.75, 0.0, 0.55);
   const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
   if (d[0].symmetric && slide_ok(d, n)) {
     long long mid = 0, small = 0, matrices = 0;
     for (int g = 0; g < n; ++g) { mid += tiles_of<Mid>(d[g]); small += tiles_of<Small>(d[g]); matrices += d[g].batch; }
-    const double cost_mid = launch_cost<Mid>(d, n, 256, 2.75);
-    if (big) {
-      // (several matrices over many rounds: 4 of 4096 x 10560, a round in twelve less by this count, were 1.4 % slower)
-      if (cost_mid * (mid > 512 && matrices > 1 ? 1.1 : 1.0) < cost_big) return Mid::BT;
-    } else if (small > 256 && 2.25 * mid <= 1.15 * small && cost_mid * (mid > 256 ? 1.13 : 1.0) < cost_small) {
-      // (128-tiles two to a unit hide one another's epilogues: only where sliding computes little again, and over several
-      // rounds, where a 192-tile's stage takes 1.12 us, only for a round less)
+    const double cost_mid = launch_cost<Mid>(d, n, 256, 2.75, 0.0, 1.0);
+    if (addend && !big) {
+      if (small > 256 && 2.25 * mid <= 1.15 * small && cost_mid * (mid > 256 ? 1.13 : 1.0) < cost_small) return Mid::BT;
+    } else if (cost_mid * (mid > 512 && matrices > 1 ? 1.1 : 1.0) < (big ? cost_big : cost_small)) {
+      // (several matrices over many rounds: 4 of 4096 x 10560, a round in twelve less by this count, are 5 % slower)
       return Mid::BT;
     }
   }
@@ -438,12 +437,12 @@ int da_gemm_bf16_grouped(const GemmDesc* din, int n, hipStream_t stream) {
     d[pos] = a;
   }
   if (d[0].mi32) {
-    if (choose_tile(d, n) == 256) return launch<Big32, false, false, false>(d, n, stream);
-    return launch<Small32, false, false, false>(d, n, stream);
+    if (choose_tile(d, n) == 256) return launch<Big32, Big32, false, false, false>(d, n, stream);
+    return launch<Small32, Small32, false, false, false>(d, n, stream);
   }
   const int bt = choose_tile(d, n);
-  if (bt == Mid::BT) return launch<Mid, false, false, true>(d, n, stream);
-  return bt == 256 ? dispatch_layout<Big>(d, n, stream) : dispatch_layout<Small>(d, n, stream);
+  if (bt == Mid::BT) return launch<Mid, Mid, false, false, true>(d, n, stream);
+  return bt == 256 ? dispatch_layout<Big, BigChecked>(d, n, stream) : dispatch_layout<Small, Small>(d, n, stream);
 }
 
 void da_gemm_bf16_set_edge_loop(int v) { g_opt_edge_loop.store(v < 0 ? -1 : (v != 0), std::memory_order_relaxed); }

@@ -7,6 +7,7 @@
 #pragma once
 #include "common.h"
 #include "mfma_tile.h"
+#include <type_traits>
 
 namespace {
 
@@ -18,9 +19,6 @@ template <> struct AccOf<16> { typedef f32x4_t type; };
 
 #ifndef DA_MI
 #define DA_MI 16   // the MFMA shape the kernels of this library are built with (32: the 32x32x16 form)
-#endif
-#ifndef DA_KLOOP_ABLATE
-#define DA_KLOOP_ABLATE 0   // see gemm_tile_k_loop: measurement builds only
 #endif
 
 template <int BT_, int WGM_, int WGN_, int MI_ = DA_MI>
@@ -35,6 +33,11 @@ struct Cfg {
   static constexpr int NB = WROWS / 32;            // 32-row bands of a wavefront's sub-tile (the epilogue's unit)
   // the last row and column of tiles lies against the matrix's end, over part of its neighbour (gemm_bf16.hip, Mid)
   static constexpr bool SLIDE = BT == 192;
+  // interior and edge tiles run gemm_tile_k_loop_quad
+  static constexpr bool QUAD = MI == 16 && WGM == 2 && WGN == 2;
+  // A k-strided operand of 128-tiles there: a wavefront has two runs of 32 rows (columns) 64 apart, so that what it reads in one phase
+  // is half a k-row of the tile, a whole cache line (two half lines otherwise: both operands k-strided 1720 - 1880 clocks a stage).
+  static constexpr bool split(bool full, bool ks) { return QUAD && full && BT == 128 && ks; }
   typedef typename AccOf<MI>::type acc_t;
 };
 
@@ -136,7 +139,9 @@ __device__ __forceinline__ void update_weights8(char* Wp, bool w_f32, u32x4_t x0
 
 // UPD: 0 the result is stored in C; 1 / 2 it is not stored but updates the weights d.upd_tab[b] in place (2: those are
 // stored transposed), see GemmDesc.
-template <typename C, bool SYM, bool FULL, bool CF32, bool HAS_E, bool FAITHFUL, bool S1_ONE, int UPD = 0, bool WF32 = false>
+// RSPLIT, CSPLIT: a wavefront's rows (columns) are two runs, see Cfg::split.
+template <typename C, bool SYM, bool FULL, bool CF32, bool HAS_E, bool FAITHFUL, bool S1_ONE, int UPD = 0, bool WF32 = false,
+          bool RSPLIT = false, bool CSPLIT = false>
 __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, char* lds, int b,
                                               bool mirror, int m0, int n0, int wave, int lane, int wm, int wn) {
   constexpr int W = C::WCOLS;        // columns of a wavefront's sub-tile
@@ -154,13 +159,15 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   const long long c2 = (!HAS_E && !FAITHFUL && !SYM && !CF32) ? d.c2_off * 2 : 0;   // bytes to the second output
   const int dM = d.M, dN = d.N;
   const long long ldc = d.ldc, lde = d.lde;
-  const int wm0 = m0 + wm * C::WROWS, wn0 = n0 + wn * W;
+  const int wm0 = m0 + wm * (RSPLIT ? 32 : C::WROWS), wn0 = n0 + wn * (CSPLIT ? 32 : W);
+  auto row_of = [&](int band) { return wm0 + band * (RSPLIT ? 64 : 32); };            // first row of a band
+  auto col_of = [&](int c) { return wn0 + (CSPLIT ? (c & 31) + (c >> 5) * 64 : c); };   // column c of the wavefront's
   char* const Cbase = d.Ctab ? static_cast<char*>(d.Ctab[b]) : static_cast<char*>(d.C) + (long long)b * d.sC * CSZ;
   const char* const Ebase = !HAS_E ? nullptr
                             : d.Etab ? static_cast<const char*>(d.Etab[b])
                                      : static_cast<const char*>(d.E) + (long long)b * d.sE * CSZ;
-  const int lr = lane / CPR, c8 = (lane % CPR) * 8;
-  const bool col_ok = (FULL || wn0 + c8 < dN) && (!ODD || lane < RPP * CPR);
+  const int lr = lane / CPR, c8 = (lane % CPR) * 8, cn = col_of(c8);
+  const bool col_ok = (FULL || cn < dN) && (!ODD || lane < RPP * CPR);
   char* const Wbase = UPD ? static_cast<char*>(d.upd_tab[b]) : nullptr;
   constexpr bool w_f32 = WF32;   // (a compile-time variant: the prefetch buffers differ in size)
   constexpr int wsz = w_f32 ? 4 : 2;
@@ -177,11 +184,11 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   u32x4_t wv[NWP][NWV];
   auto weight_ptr = [&](int band, int pass) -> char* {
     if (UPD == 2) {
-      const int n = wn0 + (pass >> 2) * 64 + lane, m = wm0 + band * 32 + (pass & 3) * 8;
+      const int n = col_of((pass >> 2) * 64 + lane), m = row_of(band) + (pass & 3) * 8;
       return Wbase + ((long long)n * ldw + m) * wsz;
     }
-    const int m = wm0 + band * 32 + pass * RPP + lr;
-    return Wbase + ((long long)m * ldw + wn0 + c8) * wsz;
+    const int m = row_of(band) + pass * RPP + lr;
+    return Wbase + ((long long)m * ldw + cn) * wsz;
   };
   auto load_w = [&](int band, u32x4_t (&dst)[NWP][NWV]) {
 #pragma unroll
@@ -195,12 +202,12 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   auto load_e = [&](int band, u32x4_t (&dst)[NPASS][NV]) {
 #pragma unroll
     for (int pass = 0; pass < NPASS; ++pass) {
-      const int m = wm0 + band * 32 + pass * RPP + lr;
+      const int m = row_of(band) + pass * RPP + lr;
       const u32x4_t z = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int h = 0; h < NV; ++h) dst[pass][h] = z;
       if (col_ok && (FULL || m < dM) && (!ODD || pass * RPP + lr < 32)) {
-        const char* Ep = Ebase + ((long long)m * lde + wn0 + c8) * CSZ;
+        const char* Ep = Ebase + ((long long)m * lde + cn) * CSZ;
 #pragma unroll
         for (int h = 0; h < NV; ++h) dst[pass][h] = ldg16(Ep + 16 * h);
       }
@@ -233,7 +240,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
         }
     }
     wave_sync_lds();
-    const int band_m = wm0 + i * 32;
+    const int band_m = row_of(i);
     u32x4_t ec[NPASS][NV];
     if (HAS_E) {
 #pragma unroll
@@ -253,7 +260,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
         const float4 a1 = *reinterpret_cast<const float4*>(sp + 4);
         float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
         float e[8];
-        char* Cp = Cbase + ((long long)m * ldc + wn0 + c8) * CSZ;
+        char* Cp = Cbase + ((long long)m * ldc + cn) * CSZ;
         if (CF32) {
 #pragma unroll
           for (int q = 0; q < 8; ++q) {
@@ -307,7 +314,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
       for (int pass = 0; pass < (W / 64) * 4; ++pass) {
         const int nl = (pass >> 2) * 64 + lane;
         const int mg = (pass & 3) * 8;
-        const int n = wn0 + nl, m = band_m + mg;
+        const int n = col_of(nl), m = band_m + mg;
         if (FULL || (n < dN && m < dM)) {
           u32x4_t pk;
 #pragma unroll
@@ -353,16 +360,16 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   }
 }
 
-template <typename C, bool SYM, bool FULL>
+template <typename C, bool SYM, bool FULL, bool RSPLIT = false, bool CSPLIT = false>
 __device__ __forceinline__ void epilogue(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, char* lds, int b, int ti,
                                          int tj, int m0, int n0, int wave, int lane, int wm, int wn) {
   const bool mirror = SYM && (ti != tj);
   const bool cf32 = d.c_dtype == DA_F32, has_e = d.epilogue == DA_EPI_AXPBY, fa = d.faithful != 0;
   const bool one = d.s1 == 1.f;   // rounding-faithful bf16 output: the exact multiplication by 1 is left out
 #define DA_EPI(CF, HE, FA, S1) \
-  epilogue_impl<C, SYM, FULL, CF, HE, FA, S1>(acc, d, lds, b, mirror, m0, n0, wave, lane, wm, wn)
+  epilogue_impl<C, SYM, FULL, CF, HE, FA, S1, 0, false, RSPLIT, CSPLIT>(acc, d, lds, b, mirror, m0, n0, wave, lane, wm, wn)
 #define DA_EPI_UPD(FA, S1, U, WF) \
-  epilogue_impl<C, false, FULL, false, true, FA, S1, U, WF>(acc, d, lds, b, false, m0, n0, wave, lane, wm, wn)
+  epilogue_impl<C, false, FULL, false, true, FA, S1, U, WF, RSPLIT, CSPLIT>(acc, d, lds, b, false, m0, n0, wave, lane, wm, wn)
 #define DA_EPI_UPD_FA(U, WF)                                                              \
   do {                                                                                    \
     if (fa) { if (one) DA_EPI_UPD(true, true, U, WF); else DA_EPI_UPD(true, false, U, WF); } \
@@ -395,10 +402,225 @@ __device__ __forceinline__ void epilogue(typename C::acc_t (&acc)[C::TMI][C::TNJ
 
 constexpr int DA_LOOP_CHECKED = 0, DA_LOOP_INTERIOR = 1, DA_LOOP_EDGE = 2;
 
+__device__ __forceinline__ unsigned long long wave_uniform64(unsigned long long x) {
+  return ((unsigned long long)(unsigned)wave_uniform((int)(x >> 32)) << 32) | (unsigned)wave_uniform((int)x);
+}
+template <int N> __device__ __forceinline__ void dma_wait_all_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// 16 bytes per lane from a raw buffer into LDS at `lbase` + `l` + 16 * lane (dma16, addressed by scalars: a request costs the wavefront
+// three instructions).  From a buffer of no records nothing is fetched, the request is counted all the same.
+__device__ __forceinline__ void dma16_buf(u32x4_t buf, unsigned off, unsigned soff, unsigned lbase, unsigned l) {
+  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+               :
+               : "v"(off), "s"(buf), "s"(soff), "s"(lbase), "s"(l)
+               : "memory", "scc");
+}
+
+// One product added to accumulators that stay in their AGPRs.  As assembly: the compiler, given 256 of them, moved some about on every
+// pass of the loop (56 v_accvgpr_mov a stage with both operands k-contiguous, 3400 clocks instead of 2600).  It does not know the
+// instruction's hazards then: no accumulator is touched again within four products, and mfma_drain() comes before they are read.
+__device__ __forceinline__ void mfma16_in_place(f32x4_t& c, bf16x8_t col, bf16x8_t row) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(col), "v"(row));
+}
+__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+
+// Addresses of one operand in gemm_tile_k_loop_quad.  The unit of a request is half an operand stage, what every wavefront reads in one
+// phase: H rows of each of the two wavefronts along the operand.  In LDS a k-contiguous operand has the layout of read_frag16
+// ([BT][64], the halves are blocks of its rows), a k-strided one two tiles [64][BT / 2], a unit each.
+template <typename C, bool KS>
+struct UnitAddr {
+  static constexpr int H = C::BT / 4;
+  static constexpr int NU = H / 16;                      // wave instructions (1024 bytes) of a wavefront per unit
+  static constexpr int LHALF = KS ? H * 2 * BK * 2 : H * 128;
+  unsigned long long base;                               // bytes; wave-uniform, as step and l
+  unsigned step[2][NU], l[NU];                           // to the instructions' blocks, in memory (both units) and in LDS
+  unsigned off[KS ? 2 : 1];                              // per lane
+  __device__ __forceinline__ UnitAddr(const bf16_t* P, int ld, int row0, int dim, int lane, int wave) {
+    const unsigned pitch = (unsigned)ld * 2u;
+    if (!KS) {
+      constexpr int HB = H / 8;                          // blocks of eight rows in a half
+      const int r = lane >> 3;
+      base = wave_uniform64(reinterpret_cast<unsigned long long>(P + (long long)row0 * ld));
+      off[0] = (unsigned)r * pitch + (unsigned)kc_swizzle(lane & 7, (wave & 1) * 8 + r) * 16u;   // (a block's parity is the wavefront's)
+#pragma unroll
+      for (int e = 0; e < NU; ++e) {
+        const int q = e * 4 + wave, blk = q / HB * (2 * HB) + q % HB;
+        step[0][e] = (unsigned)wave_uniform((int)((unsigned)blk * 8u * pitch));
+        step[1][e] = (unsigned)wave_uniform((int)((unsigned)(blk * 8 + H) * pitch));
+        l[e] = (unsigned)blk * 1024u;
+      }
+    } else {
+      constexpr int CPR = H / 4, RPB = 64 / CPR;         // chunks of a unit's k-row, k-rows of an instruction
+      const int kr = lane / CPR, c = ks_swizzle(lane % CPR, kr) * 8;
+      base = wave_uniform64(reinterpret_cast<unsigned long long>(P + row0));
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        int col = C::split(true, true) ? h * (2 * H) + c : c / H * (2 * H) + h * H + c % H;
+        if (row0 + col > dim - 8) col = dim - 8 - row0;  // (StageAddr: an edge tile stays inside the matrix)
+        off[h] = (unsigned)kr * pitch + (unsigned)col * 2u;
+      }
+#pragma unroll
+      for (int e = 0; e < NU; ++e) {
+        step[0][e] = step[1][e] = (unsigned)wave_uniform((int)((unsigned)((e * 4 + wave) * RPB) * pitch));
+        l[e] = (unsigned)(e * 4 + wave) * 1024u;
+      }
+    }
+  }
+};
+template <typename C, bool KS>
+__device__ __forceinline__ bf16x8_t unit_frag(const char* op, int w, int h, int i, int ks, int lane) {
+  constexpr int H = C::BT / 4;
+  if (!KS) return read_frag16<C::BT, false>(op, w * (2 * H) + h * H + i * 16, ks, lane);
+  return read_frag16<C::BT / 2, true>(op + h * UnitAddr<C, true>::LHALF, w * H + i * 16, ks, lane);
+}
+
+// The direct-to-LDS K loop of four wavefronts, a quarter of the tile each (of a 256-tile 128 x 128: 256 accumulators, in AGPRs).
+// A wavefront's results are four quadrants; a 64-deep stage is four phases, a quadrant's products each:
+//   phase            0              1              2                3
+//   products         A0 B0          A0 B1          A1 B0            A1 B1          (A0, A1: halves of the wavefront's rows; B: of its columns)
+//   LDS reads        B1             A1             A0 of the next   B0 of the next stage
+//   requests         A0 of t + 2    B0 of t + 2    B1 of t + 2      A1 of t + 2    (into the buffer of stage t)
+// Two barriers to a stage, behind phases 1 and 3: what the next two phases read has landed (four to six phases after its request; the
+// wait leaves the 16 younger requests in flight) and what they request anew has been read.  Reads and requests stand singly between
+// products, in a fixed order: with one wavefront to a SIMD nothing else covers them, and a product covers three instructions.  The loop
+// has no branches: the two stages past the last one are requested from a buffer of no records.
+// What bounds it: eight wavefronts of 128 x 64 read 192 KB a stage from LDS (128 bytes a clock) and the requests write 64 KB, 2048 clocks
+// of the matrix cores' 2048; four of 128 x 128 read 128 KB.  Clocks per stage of a 256-tile on every CU, eight wavefronts -> four: both
+// operands k-contiguous 2990 -> 2610, one k-strided 3130 -> 2640, both - -> 2690 (products and barriers alone 2180).  Under random data
+// the chip lowers its clock as the loop gets denser (2.2 GHz for zeros, 1.7 here): 1.22-1.26 -> 1.36-1.39 PFLOP/s.
+// `hook`, `a_wrap`, `b_jump`: gemm_tile_k_loop.
+template <typename C, bool A_KS, bool B_KS, typename Hook>
+__device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, const bf16_t* A,
+                                                      const bf16_t* B, int dK, int m0, int n0, char* lds, int lane, int wave,
+                                                      int wm, int wn, Hook hook, int a_wrap, unsigned b_jump) {
+  static_assert(C::MI == 16 && C::WGM == 2 && C::WGN == 2 && (C::BT == 256 || C::BT == 128 || (C::BT == 192 && !A_KS && !B_KS)), "");
+  constexpr int OP = C::BT * BK * 2, STAGE = 2 * OP;
+  constexpr int HI = C::BT / 64;                         // 16-row blocks of a half
+  constexpr int NR = 2 * HI, NU = UnitAddr<C, false>::NU;
+  typedef UnitAddr<C, A_KS> UA;
+  typedef UnitAddr<C, B_KS> UB;
+  const int KT = wave_uniform(dK / BK);
+  const unsigned wrap = (unsigned)wave_uniform(a_wrap < 0 ? d.a_kwrap : a_wrap) * 2u;
+  const unsigned jump = (unsigned)wave_uniform((int)b_jump);
+  const UA ua(A, d.lda, m0, d.M, lane, wave);
+  const UB ub(B, d.ldb, n0, d.N, lane, wave);
+  const unsigned long long a_stage = wave_uniform64(A_KS ? (unsigned long long)d.lda * (BK * 2) : BK * 2);
+  const unsigned long long b_stage = wave_uniform64(B_KS ? (unsigned long long)d.ldb * (BK * 2) : BK * 2);
+  const unsigned l0 = lds_addr(lds);
+  unsigned long long pa = ua.base, pb = ub.base;         // the stage being requested
+  unsigned in_turn = 0;
+  u32x4_t ba, bb;
+  // `more` >= 0: the stage exists.  (Left to the compiler the choice of the record count ends up on the vector unit.)
+  auto set_buffers = [&](int more) {
+    unsigned n;
+    asm("s_cmp_ge_i32 %1, 0\n\ts_cselect_b32 %0, -1, 0" : "=s"(n) : "s"(more) : "scc");
+    ba = u32x4_t{(unsigned)wave_uniform((int)pa), (unsigned)wave_uniform((int)(pa >> 32)), n, 0x00020000u};
+    bb = u32x4_t{(unsigned)wave_uniform((int)pb), (unsigned)wave_uniform((int)(pb >> 32)), n, 0x00020000u};
+  };
+  auto load_a = [&](int h, int e, unsigned l) { dma16_buf(ba, ua.off[A_KS ? h : 0], ua.step[h][e], l + h * UA::LHALF, ua.l[e]); };
+  auto load_b = [&](int h, int e, unsigned l) { dma16_buf(bb, ub.off[B_KS ? h : 0], ub.step[h][e], l + OP + h * UB::LHALF, ub.l[e]); };
+  auto next_stage = [&](int more) {
+    pa += a_stage;
+    pb += b_stage;
+    in_turn += BK * 2;
+    if (in_turn == wrap) { pa = ua.base; in_turn = 0; pb += jump; }   // (0: never, in_turn > 0 here)
+    set_buffers(more);
+  };
+
+  bf16x8_t a0[HI][2], a1[HI][2], b0[HI][2], b1[HI][2];
+  // the products of quadrant (ah, bh), the NR reads and NU requests of the phase at fixed places between them
+  auto phase = [&](auto ah, auto bh, bf16x8_t (&a)[HI][2], bf16x8_t (&b)[HI][2], auto read, auto request) {
+    int n = 0;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < HI; ++i)
+#pragma unroll
+        for (int j = 0; j < HI; ++j) {
+          constexpr int EVERY = HI == 4 ? 3 : HI == 3 ? 2 : 1;   // (early: the barrier waits for the last of them)
+          if (n % EVERY == 0 && n / EVERY < NR) {
+            read((n / EVERY) % HI, (n / EVERY) / HI);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          const int e = HI == 4   ? (n == 1 ? 0 : n == 8 ? 1 : n == 16 ? 2 : n == 23 ? 3 : -1)
+                        : HI == 3 ? (n == 1 ? 0 : n == 7 ? 1 : n == 13 ? 2 : -1)
+                                  : (n == 4 ? 0 : n == 6 ? 1 : -1);
+          if (e >= 0) {
+            request(e);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          mfma16_in_place(acc[decltype(ah)::value * HI + i][decltype(bh)::value * HI + j], b[j][ks], a[i][ks]);
+          __builtin_amdgcn_sched_barrier(0);
+          ++n;
+        }
+  };
+  auto meet = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  set_buffers(0);
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int e = 0; e < NU; ++e) load_a(h, e, l0 + s * STAGE);
+#pragma unroll
+      for (int e = 0; e < NU; ++e) load_b(h, e, l0 + s * STAGE);
+    }
+    next_stage(KT - 2 - s);
+  }
+  __builtin_amdgcn_sched_barrier(0);   // (256 registers are cleared while the first stage is on its way)
+#pragma unroll
+  for (int i = 0; i < C::TMI; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TNJ; ++j)
+#pragma unroll
+      for (int v = 0; v < C::AV; ++v) acc[i][j][v] = 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+  dma_wait_all_but<6 * NU>();   // A0, B0
+  meet();
+  hook();
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int i = 0; i < HI; ++i) {
+      a0[i][ks] = unit_frag<C, A_KS>(lds, wm, 0, i, ks, lane);
+      b0[i][ks] = unit_frag<C, B_KS>(lds + OP, wn, 0, i, ks, lane);
+    }
+  dma_wait_all_but<4 * NU>();   // the rest of stage 0
+  meet();
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, 1> I1;
+  for (int left = KT - 1, buf = 0; left >= 0; --left, buf ^= STAGE) {   // (`left` stages follow this one)
+    const char* const cur = lds + buf;
+    const char* const nxt = lds + (buf ^ STAGE);
+    const unsigned l = l0 + buf;
+    phase(I0(), I0(), a0, b0, [&](int i, int ks) { b1[i][ks] = unit_frag<C, B_KS>(cur + OP, wn, 1, i, ks, lane); },
+          [&](int e) { load_a(0, e, l); });
+    phase(I0(), I1(), a0, b1, [&](int i, int ks) { a1[i][ks] = unit_frag<C, A_KS>(cur, wm, 1, i, ks, lane); },
+          [&](int e) { load_b(0, e, l); });
+    dma_wait_all_but<4 * NU>();
+    meet();
+    // (behind the last stage these reads return what lies in the other buffer, for no product)
+    phase(I1(), I0(), a1, b0, [&](int i, int ks) { a0[i][ks] = unit_frag<C, A_KS>(nxt, wm, 0, i, ks, lane); },
+          [&](int e) { load_b(1, e, l); });
+    phase(I1(), I1(), a1, b1, [&](int i, int ks) { b0[i][ks] = unit_frag<C, B_KS>(nxt + OP, wn, 0, i, ks, lane); },
+          [&](int e) { load_a(1, e, l); });
+    next_stage(left - 3);
+    dma_wait_all_but<4 * NU>();
+    meet();
+  }
+  dma_wait();   // (requests of no records: what they leave in LDS comes before the epilogue's use of it)
+  mfma_drain();
+  meet();
+}
+
 // K loop of one BT x BT tile: acc += sum over dK elements of k of A-rows (m0 ...) x B-rows (n0 ...).  `A`, `B`: the
 // matrix's operands at the first k of the sum.  Three forms (MODE):
-//   DA_LOOP_INTERIOR: every tile is interior (M, N multiples of BT, K a multiple of 64).  Stages are
-//     fetched with direct-to-LDS loads issued one stage ahead; the only wait is the
+//   DA_LOOP_INTERIOR: every tile is interior (M, N multiples of BT, K a multiple of 64): gemm_tile_k_loop_quad where four
+//     wavefronts run the 16 x 16 form, else stages fetched with direct-to-LDS loads one stage ahead, the only wait the
 //     vmcnt(0) in front of the per-stage barrier.  No bounds checks anywhere.
 //   DA_LOOP_EDGE: the same K loop for products whose ragged dimension belongs to a k-strided operand (its chunks
 //     are kept inside the matrix) and whose other operand has whole tiles; the epilogue checks bounds.  Dion's
@@ -408,8 +630,6 @@ constexpr int DA_LOOP_CHECKED = 0, DA_LOOP_INTERIOR = 1, DA_LOOP_EDGE = 2;
 // Ends with a workgroup barrier: the stage buffers are free for the epilogue.
 // `after_first_stage` (direct-to-LDS forms) is called once, behind the barrier that publishes the first stage: every
 // wavefront has waited for all of its outstanding memory operations by then, stores of earlier work included.
-// `same_panel` (direct-to-LDS forms, both operands k-contiguous): the two operands are the same rows of the same
-// matrix -- a diagonal tile of X X^T or A A -- so one panel is staged and both fragment sets are read from it.
 // `a_wrap`, `b_jump` (direct-to-LDS forms): A is read again from its first column after a_wrap of its columns instead of
 // GemmDesc::a_kwrap of them, and B then goes on b_jump bytes further.
 struct DaNoHook { __device__ __forceinline__ void operator()() const {} };
@@ -417,8 +637,12 @@ template <typename C, bool A_KS, bool B_KS, int MODE, typename Hook = DaNoHook>
 __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, const bf16_t* A,
                                                  const bf16_t* B, int dK, int m0, int n0, char* lds, int tid, int lane,
                                                  int wave, int wm, int wn, Hook after_first_stage = Hook(),
-                                                 bool same_panel = false, int a_wrap = -1, unsigned b_jump = 0) {
+                                                 int a_wrap = -1, unsigned b_jump = 0) {
   constexpr bool FULL = MODE != DA_LOOP_CHECKED;   // the direct-to-LDS K loop
+  if constexpr (FULL && C::QUAD) {
+    gemm_tile_k_loop_quad<C, A_KS, B_KS>(acc, d, A, B, dK, m0, n0, lds, lane, wave, wm, wn, after_first_stage, a_wrap, b_jump);
+    return;
+  }
   constexpr int BT = C::BT, TMI = C::TMI, TNJ = C::TNJ, NCH = C::NCH, NW = C::NT / 64;
   constexpr int A_BYTES = Tile<BT, A_KS>::bytes;
   constexpr int B_BYTES = Tile<BT, B_KS>::bytes;
@@ -436,21 +660,20 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
   const int KT = (dK + BK - 1) / BK;
   bf16x8_t fa[C::MI == 32 ? TMI : 1], fb[C::MI == 32 ? TNJ : 1];   // (the 16 x 16 form keeps its own sets below)
 
-  const int b_at = (FULL && !A_KS && !B_KS && same_panel) ? 0 : A_BYTES;   // where the column operand's panel lies in a stage
   if constexpr (C::MI == 32) {
 #define DA_FREAD(st, ks)                                                                           \
   do {                                                                                             \
     _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
         fa[i] = read_frag<BT, A_KS>((st), ar0 + i * 32, (ks), lane);                               \
     _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
-        fb[j] = read_frag<BT, B_KS>((st) + b_at, br0 + j * 32, (ks), lane);                        \
+        fb[j] = read_frag<BT, B_KS>((st) + A_BYTES, br0 + j * 32, (ks), lane);                        \
   } while (0)
 #define DA_FREAD2(st, ks, FA, FB)                                                                  \
   do {                                                                                             \
     _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
         FA[i] = read_frag<BT, A_KS>((st), ar0 + i * 32, (ks), lane);                               \
     _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
-        FB[j] = read_frag<BT, B_KS>((st) + b_at, br0 + j * 32, (ks), lane);                        \
+        FB[j] = read_frag<BT, B_KS>((st) + A_BYTES, br0 + j * 32, (ks), lane);                        \
   } while (0)
 #define DA_MMA2(FA, FB)                                                                            \
   do {                                                                                             \
@@ -471,10 +694,8 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
   do {                                                                                             \
     _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
         dma16(sa.dbase, sa.doff + i * sa.dstep + koff_a, lds_addr(st) + (i * NW + wave) * 1024);   \
-    if (b_at != 0) {                                                                               \
-      _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                              \
-          dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
-    }                                                                                              \
+    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
+        dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
     koff_a += (unsigned)(sa.tstep * 2);                                                            \
     koff_b += (unsigned)(sb.tstep * 2);                                                            \
     if (koff_a == wrap_a) { koff_a = 0; koff_b += b_jump; }                                        \
@@ -572,102 +793,27 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
 #undef DA_FREAD2
 #undef DA_MMA2
   } else {
-  // ---- v_mfma_f32_16x16x32_bf16: a stage is two 32-deep k-steps; per k-step TMI row fragments (two halves H0, H1) and
-  // TNJ column fragments.  Read-ahead in registers: while the MFMAs of one half run, the other half's row fragments
-  // (and, under H1, the next k-step's column fragments and H0 row fragments) are fetched.
+  // ---- v_mfma_f32_16x16x32_bf16, bounds-checked: a stage is two 32-deep k-steps of TMI row fragments (in two halves) and TNJ
+  // column fragments
   constexpr int TH = TMI / 2;
-  // Measurement builds (-DDA_KLOOP_ABLATE=<bits>, WRONG RESULTS): what the direct-to-LDS loop costs without 1 its
-  // fragment reads (the first stage's are kept), 2 its staging loads (after the first two stages), 4 the per-stage
-  // wait and barrier, 8 its matrix-core instructions.
-  constexpr bool ABL_READ = (DA_KLOOP_ABLATE & 1) != 0, ABL_DMA = (DA_KLOOP_ABLATE & 2) != 0,
-                 ABL_BAR = (DA_KLOOP_ABLATE & 4) != 0, ABL_MMA = (DA_KLOOP_ABLATE & 8) != 0;
-  bool abl_first = true;
 #define DA16_RA(FA, st, ks, h)                                                                     \
   do {                                                                                             \
-    if (!(FULL && ABL_READ) || abl_first) {                                                        \
-      _Pragma("unroll") for (int i = 0; i < TH; ++i)                                               \
-          FA[i] = read_frag16<BT, A_KS>((st), ar0 + ((h) * TH + i) * 16, (ks), lane);              \
-    }                                                                                              \
+    _Pragma("unroll") for (int i = 0; i < TH; ++i)                                                 \
+        FA[i] = read_frag16<BT, A_KS>((st), ar0 + ((h) * TH + i) * 16, (ks), lane);                \
   } while (0)
 #define DA16_RB(FB, st, ks)                                                                        \
   do {                                                                                             \
-    if (!(FULL && ABL_READ) || abl_first) {                                                        \
-      _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                              \
-          FB[j] = read_frag16<BT, B_KS>((st) + b_at, br0 + j * 16, (ks), lane);                    \
-    }                                                                                              \
+    _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
+        FB[j] = read_frag16<BT, B_KS>((st) + A_BYTES, br0 + j * 16, (ks), lane);                      \
   } while (0)
 #define DA16_MMA(FA, FB, h)                                                                        \
   do {                                                                                             \
-    if (FULL && ABL_MMA) {   /* the fragments are consumed (waited for), nothing is computed */   \
-      _Pragma("unroll") for (int i = 0; i < TH; ++i) asm volatile("" ::"v"(FA[i]));               \
-      _Pragma("unroll") for (int j = 0; j < TNJ; ++j) asm volatile("" ::"v"(FB[j]));              \
-    } else {                                                                                       \
-      _Pragma("unroll") for (int i = 0; i < TH; ++i)                                               \
-          _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                          \
-              acc[(h) * TH + i][j] =                                                               \
-                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(FB[j], FA[i], acc[(h) * TH + i][j], 0, 0, 0); \
-    }                                                                                              \
+    _Pragma("unroll") for (int i = 0; i < TH; ++i)                                                 \
+        _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                            \
+            acc[(h) * TH + i][j] =                                                                 \
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(FB[j], FA[i], acc[(h) * TH + i][j], 0, 0, 0); \
   } while (0)
-  if (FULL) {
-#define DA16_DMA(st)                                                                               \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
-        dma16(sa.dbase, sa.doff + i * sa.dstep + koff_a, lds_addr(st) + (i * NW + wave) * 1024);   \
-    if (b_at != 0) {                                                                               \
-      _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                              \
-          dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
-    }                                                                                              \
-    koff_a += (unsigned)(sa.tstep * 2);                                                            \
-    koff_b += (unsigned)(sb.tstep * 2);                                                            \
-    if (koff_a == wrap_a) { koff_a = 0; koff_b += b_jump; }                                        \
-  } while (0)
-    unsigned koff_a = 0, koff_b = 0;
-    const unsigned wrap_a = (unsigned)(a_wrap < 0 ? d.a_kwrap : a_wrap) * 2u;
-    DA16_DMA(lds);
-    dma_wait();
-    __syncthreads();
-    after_first_stage();
-    bf16x8_t a0[TH], a1[TH], b0[TNJ], b1[TNJ];
-    if (KT > 1) DA16_DMA(lds + STAGE);
-    DA16_RB(b0, lds, 0);
-    DA16_RA(a0, lds, 0, 0);
-    for (int kt = 0; kt < KT; ++kt) {
-      char* cur = lds + (kt & 1) * STAGE;
-      char* nxt = lds + ((kt + 1) & 1) * STAGE;
-      const bool more = kt + 1 < KT;
-      DA16_RA(a1, cur, 0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_MMA(a0, b0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_RB(b1, cur, 1);
-      DA16_RA(a0, cur, 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_MMA(a1, b0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_RA(a1, cur, 1, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_MMA(a0, b1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (!ABL_BAR) {
-        dma_wait();
-        __syncthreads();
-      }
-      // this stage's buffer is free (every wavefront holds its last fragments): the stage after the next is requested
-      // here, a full stage ahead of the barrier that needs it
-      if (!ABL_DMA && kt + 2 < KT) DA16_DMA(cur);
-      if (more) {
-        DA16_RB(b0, nxt, 0);
-        DA16_RA(a0, nxt, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      DA16_MMA(a1, b1, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      abl_first = false;
-    }
-    if (ABL_BAR) dma_wait();
-    __syncthreads();
-#undef DA16_DMA
-  } else {
+  {
     u32x4_t ra[NCH], rb[NCH];
     constexpr int A_RSTEP = A_KS ? C::NT / (BT / 8) : C::NT / 8;
     constexpr int B_RSTEP = B_KS ? C::NT / (BT / 8) : C::NT / 8;

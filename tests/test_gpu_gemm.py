@@ -94,6 +94,36 @@ def test_gemm_layouts(dev, a_ks, b_ks, dtype, M, N, K, batch):
     assert rel_fro(got2, ref2) < (6e-3 if dtype == torch.bfloat16 else 1e-6)
 
 
+# (two 128-tiles to a unit, the last two with columns that end inside a tile; 256-tiles, from eight stages on)
+@pytest.mark.parametrize("batch, M, N", [(3, 256, 384), (2, 256, 200), (2, 384, 8), (64, 512, 512)])
+@pytest.mark.parametrize("a_ks", [False, True])
+@pytest.mark.parametrize("b_ks", [False, True])
+def test_gemm_by_number_of_stages(dev, a_ks, b_ks, batch, M, N):
+    """One 64-deep stage, two, three, odd and even ones.  Small integers: every sum is exact, whatever its order."""
+    from dion_amd.newton_schulz import gemm
+
+    torch.manual_seed(6)
+    for K in (64, 128, 192, 256, 320) if batch < 64 else (512, 576, 640):
+        A, B = torch.randint(-2, 3, (batch, M, K)).float(), torch.randint(-2, 3, (batch, N, K)).float()
+        E = torch.randint(-9, 10, (batch, M, N)).float()
+        want = A @ B.mT
+        a, b = (t.bfloat16().mT.contiguous().to(dev) if ks else t.bfloat16().to(dev) for t, ks in ((A, a_ks), (B, b_ks)))
+        got = gemm(a, b, a_kstrided=a_ks, b_kstrided=b_ks, E=E.to(dev), s0=1.0, s1=1.0, out_dtype=torch.float32)
+        assert torch.equal(got.cpu(), want + E), K
+        assert torch.equal(gemm(a, b, a_kstrided=a_ks, b_kstrided=b_ks).cpu(), want.bfloat16()), K
+
+
+@pytest.mark.parametrize("m", [4096, 3912])
+def test_symmetric_products_by_number_of_stages(dev, m):
+    """192-tiles, whole and sliding ones."""
+    from dion_amd.newton_schulz import ns_line_1
+
+    torch.manual_seed(7)
+    for K in (64, 128, 192, 320):
+        A = torch.randint(-2, 3, (m, K)).float()
+        assert torch.equal(ns_line_1(A.bfloat16().to(dev)).cpu(), (A @ A.mT).bfloat16()), K
+
+
 def test_gemm_faithful_rounding_sequence(dev):
     """faithful=1 must reproduce torch's separate bf16 ops bit for bit when the matmul itself is exact
     (small integers: every product and partial sum is representable, so accumulation order is moot)."""
