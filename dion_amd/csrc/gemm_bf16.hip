@@ -244,7 +244,7 @@ int launch(const GemmDesc* d, int n, hipStream_t stream) {
   constexpr int BT = C::BT;
   static_assert(CG::BT == BT, "");
   constexpr int stage2 = 2 * (Tile<BT, A_KS>::bytes + Tile<BT, B_KS>::bytes);
-  constexpr int epi = (C::NT / 64) * 32 * (C::WCOLS + 4) * 4, epi_g = (CG::NT / 64) * 32 * (CG::WCOLS + 4) * 4;
+  constexpr int epi = epilogue_lds<C>(), epi_g = epilogue_lds<CG>();
   constexpr int smem = stage2 > epi ? (stage2 > epi_g ? stage2 : epi_g) : (epi > epi_g ? epi : epi_g);
   auto kfull = gemm_bf16_kernel<C, A_KS, B_KS, SYM, DA_LOOP_INTERIOR>;
   constexpr int CHECKED = C::SLIDE ? DA_LOOP_INTERIOR : DA_LOOP_CHECKED;
@@ -383,6 +383,7 @@ bool slide_ok(const GemmDesc* d, int n) {
 // 56 / 59;  and not: 12 of 768 x 3072 61 / 58;  5120 x 5120 293 / 235;  4096 x 14336 518 / 435.
 // Plain stores have less for two tiles to hide of one another.  (M, N, K), operands k-contiguous (c) or k-strided (s): 48 of
 // (768, 768, 768) c s 64 / 58, s s 62 / 57, c c 52 / 54;  12 of (3072, 768, 768) c s 61 / 55;  12 of (768, 768, 3072) c s 47 / 67.
+// (A little more still: beside the launches of two other streams, as in a full-rank Dion step, ties go to the 256-tiles, 3705 / 3612.)
 int choose_tile(const GemmDesc* d, int n) {
   static const int forced = [] { const char* e = getenv("DION_AMD_TILE"); return e ? atoi(e) : 0; }();
   if (forced == 128 || forced == 256) return forced;
@@ -400,7 +401,7 @@ int choose_tile(const GemmDesc* d, int n) {
   const bool addend = d[0].symmetric && d[0].epilogue == DA_EPI_AXPBY;
   const double cost_big = launch_cost<Big>(d, n, 256, 4.0, addend ? 0.0 : 3.0, 1.0);
   const double cost_small = addend ? launch_cost<Small>(d, n, 512, 3.0, 0.0, 1.0)
-                                   : launch_cost<Small>(d, n, 512, may_edge && d[0].epilogue == DA_EPI_STORE ? 3.0 : 2.75, 0.0, 0.55);
+                                   : launch_cost<Small>(d, n, 512, may_edge && d[0].epilogue == DA_EPI_STORE ? 3.2 : 2.75, 0.0, 0.55);
   const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
   if (d[0].symmetric && slide_ok(d, n)) {
     long long mid = 0, small = 0, matrices = 0;

@@ -137,6 +137,10 @@ __device__ __forceinline__ void update_weights8(char* Wp, bool w_f32, u32x4_t x0
   }
 }
 
+// LDS bytes of the epilogue: a band of fp32 results and one of bf16 results (to be turned) for each wavefront.
+template <typename C> constexpr int epilogue_lds() {
+  return (C::NT / 64) * 32 * ((C::WCOLS + 4) * 4 + (C::WCOLS <= 64 ? 128 : 256));
+}
 // UPD: 0 the result is stored in C; 1 / 2 it is not stored but updates the weights d.upd_tab[b] in place (2: those are
 // stored transposed), see GemmDesc.
 // RSPLIT, CSPLIT: a wavefront's rows (columns) are two runs, see Cfg::split.
@@ -148,11 +152,21 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   constexpr int PITCH = W + 4;       // floats; 16-byte aligned rows, conflict-free float4 writes
   constexpr int CPR = W / 8;         // 8-column chunks per row
   constexpr int RPP = 64 / CPR;      // rows per pass of the wavefront
-  constexpr int NPASS = (32 + RPP - 1) / RPP;
+  constexpr bool PIPE = C::QUAD && !(SYM && CF32);   // (see below)
+  // rows of a band; 16 of 128 columns, for the registers' sake: two staging areas then, taken in turns
+  constexpr int BR = PIPE && W == 128 ? 16 : 32, NB = C::WROWS / BR;
+  constexpr int NPASS = (BR + RPP - 1) / RPP;
   constexpr bool ODD = 64 % CPR != 0;   // (six chunks to a row: ten rows a pass, four lanes and most of the last pass idle)
   constexpr int CSZ = CF32 ? 4 : 2;
   constexpr int NV = CF32 ? 2 : 1;   // 16-byte vectors per 8 elements
+  // TURN: the bf16 results go through LDS a second time, to be stored transposed: 32 rows of the band as a k-strided tile ([32][W] in
+  // 32-byte slots, read_frag16), whose transpose read hands a lane eight consecutive rows of a column.
+  constexpr bool TURN = (SYM && !CF32) || UPD == 2;
+  constexpr int TPITCH = W <= 64 ? 128 : 256;
+  // PIPE: a band is written to LDS and requested back before the arithmetic of the one before it (with one wavefront to a SIMD
+  // nothing else covers the round trip; a wavefront's LDS operations run in order).
   float* stg = reinterpret_cast<float*>(lds) + wave * (32 * PITCH);
+  char* const trn = lds + (C::NT / 64) * (32 * PITCH * 4) + wave * (32 * TPITCH);
   // the descriptor lives in the kernel-argument segment: fields read inside the band loop would be fetched
   // again after every store (scalar load + a full wait in the middle of the band), so they are copied first
   const float s0 = d.s0, s1 = d.s1;
@@ -160,7 +174,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   const int dM = d.M, dN = d.N;
   const long long ldc = d.ldc, lde = d.lde;
   const int wm0 = m0 + wm * (RSPLIT ? 32 : C::WROWS), wn0 = n0 + wn * (CSPLIT ? 32 : W);
-  auto row_of = [&](int band) { return wm0 + band * (RSPLIT ? 64 : 32); };            // first row of a band
+  auto row_of = [&](int band) { return wm0 + (RSPLIT ? band * 64 : band * BR); };        // first row of a band
   auto col_of = [&](int c) { return wn0 + (CSPLIT ? (c & 31) + (c >> 5) * 64 : c); };   // column c of the wavefront's
   char* const Cbase = d.Ctab ? static_cast<char*>(d.Ctab[b]) : static_cast<char*>(d.C) + (long long)b * d.sC * CSZ;
   const char* const Ebase = !HAS_E ? nullptr
@@ -175,16 +189,16 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   const float w_decay = d.upd_decay, w_step = d.upd_step;
   // E is requested up to three bands ahead (registers that the K loop's fragments no longer need), so that a
   // tile's epilogue pays one memory latency and not one per band; an fp32 E (twice the registers) one band ahead.
-  constexpr int DEPTH = (!HAS_E || CF32) ? 1 : (UPD ? 2 : (C::NB < 3 ? C::NB : 3));
+  constexpr int DEPTH = (!HAS_E || CF32) ? 1 : BR == 16 ? (UPD ? 2 : 4) : (UPD ? 2 : (NB < 3 ? NB : 3));
   u32x4_t ev[DEPTH][NPASS][NV];
   // the weights a band updates are requested when the band starts, ahead of its staging through LDS and of the
   // arithmetic on E (two vectors per 8 elements when they are fp32)
-  constexpr int NWP = UPD == 2 ? (W + 63) / 64 * 4 : NPASS;
+  constexpr int NWP = UPD == 2 ? W / 16 : NPASS;
   constexpr int NWV = WF32 ? 2 : 1;
   u32x4_t wv[NWP][NWV];
   auto weight_ptr = [&](int band, int pass) -> char* {
     if (UPD == 2) {
-      const int n = col_of((pass >> 2) * 64 + lane), m = row_of(band) + (pass & 3) * 8;
+      const int n = col_of(pass * 16 + (lane & 15)), m = row_of(band / (32 / BR) * (32 / BR)) + (lane >> 4) * 8;
       return Wbase + ((long long)n * ldw + m) * wsz;
     }
     const int m = row_of(band) + pass * RPP + lr;
@@ -206,7 +220,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
       const u32x4_t z = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int h = 0; h < NV; ++h) dst[pass][h] = z;
-      if (col_ok && (FULL || m < dM) && (!ODD || pass * RPP + lr < 32)) {
+      if (col_ok && (FULL || m < dM) && (!ODD || pass * RPP + lr < BR)) {
         const char* Ep = Ebase + ((long long)m * lde + cn) * CSZ;
 #pragma unroll
         for (int h = 0; h < NV; ++h) dst[pass][h] = ldg16(Ep + 16 * h);
@@ -217,9 +231,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
 #pragma unroll
     for (int q = 0; q < DEPTH; ++q) load_e(q, ev[q]);
   }
-#pragma unroll
-  for (int i = 0; i < C::NB; ++i) {
-    if (UPD) load_w(i, wv);
+  auto put_band = [&](int i) {
     if (C::MI == 32) {
       float* row = stg + (lane & 31) * PITCH + (lane >> 5) * 4;
 #pragma unroll
@@ -230,16 +242,42 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
               make_float4(acc[i][j][vq * 4], acc[i][j][vq * 4 + 1], acc[i][j][vq * 4 + 2], acc[i][j][vq * 4 + 3]);
     } else {
       // 16 x 16 blocks: a lane holds, for row (lane & 15) of a block, the four columns 4 (lane >> 4) .. + 3
-      float* row = stg + (lane & 15) * PITCH + (lane >> 4) * 4;
+      float* row = stg + (BR == 16 ? (i & 1) * 16 * PITCH : 0) + (lane & 15) * PITCH + (lane >> 4) * 4;
 #pragma unroll
-      for (int ib = 0; ib < 2; ++ib)
+      for (int ib = 0; ib < BR / 16; ++ib)
 #pragma unroll
         for (int j = 0; j < C::TNJ; ++j) {
-          const typename C::acc_t& a = acc[(2 * i + ib) % C::TMI][j];
+          const typename C::acc_t& a = acc[(BR / 16 * i + ib) % C::TMI][j];
           *reinterpret_cast<float4*>(row + ib * 16 * PITCH + j * 16) = make_float4(a[0], a[1], a[2], a[3]);
         }
     }
     wave_sync_lds();
+  };
+  float4 raw[PIPE ? 2 : 1][NPASS][2];
+  auto get_pass = [&](int i, int pass, float4 (&dst)[2]) {
+    if (!ODD || pass * RPP + lr < BR) {
+      const float* sp = stg + (BR == 16 ? (i & 1) * 16 * PITCH : 0) + (pass * RPP + lr) * PITCH + c8;
+      dst[0] = *reinterpret_cast<const float4*>(sp);
+      dst[1] = *reinterpret_cast<const float4*>(sp + 4);
+    }
+  };
+  auto get_band = [&](int i, float4 (&dst)[NPASS][2]) {
+#pragma unroll
+    for (int pass = 0; pass < NPASS; ++pass) get_pass(i, pass, dst[pass]);
+    wave_sync_lds();
+  };
+  if (PIPE) {
+    put_band(0);
+    get_band(0, raw[0]);
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if (UPD == 1 || (UPD == 2 && i % (32 / BR) == 0)) load_w(i, wv);
+    if (!PIPE) put_band(i);
+    else if (i + 1 < NB) {
+      put_band(i + 1);
+      get_band(i + 1, raw[(i + 1) & (PIPE ? 1 : 0)]);
+    }
     const int band_m = row_of(i);
     u32x4_t ec[NPASS][NV];
     if (HAS_E) {
@@ -247,17 +285,17 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
       for (int pass = 0; pass < NPASS; ++pass)
 #pragma unroll
         for (int h = 0; h < NV; ++h) ec[pass][h] = ev[i % DEPTH][pass][h];
-      if (i + DEPTH < C::NB) load_e(i + DEPTH, ev[i % DEPTH]);
+      if (i + DEPTH < NB) load_e(i + DEPTH, ev[i % DEPTH]);
     }
 
 #pragma unroll
     for (int pass = 0; pass < NPASS; ++pass) {
       const int r = pass * RPP + lr;
       const int m = band_m + r;
-      if (col_ok && (FULL || m < dM) && (!ODD || r < 32)) {
+      if (col_ok && (FULL || m < dM) && (!ODD || r < BR)) {
         float* sp = stg + r * PITCH + c8;
-        const float4 a0 = *reinterpret_cast<const float4*>(sp);
-        const float4 a1 = *reinterpret_cast<const float4*>(sp + 4);
+        if (!PIPE) get_pass(i, pass, raw[0][pass]);
+        const float4 a0 = raw[PIPE ? i & 1 : 0][pass][0], a1 = raw[PIPE ? i & 1 : 0][pass][1];
         float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
         float e[8];
         char* Cp = Cbase + ((long long)m * ldc + cn) * CSZ;
@@ -282,17 +320,11 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
             const unsigned w = HAS_E ? ec[pass][0][q] : 0u;   // (copied out: see the note on bit_cast above)
             const unsigned o = epi_pair<HAS_E, FAITHFUL, S1_ONE>(s0, s1, v[2 * q], v[2 * q + 1], w);
             pk[q] = o;
-            if (SYM) {
-              v[2 * q] = lo_f(o);
-              v[2 * q + 1] = hi_f(o);
-            }
           }
           if (UPD == 0) stg16(Cp, pk);
           if (UPD == 1) update_weights8(weight_ptr(i, pass), w_f32, wv[pass][0], wv[pass][NWV - 1], pk, w_decay, w_step);
-          if (UPD == 2) {   // the final values stay in the staging area for the transposed pass below
-            *reinterpret_cast<float4*>(sp) = make_float4(lo_f(pk[0]), hi_f(pk[0]), lo_f(pk[1]), hi_f(pk[1]));
-            *reinterpret_cast<float4*>(sp + 4) = make_float4(lo_f(pk[2]), hi_f(pk[2]), lo_f(pk[3]), hi_f(pk[3]));
-          }
+          if (TURN && (UPD == 2 || mirror))
+            *reinterpret_cast<u32x4_t*>(trn + (r + i % (32 / BR) * BR) * TPITCH + (((c8 >> 4) ^ (r & 3)) * 32 + (c8 & 8) * 2)) = pk;
           if (!HAS_E && !FAITHFUL && !SYM && c2) {
             // what the stored bf16 leaves of s1 * acc, as a second bf16 matrix
             u32x4_t lo;
@@ -301,58 +333,54 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
             stg16(Cp + c2, lo);
           }
         }
-        if (SYM && mirror) {  // keep the final values for the transposed store
+        if (SYM && CF32 && mirror) {  // keep the final values for the transposed store
           *reinterpret_cast<float4*>(sp) = make_float4(v[0], v[1], v[2], v[3]);
           *reinterpret_cast<float4*>(sp + 4) = make_float4(v[4], v[5], v[6], v[7]);
         }
       }
     }
-    if (UPD == 2) {
+    // Transposed: row n of the mirrored tile (of the weights) holds 32 consecutive m of this band.  Where sliding tiles overlap, what a
+    // diagonal tile stores (from E itself) is left to it: with E(m, n) here and E(n, m) there, an E that is not symmetric would leave either.
+    const int n_own = C::SLIDE && n0 + C::BT >= dN ? (dN - 1) / C::BT * C::BT : 0;
+    const int m_end = C::SLIDE ? dM - C::BT : 0;
+    if (TURN && (UPD == 2 || mirror) && (i + 1) % (32 / BR) == 0) {
       wave_sync_lds();
-      // the weights are stored transposed: row n of W holds 32 consecutive m of this band
 #pragma unroll
-      for (int pass = 0; pass < (W / 64) * 4; ++pass) {
-        const int nl = (pass >> 2) * 64 + lane;
-        const int mg = (pass & 3) * 8;
-        const int n = col_of(nl), m = band_m + mg;
-        if (FULL || (n < dN && m < dM)) {
-          u32x4_t pk;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) pk[q] = cvt_pk_bf16(stg[(mg + 2 * q) * PITCH + nl], stg[(mg + 2 * q + 1) * PITCH + nl]);
-          update_weights8(weight_ptr(i, pass), w_f32, wv[pass][0], wv[pass][NWV - 1], pk, w_decay, w_step);
+      for (int slot = 0; slot < W / 16; ++slot) {
+        const int g = lane >> 4, q = (lane & 15) >> 2;
+        const char* p = trn + (g * 8 + q) * TPITCH + (slot ^ q) * 32 + (lane & 3) * 8;
+        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(DA_LDS_PTR(s16x4_t, p));
+        const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(DA_LDS_PTR(s16x4_t, p + 4 * TPITCH));
+        typedef short s16x8_t __attribute__((ext_vector_type(8)));
+        const s16x8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        const u32x4_t pk = __builtin_bit_cast(u32x4_t, v);
+        const int n = col_of(slot * 16 + (lane & 15)), m = row_of(i + 1 - 32 / BR) + g * 8;
+        if (C::SLIDE && (n < n_own || m >= m_end)) continue;
+        if (FULL || (n < dN && m < dM)) {   // M is a multiple of 8 for symmetric outputs
+          if (UPD == 2) update_weights8(weight_ptr(i, slot), w_f32, wv[slot][0], wv[slot][NWV - 1], pk, w_decay, w_step);
+          else stg16(Cbase + ((long long)n * ldc + m) * CSZ, pk);
         }
       }
     }
-    if (SYM && mirror) {
+    if (SYM && CF32 && mirror) {
       wave_sync_lds();
-      // C^T: row n of the mirrored tile holds 32 consecutive m of this band.  Where sliding tiles overlap, what a diagonal tile stores
-      // (from E itself) is left to it: with E(m, n) here and E(n, m) there, an E that is not symmetric would leave either.
-      const int n_own = C::SLIDE && n0 + C::BT >= dN ? (dN - 1) / C::BT * C::BT : 0;
-      const int m_end = C::SLIDE ? dM - C::BT : 0;
 #pragma unroll
       for (int pass = 0; pass < (W + 63) / 64 * 4; ++pass) {
         const int nl = (pass >> 2) * 64 + lane;
         const int mg = (pass & 3) * 8;
         const int n = wn0 + nl, m = band_m + mg;
         if (C::SLIDE && (n < n_own || m >= m_end)) continue;
-        if ((FULL || (n < dN && m < dM)) && (W % 64 == 0 || nl < W)) {  // M is a multiple of 8 for symmetric outputs
+        if ((FULL || (n < dN && m < dM)) && (W % 64 == 0 || nl < W)) {
           float v[8];
 #pragma unroll
           for (int q = 0; q < 8; ++q) v[q] = stg[(mg + q) * PITCH + nl];
           char* Cp = Cbase + ((long long)n * ldc + m) * CSZ;
-          if (CF32) {
-            const u32x4_t o0 = {__builtin_bit_cast(unsigned, v[0]), __builtin_bit_cast(unsigned, v[1]),
-                                __builtin_bit_cast(unsigned, v[2]), __builtin_bit_cast(unsigned, v[3])};
-            const u32x4_t o1 = {__builtin_bit_cast(unsigned, v[4]), __builtin_bit_cast(unsigned, v[5]),
-                                __builtin_bit_cast(unsigned, v[6]), __builtin_bit_cast(unsigned, v[7])};
-            stg16(Cp, o0);
-            stg16(Cp + 16, o1);
-          } else {
-            u32x4_t pk;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) pk[q] = cvt_pk_bf16(v[2 * q], v[2 * q + 1]);
-            stg16(Cp, pk);
-          }
+          const u32x4_t o0 = {__builtin_bit_cast(unsigned, v[0]), __builtin_bit_cast(unsigned, v[1]),
+                              __builtin_bit_cast(unsigned, v[2]), __builtin_bit_cast(unsigned, v[3])};
+          const u32x4_t o1 = {__builtin_bit_cast(unsigned, v[4]), __builtin_bit_cast(unsigned, v[5]),
+                              __builtin_bit_cast(unsigned, v[6]), __builtin_bit_cast(unsigned, v[7])};
+          stg16(Cp, o0);
+          stg16(Cp + 16, o1);
         }
       }
     }
