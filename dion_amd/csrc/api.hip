@@ -540,12 +540,18 @@ bool dtype_ok(int d) { return d == DA_BF16 || d == DA_F32; }
 // Run-time options (dion_amd_set_option).  -1: not set by the caller, the environment decides.
 std::atomic<int> g_opt_fused_update{-1};
 
-// Error feedback and weight update as one pass (the default) or as two AXPBY products.
-bool fused_update_enabled() {
+// Dion's error feedback and weight update, bf16 momentum: 1 as one pass over M and X, 0 as two AXPBY products with that pass's
+// bits, -1 (nobody asked for either) as the products of the 16x16x32 instruction, M's and X's in one launch, or with fp32 weights
+// as the one pass where it applies.
+// (us a step, the pass / the products in one launch.  Several buckets on their streams, which the pass's workgroups, one to a CU
+// from start to end, keep waiting: GPT-small at rank 192 712 / 697, at full rank 3605 / 3560, MLP matrices of a Llama-70B
+// layer 4645 / 4570.  One bucket: 48 of 768 x 768 at rank 64 213 / 211, 4 of 4096 x 4096 at rank 512 775 / 761, at rank 256 580 / 588,
+// 2 of 14336 x 4096 at rank 64 600 / 593, 2 of 4096 x 14336 at rank 256 813 / 832;  fp32 weights, two launches: 947 / 970, 422 / 438.)
+int update_form() {
   const int v = g_opt_fused_update.load(std::memory_order_relaxed);
   if (v >= 0) return v != 0;
   static const bool env_off = getenv("DION_AMD_NO_FUSED") != nullptr;
-  return !env_off;
+  return env_off ? 0 : -1;
 }
 
 // B = M + G inside the launch of P = B Q (the default where it applies) or as a pass of its own.
@@ -1228,7 +1234,8 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
       }
     }  // power iterations
     // ---- error feedback, column normalisation and weight update (reference dion/dion.py:851-872)
-    if (faithful && fused_update_enabled() && da_dion_ef_update_applicable(mp, np, r, m_dtype)) {
+    const int form = update_form();
+    if (faithful && (form > 0 || (form < 0 && x_dtype == DA_F32)) && da_dion_ef_update_applicable(mp, np, r, m_dtype)) {
       // Q_new first (it only needs R), then both rank-r updates in one pass over M and X
       {
         DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);
@@ -1242,32 +1249,34 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
       continue;
     }
     // ---- error feedback  M <- M - (1 - mu) P R^T  (or R P^T)   (reference dion/dion.py:851-853)
-    g = GemmDesc{};
-    g.batch = cb; g.faithful = faithful;
-    if (!transposed) { g.A = P; g.sA = sP; g.B = R; g.sB = sQ; g.M = mp; g.N = np; }
-    else             { g.A = R; g.sA = sQ; g.B = P; g.sB = sP; g.M = np; g.N = mp; }
-    g.lda = r; g.ldb = r; g.K = r;
-    g.Ctab = tabM; g.Etab = const_cast<const void* const*>(tabM); g.ldc = n; g.lde = n; g.c_dtype = m_dtype;
-    g.epilogue = DA_EPI_AXPBY; g.s0 = 1.f; g.s1 = ef_alpha;
-    g.mi32 = 1;   // (the bits of the one-pass kernel)
-    rc = gemm_any(g, m_dtype, s, DA_PROF_DION_EF);
-    if (rc) return rc;
+    GemmDesc up[2] = {GemmDesc{}, GemmDesc{}};
+    for (int k = 0; k < 2; ++k) {
+      GemmDesc& u = up[k];
+      const char* const D = k == 0 ? R : Qn;
+      u.batch = cb; u.faithful = faithful;
+      if (!transposed) { u.A = P; u.sA = sP; u.B = D; u.sB = sQ; u.M = mp; u.N = np; }
+      else             { u.A = D; u.sA = sQ; u.B = P; u.sB = sP; u.M = np; u.N = mp; }
+      u.lda = r; u.ldb = r; u.K = r; u.ldc = n; u.lde = n;
+      u.epilogue = DA_EPI_AXPBY;
+      u.mi32 = form == 0;   // (the bits of the one-pass kernel)
+    }
+    up[0].Ctab = tabM; up[0].Etab = const_cast<const void* const*>(tabM); up[0].c_dtype = m_dtype;
+    up[0].s0 = 1.f; up[0].s1 = ef_alpha;
+    // ---- X <- (1 - lr wd) X - scaled_lr P Q_new^T  (or Q_new P^T)   (reference dion/dion.py:865-872)
+    up[1].Ctab = tabX; up[1].Etab = const_cast<const void* const*>(tabX); up[1].c_dtype = x_dtype;
+    up[1].s0 = decay; up[1].s1 = -scaled_lr;
+    const bool together = form < 0 && m_dtype == DA_BF16 && x_dtype == DA_BF16;
+    if (!together) {
+      rc = gemm_any(up[0], m_dtype, s, DA_PROF_DION_EF);
+      if (rc) return rc;
+    }
     // ---- Q_new = column-normalised R   (reference dion/dion.py:856, 875, 1460-1491, 1533-1561)
     {
       DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);
       rc = da_colnorm(R, Qn, m_dtype, tq, q_dtype, np, r, rank, eps, cb, reinterpret_cast<double*>(orth_ws), s);
       if (rc) return rc;
     }
-    // ---- X <- (1 - lr wd) X - scaled_lr P Q_new^T  (or Q_new P^T)   (reference dion/dion.py:865-872)
-    g = GemmDesc{};
-    g.batch = cb; g.faithful = faithful;
-    if (!transposed) { g.A = P; g.sA = sP; g.B = Qn; g.sB = sQ; g.M = mp; g.N = np; }
-    else             { g.A = Qn; g.sA = sQ; g.B = P; g.sB = sP; g.M = np; g.N = mp; }
-    g.lda = r; g.ldb = r; g.K = r;
-    g.Ctab = tabX; g.Etab = const_cast<const void* const*>(tabX); g.ldc = n; g.lde = n; g.c_dtype = x_dtype;
-    g.epilogue = DA_EPI_AXPBY; g.s0 = decay; g.s1 = -scaled_lr;
-    g.mi32 = 1;
-    rc = gemm_any(g, m_dtype, s, DA_PROF_DION_UPD);
+    rc = together ? gemm_group(up, 2, m_dtype, s, DA_PROF_DION_EFUPD) : gemm_any(up[1], m_dtype, s, DA_PROF_DION_UPD);
     if (rc) return rc;
   }
   return DA_OK;
