@@ -712,7 +712,7 @@ int dion_amd_sym_poly(const void* A, long long a_stride, int lda, void* C, long 
   g.sA = a_stride; g.sB = a_stride; g.sC = c_stride; g.sE = a_stride;
   g.lda = lda; g.ldb = lda; g.ldc = ldc; g.lde = lda;
   g.M = m; g.N = m; g.K = m; g.batch = batch;
-  g.symmetric = 1; g.epilogue = DA_EPI_AXPBY; g.s0 = beta; g.s1 = alpha; g.faithful = faithful; g.c_dtype = dtype;
+  g.symmetric = 1; g.any_addend = 1; g.epilogue = DA_EPI_AXPBY; g.s0 = beta; g.s1 = alpha; g.faithful = faithful; g.c_dtype = dtype;
   return gemm_any(g, dtype, static_cast<hipStream_t>(stream));
 }
 

@@ -112,6 +112,8 @@ struct GemmDesc {
   int batch;
   int a_kstrided, b_kstrided;
   int symmetric;      // 1: C is symmetric (M == N); compute upper tiles and mirror
+  int any_addend;     // bf16, symmetric with an E from a caller, who may hand one in that is not symmetric: the tile edge, which decides
+                      // between E(m, n) and E(n, m) then, follows its own rule (choose_tile)
   int epilogue;       // DA_EPI_*
   int faithful;       // 1: reproduce every bf16 rounding of the op-by-op reference
   float s0, s1;       // epilogue scalars

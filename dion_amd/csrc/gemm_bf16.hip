@@ -396,11 +396,13 @@ int choose_tile(const GemmDesc* d, int n) {
   const bool may_edge = !d[0].symmetric && (d[0].a_kstrided || d[0].b_kstrided);
   const bool full_big = all_interior(d, n, 256) || (may_edge && edge_loop_ok(d, n, 256));
   const bool full_small = all_interior(d, n, 128) || (may_edge && edge_loop_ok(d, n, 128));
-  // A symmetric product with an addend: where a caller's addend is not symmetric the tile edge decides which of E(m, n) and E(n, m)
-  // an element gets.  Its rule (constants of an older K loop, up to 12 % from the best edge for b A + c A A) stays as it is for that.
-  const bool addend = d[0].symmetric && d[0].epilogue == DA_EPI_AXPBY;
-  const double cost_big = launch_cost<Big>(d, n, 256, 4.0, addend ? 0.0 : 3.0, 1.0);
-  const double cost_small = addend ? launch_cost<Small>(d, n, 512, 3.0, 0.0, 1.0)
+  // Where a caller's addend is not symmetric the tile edge decides which of E(m, n) and E(n, m) an element gets: the rule for those
+  // products (constants of an older K loop, up to 12 % from the best edge) stays as it is.  (Newton-Schulz's own A is symmetric.)
+  const bool addend = d[0].symmetric && d[0].any_addend && d[0].epilogue == DA_EPI_AXPBY;
+  // (The older constants also where the bounds-checked loop runs, for which they were measured.)
+  const bool older = addend || !(full_big || full_small);
+  const double cost_big = launch_cost<Big>(d, n, 256, 4.0, older ? 0.0 : 3.0, 1.0);
+  const double cost_small = older ? launch_cost<Small>(d, n, 512, 3.0, 0.0, 1.0)
                                    : launch_cost<Small>(d, n, 512, may_edge && d[0].epilogue == DA_EPI_STORE ? 3.2 : 2.75, 0.0, 0.55);
   const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
   if (d[0].symmetric && slide_ok(d, n)) {
@@ -429,7 +431,7 @@ int da_gemm_bf16_grouped(const GemmDesc* din, int n, hipStream_t stream) {
     if (rc) return rc;
     const GemmDesc &a = din[g], &f = din[0];
     if (a.symmetric != f.symmetric || a.a_kstrided != f.a_kstrided || a.b_kstrided != f.b_kstrided ||
-        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || (a.mi32 != 0) != (f.mi32 != 0))
+        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || (a.mi32 != 0) != (f.mi32 != 0) || a.any_addend != f.any_addend)
       return DA_ERR_ARG;
     if (a.mi32 && (a.symmetric || a.a_kstrided || a.b_kstrided)) return DA_ERR_ARG;
     // insertion sort, longest K first: long tiles start early, short ones fill the tail
