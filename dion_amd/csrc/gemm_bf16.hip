@@ -1,5 +1,5 @@
 // Batched bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16, fp32 accumulate; the 32x32x16 form of the
-// instruction is kept as a build variant and for GemmDesc::mi32: under the 16x16x32 form the chip holds a 13 % higher
+// instruction is kept for GemmDesc::mi32 and as a build variant: under the 16x16x32 form the chip holds a 13 % higher
 // clock at the same flops per pass, which is worth 3 % to the whole K loop).
 //
 //   C[b] (M x N) = epilogue( sum_k Aop[b](i,k) * Bop[b](j,k) )

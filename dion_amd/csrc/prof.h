@@ -18,7 +18,7 @@ enum DaProfKind {
   DA_PROF_DION_ORTH = 11, // orthonormalisation of P (all of its launches)
   DA_PROF_DION_ELEM = 12, // B = M + G, column norms, guards
   DA_PROF_SCALAR_OPT = 13,// fused Lion / AdamW pass over non-matrix parameters
-  DA_PROF_DION_EFUPD = 14,// error feedback and weight update in one pass
+  DA_PROF_DION_EFUPD = 14,// error feedback and weight update in one launch
   DA_PROF_NS_FLOW = 15,   // all Newton-Schulz iterations of a set of buckets in one persistent launch
   DA_PROF_DION_SMALL = 16,// a whole Dion step of small matrices
   DA_PROF_KINDS = 17
