@@ -222,7 +222,7 @@ def summarize(name, wl, res):
             r = min(math.ceil(wl["rank_fraction"] * min(m, n)), m, n)
             rd += 2.0 * (m * n + (m + n) * r)
             upd += 2.0 * (2 * m * n + (m + n) * r)
-            # error feedback and weight update as one pass: M and X read and written once, P, R and Q_new read
+            # error feedback and weight update in one launch: M and X read and written once, P, R and Q_new read
             fused += 2.0 * (4 * m * n + (max(m, n) + 2 * min(m, n)) * r)
         for name, nbytes in (("dion_bq", bq), ("dion_btp", rd), ("dion_ef", upd), ("dion_upd", upd),
                              ("dion_ef_upd", fused)):
@@ -236,24 +236,24 @@ def summarize(name, wl, res):
 # HBM bytes per launch of the dominant kernel, from two `rocprofv3 --pmc` runs (FETCH_SIZE x 2.000 and
 # WRITE_SIZE x 1.000, in KiB, the factors being what the same counters read for a plain 512 MiB copy);
 # the runs used the workload named in the key with three 512 MiB copies first (--calibrate-copy).  Keyed by
-# (workload, kernel); measured 2026-11-25 on the kernels of this revision (profiles/*_hbm_traffic.md hold the runs);
+# (workload, kernel); measured 2026-12-02 on the kernels of this revision (profiles/*_hbm_traffic.md hold the runs);
 # a kernel kind that is not listed has not been measured since it last changed and reports null.
 MEASURED_TRAFFIC_BYTES = {
     # the persistent Newton-Schulz launch: all 15 products of all 72 matrices
-    ("muon_gpt_small", "ns_flow"): 5910473 * 1024,
+    ("muon_gpt_small", "ns_flow"): 5997609 * 1024,
     # X' = aX + BX over the 32 matrices (mean of the five launches; the last one updates the weights instead of storing X')
-    ("muon_4096x14336", "ns_axpy"): 29839601 * 1024,
+    ("muon_4096x14336", "ns_axpy"): 30044150 * 1024,
     # one Llama-3-8B layer: the grouped X' = aX + BX launch over its four buckets
-    ("muon_llama8b_layer", "ns_axpy"): 3534072 * 1024,
-    # error feedback + weight update in one pass: mean over the buckets of the workload
-    ("dion_gpt_small_r025", "dion_ef_upd"): 277687 * 1024,
-    ("dion_llama70b_layer", "dion_ef_upd"): 4027315 * 1024,
-    # mean over the three buckets (two launches of the non-transposed kernel, one of the transposed one)
-    ("dion_gpt_small_r1", "dion_ef_upd"): 446671 * 1024,
+    ("muon_llama8b_layer", "ns_axpy"): 3544863 * 1024,
+    # error feedback + weight update in one launch: mean over the buckets of the workload
+    ("dion_gpt_small_r025", "dion_ef_upd"): 266764 * 1024,
+    ("dion_llama70b_layer", "dion_ef_upd"): 3511913 * 1024,
+    # mean over the three buckets
+    ("dion_gpt_small_r1", "dion_ef_upd"): 524478 * 1024,
     # the 16-matrix and the 8-matrix bucket: mean of the two launches
-    ("dion_llama70b_mlp", "dion_ef_upd"): 33113826 * 1024,
+    ("dion_llama70b_mlp", "dion_ef_upd"): 32323032 * 1024,
     # the grouped X' = aX + BX launch over all 224 matrices
-    ("muon_llama8b", "ns_axpy"): 108596291 * 1024,
+    ("muon_llama8b", "ns_axpy"): 109270265 * 1024,
     # mean of the AdamW launch (lm_head) and the Lion launch (embedding, norms)
     ("scalar_gpt_small", "scalar_opt"): 453078 * 1024,
 }
