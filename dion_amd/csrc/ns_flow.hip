@@ -349,7 +349,8 @@ std::atomic<int> g_flow_fail{0};           // test hook: the launch starts with 
 std::atomic<long long> g_flow_spin{-1};    // ticks of the 100 MHz counter; -1: default
 
 double tile_cost(int stages, int product) {
-  // microseconds, from the tile time lines of the batched kernel: 1.7 per 64-deep stage, epilogue, ticket + wait
+  // microseconds, from tile time lines: 1.7 per 64-deep stage, epilogue, ticket + wait (now 1.5, 5.8 - 10 and the first stage's 5:
+  // only the ratios of the queues' loads are used)
   const double epi = product == 2 ? 5.5 : (product == 1 ? 4.5 : 4.0);
   return 1.7 * stages + epi + 1.0;
 }
