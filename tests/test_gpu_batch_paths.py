@@ -80,6 +80,45 @@ def test_fused_update_pass_equals_the_two_products_bit_for_bit(dev, shapes, rank
     assert not torch.equal(runs[0][1][0].detach(), X[0])
 
 
+@pytest.mark.parametrize("shapes,rank_fraction", [
+    ([(768, 512)] * 3 + [(512, 1024)] * 2, 0.25),      # whole tiles, tall and wide
+    ([(648, 264)] * 2 + [(200, 1032)], 0.3),           # rank 80 and 60, edges of tiles: the bounds-checked loop
+    ([(4096, 64)] * 2, 1.0),                           # one stage
+])
+def test_update_in_one_launch_is_the_two_products(dev, shapes, rank_fraction):
+    """The default form (both products of bf16 weights in one launch) against the two launches of the other matrix instruction: the
+    same fp32 sums in another order inside an instruction, then bf16 roundings of the product, at most as large as the old and the new
+    value together, and of the result that may each fall one step (2^-7) apart."""
+    from dion_amd import _lib
+
+    X, gen = _dion_problem(dev, shapes, 22)
+    G = [(torch.randn(s, generator=gen, device=dev) * 1e-3).to(BF) for s in shapes]
+    runs = []
+    try:
+        _lib.set_option("dion_small", 0)
+        for form in (0, -1):
+            _lib.set_option("fused_update", form)
+            torch.manual_seed(5)
+            opt, params, states = _make_dion(dev, X, rank_fraction)
+            if runs:
+                for st, ref in zip(states, runs[0][2]):
+                    st["Q"].copy_(ref)
+            q0 = [st["Q"].clone() for st in states]
+            for p, g in zip(params, G):
+                p.grad = g
+            opt.step()
+            torch.cuda.synchronize()
+            runs.append((params, states, q0))
+    finally:
+        _lib.set_option("fused_update", -1)
+        _lib.set_option("dion_small", -1)
+    for p, q, s, t, x, g in zip(runs[0][0], runs[1][0], runs[0][1], runs[1][1], X, G):
+        assert torch.equal(s["Q"], t["Q"])
+        assert not torch.equal(q.detach(), x)
+        for a, b, old in ((p.detach(), q.detach(), x), (s["momentum"], t["momentum"], g)):   # (the momentum was zero before g)
+            assert torch.all((a.float() - b.float()).abs() <= 2.0**-7 * (2 * a.float().abs() + old.float().abs()))
+
+
 def test_dion_step_serial_and_threaded_enqueue_give_the_same_bits(dev, monkeypatch):
     """Three buckets: once with the default path (one worker thread and stream per bucket of a wave), once with
     DION_AMD_DION_SERIAL=1 (the caller's thread, one call after the other; also what runs under stream capture)."""
