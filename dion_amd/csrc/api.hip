@@ -300,8 +300,10 @@ int ns_iterate(const NsSet* sets, int nsets, int dtype, const float* coeffs, int
       g[i].a_kstrided = 0; g[i].b_kstrided = 1; g[i].symmetric = 0;
       g[i].epilogue = DA_EPI_AXPBY; g[i].s0 = a; g[i].s1 = 1.f;
     }
-    if (want_update && it + 1 == steps && da_gemm_bf16_all_interior(g, nsets)) {
+    const int plan = want_update && it + 1 == steps ? da_gemm_bf16_group_plan(g, nsets) : 0;
+    if (plan > 0 && (plan & 1)) {
       for (int i = 0; i < nsets; ++i) {
+        g[i].tile = plan - 1;
         g[i].upd_tab = sets[i].W.xtab; g[i].upd_dtype = sets[i].x_dtype; g[i].upd_ld = sets[i].x_ld;
         g[i].upd_transposed = sets[i].tall; g[i].upd_decay = sets[i].decay; g[i].upd_step = sets[i].step;
       }
@@ -878,6 +880,21 @@ int dion_amd_gemm_plan(int M, int N, int K, int lda, int a_kstrided, int ldb, in
   g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldb = ldb; g.batch = 1;
   g.a_kstrided = a_kstrided != 0; g.b_kstrided = b_kstrided != 0;
   return da_gemm_bf16_plan(g);
+}
+
+int dion_amd_gemm_group_plan(const int* batch, const int* M, const int* N, const int* K, int n, int a_kstrided, int b_kstrided,
+                             int epilogue) {
+  if (!batch || !M || !N || !K || n <= 0 || n > DA_MAX_GROUPS) return DA_ERR_ARG;
+  GemmDesc g[DA_MAX_GROUPS];
+  for (int i = 0; i < n; ++i) {
+    if (batch[i] <= 0 || M[i] <= 0 || N[i] <= 0 || K[i] <= 0) return DA_ERR_ARG;
+    g[i] = GemmDesc{};
+    g[i].batch = batch[i]; g[i].M = M[i]; g[i].N = N[i]; g[i].K = K[i];
+    g[i].a_kstrided = a_kstrided != 0; g[i].b_kstrided = b_kstrided != 0;
+    g[i].lda = a_kstrided ? M[i] : K[i]; g[i].ldb = b_kstrided ? N[i] : K[i];
+    g[i].epilogue = epilogue;
+  }
+  return da_gemm_bf16_group_plan(g, n);
 }
 
 size_t dion_amd_muon_buckets_workspace_bytes(const dion_amd_muon_bucket* buckets, int nbuckets) {

@@ -149,6 +149,9 @@ struct GemmDesc {
   // per instruction instead of 32: another order of the fp32 sums).  Dion's error-feedback and weight-update products
   // use it where their bits have to be those of the one-pass kernel (dion_fused.hip), which is built on that instruction.
   int mi32;
+  // bf16 only.  The tile edge to run (0: the launcher chooses).  A caller whose descriptors depend on the choice, as upd_tab does,
+  // asks da_gemm_bf16_group_plan for it and hands it on, so that what was asked about is what runs.
+  int tile;
 };
 
 // Epilogues.  With `faithful` set the rounding points of the reference's separate
@@ -171,5 +174,6 @@ int da_gemm_f32(const GemmDesc& d, hipStream_t stream);
 int da_gemm_bf16_plan(const GemmDesc& d);
 // -1 / 0 / 1: whether ragged products may take the direct-to-LDS K loop with edge tiles (see dion_amd_set_option)
 void da_gemm_bf16_set_edge_loop(int v);
-// Whether da_gemm_bf16_grouped would run every tile of these products in its interior (unchecked) form.
-bool da_gemm_bf16_all_interior(const GemmDesc* d, int n);
+// The tile edge (128, 192 or 256) da_gemm_bf16_grouped picks for these products, in whatever order they are given, + 1 if every tile
+// then runs in the interior (unchecked) form, the one the weight-update epilogue (GemmDesc::upd_tab) exists in.
+int da_gemm_bf16_group_plan(const GemmDesc* d, int n);

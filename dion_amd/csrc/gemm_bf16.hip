@@ -419,31 +419,39 @@ int choose_tile(const GemmDesc* d, int n) {
   return big ? 256 : 128;
 }
 
+// The products in the order they are launched in: longest K first, so that long tiles start early and short ones fill the tail.
+// launch_cost counts on that order: whoever asks for a tile edge has to ask in it.
+void by_longest_k(const GemmDesc* in, int n, GemmDesc* d) {
+  for (int g = 0; g < n; ++g) {
+    int pos = g;
+    while (pos > 0 && d[pos - 1].K < in[g].K) { d[pos] = d[pos - 1]; --pos; }
+    d[pos] = in[g];
+  }
+}
+
 }  // namespace
 
 // Alignment contract: K, N, every leading dimension and every batch stride are multiples
 // of 8 elements (16-byte chunks); M too when A is k-strided; pointers 16-byte aligned.
 int da_gemm_bf16_grouped(const GemmDesc* din, int n, hipStream_t stream) {
   if (!din || n <= 0 || n > DA_MAX_GROUPS) return DA_ERR_ARG;
-  GemmDesc d[DA_MAX_GROUPS];
   for (int g = 0; g < n; ++g) {
     const int rc = check_desc(din[g]);
     if (rc) return rc;
     const GemmDesc &a = din[g], &f = din[0];
     if (a.symmetric != f.symmetric || a.a_kstrided != f.a_kstrided || a.b_kstrided != f.b_kstrided ||
-        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || (a.mi32 != 0) != (f.mi32 != 0) || a.any_addend != f.any_addend)
+        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || (a.mi32 != 0) != (f.mi32 != 0) || a.any_addend != f.any_addend || a.tile != f.tile)
       return DA_ERR_ARG;
     if (a.mi32 && (a.symmetric || a.a_kstrided || a.b_kstrided)) return DA_ERR_ARG;
-    // insertion sort, longest K first: long tiles start early, short ones fill the tail
-    int pos = g;
-    while (pos > 0 && d[pos - 1].K < a.K) { d[pos] = d[pos - 1]; --pos; }
-    d[pos] = a;
   }
+  GemmDesc d[DA_MAX_GROUPS];
+  by_longest_k(din, n, d);
+  const int bt = d[0].tile ? d[0].tile : choose_tile(d, n);
+  if (bt != 128 && bt != 256 && !(bt == Mid::BT && slide_ok(d, n))) return DA_ERR_ARG;
   if (d[0].mi32) {
-    if (choose_tile(d, n) == 256) return launch<Big32, Big32, false, false, false>(d, n, stream);
+    if (bt == 256) return launch<Big32, Big32, false, false, false>(d, n, stream);
     return launch<Small32, Small32, false, false, false>(d, n, stream);
   }
-  const int bt = choose_tile(d, n);
   if (bt == Mid::BT) return launch<Mid, Mid, false, false, true>(d, n, stream);
   return bt == 256 ? dispatch_layout<Big, BigChecked>(d, n, stream) : dispatch_layout<Small, Small>(d, n, stream);
 }
@@ -459,11 +467,12 @@ int da_gemm_bf16_plan(const GemmDesc& d) {
 
 int da_gemm_bf16(const GemmDesc& d, hipStream_t stream) { return da_gemm_bf16_grouped(&d, 1, stream); }
 
-// Whether the grouped launch of these products runs the interior (direct-to-LDS, unchecked) form for every tile:
-// the form the weight-update epilogue (GemmDesc::upd_tab) exists in.
-bool da_gemm_bf16_all_interior(const GemmDesc* d, int n) {
-  if (!d || n <= 0 || n > DA_MAX_GROUPS) return false;
-  return all_interior(d, n, choose_tile(d, n));
+int da_gemm_bf16_group_plan(const GemmDesc* din, int n) {
+  if (!din || n <= 0 || n > DA_MAX_GROUPS) return DA_ERR_ARG;
+  GemmDesc d[DA_MAX_GROUPS];
+  by_longest_k(din, n, d);
+  const int bt = choose_tile(d, n);
+  return bt + (all_interior(d, n, bt) ? 1 : 0);
 }
 
 // ---- measurement hook: time stamps of the tiles of the bf16 GEMM launches (see include/dion_amd.h)

@@ -2,6 +2,7 @@
 host-side mirror of the reference's optimizer interface validates and dispatches like the reference
 (reference dion/muon.py:55-131, dion/dion.py:105-231).  No GPU compute is launched here."""
 import ctypes
+import itertools
 import os
 import re
 
@@ -70,6 +71,26 @@ def test_gemm_plan_keeps_huge_operands_off_the_32_bit_offset_path():
     # ragged sizes never take it
     assert lib.dion_amd_gemm_plan(200, 136, 72, 72, 0, 72, 0) % 2 == 0
     assert lib.dion_amd_gemm_plan(0, 8, 8, 8, 0, 8, 0) == -1
+
+
+@pytest.mark.parametrize("groups", [   # (batch, M, N, K) of X' = a X + B X
+    [(48, 512, 896, 512), (48, 768, 1152, 768)],
+    [(16, 768, 1408, 768), (4, 1280, 1664, 1280)],
+    [(3, 512, 1408, 512), (12, 1280, 1664, 1280)],
+    [(4, 768, 896, 768), (24, 1024, 1152, 1024)],
+    [(4, 768, 896, 768), (24, 1024, 1152, 1024), (7, 640, 2048, 640), (2, 1536, 1664, 1536)],
+])
+def test_tile_of_a_grouped_launch_does_not_depend_on_the_order_of_its_products(groups):
+    """The epilogue that updates the weights is asked for where the launch has whole tiles: the answer is that of the order in which
+    the products are launched, longest K first, whatever order the caller's buckets have.  Host-side query, nothing is launched."""
+    from dion_amd import _lib
+
+    def plan(order):
+        return _lib.load().dion_amd_gemm_group_plan(*((ctypes.c_int * len(order))(*v) for v in zip(*order)), len(order), 0, 1, _lib.EPI_AXPBY)
+
+    want = plan(sorted(groups, key=lambda g: -g[3]))
+    assert want // 2 * 2 in (128, 256)
+    assert all(plan(order) == want for order in itertools.permutations(groups))
 
 
 def test_no_cpu_fallback():

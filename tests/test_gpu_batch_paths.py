@@ -250,6 +250,9 @@ def test_momentum_plus_gradient_inside_the_first_product_equals_the_separate_pas
 @pytest.mark.parametrize("shapes", [
     [(768, 768)] * 2 + [(3072, 768)] * 2 + [(768, 3072)] * 2,      # product launches: square, tall (transposed), wide
     [(768, 768)] * 16 + [(3072, 768)] * 8 + [(768, 3072)] * 8,     # enough matrices for the persistent launch
+    # whole 128-tiles, shorter K first: together they run 256-tiles, whose edges leave the update to the pass
+    [(512, 896)] * 48 + [(768, 1152)] * 48,
+    [(768, 896)] * 4 + [(1024, 1152)] * 24,
 ])
 def test_muon_update_in_the_last_epilogue_equals_the_stand_alone_pass(dev, shapes, wdtype):
     """`Muon.step` (momentum pass, Newton-Schulz whose last X' = aX + BX applies the weight update in its epilogue)
