@@ -12,7 +12,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
-# Measurement builds: DION_AMD_BUILD_DEFINES holds extra compiler options (e.g. "-DDA_MI=32"), DION_AMD_BUILD_LIB the
+# Measurement builds: DION_AMD_BUILD_DEFINES holds extra compiler options (e.g. "-save-temps"), DION_AMD_BUILD_LIB the
 # library to write instead of the in-tree one (its objects go beside it); load it with DION_AMD_LIB.
 LIB = os.environ.get("DION_AMD_BUILD_LIB") or os.path.join(HERE, "libdion_amd.so")
 if os.environ.get("DION_AMD_BUILD_LIB"):

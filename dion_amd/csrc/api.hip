@@ -542,9 +542,9 @@ bool dtype_ok(int d) { return d == DA_BF16 || d == DA_F32; }
 // Run-time options (dion_amd_set_option).  -1: not set by the caller, the environment decides.
 std::atomic<int> g_opt_fused_update{-1};
 
-// Dion's error feedback and weight update, bf16 momentum: 1 as one pass over M and X, 0 as two AXPBY products with that pass's
-// bits, -1 (nobody asked for either) as the products of the 16x16x32 instruction, M's and X's in one launch, or with fp32 weights
-// as the one pass where it applies.
+// Dion's error feedback and weight update, bf16 momentum: 1 as one pass over M and X where that applies, 0 as two AXPBY products,
+// -1 (nobody asked for either) as these products, M's and X's in one launch, or with fp32 weights as the one pass where it applies.
+// All give the same bits (dion_fused.hip uses the 32x32x16 instruction, the products 16x16x32, which form the same sums).
 // (us a step, the pass / the products in one launch.  Several buckets on their streams, which the pass's workgroups, one to a CU
 // from start to end, keep waiting: GPT-small at rank 192 712 / 697, at full rank 3605 / 3560, MLP matrices of a Llama-70B
 // layer 4645 / 4570.  One bucket: 48 of 768 x 768 at rank 64 213 / 211, 4 of 4096 x 4096 at rank 512 775 / 761, at rank 256 580 / 588,
@@ -1275,7 +1275,6 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
       else             { u.A = D; u.sA = sQ; u.B = P; u.sB = sP; u.M = np; u.N = mp; }
       u.lda = r; u.ldb = r; u.K = r; u.ldc = n; u.lde = n;
       u.epilogue = DA_EPI_AXPBY;
-      u.mi32 = form == 0;   // (the bits of the one-pass kernel)
     }
     up[0].Ctab = tabM; up[0].Etab = const_cast<const void* const*>(tabM); up[0].c_dtype = m_dtype;
     up[0].s0 = 1.f; up[0].s1 = ef_alpha;

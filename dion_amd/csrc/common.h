@@ -145,10 +145,6 @@ struct GemmDesc {
   void* const* upd_tab;
   int upd_dtype, upd_ld, upd_transposed;
   float upd_decay, upd_step;
-  // bf16 only, both operands k-contiguous, not symmetric: run the product with v_mfma_f32_32x32x16_bf16 (16 values of k
-  // per instruction instead of 32: another order of the fp32 sums).  Dion's error-feedback and weight-update products
-  // use it where their bits have to be those of the one-pass kernel (dion_fused.hip), which is built on that instruction.
-  int mi32;
   // bf16 only.  The tile edge to run (0: the launcher chooses).  A caller whose descriptors depend on the choice, as upd_tab does,
   // asks da_gemm_bf16_group_plan for it and hands it on, so that what was asked about is what runs.
   int tile;

@@ -1,12 +1,13 @@
-// Batched bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16, fp32 accumulate; the 32x32x16 form of the
-// instruction is kept for GemmDesc::mi32 and as a build variant: under the 16x16x32 form the chip holds a 13 % higher
-// clock at the same flops per pass, which is worth 3 % to the whole K loop).
+// Batched bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16, fp32 accumulate: under this form of the
+// instruction the chip holds a 13 % higher clock than under 32x32x16 at the same flops per pass, which is worth 3 % to the whole
+// K loop.  Both form the same fp32 sums, bit for bit: 10 million of 32 to 1024 products, normal, over 80 binary orders of magnitude,
+// subnormal and sparse ones.)
 //
 //   C[b] (M x N) = epilogue( sum_k Aop[b](i,k) * Bop[b](j,k) )
 //
 // Work decomposition: one workgroup of four wavefronts (2 x 2) per BT x BT output tile:
 //   * BT = 256, a CU each: 128 x 128 per wavefront as 8 x 8 accumulator blocks of 16 x 16, so that LDS is read for 128 KB a
-//     stage (eight wavefronts of 128 x 64, as the bounds-checked form and GemmDesc::mi32 have them, read 192 KB and are bound by it).
+//     stage (eight wavefronts of 128 x 64, as the bounds-checked form has them, read 192 KB and are bound by it).
 //   * BT = 192, symmetric products, a CU each.
 //   * BT = 128, two to a CU: for problems too small to fill the 256 CUs with large tiles.
 // The K loop advances 64 elements per stage and is double buffered through LDS (gemm_tile_k_loop_quad).
@@ -358,8 +359,6 @@ typedef Cfg<256, 2, 2> Big;
 typedef Cfg<256, 2, 4> BigChecked;     // (the operand stages go through registers: eight wavefronts)
 typedef Cfg<128, 2, 2> Small;
 typedef Cfg<192, 2, 2> Mid;            // (symmetric products)
-typedef Cfg<256, 2, 4, 32> Big32;      // (GemmDesc::mi32)
-typedef Cfg<128, 2, 2, 32> Small32;
 
 // Whether 192 x 192 tiles can run: every operand at least a tile, whole stages, 32-bit offsets (as all_interior); the last tile of
 // a dimension is moved back over its neighbour, whose results it computes again, the same bits, so E must not be C.  (An E that is not
@@ -440,18 +439,13 @@ int da_gemm_bf16_grouped(const GemmDesc* din, int n, hipStream_t stream) {
     if (rc) return rc;
     const GemmDesc &a = din[g], &f = din[0];
     if (a.symmetric != f.symmetric || a.a_kstrided != f.a_kstrided || a.b_kstrided != f.b_kstrided ||
-        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || (a.mi32 != 0) != (f.mi32 != 0) || a.any_addend != f.any_addend || a.tile != f.tile)
+        a.epilogue != f.epilogue || a.c_dtype != f.c_dtype || a.faithful != f.faithful || a.any_addend != f.any_addend || a.tile != f.tile)
       return DA_ERR_ARG;
-    if (a.mi32 && (a.symmetric || a.a_kstrided || a.b_kstrided)) return DA_ERR_ARG;
   }
   GemmDesc d[DA_MAX_GROUPS];
   by_longest_k(din, n, d);
   const int bt = d[0].tile ? d[0].tile : choose_tile(d, n);
   if (bt != 128 && bt != 256 && !(bt == Mid::BT && slide_ok(d, n))) return DA_ERR_ARG;
-  if (d[0].mi32) {
-    if (bt == 256) return launch<Big32, Big32, false, false, false>(d, n, stream);
-    return launch<Small32, Small32, false, false, false>(d, n, stream);
-  }
   if (bt == Mid::BT) return launch<Mid, Mid, false, false, true>(d, n, stream);
   return bt == 256 ? dispatch_layout<Big, BigChecked>(d, n, stream) : dispatch_layout<Small, Small>(d, n, stream);
 }

@@ -11,34 +11,22 @@
 
 namespace {
 
-// MI: edge of the MFMA's output block -- 32: v_mfma_f32_32x32x16_bf16 (16 accumulator registers per block, 16-deep
-// k-steps), 16: v_mfma_f32_16x16x32_bf16 (4 registers, 32-deep k-steps; the chip holds a higher clock under it).
-template <int MI> struct AccOf;
-template <> struct AccOf<32> { typedef f32x16_t type; };
-template <> struct AccOf<16> { typedef f32x4_t type; };
-
-#ifndef DA_MI
-#define DA_MI 16   // the MFMA shape the kernels of this library are built with (32: the 32x32x16 form)
-#endif
-
-template <int BT_, int WGM_, int WGN_, int MI_ = DA_MI>
+template <int BT_, int WGM_, int WGN_>
 struct Cfg {
-  static constexpr int BT = BT_, WGM = WGM_, WGN = WGN_, MI = MI_;
+  static constexpr int BT = BT_, WGM = WGM_, WGN = WGN_;
   static constexpr int NT = 64 * WGM * WGN;        // threads
-  static constexpr int TMI = BT / (MI * WGM);      // accumulator blocks per wavefront, row direction
-  static constexpr int TNJ = BT / (MI * WGN);      // ... column direction
-  static constexpr int AV = MI * MI / 64;          // accumulator registers per block
+  static constexpr int TMI = BT / (16 * WGM);      // 16 x 16 accumulator blocks per wavefront, row direction
+  static constexpr int TNJ = BT / (16 * WGN);      // ... column direction
   static constexpr int NCH = BT * 8 / NT;          // 16-byte chunks per thread per operand stage
   static constexpr int WROWS = BT / WGM, WCOLS = BT / WGN;
-  static constexpr int NB = WROWS / 32;            // 32-row bands of a wavefront's sub-tile (the epilogue's unit)
   // the last row and column of tiles lies against the matrix's end, over part of its neighbour (gemm_bf16.hip, Mid)
   static constexpr bool SLIDE = BT == 192;
   // interior and edge tiles run gemm_tile_k_loop_quad
-  static constexpr bool QUAD = MI == 16 && WGM == 2 && WGN == 2;
+  static constexpr bool QUAD = WGM == 2 && WGN == 2;
   // A k-strided operand of 128-tiles there: a wavefront has two runs of 32 rows (columns) 64 apart, so that what it reads in one phase
   // is half a k-row of the tile, a whole cache line (two half lines otherwise: both operands k-strided 1720 - 1880 clocks a stage).
   static constexpr bool split(bool full, bool ks) { return QUAD && full && BT == 128 && ks; }
-  typedef typename AccOf<MI>::type acc_t;
+  typedef f32x4_t acc_t;
 };
 
 template <int BT, bool KS>
@@ -232,25 +220,15 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
     for (int q = 0; q < DEPTH; ++q) load_e(q, ev[q]);
   }
   auto put_band = [&](int i) {
-    if (C::MI == 32) {
-      float* row = stg + (lane & 31) * PITCH + (lane >> 5) * 4;
+    // a lane holds, for row (lane & 15) of a block, the four columns 4 (lane >> 4) .. + 3
+    float* row = stg + (BR == 16 ? (i & 1) * 16 * PITCH : 0) + (lane & 15) * PITCH + (lane >> 4) * 4;
 #pragma unroll
-      for (int j = 0; j < C::TNJ; ++j)
+    for (int ib = 0; ib < BR / 16; ++ib)
 #pragma unroll
-        for (int vq = 0; vq < C::AV / 4; ++vq)
-          *reinterpret_cast<float4*>(row + j * 32 + vq * 8) =
-              make_float4(acc[i][j][vq * 4], acc[i][j][vq * 4 + 1], acc[i][j][vq * 4 + 2], acc[i][j][vq * 4 + 3]);
-    } else {
-      // 16 x 16 blocks: a lane holds, for row (lane & 15) of a block, the four columns 4 (lane >> 4) .. + 3
-      float* row = stg + (BR == 16 ? (i & 1) * 16 * PITCH : 0) + (lane & 15) * PITCH + (lane >> 4) * 4;
-#pragma unroll
-      for (int ib = 0; ib < BR / 16; ++ib)
-#pragma unroll
-        for (int j = 0; j < C::TNJ; ++j) {
-          const typename C::acc_t& a = acc[(BR / 16 * i + ib) % C::TMI][j];
-          *reinterpret_cast<float4*>(row + ib * 16 * PITCH + j * 16) = make_float4(a[0], a[1], a[2], a[3]);
-        }
-    }
+      for (int j = 0; j < C::TNJ; ++j) {
+        const typename C::acc_t& a = acc[(BR / 16 * i + ib) % C::TMI][j];
+        *reinterpret_cast<float4*>(row + ib * 16 * PITCH + j * 16) = make_float4(a[0], a[1], a[2], a[3]);
+      }
     wave_sync_lds();
   };
   float4 raw[PIPE ? 2 : 1][NPASS][2];
@@ -520,7 +498,7 @@ template <typename C, bool A_KS, bool B_KS, typename Hook>
 __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, const bf16_t* A,
                                                       const bf16_t* B, int dK, int m0, int n0, char* lds, int lane, int wave,
                                                       int wm, int wn, Hook hook, int a_wrap, unsigned b_jump) {
-  static_assert(C::MI == 16 && C::WGM == 2 && C::WGN == 2 && (C::BT == 256 || C::BT == 128 || (C::BT == 192 && !A_KS && !B_KS)), "");
+  static_assert(C::QUAD && (C::BT == 256 || C::BT == 128 || (C::BT == 192 && !A_KS && !B_KS)), "");
   constexpr int OP = C::BT * BK * 2, STAGE = 2 * OP;
   constexpr int HI = C::BT / 64;                         // 16-row blocks of a half
   constexpr int NR = 2 * HI, NU = UnitAddr<C, false>::NU;
@@ -605,7 +583,7 @@ __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C
 #pragma unroll
     for (int j = 0; j < C::TNJ; ++j)
 #pragma unroll
-      for (int v = 0; v < C::AV; ++v) acc[i][j][v] = 0.f;
+      for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
   __builtin_amdgcn_sched_barrier(0);
   dma_wait_all_but<6 * NU>();   // A0, B0
   meet();
@@ -647,9 +625,8 @@ __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C
 
 // K loop of one BT x BT tile: acc += sum over dK elements of k of A-rows (m0 ...) x B-rows (n0 ...).  `A`, `B`: the
 // matrix's operands at the first k of the sum.  Three forms (MODE):
-//   DA_LOOP_INTERIOR: every tile is interior (M, N multiples of BT, K a multiple of 64): gemm_tile_k_loop_quad where four
-//     wavefronts run the 16 x 16 form, else stages fetched with direct-to-LDS loads one stage ahead, the only wait the
-//     vmcnt(0) in front of the per-stage barrier.  No bounds checks anywhere.
+//   DA_LOOP_INTERIOR: every tile is interior (M, N multiples of BT, K a multiple of 64): gemm_tile_k_loop_quad.  No
+//     bounds checks anywhere.
 //   DA_LOOP_EDGE: the same K loop for products whose ragged dimension belongs to a k-strided operand (its chunks
 //     are kept inside the matrix) and whose other operand has whole tiles; the epilogue checks bounds.  Dion's
 //     rank-r products at a rank that is not a multiple of the tile edge (r = 192).
@@ -667,11 +644,12 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
                                                  int wave, int wm, int wn, Hook after_first_stage = Hook(),
                                                  int a_wrap = -1, unsigned b_jump = 0) {
   constexpr bool FULL = MODE != DA_LOOP_CHECKED;   // the direct-to-LDS K loop
-  if constexpr (FULL && C::QUAD) {
+  static_assert(!FULL || C::QUAD, "");
+  if constexpr (FULL) {
     gemm_tile_k_loop_quad<C, A_KS, B_KS>(acc, d, A, B, dK, m0, n0, lds, lane, wave, wm, wn, after_first_stage, a_wrap, b_jump);
     return;
   }
-  constexpr int BT = C::BT, TMI = C::TMI, TNJ = C::TNJ, NCH = C::NCH, NW = C::NT / 64;
+  constexpr int BT = C::BT, TMI = C::TMI, TNJ = C::TNJ, NCH = C::NCH;
   constexpr int A_BYTES = Tile<BT, A_KS>::bytes;
   constexpr int B_BYTES = Tile<BT, B_KS>::bytes;
   constexpr int STAGE = A_BYTES + B_BYTES;
@@ -680,149 +658,13 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
 #pragma unroll
     for (int j = 0; j < TNJ; ++j)
 #pragma unroll
-      for (int v = 0; v < C::AV; ++v) acc[i][j][v] = 0.f;
+      for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
 
   StageAddr<C, A_KS> sa(A, d.lda, m0, tid, d.M);
   StageAddr<C, B_KS> sb(B, d.ldb, n0, tid, d.N);
   const int ar0 = wm * C::WROWS, br0 = wn * C::WCOLS;
   const int KT = (dK + BK - 1) / BK;
-  bf16x8_t fa[C::MI == 32 ? TMI : 1], fb[C::MI == 32 ? TNJ : 1];   // (the 16 x 16 form keeps its own sets below)
-
-  if constexpr (C::MI == 32) {
-#define DA_FREAD(st, ks)                                                                           \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        fa[i] = read_frag<BT, A_KS>((st), ar0 + i * 32, (ks), lane);                               \
-    _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
-        fb[j] = read_frag<BT, B_KS>((st) + A_BYTES, br0 + j * 32, (ks), lane);                        \
-  } while (0)
-#define DA_FREAD2(st, ks, FA, FB)                                                                  \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        FA[i] = read_frag<BT, A_KS>((st), ar0 + i * 32, (ks), lane);                               \
-    _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
-        FB[j] = read_frag<BT, B_KS>((st) + A_BYTES, br0 + j * 32, (ks), lane);                        \
-  } while (0)
-#define DA_MMA2(FA, FB)                                                                            \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                            \
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(FB[j], FA[i], acc[i][j], 0, 0, 0); \
-  } while (0)
-#define DA_MMA()                                                                                   \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                            \
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0); \
-  } while (0)
-
-  if (FULL) {
-// one stage of both operands, straight into LDS: NCH wave-instructions of 1024 bytes each
-#define DA_DMA(st)                                                                                 \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
-        dma16(sa.dbase, sa.doff + i * sa.dstep + koff_a, lds_addr(st) + (i * NW + wave) * 1024);   \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
-        dma16(sb.dbase, sb.doff + i * sb.dstep + koff_b, lds_addr(st) + A_BYTES + (i * NW + wave) * 1024); \
-    koff_a += (unsigned)(sa.tstep * 2);                                                            \
-    koff_b += (unsigned)(sb.tstep * 2);                                                            \
-    if (koff_a == wrap_a) { koff_a = 0; koff_b += b_jump; }                                        \
-  } while (0)
-    unsigned koff_a = 0, koff_b = 0;   // byte offset of the stage within the operand (< 4 GiB: checked by the launcher)
-    const unsigned wrap_a = (unsigned)(a_wrap < 0 ? d.a_kwrap : a_wrap) * 2u;   // A read again from its first column (0: never, koff_a > 0 here)
-    DA_DMA(lds);
-    dma_wait();
-    __syncthreads();
-    after_first_stage();
-    // Fragments are double buffered in registers: the ds_reads of k-step s+1 are issued before
-    // the MFMAs of k-step s (scheduling fences keep the compiler from sinking them back down to
-    // their first use), and the stage barrier sits before the last k-step so that the first
-    // fragments of the next stage are fetched under the last MFMAs of this one.
-    bf16x8_t ga[TMI], gb[TNJ];
-    DA_FREAD(lds, 0);
-    for (int kt = 0; kt < KT; ++kt) {
-      char* cur = lds + (kt & 1) * STAGE;
-      char* nxt = lds + ((kt + 1) & 1) * STAGE;
-      const bool more = kt + 1 < KT;
-      if (more) DA_DMA(nxt);
-      DA_FREAD2(cur, 1, ga, gb);
-      __builtin_amdgcn_sched_barrier(0);
-      DA_MMA();
-      __builtin_amdgcn_sched_barrier(0);
-      DA_FREAD(cur, 2);
-      __builtin_amdgcn_sched_barrier(0);
-      DA_MMA2(ga, gb);
-      __builtin_amdgcn_sched_barrier(0);
-      DA_FREAD2(cur, 3, ga, gb);
-      __builtin_amdgcn_sched_barrier(0);
-      DA_MMA();
-      __builtin_amdgcn_sched_barrier(0);
-      dma_wait();
-      __syncthreads();
-      if (more) DA_FREAD(nxt, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      DA_MMA2(ga, gb);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();
-#undef DA_DMA
-  } else {
-    u32x4_t ra[NCH], rb[NCH];
-    constexpr int A_RSTEP = A_KS ? C::NT / (BT / 8) : C::NT / 8;  // tile rows (k rows if k-strided) per chunk
-    constexpr int B_RSTEP = B_KS ? C::NT / (BT / 8) : C::NT / 8;
-#define DA_GLOAD(kt)                                                                               \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i) {                                              \
-      const int r_ = sa.row + i * A_RSTEP;                                                         \
-      const bool ok = A_KS ? ((kt) * BK + r_ < dK && m0 + sa.col < d.M)                            \
-                           : (m0 + r_ < d.M && (kt) * BK + sa.col < dK);                           \
-      const u32x4_t z_ = {0u, 0u, 0u, 0u};                                                         \
-      ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(sa.g + i * sa.gstep) : z_;                    \
-    }                                                                                              \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i) {                                              \
-      const int r_ = sb.row + i * B_RSTEP;                                                         \
-      const bool ok = B_KS ? ((kt) * BK + r_ < dK && n0 + sb.col < d.N)                            \
-                           : (n0 + r_ < d.N && (kt) * BK + sb.col < dK);                           \
-      const u32x4_t z_ = {0u, 0u, 0u, 0u};                                                         \
-      rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(sb.g + i * sb.gstep) : z_;                    \
-    }                                                                                              \
-    sa.g += sa.tstep;                                                                              \
-    if (!A_KS && d.a_kwrap && (((kt) + 1) * BK) % d.a_kwrap == 0) sa.g -= d.a_kwrap;               \
-    sb.g += sb.tstep;                                                                              \
-  } while (0)
-#define DA_LSTORE(st)                                                                              \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
-        *reinterpret_cast<u32x4_t*>((st) + sa.l + i * sa.lstep) = ra[i];                           \
-    _Pragma("unroll") for (int i = 0; i < NCH; ++i)                                                \
-        *reinterpret_cast<u32x4_t*>((st) + A_BYTES + sb.l + i * sb.lstep) = rb[i];                 \
-  } while (0)
-    DA_GLOAD(0);
-    DA_LSTORE(lds);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      char* cur = lds + (kt & 1) * STAGE;
-      char* nxt = lds + ((kt + 1) & 1) * STAGE;
-      const bool more = kt + 1 < KT;
-      if (more) DA_GLOAD(kt + 1);
-#pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        DA_FREAD(cur, ks);
-        DA_MMA();
-      }
-      if (more) DA_LSTORE(nxt);
-      __syncthreads();
-    }
-#undef DA_GLOAD
-#undef DA_LSTORE
-  }
-#undef DA_FREAD
-#undef DA_MMA
-#undef DA_FREAD2
-#undef DA_MMA2
-  } else {
-  // ---- v_mfma_f32_16x16x32_bf16, bounds-checked: a stage is two 32-deep k-steps of TMI row fragments (in two halves) and TNJ
-  // column fragments
+  // bounds-checked: a stage is two 32-deep k-steps of TMI row fragments (in two halves) and TNJ column fragments
   constexpr int TH = TMI / 2;
 #define DA16_RA(FA, st, ks, h)                                                                     \
   do {                                                                                             \
@@ -841,71 +683,57 @@ __device__ __forceinline__ void gemm_tile_k_loop(typename C::acc_t (&acc)[C::TMI
             acc[(h) * TH + i][j] =                                                                 \
                 __builtin_amdgcn_mfma_f32_16x16x32_bf16(FB[j], FA[i], acc[(h) * TH + i][j], 0, 0, 0); \
   } while (0)
-  {
-    u32x4_t ra[NCH], rb[NCH];
-    constexpr int A_RSTEP = A_KS ? C::NT / (BT / 8) : C::NT / 8;
-    constexpr int B_RSTEP = B_KS ? C::NT / (BT / 8) : C::NT / 8;
-    auto gload = [&](int kt) {
+  u32x4_t ra[NCH], rb[NCH];
+  constexpr int A_RSTEP = A_KS ? C::NT / (BT / 8) : C::NT / 8;
+  constexpr int B_RSTEP = B_KS ? C::NT / (BT / 8) : C::NT / 8;
+  auto gload = [&](int kt) {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        const int r_ = sa.row + i * A_RSTEP;
-        const bool ok = A_KS ? (kt * BK + r_ < dK && m0 + sa.col < d.M) : (m0 + r_ < d.M && kt * BK + sa.col < dK);
-        const u32x4_t z_ = {0u, 0u, 0u, 0u};
-        ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(sa.g + i * sa.gstep) : z_;
-      }
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        const int r_ = sb.row + i * B_RSTEP;
-        const bool ok = B_KS ? (kt * BK + r_ < dK && n0 + sb.col < d.N) : (n0 + r_ < d.N && kt * BK + sb.col < dK);
-        const u32x4_t z_ = {0u, 0u, 0u, 0u};
-        rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(sb.g + i * sb.gstep) : z_;
-      }
-      sa.g += sa.tstep;
-      if (!A_KS && d.a_kwrap && ((kt + 1) * BK) % d.a_kwrap == 0) sa.g -= d.a_kwrap;   // A again from its first column
-      sb.g += sb.tstep;
-    };
-    auto lstore = [&](char* st) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) *reinterpret_cast<u32x4_t*>(st + sa.l + i * sa.lstep) = ra[i];
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) *reinterpret_cast<u32x4_t*>(st + A_BYTES + sb.l + i * sb.lstep) = rb[i];
-    };
-    bf16x8_t a0[TH], a1[TH], b0[TNJ];
-    gload(0);
-    lstore(lds);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-      char* cur = lds + (kt & 1) * STAGE;
-      char* nxt = lds + ((kt + 1) & 1) * STAGE;
-      const bool more = kt + 1 < KT;
-      if (more) gload(kt + 1);
-#pragma unroll
-      for (int ks = 0; ks < BK / 32; ++ks) {
-        DA16_RB(b0, cur, ks);
-        DA16_RA(a0, cur, ks, 0);
-        DA16_RA(a1, cur, ks, 1);
-        DA16_MMA(a0, b0, 0);
-        DA16_MMA(a1, b0, 1);
-      }
-      if (more) lstore(nxt);
-      __syncthreads();
+    for (int i = 0; i < NCH; ++i) {
+      const int r_ = sa.row + i * A_RSTEP;
+      const bool ok = A_KS ? (kt * BK + r_ < dK && m0 + sa.col < d.M) : (m0 + r_ < d.M && kt * BK + sa.col < dK);
+      const u32x4_t z_ = {0u, 0u, 0u, 0u};
+      ra[i] = ok ? *reinterpret_cast<const u32x4_t*>(sa.g + i * sa.gstep) : z_;
     }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int r_ = sb.row + i * B_RSTEP;
+      const bool ok = B_KS ? (kt * BK + r_ < dK && n0 + sb.col < d.N) : (n0 + r_ < d.N && kt * BK + sb.col < dK);
+      const u32x4_t z_ = {0u, 0u, 0u, 0u};
+      rb[i] = ok ? *reinterpret_cast<const u32x4_t*>(sb.g + i * sb.gstep) : z_;
+    }
+    sa.g += sa.tstep;
+    if (!A_KS && d.a_kwrap && ((kt + 1) * BK) % d.a_kwrap == 0) sa.g -= d.a_kwrap;   // A again from its first column
+    sb.g += sb.tstep;
+  };
+  auto lstore = [&](char* st) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) *reinterpret_cast<u32x4_t*>(st + sa.l + i * sa.lstep) = ra[i];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) *reinterpret_cast<u32x4_t*>(st + A_BYTES + sb.l + i * sb.lstep) = rb[i];
+  };
+  bf16x8_t a0[TH], a1[TH], b0[TNJ];
+  gload(0);
+  lstore(lds);
+  __syncthreads();
+  for (int kt = 0; kt < KT; ++kt) {
+    char* cur = lds + (kt & 1) * STAGE;
+    char* nxt = lds + ((kt + 1) & 1) * STAGE;
+    const bool more = kt + 1 < KT;
+    if (more) gload(kt + 1);
+#pragma unroll
+    for (int ks = 0; ks < BK / 32; ++ks) {
+      DA16_RB(b0, cur, ks);
+      DA16_RA(a0, cur, ks, 0);
+      DA16_RA(a1, cur, ks, 1);
+      DA16_MMA(a0, b0, 0);
+      DA16_MMA(a1, b0, 1);
+    }
+    if (more) lstore(nxt);
+    __syncthreads();
   }
 #undef DA16_RA
 #undef DA16_RB
 #undef DA16_MMA
-  }
-}
-
-template <typename C, bool KS>
-__device__ __forceinline__ bf16x8_t read_frag_of(const char* lds, int r0, int ks, int lane) {
-  if constexpr (C::MI == 32) return read_frag<C::BT, KS>(lds, r0, ks, lane);
-  else return read_frag16<C::BT, KS>(lds, r0, ks, lane);
-}
-template <typename C>
-__device__ __forceinline__ void mma_of(typename C::acc_t& acc, bf16x8_t col, bf16x8_t row) {
-  if constexpr (C::MI == 32) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(col, row, acc, 0, 0, 0);
-  else acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(col, row, acc, 0, 0, 0);
 }
 
 // K loop of one BT x BT tile whose row operand is the SUM of two bf16 matrices of the same layout, formed on the way
@@ -931,7 +759,7 @@ __device__ __forceinline__ void gemm_tile_k_loop_sum(typename C::acc_t (&acc)[C:
 #pragma unroll
     for (int j = 0; j < TNJ; ++j)
 #pragma unroll
-      for (int v = 0; v < C::AV; ++v) acc[i][j][v] = 0.f;
+      for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.f;
 
   StageAddr<C, A_KS> sa(M, d.lda, m0, tid, d.M);
   StageAddr<C, B_KS> sb(B, d.ldb, n0, tid, d.N);
@@ -942,7 +770,7 @@ __device__ __forceinline__ void gemm_tile_k_loop_sum(typename C::acc_t (&acc)[C:
   const unsigned gs2 = (unsigned)(sa.gstep * 2), ts2 = (unsigned)(sa.tstep * 2);
   const int ar0 = wm * C::WROWS, br0 = wn * C::WCOLS;
   const int KT = dK / BK;
-  bf16x8_t fa[C::MI == 32 ? TMI : TMI / 2], fb[TNJ];
+  bf16x8_t fa[TMI / 2], fb[TNJ];
   u32x4_t rm[NCH], rg[NCH];
   unsigned nz = 0u;
   unsigned koff_b = 0;
@@ -976,20 +804,6 @@ __device__ __forceinline__ void gemm_tile_k_loop_sum(typename C::acc_t (&acc)[C:
     }                                                                                              \
     aoff += ts2;                                                                                   \
   } while (0)
-#define DA_SUM_FREAD(st, ks, FA, FB)                                                               \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        FA[i] = read_frag_of<C, A_KS>((st), ar0 + i * C::MI, (ks), lane);                          \
-    _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                                \
-        FB[j] = read_frag_of<C, B_KS>((st) + A_BYTES, br0 + j * C::MI, (ks), lane);                \
-  } while (0)
-#define DA_SUM_MMA(FA, FB)                                                                         \
-  do {                                                                                             \
-    _Pragma("unroll") for (int i = 0; i < TMI; ++i)                                                \
-        _Pragma("unroll") for (int j = 0; j < TNJ; ++j)                                            \
-            mma_of<C>(acc[i][j], FB[j], FA[i]);                                                    \
-  } while (0)
-
   // (fragments are not double buffered here: the registers hold a stage of M and of G instead, and the loop is
   // bound by the stream of M and G from HBM, not by the matrix cores)
   DA_SUM_LOAD();
@@ -1005,27 +819,19 @@ __device__ __forceinline__ void gemm_tile_k_loop_sum(typename C::acc_t (&acc)[C:
       DA_SUM_LOAD();
       DA_SUM_DMA(nxt);
     }
-    if constexpr (C::MI == 32) {
+    // (the row fragments of a 32-deep k-step in two halves through the same registers)
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        DA_SUM_FREAD(cur, ks, fa, fb);
-        DA_SUM_MMA(fa, fb);
-      }
-    } else {
-      // (16 x 16 blocks: the row fragments of a 32-deep k-step in two halves through the same registers)
+    for (int ks = 0; ks < BK / 32; ++ks) {
 #pragma unroll
-      for (int ks = 0; ks < BK / 32; ++ks) {
+      for (int j = 0; j < TNJ; ++j) fb[j] = read_frag16<BT, B_KS>(cur + A_BYTES, br0 + j * 16, ks, lane);
 #pragma unroll
-        for (int j = 0; j < TNJ; ++j) fb[j] = read_frag16<BT, B_KS>(cur + A_BYTES, br0 + j * 16, ks, lane);
+      for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int i = 0; i < TMI / 2; ++i) fa[i] = read_frag16<BT, A_KS>(cur, ar0 + (h * (TMI / 2) + i) * 16, ks, lane);
 #pragma unroll
-          for (int i = 0; i < TMI / 2; ++i) fa[i] = read_frag16<BT, A_KS>(cur, ar0 + (h * (TMI / 2) + i) * 16, ks, lane);
+        for (int i = 0; i < TMI / 2; ++i)
 #pragma unroll
-          for (int i = 0; i < TMI / 2; ++i)
-#pragma unroll
-            for (int j = 0; j < TNJ; ++j) mma_of<C>(acc[h * (TMI / 2) + i][j], fb[j], fa[i]);
-        }
+          for (int j = 0; j < TNJ; ++j) acc[h * (TMI / 2) + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[h * (TMI / 2) + i][j], 0, 0, 0);
       }
     }
     if (more) DA_SUM_STORE(nxt);
@@ -1039,8 +845,6 @@ __device__ __forceinline__ void gemm_tile_k_loop_sum(typename C::acc_t (&acc)[C:
 #undef DA_SUM_LOAD
 #undef DA_SUM_DMA
 #undef DA_SUM_STORE
-#undef DA_SUM_FREAD
-#undef DA_SUM_MMA
 }
 
 }  // namespace

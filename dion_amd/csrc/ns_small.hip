@@ -34,7 +34,7 @@
 
 namespace {
 
-typedef Cfg<64, 2, 2, 16> Sm;
+typedef Cfg<64, 2, 2> Sm;
 constexpr int BT = DA_SMALL_BT;
 constexpr int NQ = DA_QUEUES;
 constexpr int NST = 4;                     // LDS stage buffers

@@ -398,9 +398,9 @@ int dion_amd_profile_read(int kind, long long* launches, double* total_ms, doubl
  *   "fused_update"  1: dion_amd_dion_step(_qr) applies error feedback and weight update in one pass over M and X
  *                   where that kernel applies (bf16 momentum, dimensions multiples of 128, rank a multiple of 64);
  *                   0: always as two products with the update in their epilogues (reference dion/dion.py:851-853
- *                   and 865-872 as two calls); both roads give the same bits.  -1: the default, bf16 weights by two
- *                   products of another matrix instruction (the same sums) in one launch, fp32 weights in one pass where
- *                   that applies (DION_AMD_NO_FUSED in the environment: as 0).
+ *                   and 865-872 as two calls); -1: the default, bf16 weights by the two products in one
+ *                   launch, fp32 weights in one pass where that applies (DION_AMD_NO_FUSED in the environment: as 0).
+ *                   All give the same bits.
  *   "fused_bq"      Dion's B = M + G: 1 formed inside the launch of P = B Q where that applies (bf16 momentum and
  *                   gradients, the longer dimension a multiple of 256, the shorter of 64); 0 as a pass of its own
  *                   (reference dion/dion.py:794 and 801 as two calls); -1 the default (inside, unless

@@ -80,15 +80,50 @@ def test_fused_update_pass_equals_the_two_products_bit_for_bit(dev, shapes, rank
     assert not torch.equal(runs[0][1][0].detach(), X[0])
 
 
+@pytest.mark.parametrize("wdtype", [BF, torch.float32])
+@pytest.mark.parametrize("shapes,rank_fraction", [
+    # (matrices of millions of elements: an fp32 sum in another order would seldom end in another bf16 value)
+    ([(4096, 2048)], 0.25),                            # on the one-pass kernel's grid
+    ([(2048, 4096), (4096, 1024)], 0.15),              # ranks off it (312, 160)
+    ([(4104, 2056), (200, 1032)], 0.3),                # dimensions off it
+])
+def test_forms_of_the_update_have_the_same_bits(dev, shapes, rank_fraction, wdtype):
+    """One pass (where it applies), two products, the default.  mu = 0, lr = 1: the products are not small against what they are added
+    to, so that a difference would show in the sums."""
+    from dion_amd import _lib
+
+    X, gen = _dion_problem(dev, shapes, 23)
+    G = [(torch.randn(s, generator=gen, device=dev) * 1e-3).to(wdtype) for s in shapes]
+    runs = []
+    try:
+        _lib.set_option("dion_small", 0)
+        for form in (1, 0, -1):
+            _lib.set_option("fused_update", form)
+            opt, params, states = _make_dion(dev, [x.to(wdtype) for x in X], rank_fraction, runs and runs[0][2])
+            opt.param_groups[0].update(lr=1.0, mu=0.0, weight_decay=0.0)
+            q0 = [st["Q"].clone() for st in states]
+            for p, g in zip(params, G):
+                p.grad = g
+            opt.step()
+            torch.cuda.synchronize()
+            runs.append((params, states, q0))
+    finally:
+        _lib.set_option("fused_update", -1)
+        _lib.set_option("dion_small", -1)
+    for other in runs[1:]:
+        _assert_same("forms of the update", *runs[0][:2], *other[:2])
+    assert not torch.equal(runs[0][0][0].detach(), X[0].to(wdtype))
+
+
 @pytest.mark.parametrize("shapes,rank_fraction", [
     ([(768, 512)] * 3 + [(512, 1024)] * 2, 0.25),      # whole tiles, tall and wide
     ([(648, 264)] * 2 + [(200, 1032)], 0.3),           # rank 80 and 60, edges of tiles: the bounds-checked loop
     ([(4096, 64)] * 2, 1.0),                           # one stage
 ])
 def test_update_in_one_launch_is_the_two_products(dev, shapes, rank_fraction):
-    """The default form (both products of bf16 weights in one launch) against the two launches of the other matrix instruction: the
-    same fp32 sums in another order inside an instruction, then bf16 roundings of the product, at most as large as the old and the new
-    value together, and of the result that may each fall one step (2^-7) apart."""
+    """The default form (both products of bf16 weights in one launch) against the two launches.  The bound is that of the same fp32
+    sums in another order: bf16 roundings of the product, at most as large as the old and the new value together, and of the result
+    that may each fall one step (2^-7) apart."""
     from dion_amd import _lib
 
     X, gen = _dion_problem(dev, shapes, 22)
