@@ -543,18 +543,30 @@ bool dtype_ok(int d) { return d == DA_BF16 || d == DA_F32; }
 std::atomic<int> g_opt_fused_update{-1};
 
 // Dion's error feedback and weight update, bf16 momentum: 1 as one pass over M and X where that applies, 0 as two AXPBY products,
-// -1 (nobody asked for either) as these products, M's and X's in one launch, or with fp32 weights as the one pass where it applies.
+// -1 (nobody asked for either) by one_pass_update.
 // All give the same bits (dion_fused.hip uses the 32x32x16 instruction, the products 16x16x32, which form the same sums).
-// (us a step, the pass / the products in one launch.  Several buckets on their streams, which the pass's workgroups, one to a CU
-// from start to end, keep waiting: GPT-small at rank 192 712 / 697, at full rank 3605 / 3560, MLP matrices of a Llama-70B
-// layer 4645 / 4570.  One bucket: 48 of 768 x 768 at rank 64 213 / 211, 4 of 4096 x 4096 at rank 512 775 / 761, at rank 256 580 / 588,
-// 2 of 14336 x 4096 at rank 64 600 / 593, 2 of 4096 x 14336 at rank 256 813 / 832;  fp32 weights, two launches: 947 / 970, 422 / 438.)
 int update_form() {
   const int v = g_opt_fused_update.load(std::memory_order_relaxed);
   if (v >= 0) return v != 0;
   static const bool env_off = getenv("DION_AMD_NO_FUSED") != nullptr;
   return env_off ? 0 : -1;
 }
+
+// The form nobody asked for: one pass, or (false) both products in one launch, with fp32 weights one after the other.  `beside`:
+// other buckets' launches run on other streams, and the pass's workgroups, one to a CU from start to end, keep them waiting.
+// us a step, the pass / the products:
+//   one bucket, at rank     64             128            256            384            512            1024
+//   1 of 8192 x 28672       1123 / 1164    1208 / 1266    1364 / 1468    1612 / 1708    1775 / 1811    3027 / 2938
+//   4 of 4096 x 4096        435 / 440      476 / 492      579 / 595      643 / 648      784 / 772      1405 / 1360
+//   16 of 2048 x 2048       368 / 372      412 / 421      545 / 551      695 / 680      868 / 861      3039 / 2943
+//   2 of 4096 x 14336       602 / 582      654 / 649      807 / 819      971 / 985      1098 / 1092    1994 / 1894
+//   2 of 14336 x 4096       571 / 560      617 / 618      769 / 779      942 / 938      1071 / 1064    1975 / 1839
+//   (48 of 768 x 768 and 12 of 3072 x 768, ranks 64 to 384: within 1 %)
+//   several: a Llama-8B layer at rank 64 1118 / 1095, 256 1523 / 1473, 512 2246 / 2184;  MLP matrices of a Llama-70B layer at rank 128
+//   2901 / 2779, 256 3286 / 3314, 512 4640 / 4587;  GPT-small at rank 192 701 / 684, 768 3640 / 3564.
+// The shorter the products' sums, the more of their tiles is the trip to memory that the pass has under the next tile's sums.
+// fp32 weights (not grouped: two output types): 947 / 970, 422 / 438.
+bool one_pass_update(bool x_f32, int r, bool beside) { return x_f32 || (!beside && r < 512); }
 
 // B = M + G inside the launch of P = B Q (the default where it applies) or as a pass of its own.
 std::atomic<int> g_opt_fused_bq{-1};
@@ -1252,7 +1264,8 @@ int dion_step_impl(void* const* X, const void* const* G, void* const* M, void* c
     }  // power iterations
     // ---- error feedback, column normalisation and weight update (reference dion/dion.py:851-872)
     const int form = update_form();
-    if (faithful && (form > 0 || (form < 0 && x_dtype == DA_F32)) && da_dion_ef_update_applicable(mp, np, r, m_dtype)) {
+    if (faithful && (form > 0 || (form < 0 && one_pass_update(x_dtype == DA_F32, r, faithful == 2))) &&
+        da_dion_ef_update_applicable(mp, np, r, m_dtype)) {
       // Q_new first (it only needs R), then both rank-r updates in one pass over M and X
       {
         DaProfScope prof(DA_PROF_DION_ELEM, 0.0, s);

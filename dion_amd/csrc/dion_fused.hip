@@ -17,7 +17,7 @@
 // tiles, filled by direct-to-LDS loads) is shared: only one group is in a K loop at a time, and it also requests the
 // first stage of the other group's next tile during its own last stage, so the epilogue group never waits for a
 // load it has not asked for.
-// Taken for fp32 weights; bf16 weights are updated by two products in one launch (update_form in api.hip has the figures).
+// Taken for fp32 weights, and for bf16 weights of one bucket at ranks below 512 (one_pass_update in api.hip has the figures).
 #include "dion.h"
 #include "mfma_tile.h"
 #include <cstdlib>

@@ -347,7 +347,9 @@ class Dion(_lib.HookedOptimizer):
                             _lib.ptr_array(Xs), _lib.ptr_array(Gs), _lib.ptr_array(Ms), _lib.ptr_array(Qs),
                             len(plist), m, n, r,
                             _lib.dtype_code(dtype), _lib.dtype_code(gdtype), mcode, _lib.dtype_code(Qs[0].dtype),
-                            ef_alpha.item(), decay.item(), scaled_lr.item(), epsilon.item(), 1, self._power_iters,
+                            ef_alpha.item(), decay.item(), scaled_lr.item(), epsilon.item(),
+                            2 if slots > 1 else 1,   # (faithful rounding; 2: beside other buckets' launches)
+                            self._power_iters,
                         )
                         sketch = None
                         if self._REFERENCE_OPTIONS and qr_method == "rcqr" and max(m, n) > r:

@@ -293,6 +293,8 @@ int dion_amd_dion_bq_fused(int batch, int m, int n, int rank, int m_dtype, int g
  *   B = M + G;  P = orth(B' Q);  R = B'^T P;  (all-zero / NaN guard on P, R)
  *   M <- B - (1-mu) P R^T  (transposed back when m < n);   Q <- R / (||R||_col + eps);
  *   X <- decay X - scaled_lr P Q^T.
+ * faithful: as above; 2 as 1, and other buckets' steps run on other streams meanwhile (a hint: the same results, by launches that
+ * leave room for those).
  * ef_alpha = -(1 - mu), decay = 1 - lr*wd and scaled_lr = sqrt(m/n)*lr are passed as
  * already-evaluated fp32 values.  Every combination of bf16 / f32 for x, g, m and q is accepted.  info as above.
  * power_iters >= 1 repeats P = orth(B' Q), Q = B'^T P before the updates, the unnormalised R serving as the
@@ -398,8 +400,9 @@ int dion_amd_profile_read(int kind, long long* launches, double* total_ms, doubl
  *   "fused_update"  1: dion_amd_dion_step(_qr) applies error feedback and weight update in one pass over M and X
  *                   where that kernel applies (bf16 momentum, dimensions multiples of 128, rank a multiple of 64);
  *                   0: always as two products with the update in their epilogues (reference dion/dion.py:851-853
- *                   and 865-872 as two calls); -1: the default, bf16 weights by the two products in one
- *                   launch, fp32 weights in one pass where that applies (DION_AMD_NO_FUSED in the environment: as 0).
+ *                   and 865-872 as two calls); -1: the default, fp32 weights and bf16 weights of
+ *                   one bucket at ranks below 512 in one pass where that applies, else bf16 weights by the two products
+ *                   in one launch (DION_AMD_NO_FUSED in the environment: as 0).
  *                   All give the same bits.
  *   "fused_bq"      Dion's B = M + G: 1 formed inside the launch of P = B Q where that applies (bf16 momentum and
  *                   gradients, the longer dimension a multiple of 256, the shorter of 64); 0 as a pass of its own

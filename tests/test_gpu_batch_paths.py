@@ -83,7 +83,7 @@ def test_fused_update_pass_equals_the_two_products_bit_for_bit(dev, shapes, rank
 @pytest.mark.parametrize("wdtype", [BF, torch.float32])
 @pytest.mark.parametrize("shapes,rank_fraction", [
     # (matrices of millions of elements: an fp32 sum in another order would seldom end in another bf16 value)
-    ([(4096, 2048)], 0.25),                            # on the one-pass kernel's grid
+    ([(4096, 2048)], 0.125),                           # on the one-pass kernel's grid, which the default takes
     ([(2048, 4096), (4096, 1024)], 0.15),              # ranks off it (312, 160)
     ([(4104, 2056), (200, 1032)], 0.3),                # dimensions off it
 ])
