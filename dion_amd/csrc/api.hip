@@ -895,12 +895,13 @@ int dion_amd_gemm_plan(int M, int N, int K, int lda, int a_kstrided, int ldb, in
 }
 
 int dion_amd_gemm_group_plan(const int* batch, const int* M, const int* N, const int* K, int n, int a_kstrided, int b_kstrided,
-                             int epilogue) {
+                             int symmetric, int epilogue) {
   if (!batch || !M || !N || !K || n <= 0 || n > DA_MAX_GROUPS) return DA_ERR_ARG;
   GemmDesc g[DA_MAX_GROUPS];
   for (int i = 0; i < n; ++i) {
-    if (batch[i] <= 0 || M[i] <= 0 || N[i] <= 0 || K[i] <= 0) return DA_ERR_ARG;
+    if (batch[i] <= 0 || M[i] <= 0 || N[i] <= 0 || K[i] <= 0 || (symmetric && M[i] != N[i])) return DA_ERR_ARG;
     g[i] = GemmDesc{};
+    g[i].symmetric = symmetric != 0;
     g[i].batch = batch[i]; g[i].M = M[i]; g[i].N = N[i]; g[i].K = K[i];
     g[i].a_kstrided = a_kstrided != 0; g[i].b_kstrided = b_kstrided != 0;
     g[i].lda = a_kstrided ? M[i] : K[i]; g[i].ldb = b_kstrided ? N[i] : K[i];

@@ -365,7 +365,7 @@ typedef Cfg<192, 2, 2> Mid;            // (symmetric products)
 // symmetric gives E(m, n) above the diagonal and on the diagonal tiles and E(n, m) elsewhere, as with the other tiles: epilogue_impl.)
 bool slide_ok(const GemmDesc* d, int n) {
   for (int g = 0; g < n; ++g) {
-    if (!d[g].symmetric || d[g].M < Mid::BT || d[g].K % BK || d[g].Ctab || d[g].Etab || d[g].E == d[g].C) return false;
+    if (!d[g].symmetric || d[g].M < Mid::BT || d[g].K % BK || d[g].Ctab || d[g].Etab || (d[g].E && d[g].E == d[g].C)) return false;
     if (da_tile_span_bytes(false, Mid::BT, d[g].lda, d[g].K) >= (1LL << 32) || da_tile_span_bytes(false, Mid::BT, d[g].ldb, d[g].K) >= (1LL << 32)) return false;
   }
   return true;
@@ -373,11 +373,17 @@ bool slide_ok(const GemmDesc* d, int n) {
 
 // Tile choice by cost model: 256 x 256 tiles run one per CU, 128 x 128 tiles two per CU, 192 x 192 tiles (symmetric products:
 // 136 tiles of 256 x 256 of a 4096 x 4096 result leave half the chip idle, 253 of 192 x 192 fill it) one.  Of two 128-tiles a stage
-// takes 0.7 of a 256-tile's time for half its work, of one alone 0.4, of a 192-tile 0.7; the constants are the best of a grid over the
-// 38 products of which these are some.  Interior-only (direct-to-LDS) eligibility wins over either.
-// X X^T (us, 128 / 192 / 256): 4096 x 14336 334 / 260 / 310;  2 of 4096 x 4096 161 / 147 / 189;  8192 x 8192 720 / 515 / 544;  6 of
-// 1536 x 6144 89 / 96 / 131;  3072 x 8192 102 / 113 / 159;  5 of 4096 x 4096 364 / 353 / 317;  5120 x 5120 183 / 165 / 131;
-// 2048 x 8192 61 / 105 / 150;  24 of 1024 x 4096 113 / 136 / 104;  12 of 1024 x 1024 24 / 30 / 37;  48 of 768 x 768 40 / 47 / 52.
+// takes 0.7 of a 256-tile's time for half its work, of one alone 0.4, of a 192-tile 0.7.  Interior-only (direct-to-LDS) eligibility
+// wins over either, but for the 192-tiles, which are interior always.
+// Symmetric products: a tile's start and end cost two stages of a 128-tile's, five of a 192-tile's, four of a 256-tile's; where M or K
+// is off the grid the 128- and 256-tiles run the bounds-checked loop; one matrix alone in 128-tiles two to a CU has every XCD read all
+// of it, a tenth more.  The constants are the best of a grid over 580 products (batches of 1 to 48, M 200 to 8192, K 64 to 14848), half of
+// them off the grid: on average 0.2 % from each one's best edge.
+// X X^T (us, 128 / 192 / 256), whole 128-tiles: 3712 x 14848 245 / 199 / 441;  3840 x 8256 165 / 114 / 154;  3200 x 12288 208 / 149 /
+// 373;  2 of 4096 x 4096 161 / 147 / 189;  8192 x 8192 720 / 515 / 544;  5 of 4096 x 4096 364 / 353 / 317;  5120 x 5120 183 / 165 /
+// 131;  3072 x 4096 52 / 58 / 82;  2 of 2048 x 8192 89 / 103 / 150;  24 of 1024 x 4096 113 / 136 / 104;  48 of 768 x 768 40 / 47 / 52;
+// and not: 3 of 2048 x 6144 87 / 83 / 116.   Checked: 2 of 328 x 256 9 / 13 / 16;  3 of 832 x 384 11 / 15 / 21;  1728 x 128 8 / 12 / 14;
+// 1344 x 3968 57 / 53 / 127;  4 of 192 x 10560 142 / 121 / 302;  8 of 4544 x 960 265 / 232 / 253.
 // B X, B of m x m (us, 128 / 256): 3072 x 8192 141 / 148;  3 of 2048 x 5632 148 / 160;  12 of 1024 x 1024 34 / 37;  48 of 768 x 768
 // 56 / 59;  and not: 12 of 768 x 3072 61 / 58;  5120 x 5120 293 / 235;  4096 x 14336 518 / 435.
 // Plain stores have less for two tiles to hide of one another.  (M, N, K), operands k-contiguous (c) or k-strided (s): 48 of
@@ -398,20 +404,28 @@ int choose_tile(const GemmDesc* d, int n) {
   // Where a caller's addend is not symmetric the tile edge decides which of E(m, n) and E(n, m) an element gets: the rule for those
   // products (constants of an older K loop, up to 12 % from the best edge) stays as it is.  (Newton-Schulz's own A is symmetric.)
   const bool addend = d[0].symmetric && d[0].any_addend && d[0].epilogue == DA_EPI_AXPBY;
+  const bool checked = !(full_big || full_small), slide = d[0].symmetric && slide_ok(d, n);
+  if (slide && !addend) {
+    const bool lone = n == 1 && d[0].batch == 1 && tiles_of<Small>(d[0]) > 256;
+    const double cost_big = launch_cost<Big>(d, n, 256, checked ? 6.0 : 4.0, 4.0, 1.0);
+    const double cost_small = checked ? launch_cost<Small>(d, n, 512, 3.4, 1.0, 0.9)
+                                      : launch_cost<Small>(d, n, 512, lone ? 2.86 : 2.6, 2.0, 0.55);
+    const bool big = (full_big || !full_small) && cost_big <= cost_small;
+    return launch_cost<Mid>(d, n, 256, 2.75, 5.0, 1.0) < (big ? cost_big : cost_small) ? Mid::BT : big ? 256 : 128;
+  }
   // (The older constants also where the bounds-checked loop runs, for which they were measured.)
-  const bool older = addend || !(full_big || full_small);
+  const bool older = addend || checked;
   const double cost_big = launch_cost<Big>(d, n, 256, 4.0, older ? 0.0 : 3.0, 1.0);
   const double cost_small = older ? launch_cost<Small>(d, n, 512, 3.0, 0.0, 1.0)
                                    : launch_cost<Small>(d, n, 512, may_edge && d[0].epilogue == DA_EPI_STORE ? 3.2 : 2.75, 0.0, 0.55);
   const bool big = fits_big && (full_big || !full_small) && cost_big <= cost_small;
-  if (d[0].symmetric && slide_ok(d, n)) {
+  if (slide) {
     long long mid = 0, small = 0, matrices = 0;
     for (int g = 0; g < n; ++g) { mid += tiles_of<Mid>(d[g]); small += tiles_of<Small>(d[g]); matrices += d[g].batch; }
     const double cost_mid = launch_cost<Mid>(d, n, 256, 2.75, 0.0, 1.0);
-    if (addend && !big) {
+    if (!big) {
       if (small > 256 && 2.25 * mid <= 1.15 * small && cost_mid * (mid > 256 ? 1.13 : 1.0) < cost_small) return Mid::BT;
-    } else if (cost_mid * (mid > 512 && matrices > 1 ? 1.1 : 1.0) < (big ? cost_big : cost_small)) {
-      // (several matrices over many rounds: 4 of 4096 x 10560, a round in twelve less by this count, are 5 % slower)
+    } else if (cost_mid * (mid > 512 && matrices > 1 ? 1.1 : 1.0) < cost_big) {
       return Mid::BT;
     }
   }
@@ -466,7 +480,7 @@ int da_gemm_bf16_group_plan(const GemmDesc* din, int n) {
   GemmDesc d[DA_MAX_GROUPS];
   by_longest_k(din, n, d);
   const int bt = choose_tile(d, n);
-  return bt + (all_interior(d, n, bt) ? 1 : 0);
+  return bt + (bt == Mid::BT || all_interior(d, n, bt) ? 1 : 0);
 }
 
 // ---- measurement hook: time stamps of the tiles of the bf16 GEMM launches (see include/dion_amd.h)

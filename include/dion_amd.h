@@ -132,10 +132,10 @@ int dion_amd_gemm(const void* A, long long a_stride, int lda, int a_kstrided,
  * an operand whose tile spans 4 GiB or more takes the bounds-checked loop instead. */
 int dion_amd_gemm_plan(int M, int N, int K, int lda, int a_kstrided, int ldb, int b_kstrided);
 
-/* The same for up to 4 batched products that share a launch (dense operands; as in a Muon step of several shapes): the tile edge of
- * all of them, plus 1 if every tile is interior.  The order they are given in does not matter where their K differ. */
+/* The same for up to 4 batched products that share a launch (dense operands; as in a Muon step of several shapes; `symmetric`: A A^T):
+ * the tile edge of all of them (128, 192 for symmetric ones, 256), plus 1 if every tile is interior.  The order they are given in does not matter where their K differ. */
 int dion_amd_gemm_group_plan(const int* batch, const int* M, const int* N, const int* K, int n, int a_kstrided, int b_kstrided,
-                             int epilogue);
+                             int symmetric, int epilogue);
 
 /* ---------------------------------------------------------------------------------------
  * Muon step for one bucket of same-shape matrices

@@ -86,11 +86,25 @@ def test_tile_of_a_grouped_launch_does_not_depend_on_the_order_of_its_products(g
     from dion_amd import _lib
 
     def plan(order):
-        return _lib.load().dion_amd_gemm_group_plan(*((ctypes.c_int * len(order))(*v) for v in zip(*order)), len(order), 0, 1, _lib.EPI_AXPBY)
+        return _lib.load().dion_amd_gemm_group_plan(*((ctypes.c_int * len(order))(*v) for v in zip(*order)), len(order), 0, 1, 0,
+                                                    _lib.EPI_AXPBY)
 
     want = plan(sorted(groups, key=lambda g: -g[3]))
     assert want // 2 * 2 in (128, 256)
     assert all(plan(order) == want for order in itertools.permutations(groups))
+
+
+@pytest.mark.parametrize("batch, m, k, edge", [   # each one's fastest, by 6 % or more (choose_tile has the times)
+    (1, 3712, 14848, 192), (1, 3840, 8256, 192), (1, 3200, 12288, 192), (1, 3072, 4096, 128), (2, 2048, 8192, 128), (2, 4096, 4096, 192),
+    (1, 5120, 5120, 256), (5, 4096, 4096, 256), (24, 1024, 4096, 256), (48, 768, 768, 128),
+    # off the grid: the bounds-checked loop in 128-tiles, or 192-tiles
+    (2, 328, 256, 128), (3, 832, 384, 128), (1, 1728, 128, 128), (1, 1344, 3968, 192), (4, 192, 10560, 192), (8, 4544, 960, 192),
+])
+def test_tile_of_symmetric_products(batch, m, k, edge):
+    from dion_amd import _lib
+
+    dims = [(ctypes.c_int * 1)(v) for v in (batch, m, m, k)]
+    assert _lib.load().dion_amd_gemm_group_plan(*dims, 1, 0, 0, 1, _lib.EPI_STORE) // 2 * 2 == edge
 
 
 def test_no_cpu_fallback():

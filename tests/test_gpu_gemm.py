@@ -115,11 +115,11 @@ def test_gemm_by_number_of_stages(dev, a_ks, b_ks, batch, M, N):
 
 @pytest.mark.parametrize("m", [4096, 3912])
 def test_symmetric_products_by_number_of_stages(dev, m):
-    """192-tiles, whole and sliding ones."""
+    """128-tiles, and from 3 and 16 stages on 192-tiles, whole and sliding ones."""
     from dion_amd.newton_schulz import ns_line_1
 
     torch.manual_seed(7)
-    for K in (64, 128, 192, 320):
+    for K in (64, 128, 192, 320, 1024, 1088):
         A = torch.randint(-2, 3, (m, K)).float()
         assert torch.equal(ns_line_1(A.bfloat16().to(dev)).cpu(), (A @ A.mT).bfloat16()), K
 
