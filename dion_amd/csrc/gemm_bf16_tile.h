@@ -413,7 +413,9 @@ __device__ __forceinline__ unsigned long long wave_uniform64(unsigned long long 
 }
 template <int N> __device__ __forceinline__ void dma_wait_all_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // 16 bytes per lane from a raw buffer into LDS at `lbase` + `l` + 16 * lane (dma16, addressed by scalars: a request costs the wavefront
-// three instructions).  From a buffer of no records nothing is fetched, the request is counted all the same.
+// three instructions).  From a buffer of no records nothing is fetched, the request is counted all the same.  The wait states between
+// the vector unit's scalars and the request are the caller's (buffers_ready): five in every request, as in dma16, cost 2 to 4 % of a step
+// of large products, one set of them a stage 0.3 %.  tests/test_wait_states.py looks for a scalar that the compiler moves in between.
 __device__ __forceinline__ void dma16_buf(u32x4_t buf, unsigned off, unsigned soff, unsigned lbase, unsigned l) {
   asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                :
@@ -421,9 +423,12 @@ __device__ __forceinline__ void dma16_buf(u32x4_t buf, unsigned off, unsigned so
                : "memory", "scc");
 }
 
+__device__ __forceinline__ void buffers_ready(u32x4_t& a, u32x4_t& b) { asm volatile("s_nop 4" : "+s"(a), "+s"(b)); }
+
 // One product added to accumulators that stay in their AGPRs.  As assembly: the compiler, given 256 of them, moved some about on every
 // pass of the loop (56 v_accvgpr_mov a stage with both operands k-contiguous, 3400 clocks instead of 2600).  It does not know the
-// instruction's hazards then: no accumulator is touched again within four products, and mfma_drain() comes before they are read.
+// instruction's hazards then: no accumulator is touched again within four products, mfma_drain() comes before they are read, and no
+// fragment is moved by the vector unit within two wait states of its product, which tests/test_wait_states.py holds the build to.
 __device__ __forceinline__ void mfma16_in_place(f32x4_t& c, bf16x8_t col, bf16x8_t row) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(col), "v"(row));
 }
@@ -568,6 +573,7 @@ __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C
   set_buffers(0);
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
+    buffers_ready(ba, bb);   // (in the loop a barrier, its waits and a product stand between the buffers and the first request)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
