@@ -349,10 +349,9 @@ std::atomic<int> g_flow_fail{0};           // test hook: the launch starts with 
 std::atomic<long long> g_flow_spin{-1};    // ticks of the 100 MHz counter; -1: default
 
 double tile_cost(int stages, int product) {
-  // microseconds, from tile time lines: 1.7 per 64-deep stage, epilogue, ticket + wait (now 1.5, 5.8 - 10 and the first stage's 5:
-  // only the ratios of the queues' loads are used)
-  const double epi = product == 2 ? 5.5 : (product == 1 ? 4.5 : 4.0);
-  return 1.7 * stages + epi + 1.0;
+  // microseconds, from tile time lines: 1.5 per 64-deep stage, the epilogue, the first stage's trip, ticket and wait
+  const double epi = product == 2 ? 8.5 : (product == 1 ? 10.0 : 5.7);
+  return 1.5 * stages + epi + 6.0;
 }
 
 }  // namespace
@@ -407,7 +406,10 @@ bool da_ns_flow_applicable(const DaNsFlowGroup* g, int n, int steps, int faithfu
   if (nmat < 16) return false;
   double mx = 0, sum = 0;
   for (int q = 0; q < NQ; ++q) { mx = load[q] > mx ? load[q] : mx; sum += load[q]; }
-  if (mx > 1.06 * sum / NQ) return false;
+  // (us a Muon step, this launch / the product launches, of sets about that line: 52 of 768 x 768 with 43 of 768 x 3072 2473 / 2696, 6 of
+  // 1024 x 2816 with 26 of 1024 x 1024 1081 / 1249, 62 of 768 x 768 with 7 of 768 x 3072 1145 / 1313.  At 6 %, the line that an estimate
+  // with an older K loop's times went with, 0.2 % of the sets of two shapes would go the slower way that did not before.)
+  if (mx > 1.065 * sum / NQ) return false;
   for (int q = 0; q < NQ; ++q) {
     double tiles = 0;
     long long s = 0;
