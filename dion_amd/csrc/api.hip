@@ -581,9 +581,9 @@ bool fused_bq_enabled() {
 std::atomic<int> g_opt_dion_small{-1};
 
 // Number of slices (1, 2 or 4) of the inner dimension `mp` for the product R = B^T P (np x r per matrix, `cb`
-// matrices), by the bf16 launcher's own estimate: workgroup rounds x 64-deep stages per tile, a 256 x 256 tile
-// costing 4 per stage on a whole CU and a 128 x 128 tile 3 on half a CU; a sliced product also pays for writing
-// and adding its fp32 partial sums.
+// matrices): workgroup rounds x 64-deep stages per tile, a 256 x 256 tile costing 4 per stage on a whole CU and a
+// 128 x 128 tile 3 on half a CU; a sliced product also pays for writing and adding its fp32 partial sums.  (The times of
+// an older K loop than choose_tile's; they stay because the number of slices is the order of the sums.)
 int btp_slices(int np, int r, int mp, int cb) {
   int best = 1;
   double best_cost = 0.0;

@@ -144,7 +144,7 @@ __device__ __forceinline__ void epilogue_impl(typename C::acc_t (&acc)[C::TMI][C
   // rows of a band; 16 of 128 columns, for the registers' sake: two staging areas then, taken in turns
   constexpr int BR = PIPE && W == 128 ? 16 : 32, NB = C::WROWS / BR;
   constexpr int NPASS = (BR + RPP - 1) / RPP;
-  constexpr bool ODD = 64 % CPR != 0;   // (six chunks to a row: ten rows a pass, four lanes and most of the last pass idle)
+  constexpr bool ODD = 64 % CPR != 0;   // (twelve chunks to a row: five rows a pass, four lanes and most of the last pass idle)
   constexpr int CSZ = CF32 ? 4 : 2;
   constexpr int NV = CF32 ? 2 : 1;   // 16-byte vectors per 8 elements
   // TURN: the bf16 results go through LDS a second time, to be stored transposed: 32 rows of the band as a k-strided tile ([32][W] in
@@ -497,7 +497,7 @@ __device__ __forceinline__ bf16x8_t unit_frag(const char* op, int w, int h, int 
 // What bounds it: eight wavefronts of 128 x 64 read 192 KB a stage from LDS (128 bytes a clock) and the requests write 64 KB, 2048 clocks
 // of the matrix cores' 2048; four of 128 x 128 read 128 KB.  Clocks per stage of a 256-tile on every CU, eight wavefronts -> four: both
 // operands k-contiguous 2990 -> 2610, one k-strided 3130 -> 2640, both - -> 2690 (products and barriers alone 2180).  Under random data
-// the chip lowers its clock as the loop gets denser (2.2 GHz for zeros, 1.7 here): 1.22-1.26 -> 1.36-1.39 PFLOP/s.
+// the chip lowers its clock as the loop gets denser (2.2 GHz for zeros, 1.7 here): 1.21-1.26 -> 1.32-1.39 PFLOP/s.
 // `hook`, `a_wrap`, `b_jump`: gemm_tile_k_loop.
 template <typename C, bool A_KS, bool B_KS, typename Hook>
 __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C::TMI][C::TNJ], const GemmDesc& d, const bf16_t* A,
@@ -639,8 +639,9 @@ __device__ __forceinline__ void gemm_tile_k_loop_quad(typename C::acc_t (&acc)[C
 //   DA_LOOP_CHECKED: bounds-checked 16-byte loads into registers (out-of-range chunks zero filled),
 //     written to LDS after the stage's MFMAs.
 // Ends with a workgroup barrier: the stage buffers are free for the epilogue.
-// `after_first_stage` (direct-to-LDS forms) is called once, behind the barrier that publishes the first stage: every
-// wavefront has waited for all of its outstanding memory operations by then, stores of earlier work included.
+// `after_first_stage` (direct-to-LDS forms) is called once, behind the loop's first barrier.  Every wavefront has waited there until no
+// more than its youngest requests of this loop are outstanding (loads and stores count down in the order they were issued): whatever it
+// issued before the loop, stores of earlier work included, has completed; most of the first two stages is still on its way.
 // `a_wrap`, `b_jump` (direct-to-LDS forms): A is read again from its first column after a_wrap of its columns instead of
 // GemmDesc::a_kwrap of them, and B then goes on b_jump bytes further.
 struct DaNoHook { __device__ __forceinline__ void operator()() const {} };

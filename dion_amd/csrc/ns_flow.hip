@@ -476,6 +476,7 @@ int da_ns_flow(const DaNsFlowGroup* g, int n, const float* coeffs, int steps, in
   int rc = da_launch_status();
   if (rc) return rc;
   constexpr int smem = 2 * (Tile<BT, false>::bytes + Tile<BT, false>::bytes);
+  static_assert(epilogue_lds<Big>() <= smem, "the epilogue stages through the K loop's buffers");
   static DaOncePerDevice configured;
   rc = configured.run([&]() -> int {
     DA_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(ns_flow_kernel),
