@@ -245,8 +245,9 @@ MEASURED_TRAFFIC_BYTES = {
     ("muon_4096x14336", "ns_axpy"): 30044150 * 1024,
     # one Llama-3-8B layer: the grouped X' = aX + BX launch over its four buckets
     ("muon_llama8b_layer", "ns_axpy"): 3544863 * 1024,
-    # error feedback + weight update in one launch: mean over the buckets of the workload
-    ("dion_gpt_small_r025", "dion_ef_upd"): 266764 * 1024,
+    # error feedback + weight update, mean over the buckets of the workload.  Launches are timed one bucket at a time, where a rank
+    # below 512 is updated in one pass (277 687 KiB; the step's buckets, side by side, by two products in one launch, 266 764)
+    ("dion_gpt_small_r025", "dion_ef_upd"): 277687 * 1024,
     ("dion_llama70b_layer", "dion_ef_upd"): 3511913 * 1024,
     # mean over the three buckets
     ("dion_gpt_small_r1", "dion_ef_upd"): 524478 * 1024,
